@@ -8,7 +8,12 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from .ops import mhc_layer_fused, mhc_layer_fused_dynamic, mhc_layer_fused_inference
+from .ops import _ext
+
+# in the order of the operators' arguments
+_DYNAMIC_PARAMS = ("rmsnorm_weight", "phi_pre", "phi_post", "phi_res", "alpha_pre", "alpha_post", "alpha_res",
+                   "b_pre", "b_post", "b_res")
+_STATIC_PARAMS = ("rmsnorm_weight", "H_pre", "H_post", "H_res")
 
 
 class MHCLayer(nn.Module):
@@ -62,25 +67,33 @@ class MHCLayer(nn.Module):
             self.H_post = nn.Parameter(torch.zeros(n, dtype=torch.float32))
             self.H_res = nn.Parameter((alpha_init * torch.randn(n, n)).float())
 
+    def _params(self, names):
+        # nn.Module.__getattr__ is a Python call per parameter, which adds up at the sizes where the host
+        # decides the time of a call; a parameter that was replaced by a property (parametrizations,
+        # pruning) is not in the dictionary and goes the ordinary way
+        p = self._parameters
+        try:
+            return [p[k] for k in names]
+        except KeyError:
+            return [getattr(self, k) for k in names]
+
     def forward(self, x_expanded: torch.Tensor) -> torch.Tensor:
         B, n, C = x_expanded.shape
         assert n == self.expansion_rate
         assert C == self.hidden_dim
+        compute = self.compute_dtype
+        cast = compute is not None and x_expanded.dtype != compute
         if self.use_dynamic_h:
             # float32 activations with compute_dtype=bfloat16: the operator rounds them inside its kernels
             # where it can and casts them itself elsewhere
-            in_op = self.compute_dtype == torch.bfloat16 and x_expanded.dtype == torch.float32
-            if self.compute_dtype is not None and x_expanded.dtype != self.compute_dtype and not in_op:
-                x_expanded = x_expanded.to(self.compute_dtype)
-            return mhc_layer_fused_dynamic(
-                x_expanded, self.rmsnorm_weight, self.phi_pre, self.phi_post, self.phi_res,
-                self.alpha_pre, self.alpha_post, self.alpha_res, self.b_pre, self.b_post, self.b_res,
-                self.sinkhorn_iters, self.eps, self.output_dtype, None, in_op)
-        if self.compute_dtype is not None and x_expanded.dtype != self.compute_dtype:
-            x_expanded = x_expanded.to(self.compute_dtype)
+            in_op = cast and compute == torch.bfloat16 and x_expanded.dtype == torch.float32
+            if cast and not in_op:
+                x_expanded = x_expanded.to(compute)
+            return _ext.mhc_layer_dynamic(x_expanded, *self._params(_DYNAMIC_PARAMS), self.sinkhorn_iters, self.eps,
+                                          self.output_dtype, None, in_op)
+        if cast:
+            x_expanded = x_expanded.to(compute)
+        params = self._params(_STATIC_PARAMS)
         if not self.training and not torch.is_grad_enabled():
-            return mhc_layer_fused_inference(x_expanded, self.rmsnorm_weight, self.H_pre, self.H_post,
-                                             self.H_res, self.sinkhorn_iters, self.eps,
-                                             self.output_dtype)
-        return mhc_layer_fused(x_expanded, self.rmsnorm_weight, self.H_pre, self.H_post, self.H_res,
-                               self.sinkhorn_iters, self.eps, self.output_dtype)
+            return _ext.mhc_layer_inference(x_expanded, *params, self.sinkhorn_iters, self.eps, self.output_dtype)
+        return _ext.mhc_layer_static(x_expanded, *params, self.sinkhorn_iters, self.eps, self.output_dtype, None)
