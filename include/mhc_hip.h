@@ -151,6 +151,34 @@ MHC_API int mhc_pack_dynamic_params(const void *phi_pre, const void *phi_post, c
                             void *phi, int phi_dtype, float *bias, float *alpha, int n, int C, void *stream);
 
 /*
+ * mhc_layer_fwd_dynamic on the parameters as they are stored: what mhc_pack_dynamic_params followed by
+ * mhc_layer_fwd_dynamic do, with the packing inside the projection kernel where that is the faster way.
+ * phi [D, nC] (phi_dtype), bias [D] and alpha [3] receive the packed parameters, which the backward
+ * call takes.  The structure is read during the call only.
+ */
+struct mhc_dynamic_params {
+    const void *phi_pre, *phi_post, *phi_res; /* [n, nC], [n, nC], [n*n, nC] */
+    int phi_dtype;
+    const float *b_pre, *b_post, *b_res;      /* [n], [n], [n, n] */
+    const float *alpha_pre, *alpha_post, *alpha_res;
+};
+MHC_API int mhc_layer_fwd_dynamic_params(const void *x, int x_dtype, const void *w, int w_dtype,
+                                 const struct mhc_dynamic_params *p, void *phi, int phi_dtype, float *bias, float *alpha,
+                                 const void *f_inject, void *y, int y_dtype, float *H_pre, float *H_post, float *M,
+                                 float *P, float *r, float *q, float *sk_state, int B, int n, int C, int iters,
+                                 float eps, void *workspace, size_t workspace_bytes, void *stream);
+
+/* mhc_layer_bwd_dynamic with dw in a dtype of the caller's choice (fp32 or bf16, rounded once). */
+MHC_API int mhc_layer_bwd_dynamic_dw(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w,
+                          int w_dtype, const void *phi, int phi_dtype, const float *bias,
+                          const float *alpha, const void *f_inject, const float *H_pre,
+                          const float *H_post, const float *M, const float *P, const float *r,
+                          const float *q, const float *sk_state, void *dx, void *df, void *dw, int dw_dtype,
+                          float *dphi,
+                          float *dbias, float *dalpha, int B, int n, int C, int iters, float eps,
+                          void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * mhc_layer_fwd_dynamic for callers that cannot allocate device memory or pass a workspace: code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no
  * counterpart in the reference.  Same arguments and results as mhc_layer_fwd_dynamic minus the
@@ -197,6 +225,14 @@ MHC_API int mhc_layer_bwd(const void *dy, int y_dtype, const void *x, int x_dtyp
                   const float *H_res_logits, const void *f_inject, const float *H_pre,
                   const float *H_post, const float *M, const float *q, void *dx, void *df,
                   float *dw, float *dH_pre, float *dH_post, float *dH_res, int B, int n, int C,
+                  int iters, float eps, void *workspace, size_t workspace_bytes, void *stream);
+
+/* mhc_layer_bwd with dw in a dtype of the caller's choice (fp32 or bf16, rounded once). */
+MHC_API int mhc_layer_bwd_dw(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w,
+                  int w_dtype, const float *H_pre_logits, const float *H_post_logits,
+                  const float *H_res_logits, const void *f_inject, const float *H_pre,
+                  const float *H_post, const float *M, const float *q, void *dx, void *df,
+                  void *dw, int dw_dtype, float *dH_pre, float *dH_post, float *dH_res, int B, int n, int C,
                   int iters, float eps, void *workspace, size_t workspace_bytes, void *stream);
 
 /* ------------------------------------------------------------------------------------------

@@ -8,20 +8,29 @@
 // hundred times smaller than the terms, and a float32 running sum loses what the 1e-5 parity tier
 // needs.  The terms themselves stay float32.
 #pragma once
-#include <hip/hip_runtime.h>
+#include "mhc_common.h"
 
 namespace mhc {
 
-struct BatchSumArgs {
-    const float *u; int rows_u, C; float *dw;
-    const float *dt; int rows_dt, D; float *dbias, *dalpha;
-    int nblk;  // blocks of 64 columns
+// Where dw goes: fp32, or bf16 (rounded once from the float64 sum's float32 value) for a bf16 weight whose
+// gradient the caller hands back in the weight's type, which saves a conversion launch.
+struct DwOut {
+    void *p;
+    bool bf16;
+    explicit operator bool() const { return p != nullptr; }
 };
 
-inline BatchSumArgs make_batch_sums(const float *u, int rows_u, int C, float *dw, const float *dt, int rows_dt,
+struct BatchSumArgs {
+    const float *u; int rows_u, C; void *dw;
+    const float *dt; int rows_dt, D; float *dbias, *dalpha;
+    int nblk;  // blocks of 64 columns
+    bool dw_bf16;
+};
+
+inline BatchSumArgs make_batch_sums(const float *u, int rows_u, int C, DwOut dw, const float *dt, int rows_dt,
                                     int D, float *dbias, float *dalpha) {
     const int ncols = (dw ? C : 0) + (dt ? D + 3 : 0);  // dt == nullptr: the u columns only
-    return BatchSumArgs{u, rows_u, C, dw, dt, rows_dt, D, dbias, dalpha, (ncols + 63) / 64};
+    return BatchSumArgs{u, rows_u, C, dw.p, dt, rows_dt, D, dbias, dalpha, (ncols + 63) / 64, dw.bf16};
 }
 
 // red: RG * (CW + 1) doubles of LDS; called by all CW * RG threads of the workgroup (contains a barrier).
@@ -65,7 +74,10 @@ __device__ __forceinline__ void batch_sum_block(const BatchSumArgs &a, int blk, 
         double v = 0.0;
 #pragma unroll
         for (int i = 0; i < RG; i++) v += red[i * (CW + 1) + cl];
-        if (col < ncol_u) a.dw[col] = (float)v;
+        if (col < ncol_u) {
+            if (a.dw_bf16) static_cast<unsigned short *>(a.dw)[col] = f32_to_bf16((float)v);
+            else static_cast<float *>(a.dw)[col] = (float)v;
+        }
         else if (col - ncol_u < a.D) a.dbias[col - ncol_u] = (float)v;
         else a.dalpha[col - ncol_u - a.D] = (float)v;
     }

@@ -184,6 +184,25 @@ __device__ unsigned long long g_phase[kPhaseKernels][kPhaseMaxWg][kPhaseMaxMarks
 }
 #endif
 
+namespace {
+
+int fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype, const ParamGather *gather, const void *phi,
+                int phi_dtype, const float *bias, const float *alpha, const void *f_inject, void *y, int y_dtype,
+                float *H_pre, float *H_post, float *M, float *P, float *r, float *q, float *sk_state, int B, int n,
+                int C, int iters, float eps, void *workspace, size_t workspace_bytes, void *stream);
+int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w, int w_dtype, const void *phi,
+                int phi_dtype, const float *bias, const float *alpha, const void *f_inject, const float *H_pre,
+                const float *H_post, const float *M, const float *P, const float *r, const float *q,
+                const float *sk_state, void *dx, void *df, DwOut dw, float *dphi, float *dbias, float *dalpha, int B,
+                int n, int C, int iters, float eps, void *workspace, size_t workspace_bytes, void *stream);
+int bwd_static(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w, int w_dtype,
+               const float *H_pre_logits, const float *H_post_logits, const float *H_res_logits, const void *f_inject,
+               const float *H_pre, const float *H_post, const float *M, const float *q, void *dx, void *df, DwOut dw,
+               float *dH_pre, float *dH_post, float *dH_res, int B, int n, int C, int iters, float eps,
+               void *workspace, size_t workspace_bytes, void *stream);
+
+}  // namespace
+
 extern "C" {
 
 #ifdef MHC_PHASE_PROFILE
@@ -254,42 +273,23 @@ int mhc_layer_fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype
                           const void *f_inject, void *y, int y_dtype, float *H_pre, float *H_post,
                           float *M, float *P, float *r, float *q, float *sk_state, int B, int n, int C,
                           int iters, float eps, void *workspace, size_t workspace_bytes, void *stream) {
-    if (int s = check_shape(B, n, C, iters)) return s;
-    if (!x || !phi || !bias || !alpha || !y || !H_pre || !H_post || !M || !P || !r || !q)
+    return fwd_dynamic(x, x_dtype, w, w_dtype, nullptr, phi, phi_dtype, bias, alpha, f_inject, y, y_dtype, H_pre, H_post, M, P,
+                       r, q, sk_state, B, n, C, iters, eps, workspace, workspace_bytes, stream);
+}
+
+int mhc_layer_fwd_dynamic_params(const void *x, int x_dtype, const void *w, int w_dtype,
+                                 const struct mhc_dynamic_params *p, void *phi, int phi_dtype, float *bias, float *alpha,
+                                 const void *f_inject, void *y, int y_dtype, float *H_pre, float *H_post, float *M,
+                                 float *P, float *r, float *q, float *sk_state, int B, int n, int C, int iters,
+                                 float eps, void *workspace, size_t workspace_bytes, void *stream) {
+    if (!p || !p->phi_pre || !p->phi_post || !p->phi_res || !p->b_pre || !p->b_post || !p->b_res || !p->alpha_pre ||
+        !p->alpha_post || !p->alpha_res)
         return MHC_ERR_NULL_POINTER;
-    if (!f_inject && !w) return MHC_ERR_NULL_POINTER;
-    if (!valid_io(x_dtype, y_dtype) || !valid_dtype(phi_dtype) || (w && !valid_dtype(w_dtype)))
-        return MHC_ERR_BAD_DTYPE;
-    if (x_dtype == MHC_F32_AS_BF16 && (phi_dtype != MHC_BF16 || !f32_as_bf16_accepted(B, n, C, iters)))
-        return MHC_ERR_BAD_DTYPE;
-    if (!aligned16(x) || !aligned16(y) || !aligned16(phi) || (f_inject && !aligned16(f_inject)))
-        return MHC_ERR_MISALIGNED;
-    const DynFwdWs ws = carve_dyn_fwd(workspace, B, n, C);
-    if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C)) {
-        // projection, coefficients and mix in one launch; x crosses HBM once
-        MHC_LAUNCH(launch_layer_fwd_onepass(x, w, w_dtype, f_inject, y, y_dtype, phi, alpha, bias, H_pre, H_post,
-                                            M, P, r, q, sk_state, B, n, C, iters, eps, st));
-        return MHC_OK;
-    }
-    const int KS = proj_fwd_ksplit(x_dtype, phi_dtype, B, n, C);
-    MHC_LAUNCH(launch_proj_fwd(x, x_dtype, phi, phi_dtype, ws.Ppart, ws.ssqpart, KS, B, n, C, st));
-    if (layer_fwd_fused_supported(n, C, x_dtype)) {
-        MHC_LAUNCH(launch_layer_fwd_fused(x, x_dtype, w, w_dtype, f_inject, y, y_dtype, ws.Ppart,
-                                          ws.ssqpart, KS, padded_D(n), alpha, bias, bias + n,
-                                          bias + 2 * n, H_pre, H_post, M, P, r, q, sk_state, B, n, C, iters,
-                                          eps, st));
-        return MHC_OK;
-    }
-    // n > 8 in the bf16 tier: the coefficient launch also forms the stream aggregate and its RMS
-    const bool agg = !f_inject && ws.agg && coef_fwd_aggregates(n, C, x_dtype);
-    MHC_LAUNCH(launch_coef_fwd(ws.Ppart, ws.ssqpart, KS, padded_D(n), alpha, bias, bias + n,
-                               bias + 2 * n, H_pre, H_post, M, P, r, B, n, n * C, iters, eps,
-                               x_dtype == kF32, agg ? x : nullptr, ws.agg, q, sk_state, st));
-    MHC_LAUNCH(launch_mix_fwd(x, x_dtype, w, w_dtype, f_inject, y, y_dtype, H_pre, H_post, M, n, q,
-                              ws.agg, B, n, C, eps, agg, st));
-    return MHC_OK;
+    if (!valid_dtype(p->phi_dtype)) return MHC_ERR_BAD_DTYPE;
+    const ParamGather g{{p->phi_pre, p->phi_post, p->phi_res}, p->phi_dtype, {p->b_pre, p->b_post, p->b_res},
+                        {p->alpha_pre, p->alpha_post, p->alpha_res}, phi, phi_dtype, bias, alpha};
+    return fwd_dynamic(x, x_dtype, w, w_dtype, &g, phi, phi_dtype, bias, alpha, f_inject, y, y_dtype, H_pre, H_post, M, P,
+                       r, q, sk_state, B, n, C, iters, eps, workspace, workspace_bytes, stream);
 }
 
 int mhc_layer_bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w,
@@ -299,130 +299,23 @@ int mhc_layer_bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtyp
                           const float *q, const float *sk_state, void *dx, void *df, float *dw, float *dphi,
                           float *dbias, float *dalpha, int B, int n, int C, int iters, float eps,
                           void *workspace, size_t workspace_bytes, void *stream) {
-    if (int s = check_shape(B, n, C, iters)) return s;
-    if (!dy || !x || !phi || !bias || !alpha || !H_pre || !H_post || !M || !P || !r || !q || !dx ||
-        !dphi || !dbias || !dalpha)
-        return MHC_ERR_NULL_POINTER;
-    if (!f_inject && (!w || !dw)) return MHC_ERR_NULL_POINTER;
-    if (!valid_io(x_dtype, y_dtype) || !valid_dtype(phi_dtype) || (w && !valid_dtype(w_dtype)))
-        return MHC_ERR_BAD_DTYPE;
-    if (x_dtype == MHC_F32_AS_BF16 && (phi_dtype != MHC_BF16 || !f32_as_bf16_accepted(B, n, C, iters)))
-        return MHC_ERR_BAD_DTYPE;
-    if (!aligned16(dy) || !aligned16(x) || !aligned16(dx) || !aligned16(phi) || !aligned16(dphi) ||
-        (f_inject && !aligned16(f_inject)) || (df && !aligned16(df)))
-        return MHC_ERR_MISALIGNED;
-    const DynBwdWs ws = carve_dyn_bwd(workspace, B, n, C);
-    if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const int D = n * n + 2 * n, DP = padded_D(n);
-    const bool mfma = proj_bwd_mfma_supported(x_dtype == kF32AsBF16 ? kBF16 : x_dtype, phi_dtype, C);
-    BwdCoefOut out{ws.dt, ws.dP, ws.cx, ws.s1, nullptr, mfma ? ws.dPb : nullptr, ws.dPT, ws.BP};
-    if (mfma && bwd_resident_supported(x_dtype, y_dtype, phi_dtype, n, C, iters) && proj_bwd_addx_supported(n) &&
-        (bwd_resident_preferred(B, n, C) || x_dtype == kF32AsBF16)) {
-        // two launches: (1) one workgroup per sample keeps the sample's rows of dy and x in registers for
-        // the channel sums, the coefficient backward and the mixing part of dx; (2) a column-slab
-        // kernel over all samples adds dP phi - cx x, finishes dphi without batch-split partial sums
-        // and sums dw, dbias and dalpha in a few extra workgroups
-        BwdCoefOut out2 = out;
-        out2.dP = nullptr;  // the second launch takes dP as matrix-core operands only
-        MHC_LAUNCH(launch_bwd_resident(dy, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, q, P, r, alpha, bias + 2 * n,
-                                       sk_state, out2, dx, df, ws.u, B, n, C, iters, eps, st));
-        const BatchSumArgs sums = make_batch_sums(ws.u, B, C, f_inject ? nullptr : dw, ws.dt, B, D, dbias, dalpha);
-        bool tail_taken = false;
-        MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, dphi, dx, B, n, C,
-                                        tuning_get(kTuneSeparateFinalize) == 1 ? nullptr : &sums, &tail_taken, st));
-        if (!tail_taken)
-            MHC_LAUNCH(launch_finalize(ws.u, B, C, f_inject ? nullptr : dw, ws.dt, B, D, dbias, dalpha, nullptr, 1,
-                                       0, nullptr, st));
-        return MHC_OK;
-    }
-    if (x_dtype == kF32AsBF16) return MHC_ERR_BAD_DTYPE;  // not reached: accepted shapes take the path above
-    if (mfma && x_dtype == kBF16 && y_dtype == kBF16 && wide_dx_beside(B, n, C) && tuning_get(kTuneWideDxBeside) != 1) {
-        // wide projection (n > 18), four launches.  The coefficient backward is one workgroup per sample,
-        // all dependent chains; the part of dx that needs none of its results (M^T dy + Hpre (x) da,
-        // with s1 from the channel sums) runs beside it in the same launch and is handed over in fp32;
-        // the dP phi kernel then completes dx (+ dP phi - cx x, one rounding); dphi comes last and carries
-        // the batch sums.
-        // B=128 n=32 C=1280, backward in graphs of ten, same box: five launches 99.8 us, these four 93.0 us
-        MHC_LAUNCH(launch_mix_bwd_reduce_with_dx(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, n, q, P, r, alpha,
-                                                 bias + 2 * n, sk_state, out, ws.raw, ws.s1part, ws.dx_part, df, ws.u, B, n, C,
-                                                 iters, eps, st));
-        MHC_LAUNCH(launch_dxflat_wide(phi, ws.dPb, ws.BP, dx, x, ws.cx, ws.dx_part, B, n, C, st));
-        const BatchSumArgs sums = make_batch_sums(ws.u, B, C, f_inject ? nullptr : dw, ws.dt, B, D, dbias, dalpha);
-        bool tail_taken = false;
-        MHC_LAUNCH(launch_dphi_large(x, ws.dPT, ws.BP, dphi, 1, B, n, C,
-                                     tuning_get(kTuneSeparateFinalize) != 1 ? &sums : nullptr, &tail_taken, st));
-        if (!tail_taken)
-            MHC_LAUNCH(launch_finalize(ws.u, B, C, f_inject ? nullptr : dw, ws.dt, B, D, dbias, dalpha, nullptr, 1,
-                                       (size_t)D * n * C, dphi, st));
-        return MHC_OK;
-    }
-    MHC_LAUNCH(launch_mix_bwd_reduce(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
-                                     n, q, P, r, alpha, bias + 2 * n, sk_state, out, ws.raw, B, n, C, iters, eps,
-                                     st));
-    if (mfma && bwd_slab_supported(x_dtype, y_dtype, phi_dtype, n, C)) {
-        // n <= 4: one slab kernel finishes dx and produces every batch-split partial sum
-        const int S = bwd_slab_batch_splits(B, n, C);
-        MHC_LAUNCH(launch_bwd_slab(dy, y_dtype, x, w, w_dtype, f_inject, phi, H_pre, H_post, M, q, ws.s1,
-                                   ws.cx, ws.dPb, ws.dPT, ws.BP, ws.dt, dx, df,
-                                   S > 1 ? ws.dphi_part : dphi, ws.u, ws.dtpart, S, B, n, C, st));
-        MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? nullptr : dw, ws.dtpart, S, D, dbias, dalpha,
-                                   ws.dphi_part, S, (size_t)D * n * C, dphi, st));
-        return MHC_OK;
-    }
-    const int spg = bwd_dx_samples_per_group(B, n);
-    const int groups = (B + spg - 1) / spg;
-    int S = 1;
-    if (mfma) {
-        // matrix cores: dphi and the projection term of dx (written into dx, then completed in place)
-        S = proj_bwd_batch_splits(B, n, C);
-        // From D > 128 on the two products run as launches of their own (they share no operand but dP
-        // and no output): dP phi first, then the dx kernel that consumes it, dphi = dP^T x last.  The
-        // last launch carries the batch sums (dw, dbias, dalpha) in an extra row of workgroups, which
-        // run in the shadow of the dphi stores instead of as a launch of their own.  Measured on whole
-        // steps, graphs of ten (one launch for both products + finalize launch -> apart + carried sums):
-        //   B=256 n=8   47.7 -> 48.8 us (not taken)    B=256 n=10   79.8 -> 80.0 (not taken)
-        //   B=512 n=12 126.6 -> 125.9    B=256 n=13 101.6 -> 96.6    B=256 n=16 111.9 -> 104.4
-        //   B=256 n=18 127.5 -> 119.0    B=128 n=32 148.6 -> 145.8 (always two product kernels; sums carried)
-        const bool wide = proj_bwd_is_wide(n);
-        const int hook = tuning_get(kTuneProjApart);
-        const bool apart = wide || (hook ? hook == 2 : proj_bwd_products_apart(n));
-        if (apart) {
-            if (wide) MHC_LAUNCH(launch_dxflat_wide(phi, ws.dPb, ws.BP, dx, nullptr, nullptr, nullptr, B, n, C, st));
-            else MHC_LAUNCH(launch_proj_bwd_mfma(x, phi, ws.dPb, ws.dPT, ws.BP, dphi, ws.dphi_part, dx, B, n, C, st, kProjPartDx));
-        } else {
-            MHC_LAUNCH(launch_proj_bwd_mfma(x, phi, ws.dPb, ws.dPT, ws.BP, dphi, ws.dphi_part, dx, B, n, C, st));
-        }
-        MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
-                                     n, q, ws.s1, ws.cx, ws.dP, DP, nullptr, 0, dx, dx, df, ws.u, ws.dt,
-                                     ws.dtpart, spg, B, n, C, st));
-        if (apart) {
-            const BatchSumArgs sums = make_batch_sums(ws.u, groups, C, f_inject ? nullptr : dw, ws.dtpart, groups,
-                                                      D, dbias, dalpha);
-            const BatchSumArgs *tail = S == 1 && tuning_get(kTuneSeparateFinalize) != 1 ? &sums : nullptr;
-            bool tail_taken = false;
-            if (wide) MHC_LAUNCH(launch_dphi_large(x, ws.dPT, ws.BP, S > 1 ? ws.dphi_part : dphi, S, B, n, C, tail, &tail_taken, st));
-            else MHC_LAUNCH(launch_proj_bwd_mfma(x, phi, ws.dPb, ws.dPT, ws.BP, dphi, ws.dphi_part, dx, B, n, C, st,
-                                                 kProjPartDphi, tail, &tail_taken));
-            if (tail_taken) return MHC_OK;
-        }
-    } else if (gemm_f32_supported(x_dtype, phi_dtype, n, C)) {
-        // exact float32 tier, wide projection: both products on the fp32 matrix cores; the projection
-        // term of dx is written into dx and completed in place
-        MHC_LAUNCH(launch_gemm_f32_dxflat(ws.dP, static_cast<const float *>(phi), static_cast<float *>(dx), B, n, C, st));
-        MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
-                                     n, q, ws.s1, ws.cx, ws.dP, DP, nullptr, 0, dx, dx, df, ws.u, ws.dt,
-                                     ws.dtpart, spg, B, n, C, st));
-        MHC_LAUNCH(launch_gemm_f32_dphi(ws.dP, static_cast<const float *>(x), dphi, B, n, C, st));
-    } else {
-        MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
-                                     n, q, ws.s1, ws.cx, ws.dP, DP, phi, phi_dtype, nullptr, dx, df,
-                                     ws.u, ws.dt, ws.dtpart, spg, B, n, C, st));
-        MHC_LAUNCH(launch_dphi(x, x_dtype, ws.dP, DP, dphi, B, n, C, ws.dphi_part, st));
-    }
-    MHC_LAUNCH(launch_finalize(ws.u, groups, C, f_inject ? nullptr : dw, ws.dtpart, groups, D, dbias,
-                               dalpha, ws.dphi_part, S, (size_t)D * n * C, dphi, st));
-    return MHC_OK;
+    return bwd_dynamic(dy, y_dtype, x, x_dtype, w, w_dtype, phi, phi_dtype, bias, alpha, f_inject, H_pre, H_post, M, P, r, q,
+                       sk_state, dx, df, DwOut{dw, false}, dphi, dbias, dalpha, B, n, C, iters, eps, workspace,
+                       workspace_bytes, stream);
+}
+
+int mhc_layer_bwd_dynamic_dw(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w,
+                          int w_dtype, const void *phi, int phi_dtype, const float *bias,
+                          const float *alpha, const void *f_inject, const float *H_pre,
+                          const float *H_post, const float *M, const float *P, const float *r,
+                          const float *q, const float *sk_state, void *dx, void *df, void *dw, int dw_dtype,
+                          float *dphi,
+                          float *dbias, float *dalpha, int B, int n, int C, int iters, float eps,
+                          void *workspace, size_t workspace_bytes, void *stream) {
+    if (!valid_dtype(dw_dtype)) return MHC_ERR_BAD_DTYPE;
+    return bwd_dynamic(dy, y_dtype, x, x_dtype, w, w_dtype, phi, phi_dtype, bias, alpha, f_inject, H_pre, H_post, M, P, r, q,
+                       sk_state, dx, df, DwOut{dw, dw_dtype == MHC_BF16}, dphi, dbias, dalpha, B, n, C, iters, eps,
+                       workspace, workspace_bytes, stream);
 }
 
 int mhc_pack_dynamic_params(const void *phi_pre, const void *phi_post, const void *phi_res, int src_dtype,
@@ -435,9 +328,9 @@ int mhc_pack_dynamic_params(const void *phi_pre, const void *phi_post, const voi
         !alpha_res || !phi || !bias || !alpha)
         return MHC_ERR_NULL_POINTER;
     if (!valid_dtype(src_dtype) || !valid_dtype(phi_dtype)) return MHC_ERR_BAD_DTYPE;
-    MHC_LAUNCH(launch_pack_params(phi_pre, phi_post, phi_res, src_dtype, b_pre, b_post, b_res, alpha_pre,
-                                  alpha_post, alpha_res, phi, phi_dtype, bias, alpha, n, C,
-                                  static_cast<hipStream_t>(stream)));
+    MHC_LAUNCH(launch_pack_params(ParamGather{{phi_pre, phi_post, phi_res}, src_dtype, {b_pre, b_post, b_res},
+                                              {alpha_pre, alpha_post, alpha_res}, phi, phi_dtype, bias, alpha},
+                                  n, C, static_cast<hipStream_t>(stream)));
     return MHC_OK;
 }
 
@@ -495,57 +388,21 @@ int mhc_layer_bwd(const void *dy, int y_dtype, const void *x, int x_dtype, const
                   const float *H_post, const float *M, const float *q, void *dx, void *df,
                   float *dw, float *dH_pre, float *dH_post, float *dH_res, int B, int n, int C,
                   int iters, float eps, void *workspace, size_t workspace_bytes, void *stream) {
-    if (int s = check_shape(B, n, C, iters)) return s;
-    if (!dy || !x || !H_pre_logits || !H_post_logits || !H_res_logits || !H_pre || !H_post || !M ||
-        !q || !dx || !dH_pre || !dH_post || !dH_res)
-        return MHC_ERR_NULL_POINTER;
-    if (!f_inject && (!w || !dw)) return MHC_ERR_NULL_POINTER;
-    if (!valid_io(x_dtype, y_dtype) || (w && !valid_dtype(w_dtype))) return MHC_ERR_BAD_DTYPE;
-    if (!aligned16(dy) || !aligned16(x) || !aligned16(dx) || (f_inject && !aligned16(f_inject)) ||
-        (df && !aligned16(df)))
-        return MHC_ERR_MISALIGNED;
-    const StaBwdWs ws = carve_sta_bwd(workspace, B, n, C);
-    if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    BwdCoefOut out{nullptr, nullptr, nullptr, ws.s1, ws.red, nullptr, nullptr, 0};
-    if (bwd_resident_supported(x_dtype, y_dtype, kBF16, n, C, 0) && tuning_get(kTuneResident) != 1) {
-        // bf16 activations, n <= 8: with shared coefficients nothing of dx depends on a batch-wide
-        // result, so ONE pass over dy and x (a workgroup keeps its sample's rows in registers) forms
-        // the channel sums, the sample's raw coefficient gradients and the complete dx
-        MHC_LAUNCH(launch_bwd_resident_static(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, q, out, dx, df, ws.u,
-                                              B, n, C, st));
-        MHC_LAUNCH(launch_finalize_static(ws.u, B, C, f_inject ? nullptr : dw, ws.red, B, ws.red_sum, H_pre, H_post,
-                                          H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st));
-        return MHC_OK;
-    }
-    if (n > 16 && x_dtype == kBF16 && y_dtype == kBF16 && C % 8 == 0) {
-        // three launches: channel sums (+ the Sinkhorn forward recompute), the per-sample coefficient sums
-        // with the complete dx beside them, batch sums + coefficient backward
-        // (cold, B=128 n=32 C=1280: 44.7 us -> see profiles/native_bench_all_configs.txt)
-        MHC_LAUNCH(launch_mix_bwd_reduce_with_dx_static(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, q, out, ws.raw,
-                                                        ws.s1part, dx, df, ws.u, B, n, C, iters, eps, st, H_res_logits,
-                                                        ws.sk));
-        MHC_LAUNCH(launch_finalize_static(ws.u, B, C, f_inject ? nullptr : dw, ws.red, B, ws.red_sum, H_pre, H_post,
-                                          H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st, ws.sk));
-        return MHC_OK;
-    }
-    MHC_LAUNCH(launch_mix_bwd_reduce(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
-                                     0, q, nullptr, nullptr, nullptr, nullptr, nullptr, out, n > 8 ? ws.raw : nullptr,
-                                     B, n, C, iters, eps, st, H_res_logits, n > 8 ? ws.sk : nullptr));
-    // samples per workgroup of the dx kernel: with a large batch a workgroup adds up the dw terms of a
-    // few samples itself, so that the batch-sum launch reads fewer rows
-    const int hook = tuning_get(kTuneStaticSpg);
-    // (measured cold, bf16: B=1280 C=2560 n=4 60.5 -> 58.6 us with four; B=1024 n=8 and small batches lose)
-    const int spg = n > 8 ? 1 : (hook > 0 ? hook : (n <= 4 && B >= 1024 ? 4 : 1));
-    const int groups = (B + spg - 1) / spg;
-    MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, 0,
-                                 q, ws.s1, nullptr, nullptr, 0, nullptr, 0, nullptr, dx, df, ws.u, nullptr,
-                                 nullptr, spg, B, n, C, st));
-    // the batch sums (dw = sum_b u, sum_b red) and the coefficient backward on them: one launch for
-    // n <= 8, two beyond
-    MHC_LAUNCH(launch_finalize_static(ws.u, groups, C, f_inject ? nullptr : dw, ws.red, B, ws.red_sum, H_pre, H_post,
-                                      H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st, n > 8 ? ws.sk : nullptr));
-    return MHC_OK;
+    return bwd_static(dy, y_dtype, x, x_dtype, w, w_dtype, H_pre_logits, H_post_logits, H_res_logits, f_inject, H_pre, H_post,
+                      M, q, dx, df, DwOut{dw, false}, dH_pre, dH_post, dH_res, B, n, C, iters, eps, workspace,
+                      workspace_bytes, stream);
+}
+
+int mhc_layer_bwd_dw(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w,
+                  int w_dtype, const float *H_pre_logits, const float *H_post_logits,
+                  const float *H_res_logits, const void *f_inject, const float *H_pre,
+                  const float *H_post, const float *M, const float *q, void *dx, void *df,
+                  void *dw, int dw_dtype, float *dH_pre, float *dH_post, float *dH_res, int B, int n, int C,
+                  int iters, float eps, void *workspace, size_t workspace_bytes, void *stream) {
+    if (!valid_dtype(dw_dtype)) return MHC_ERR_BAD_DTYPE;
+    return bwd_static(dy, y_dtype, x, x_dtype, w, w_dtype, H_pre_logits, H_post_logits, H_res_logits, f_inject, H_pre, H_post,
+                      M, q, dx, df, DwOut{dw, dw_dtype == MHC_BF16}, dH_pre, dH_post, dH_res, B, n, C, iters, eps, workspace,
+                      workspace_bytes, stream);
 }
 
 // ===============================================================================================
@@ -681,3 +538,246 @@ int mhc_layer_fwd_dynamic_static_scratch(const void *x, int x_dtype, const void 
 }
 
 }  // extern "C"
+
+// ===============================================================================================
+// the launch sequences behind the entry points above
+// ===============================================================================================
+namespace {
+
+int fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype, const ParamGather *gather, const void *phi,
+                int phi_dtype, const float *bias, const float *alpha, const void *f_inject, void *y, int y_dtype,
+                float *H_pre, float *H_post, float *M, float *P, float *r, float *q, float *sk_state, int B, int n,
+                int C, int iters, float eps, void *workspace, size_t workspace_bytes, void *stream) {
+    if (int s = check_shape(B, n, C, iters)) return s;
+    if (!x || !phi || !bias || !alpha || !y || !H_pre || !H_post || !M || !P || !r || !q)
+        return MHC_ERR_NULL_POINTER;
+    if (!f_inject && !w) return MHC_ERR_NULL_POINTER;
+    if (!valid_io(x_dtype, y_dtype) || !valid_dtype(phi_dtype) || (w && !valid_dtype(w_dtype)))
+        return MHC_ERR_BAD_DTYPE;
+    if (x_dtype == MHC_F32_AS_BF16 && (phi_dtype != MHC_BF16 || !f32_as_bf16_accepted(B, n, C, iters)))
+        return MHC_ERR_BAD_DTYPE;
+    if (!aligned16(x) || !aligned16(y) || !aligned16(phi) || (f_inject && !aligned16(f_inject)))
+        return MHC_ERR_MISALIGNED;
+    const DynFwdWs ws = carve_dyn_fwd(workspace, B, n, C);
+    if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    // the caller's own parameters: read by the projection where it can, otherwise packed by a launch of their own
+    const bool in_proj = gather && !layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C) &&
+                         proj_fwd_gathers(*gather, x_dtype, B, n, C);
+    if (gather && !in_proj) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
+    if (layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C)) {
+        // projection, coefficients and mix in one launch; x crosses HBM once
+        MHC_LAUNCH(launch_layer_fwd_onepass(x, w, w_dtype, f_inject, y, y_dtype, phi, alpha, bias, H_pre, H_post,
+                                            M, P, r, q, sk_state, B, n, C, iters, eps, st));
+        return MHC_OK;
+    }
+    const int KS = proj_fwd_ksplit(x_dtype, phi_dtype, B, n, C);
+    MHC_LAUNCH(launch_proj_fwd(x, x_dtype, phi, phi_dtype, ws.Ppart, ws.ssqpart, KS, B, n, C, st,
+                               in_proj ? gather : nullptr));
+    if (layer_fwd_fused_supported(n, C, x_dtype)) {
+        MHC_LAUNCH(launch_layer_fwd_fused(x, x_dtype, w, w_dtype, f_inject, y, y_dtype, ws.Ppart,
+                                          ws.ssqpart, KS, padded_D(n), alpha, bias, bias + n,
+                                          bias + 2 * n, H_pre, H_post, M, P, r, q, sk_state, B, n, C, iters,
+                                          eps, st));
+        return MHC_OK;
+    }
+    // n > 8 in the bf16 tier: the coefficient launch also forms the stream aggregate and its RMS
+    const bool agg = !f_inject && ws.agg && coef_fwd_aggregates(n, C, x_dtype);
+    MHC_LAUNCH(launch_coef_fwd(ws.Ppart, ws.ssqpart, KS, padded_D(n), alpha, bias, bias + n,
+                               bias + 2 * n, H_pre, H_post, M, P, r, B, n, n * C, iters, eps,
+                               x_dtype == kF32, agg ? x : nullptr, ws.agg, q, sk_state, st));
+    MHC_LAUNCH(launch_mix_fwd(x, x_dtype, w, w_dtype, f_inject, y, y_dtype, H_pre, H_post, M, n, q,
+                              ws.agg, B, n, C, eps, agg, st));
+    return MHC_OK;
+}
+
+int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w, int w_dtype, const void *phi,
+                int phi_dtype, const float *bias, const float *alpha, const void *f_inject, const float *H_pre,
+                const float *H_post, const float *M, const float *P, const float *r, const float *q,
+                const float *sk_state, void *dx, void *df, DwOut dw, float *dphi, float *dbias, float *dalpha, int B,
+                int n, int C, int iters, float eps, void *workspace, size_t workspace_bytes, void *stream) {
+    if (int s = check_shape(B, n, C, iters)) return s;
+    if (!dy || !x || !phi || !bias || !alpha || !H_pre || !H_post || !M || !P || !r || !q || !dx ||
+        !dphi || !dbias || !dalpha)
+        return MHC_ERR_NULL_POINTER;
+    if (!f_inject && (!w || !dw)) return MHC_ERR_NULL_POINTER;
+    if (!valid_io(x_dtype, y_dtype) || !valid_dtype(phi_dtype) || (w && !valid_dtype(w_dtype)))
+        return MHC_ERR_BAD_DTYPE;
+    if (x_dtype == MHC_F32_AS_BF16 && (phi_dtype != MHC_BF16 || !f32_as_bf16_accepted(B, n, C, iters)))
+        return MHC_ERR_BAD_DTYPE;
+    if (!aligned16(dy) || !aligned16(x) || !aligned16(dx) || !aligned16(phi) || !aligned16(dphi) ||
+        (f_inject && !aligned16(f_inject)) || (df && !aligned16(df)))
+        return MHC_ERR_MISALIGNED;
+    const DynBwdWs ws = carve_dyn_bwd(workspace, B, n, C);
+    if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int D = n * n + 2 * n, DP = padded_D(n);
+    const bool mfma = proj_bwd_mfma_supported(x_dtype == kF32AsBF16 ? kBF16 : x_dtype, phi_dtype, C);
+    BwdCoefOut out{ws.dt, ws.dP, ws.cx, ws.s1, nullptr, mfma ? ws.dPb : nullptr, ws.dPT, ws.BP};
+    if (mfma && bwd_resident_supported(x_dtype, y_dtype, phi_dtype, n, C, iters) && proj_bwd_addx_supported(n) &&
+        (bwd_resident_preferred(B, n, C) || x_dtype == kF32AsBF16)) {
+        // two launches: (1) one workgroup per sample keeps the sample's rows of dy and x in registers for
+        // the channel sums, the coefficient backward and the mixing part of dx; (2) a column-slab
+        // kernel over all samples adds dP phi - cx x, finishes dphi without batch-split partial sums
+        // and sums dw, dbias and dalpha in a few extra workgroups
+        BwdCoefOut out2 = out;
+        out2.dP = nullptr;  // the second launch takes dP as matrix-core operands only
+        MHC_LAUNCH(launch_bwd_resident(dy, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, q, P, r, alpha, bias + 2 * n,
+                                       sk_state, out2, dx, df, ws.u, B, n, C, iters, eps, st));
+        const BatchSumArgs sums = make_batch_sums(ws.u, B, C, f_inject ? DwOut{} : dw, ws.dt, B, D, dbias, dalpha);
+        bool tail_taken = false;
+        MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, dphi, dx, B, n, C,
+                                        tuning_get(kTuneSeparateFinalize) == 1 ? nullptr : &sums, &tail_taken, st));
+        if (!tail_taken)
+            MHC_LAUNCH(launch_finalize(ws.u, B, C, f_inject ? DwOut{} : dw, ws.dt, B, D, dbias, dalpha, nullptr, 1,
+                                       0, nullptr, st));
+        return MHC_OK;
+    }
+    if (x_dtype == kF32AsBF16) return MHC_ERR_BAD_DTYPE;  // not reached: accepted shapes take the path above
+    if (mfma && x_dtype == kBF16 && y_dtype == kBF16 && wide_dx_beside(B, n, C) && tuning_get(kTuneWideDxBeside) != 1) {
+        // wide projection (n > 18), four launches.  The coefficient backward is one workgroup per sample,
+        // all dependent chains; the part of dx that needs none of its results (M^T dy + Hpre (x) da,
+        // with s1 from the channel sums) runs beside it in the same launch and is handed over in fp32;
+        // the dP phi kernel then completes dx (+ dP phi - cx x, one rounding); dphi comes last and carries
+        // the batch sums.
+        // B=128 n=32 C=1280, backward in graphs of ten, same box: five launches 99.8 us, these four 93.0 us
+        MHC_LAUNCH(launch_mix_bwd_reduce_with_dx(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, n, q, P, r, alpha,
+                                                 bias + 2 * n, sk_state, out, ws.raw, ws.s1part, ws.dx_part, df, ws.u, B, n, C,
+                                                 iters, eps, st));
+        MHC_LAUNCH(launch_dxflat_wide(phi, ws.dPb, ws.BP, dx, x, ws.cx, ws.dx_part, B, n, C, st));
+        const BatchSumArgs sums = make_batch_sums(ws.u, B, C, f_inject ? DwOut{} : dw, ws.dt, B, D, dbias, dalpha);
+        bool tail_taken = false;
+        MHC_LAUNCH(launch_dphi_large(x, ws.dPT, ws.BP, dphi, 1, B, n, C,
+                                     tuning_get(kTuneSeparateFinalize) != 1 ? &sums : nullptr, &tail_taken, st));
+        if (!tail_taken)
+            MHC_LAUNCH(launch_finalize(ws.u, B, C, f_inject ? DwOut{} : dw, ws.dt, B, D, dbias, dalpha, nullptr, 1,
+                                       (size_t)D * n * C, dphi, st));
+        return MHC_OK;
+    }
+    MHC_LAUNCH(launch_mix_bwd_reduce(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
+                                     n, q, P, r, alpha, bias + 2 * n, sk_state, out, ws.raw, B, n, C, iters, eps,
+                                     st));
+    if (mfma && bwd_slab_supported(x_dtype, y_dtype, phi_dtype, n, C)) {
+        // n <= 4: one slab kernel finishes dx and produces every batch-split partial sum
+        const int S = bwd_slab_batch_splits(B, n, C);
+        MHC_LAUNCH(launch_bwd_slab(dy, y_dtype, x, w, w_dtype, f_inject, phi, H_pre, H_post, M, q, ws.s1,
+                                   ws.cx, ws.dPb, ws.dPT, ws.BP, ws.dt, dx, df,
+                                   S > 1 ? ws.dphi_part : dphi, ws.u, ws.dtpart, S, B, n, C, st));
+        MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S, D, dbias, dalpha,
+                                   ws.dphi_part, S, (size_t)D * n * C, dphi, st));
+        return MHC_OK;
+    }
+    const int spg = bwd_dx_samples_per_group(B, n);
+    const int groups = (B + spg - 1) / spg;
+    int S = 1;
+    if (mfma) {
+        // matrix cores: dphi and the projection term of dx (written into dx, then completed in place)
+        S = proj_bwd_batch_splits(B, n, C);
+        // From D > 128 on the two products run as launches of their own (they share no operand but dP
+        // and no output): dP phi first, then the dx kernel that consumes it, dphi = dP^T x last.  The
+        // last launch carries the batch sums (dw, dbias, dalpha) in an extra row of workgroups, which
+        // run in the shadow of the dphi stores instead of as a launch of their own.  Measured on whole
+        // steps, graphs of ten (one launch for both products + finalize launch -> apart + carried sums):
+        //   B=256 n=8   47.7 -> 48.8 us (not taken)    B=256 n=10   79.8 -> 80.0 (not taken)
+        //   B=512 n=12 126.6 -> 125.9    B=256 n=13 101.6 -> 96.6    B=256 n=16 111.9 -> 104.4
+        //   B=256 n=18 127.5 -> 119.0    B=128 n=32 148.6 -> 145.8 (always two product kernels; sums carried)
+        const bool wide = proj_bwd_is_wide(n);
+        const int hook = tuning_get(kTuneProjApart);
+        const bool apart = wide || (hook ? hook == 2 : proj_bwd_products_apart(n));
+        if (apart) {
+            if (wide) MHC_LAUNCH(launch_dxflat_wide(phi, ws.dPb, ws.BP, dx, nullptr, nullptr, nullptr, B, n, C, st));
+            else MHC_LAUNCH(launch_proj_bwd_mfma(x, phi, ws.dPb, ws.dPT, ws.BP, dphi, ws.dphi_part, dx, B, n, C, st, kProjPartDx));
+        } else {
+            MHC_LAUNCH(launch_proj_bwd_mfma(x, phi, ws.dPb, ws.dPT, ws.BP, dphi, ws.dphi_part, dx, B, n, C, st));
+        }
+        MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
+                                     n, q, ws.s1, ws.cx, ws.dP, DP, nullptr, 0, dx, dx, df, ws.u, ws.dt,
+                                     ws.dtpart, spg, B, n, C, st));
+        if (apart) {
+            const BatchSumArgs sums = make_batch_sums(ws.u, groups, C, f_inject ? DwOut{} : dw, ws.dtpart, groups,
+                                                      D, dbias, dalpha);
+            const BatchSumArgs *tail = S == 1 && tuning_get(kTuneSeparateFinalize) != 1 ? &sums : nullptr;
+            bool tail_taken = false;
+            if (wide) MHC_LAUNCH(launch_dphi_large(x, ws.dPT, ws.BP, S > 1 ? ws.dphi_part : dphi, S, B, n, C, tail, &tail_taken, st));
+            else MHC_LAUNCH(launch_proj_bwd_mfma(x, phi, ws.dPb, ws.dPT, ws.BP, dphi, ws.dphi_part, dx, B, n, C, st,
+                                                 kProjPartDphi, tail, &tail_taken));
+            if (tail_taken) return MHC_OK;
+        }
+    } else if (gemm_f32_supported(x_dtype, phi_dtype, n, C)) {
+        // exact float32 tier, wide projection: both products on the fp32 matrix cores; the projection
+        // term of dx is written into dx and completed in place
+        MHC_LAUNCH(launch_gemm_f32_dxflat(ws.dP, static_cast<const float *>(phi), static_cast<float *>(dx), B, n, C, st));
+        MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
+                                     n, q, ws.s1, ws.cx, ws.dP, DP, nullptr, 0, dx, dx, df, ws.u, ws.dt,
+                                     ws.dtpart, spg, B, n, C, st));
+        MHC_LAUNCH(launch_gemm_f32_dphi(ws.dP, static_cast<const float *>(x), dphi, B, n, C, st));
+    } else {
+        MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
+                                     n, q, ws.s1, ws.cx, ws.dP, DP, phi, phi_dtype, nullptr, dx, df,
+                                     ws.u, ws.dt, ws.dtpart, spg, B, n, C, st));
+        MHC_LAUNCH(launch_dphi(x, x_dtype, ws.dP, DP, dphi, B, n, C, ws.dphi_part, st));
+    }
+    MHC_LAUNCH(launch_finalize(ws.u, groups, C, f_inject ? DwOut{} : dw, ws.dtpart, groups, D, dbias,
+                               dalpha, ws.dphi_part, S, (size_t)D * n * C, dphi, st));
+    return MHC_OK;
+}
+
+int bwd_static(const void *dy, int y_dtype, const void *x, int x_dtype, const void *w, int w_dtype,
+               const float *H_pre_logits, const float *H_post_logits, const float *H_res_logits, const void *f_inject,
+               const float *H_pre, const float *H_post, const float *M, const float *q, void *dx, void *df, DwOut dw,
+               float *dH_pre, float *dH_post, float *dH_res, int B, int n, int C, int iters, float eps,
+               void *workspace, size_t workspace_bytes, void *stream) {
+    if (int s = check_shape(B, n, C, iters)) return s;
+    if (!dy || !x || !H_pre_logits || !H_post_logits || !H_res_logits || !H_pre || !H_post || !M ||
+        !q || !dx || !dH_pre || !dH_post || !dH_res)
+        return MHC_ERR_NULL_POINTER;
+    if (!f_inject && (!w || !dw)) return MHC_ERR_NULL_POINTER;
+    if (!valid_io(x_dtype, y_dtype) || (w && !valid_dtype(w_dtype))) return MHC_ERR_BAD_DTYPE;
+    if (!aligned16(dy) || !aligned16(x) || !aligned16(dx) || (f_inject && !aligned16(f_inject)) ||
+        (df && !aligned16(df)))
+        return MHC_ERR_MISALIGNED;
+    const StaBwdWs ws = carve_sta_bwd(workspace, B, n, C);
+    if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    BwdCoefOut out{nullptr, nullptr, nullptr, ws.s1, ws.red, nullptr, nullptr, 0};
+    if (bwd_resident_supported(x_dtype, y_dtype, kBF16, n, C, 0) && tuning_get(kTuneResident) != 1) {
+        // bf16 activations, n <= 8: with shared coefficients nothing of dx depends on a batch-wide
+        // result, so ONE pass over dy and x (a workgroup keeps its sample's rows in registers) forms
+        // the channel sums, the sample's raw coefficient gradients and the complete dx
+        MHC_LAUNCH(launch_bwd_resident_static(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, q, out, dx, df, ws.u,
+                                              B, n, C, st));
+        MHC_LAUNCH(launch_finalize_static(ws.u, B, C, f_inject ? DwOut{} : dw, ws.red, B, ws.red_sum, H_pre, H_post,
+                                          H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st));
+        return MHC_OK;
+    }
+    if (n > 16 && x_dtype == kBF16 && y_dtype == kBF16 && C % 8 == 0) {
+        // three launches: channel sums (+ the Sinkhorn forward recompute), the per-sample coefficient sums
+        // with the complete dx beside them, batch sums + coefficient backward
+        // (cold, B=128 n=32 C=1280: 44.7 us -> see profiles/native_bench_all_configs.txt)
+        MHC_LAUNCH(launch_mix_bwd_reduce_with_dx_static(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, q, out, ws.raw,
+                                                        ws.s1part, dx, df, ws.u, B, n, C, iters, eps, st, H_res_logits,
+                                                        ws.sk));
+        MHC_LAUNCH(launch_finalize_static(ws.u, B, C, f_inject ? DwOut{} : dw, ws.red, B, ws.red_sum, H_pre, H_post,
+                                          H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st, ws.sk));
+        return MHC_OK;
+    }
+    MHC_LAUNCH(launch_mix_bwd_reduce(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
+                                     0, q, nullptr, nullptr, nullptr, nullptr, nullptr, out, n > 8 ? ws.raw : nullptr,
+                                     B, n, C, iters, eps, st, H_res_logits, n > 8 ? ws.sk : nullptr));
+    // samples per workgroup of the dx kernel: with a large batch a workgroup adds up the dw terms of a
+    // few samples itself, so that the batch-sum launch reads fewer rows
+    const int hook = tuning_get(kTuneStaticSpg);
+    // (measured cold, bf16: B=1280 C=2560 n=4 60.5 -> 58.6 us with four; B=1024 n=8 and small batches lose)
+    const int spg = n > 8 ? 1 : (hook > 0 ? hook : (n <= 4 && B >= 1024 ? 4 : 1));
+    const int groups = (B + spg - 1) / spg;
+    MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, 0,
+                                 q, ws.s1, nullptr, nullptr, 0, nullptr, 0, nullptr, dx, df, ws.u, nullptr,
+                                 nullptr, spg, B, n, C, st));
+    // the batch sums (dw = sum_b u, sum_b red) and the coefficient backward on them: one launch for
+    // n <= 8, two beyond
+    MHC_LAUNCH(launch_finalize_static(ws.u, groups, C, f_inject ? DwOut{} : dw, ws.red, B, ws.red_sum, H_pre, H_post,
+                                      H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st, n > 8 ? ws.sk : nullptr));
+    return MHC_OK;
+}
+
+}  // namespace

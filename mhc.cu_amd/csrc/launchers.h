@@ -29,6 +29,17 @@ template <typename K> inline hipError_t allow_dynamic_lds(K kernel, size_t bytes
 // Projection row count padded to whole 32-wide MFMA tiles.
 inline int padded_D(int n) { return ((n * n + 2 * n) + 31) / 32 * 32; }
 
+// The parameters of a dynamic layer as the caller stores them (three phi matrices, three biases, three
+// scalars) and where their packed form goes: phi_out [D, nC] in the compute dtype, bias_out [D], alpha_out [3].
+struct ParamGather {
+    const void *phi[3];  // pre [n, nC], post [n, nC], res [n*n, nC]
+    int phi_dtype;
+    const float *b[3], *alpha[3];
+    void *phi_out;
+    int out_dtype;
+    float *bias_out, *alpha_out;
+};
+
 // ---- forward ---------------------------------------------------------------------------------
 
 // Number of K-splits launch_proj_fwd produces for this shape and dtype pair (never more than
@@ -38,8 +49,12 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C);
 
 // Ppart[ks][b][d] = sum over K-slab ks of x_flat[b,k] * phi[d,k]   (d < D; padded rows zero)
 // ssqpart[ks][b]  = sum over the slab of x_flat[b,k]^2
+// gather (optional, only where proj_fwd_gathers() holds): the kernel reads the caller's fp32 parameters
+// itself and leaves their packed form behind (phi, = gather->phi_out, is then written, not read).
 hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_dtype, float *Ppart,
-                           float *ssqpart, int KS, int B, int n, int C, hipStream_t stream);
+                           float *ssqpart, int KS, int B, int n, int C, hipStream_t stream,
+                           const ParamGather *gather = nullptr);
+bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C);
 
 // Coefficients from projection partials (dynamic: Ppart != nullptr) or logits (static: B == 1).
 hipError_t launch_coef_fwd(const float *Ppart, const float *ssqpart, int KS, int DP,
@@ -169,7 +184,7 @@ int bwd_dx_samples_per_group(int B, int n);
 
 // One launch for all remaining batch sums: u [rows_u, C] -> dw (skipped when dw == nullptr),
 // dt [rows_dt, D+3] -> dbias, dalpha, and (S > 1) dphi_part [S, dphi_elems] -> dphi.
-hipError_t launch_finalize(const float *u, int rows_u, int C, float *dw, const float *dt, int rows_dt,
+hipError_t launch_finalize(const float *u, int rows_u, int C, DwOut dw, const float *dt, int rows_dt,
                            int D, float *dbias, float *dalpha, const float *dphi_part, int S,
                            size_t dphi_elems, float *dphi, hipStream_t stream);
 
@@ -241,18 +256,14 @@ hipError_t launch_colsum_split(const float *in, int rows, int cols, int ld, floa
 hipError_t launch_coef_bwd_static(const float *red_sum, const float *Hpre, const float *Hpost,
                                   const float *H_res_logits, float *dH_pre, float *dH_post,
                                   float *dH_res, int n, int T, float eps, hipStream_t stream, const float *state = nullptr);
-hipError_t launch_finalize_static(const float *u, int rows_u, int C, float *dw, const float *red, int rows,
+hipError_t launch_finalize_static(const float *u, int rows_u, int C, DwOut dw, const float *red, int rows,
                                   float *red_sum, const float *Hpre, const float *Hpost,
                                   const float *H_res_logits, float *dH_pre, float *dH_post, float *dH_res, int n,
                                   int T, float eps, hipStream_t stream, const float *static_state = nullptr);
 
 // phi [D, nC] (out_dtype) = rows [pre | post | res] of the three parameter matrices (src_dtype),
 // bias [D] and alpha [3] likewise, in one launch.
-hipError_t launch_pack_params(const void *phi_pre, const void *phi_post, const void *phi_res, int src_dtype,
-                              const float *b_pre, const float *b_post, const float *b_res,
-                              const float *alpha_pre, const float *alpha_post, const float *alpha_res,
-                              void *phi_out, int out_dtype, float *bias, float *alpha, int n, int C,
-                              hipStream_t stream);
+hipError_t launch_pack_params(const ParamGather &g, int n, int C, hipStream_t stream);
 
 // ---- stand-alone operators -------------------------------------------------------------------
 hipError_t launch_sinkhorn_plain_fwd(const float *inp, float *out, int batch, int rows, int cols,

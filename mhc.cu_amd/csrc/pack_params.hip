@@ -76,29 +76,29 @@ __global__ __launch_bounds__(256) void pack_params_stream_kernel(PackArgs a) {
     }
 }
 
-hipError_t launch_pack_params(const void *phi_pre, const void *phi_post, const void *phi_res, int src_dtype,
-                              const float *b_pre, const float *b_post, const float *b_res,
-                              const float *alpha_pre, const float *alpha_post, const float *alpha_res,
-                              void *phi_out, int out_dtype, float *bias, float *alpha, int n, int C,
-                              hipStream_t stream) {
+hipError_t launch_pack_params(const ParamGather &g, int n, int C, hipStream_t stream) {
     const size_t nC = (size_t)n * C, rows[3] = {(size_t)n, (size_t)n, (size_t)n * n};
     PackArgs a;
-    a.src[0] = phi_pre; a.src[1] = phi_post; a.src[2] = phi_res;
     size_t end = 0;
-    for (int i = 0; i < 3; i++) { end += rows[i] * nC; a.end[i] = end; }
-    a.b[0] = b_pre; a.b[1] = b_post; a.b[2] = b_res;
-    a.bn[0] = n; a.bn[1] = n; a.bn[2] = n * n;
-    a.alpha_in[0] = alpha_pre; a.alpha_in[1] = alpha_post; a.alpha_in[2] = alpha_res;
-    a.phi_out = phi_out; a.bias = bias; a.alpha = alpha; a.total = end;
+    for (int i = 0; i < 3; i++) {
+        a.src[i] = g.phi[i];
+        end += rows[i] * nC;
+        a.end[i] = end;
+        a.b[i] = g.b[i];
+        a.bn[i] = (int)rows[i];
+        a.alpha_in[i] = g.alpha[i];
+    }
+    a.phi_out = g.phi_out; a.bias = g.bias_out; a.alpha = g.alpha_out; a.total = end;
+    const int src_dtype = g.phi_dtype, out_dtype = g.out_dtype;
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     // the streaming kernel: fp32 -> bf16, whole 16-byte chunks in every source, enough of them to matter
-    if (src_dtype == kF32 && out_dtype == kBF16 && (n * nC) % 4 == 0 && al16(phi_pre) && al16(phi_post) &&
-        al16(phi_res) && (reinterpret_cast<uintptr_t>(phi_out) & 7u) == 0 && end >= (size_t)1 << 20) {
+    if (src_dtype == kF32 && out_dtype == kBF16 && (n * nC) % 4 == 0 && al16(g.phi[0]) && al16(g.phi[1]) &&
+        al16(g.phi[2]) && (reinterpret_cast<uintptr_t>(g.phi_out) & 7u) == 0 && end >= (size_t)1 << 20) {
         const size_t rounds = (end / 4 + (size_t)kPackU * 256 - 1) / ((size_t)kPackU * 256);
         pack_params_stream_kernel<<<(unsigned)(rounds < 2048 ? rounds : 2048), 256, 0, stream>>>(a);
         return hipGetLastError();
     }
-    const bool vec = (n * nC) % 8 == 0 && al16(phi_pre) && al16(phi_post) && al16(phi_res) && al16(phi_out);
+    const bool vec = (n * nC) % 8 == 0 && al16(g.phi[0]) && al16(g.phi[1]) && al16(g.phi[2]) && al16(g.phi_out);
     const int V = vec ? 8 : 1;
     const size_t chunks = (end + V - 1) / V;
     const unsigned grid = (unsigned)((chunks + 255) / 256);

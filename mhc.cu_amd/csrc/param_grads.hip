@@ -172,7 +172,7 @@ __global__ __launch_bounds__(1024) void finalize_kernel(FinalizeArgs a) {
     }
 }
 
-hipError_t launch_finalize(const float *u, int rows_u, int C, float *dw, const float *dt, int rows_dt,
+hipError_t launch_finalize(const float *u, int rows_u, int C, DwOut dw, const float *dt, int rows_dt,
                            int D, float *dbias, float *dalpha, const float *dphi_part, int S,
                            size_t dphi_elems, float *dphi, hipStream_t stream) {
     const BatchSumArgs sums = make_batch_sums(u, rows_u, C, dw, dt, rows_dt, D, dbias, dalpha);
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(1024) void finalize_static_kernel(FinalizeStaticArg
 
 // Batch sums + coefficient backward of the static path.  n <= 8: one launch (above); wider matrices: the
 // finalize launch writes the sums to red_sum [D + 3] and the workgroup-wide Sinkhorn kernel follows.
-hipError_t launch_finalize_static(const float *u, int rows_u, int C, float *dw, const float *red, int rows,
+hipError_t launch_finalize_static(const float *u, int rows_u, int C, DwOut dw, const float *red, int rows,
                                   float *red_sum, const float *Hpre, const float *Hpost,
                                   const float *H_res_logits, float *dH_pre, float *dH_post, float *dH_res, int n,
                                   int T, float eps, hipStream_t stream, const float *static_state) {

@@ -80,17 +80,42 @@ __global__ __launch_bounds__(256) void proj_fwd_generic_kernel(const TX *__restr
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2_t;
 constexpr int kNarrowPitch = 72;  // LDS row of a 64-element chunk: 128 data bytes + 16 pad (bf16 elements)
 
+// The caller's fp32 parameters, read by the projection itself (PF32 of the two kernels below): projection row d
+// is a row of one of the three matrices, rounded to bf16 on its way into the LDS tile; the workgroups of the
+// first sample tile also store the rounded rows, [bias] and [alpha] for the kernels that follow and for the
+// backward call.  Saves a packing launch (about 3 us of device and 5 us of host time per call, and for n = 32
+// a read of the 89 MB that it wrote).
+struct PhiSrc {
+    const float *phi[3];
+    const float *b[3], *alpha[3];
+    bf16_t *phi_out;
+    float *bias_out, *alpha_out;
+    int n;
+};
+__device__ __forceinline__ const float *phi_src_row(const PhiSrc &g, int d, int nC) {
+    const float *base = d < g.n ? g.phi[0] : (d < 2 * g.n ? g.phi[1] : g.phi[2]);
+    const int r = d < g.n ? d : (d < 2 * g.n ? d - g.n : d - 2 * g.n);
+    return base + (size_t)r * nC;
+}
+__device__ __forceinline__ void gather_small(const PhiSrc &g, int tid, int nthr, int D) {
+    if (tid < 3) g.alpha_out[tid] = g.alpha[tid][0];
+    for (int i = tid; i < D; i += nthr)
+        g.bias_out[i] = i < g.n ? g.b[0][i] : (i < 2 * g.n ? g.b[1][i - g.n] : g.b[2][i - 2 * g.n]);
+}
+
 // XF32: x is stored as fp32 and rounded to bf16 (nearest even) on its way into the LDS tile; everything
 // behind the tile, the sum of squares included, sees the rounded values.
-template <int NT, bool XF32 = false>
+template <int NT, bool XF32 = false, bool PF32 = false>
 __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
                                                             const bf16_t *__restrict__ phi,
                                                             float *__restrict__ Ppart,
                                                             float *__restrict__ ssqpart, int B,
                                                             int D, int DP, int nC, int tiles_s, int KS,
-                                                            int sub /* K per wave, multiple of 64 */) {
+                                                            int sub /* K per wave, multiple of 64 */,
+                                                            PhiSrc src /* PF32 */) {
     extern __shared__ __align__(16) float lds[];  // per wave [(1 + NT) * 32][pitch] bf16; later [4][NT*16 + 1][64] fp32
     using TXS = typename std::conditional<XF32, float, bf16_t>::type;  // storage type of x
+    using TPS = typename std::conditional<PF32, float, bf16_t>::type;  // storage type of phi
     const TXS *__restrict__ x = static_cast<const TXS *>(x_);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int set = (blockIdx.x >> 3) / tiles_s;
@@ -114,7 +139,7 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     bf16_t *cb = reinterpret_cast<bf16_t *>(lds) + (size_t)wave * (1 + NT) * 32 * kNarrowPitch;
     const int lr = lane >> 3, seg = lane & 7;
     const TXS *xrow[4];
-    const bf16_t *prow[NT][4];
+    const TPS *prow[NT][4];
     bool xval[4], pval[NT][4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -125,15 +150,17 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
         for (int t = 0; t < NT; t++) {
             const int d = dbase + t * 32 + lr + 8 * j;
             pval[t][j] = d < D;
-            prow[t][j] = phi + (size_t)(pval[t][j] ? d : 0) * nC;
+            if constexpr (PF32) prow[t][j] = phi_src_row(src, pval[t][j] ? d : 0, nC);
+            else prow[t][j] = phi + (size_t)(pval[t][j] ? d : 0) * nC;
         }
     }
     constexpr int XW = XF32 ? 8 : 4;  // words of a lane's 8 elements of x as loaded
-    uint32_t xq[4][XW], pq[NT][4][4];  // scalar words: whole-uint4 array elements can end up in scratch
-    auto load_x8 = [&](const TXS *p, uint32_t (&q)[XW], bool ok) {
+    constexpr int PW = PF32 ? 8 : 4;
+    uint32_t xq[4][XW], pq[NT][4][PW];  // scalar words: whole-uint4 array elements can end up in scratch
+    auto load8 = [&](const auto *p, auto &q, bool ok) {
         const uint4 v = load16_masked(reinterpret_cast<const uint4 *>(p), ok);
         q[0] = v.x; q[1] = v.y; q[2] = v.z; q[3] = v.w;
-        if constexpr (XF32) {
+        if constexpr (sizeof(q) == 32) {
             const uint4 v2 = load16_masked(reinterpret_cast<const uint4 *>(p) + 1, ok);
             q[4] = v2.x; q[5] = v2.y; q[6] = v2.z; q[7] = v2.w;
         }
@@ -147,17 +174,9 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
         if (k0 + 64 <= kend) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                if constexpr (XF32) {
-                    load_x8(xrow[j] + k, xq[j], true);
-                } else {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(xrow[j] + k);
-                    xq[j][0] = v.x; xq[j][1] = v.y; xq[j][2] = v.z; xq[j][3] = v.w;
-                }
+                load8(xrow[j] + k, xq[j], true);
 #pragma unroll
-                for (int t = 0; t < NT; t++) {
-                    const uint4 p = *reinterpret_cast<const uint4 *>(prow[t][j] + k);
-                    pq[t][j][0] = p.x; pq[t][j][1] = p.y; pq[t][j][2] = p.z; pq[t][j][3] = p.w;
-                }
+                for (int t = 0; t < NT; t++) load8(prow[t][j] + k, pq[t][j], true);
             }
             return;
         }
@@ -165,30 +184,35 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
         const int off = kv ? k : 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            load_x8(xrow[j] + off, xq[j], kv);
+            load8(xrow[j] + off, xq[j], kv);
 #pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const uint4 p = load16_masked(reinterpret_cast<const uint4 *>(prow[t][j] + off), kv);
-                pq[t][j][0] = p.x; pq[t][j][1] = p.y; pq[t][j][2] = p.z; pq[t][j][3] = p.w;
-            }
+            for (int t = 0; t < NT; t++) load8(prow[t][j] + off, pq[t][j], kv);
         }
     };
-    auto park = [&]() {
+    auto as_bf16 = [&](const auto &q) {
+        if constexpr (sizeof(q) == 32)
+            return make_uint4(pack_bf16x2(__uint_as_float(q[0]), __uint_as_float(q[1])),
+                              pack_bf16x2(__uint_as_float(q[2]), __uint_as_float(q[3])),
+                              pack_bf16x2(__uint_as_float(q[4]), __uint_as_float(q[5])),
+                              pack_bf16x2(__uint_as_float(q[6]), __uint_as_float(q[7])));
+        else
+            return make_uint4(q[0], q[1], q[2], q[3]);
+    };
+    auto park = [&](int k0) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            if constexpr (XF32)
-                *reinterpret_cast<uint4 *>(cb + (size_t)(lr + 8 * j) * kNarrowPitch + seg * 8) =
-                    make_uint4(pack_bf16x2(__uint_as_float(xq[j][0]), __uint_as_float(xq[j][1])),
-                               pack_bf16x2(__uint_as_float(xq[j][2]), __uint_as_float(xq[j][3])),
-                               pack_bf16x2(__uint_as_float(xq[j][4]), __uint_as_float(xq[j][5])),
-                               pack_bf16x2(__uint_as_float(xq[j][6]), __uint_as_float(xq[j][7])));
-            else
-            *reinterpret_cast<uint4 *>(cb + (size_t)(lr + 8 * j) * kNarrowPitch + seg * 8) =
-                make_uint4(xq[j][0], xq[j][1], xq[j][2], xq[j][3]);
+            *reinterpret_cast<uint4 *>(cb + (size_t)(lr + 8 * j) * kNarrowPitch + seg * 8) = as_bf16(xq[j]);
 #pragma unroll
-            for (int t = 0; t < NT; t++)
-                *reinterpret_cast<uint4 *>(cb + (size_t)(32 + t * 32 + lr + 8 * j) * kNarrowPitch + seg * 8) =
-                    make_uint4(pq[t][j][0], pq[t][j][1], pq[t][j][2], pq[t][j][3]);
+            for (int t = 0; t < NT; t++) {
+                const uint4 p = as_bf16(pq[t][j]);
+                *reinterpret_cast<uint4 *>(cb + (size_t)(32 + t * 32 + lr + 8 * j) * kNarrowPitch + seg * 8) = p;
+                if constexpr (PF32) {
+                    // rows of D * nC elements, nC % 8 == 0: the chunk is 16-byte aligned and whole
+                    const int k = k0 + seg * 8;
+                    if (st == 0 && pval[t][j] && k < kend)
+                        *reinterpret_cast<uint4 *>(src.phi_out + (size_t)(dbase + t * 32 + lr + 8 * j) * nC + k) = p;
+                }
+            }
         }
     };
 
@@ -200,9 +224,11 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     float ssq = 0.f;
 
     if (kbeg < kend) fetch(kbeg);
+    if constexpr (PF32)
+        if (blockIdx.x == 0 && blockIdx.y == 0) gather_small(src, threadIdx.x, 256, D);
     MHC_PHASE_ADD(kPhaseProjFwd, pwg, 0, pclk);
     for (int k0 = kbeg; k0 < kend; k0 += 64) {
-        park();
+        park(k0);
         // (a wave's LDS accesses complete in order; the fence keeps the compiler from moving the
         // fragment reads above the writes of its own tile)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -292,14 +318,15 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
 // --------------------------------------------------------------------------------------------
 constexpr int kWideLd = 72;  // LDS row stride in bf16 elements: 128 data bytes + 16 pad
 
-template <int NT, int P, int NWM = 2, int NWN = 2>
+// PF32: phi comes from the caller's fp32 matrices, see PhiSrc
+template <int NT, int P, int NWM = 2, int NWN = 2, bool PF32 = false>
 __global__ __launch_bounds__(64 * NWM * NWN) void proj_fwd_wide_kernel(const bf16_t *__restrict__ x,
                                                             const bf16_t *__restrict__ phi,
                                                             float *__restrict__ Ppart,
                                                             float *__restrict__ ssqpart, int B,
                                                             int D, int DP, int nC, int groups,
                                                             int sgroups, int KS,
-                                                            int cpk /* chunks per K slab */) {
+                                                            int cpk /* chunks per K slab */, PhiSrc src) {
     static_assert(P % 2 == 0, "buffer parity is tied to the FIFO slot");
     constexpr int R = NT * 32 * NWN;   // projection rows per workgroup
     constexpr int NTHR = 64 * NWM * NWN;     // NWM x NWN waves: a wave owns 128 / NWM samples x NT*32 rows
@@ -338,15 +365,19 @@ __global__ __launch_bounds__(64 * NWM * NWN) void proj_fwd_wide_kernel(const bf1
     for (int j = 0; j < PJ; j++) {
         const int d = group * R + lrow + RSTEP * j;
         pv[j] = d < D;
-        pg[j] = reinterpret_cast<const uint4 *>(phi + (size_t)(pv[j] ? d : 0) * nC) + seg;
+        if constexpr (PF32) pg[j] = reinterpret_cast<const uint4 *>(phi_src_row(src, pv[j] ? d : 0, nC)) + 2 * seg;
+        else pg[j] = reinterpret_cast<const uint4 *>(phi + (size_t)(pv[j] ? d : 0) * nC) + seg;
     }
     // No per-lane predicate on the loads: rows beyond B / D alias row 0 (their products are never
     // stored) and nC % 64 == 0, so a loaded value is not touched until it is parked in LDS and
     // the loads of all P slots stay in flight.
-    uint4 rg[P][XJ + PJ];  // per slot: XJ segments of x, then PJ of phi
+    constexpr int PS = PF32 ? 2 : 1;            // 16-byte pieces per segment of phi
+    uint4 rg[P][XJ + PJ * PS];  // per slot: XJ segments of x, then PJ of phi
     auto issue = [&](int slot_, int c) {
 #pragma unroll
-        for (int j = 0; j < PJ; j++) rg[slot_][XJ + j] = pg[j][c * 8];
+        for (int j = 0; j < PJ; j++)
+#pragma unroll
+            for (int h = 0; h < PS; h++) rg[slot_][XJ + j * PS + h] = pg[j][c * 8 * PS + h];
 #pragma unroll
         for (int j = 0; j < XJ; j++) rg[slot_][j] = xg[j][c * 8];
     };
@@ -364,15 +395,26 @@ __global__ __launch_bounds__(64 * NWM * NWN) void proj_fwd_wide_kernel(const bf1
 
     // park slot j in LDS buffer j & 1, then multiply that buffer; with prefetch, `next` is the
     // chunk whose loads refill the slot
-    auto step = [&](int j, int next, auto prefetch) {
+    auto step = [&](int j, int cur, int next, auto prefetch) {
         bf16_t *xs = lds_w + (size_t)(j & 1) * (128 + R) * kWideLd;
         bf16_t *ps = xs + 128 * kWideLd;
 #pragma unroll
         for (int q = 0; q < XJ; q++)
             *reinterpret_cast<uint4 *>(xs + (lrow + RSTEP * q) * kWideLd + seg * 8) = rg[j][q];
 #pragma unroll
-        for (int q = 0; q < PJ; q++)
-            *reinterpret_cast<uint4 *>(ps + (lrow + RSTEP * q) * kWideLd + seg * 8) = rg[j][XJ + q];
+        for (int q = 0; q < PJ; q++) {
+            uint4 p = rg[j][XJ + q * PS];
+            if constexpr (PF32) {
+                const uint4 p2 = rg[j][XJ + q * PS + 1];
+                p = make_uint4(pack_bf16x2(__uint_as_float(p.x), __uint_as_float(p.y)),
+                               pack_bf16x2(__uint_as_float(p.z), __uint_as_float(p.w)),
+                               pack_bf16x2(__uint_as_float(p2.x), __uint_as_float(p2.y)),
+                               pack_bf16x2(__uint_as_float(p2.z), __uint_as_float(p2.w)));
+                if (sg == 0 && pv[q])  // every (row group, K slab) stores its part of the packed phi once
+                    *reinterpret_cast<uint4 *>(src.phi_out + (size_t)(group * R + lrow + RSTEP * q) * nC + cur * 64 + seg * 8) = p;
+            }
+            *reinterpret_cast<uint4 *>(ps + (lrow + RSTEP * q) * kWideLd + seg * 8) = p;
+        }
         if (want_ssq) {
 #pragma unroll
             for (int q = 0; q < XJ; q++) {
@@ -405,18 +447,20 @@ __global__ __launch_bounds__(64 * NWM * NWN) void proj_fwd_wide_kernel(const bf1
         }
     };
 
+    if constexpr (PF32)
+        if (item == 0) gather_small(src, tid, NTHR, D);
     // prologue: fill the FIFO (indices beyond the slab are clamped: redundant, never consumed)
 #pragma unroll
     for (int j = 0; j < P; j++) issue(j, min(cbeg + j, cend - 1));
     int c = cbeg;
     for (; c + P <= cend; c += P) {
 #pragma unroll
-        for (int j = 0; j < P; j++) step(j, min(c + j + P, cend - 1), std::true_type{});
+        for (int j = 0; j < P; j++) step(j, c + j, min(c + j + P, cend - 1), std::true_type{});
     }
     const int rem = cend - c;  // < P chunks left, all already in flight
 #pragma unroll
     for (int j = 0; j < P - 1; j++)
-        if (j < rem) step(j, 0, std::false_type{});
+        if (j < rem) step(j, c + j, 0, std::false_type{});
 
     // accumulator layout of a 32x32 tile: lane -> column (lane & 31),
     // register i -> row 8 * (i / 4) + 4 * (lane / 32) + (i % 4)
@@ -444,9 +488,9 @@ __global__ __launch_bounds__(64 * NWM * NWN) void proj_fwd_wide_kernel(const bf1
     }
 }
 
-template <int NT, int P, int NWM = 2, int NWN = 2>
+template <int NT, int P, int NWM = 2, int NWN = 2, bool PF32 = false>
 static hipError_t launch_wide(const void *x, const void *phi, float *Ppart, float *ssqpart, int KS,
-                              int B, int D, int DP, int nC, hipStream_t stream) {
+                              int B, int D, int DP, int nC, hipStream_t stream, const PhiSrc &src = PhiSrc{}) {
     const int sgroups = (B + 127) / 128;
     constexpr int R = NT * 32 * NWN;
     const int groups = (DP + R - 1) / R;
@@ -455,13 +499,13 @@ static hipError_t launch_wide(const void *x, const void *phi, float *Ppart, floa
     const int grid = 8 * ((groups * sgroups * KS + 7) / 8);
     const size_t smem = sizeof(bf16_t) * 2 * (128 + R) * kWideLd;
     if (smem > 64 * 1024) {  // above the default dynamic-LDS limit (the CU has 160 KB)
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&proj_fwd_wide_kernel<NT, P, NWM, NWN>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&proj_fwd_wide_kernel<NT, P, NWM, NWN, PF32>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         if (e != hipSuccess) return e;
     }
-    proj_fwd_wide_kernel<NT, P, NWM, NWN><<<grid, 64 * NWM * NWN, smem, stream>>>(
+    proj_fwd_wide_kernel<NT, P, NWM, NWN, PF32><<<grid, 64 * NWM * NWN, smem, stream>>>(
         static_cast<const bf16_t *>(x), static_cast<const bf16_t *>(phi), Ppart, ssqpart, B, D, DP,
-        nC, groups, sgroups, KS, cpk);
+        nC, groups, sgroups, KS, cpk, src);
     return hipGetLastError();
 }
 
@@ -539,9 +583,9 @@ static hipError_t launch_generic(const void *x, const void *phi, float *Ppart, f
     return hipGetLastError();
 }
 
-template <int NT, bool XF32 = false>
+template <int NT, bool XF32 = false, bool PF32 = false>
 static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, float *ssqpart, int KS,
-                              int B, int D, int DP, int nC, hipStream_t stream) {
+                              int B, int D, int DP, int nC, hipStream_t stream, const PhiSrc &src = PhiSrc{}) {
     const int tiles_s = (B + 31) / 32;
     const int groups = (DP / 32 + NT - 1) / NT;
     const int sub = round_up((nC + KS * 4 - 1) / (KS * 4), 64);  // whole 128-byte lines per lane pair
@@ -549,15 +593,58 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
     const size_t smem_chunks = sizeof(bf16_t) * 4 * (1 + NT) * 32 * kNarrowPitch;
     const size_t smem_sum = sizeof(float) * 4 * (NT * 16 + 1) * 64;
     const size_t smem = smem_chunks > smem_sum ? smem_chunks : smem_sum;
-    if (hipError_t e = allow_dynamic_lds(&proj_fwd_mfma_kernel<NT, XF32>, smem); e != hipSuccess) return e;
-    proj_fwd_mfma_kernel<NT, XF32><<<grid, 256, smem, stream>>>(x, static_cast<const bf16_t *>(phi), Ppart,
-                                                                 ssqpart, B, D, DP, nC, tiles_s, KS, sub);
+    if (hipError_t e = allow_dynamic_lds(&proj_fwd_mfma_kernel<NT, XF32, PF32>, smem); e != hipSuccess) return e;
+    proj_fwd_mfma_kernel<NT, XF32, PF32><<<grid, 256, smem, stream>>>(x, static_cast<const bf16_t *>(phi), Ppart,
+                                                                 ssqpart, B, D, DP, nC, tiles_s, KS, sub, src);
     return hipGetLastError();
 }
 
+// Where the projection reads the caller's fp32 parameters itself.  In a narrow projection every tile of 32
+// samples reads all of phi, so fp32 doubles what the tiles pull through L1 and a large batch pays more than the
+// packing launch costs; the more row tiles of phi (n), the sooner.  In a wide one a workgroup covers 128 samples
+// and every element of phi is read once per 128.  Forward in graphs of ten, packing launch -> in the projection (us):
+//   n=4 C=1280: B=8 12.3 -> 10.8, 320 13.3 -> 12.0, 2560 29.6 -> 29.2, 4096 38.2 -> 38.2, 8192 66.8 -> 69.9
+//   n=6 C=1280: B=512 18.6 -> 17.9, 1024 27.3 -> 27.2, 2048 41.4 -> 43.4
+//   n=8 C=1280: B=256 18.7 -> 18.9, 512 22.9 -> 28.1;  C=2560: B=384 30.8 -> 30.1  (and one launch less on the host)
+//   n=32 C=1280: B=64 89.0 -> 66.5, 128 91.5 -> 75.0, 256 112.5 -> 109.5, 384 137.9 -> 140.2;  n=16: B=128 39.2 -> 30.6
+bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
+    auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    if (g.phi_dtype != kF32 || g.out_dtype != kBF16 || !al16(g.phi[0]) || !al16(g.phi[1]) || !al16(g.phi[2]) ||
+        !use_mfma(x_dtype, kBF16, C))
+        return false;
+    if (const int hook = tuning_get(kTuneGather)) return hook == 2 && (use_wide(n, C) || mfma_nt(n) <= 3);
+    if (use_wide(n, C)) return B <= 320;
+    const int nt = mfma_nt(n);
+    return B <= (nt == 1 ? 4096 : (nt == 2 ? 1024 : 384)) && nt <= 3;
+}
+
 hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_dtype, float *Ppart,
-                           float *ssqpart, int KS, int B, int n, int C, hipStream_t stream) {
+                           float *ssqpart, int KS, int B, int n, int C, hipStream_t stream,
+                           const ParamGather *gather) {
     const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n);
+    if (gather) {
+        PhiSrc src;
+        for (int i = 0; i < 3; i++) {
+            src.phi[i] = static_cast<const float *>(gather->phi[i]);
+            src.b[i] = gather->b[i];
+            src.alpha[i] = gather->alpha[i];
+        }
+        src.phi_out = static_cast<bf16_t *>(gather->phi_out);
+        src.bias_out = gather->bias_out;
+        src.alpha_out = gather->alpha_out;
+        src.n = n;
+        if (use_wide(n, C)) return launch_wide<1, 2, 4, 2, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+        const bool xf32 = x_dtype == kF32AsBF16;
+        switch (mfma_nt(n)) {
+            case 1: return xf32 ? launch_mfma<1, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src)
+                                : launch_mfma<1, false, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+            case 2: return xf32 ? launch_mfma<2, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src)
+                                : launch_mfma<2, false, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+            case 3: return xf32 ? launch_mfma<3, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src)
+                                : launch_mfma<3, false, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+            default: return hipErrorInvalidValue;
+        }
+    }
     if (use_mfma(x_dtype, phi_dtype, C)) {
         if (x_dtype == kF32AsBF16) {  // fp32 storage, rounded on load: the narrow kernel only (n <= 8)
             switch (use_wide(n, C) ? 0 : mfma_nt(n)) {

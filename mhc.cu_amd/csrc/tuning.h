@@ -18,7 +18,8 @@ enum TuneKey {
     kTuneResident = 7,      // n <= 8 sample-resident backward: 0 = by heuristic, 1 = never, 2 = whenever the shape allows
     kTuneWideDxBeside = 8,  // wide projections (n > 18): dx workgroups beside the coefficient launch: 1 = never, 2 = always
     kTuneSpareB = 9,        // projection forward (matrix-core kernels): K splits, 0 = by heuristic
-    kTuneCount = 10
+    kTuneGather = 10,       // projection reads the caller's fp32 parameters itself: 1 = never, 2 = whenever the shape allows
+    kTuneCount = 11
 };
 
 #ifdef MHC_TUNING

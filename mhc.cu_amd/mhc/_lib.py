@@ -40,6 +40,10 @@ _SIGNATURES = {
                                       _P, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),
     "mhc_layer_bwd_dynamic": (c_int, [_P, _I, _P, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P,
                                       _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),
+    "mhc_layer_fwd_dynamic_params": (c_int, [_P, _I, _P, _I, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P,
+                                             _P, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),
+    "mhc_layer_bwd_dynamic_dw": (c_int, [_P, _I, _P, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P,
+                                         _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),
     "mhc_pack_dynamic_params": (c_int, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _P]),
     "mhc_static_scratch_capacity": (_Z, []),
     "mhc_layer_fwd_dynamic_scratch_bytes": (_Z, [_I, _I, _I]),
@@ -51,6 +55,8 @@ _SIGNATURES = {
                               _F, _P, _Z, _P]),
     "mhc_layer_bwd": (c_int, [_P, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                               _P, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),
+    "mhc_layer_bwd_dw": (c_int, [_P, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P,
+                                 _P, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),
     "mhc_sinkhorn_knopp_fwd": (c_int, [_P, _P, _I, _I, _I, _I, _F, _P]),
     "mhc_sinkhorn_knopp_bwd": (c_int, [_P, _P, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),
     "mhc_sinkhorn_knopp_bwd_workspace_bytes": (_Z, [_I, _I, _I, _I]),

@@ -148,11 +148,11 @@ struct DynParams {
     const Tensor *src[9];  // phi_pre, phi_post, phi_res, alpha_pre, alpha_post, alpha_res, b_pre, b_post, b_res
 };
 
-void pack_params_into(const DynParams &p, int n, int C, int cd, void *phi, float *ba) {
-    // the three phi matrices in one source dtype the kernel reads (float32 or bfloat16)
+// the parameters as the library takes them: device, dtype and shape checked; m keeps converted copies alive
+struct mhc_dynamic_params library_params(const DynParams &p, int n, int C, Tensor (&m)[9]) {
+    // the three phi matrices in one source dtype the kernels read (float32 or bfloat16)
     const bool same_dt = p.src[0]->scalar_type() == p.src[1]->scalar_type() && p.src[0]->scalar_type() == p.src[2]->scalar_type() &&
                          is_act_dtype(*p.src[0]);
-    Tensor m[9];
     for (int i = 0; i < 9; i++) {
         require_gpu(*p.src[i]);
         m[i] = i < 3 && same_dt ? p.src[i]->contiguous() : f32c(*p.src[i]);
@@ -160,11 +160,8 @@ void pack_params_into(const DynParams &p, int n, int C, int cd, void *phi, float
     TORCH_CHECK(m[0].numel() == (int64_t)n * n * C && m[1].numel() == m[0].numel() && m[2].numel() == (int64_t)n * n * n * C,
                 "mhc: phi shapes do not match expansion rate ", n, " and hidden size ", C);
     TORCH_CHECK(m[6].numel() == n && m[7].numel() == n && m[8].numel() == n * n, "mhc: bias shapes do not match n = ", n);
-    const int D = n * n + 2 * n;
-    check("mhc_pack_dynamic_params",
-          mhc_pack_dynamic_params(ptr(m[0]), ptr(m[1]), ptr(m[2]), dt(m[0]), m[6].data_ptr<float>(), m[7].data_ptr<float>(),
-                                  m[8].data_ptr<float>(), m[3].data_ptr<float>(), m[4].data_ptr<float>(),
-                                  m[5].data_ptr<float>(), phi, cd, ba, ba + D, n, C, stream_of(m[0])));
+    return {ptr(m[0]), ptr(m[1]), ptr(m[2]), dt(m[0]), m[6].data_ptr<float>(), m[7].data_ptr<float>(), m[8].data_ptr<float>(),
+            m[3].data_ptr<float>(), m[4].data_ptr<float>(), m[5].data_ptr<float>()};
 }
 
 bool g_param_cache = false;
@@ -203,7 +200,12 @@ Packed cached_params(const DynParams &p, const Tensor &x, int n, int C, int cd) 
     Packed out;
     out.phi = at::empty({D, (int64_t)n * C}, x.options().dtype(cd == MHC_BF16 ? at::kBFloat16 : at::kFloat));
     out.ba = at::empty({D + 3}, x.options().dtype(at::kFloat));
-    pack_params_into(p, n, C, cd, out.phi.data_ptr(), out.ba.data_ptr<float>());
+    Tensor m[9];
+    const struct mhc_dynamic_params lp = library_params(p, n, C, m);
+    float *ba = out.ba.data_ptr<float>();
+    check("mhc_pack_dynamic_params",
+          mhc_pack_dynamic_params(lp.phi_pre, lp.phi_post, lp.phi_res, lp.phi_dtype, lp.b_pre, lp.b_post, lp.b_res, lp.alpha_pre,
+                                  lp.alpha_post, lp.alpha_res, out.phi.data_ptr(), cd, ba, ba + D, n, C, stream_of(x)));
     std::lock_guard<std::mutex> lock(mu);
     if (cache.size() >= 4096) cache.clear();
     CacheEntry e;
@@ -282,20 +284,21 @@ struct MHCDynamicBackward final : public torch::autograd::Node {
         const Tensor dy = incoming_gradient(grads[0], x, y_type);
         Tensor dx = at::empty(x.sizes(), x.options());
         Tensor df = has_f ? at::empty(f.sizes(), f.options()) : Tensor();
-        // dphi [D, nC] | dbias [D] dalpha [3] | dw [C], fp32
+        // dphi [D, nC] | dbias [D] dalpha [3], fp32 | dw [C] in the weight's type where the library writes it
+        const at::ScalarType dw_type = w_type == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
         const size_t off_ba = align256((size_t)D * nC * 4), off_w = off_ba + align256((size_t)(D + 3) * 4);
         Tensor g = byte_buffer(x, off_w + (size_t)C * 4);
         char *gp = static_cast<char *>(g.data_ptr());
         float *dphi = reinterpret_cast<float *>(gp), *dba = reinterpret_cast<float *>(gp + off_ba);
         Tensor ws = workspace(x, mhc_layer_dynamic_workspace_bytes(B, n, C));
         check("mhc_layer_bwd_dynamic",
-              mhc_layer_bwd_dynamic(ptr(dy), dt(dy), ptr(x), x_code, ptr(w), has_w ? dt(w) : 0, v.phi, cd, v.ba, v.ba + D, ptr(f),
+              mhc_layer_bwd_dynamic_dw(ptr(dy), dt(dy), ptr(x), x_code, ptr(w), has_w ? dt(w) : 0, v.phi, cd, v.ba, v.ba + D, ptr(f),
                                     v.Hp, v.Ho, v.M, v.P, v.r, v.q, v.sk, ptr(dx), ptr(df),
-                                    has_f ? nullptr : reinterpret_cast<float *>(gp + off_w), dphi, dba, dba + D, B, n, C, iters,
+                                    has_f ? nullptr : gp + off_w, dw_type == at::kBFloat16 ? MHC_BF16 : MHC_F32, dphi, dba, dba + D, B, n, C, iters,
                                     (float)eps, ws.data_ptr(), (size_t)ws.numel(), stream_of(x)));
         variable_list out(12);
         if (task_should_compute_output(0)) out[0] = cast_to(dx, x_type);
-        if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(g, at::kFloat, off_w, {C}), w_type);
+        if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(g, dw_type, off_w, {C}), w_type);
         if (has_f && task_should_compute_output(2)) out[2] = cast_to(df, f_type);
         const int64_t rows[3] = {n, n, (int64_t)n * n}, row0[3] = {0, n, 2 * n};
         for (int i = 0; i < 3; i++) {
@@ -356,17 +359,23 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
         const DynLayout l(B, n, C, (int)iters, record, cd, !cached);
         Tensor kept = byte_buffer(x, l.bytes);
         DynViews v(static_cast<char *>(kept.data_ptr()), l);
+        Tensor ws = workspace(x, mhc_layer_dynamic_workspace_bytes(B, n, C));
+        const int w_dt = w.defined() ? dt(w) : 0;
         if (cached) {
             v.phi = pk.phi.data_ptr();
             v.ba = pk.ba.data_ptr<float>();
+            check("mhc_layer_fwd_dynamic",
+                  mhc_layer_fwd_dynamic(ptr(x), x_code, ptr(w), w_dt, v.phi, cd, v.ba, v.ba + D, ptr(f), ptr(y), dt(y), v.Hp, v.Ho,
+                                        v.M, v.P, v.r, v.q, v.sk, B, n, C, (int)iters, (float)eps, ws.data_ptr(),
+                                        (size_t)ws.numel(), stream_of(x)));
         } else {
-            pack_params_into(params, n, C, cd, v.phi, v.ba);
+            Tensor m[9];
+            const struct mhc_dynamic_params lp = library_params(params, n, C, m);
+            check("mhc_layer_fwd_dynamic",
+                  mhc_layer_fwd_dynamic_params(ptr(x), x_code, ptr(w), w_dt, &lp, v.phi, cd, v.ba, v.ba + D, ptr(f), ptr(y), dt(y),
+                                               v.Hp, v.Ho, v.M, v.P, v.r, v.q, v.sk, B, n, C, (int)iters, (float)eps,
+                                               ws.data_ptr(), (size_t)ws.numel(), stream_of(x)));
         }
-        Tensor ws = workspace(x, mhc_layer_dynamic_workspace_bytes(B, n, C));
-        check("mhc_layer_fwd_dynamic",
-              mhc_layer_fwd_dynamic(ptr(x), x_code, ptr(w), w.defined() ? dt(w) : 0, v.phi, cd, v.ba, v.ba + D, ptr(f), ptr(y),
-                                    dt(y), v.Hp, v.Ho, v.M, v.P, v.r, v.q, v.sk, B, n, C, (int)iters, (float)eps, ws.data_ptr(),
-                                    (size_t)ws.numel(), stream_of(x)));
         if (record) {
             node->x_ = SavedVariable(x, false);
             node->kept_ = SavedVariable(kept, false);
@@ -422,19 +431,20 @@ struct MHCStaticBackward final : public torch::autograd::Node {
         const Tensor dy = incoming_gradient(grads[0], x, y_type);
         Tensor dx = at::empty(x.sizes(), x.options());
         Tensor df = has_f ? at::empty(f.sizes(), f.options()) : Tensor();
-        // dH_pre | dH_post | dH_res, dw [C], fp32
+        // dH_pre | dH_post | dH_res, fp32 | dw [C] in the weight's type where the library writes it
+        const at::ScalarType dw_type = w_type == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
         const size_t off_w = align256((size_t)(2 * n + n * n) * 4);
         Tensor g = byte_buffer(x, off_w + (size_t)C * 4);
         float *d = static_cast<float *>(g.data_ptr()), *s = kept.data_ptr<float>();
         Tensor ws = workspace(x, mhc_layer_static_workspace_bytes(B, n, C));
         check("mhc_layer_bwd",
-              mhc_layer_bwd(ptr(dy), dt(dy), ptr(x), dt(x), ptr(w), has_w ? dt(w) : 0, hp.data_ptr<float>(), ho.data_ptr<float>(),
+              mhc_layer_bwd_dw(ptr(dy), dt(dy), ptr(x), dt(x), ptr(w), has_w ? dt(w) : 0, hp.data_ptr<float>(), ho.data_ptr<float>(),
                             hr.data_ptr<float>(), ptr(f), s, s + n, s + 2 * n, s + 2 * n + n * n, ptr(dx), ptr(df),
-                            has_f ? nullptr : d + off_w / 4, d, d + n, d + 2 * n, B, n, C, iters, (float)eps, ws.data_ptr(),
+                            has_f ? nullptr : d + off_w / 4, dw_type == at::kBFloat16 ? MHC_BF16 : MHC_F32, d, d + n, d + 2 * n, B, n, C, iters, (float)eps, ws.data_ptr(),
                             (size_t)ws.numel(), stream_of(x)));
         variable_list out(6);
         if (task_should_compute_output(0)) out[0] = cast_to(dx, x_type);
-        if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(g, at::kFloat, off_w, {C}), w_type);
+        if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(g, dw_type, off_w, {C}), w_type);
         if (has_f && task_should_compute_output(2)) out[2] = cast_to(df, f_type);
         if (task_should_compute_output(3)) out[3] = cast_to(over(g, at::kFloat, 0, {n}), h_type[0]);
         if (task_should_compute_output(4)) out[4] = cast_to(over(g, at::kFloat, (size_t)n * 4, {n}), h_type[1]);
