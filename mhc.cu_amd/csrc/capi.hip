@@ -140,6 +140,10 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     if (bs2 > bs) bs = bs2;
     const int bs3 = n <= 4 ? bwd_slab_batch_splits(B, n, C) : 1;
     if (bs3 > bs) bs = bs3;
+    const int bs4 = dphi_f32_splits(B, n, C);
+    if (bs4 > bs) bs = bs4;
+    const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1;
+    if (bs5 > bs) bs = bs5;
     w.dphi_part = c.floats(bs > 1 ? (size_t)bs * D * nC : 0);
     w.BP = (B + 31) / 32 * 32;
     w.dPb = reinterpret_cast<unsigned short *>(c.floats(((size_t)w.BP * padded_D(n) + 1) / 2));
@@ -667,6 +671,15 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
                                    ws.dphi_part, S, (size_t)D * n * C, dphi, st));
         return MHC_OK;
     }
+    if (bwd_slab_f32_supported(x_dtype, phi_dtype, n, C)) {
+        const int S = bwd_slab_f32_splits(B, C);
+        MHC_LAUNCH(launch_bwd_slab_f32(static_cast<const float *>(dy), static_cast<const float *>(x), w, w_dtype, f_inject,
+                                       static_cast<const float *>(phi), H_pre, H_post, M, q, out, static_cast<float *>(dx),
+                                       static_cast<float *>(df), S > 1 ? ws.dphi_part : dphi, ws.u, ws.dtpart, B, n, C, st));
+        MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S, D, dbias, dalpha, ws.dphi_part, S,
+                                   (size_t)D * n * C, dphi, st));
+        return MHC_OK;
+    }
     const int spg = bwd_dx_samples_per_group(B, n);
     const int groups = (B + spg - 1) / spg;
     int S = 1;
@@ -710,7 +723,12 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
                                      n, q, ws.s1, ws.cx, ws.dP, DP, nullptr, 0, dx, dx, df, ws.u, ws.dt,
                                      ws.dtpart, spg, B, n, C, st));
-        MHC_LAUNCH(launch_gemm_f32_dphi(ws.dP, static_cast<const float *>(x), dphi, B, n, C, st));
+        if (n <= 8) {
+            S = dphi_f32_splits(B, n, C);
+            MHC_LAUNCH(launch_dphi_f32(ws.dP, static_cast<const float *>(x), S > 1 ? ws.dphi_part : dphi, S, B, n, C, st));
+        } else {
+            MHC_LAUNCH(launch_gemm_f32_dphi(ws.dP, static_cast<const float *>(x), dphi, B, n, C, st));
+        }
     } else {
         MHC_LAUNCH(launch_mix_bwd_dx(dy, y_dtype, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M,
                                      n, q, ws.s1, ws.cx, ws.dP, DP, phi, phi_dtype, nullptr, dx, df,

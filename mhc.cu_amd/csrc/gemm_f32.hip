@@ -164,6 +164,124 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs a) {
     }
 }
 
+// --------------------------------------------------------------------------------------------
+// dphi of a narrow projection (n <= 8, D <= 96): dphi[d, k] = sum_b dP[b, d] x[b, k]
+//
+// A contraction over the batch with few output rows: bound by reading x once.  The 128 x 128 tiles above pad
+// D = 24 to 128 rows and leave nC / 128 workgroups; here a wave owns all D rows (NT tiles of 32) x 32 CPL
+// columns, the four waves of a workgroup and grid.z split the batch.  Both operands come straight from memory
+// in matrix-core layout, no LDS: lane (l, h) of product s holds dP[b, l] and x[b, columns CPL l ..] of sample
+// b = 2 s + h, i.e. whole 128-byte rows of dP and 512-byte rows of x per half-wave; the CPL columns of a lane
+// feed CPL tiles, so column CPL l + t belongs to tile t and a lane stores CPL consecutive columns.
+// B=2560 n=4 C=1280: 205 -> MEASURED_DPHI us.
+// --------------------------------------------------------------------------------------------
+template <int NT, int CPL>
+__global__ __launch_bounds__(256) void dphi_f32_kernel(const float *__restrict__ dP, const float *__restrict__ x,
+                                                       float *__restrict__ out, int B, int D, int DP, int nC,
+                                                       int per_wave /* samples, even */) {
+    extern __shared__ __align__(16) float lds[];  // [4 waves][NT * CPL * 16][64]
+    constexpr int U = 8;                          // products (pairs of samples) in flight
+    typedef float vec_t __attribute__((ext_vector_type(CPL)));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 31, h = lane >> 5;
+    const int col = blockIdx.x * 32 * CPL + CPL * l;
+    const float *xc = x + (col < nC ? col : 0);  // nC % 4 == 0: a lane's columns are all inside or all outside
+    const float *pc = dP + l;
+    const int b0 = (blockIdx.z * 4 + wave) * per_wave, b1 = min(B, b0 + per_wave);
+
+    f32x16_t acc[NT][CPL];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int c = 0; c < CPL; c++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[t][c][i] = 0.f;
+    vec_t xv[U];
+    float pv[U][NT];
+    auto fetch = [&](int b) {
+#pragma unroll
+        for (int s = 0; s < U; s++) {
+            const int bs = min(b + 2 * s + h, B - 1);  // samples beyond the range meet a zero of dP below
+            xv[s] = *reinterpret_cast<const vec_t *>(xc + (size_t)bs * nC);
+#pragma unroll
+            for (int t = 0; t < NT; t++) pv[s][t] = pc[(size_t)bs * DP + 32 * t];
+        }
+    };
+    if (b0 < b1) fetch(b0);
+    for (int b = b0; b < b1; b += 2 * U) {
+        vec_t xs[U];
+        float ps[U][NT];
+#pragma unroll
+        for (int s = 0; s < U; s++) {
+            xs[s] = xv[s];
+#pragma unroll
+            for (int t = 0; t < NT; t++) ps[s][t] = b + 2 * s + h < b1 ? pv[s][t] : 0.f;
+        }
+        if (b + 2 * U < b1) fetch(b + 2 * U);  // in flight during the products
+#pragma unroll
+        for (int s = 0; s < U; s++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int c = 0; c < CPL; c++)
+                    acc[t][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(ps[s][t], xs[s][c], acc[t][c], 0, 0, 0);
+    }
+    // sum of the four waves: wave w adds and stores accumulator registers 4w .. 4w+3 of every tile
+    constexpr int R = NT * CPL * 16;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int c = 0; c < CPL; c++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) lds[((size_t)wave * R + (t * CPL + c) * 16 + i) * 64 + lane] = acc[t][c][i];
+    __syncthreads();
+    float *o = out + (size_t)blockIdx.z * D * nC + col;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            vec_t v;
+#pragma unroll
+            for (int c = 0; c < CPL; c++) {
+                const float *p = lds + (size_t)((t * CPL + c) * 16 + 4 * wave + q) * 64 + lane;
+                v[c] = (p[0] + p[(size_t)R * 64]) + (p[(size_t)2 * R * 64] + p[(size_t)3 * R * 64]);
+            }
+            const int d = 32 * t + 8 * wave + 4 * h + q;  // accumulator register 4w + q: row 8 w + 4 h + q
+            if (d < D && col < nC) *reinterpret_cast<vec_t *>(o + (size_t)d * nC) = v;
+        }
+}
+
+// columns per lane: accumulators are NT * CPL * 16 registers, two workgroups per CU at most 96 of them
+static int dphi_f32_cpl(int n) { return padded_D(n) == 32 ? 4 : 2; }
+
+int dphi_f32_splits(int B, int n, int C) {
+    if (n > 8) return 1;
+    const int blocks = (n * C + 32 * dphi_f32_cpl(n) - 1) / (32 * dphi_f32_cpl(n));
+    int s = (512 + blocks - 1) / blocks;         // two workgroups per CU
+    if (s > (B + 63) / 64) s = (B + 63) / 64;     // a wave takes at least 16 samples
+    if (s > 16) s = 16;                           // the finalize launch sums sixteen copies per round
+    return s < 1 ? 1 : s;
+}
+
+hipError_t launch_dphi_f32(const float *dP, const float *x, float *out, int S, int B, int n, int C, hipStream_t stream) {
+    const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n), cpl = dphi_f32_cpl(n);
+    const int per_wave = round_up((B + 4 * S - 1) / (4 * S), 2);
+    const dim3 grid((nC + 32 * cpl - 1) / (32 * cpl), 1, S);
+    const size_t smem = sizeof(float) * 4 * (DP / 32) * cpl * 16 * 64;
+#define MHC_DPHI_F32(NT, CPL)                                                                                          \
+    do {                                                                                                               \
+        if (hipError_t e = allow_dynamic_lds(&dphi_f32_kernel<NT, CPL>, smem); e != hipSuccess) return e;              \
+        dphi_f32_kernel<NT, CPL><<<grid, 256, smem, stream>>>(dP, x, out, B, D, DP, nC, per_wave);                     \
+    } while (0)
+    switch (DP / 32) {
+        case 1: MHC_DPHI_F32(1, 4); break;
+        case 2: MHC_DPHI_F32(2, 2); break;
+        case 3: MHC_DPHI_F32(3, 2); break;
+        default: return hipErrorInvalidValue;
+    }
+#undef MHC_DPHI_F32
+    return hipGetLastError();
+}
+
 template <bool AK, bool BK> static hipError_t launch_gemm(const GemmArgs &a, int splits, hipStream_t stream) {
     dim3 grid((a.n_store + kGT - 1) / kGT, (a.M + kGT - 1) / kGT, splits);
     gemm_f32_kernel<AK, BK><<<grid, 256, 0, stream>>>(a);

@@ -107,6 +107,9 @@ hipError_t launch_gemm_f32_proj(const float *x, const float *phi, float *Ppart, 
                                 int B, int n, int C, hipStream_t stream);
 hipError_t launch_gemm_f32_dphi(const float *dP, const float *x, float *dphi, int B, int n, int C,
                                 hipStream_t stream);
+// n <= 8: dphi with the batch split into dphi_f32_splits() copies [S][D][nC] (S == 1: the result itself)
+int dphi_f32_splits(int B, int n, int C);
+hipError_t launch_dphi_f32(const float *dP, const float *x, float *out, int S, int B, int n, int C, hipStream_t stream);
 hipError_t launch_gemm_f32_dxflat(const float *dP, const float *phi, float *dxflat, int B, int n, int C,
                                   hipStream_t stream);
 
@@ -178,6 +181,15 @@ hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const voi
                            const float *cx, const void *dPb, const void *dPT, int BP, const float *dt,
                            void *dx, void *df, float *dphi_part, float *dw_part, float *dt_part, int S,
                            int B, int n, int C, hipStream_t stream);
+
+// The same for the fp32 tier (n <= 4, even C), behind launch_mix_bwd_reduce (dP [B, 32], cx, s1, dt of `co`):
+// dx, df and the batch-split partial sums of dphi [S][D][nC], dw [S][C] and dt [S][D+3], S = bwd_slab_f32_splits().
+bool bwd_slab_f32_supported(int x_dtype, int phi_dtype, int n, int C);
+int bwd_slab_f32_splits(int B, int C);
+hipError_t launch_bwd_slab_f32(const float *dy, const float *x, const void *w, int w_dtype, const void *f_inject,
+                               const float *phi, const float *Hpre, const float *Hpost, const float *M, const float *q,
+                               const BwdCoefOut &co, float *dx, float *df, float *dphi, float *dw_part, float *dt_part,
+                               int B, int n, int C, hipStream_t stream);
 
 // Samples per workgroup of launch_mix_bwd_dx and the resulting row count of u / dtpart.
 int bwd_dx_samples_per_group(int B, int n);

@@ -5,11 +5,13 @@
 // Replaces compute_rms (reference src/csrc/kernels/fused_rmsnorm_matmul.cuh:119-153) and the
 // cuBLASLt projection GEMM (src/python/bindings.cu:34-81, :436-443) with one pass over x.
 //
-// Two kernels:
-//   proj_fwd_mfma_kernel    x and phi both bf16, C % 8 == 0: v_mfma_f32_32x32x16_bf16 tiles
-//                           (32 samples x 32 projection rows), operands fetched row-contiguously
+// Three kernels:
+//   proj_fwd_mfma_kernel    n <= 10; x and phi both bf16 (C % 8 == 0): v_mfma_f32_32x32x16_bf16 tiles
+//                           (32 samples x 32 projection rows), or both fp32 (n <= 8, nC % 4 == 0):
+//                           v_mfma_f32_32x32x2_f32, IEEE products; operands fetched row-contiguously
 //                           through a wave-private LDS tile.
-//   proj_fwd_generic_kernel any dtype / any C: fp32 FMA, exact products (the fp32 parity tier).
+//   proj_fwd_wide_kernel    bf16, wider phi.
+//   proj_fwd_generic_kernel any dtype / any C: fp32 FMA.
 #include "launchers.h"
 
 #include <type_traits>
@@ -88,7 +90,7 @@ constexpr int kNarrowPitch = 72;  // LDS row of a 64-element chunk: 128 data byt
 struct PhiSrc {
     const float *phi[3];
     const float *b[3], *alpha[3];
-    bf16_t *phi_out;
+    void *phi_out;  // in the compute type: bf16, or fp32 in the exact tier
     float *bias_out, *alpha_out;
     int n;
 };
@@ -105,17 +107,24 @@ __device__ __forceinline__ void gather_small(const PhiSrc &g, int tid, int nthr,
 
 // XF32: x is stored as fp32 and rounded to bf16 (nearest even) on its way into the LDS tile; everything
 // behind the tile, the sum of squares included, sees the rounded values.
-template <int NT, bool XF32 = false, bool PF32 = false>
+// EXACT: the fp32 tier.  x and phi stay fp32 and are multiplied as they are; a 16-byte piece of a row is then
+// four elements instead of eight and a chunk 32 instead of 64, everything else (LDS tile, pieces per lane,
+// accumulators) is the same.  With 32 samples per tile and D padded to 32 instead of 128 x 128 tiles the fp32
+// projection of B=2560 n=4 C=1280 went from 58 to MEASURED_PROJ us.
+template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false>
 __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
-                                                            const bf16_t *__restrict__ phi,
+                                                            const void *__restrict__ phi_,
                                                             float *__restrict__ Ppart,
                                                             float *__restrict__ ssqpart, int B,
                                                             int D, int DP, int nC, int tiles_s, int KS,
-                                                            int sub /* K per wave, multiple of 64 */,
+                                                            int sub /* K per wave, whole chunks */,
                                                             PhiSrc src /* PF32 */) {
     extern __shared__ __align__(16) float lds[];  // per wave [(1 + NT) * 32][pitch] bf16; later [4][NT*16 + 1][64] fp32
-    using TXS = typename std::conditional<XF32, float, bf16_t>::type;  // storage type of x
-    using TPS = typename std::conditional<PF32, float, bf16_t>::type;  // storage type of phi
+    static_assert(!(EXACT && XF32), "XF32 rounds");
+    using TXS = typename std::conditional<XF32 || EXACT, float, bf16_t>::type;  // storage type of x
+    using TPS = typename std::conditional<PF32 || EXACT, float, bf16_t>::type;  // storage type of phi
+    using TC = typename std::conditional<EXACT, float, bf16_t>::type;           // compute type
+    constexpr int EL = 16 / sizeof(TC), CH = 8 * EL;  // elements of a 16-byte piece, of a chunk (8 pieces)
     const TXS *__restrict__ x = static_cast<const TXS *>(x_);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int set = (blockIdx.x >> 3) / tiles_s;
@@ -136,7 +145,8 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     // layout of the matrix cores has every lane on a different row, which the memory pipeline
     // serves at a quarter of this rate.  The chunk goes through a wave-private LDS tile and comes
     // back as fragments; no barrier is involved (a wave's LDS accesses complete in order).
-    bf16_t *cb = reinterpret_cast<bf16_t *>(lds) + (size_t)wave * (1 + NT) * 32 * kNarrowPitch;
+    constexpr int PITCH = kNarrowPitch * 2;  // bytes
+    char *cb = reinterpret_cast<char *>(lds) + (size_t)wave * (1 + NT) * 32 * PITCH;
     const int lr = lane >> 3, seg = lane & 7;
     const TXS *xrow[4];
     const TPS *prow[NT][4];
@@ -151,11 +161,11 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
             const int d = dbase + t * 32 + lr + 8 * j;
             pval[t][j] = d < D;
             if constexpr (PF32) prow[t][j] = phi_src_row(src, pval[t][j] ? d : 0, nC);
-            else prow[t][j] = phi + (size_t)(pval[t][j] ? d : 0) * nC;
+            else prow[t][j] = static_cast<const TPS *>(phi_) + (size_t)(pval[t][j] ? d : 0) * nC;
         }
     }
-    constexpr int XW = XF32 ? 8 : 4;  // words of a lane's 8 elements of x as loaded
-    constexpr int PW = PF32 ? 8 : 4;
+    constexpr int XW = EL * sizeof(TXS) / 4;  // words of a lane's piece of x as loaded
+    constexpr int PW = EL * sizeof(TPS) / 4;
     uint32_t xq[4][XW], pq[NT][4][PW];  // scalar words: whole-uint4 array elements can end up in scratch
     auto load8 = [&](const auto *p, auto &q, bool ok) {
         const uint4 v = load16_masked(reinterpret_cast<const uint4 *>(p), ok);
@@ -170,8 +180,8 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     // slab needs a mask - a uniform test per chunk instead of four selects per load (the kernel is
     // bound by VALU issue, not by memory, with four waves per SIMD).
     auto fetch = [&](int k0) {
-        const int k = k0 + seg * 8;
-        if (k0 + 64 <= kend) {
+        const int k = k0 + seg * EL;
+        if (k0 + CH <= kend) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 load8(xrow[j] + k, xq[j], true);
@@ -180,7 +190,7 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
             }
             return;
         }
-        const bool kv = k < kend;  // kend and k are multiples of 8
+        const bool kv = k < kend;  // kend and k are multiples of EL
         const int off = kv ? k : 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -189,7 +199,7 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
             for (int t = 0; t < NT; t++) load8(prow[t][j] + off, pq[t][j], kv);
         }
     };
-    auto as_bf16 = [&](const auto &q) {
+    auto as_tile = [&](const auto &q) {
         if constexpr (sizeof(q) == 32)
             return make_uint4(pack_bf16x2(__uint_as_float(q[0]), __uint_as_float(q[1])),
                               pack_bf16x2(__uint_as_float(q[2]), __uint_as_float(q[3])),
@@ -201,16 +211,16 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     auto park = [&](int k0) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            *reinterpret_cast<uint4 *>(cb + (size_t)(lr + 8 * j) * kNarrowPitch + seg * 8) = as_bf16(xq[j]);
+            *reinterpret_cast<uint4 *>(cb + (size_t)(lr + 8 * j) * PITCH + seg * 16) = as_tile(xq[j]);
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                const uint4 p = as_bf16(pq[t][j]);
-                *reinterpret_cast<uint4 *>(cb + (size_t)(32 + t * 32 + lr + 8 * j) * kNarrowPitch + seg * 8) = p;
+                const uint4 p = as_tile(pq[t][j]);
+                *reinterpret_cast<uint4 *>(cb + (size_t)(32 + t * 32 + lr + 8 * j) * PITCH + seg * 16) = p;
                 if constexpr (PF32) {
-                    // rows of D * nC elements, nC % 8 == 0: the chunk is 16-byte aligned and whole
-                    const int k = k0 + seg * 8;
+                    // nC is a multiple of EL: the piece is 16-byte aligned and whole
+                    const int k = k0 + seg * EL;
                     if (st == 0 && pval[t][j] && k < kend)
-                        *reinterpret_cast<uint4 *>(src.phi_out + (size_t)(dbase + t * 32 + lr + 8 * j) * nC + k) = p;
+                        *reinterpret_cast<uint4 *>(static_cast<TC *>(src.phi_out) + (size_t)(dbase + t * 32 + lr + 8 * j) * nC + k) = p;
                 }
             }
         }
@@ -227,30 +237,42 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     if constexpr (PF32)
         if (blockIdx.x == 0 && blockIdx.y == 0) gather_small(src, threadIdx.x, 256, D);
     MHC_PHASE_ADD(kPhaseProjFwd, pwg, 0, pclk);
-    for (int k0 = kbeg; k0 < kend; k0 += 64) {
+    for (int k0 = kbeg; k0 < kend; k0 += CH) {
         park(k0);
         // (a wave's LDS accesses complete in order; the fence keeps the compiler from moving the
         // fragment reads above the writes of its own tile)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         MHC_PHASE_ADD(kPhaseProjFwd, pwg, 1, pclk);
-        if (k0 + 64 < kend) fetch(k0 + 64);  // in flight while this chunk is multiplied
+        if (k0 + CH < kend) fetch(k0 + CH);  // in flight while this chunk is multiplied
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            // fragment of k-step u: lane (row, kh) holds elements u*16 + kh*8 .. +8 of its row
-            const uint4 av = *reinterpret_cast<const uint4 *>(cb + (size_t)row * kNarrowPitch + u * 16 + kh * 8);
-            const bf16x8_t af = __builtin_bit_cast(bf16x8_t, av);
+            // fragment of k-step u: lane (row, kh) holds the 16 bytes at u*32 + kh*16 of its row
+            const uint4 av = *reinterpret_cast<const uint4 *>(cb + (size_t)row * PITCH + u * 32 + kh * 16);
+            const uint32_t w4[4] = {av.x, av.y, av.z, av.w};
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                const uint4 bv = *reinterpret_cast<const uint4 *>(cb + (size_t)(32 + t * 32 + row) * kNarrowPitch + u * 16 + kh * 8);
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, __builtin_bit_cast(bf16x8_t, bv), acc[t], 0, 0, 0);
+                const uint4 bv = *reinterpret_cast<const uint4 *>(cb + (size_t)(32 + t * 32 + row) * PITCH + u * 32 + kh * 16);
+                if constexpr (EXACT) {
+                    // four products of depth 2: product i contracts element i of both lane halves' pieces
+                    const uint32_t b4[4] = {bv.x, bv.y, bv.z, bv.w};
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w4[i]), __uint_as_float(b4[i]), acc[t], 0, 0, 0);
+                } else {
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, av), __builtin_bit_cast(bf16x8_t, bv),
+                                                                    acc[t], 0, 0, 0);
+                }
             }
-            if (blockIdx.y == 0) {  // sum of squares: v_dot2c_f32_bf16, two elements per instruction
-                const uint32_t w4[4] = {av.x, av.y, av.z, av.w};
+            if (blockIdx.y == 0) {  // sum of squares; bf16: v_dot2c_f32_bf16, two elements per instruction
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const bf16x2_t pr = __builtin_bit_cast(bf16x2_t, w4[i]);
-                    ssq = __builtin_amdgcn_fdot2_f32_bf16(pr, pr, ssq, false);
+                    if constexpr (EXACT) {
+                        ssq = fmaf(__uint_as_float(w4[i]), __uint_as_float(w4[i]), ssq);
+                    } else {
+                        const bf16x2_t pr = __builtin_bit_cast(bf16x2_t, w4[i]);
+                        ssq = __builtin_amdgcn_fdot2_f32_bf16(pr, pr, ssq, false);
+                    }
                 }
             }
         }
@@ -411,7 +433,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void proj_fwd_wide_kernel(const bf1
                                pack_bf16x2(__uint_as_float(p2.x), __uint_as_float(p2.y)),
                                pack_bf16x2(__uint_as_float(p2.z), __uint_as_float(p2.w)));
                 if (sg == 0 && pv[q])  // every (row group, K slab) stores its part of the packed phi once
-                    *reinterpret_cast<uint4 *>(src.phi_out + (size_t)(group * R + lrow + RSTEP * q) * nC + cur * 64 + seg * 8) = p;
+                    *reinterpret_cast<uint4 *>(static_cast<bf16_t *>(src.phi_out) + (size_t)(group * R + lrow + RSTEP * q) * nC + cur * 64 + seg * 8) = p;
             }
             *reinterpret_cast<uint4 *>(ps + (lrow + RSTEP * q) * kWideLd + seg * 8) = p;
         }
@@ -521,13 +543,19 @@ static int mfma_nt(int n) {
 // LDS-staged kernel
 static bool use_wide(int n, int C) { return padded_D(n) / 32 > 4 && (n * C) % 64 == 0; }
 
+// fp32 tier, n <= 8: the narrow kernel in fp32 arithmetic (rows in whole 16-byte pieces)
+static bool use_exact(int x_dtype, int phi_dtype, int n, int C) {
+    return n <= 8 && gemm_f32_supported(x_dtype, phi_dtype, n, C);
+}
+
 int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
     // The generic path always uses one split.  MFMA path: enough workgroups to fill 256 CUs
     // several times over (the K loop is latency-bound per wave), at least 64 K elements per wave.
-    if (gemm_f32_supported(x_dtype, phi_dtype, n, C)) return gemm_f32_proj_ksplit(B, n, C, kMaxKSplit);
-    if (!use_mfma(x_dtype, phi_dtype, C)) return 1;
+    const bool exact = use_exact(x_dtype, phi_dtype, n, C);
+    if (!exact && gemm_f32_supported(x_dtype, phi_dtype, n, C)) return gemm_f32_proj_ksplit(B, n, C, kMaxKSplit);
+    if (!exact && !use_mfma(x_dtype, phi_dtype, C)) return 1;
     const int nC = n * C, DP = padded_D(n);
-    if (use_wide(n, C)) {
+    if (!exact && use_wide(n, C)) {
         // Workgroups = (64-row groups) x (128-sample tiles) x splits.  The chip has 256 CUs and a workgroup
         // (8 waves) loads one: the count that fills every CU once, or twice where that still keeps the
         // splits within the 24 that the coefficient kernel sums in one round of loads, beats the counts in
@@ -553,9 +581,11 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
     const int tiles_s = (B + 31) / 32;
     const int groups = DP / 32 / mfma_nt(n);
     int ks = (1024 + tiles_s * groups - 1) / (tiles_s * groups);
-    const int cap_slab = nC / 256;
+    const int chunk = exact ? 32 : 64;
+    const double esize = exact ? 4.0 : 2.0;
+    const int cap_slab = nC / (4 * chunk);
     // partial sums (KS * B * DP fp32) at most ~1/3 of the bytes this kernel streams (x and phi)
-    const int cap_bytes = (int)(0.35 * (2.0 * B * nC + 2.0 * DP * nC) / (4.0 * B * DP));
+    const int cap_bytes = (int)(0.35 * (esize * B * nC + esize * DP * nC) / (4.0 * B * DP));
     if (ks > cap_slab) ks = cap_slab;
     if (ks > cap_bytes) ks = cap_bytes;
     // the fused forward kernel (n <= 8) sums up to 24 splits (16 when a thread holds two chunks of
@@ -569,7 +599,7 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
     // a wave's share is whole 64-element chunks (launch_mfma): with that share fixed, only as many
     // splits as have work (B=1280 n=4 C=2560: 16 splits of 4 x 192 elements would leave the last two
     // and a half empty; 14 do the same work and the forward sums two partial rows fewer per sample)
-    const int sub = round_up((nC + ks * 4 - 1) / (ks * 4), 64);
+    const int sub = round_up((nC + ks * 4 - 1) / (ks * 4), chunk);
     ks = (nC + 4 * sub - 1) / (4 * sub);
     return ks;
 }
@@ -583,18 +613,18 @@ static hipError_t launch_generic(const void *x, const void *phi, float *Ppart, f
     return hipGetLastError();
 }
 
-template <int NT, bool XF32 = false, bool PF32 = false>
+template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false>
 static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, float *ssqpart, int KS,
                               int B, int D, int DP, int nC, hipStream_t stream, const PhiSrc &src = PhiSrc{}) {
     const int tiles_s = (B + 31) / 32;
     const int groups = (DP / 32 + NT - 1) / NT;
-    const int sub = round_up((nC + KS * 4 - 1) / (KS * 4), 64);  // whole 128-byte lines per lane pair
+    const int sub = round_up((nC + KS * 4 - 1) / (KS * 4), EXACT ? 32 : 64);  // whole chunks: 128-byte lines
     dim3 grid(tiles_s * round_up(KS, 8), groups);
     const size_t smem_chunks = sizeof(bf16_t) * 4 * (1 + NT) * 32 * kNarrowPitch;
     const size_t smem_sum = sizeof(float) * 4 * (NT * 16 + 1) * 64;
     const size_t smem = smem_chunks > smem_sum ? smem_chunks : smem_sum;
-    if (hipError_t e = allow_dynamic_lds(&proj_fwd_mfma_kernel<NT, XF32, PF32>, smem); e != hipSuccess) return e;
-    proj_fwd_mfma_kernel<NT, XF32, PF32><<<grid, 256, smem, stream>>>(x, static_cast<const bf16_t *>(phi), Ppart,
+    if (hipError_t e = allow_dynamic_lds(&proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT>, smem); e != hipSuccess) return e;
+    proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT><<<grid, 256, smem, stream>>>(x, phi, Ppart,
                                                                  ssqpart, B, D, DP, nC, tiles_s, KS, sub, src);
     return hipGetLastError();
 }
@@ -609,9 +639,9 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
 //   n=32 C=1280: B=64 89.0 -> 66.5, 128 91.5 -> 75.0, 256 112.5 -> 109.5, 384 137.9 -> 140.2;  n=16: B=128 39.2 -> 30.6
 bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    if (g.phi_dtype != kF32 || g.out_dtype != kBF16 || !al16(g.phi[0]) || !al16(g.phi[1]) || !al16(g.phi[2]) ||
-        !use_mfma(x_dtype, kBF16, C))
-        return false;
+    if (g.phi_dtype != kF32 || !al16(g.phi[0]) || !al16(g.phi[1]) || !al16(g.phi[2])) return false;
+    if (g.out_dtype == kF32) return use_exact(x_dtype, kF32, n, C) && B <= 4096 && tuning_get(kTuneGather) != 1;
+    if (!use_mfma(x_dtype, kBF16, C)) return false;
     if (const int hook = tuning_get(kTuneGather)) return hook == 2 && (use_wide(n, C) || mfma_nt(n) <= 3);
     if (use_wide(n, C)) return B <= 320;
     const int nt = mfma_nt(n);
@@ -629,10 +659,18 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
             src.b[i] = gather->b[i];
             src.alpha[i] = gather->alpha[i];
         }
-        src.phi_out = static_cast<bf16_t *>(gather->phi_out);
+        src.phi_out = gather->phi_out;
         src.bias_out = gather->bias_out;
         src.alpha_out = gather->alpha_out;
         src.n = n;
+        if (x_dtype == kF32) {
+            switch (mfma_nt(n)) {
+                case 1: return launch_mfma<1, false, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+                case 2: return launch_mfma<2, false, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+                case 3: return launch_mfma<3, false, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+                default: return hipErrorInvalidValue;
+            }
+        }
         if (use_wide(n, C)) return launch_wide<1, 2, 4, 2, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
         const bool xf32 = x_dtype == kF32AsBF16;
         switch (mfma_nt(n)) {
@@ -660,6 +698,14 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
             case 2: return launch_mfma<2>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
             case 3: return launch_mfma<3>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
             default: return launch_mfma<4>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
+        }
+    }
+    if (use_exact(x_dtype, phi_dtype, n, C)) {
+        switch (mfma_nt(n)) {
+            case 1: return launch_mfma<1, false, false, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
+            case 2: return launch_mfma<2, false, false, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
+            case 3: return launch_mfma<3, false, false, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
+            default: return hipErrorInvalidValue;
         }
     }
     if (gemm_f32_supported(x_dtype, phi_dtype, n, C))
