@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs a) {
 // in matrix-core layout, no LDS: lane (l, h) of product s holds dP[b, l] and x[b, columns CPL l ..] of sample
 // b = 2 s + h, i.e. whole 128-byte rows of dP and 512-byte rows of x per half-wave; the CPL columns of a lane
 // feed CPL tiles, so column CPL l + t belongs to tile t and a lane stores CPL consecutive columns.
-// B=2560 n=4 C=1280: 205 -> MEASURED_DPHI us.
+// B=2560 n=4 C=1280: 205 -> 22 us (n <= 4 has since moved into bwd_slab_f32.hip).
 // --------------------------------------------------------------------------------------------
 template <int NT, int CPL>
 __global__ __launch_bounds__(256) void dphi_f32_kernel(const float *__restrict__ dP, const float *__restrict__ x,

@@ -110,7 +110,7 @@ __device__ __forceinline__ void gather_small(const PhiSrc &g, int tid, int nthr,
 // EXACT: the fp32 tier.  x and phi stay fp32 and are multiplied as they are; a 16-byte piece of a row is then
 // four elements instead of eight and a chunk 32 instead of 64, everything else (LDS tile, pieces per lane,
 // accumulators) is the same.  With 32 samples per tile and D padded to 32 instead of 128 x 128 tiles the fp32
-// projection of B=2560 n=4 C=1280 went from 58 to MEASURED_PROJ us.
+// projection of B=2560 n=4 C=1280 went from 58 to 20 us.
 template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false>
 __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
                                                             const void *__restrict__ phi_,
@@ -127,9 +127,14 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     constexpr int EL = 16 / sizeof(TC), CH = 8 * EL;  // elements of a 16-byte piece, of a chunk (8 pieces)
     const TXS *__restrict__ x = static_cast<const TXS *>(x_);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int set = (blockIdx.x >> 3) / tiles_s;
-    const int st = (blockIdx.x >> 3) % tiles_s, ks = (blockIdx.x & 7) + 8 * set;
-    if (ks >= KS) return;  // the whole workgroup, before any barrier
+    // Work item = (K slab, sample tile), tiles fastest.  Workgroup ids go round the 8 XCDs and XCD j takes the
+    // contiguous items [j * per_xcd, (j + 1) * per_xcd): every XCD gets the same number, and a slab of phi is
+    // fetched into one L2 (two where it straddles a border).  (One slab per XCD left XCDs without work whenever
+    // KS was not a multiple of 8: half of the chip at B=8192, KS=4.)
+    const int items = tiles_s * KS, per_xcd = (items + 7) >> 3;
+    const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (item >= items) return;  // the whole workgroup, before any barrier
+    const int st = item % tiles_s, ks = item / tiles_s;
     const int pwg = blockIdx.y * gridDim.x + blockIdx.x;
     (void)pwg;
     MHC_PHASE_ZERO(kPhaseProjFwd, pwg);
@@ -148,25 +153,32 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
     constexpr int PITCH = kNarrowPitch * 2;  // bytes
     char *cb = reinterpret_cast<char *>(lds) + (size_t)wave * (1 + NT) * 32 * PITCH;
     const int lr = lane >> 3, seg = lane & 7;
-    const TXS *xrow[4];
+    // rows as 32-bit byte offsets from a uniform base (32 rows of x, all of phi: far below 4 GB), except where the
+    // rows of phi lie in three matrices: eight registers less, which is one more wave per SIMD
+    const char *xbase = reinterpret_cast<const char *>(x + (size_t)st * 32 * nC);
+    uint32_t xoff[4], poff[NT][4];
     const TPS *prow[NT][4];
-    bool xval[4], pval[NT][4];
+    bool pval[NT][4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int bs = st * 32 + lr + 8 * j;
-        xval[j] = bs < B;
-        xrow[j] = x + (size_t)(xval[j] ? bs : 0) * nC;
+        xoff[j] = (bs < B ? (uint32_t)(lr + 8 * j) * nC : 0u) * (uint32_t)sizeof(TXS);
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const int d = dbase + t * 32 + lr + 8 * j;
             pval[t][j] = d < D;
             if constexpr (PF32) prow[t][j] = phi_src_row(src, pval[t][j] ? d : 0, nC);
-            else prow[t][j] = static_cast<const TPS *>(phi_) + (size_t)(pval[t][j] ? d : 0) * nC;
+            else poff[t][j] = (uint32_t)(pval[t][j] ? d : 0) * (uint32_t)nC * (uint32_t)sizeof(TPS);
         }
     }
     constexpr int XW = EL * sizeof(TXS) / 4;  // words of a lane's piece of x as loaded
     constexpr int PW = EL * sizeof(TPS) / 4;
     uint32_t xq[4][XW], pq[NT][4][PW];  // scalar words: whole-uint4 array elements can end up in scratch
+    auto xat = [&](int j, int k) { return reinterpret_cast<const TXS *>(xbase + (xoff[j] + (uint32_t)k * (uint32_t)sizeof(TXS))); };
+    auto pat = [&](int t, int j, int k) {
+        if constexpr (PF32) return prow[t][j] + k;
+        else return reinterpret_cast<const TPS *>(static_cast<const char *>(phi_) + (poff[t][j] + (uint32_t)k * (uint32_t)sizeof(TPS)));
+    };
     auto load8 = [&](const auto *p, auto &q, bool ok) {
         const uint4 v = load16_masked(reinterpret_cast<const uint4 *>(p), ok);
         q[0] = v.x; q[1] = v.y; q[2] = v.z; q[3] = v.w;
@@ -184,9 +196,9 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
         if (k0 + CH <= kend) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                load8(xrow[j] + k, xq[j], true);
+                load8(xat(j, k), xq[j], true);
 #pragma unroll
-                for (int t = 0; t < NT; t++) load8(prow[t][j] + k, pq[t][j], true);
+                for (int t = 0; t < NT; t++) load8(pat(t, j, k), pq[t][j], true);
             }
             return;
         }
@@ -194,9 +206,9 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
         const int off = kv ? k : 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            load8(xrow[j] + off, xq[j], kv);
+            load8(xat(j, off), xq[j], kv);
 #pragma unroll
-            for (int t = 0; t < NT; t++) load8(prow[t][j] + off, pq[t][j], kv);
+            for (int t = 0; t < NT; t++) load8(pat(t, j, off), pq[t][j], kv);
         }
     };
     auto as_tile = [&](const auto &q) {
@@ -233,18 +245,21 @@ __global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restri
         for (int i = 0; i < 16; i++) acc[t][i] = 0.f;
     float ssq = 0.f;
 
-    if (kbeg < kend) fetch(kbeg);
+    const int nch = kbeg < kend ? (kend - kbeg + CH - 1) / CH : 0;
+    int kc = kbeg + (nch ? st % nch : 0) * CH;  // first chunk
+    if (nch) fetch(kc);
     if constexpr (PF32)
-        if (blockIdx.x == 0 && blockIdx.y == 0) gather_small(src, threadIdx.x, 256, D);
+        if (item == 0 && blockIdx.y == 0) gather_small(src, threadIdx.x, 256, D);
     MHC_PHASE_ADD(kPhaseProjFwd, pwg, 0, pclk);
-    for (int k0 = kbeg; k0 < kend; k0 += CH) {
-        park(k0);
+    for (int it = 0; it < nch; it++) {
+        park(kc);
+        kc = kc + CH < kend ? kc + CH : kbeg;
         // (a wave's LDS accesses complete in order; the fence keeps the compiler from moving the
         // fragment reads above the writes of its own tile)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         MHC_PHASE_ADD(kPhaseProjFwd, pwg, 1, pclk);
-        if (k0 + CH < kend) fetch(k0 + CH);  // in flight while this chunk is multiplied
+        if (it + 1 < nch) fetch(kc);  // in flight while this chunk is multiplied
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             // fragment of k-step u: lane (row, kh) holds the 16 bytes at u*32 + kh*16 of its row
@@ -595,6 +610,19 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
     if (n <= 8 && ks > fused_cap) ks = fused_cap;
     if (ks > 64) ks = 64;
     if (ks < 1) ks = 1;
+    // splits with work when ks are asked for (see below)
+    auto effective = [&](int k) { const int s_ = round_up((nC + k * 4 - 1) / (k * 4), chunk); return (nC + 4 * s_ - 1) / (4 * s_); };
+    if (mfma_nt(n) == 1) {
+        // one row tile of phi: a multiple of 8 gives every XCD whole slabs of phi (forward us, default count -> 8:
+        // B=8192 C=2560 4: 112.7 -> 107.5, B=3001 C=2560 5: 43.3 -> 41.9, fp32 B=2560 C=1280 13: 41.4 -> 38.8)
+        const int k8 = ks < 8 ? 8 : ks / 8 * 8;
+        if (ks >= 4 && k8 <= cap_slab && effective(k8) == k8) ks = k8;
+    } else if (const int wgs = tiles_s * groups; wgs * effective(ks) > 256) {
+        // more row tiles (two workgroups per CU): once per CU instead of once and a bit, but not below 8 (forward us,
+        // n=8 C=1280: bf16 B=1024 16 -> 8 splits 33.7 -> 30.1, B=2048 49.2 -> 44.8, fp32 B=512 20 -> 16 36.9 -> 30.6)
+        const int k = 256 / wgs > 8 ? 256 / wgs : 8;
+        if (k < ks) ks = k;
+    }
     if (const int forced = tuning_get(kTuneSpareB); forced > 0) ks = forced;  // experiment hook
     // a wave's share is whole 64-element chunks (launch_mfma): with that share fixed, only as many
     // splits as have work (B=1280 n=4 C=2560: 16 splits of 4 x 192 elements would leave the last two
@@ -619,7 +647,7 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
     const int tiles_s = (B + 31) / 32;
     const int groups = (DP / 32 + NT - 1) / NT;
     const int sub = round_up((nC + KS * 4 - 1) / (KS * 4), EXACT ? 32 : 64);  // whole chunks: 128-byte lines
-    dim3 grid(tiles_s * round_up(KS, 8), groups);
+    dim3 grid(8 * ((tiles_s * KS + 7) / 8), groups);
     const size_t smem_chunks = sizeof(bf16_t) * 4 * (1 + NT) * 32 * kNarrowPitch;
     const size_t smem_sum = sizeof(float) * 4 * (NT * 16 + 1) * 64;
     const size_t smem = smem_chunks > smem_sum ? smem_chunks : smem_sum;
@@ -633,9 +661,9 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
 // samples reads all of phi, so fp32 doubles what the tiles pull through L1 and a large batch pays more than the
 // packing launch costs; the more row tiles of phi (n), the sooner.  In a wide one a workgroup covers 128 samples
 // and every element of phi is read once per 128.  Forward in graphs of ten, packing launch -> in the projection (us):
-//   n=4 C=1280: B=8 12.3 -> 10.8, 320 13.3 -> 12.0, 2560 29.6 -> 29.2, 4096 38.2 -> 38.2, 8192 66.8 -> 69.9
-//   n=6 C=1280: B=512 18.6 -> 17.9, 1024 27.3 -> 27.2, 2048 41.4 -> 43.4
-//   n=8 C=1280: B=256 18.7 -> 18.9, 512 22.9 -> 28.1;  C=2560: B=384 30.8 -> 30.1  (and one launch less on the host)
+//   n=4 C=1280: B=8 12.3 -> 10.7, 320 13.4 -> 11.9, 4096 37.1 -> 36.1;  C=2560: B=3001 43.8 -> 43.4, 8192 113.6 -> 116.4
+//   n=6 C=1280: B=1024 27.2 -> 26.7, 2048 41.2 -> 42.5
+//   n=8 C=1280: B=256 17.9 -> 18.3, 512 23.0 -> 23.5, 1024 34.0 -> 36.5  (and one launch less on the host)
 //   n=32 C=1280: B=64 89.0 -> 66.5, 128 91.5 -> 75.0, 256 112.5 -> 109.5, 384 137.9 -> 140.2;  n=16: B=128 39.2 -> 30.6
 bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
@@ -645,7 +673,7 @@ bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
     if (const int hook = tuning_get(kTuneGather)) return hook == 2 && (use_wide(n, C) || mfma_nt(n) <= 3);
     if (use_wide(n, C)) return B <= 320;
     const int nt = mfma_nt(n);
-    return B <= (nt == 1 ? 4096 : (nt == 2 ? 1024 : 384)) && nt <= 3;
+    return B <= (nt == 1 ? 4096 : (nt == 2 ? 1024 : 512)) && nt <= 3;
 }
 
 hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_dtype, float *Ppart,
