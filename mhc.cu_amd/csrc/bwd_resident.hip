@@ -77,7 +77,7 @@ template <> struct Act8<true> {
 // the complete dx; wave 0 only turns the sums into the sample's row of raw coefficient gradients
 // (dM | dHpre | dHpost), whose batch sum feeds the one Sinkhorn backward of the static layer.
 template <int NP, int WMODE, int ITEMS, bool F32, bool STATIC = false, int TWV = kResTileWaves>
-__global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1))) void bwd_resident_kernel(BwdResidentArgs ra) {
+__global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void bwd_resident_kernel(BwdResidentArgs ra) {
     using TS = typename std::conditional<F32, float, bf16_t>::type;  // storage type of the activations
     static_assert(NP == 4 || NP == 8, "stream groups of four");
     using SK = SkSmall<NP>;

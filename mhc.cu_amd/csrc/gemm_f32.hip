@@ -85,7 +85,7 @@ __device__ __forceinline__ void park_rc(const Slice &s, float *Xs, int tid) {
 
 // AK / BK: the operand's contiguous index is k.  grid: (N tiles, M tiles, splits)
 template <bool AK, bool BK>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs a) {
+__global__ __launch_bounds__(256, kMfmaMinWaves) void gemm_f32_kernel(GemmArgs a) {
     __shared__ __align__(16) float As[kGK * kGLD];
     __shared__ __align__(16) float Bs[kGK * kGLD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs a) {
 // B=2560 n=4 C=1280: 205 -> 22 us (n <= 4 has since moved into bwd_slab_f32.hip).
 // --------------------------------------------------------------------------------------------
 template <int NT, int CPL>
-__global__ __launch_bounds__(256) void dphi_f32_kernel(const float *__restrict__ dP, const float *__restrict__ x,
+__global__ __launch_bounds__(256, kMfmaMinWaves) void dphi_f32_kernel(const float *__restrict__ dP, const float *__restrict__ x,
                                                        float *__restrict__ out, int B, int D, int DP, int nC,
                                                        int per_wave /* samples, even */) {
     extern __shared__ __align__(16) float lds[];  // [4 waves][NT * CPL * 16][64]

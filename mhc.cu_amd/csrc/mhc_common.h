@@ -209,6 +209,13 @@ __device__ __forceinline__ uint4 load16_masked(const uint4 *p, bool ok) {
 // ---------------------------------------------------------------------------------------------
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short bf16x4_t;
 
+// Second argument of __launch_bounds__ (waves per SIMD at least) of kernels with matrix instructions.  At one
+// wave the register budget is 512, which is only reachable with the accumulation half of the file, and the
+// compiler then gives every matrix result to that half: moves to and from it, and a register count that is
+// the sum of both halves (the 8 x 8 fused forward: 87 + 80, two or three waves per SIMD instead of four).  At two
+// waves everything lives in ordinary registers.
+constexpr int kMfmaMinWaves = 2;
+
 // ---------------------------------------------------------------------------------------------
 // Transposed MFMA operand from a row-major [k][column] bf16 tile in LDS (pitch ld elements, a
 // multiple of 4; col0 a multiple of 4; tile 8-byte aligned): lane (n = lane & 31, kg = lane >> 5)

@@ -232,7 +232,7 @@ __global__ __launch_bounds__(64) void coef_bwd_small_kernel(BwdReduceArgs a) {
 // STATIC (with FUSED): shared coefficients; the tail only converts the sums into the sample's row of raw
 // gradients (see CoefBwdSmall).
 template <int NP, int WMODE, bool FUSED, bool STATIC = false>
-__global__ __launch_bounds__(256, NP == 4 ? 4 : 1) void gram_small_kernel(BwdReduceArgs a) {
+__global__ __launch_bounds__(256, NP == 4 ? 4 : kMfmaMinWaves) void gram_small_kernel(BwdReduceArgs a) {
     static_assert(NP == 4 || NP == 8, "stream groups of four");
     static_assert(FUSED || !STATIC, "the static tail runs inside the launch");
     using SK = SkSmall<NP>;
@@ -429,7 +429,7 @@ __device__ __forceinline__ void static_sinkhorn_forward_block(const BwdReduceArg
 }
 
 template <typename TG, typename TX>
-__global__ __launch_bounds__(256) void gram_large_kernel(BwdReduceArgs a) {
+__global__ __launch_bounds__(256, kMfmaMinWaves) void gram_large_kernel(BwdReduceArgs a) {
     constexpr bool kBf16 = std::is_same<TG, bf16_t>::value && std::is_same<TX, bf16_t>::value;
     constexpr int VL = kBf16 ? 8 : 4;  // columns per lane and k-step
     constexpr int SW = 2 * VL;         // columns per k-step (two lane halves)

@@ -158,7 +158,7 @@ constexpr int kFwdStaggerMinB = 512;  // two or more workgroups per CU
 
 // RX: fp32 x (and f) consumed as bf16, every value rounded to bf16 as it is unpacked
 template <typename TX, typename TY, int NP, int V, int CPT, bool RX = false>
-__global__ __launch_bounds__(256, (CPT == 2 && NP == 4 && !std::is_same<TX, float>::value) ? 4 : 1)
+__global__ __launch_bounds__(256, (CPT == 2 && NP == 4 && !std::is_same<TX, float>::value) ? 4 : kMfmaMinWaves)
 void layer_fwd_small_kernel(LayerFwdArgs a) {
     using SK = SkSmall<NP>;
     __shared__ float coef_s[NP * NP + 2 * NP];  // M | Hpre | Hpost
@@ -688,7 +688,7 @@ constexpr int kMflLDT = kMflCB + 8;   // LDS pitch of the bf16 tile (elements)
 constexpr int kMflLDO = kMflCB + 4;   // LDS pitch of the fp32 output tile
 
 template <typename TY>
-__global__ __launch_bounds__(256) void mix_fwd_large_kernel(MixLargeArgs a) {
+__global__ __launch_bounds__(256, kMfmaMinWaves) void mix_fwd_large_kernel(MixLargeArgs a) {
     extern __shared__ __align__(16) unsigned char mfl_smem[];
     bf16_t *x_s = reinterpret_cast<bf16_t *>(mfl_smem);          // [32][LDT]
     float *o_s = reinterpret_cast<float *>(x_s + 32 * kMflLDT);  // [32][LDO]

@@ -46,7 +46,7 @@ __device__ __forceinline__ bf16x8_t lds_frag_t(const bf16_t *tile, int ld, int k
 enum { kProjBoth = kProjPartBoth, kProjDphi = kProjPartDphi, kProjDx = kProjPartDx };
 
 template <int NTK, int TPW, bool PHI_REGS, int WHAT = kProjBoth>
-__global__ __launch_bounds__(256) void proj_bwd_mfma_kernel(ProjBwdArgs a) {
+__global__ __launch_bounds__(256, kMfmaMinWaves) void proj_bwd_mfma_kernel(ProjBwdArgs a) {
     constexpr bool DO_DPHI = WHAT != kProjDx, DO_DX = WHAT != kProjDphi;
     constexpr int NSB = 4 / NTK;         // 32-sample tiles per block
     constexpr int KW = 32 * NTK;         // slab width

@@ -53,7 +53,7 @@ __device__ __forceinline__ bf16x8_t pl_frag_t(const bf16_t *tile, int k0, int co
 // SINGLE: the split holds one sample block, so a row tile is complete (and stored) right after its
 // MFMAs and one accumulator is live at a time; otherwise TPW accumulators persist over the blocks.
 template <int TPW, bool SINGLE>
-__global__ __launch_bounds__(256) void dphi_large_kernel(ProjBwdLargeArgs a) {
+__global__ __launch_bounds__(256, kMfmaMinWaves) void dphi_large_kernel(ProjBwdLargeArgs a) {
     extern __shared__ __align__(16) bf16_t pl_lds[];
     bf16_t *x_s = pl_lds;  // [kPL_SB][kPL_LD]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

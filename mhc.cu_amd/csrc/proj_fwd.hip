@@ -112,7 +112,7 @@ __device__ __forceinline__ void gather_small(const PhiSrc &g, int tid, int nthr,
 // accumulators) is the same.  With 32 samples per tile and D padded to 32 instead of 128 x 128 tiles the fp32
 // projection of B=2560 n=4 C=1280 went from 58 to 20 us.
 template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false>
-__global__ __launch_bounds__(256) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
+__global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
                                                             const void *__restrict__ phi_,
                                                             float *__restrict__ Ppart,
                                                             float *__restrict__ ssqpart, int B,
