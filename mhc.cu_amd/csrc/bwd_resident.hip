@@ -37,6 +37,9 @@ struct BwdResidentArgs {
 
 constexpr int kResTileWaves = 4;                         // waves that hold the tile
 constexpr int kResMaxItems = 5;                          // 128-channel steps per tile wave
+// rows of more than 4 * 5 * 128 channels: seven tile waves (eight with the coefficient wave are two per SIMD and
+// leave 256 registers; one wave more would leave 168, which 8 x 8 samples do not fit)
+constexpr int kResLongWaves = 7, kResMaxC = 4096;
 
 template <int SEL> __device__ __forceinline__ float quad_bcast(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), SEL * 0x55, 0xF, 0xF, true));
@@ -49,25 +52,28 @@ __device__ __forceinline__ float quad_allreduce(float v) {
 
 // Eight consecutive activation values as four words of bf16 pairs.  bf16 storage: the 16 bytes as
 // loaded.  fp32 storage (F32): two 16-byte loads, rounded to bf16 (nearest even) by get() - called
-// once all loads of the workgroup have been requested.
-template <bool F32> struct Act8;
-template <> struct Act8<false> {
-    uint4 r;
+// once all loads of the workgroup have been requested.  ANY: any element alignment.  The address must be
+// dereferenceable, and a chunk that does not count (ok: false) comes out as zeros.
+template <bool F32, bool ANY> struct Act8;
+template <bool ANY> struct Act8<false, ANY> {
+    uint32_t w[4];
     __device__ __forceinline__ void load(const void *base, size_t elem, bool ok) {
-        r = load16_masked(reinterpret_cast<const uint4 *>(static_cast<const bf16_t *>(base) + (ok ? elem : 0)), ok);
+        const uint4 t = ldg16<ANY>(static_cast<const bf16_t *>(base) + elem);
+        w[0] = ok ? t.x : 0u; w[1] = ok ? t.y : 0u; w[2] = ok ? t.z : 0u; w[3] = ok ? t.w : 0u;
     }
-    __device__ __forceinline__ uint4 get() const { return r; }
+    __device__ __forceinline__ uint4 get() const { return make_uint4(w[0], w[1], w[2], w[3]); }
 };
-template <> struct Act8<true> {
-    uint4 r0, r1;
+template <bool ANY> struct Act8<true, ANY> {
+    uint32_t w[8];
     __device__ __forceinline__ void load(const void *base, size_t elem, bool ok) {
-        const uint4 *p = reinterpret_cast<const uint4 *>(static_cast<const float *>(base) + (ok ? elem : 0));
-        r0 = load16_masked(p, ok);
-        r1 = load16_masked(p + 1, ok);
+        const float *p = static_cast<const float *>(base) + elem;
+        const uint4 t = ldg16<ANY>(p), u = ldg16<ANY>(p + 4);
+        w[0] = ok ? t.x : 0u; w[1] = ok ? t.y : 0u; w[2] = ok ? t.z : 0u; w[3] = ok ? t.w : 0u;
+        w[4] = ok ? u.x : 0u; w[5] = ok ? u.y : 0u; w[6] = ok ? u.z : 0u; w[7] = ok ? u.w : 0u;
     }
     __device__ __forceinline__ uint4 get() const {
-        return make_uint4(pack_bf16x2(__uint_as_float(r0.x), __uint_as_float(r0.y)), pack_bf16x2(__uint_as_float(r0.z), __uint_as_float(r0.w)),
-                          pack_bf16x2(__uint_as_float(r1.x), __uint_as_float(r1.y)), pack_bf16x2(__uint_as_float(r1.z), __uint_as_float(r1.w)));
+        return make_uint4(pack_bf16x2(__uint_as_float(w[0]), __uint_as_float(w[1])), pack_bf16x2(__uint_as_float(w[2]), __uint_as_float(w[3])),
+                          pack_bf16x2(__uint_as_float(w[4]), __uint_as_float(w[5])), pack_bf16x2(__uint_as_float(w[6]), __uint_as_float(w[7])));
     }
 };
 
@@ -76,7 +82,8 @@ template <> struct Act8<true> {
 // STATIC: shared coefficients ([n] / [n, n] instead of per sample).  There is no projection, so dxp is
 // the complete dx; wave 0 only turns the sums into the sample's row of raw coefficient gradients
 // (dM | dHpre | dHpost), whose batch sum feeds the one Sinkhorn backward of the static layer.
-template <int NP, int WMODE, int ITEMS, bool F32, bool STATIC = false, int TWV = kResTileWaves>
+// RAG: rows of any length (C % 8 != 0): the last chunk of a row is loaded from C - 8 on and shifted down.
+template <int NP, int WMODE, int ITEMS, bool F32, bool STATIC = false, int TWV = kResTileWaves, bool RAG = false>
 __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void bwd_resident_kernel(BwdResidentArgs ra) {
     using TS = typename std::conditional<F32, float, bf16_t>::type;  // storage type of the activations
     static_assert(NP == 4 || NP == 8, "stream groups of four");
@@ -134,7 +141,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
 
     // ---- tile waves: every load of the sample up front -----------------------------------------
     uint4 gr[ITEMS][NB], xr[ITEMS][NB], fr[ITEMS];
-    Act8<F32> graw[ITEMS][NB], xraw[ITEMS][NB], fraw[ITEMS];
+    Act8<F32, RAG> graw[ITEMS][NB], xraw[ITEMS][NB], fraw[ITEMS];
     // (the RMSNorm weight chunks stay in registers next to the tile: fetching them again where they are
     // used, one item ahead, to save registers measured slower - B=1280, C=2560 static backward 33.4 -> 34.1 us -
     // and forcing four workgroups per CU made the compiler spill: 50.1 us)
@@ -152,15 +159,17 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
 #pragma unroll
         for (int it = 0; it < ITEMS; it++) {
             const int c = (tw + TW * it) * 128 + blk * 8;
-            in[it] = c < C;  // C % 8 == 0: a chunk is inside or outside
-            const int cc = in[it] ? c : 0;
+            in[it] = c < C;
+            const int cc = in[it] ? (RAG ? min(c, C - 8) : c) : 0;
 #pragma unroll
             for (int I = 0; I < NB; I++) {
                 graw[it][I].load(a.dy, rowoff[I] + cc, in[it] && sv[I]);
                 xraw[it][I].load(a.x, rowoff[I] + cc, in[it] && sv[I]);
             }
             if constexpr (inject) fraw[it].load(a.f_inject, (size_t)b * C + cc, in[it] && i == 0);
+            else if constexpr (WMODE == kGramWBf16 && RAG) wb[it].load_any(static_cast<const bf16_t *>(a.w) + cc);
             else if constexpr (WMODE == kGramWBf16) wb[it].load(static_cast<const bf16_t *>(a.w) + cc);
+            else if constexpr (RAG) wf[it].load_any(static_cast<const float *>(a.w) + cc);
             else wf[it].load(static_cast<const float *>(a.w) + cc);
         }
         // this lane's coefficients for step 3 (its own streams j = 4I + i), in flight with the tile
@@ -189,6 +198,18 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
 #pragma unroll
             for (int I = 0; I < NB; I++) { gr[it][I] = graw[it][I].get(); xr[it][I] = xraw[it][I].get(); }
             if constexpr (inject) fr[it] = fraw[it].get();
+        }
+        if constexpr (RAG) {
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) {
+                const int c = (tw + TW * it) * 128 + blk * 8;
+                const int s = in[it] && c + 8 > C ? c + 8 - C : 0;
+#pragma unroll
+                for (int I = 0; I < NB; I++) { gr[it][I] = drop8(gr[it][I], s); xr[it][I] = drop8(xr[it][I], s); }
+                if constexpr (inject) fr[it] = drop8(fr[it], s);
+                else if constexpr (WMODE == kGramWBf16) wb[it].drop(s);
+                else wf[it].drop(s);
+            }
         }
     }
 
@@ -303,6 +324,11 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     if (!tile) return;  // the coefficient wave (none with STATIC) is done
 
     // ---- 3. tile waves: dxp, u, df ---------------------------------------------------------------------
+    auto put8 = [](auto *p, const float (&v)[8], int left) {  // left: elements up to the row's end
+        using T = typename std::remove_reference<decltype(*p)>::type;
+        if constexpr (RAG) store_vec_any<T, 8>(p, v, left);
+        else store_vec<T, 8>(p, v);
+    };
     float qinv = 0.f, k2 = 0.f;
     if constexpr (!inject) {
         qinv = 1.0f / qraw;
@@ -334,7 +360,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
         if constexpr (inject) {
 #pragma unroll
             for (int v = 0; v < 8; v++) da[v] = 0.f;
-            if (ra.df && i == 0) store_vec<TS, 8>(static_cast<TS *>(ra.df) + (size_t)b * C + c, dfv);
+            if (ra.df && i == 0) put8(static_cast<TS *>(ra.df) + (size_t)b * C + c, dfv, C - c);
         } else {
             float wv[8], uv[8];
             if constexpr (WMODE == kGramWBf16) wb[it].get(wv);
@@ -348,7 +374,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                 da[v] = dfv[v] * wv[v] * qinv - av * k2;
                 uv[v] = dfv[v] * av * qinv;
             }
-            if (i == 0) store_vec<float, 8>(ra.u + (size_t)b * C + c, uv);
+            if (i == 0) put8(ra.u + (size_t)b * C + c, uv, C - c);
         }
 #pragma unroll
         for (int I = 0; I < NB; I++) {
@@ -365,7 +391,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                     out[v] += Mc[I][J][3] * quad_bcast<3>(gv[J][v]);
                 }
             // plain stores: the projection-backward launch reads dxp back right away
-            if (sv[I]) store_vec<TS, 8>(static_cast<TS *>(ra.dxp) + ((size_t)b * n + 4 * I + i) * C + c, out);
+            if (sv[I]) put8(static_cast<TS *>(ra.dxp) + ((size_t)b * n + 4 * I + i) * C + c, out, C - c);
         }
     }
     MHC_PHASE_ADD_BY(64, kPhaseDxSmall, pwg, 3, tclk);
@@ -375,31 +401,49 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
 // Activations: dy and x both bf16, or both fp32 with x marked as "consumed as bf16".
 bool bwd_resident_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C, int T) {
     const bool io = (x_dtype == kBF16 && y_dtype == kBF16) || (x_dtype == kF32AsBF16 && y_dtype == kF32);
-    return io && phi_dtype == kBF16 && n <= 8 && C % 8 == 0 && C <= 128 * kResTileWaves * kResMaxItems && T <= 32;
+    return io && phi_dtype == kBF16 && n <= 8 && C <= kResMaxC && (C % 8 == 0 || (C > 8 && x_dtype == kBF16)) && T <= 32;
 }
 
-template <int NP, int WMODE, bool F32, bool STATIC, int TW>
+template <int NP, int WMODE, bool F32, bool STATIC, int TW, bool RAG = false>
 static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream) {
     using SK = SkSmall<NP>;
     using CB = CoefBwdSmall<NP, false, true, STATIC>;
     const size_t smem = sizeof(float) * ((STATIC ? 0 : SK::scaling_floats(ra.r.T)) + CB::kXch);
-    const int items = (ra.r.C + 128 * TW - 1) / (128 * TW);
+    int items = (ra.r.C + 128 * TW - 1) / (128 * TW);
     const dim3 grid(ra.r.B);
     const int threads = 64 * (TW + (STATIC ? 0 : 1));
-    constexpr int kMaxItems = TW == kResTileWaves ? kResMaxItems : 2;  // wider workgroups are for rows they hold in one or two items
+    // five and ten tile waves are for rows that they hold in one or two items, seven for the longest rows;
+    // ragged rows round the count up (fewer instantiations)
+    constexpr int kMinItems = TW == kResLongWaves ? (RAG ? 5 : 3) : 1;
+    constexpr int kMaxItems = TW == kResTileWaves || TW == kResLongWaves ? kResMaxItems : 2;
+    if (RAG && items == 4) items = 5;
+    if (items < kMinItems) items = kMinItems;
+#define MHC_RES_ITEMS(N)                                                                              \
+    case N:                                                                                           \
+        if constexpr (N >= kMinItems && N <= kMaxItems && !(RAG && N == 4)) {                         \
+            bwd_resident_kernel<NP, WMODE, N, F32, STATIC, TW, RAG><<<grid, threads, smem, stream>>>(ra); \
+            return hipGetLastError();                                                                 \
+        }                                                                                             \
+        return hipErrorInvalidValue
     switch (items) {
-        case 1: bwd_resident_kernel<NP, WMODE, 1, F32, STATIC, TW><<<grid, threads, smem, stream>>>(ra); break;
-        case 2: bwd_resident_kernel<NP, WMODE, 2, F32, STATIC, TW><<<grid, threads, smem, stream>>>(ra); break;
-        case 3: if constexpr (kMaxItems >= 3) { bwd_resident_kernel<NP, WMODE, 3, F32, STATIC, TW><<<grid, threads, smem, stream>>>(ra); break; } return hipErrorInvalidValue;
-        case 4: if constexpr (kMaxItems >= 4) { bwd_resident_kernel<NP, WMODE, 4, F32, STATIC, TW><<<grid, threads, smem, stream>>>(ra); break; } return hipErrorInvalidValue;
-        case 5: if constexpr (kMaxItems >= 5) { bwd_resident_kernel<NP, WMODE, 5, F32, STATIC, TW><<<grid, threads, smem, stream>>>(ra); break; } return hipErrorInvalidValue;
+        MHC_RES_ITEMS(1);
+        MHC_RES_ITEMS(2);
+        MHC_RES_ITEMS(3);
+        MHC_RES_ITEMS(4);
+        MHC_RES_ITEMS(5);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+#undef MHC_RES_ITEMS
 }
 
 template <int NP, int WMODE, bool F32, bool STATIC = false>
 static hipError_t launch_items(const BwdResidentArgs &ra, hipStream_t stream) {
+    if (ra.r.C % 8 != 0) {
+        if constexpr (F32) return hipErrorInvalidValue;  // fp32 storage: whole 8-element chunks only (capi.hip)
+        else if (ra.r.C > 128 * kResTileWaves * kResMaxItems) return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves, true>(ra, stream);
+        else return launch_items_tw<NP, WMODE, F32, STATIC, kResTileWaves, true>(ra, stream);
+    }
+    if (ra.r.C > 128 * kResTileWaves * kResMaxItems) return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves>(ra, stream);
     // Eight streams, rows of at most 1280 channels: ten tile waves hold the row in one item each
     // instead of four in three - the Gram and mixing products of an 8 x 8 sample are most of such a
     // workgroup's life, and one wave per SIMD has nobody to overlap them with.  Backward at B=256,

@@ -91,7 +91,7 @@ bool bwd_resident_preferred(int B, int n, int C) {
 // a cast pass over x on top of the tiled path (through the module, fp32 tensors, forward + backward:
 // B=1280 C=2560 n=4 186 -> 184 us, B=2560 C=1280 184 -> 176, B=1024 C=1280 111 -> 100).
 bool f32_as_bf16_accepted(int B, int n, int C, int iters) {
-    return n <= 8 && layer_fwd_fused_supported(n, C, kF32) &&
+    return n <= 8 && C % 8 == 0 && layer_fwd_fused_supported(n, C, kF32) &&
            bwd_resident_supported(kF32AsBF16, kF32, kBF16, n, C, iters) && proj_bwd_addx_supported(n);
 }
 
@@ -618,13 +618,15 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
     const int D = n * n + 2 * n, DP = padded_D(n);
     const bool mfma = proj_bwd_mfma_supported(x_dtype == kF32AsBF16 ? kBF16 : x_dtype, phi_dtype, C);
     BwdCoefOut out{ws.dt, ws.dP, ws.cx, ws.s1, nullptr, mfma ? ws.dPb : nullptr, ws.dPT, ws.BP};
-    if (mfma && bwd_resident_supported(x_dtype, y_dtype, phi_dtype, n, C, iters) && proj_bwd_addx_supported(n) &&
-        (bwd_resident_preferred(B, n, C) || x_dtype == kF32AsBF16)) {
+    // (rows that are no multiple of 8 elements: these two launches are the only matrix-core ones that take them)
+    if (bwd_resident_supported(x_dtype, y_dtype, phi_dtype, n, C, iters) && proj_bwd_addx_supported(n) &&
+        (bwd_resident_preferred(B, n, C) || x_dtype == kF32AsBF16 || C % 8 != 0)) {
         // two launches: (1) one workgroup per sample keeps the sample's rows of dy and x in registers for
         // the channel sums, the coefficient backward and the mixing part of dx; (2) a column-slab
         // kernel over all samples adds dP phi - cx x, finishes dphi without batch-split partial sums
         // and sums dw, dbias and dalpha in a few extra workgroups
         BwdCoefOut out2 = out;
+        out2.dPb = ws.dPb;
         out2.dP = nullptr;  // the second launch takes dP as matrix-core operands only
         MHC_LAUNCH(launch_bwd_resident(dy, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, q, P, r, alpha, bias + 2 * n,
                                        sk_state, out2, dx, df, ws.u, B, n, C, iters, eps, st));

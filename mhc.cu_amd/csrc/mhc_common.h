@@ -133,6 +133,81 @@ __device__ __forceinline__ void store_vec(T *__restrict__ p, const float (&v)[V]
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Rows whose length is no multiple of a 16-byte access ("ragged": C = 1230, 277 ...).  A row then starts at
+// any element, and the same 16-byte accesses are used with the element's alignment (global memory takes
+// them; only the touched cache lines count: B=333 n=3 C=1230, the scalar kernels took 124 us, these 31).
+// Only the last chunk of a row needs care:
+//   loads   read the last whole chunk of the row (clamped address) and drop() the elements that belong to
+//           the chunk before, which leaves zeros behind the row's end;
+//   stores  write its elements one by one.
+// A row must hold at least one whole chunk.
+// ---------------------------------------------------------------------------------------------
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
+__device__ __forceinline__ uint4 ldg16_any(const void *p) {
+    const u32x4_any_t t = *static_cast<const u32x4_any_t *>(p);
+    return make_uint4(t[0], t[1], t[2], t[3]);
+}
+template <bool ANY> __device__ __forceinline__ uint4 ldg16(const void *p) {
+    if constexpr (ANY) return ldg16_any(p);
+    else return *static_cast<const uint4 *>(p);
+}
+template <bool STREAM> __device__ __forceinline__ void st16_any(void *p, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    const u32x4_any_t v = {a, b, c, d};
+    if constexpr (STREAM) __builtin_nontemporal_store(v, static_cast<u32x4_any_t *>(p));
+    else *static_cast<u32x4_any_t *>(p) = v;
+}
+// Drops the first s elements (of ESIZE bytes) of the N words and fills up with zeros.
+template <int ESIZE, int N> __device__ __forceinline__ void drop_elems(uint32_t (&w)[N], int s) {
+    if constexpr (ESIZE == 2) {
+        const bool odd = s & 1;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t nx = i + 1 < N ? w[i + 1] : 0u;
+            w[i] = odd ? (w[i] >> 16) | (nx << 16) : w[i];
+        }
+        s >>= 1;
+    }
+#pragma unroll
+    for (int st = 1; st < N; st *= 2) {
+        const bool on = s & st;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t nx = i + st < N ? w[i + st] : 0u;
+            w[i] = on ? nx : w[i];
+        }
+    }
+}
+__device__ __forceinline__ uint4 drop8(uint4 v, int s) {  // the first s of eight bf16 values, zeros moved in behind
+    uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    drop_elems<2>(w, s);
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+// Stores `cnt` of the V values (all of them as whole vectors when cnt >= V) at any element alignment.
+template <typename T, int V, bool STREAM = false>
+__device__ __forceinline__ void store_vec_any(T *__restrict__ p, const float (&v)[V], int cnt) {
+    if (cnt >= V) {
+        if constexpr (std::is_same<T, float>::value) {
+            static_assert(V % 4 == 0, "whole 16-byte pieces");
+#pragma unroll
+            for (int i = 0; i < V / 4; i++)
+                st16_any<STREAM>(p + 4 * i, __float_as_uint(v[4 * i]), __float_as_uint(v[4 * i + 1]),
+                                 __float_as_uint(v[4 * i + 2]), __float_as_uint(v[4 * i + 3]));
+        } else {
+            static_assert(V % 8 == 0, "whole 16-byte pieces");
+#pragma unroll
+            for (int i = 0; i < V / 8; i++)
+                st16_any<STREAM>(p + 8 * i, pack_bf16x2(v[8 * i], v[8 * i + 1]), pack_bf16x2(v[8 * i + 2], v[8 * i + 3]),
+                                 pack_bf16x2(v[8 * i + 4], v[8 * i + 5]), pack_bf16x2(v[8 * i + 6], v[8 * i + 7]));
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < V; i++)
+            if (i < cnt) p[i] = from_f32<T>(v[i]);
+    }
+}
+
 // 16-byte load with the streaming (non-temporal) hint.
 __device__ __forceinline__ uint4 ldg16_stream(const uint4 *p) {
     const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p));
@@ -142,7 +217,7 @@ __device__ __forceinline__ uint4 ldg16_stream(const uint4 *p) {
 // V consecutive elements kept exactly as loaded.  No conversion instruction sits behind the load,
 // so a batch of loads stays in flight across whatever code follows (another basic block
 // included); get() widens to fp32 at the point of use.  The pointer must be dereferenceable and
-// aligned to min(V * sizeof(T), 16) bytes: callers clamp out-of-range indices to a valid element
+// aligned to min(V * sizeof(T), 16) bytes (load_any: to the element): callers clamp out-of-range indices to a valid element
 // instead of branching around the load.
 template <typename T, int V> struct RawVec {
     static constexpr int kBytes = V * (int)sizeof(T);
@@ -178,6 +253,15 @@ template <typename T, int V> struct RawVec {
             w[4 * i] = t.x; w[4 * i + 1] = t.y; w[4 * i + 2] = t.z; w[4 * i + 3] = t.w;
         }
     }
+    __device__ __forceinline__ void load_any(const T *__restrict__ p) {
+        static_assert(kBytes % 16 == 0, "whole 16-byte pieces");
+#pragma unroll
+        for (int i = 0; i < kBytes / 16; i++) {
+            const uint4 t = ldg16_any(p + i * (16 / (int)sizeof(T)));
+            w[4 * i] = t.x; w[4 * i + 1] = t.y; w[4 * i + 2] = t.z; w[4 * i + 3] = t.w;
+        }
+    }
+    __device__ __forceinline__ void drop(int s) { drop_elems<(int)sizeof(T)>(w, s); }
     __device__ __forceinline__ void get(float (&v)[V]) const {
         if constexpr (std::is_same<T, float>::value) {
 #pragma unroll

@@ -157,7 +157,10 @@ __device__ __forceinline__ void get_act(const RawVec<T, V> &r, float (&v)[V]) {
 constexpr int kFwdStaggerMinB = 512;  // two or more workgroups per CU
 
 // RX: fp32 x (and f) consumed as bf16, every value rounded to bf16 as it is unpacked
-template <typename TX, typename TY, int NP, int V, int CPT, bool RX = false>
+// RAG: rows of any length (C % V != 0): the last chunk of a row is loaded V elements wide from C - V on and
+// shifted down behind the barrier.  A template argument: as a run-time switch the clamps and compares cost the
+// whole rows 4 % (B=3001 n=4 C=2560: 27.4 -> 28.5 us).
+template <typename TX, typename TY, int NP, int V, int CPT, bool RX = false, bool RAG = false>
 __global__ __launch_bounds__(256, (CPT == 2 && NP == 4 && !std::is_same<TX, float>::value) ? 4 : kMfmaMinWaves)
 void layer_fwd_small_kernel(LayerFwdArgs a) {
     using SK = SkSmall<NP>;
@@ -169,7 +172,8 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
     TY *__restrict__ yb = static_cast<TY *>(a.y) + (size_t)b * n * C;
     const bool inject = a.f_inject != nullptr;
     const bool dyn = a.Ppart != nullptr;
-    const int nch = C / V;
+    const int nch = RAG ? (C + V - 1) / V : C / V;
+    auto chunk_at = [&](int ch) { return RAG ? (size_t)min(ch * V, C - V) : (size_t)ch * V; };  // where chunk ch is loaded from
     MHC_PHASE(kPhaseFwdFused, b, 0);
 
     // ---- 1. loads.  Wave 0 first asks for the small coefficient inputs (they return ahead of
@@ -221,15 +225,21 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
 #pragma unroll
         for (int k = 0; k < CPT; k++) {
             const int ch = tid + k * nt;
-            const TX *xc = xb + (size_t)(ch < nch ? ch : 0) * V;
+            const TX *xc = xb + chunk_at(ch < nch ? ch : 0);
 #pragma unroll
-            for (int i = 0; i < NP; i++) xr[k][i].load(xc + (size_t)(i < n ? i : 0) * C);
+            for (int i = 0; i < NP; i++) {
+                const TX *p = xc + (size_t)(i < n ? i : 0) * C;
+                if constexpr (RAG) xr[k][i].load_any(p);
+                else xr[k][i].load(p);
+            }
         }
         if (inject) {
 #pragma unroll
             for (int k = 0; k < CPT; k++) {
                 const int ch = tid + k * nt;
-                fr[k].load(static_cast<const TX *>(a.f_inject) + (size_t)b * C + (size_t)(ch < nch ? ch : 0) * V);
+                const TX *p = static_cast<const TX *>(a.f_inject) + (size_t)b * C + chunk_at(ch < nch ? ch : 0);
+                if constexpr (RAG) fr[k].load_any(p);
+                else fr[k].load(p);
             }
         }
     };
@@ -331,6 +341,16 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
     if (late) issue_tile();
     __syncthreads();
     MHC_PHASE(kPhaseFwdFused, b, 4);
+    if constexpr (RAG) {
+#pragma unroll
+        for (int k = 0; k < CPT; k++) {
+            const int ch = tid + k * nt;
+            const int s = ch == nch - 1 ? nch * V - C : 0;
+#pragma unroll
+            for (int i = 0; i < NP; i++) xr[k][i].drop(s);
+            if (inject) fr[k].drop(s);
+        }
+    }
     float hpre[NP], hpost[NP], Mr[NP][NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) {
@@ -423,7 +443,11 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
             if (inject) {
                 get_act<RX>(fr[k], f);
             } else {
-                if (a.w_bf16) load_vec<bf16_t, V>(static_cast<const bf16_t *>(a.w) + c, f);
+                if (RAG && c + V > C) {  // the row's last chunk: behind its end any finite value will do
+#pragma unroll
+                    for (int v = 0; v < V; v++) f[v] = load_w(a.w, a.w_bf16, min(c + v, C - 1));
+                }
+                else if (a.w_bf16) load_vec<bf16_t, V>(static_cast<const bf16_t *>(a.w) + c, f);
                 else load_vec<float, V>(static_cast<const float *>(a.w) + c, f);
             }
             uint32_t yw[NP][2];  // packed first half (bf16 output), stored with the second
@@ -468,14 +492,25 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
                         if (h == 0) {
                             yw[i][0] = pack_bf16x2(o0, o1); yw[i][1] = pack_bf16x2(o2, o3);
                         } else if (i < n && ch < nch) {
-                            st16<true>(yb + (size_t)i * C + c, yw[i][0], yw[i][1], pack_bf16x2(o0, o1), pack_bf16x2(o2, o3));
+                            TY *yp = yb + (size_t)i * C + c;
+                            const uint32_t w4[4] = {yw[i][0], yw[i][1], pack_bf16x2(o0, o1), pack_bf16x2(o2, o3)};
+                            if constexpr (!RAG) {
+                                st16<true>(yp, w4[0], w4[1], w4[2], w4[3]);
+                            } else if (c + V <= C) {
+                                st16_any<true>(yp, w4[0], w4[1], w4[2], w4[3]);
+                            } else {
+#pragma unroll
+                                for (int v = 0; v < V; v++)
+                                    if (c + v < C) yp[v] = (bf16_t)(v & 1 ? w4[v / 2] >> 16 : w4[v / 2] & 0xffffu);
+                            }
                         }
                     } else {
                         if (h == 0) {
                             yf[i][0] = o0; yf[i][1] = o1; yf[i][2] = o2; yf[i][3] = o3;
                         } else if (i < n && ch < nch) {
                             const float out[V] = {yf[i][0], yf[i][1], yf[i][2], yf[i][3], o0, o1, o2, o3};
-                            store_vec<TY, V, true>(yb + (size_t)i * C + c, out);
+                            if constexpr (RAG) store_vec_any<TY, V, true>(yb + (size_t)i * C + c, out, C - c);
+                            else store_vec<TY, V, true>(yb + (size_t)i * C + c, out);
                         }
                     }
                 }
@@ -483,7 +518,7 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
         }
     } else {
         // ---- 3. aggregate + RMS ------------------------------------------------------------------
-        // (VALU path: fp32 x, n > 4, or rows not a multiple of 8.)  The tile stays in registers as raw
+        // (VALU path: fp32 x.)  The tile stays in registers as raw
         // words; LEAN (two chunks per thread) widens a stream at the point of use instead of holding
         // the fp32 copy of the whole tile, which keeps the register count down; the extra
         // conversions are cheaper than a second round of the grid.
@@ -548,10 +583,10 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
                             for (int v = 0; v < V; v++) f[v] += hpre[i] * t[v];
                         }
 #pragma unroll
-                        for (int v = 0; v < V; v++) f[v] = f[v] * qinv * load_w(a.w, a.w_bf16, c + v);
+                        for (int v = 0; v < V; v++) f[v] = f[v] * qinv * load_w(a.w, a.w_bf16, RAG ? min(c + v, C - 1) : c + v);
                     } else {
 #pragma unroll
-                        for (int v = 0; v < V; v++) f[v] = av[k][v] * qinv * load_w(a.w, a.w_bf16, c + v);
+                        for (int v = 0; v < V; v++) f[v] = av[k][v] * qinv * load_w(a.w, a.w_bf16, RAG ? min(c + v, C - 1) : c + v);
                     }
                 }
 #pragma unroll
@@ -568,7 +603,8 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
 #pragma unroll
                             for (int v = 0; v < V; v++) out[v] += mij * (LEAN ? t[v] : xv[LEAN ? 0 : k][j][v]);
                         }
-                        store_vec<TY, V, true>(yb + (size_t)i * C + c, out);
+                        if constexpr (RAG) store_vec_any<TY, V, true>(yb + (size_t)i * C + c, out, C - c);
+                            else store_vec<TY, V, true>(yb + (size_t)i * C + c, out);
                     }
                 }
             }
@@ -579,19 +615,21 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
 
 // Largest CPT instantiated: tiles with more than 4 * 256 vector chunks per stream take the
 // two-kernel path (coefficient kernel + streaming mix kernel).
-template <typename TX, typename TY, int NP, bool RX = false>
+template <typename TX, typename TY, int NP, bool RX = false, bool RAG = false>
 static bool launch_fused_small(const LayerFwdArgs &a, hipStream_t stream, hipError_t *err) {
     constexpr int V = 16 / (int)sizeof(TX);
-    if (a.C % V != 0) return false;
-    const int nch = a.C / V;
+    if constexpr (!RAG) {
+        if (a.C % V != 0) return a.C > V && launch_fused_small<TX, TY, NP, RX, true>(a, stream, err);
+    }
+    const int nch = (a.C + V - 1) / V;
     const int cpt = (nch + 255) / 256;
     // as few whole waves as hold the chunks: a thread without a chunk of its own still runs the loads
     // and the arithmetic on an aliased one (320 chunks on 2 x 256 slots would waste 37 % of both)
     const int per = cpt == 3 ? 4 : cpt;  // chunks per thread of the instantiation that runs
     const int nt = NP == 8 ? 256 : round_up((nch + per - 1) / per, kWave);
-    if (cpt == 1) layer_fwd_small_kernel<TX, TY, NP, V, 1, RX><<<a.B, nt, 0, stream>>>(a);
-    else if (cpt == 2) layer_fwd_small_kernel<TX, TY, NP, V, 2, RX><<<a.B, nt, 0, stream>>>(a);
-    else if (cpt <= 4 && NP == 4) layer_fwd_small_kernel<TX, TY, 4, V, 4, RX><<<a.B, nt, 0, stream>>>(a);
+    if (cpt == 1) layer_fwd_small_kernel<TX, TY, NP, V, 1, RX, RAG><<<a.B, nt, 0, stream>>>(a);
+    else if (cpt == 2) layer_fwd_small_kernel<TX, TY, NP, V, 2, RX, RAG><<<a.B, nt, 0, stream>>>(a);
+    else if (cpt <= 4 && NP == 4) layer_fwd_small_kernel<TX, TY, 4, V, 4, RX, RAG><<<a.B, nt, 0, stream>>>(a);
     else return false;
     *err = hipGetLastError();
     return true;
@@ -600,8 +638,8 @@ static bool launch_fused_small(const LayerFwdArgs &a, hipStream_t stream, hipErr
 bool layer_fwd_fused_supported(int n, int C, int x_dtype) {
     if (n > 8) return false;
     const int V = x_dtype == kBF16 ? 8 : 4;
-    if (C % V != 0) return false;
-    const int cpt = (C / V + 255) / 256;
+    if (C < V) return false;
+    const int cpt = ((C + V - 1) / V + 255) / 256;
     return cpt <= 2 || (cpt <= 4 && n <= 4);
 }
 

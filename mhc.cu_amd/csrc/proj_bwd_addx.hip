@@ -55,7 +55,8 @@ constexpr int kAxLDR = 36;         // LDS pitch of the dphi tiles in the final c
 // F32: x and dx are stored as fp32 (x is rounded to bf16 for the products and for the -cx x term, as in
 // the bf16 storage case; dxp is read and dx written as fp32).
 // NW: waves per workgroup (a block is NW * SPW samples).
-template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4>
+// RAG: rows of any length (nC % 8 != 0): the last chunk of a row is loaded from nC - 8 on and shifted down.
+template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel(ProjAddxArgs a) {
     constexpr int NT_ = 64 * NW;  // threads
     using TS = typename std::conditional<F32, float, bf16_t>::type;
@@ -91,7 +92,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
     // the chunks of dxp this thread completes: sample SPW wave + lane / 4 + 16 t, chunk lane % 4 ------
     const int ech = lane & 3, erow = SPW * wave + (lane >> 2);
     const int kc = k0 + ech * 8;
-    const bool kok = kc < nC;  // nC % 8 == 0: a chunk is inside or outside
+    const bool kok = kc < nC;
+    // a thread owns the same column chunk in all of its loads (they are multiples of four chunks apart), so the
+    // shift of a ragged row is one value per thread
+    const int kl = k0 + (tid & 3) * 8;  // the chunk of x and phi
+    const int kls = RAG && kl < nC && kl + 8 > nC ? kl + 8 - nC : 0, kcs = RAG && kok && kc + 8 > nC ? kc + 8 - nC : 0;
     // dxp of the next block is requested a block ahead like x, except where that costs the registers that
     // keep two workgroups on a CU (fp32 storage with a wide projection): there it is requested at the top
     // of its own block and arrives under the matrix-core phase
@@ -101,11 +106,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
     const TS *xg = static_cast<const TS *>(a.x);
     TS *dxg = static_cast<TS *>(a.dx);
     auto load_chunk = [&](const TS *p, uint32_t (&q)[AW], bool ok) {
-        const uint4 v = load16_masked(reinterpret_cast<const uint4 *>(p), ok);
-        q[0] = v.x; q[1] = v.y; q[2] = v.z; q[3] = v.w;
+        const uint4 v = ldg16<RAG>(p);
+        q[0] = ok ? v.x : 0u; q[1] = ok ? v.y : 0u; q[2] = ok ? v.z : 0u; q[3] = ok ? v.w : 0u;
         if constexpr (F32) {
-            const uint4 v2 = load16_masked(reinterpret_cast<const uint4 *>(p) + 1, ok);
-            q[4] = v2.x; q[5] = v2.y; q[6] = v2.z; q[7] = v2.w;
+            const uint4 v2 = ldg16<RAG>(p + 4);
+            q[4] = ok ? v2.x : 0u; q[5] = ok ? v2.y : 0u; q[6] = ok ? v2.z : 0u; q[7] = ok ? v2.w : 0u;
         }
     };
     auto load_block = [&](int sb, auto slot) {
@@ -113,16 +118,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 #pragma unroll
         for (int u = 0; u < KS; u++) {
             const int ch = tid + u * NT_;
-            const int b = sb + (ch >> 2), k = k0 + (ch & 3) * 8;
-            const bool ok = b < B && k < nC;
-            load_chunk(xg + (ok ? (size_t)b * nC + k : 0), xr[S][u], ok);
+            const int b = sb + (ch >> 2);
+            const bool ok = b < B && kl < nC;
+            load_chunk(xg + (ok ? (size_t)b * nC + kl - kls : 0), xr[S][u], ok);
         }
         if constexpr (PS == 2) {
 #pragma unroll
             for (int t = 0; t < KS; t++) {
                 const int b = sb + erow + 16 * t;
                 const bool ok = b < B && kok;
-                load_chunk(dxg + (ok ? (size_t)b * nC + kc : 0), pr[S][t], ok);
+                load_chunk(dxg + (ok ? (size_t)b * nC + kc - kcs : 0), pr[S][t], ok);
                 cxr[S][t] = a.cx[b < B ? b : 0];
             }
         }
@@ -132,7 +137,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         for (int t = 0; t < KS; t++) {
             const int b = sb + erow + 16 * t;
             const bool ok = b < B && kok;
-            load_chunk(dxg + (ok ? (size_t)b * nC + kc : 0), pr[0][t], ok);
+            load_chunk(dxg + (ok ? (size_t)b * nC + kc - kcs : 0), pr[0][t], ok);
             cxr[0][t] = a.cx[b < B ? b : 0];
         }
     };
@@ -173,9 +178,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 #pragma unroll
     for (int u = 0; u < (PCH + NT_ - 1) / NT_; u++) {
         const int ch = tid + u * NT_;
-        const int d = ch >> 2, k = k0 + (ch & 3) * 8;
-        const bool ok = ch < PCH && d < D && k < nC;
-        phir[u] = load16_masked(reinterpret_cast<const uint4 *>(a.phi + (ok ? (size_t)d * nC + k : 0)), ok);
+        const int d = ch >> 2;
+        const bool ok = ch < PCH && d < D && kl < nC;
+        const uint4 v = ldg16<RAG>(a.phi + (ok ? (size_t)d * nC + kl - kls : 0));
+        phir[u] = make_uint4(ok ? v.x : 0u, ok ? v.y : 0u, ok ? v.z : 0u, ok ? v.w : 0u);
     }
     load_block(0, Slot0{});
     load_ops(0, ops[0]);
@@ -186,6 +192,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 #pragma unroll
     for (int u = 0; u < (PCH + NT_ - 1) / NT_; u++) {
         const int ch = tid + u * NT_;
+        if constexpr (RAG) phir[u] = drop8(phir[u], kls);
         if (ch < PCH) *reinterpret_cast<uint4 *>(phi_s + (size_t)(ch >> 2) * kAxLD + (ch & 3) * 8) = phir[u];
     }
 
@@ -210,6 +217,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         for (int u = 0; u < KS; u++) {
             const int ch = tid + u * NT_;
             uint4 xb;
+            if constexpr (RAG) drop_elems<(int)sizeof(TS)>(xr[S][u], kls);
             if constexpr (F32)
                 xb = make_uint4(pack_bf16x2(__uint_as_float(xr[S][u][0]), __uint_as_float(xr[S][u][1])),
                                 pack_bf16x2(__uint_as_float(xr[S][u][2]), __uint_as_float(xr[S][u][3])),
@@ -260,6 +268,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
             const float4 o1 = *reinterpret_cast<const float4 *>(o_s + (size_t)r * kAxLDO + ech * 8 + 4);
             const uint4 xv = *reinterpret_cast<const uint4 *>(x_s + (size_t)r * kAxLD + ech * 8);
             const float cxv = cxr[P][t];
+            if constexpr (RAG) drop_elems<(int)sizeof(TS)>(pr[P][t], kcs);
             const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
             const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
             float res[8];
@@ -270,7 +279,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
                 res[2 * p] = plo + ov[2 * p] - cxv * bf16lo_to_f32(xw[p]);
                 res[2 * p + 1] = phi_ + ov[2 * p + 1] - cxv * bf16hi_to_f32(xw[p]);
             }
-            if (b < B && kok) store_vec<TS, 8, true>(dxg + (size_t)b * nC + kc, res);
+            if (b < B && kok) {
+                if constexpr (RAG) store_vec_any<TS, 8, true>(dxg + (size_t)b * nC + kc, res, nC - kc);
+                else store_vec<TS, 8, true>(dxg + (size_t)b * nC + kc, res);
+            }
         }
         if (sb + 2 * SBR < B) {
             load_block(sb + 2 * SBR, slot);
@@ -299,25 +311,34 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
             const float4 v = *reinterpret_cast<const float4 *>(red_s + ((size_t)w * NTD * 32 + d) * kAxLDR + c);
             s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
         }
-        // nC % 8 == 0 and k0 % 32 == 0: a quad of columns is inside or outside
-        if (d < D && k0 + c < nC) *reinterpret_cast<float4 *>(a.dphi + (size_t)d * nC + k0 + c) = s;
+        if (d < D && k0 + c < nC) {
+            if constexpr (RAG) {
+                const float out[4] = {s.x, s.y, s.z, s.w};
+                store_vec_any<float, 4>(a.dphi + (size_t)d * nC + k0 + c, out, nC - (k0 + c));
+            } else {  // k0 % 32 == 0: a quad of columns is inside or outside
+                *reinterpret_cast<float4 *>(a.dphi + (size_t)d * nC + k0 + c) = s;
+            }
+        }
     }
     MHC_PHASE_ADD(kPhaseColSlab, pwg, 4, pclk);
 }
 
 bool proj_bwd_addx_supported(int n) { return padded_D(n) / 32 <= 3; }
 
-template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4>
+template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false>
 static hipError_t launch_addx(const ProjAddxArgs &a, hipStream_t stream) {
+    if constexpr (!F32 && !RAG) {
+        if (a.nC % 8 != 0) return launch_addx<NTD, SPW, PFOP, F32, NW, true>(a, stream);
+    }
     constexpr int SBR = NW * SPW;
     const size_t tiles = sizeof(bf16_t) * (size_t)kAxLD * (32 * NTD + SBR) + sizeof(float) * SBR * kAxLDO;
     const size_t red = sizeof(float) * NW * NTD * 32 * kAxLDR;  // the final cross-wave sum reuses the tiles' memory
     const size_t smem = tiles > red ? tiles : red;
-    hipError_t e = allow_dynamic_lds(&proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW>, smem);
+    hipError_t e = allow_dynamic_lds(&proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG>, smem);
     if (e != hipSuccess) return e;
     const int slabs = (a.nC + kAxKW - 1) / kAxKW;
     dim3 grid(round_up(slabs, 16), 1 + (a.tail_row >= 0 ? 1 : 0));
-    proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW><<<grid, 64 * NW, smem, stream>>>(a);
+    proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG><<<grid, 64 * NW, smem, stream>>>(a);
     return hipGetLastError();
 }
 

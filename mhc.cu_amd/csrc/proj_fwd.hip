@@ -6,8 +6,8 @@
 // cuBLASLt projection GEMM (src/python/bindings.cu:34-81, :436-443) with one pass over x.
 //
 // Three kernels:
-//   proj_fwd_mfma_kernel    n <= 10; x and phi both bf16 (C % 8 == 0): v_mfma_f32_32x32x16_bf16 tiles
-//                           (32 samples x 32 projection rows), or both fp32 (n <= 8, nC % 4 == 0):
+//   proj_fwd_mfma_kernel    n <= 10; x and phi both bf16 (any C for n <= 8): v_mfma_f32_32x32x16_bf16 tiles
+//                           (32 samples x 32 projection rows), or both fp32 (n <= 8):
 //                           v_mfma_f32_32x32x2_f32, IEEE products; operands fetched row-contiguously
 //                           through a wave-private LDS tile.
 //   proj_fwd_wide_kernel    bf16, wider phi.
@@ -24,8 +24,9 @@ namespace mhc {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 
-static inline bool use_mfma(int x_dtype, int phi_dtype, int C) {
-    return (x_dtype == kBF16 || x_dtype == kF32AsBF16) && phi_dtype == kBF16 && C % 8 == 0;
+// n <= 8 (the narrow kernel): rows of any length from one 64-element chunk on; beyond, whole 16-byte pieces
+static inline bool use_mfma(int x_dtype, int phi_dtype, int n, int C) {
+    return (x_dtype == kBF16 || x_dtype == kF32AsBF16) && phi_dtype == kBF16 && (C % 8 == 0 || (n <= 8 && n * C >= 64));
 }
 
 // --------------------------------------------------------------------------------------------
@@ -111,7 +112,8 @@ __device__ __forceinline__ void gather_small(const PhiSrc &g, int tid, int nthr,
 // four elements instead of eight and a chunk 32 instead of 64, everything else (LDS tile, pieces per lane,
 // accumulators) is the same.  With 32 samples per tile and D padded to 32 instead of 128 x 128 tiles the fp32
 // projection of B=2560 n=4 C=1280 went from 58 to 20 us.
-template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false>
+// RAG: rows of any length (nC no multiple of the pieces): the last piece is read from nC - EL on and shifted down.
+template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false, bool RAG = false>
 __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
                                                             const void *__restrict__ phi_,
                                                             float *__restrict__ Ppart,
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
     // rows of phi lie in three matrices: eight registers less, which is one more wave per SIMD
     const char *xbase = reinterpret_cast<const char *>(x + (size_t)st * 32 * nC);
     uint32_t xoff[4], poff[NT][4];
-    const TPS *prow[NT][4];
+    const float *prow[2];
     bool pval[NT][4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -167,8 +169,11 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
         for (int t = 0; t < NT; t++) {
             const int d = dbase + t * 32 + lr + 8 * j;
             pval[t][j] = d < D;
-            if constexpr (PF32) prow[t][j] = phi_src_row(src, pval[t][j] ? d : 0, nC);
-            else poff[t][j] = (uint32_t)(pval[t][j] ? d : 0) * (uint32_t)nC * (uint32_t)sizeof(TPS);
+            // the caller's matrices: 16 rows hold all of pre and post (n <= 8), every later one is a row of res
+            if constexpr (PF32) {
+                if (t == 0 && j < 2) prow[j] = phi_src_row(src, pval[t][j] ? d : 0, nC);
+                else poff[t][j] = (uint32_t)(pval[t][j] ? d - 2 * src.n : 0) * (uint32_t)nC * (uint32_t)sizeof(TPS);
+            } else poff[t][j] = (uint32_t)(pval[t][j] ? d : 0) * (uint32_t)nC * (uint32_t)sizeof(TPS);
         }
     }
     constexpr int XW = EL * sizeof(TXS) / 4;  // words of a lane's piece of x as loaded
@@ -176,16 +181,24 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
     uint32_t xq[4][XW], pq[NT][4][PW];  // scalar words: whole-uint4 array elements can end up in scratch
     auto xat = [&](int j, int k) { return reinterpret_cast<const TXS *>(xbase + (xoff[j] + (uint32_t)k * (uint32_t)sizeof(TXS))); };
     auto pat = [&](int t, int j, int k) {
-        if constexpr (PF32) return prow[t][j] + k;
-        else return reinterpret_cast<const TPS *>(static_cast<const char *>(phi_) + (poff[t][j] + (uint32_t)k * (uint32_t)sizeof(TPS)));
+        if (PF32 && t == 0 && j < 2) return reinterpret_cast<const TPS *>(prow[j < 2 ? j : 0] + k);
+        const char *base = PF32 ? reinterpret_cast<const char *>(src.phi[2]) : static_cast<const char *>(phi_);
+        return reinterpret_cast<const TPS *>(base + (poff[t][j] + (uint32_t)k * (uint32_t)sizeof(TPS)));
     };
-    auto load8 = [&](const auto *p, auto &q, bool ok) {
-        const uint4 v = load16_masked(reinterpret_cast<const uint4 *>(p), ok);
+    auto load8 = [&](const auto *p, auto &q) {
+        const uint4 v = ldg16<RAG>(p);
         q[0] = v.x; q[1] = v.y; q[2] = v.z; q[3] = v.w;
         if constexpr (sizeof(q) == 32) {
-            const uint4 v2 = load16_masked(reinterpret_cast<const uint4 *>(p) + 1, ok);
+            const uint4 v2 = ldg16<RAG>(reinterpret_cast<const char *>(p) + 16);
             q[4] = v2.x; q[5] = v2.y; q[6] = v2.z; q[7] = v2.w;
         }
+    };
+    // the K tail: pieces behind kend are zero
+    auto mask8 = [&](auto &q, bool ok, int s) {
+        constexpr int kW = sizeof(q) / 4;
+        if constexpr (RAG) drop_elems<kW * 4 / EL>(q, s);
+#pragma unroll
+        for (int i = 0; i < kW; i++) q[i] = ok ? q[i] : 0u;
     };
     // Rows beyond B (x) or D (phi) alias row 0: what they produce is finite and is either not stored
     // (samples >= B) or zeroed at the store (projection rows >= D), so only the K tail of the last
@@ -196,19 +209,25 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
         if (k0 + CH <= kend) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                load8(xat(j, k), xq[j], true);
+                load8(xat(j, k), xq[j]);
 #pragma unroll
-                for (int t = 0; t < NT; t++) load8(pat(t, j, k), pq[t][j], true);
+                for (int t = 0; t < NT; t++) load8(pat(t, j, k), pq[t][j]);
             }
             return;
         }
-        const bool kv = k < kend;  // kend and k are multiples of EL
-        const int off = kv ? k : 0;
+        const bool kv = k < kend;  // k is a multiple of EL, and so is kend unless it is a ragged nC
+        const int off = kv ? (RAG ? min(k, nC - EL) : k) : 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            load8(xat(j, off), xq[j], kv);
+            load8(xat(j, off), xq[j]);
 #pragma unroll
-            for (int t = 0; t < NT; t++) load8(pat(t, j, off), pq[t][j], kv);
+            for (int t = 0; t < NT; t++) load8(pat(t, j, off), pq[t][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            mask8(xq[j], kv, k - off);
+#pragma unroll
+            for (int t = 0; t < NT; t++) mask8(pq[t][j], kv, k - off);
         }
     };
     auto as_tile = [&](const auto &q) {
@@ -229,10 +248,20 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
                 const uint4 p = as_tile(pq[t][j]);
                 *reinterpret_cast<uint4 *>(cb + (size_t)(32 + t * 32 + lr + 8 * j) * PITCH + seg * 16) = p;
                 if constexpr (PF32) {
-                    // nC is a multiple of EL: the piece is 16-byte aligned and whole
                     const int k = k0 + seg * EL;
-                    if (st == 0 && pval[t][j] && k < kend)
-                        *reinterpret_cast<uint4 *>(static_cast<TC *>(src.phi_out) + (size_t)(dbase + t * 32 + lr + 8 * j) * nC + k) = p;
+                    if (st == 0 && pval[t][j] && k < kend) {
+                        TC *po = static_cast<TC *>(src.phi_out) + (size_t)(dbase + t * 32 + lr + 8 * j) * nC + k;
+                        if constexpr (!RAG) {
+                            *reinterpret_cast<uint4 *>(po) = p;
+                        } else if (k + EL <= nC) {
+                            st16_any<false>(po, p.x, p.y, p.z, p.w);
+                        } else {  // the last piece of a ragged row
+                            const uint32_t w4[4] = {p.x, p.y, p.z, p.w};
+#pragma unroll
+                            for (int e = 0; e < EL; e++)
+                                if (k + e < nC) po[e] = __builtin_bit_cast(TC, (typename std::conditional<EXACT, uint32_t, uint16_t>::type)(EXACT ? w4[e * 4 / EL] : w4[e / 2] >> (16 * (e & 1))));
+                        }
+                    }
                 }
             }
         }
@@ -558,9 +587,9 @@ static int mfma_nt(int n) {
 // LDS-staged kernel
 static bool use_wide(int n, int C) { return padded_D(n) / 32 > 4 && (n * C) % 64 == 0; }
 
-// fp32 tier, n <= 8: the narrow kernel in fp32 arithmetic (rows in whole 16-byte pieces)
+// fp32 tier, n <= 8: the narrow kernel in fp32 arithmetic
 static bool use_exact(int x_dtype, int phi_dtype, int n, int C) {
-    return n <= 8 && gemm_f32_supported(x_dtype, phi_dtype, n, C);
+    return n <= 8 && x_dtype == kF32 && phi_dtype == kF32 && n * C >= 256;
 }
 
 int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
@@ -568,7 +597,7 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
     // several times over (the K loop is latency-bound per wave), at least 64 K elements per wave.
     const bool exact = use_exact(x_dtype, phi_dtype, n, C);
     if (!exact && gemm_f32_supported(x_dtype, phi_dtype, n, C)) return gemm_f32_proj_ksplit(B, n, C, kMaxKSplit);
-    if (!exact && !use_mfma(x_dtype, phi_dtype, C)) return 1;
+    if (!exact && !use_mfma(x_dtype, phi_dtype, n, C)) return 1;
     const int nC = n * C, DP = padded_D(n);
     if (!exact && use_wide(n, C)) {
         // Workgroups = (64-row groups) x (128-sample tiles) x splits.  The chip has 256 CUs and a workgroup
@@ -641,9 +670,15 @@ static hipError_t launch_generic(const void *x, const void *phi, float *Ppart, f
     return hipGetLastError();
 }
 
-template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false>
+template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false, bool RAG = false>
 static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, float *ssqpart, int KS,
                               int B, int D, int DP, int nC, hipStream_t stream, const PhiSrc &src = PhiSrc{}) {
+    if constexpr (NT <= 3 && !RAG) {
+        if (nC % (EXACT ? 4 : 8) != 0) {
+            if constexpr (XF32) return hipErrorInvalidValue;  // fp32 storage: whole pieces only (capi.hip)
+            else return launch_mfma<NT, XF32, PF32, EXACT, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+        }
+    }
     const int tiles_s = (B + 31) / 32;
     const int groups = (DP / 32 + NT - 1) / NT;
     const int sub = round_up((nC + KS * 4 - 1) / (KS * 4), EXACT ? 32 : 64);  // whole chunks: 128-byte lines
@@ -651,8 +686,8 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
     const size_t smem_chunks = sizeof(bf16_t) * 4 * (1 + NT) * 32 * kNarrowPitch;
     const size_t smem_sum = sizeof(float) * 4 * (NT * 16 + 1) * 64;
     const size_t smem = smem_chunks > smem_sum ? smem_chunks : smem_sum;
-    if (hipError_t e = allow_dynamic_lds(&proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT>, smem); e != hipSuccess) return e;
-    proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT><<<grid, 256, smem, stream>>>(x, phi, Ppart,
+    if (hipError_t e = allow_dynamic_lds(&proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG>, smem); e != hipSuccess) return e;
+    proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG><<<grid, 256, smem, stream>>>(x, phi, Ppart,
                                                                  ssqpart, B, D, DP, nC, tiles_s, KS, sub, src);
     return hipGetLastError();
 }
@@ -669,11 +704,14 @@ bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     if (g.phi_dtype != kF32 || !al16(g.phi[0]) || !al16(g.phi[1]) || !al16(g.phi[2])) return false;
     if (g.out_dtype == kF32) return use_exact(x_dtype, kF32, n, C) && B <= 4096 && tuning_get(kTuneGather) != 1;
-    if (!use_mfma(x_dtype, kBF16, C)) return false;
-    if (const int hook = tuning_get(kTuneGather)) return hook == 2 && (use_wide(n, C) || mfma_nt(n) <= 3);
+    if (!use_mfma(x_dtype, kBF16, n, C)) return false;
+    // the narrow kernel finds the rows of pre and post among its first 16 (n <= 8); beyond, rows that are not
+    // whole 64-element chunks keep the packing launch
+    if (!use_wide(n, C) && n > 8) return false;
+    if (const int hook = tuning_get(kTuneGather)) return hook == 2;
     if (use_wide(n, C)) return B <= 320;
     const int nt = mfma_nt(n);
-    return B <= (nt == 1 ? 4096 : (nt == 2 ? 1024 : 512)) && nt <= 3;
+    return B <= (nt == 1 ? 4096 : (nt == 2 ? 1024 : 512));
 }
 
 hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_dtype, float *Ppart,
@@ -700,6 +738,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
             }
         }
         if (use_wide(n, C)) return launch_wide<1, 2, 4, 2, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+        if (n > 8) return hipErrorInvalidValue;  // see proj_fwd_gathers
         const bool xf32 = x_dtype == kF32AsBF16;
         switch (mfma_nt(n)) {
             case 1: return xf32 ? launch_mfma<1, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src)
@@ -711,7 +750,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
             default: return hipErrorInvalidValue;
         }
     }
-    if (use_mfma(x_dtype, phi_dtype, C)) {
+    if (use_mfma(x_dtype, phi_dtype, n, C)) {
         if (x_dtype == kF32AsBF16) {  // fp32 storage, rounded on load: the narrow kernel only (n <= 8)
             switch (use_wide(n, C) ? 0 : mfma_nt(n)) {
                 case 1: return launch_mfma<1, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
