@@ -414,7 +414,7 @@ static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream)
     const int threads = 64 * (TW + (STATIC ? 0 : 1));
     // five and ten tile waves are for rows that they hold in one or two items, seven for the longest rows;
     // ragged rows round the count up (fewer instantiations)
-    constexpr int kMinItems = TW == kResLongWaves ? (RAG ? 5 : 3) : 1;
+    constexpr int kMinItems = TW == kResLongWaves ? (RAG ? 5 : 2) : 1;
     constexpr int kMaxItems = TW == kResTileWaves || TW == kResLongWaves ? kResMaxItems : 2;
     if (RAG && items == 4) items = 5;
     if (items < kMinItems) items = kMinItems;
@@ -451,6 +451,14 @@ static hipError_t launch_items(const BwdResidentArgs &ra, hipStream_t stream) {
     // 15.9 / 15.0: four stay).
     if constexpr (NP == 8 && !F32 && !STATIC) {
         if (ra.r.C <= 1280) return launch_items_tw<NP, WMODE, F32, STATIC, 10>(ra, stream);
+    }
+    // Longer rows of eight streams: as many tile waves as hold the row in two items (7 up to 1792 channels, 10 up to
+    // 2560).  One workgroup fits a CU at any of these register counts, so its waves are all the overlap there is
+    // (kernel us, four waves -> these: n=8 B=1300 C=1600 70.6 -> 54.4, B=2000 C=2048 106.0 -> 97.5, B=256 C=2560
+    // 16.8 -> 15.8; n=6 B=600 C=2304 38.8 -> 35.1).
+    if constexpr (NP == 8 && !F32 && !STATIC) {
+        if (ra.r.C > 128 * 2 * kResLongWaves) return launch_items_tw<NP, WMODE, F32, STATIC, 10>(ra, stream);
+        return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves>(ra, stream);
     }
     // Four streams: a fifth tile wave where it saves every wave an item (rows of 513..640 and 1025..1280
     // channels: ten 128-channel chunks are 3 + 3 + 2 + 2 on four waves, 2 each on five).  B=320, C=1280,
