@@ -295,9 +295,12 @@ hipError_t launch_bwd_slab_f32(const float *dy, const float *x, const void *w, i
     const size_t smem = sum > tile ? sum : tile;
 #define MHC_SLAB_F32(N)                                                                                    \
     do {                                                                                                   \
-        auto k = f_inject ? &bwd_slab_f32_kernel<N, true> : &bwd_slab_f32_kernel<N, false>;                \
-        if (hipError_t e = allow_dynamic_lds(k, smem); e != hipSuccess) return e;                          \
-        k<<<grid, 256, smem, stream>>>(a);                                                                 \
+        if (hipError_t e = f_inject ? allow_dynamic_lds<&bwd_slab_f32_kernel<N, true>>(smem)               \
+                                    : allow_dynamic_lds<&bwd_slab_f32_kernel<N, false>>(smem);             \
+            e != hipSuccess)                                                                               \
+            return e;                                                                                      \
+        if (f_inject) bwd_slab_f32_kernel<N, true><<<grid, 256, smem, stream>>>(a);                        \
+        else bwd_slab_f32_kernel<N, false><<<grid, 256, smem, stream>>>(a);                                \
     } while (0)
     switch (n) {
         case 1: MHC_SLAB_F32(1); break;

@@ -270,22 +270,22 @@ hipError_t launch_coef_fwd(const float *Ppart, const float *ssqpart, int KS, int
         coef_fwd_small_kernel<8><<<B, 64, 0, stream>>>(a);
     else if (n <= 16) {
         const size_t smem = sizeof(float) * (16 * 16 + 32 + SkWg<16>::lds_floats(T));
-        hipError_t e = precise ? allow_dynamic_lds(&coef_fwd_lds_kernel<16, true>, smem)
-                               : allow_dynamic_lds(&coef_fwd_lds_kernel<16, false>, smem);
+        hipError_t e = precise ? allow_dynamic_lds<&coef_fwd_lds_kernel<16, true>>(smem)
+                               : allow_dynamic_lds<&coef_fwd_lds_kernel<16, false>>(smem);
         if (e != hipSuccess) return e;
         if (agg) {
-            e = allow_dynamic_lds(&coef_fwd_lds_kernel<16, false, true>, smem);
+            e = allow_dynamic_lds<&coef_fwd_lds_kernel<16, false, true>>(smem);
             if (e != hipSuccess) return e;
             coef_fwd_lds_kernel<16, false, true><<<B, 256, smem, stream>>>(a);
         } else if (precise) coef_fwd_lds_kernel<16, true><<<B, 256, smem, stream>>>(a);
         else coef_fwd_lds_kernel<16, false><<<B, 256, smem, stream>>>(a);
     } else {
         const size_t smem = sizeof(float) * (32 * 32 + 64 + SkWg<32>::lds_floats(T));
-        hipError_t e = precise ? allow_dynamic_lds(&coef_fwd_lds_kernel<32, true>, smem)
-                               : allow_dynamic_lds(&coef_fwd_lds_kernel<32, false>, smem);
+        hipError_t e = precise ? allow_dynamic_lds<&coef_fwd_lds_kernel<32, true>>(smem)
+                               : allow_dynamic_lds<&coef_fwd_lds_kernel<32, false>>(smem);
         if (e != hipSuccess) return e;
         if (agg) {
-            e = allow_dynamic_lds(&coef_fwd_lds_kernel<32, false, true>, smem);
+            e = allow_dynamic_lds<&coef_fwd_lds_kernel<32, false, true>>(smem);
             if (e != hipSuccess) return e;
             coef_fwd_lds_kernel<32, false, true><<<B, 256, smem, stream>>>(a);
         } else if (precise) coef_fwd_lds_kernel<32, true><<<B, 256, smem, stream>>>(a);

@@ -269,7 +269,7 @@ hipError_t launch_dphi_f32(const float *dP, const float *x, float *out, int S, i
     const size_t smem = sizeof(float) * 4 * (DP / 32) * cpl * 16 * 64;
 #define MHC_DPHI_F32(NT, CPL)                                                                                          \
     do {                                                                                                               \
-        if (hipError_t e = allow_dynamic_lds(&dphi_f32_kernel<NT, CPL>, smem); e != hipSuccess) return e;              \
+        if (hipError_t e = allow_dynamic_lds<&dphi_f32_kernel<NT, CPL>>(smem); e != hipSuccess) return e;              \
         dphi_f32_kernel<NT, CPL><<<grid, 256, smem, stream>>>(dP, x, out, B, D, DP, nC, per_wave);                     \
     } while (0)
     switch (DP / 32) {

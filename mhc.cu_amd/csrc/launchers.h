@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <atomic>
+
 #include "batch_sums.h"
 
 namespace mhc {
@@ -19,11 +21,21 @@ inline size_t dtype_size(int dt) { return dt == kBF16 ? 2 : 4; }
 // denominators of the backward sweep live in LDS (160 KB per CU).
 inline int max_layer_sinkhorn_iters(int) { return 256; }
 
-// Dynamic LDS above 64 KB has to be enabled per kernel before the launch.
-template <typename K> inline hipError_t allow_dynamic_lds(K kernel, size_t bytes) {
+// Dynamic LDS above 64 KB has to be enabled per kernel and device before the launch: asked for once, not on every
+// call (the attribute only ever grows; two threads that ask at the same time set the same or the larger value).
+template <auto Kernel> inline hipError_t allow_dynamic_lds(size_t bytes) {
     if (bytes <= 64 * 1024) return hipSuccess;
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    constexpr int kDevices = 64;
+    static std::atomic<int> allowed[kDevices];
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+    const bool known = dev >= 0 && dev < kDevices;
+    int have = known ? allowed[dev].load(std::memory_order_relaxed) : 0;
+    if (have >= (int)bytes) return hipSuccess;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess && known)
+        while (have < (int)bytes && !allowed[dev].compare_exchange_weak(have, (int)bytes, std::memory_order_relaxed)) {}
+    return e;
 }
 
 // Projection row count padded to whole 32-wide MFMA tiles.

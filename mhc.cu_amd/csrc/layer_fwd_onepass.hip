@@ -482,7 +482,7 @@ hipError_t launch_layer_fwd_onepass(const void *x, const void *w, int w_dtype, c
     hipError_t e = hipSuccess;
 #define MHC_ONEPASS(TY, GH)                                                                  \
     do {                                                                                     \
-        e = allow_dynamic_lds(layer_fwd_onepass_kernel<TY, GH>, smem);                       \
+        e = allow_dynamic_lds<&layer_fwd_onepass_kernel<TY, GH>>(smem);                      \
         if (e != hipSuccess) return e;                                                       \
         layer_fwd_onepass_kernel<TY, GH><<<grid, NW * 64, smem, stream>>>(a);                \
     } while (0)

@@ -974,7 +974,7 @@ static hipError_t launch_gram_small(BwdReduceArgs a, hipStream_t stream) {
     hipError_t e = launch_gram_small_kernel<NP, false>(a, 0, stream);
     if (e != hipSuccess) return e;
     const size_t smem = sizeof(float) * (SK::scaling_floats(a.T) + SK::kPerWave * CB::kXch);
-    e = allow_dynamic_lds(&coef_bwd_small_kernel<NP, false, true>, smem);
+    e = allow_dynamic_lds<&coef_bwd_small_kernel<NP, false, true>>(smem);
     if (e != hipSuccess) return e;
     coef_bwd_small_kernel<NP, false, true><<<(a.B + SK::kPerWave - 1) / SK::kPerWave, 64, smem, stream>>>(a);
     return hipGetLastError();
@@ -1009,7 +1009,7 @@ static hipError_t launch_small(const BwdReduceArgs &a, hipStream_t stream) {
     constexpr int K = NP * NP + 3 * NP + 1;
     // the Sinkhorn area is only needed when the coefficient backward runs in the same launch
     const size_t smem = sizeof(float) * (K * 16 + K + (a.raw ? 0 : SkSmall<NP>::scaling_floats(a.T)));
-    hipError_t e = allow_dynamic_lds(&mix_bwd_reduce_small_kernel<TG, TX, NP, V>, smem);
+    hipError_t e = allow_dynamic_lds<&mix_bwd_reduce_small_kernel<TG, TX, NP, V>>(smem);
     if (e != hipSuccess) return e;
     mix_bwd_reduce_small_kernel<TG, TX, NP, V><<<dim3(a.B, a.parts), nt, smem, stream>>>(a);
     e = hipGetLastError();
@@ -1017,7 +1017,7 @@ static hipError_t launch_small(const BwdReduceArgs &a, hipStream_t stream) {
     // fp32 activations: the parity tier, IEEE divisions in the Sinkhorn chain
     constexpr bool kPrecise = std::is_same<TX, float>::value;
     const size_t smem2 = sizeof(float) * SkSmall<NP>::scaling_floats(a.T);
-    e = allow_dynamic_lds(&coef_bwd_small_kernel<NP, kPrecise>, smem2);
+    e = allow_dynamic_lds<&coef_bwd_small_kernel<NP, kPrecise>>(smem2);
     if (e != hipSuccess) return e;
     coef_bwd_small_kernel<NP, kPrecise><<<(a.B + SkSmall<NP>::kPerWave - 1) / SkSmall<NP>::kPerWave, 64, smem2, stream>>>(a);
     return hipGetLastError();
@@ -1045,11 +1045,7 @@ static hipError_t launch_large(const BwdReduceArgs &a, hipStream_t stream, const
         const size_t sk = sizeof(float) * (a.n <= 16 ? SkWg<16>::lds_floats(a.T) : SkWg<32>::lds_floats(a.T));
         if (smem1 < sk) smem1 = sk;
     }
-    if (smem1 > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gram_large_kernel<TG, TX>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem1);
-        if (e != hipSuccess) return e;
-    }
+    if (hipError_t e = allow_dynamic_lds<&gram_large_kernel<TG, TX>>(smem1); e != hipSuccess) return e;
     gram_large_kernel<TG, TX><<<dim3(a.B + (a.static_state ? 1 : 0), a.parts), 256, smem1, stream>>>(a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1059,7 +1055,7 @@ static hipError_t launch_large(const BwdReduceArgs &a, hipStream_t stream, const
             if (a.n <= 16) return hipErrorInvalidValue;
             size_t smem2 = sizeof(float) * coef_bwd_large_lds_floats<32>(a.T);
             if (smem2 < dx_large_lds_bytes()) smem2 = dx_large_lds_bytes();
-            e = allow_dynamic_lds(&coef_bwd_large_dx_kernel<32, false>, smem2);
+            e = allow_dynamic_lds<&coef_bwd_large_dx_kernel<32, false>>(smem2);
             if (e != hipSuccess) return e;
             const unsigned ncb = (unsigned)((a.C + kDxlCB - 1) / kDxlCB);
             coef_bwd_large_dx_kernel<32, false><<<(unsigned)a.B * (1u + ncb), 256, smem2, stream>>>(a, *shadow);
@@ -1069,12 +1065,12 @@ static hipError_t launch_large(const BwdReduceArgs &a, hipStream_t stream, const
     if (shadow) return hipErrorInvalidValue;
     if (a.n <= 16) {
         const size_t smem2 = sizeof(float) * coef_bwd_large_lds_floats<16>(a.T);
-        e = allow_dynamic_lds(&coef_bwd_large_kernel<16, kPrecise>, smem2);
+        e = allow_dynamic_lds<&coef_bwd_large_kernel<16, kPrecise>>(smem2);
         if (e != hipSuccess) return e;
         coef_bwd_large_kernel<16, kPrecise><<<a.B, 256, smem2, stream>>>(a);
     } else {
         const size_t smem2 = sizeof(float) * coef_bwd_large_lds_floats<32>(a.T);
-        e = allow_dynamic_lds(&coef_bwd_large_kernel<32, kPrecise>, smem2);
+        e = allow_dynamic_lds<&coef_bwd_large_kernel<32, kPrecise>>(smem2);
         if (e != hipSuccess) return e;
         coef_bwd_large_kernel<32, kPrecise><<<a.B, 256, smem2, stream>>>(a);
     }

@@ -259,20 +259,20 @@ hipError_t launch_coef_bwd_static(const float *red_sum, const float *Hpre, const
     if (n <= 8) {
         if (n <= 4) {
             const size_t smem = sizeof(float) * SkSmall<4>::scaling_floats(T);
-            if (hipError_t e = allow_dynamic_lds(&coef_bwd_static_small_kernel<4>, smem); e != hipSuccess) return e;
+            if (hipError_t e = allow_dynamic_lds<&coef_bwd_static_small_kernel<4>>(smem); e != hipSuccess) return e;
             coef_bwd_static_small_kernel<4><<<1, 64, smem, stream>>>(red_sum, Hpre, Hpost, H_res_logits, dH_pre, dH_post, dH_res, n, T, eps);
         } else {
             const size_t smem = sizeof(float) * SkSmall<8>::scaling_floats(T);
-            if (hipError_t e = allow_dynamic_lds(&coef_bwd_static_small_kernel<8>, smem); e != hipSuccess) return e;
+            if (hipError_t e = allow_dynamic_lds<&coef_bwd_static_small_kernel<8>>(smem); e != hipSuccess) return e;
             coef_bwd_static_small_kernel<8><<<1, 64, smem, stream>>>(red_sum, Hpre, Hpost, H_res_logits, dH_pre, dH_post, dH_res, n, T, eps);
         }
     } else if (n <= 16) {
         const size_t smem = sizeof(float) * SkWg<16>::lds_floats(T);
-        if (hipError_t e = allow_dynamic_lds(&coef_bwd_static_kernel<16>, smem); e != hipSuccess) return e;
+        if (hipError_t e = allow_dynamic_lds<&coef_bwd_static_kernel<16>>(smem); e != hipSuccess) return e;
         coef_bwd_static_kernel<16><<<1, 256, smem, stream>>>(red_sum, Hpre, Hpost, H_res_logits, dH_pre, dH_post, dH_res, n, T, eps, state);
     } else {
         const size_t smem = sizeof(float) * SkWg<32>::lds_floats(T);
-        if (hipError_t e = allow_dynamic_lds(&coef_bwd_static_kernel<32>, smem); e != hipSuccess) return e;
+        if (hipError_t e = allow_dynamic_lds<&coef_bwd_static_kernel<32>>(smem); e != hipSuccess) return e;
         coef_bwd_static_kernel<32><<<1, 256, smem, stream>>>(red_sum, Hpre, Hpost, H_res_logits, dH_pre, dH_post, dH_res, n, T, eps, state);
     }
     return hipGetLastError();
@@ -374,11 +374,11 @@ hipError_t launch_finalize_static(const float *u, int rows_u, int C, DwOut dw, c
     a.sums.nblk = dw ? (C + 31) / 32 : 0;  // blocks of 32 columns
     if (n <= 4) {
         const size_t smem = sizeof(float) * SkSmall<4>::scaling_floats(T);
-        if (hipError_t e = allow_dynamic_lds(&finalize_static_kernel<4>, smem); e != hipSuccess) return e;
+        if (hipError_t e = allow_dynamic_lds<&finalize_static_kernel<4>>(smem); e != hipSuccess) return e;
         finalize_static_kernel<4><<<a.sums.nblk + 1, 1024, smem, stream>>>(a);
     } else {
         const size_t smem = sizeof(float) * SkSmall<8>::scaling_floats(T);
-        if (hipError_t e = allow_dynamic_lds(&finalize_static_kernel<8>, smem); e != hipSuccess) return e;
+        if (hipError_t e = allow_dynamic_lds<&finalize_static_kernel<8>>(smem); e != hipSuccess) return e;
         finalize_static_kernel<8><<<a.sums.nblk + 1, 1024, smem, stream>>>(a);
     }
     return hipGetLastError();

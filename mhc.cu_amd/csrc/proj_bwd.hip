@@ -305,11 +305,7 @@ static hipError_t launch_what(const ProjBwdArgs &a, int S, hipStream_t stream) {
     constexpr int LD = 32 * NTK + 8;
     const size_t smem = sizeof(bf16_t) * (size_t)LD * (a.DP + 32 * (4 / NTK));
     auto kern = proj_bwd_mfma_kernel<NTK, TPW, PHI_REGS, WHAT>;
-    if (smem > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return e;
-    }
+    if (hipError_t e = allow_dynamic_lds<&proj_bwd_mfma_kernel<NTK, TPW, PHI_REGS, WHAT>>(smem); e != hipSuccess) return e;
     const int slabs = (a.nC + 32 * NTK - 1) / (32 * NTK);
     dim3 grid(NTK == 1 ? round_up(slabs, 16) : slabs, S + (WHAT == kProjDphi && a.tail_row >= 0 ? 1 : 0));
     kern<<<grid, 256, smem, stream>>>(a);

@@ -334,7 +334,7 @@ static hipError_t launch_addx(const ProjAddxArgs &a, hipStream_t stream) {
     const size_t tiles = sizeof(bf16_t) * (size_t)kAxLD * (32 * NTD + SBR) + sizeof(float) * SBR * kAxLDO;
     const size_t red = sizeof(float) * NW * NTD * 32 * kAxLDR;  // the final cross-wave sum reuses the tiles' memory
     const size_t smem = tiles > red ? tiles : red;
-    hipError_t e = allow_dynamic_lds(&proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG>, smem);
+    hipError_t e = allow_dynamic_lds<&proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG>>(smem);
     if (e != hipSuccess) return e;
     const int slabs = (a.nC + kAxKW - 1) / kAxKW;
     dim3 grid(round_up(slabs, 16), 1 + (a.tail_row >= 0 ? 1 : 0));

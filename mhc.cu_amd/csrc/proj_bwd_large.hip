@@ -428,13 +428,13 @@ hipError_t launch_dphi_large(const void *x, const void *dPT, int BP, float *dphi
         a.tpw = tpw;
         const int ytiles = (NTD + tpw - 1) / tpw;
         if (with_tail) a.tail_row = ytiles;
-        e = allow_dynamic_lds(&dphi_large_kernel<9, true>, smem);
+        e = allow_dynamic_lds<&dphi_large_kernel<9, true>>(smem);
         if (e != hipSuccess) return e;
         dphi_large_kernel<9, true><<<dim3(slabs, ytiles + (with_tail ? 1 : 0), S), 256, smem, stream>>>(a);
     } else {
         const int ytiles = (NTD + 2) / 3;
         if (with_tail) a.tail_row = ytiles;
-        e = allow_dynamic_lds(&dphi_large_kernel<3, false>, smem);
+        e = allow_dynamic_lds<&dphi_large_kernel<3, false>>(smem);
         if (e != hipSuccess) return e;
         dphi_large_kernel<3, false><<<dim3(slabs, ytiles + (with_tail ? 1 : 0), S), 256, smem, stream>>>(a);
     }

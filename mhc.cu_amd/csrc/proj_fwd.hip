@@ -564,11 +564,7 @@ static hipError_t launch_wide(const void *x, const void *phi, float *Ppart, floa
     const int cpk = (nch_all + KS - 1) / KS;
     const int grid = 8 * ((groups * sgroups * KS + 7) / 8);
     const size_t smem = sizeof(bf16_t) * 2 * (128 + R) * kWideLd;
-    if (smem > 64 * 1024) {  // above the default dynamic-LDS limit (the CU has 160 KB)
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&proj_fwd_wide_kernel<NT, P, NWM, NWN, PF32>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return e;
-    }
+    if (hipError_t e = allow_dynamic_lds<&proj_fwd_wide_kernel<NT, P, NWM, NWN, PF32>>(smem); e != hipSuccess) return e;
     proj_fwd_wide_kernel<NT, P, NWM, NWN, PF32><<<grid, 64 * NWM * NWN, smem, stream>>>(
         static_cast<const bf16_t *>(x), static_cast<const bf16_t *>(phi), Ppart, ssqpart, B, D, DP,
         nC, groups, sgroups, KS, cpk, src);
@@ -686,7 +682,7 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
     const size_t smem_chunks = sizeof(bf16_t) * 4 * (1 + NT) * 32 * kNarrowPitch;
     const size_t smem_sum = sizeof(float) * 4 * (NT * 16 + 1) * 64;
     const size_t smem = smem_chunks > smem_sum ? smem_chunks : smem_sum;
-    if (hipError_t e = allow_dynamic_lds(&proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG>, smem); e != hipSuccess) return e;
+    if (hipError_t e = allow_dynamic_lds<&proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG>>(smem); e != hipSuccess) return e;
     proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG><<<grid, 256, smem, stream>>>(x, phi, Ppart,
                                                                  ssqpart, B, D, DP, nC, tiles_s, KS, sub, src);
     return hipGetLastError();
