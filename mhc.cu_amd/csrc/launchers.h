@@ -66,6 +66,7 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C);
 hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_dtype, float *Ppart,
                            float *ssqpart, int KS, int B, int n, int C, hipStream_t stream,
                            const ParamGather *gather = nullptr);
+int fwd_splits_summed_at_once(int n, int C);  // n <= 8: the most splits that the fused forward sums in one round of loads
 bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C);
 
 // Coefficients from projection partials (dynamic: Ppart != nullptr) or logits (static: B == 1).

@@ -154,6 +154,12 @@ __device__ __forceinline__ void get_act(const RawVec<T, V> &r, float (&v)[V]) {
     }
 }
 
+// K splits of the projection that a workgroup sums from one round of loads: what its registers leave room for
+constexpr int fwd_splits_in_one_round(int NP, int CPT) { return NP == 8 ? 32 : (CPT == 1 ? 24 : 16); }
+int fwd_splits_summed_at_once(int n, int C) {  // what the projection's split count is capped to (bf16 tier chunks)
+    return fwd_splits_in_one_round(n <= 4 ? 4 : 8, C <= 2048 ? 1 : 2);
+}
+
 constexpr int kFwdStaggerMinB = 512;  // two or more workgroups per CU
 
 // RX: fp32 x (and f) consumed as bf16, every value rounded to bf16 as it is unpacked
@@ -161,13 +167,13 @@ constexpr int kFwdStaggerMinB = 512;  // two or more workgroups per CU
 // shifted down behind the barrier.  A template argument: as a run-time switch the clamps and compares cost the
 // whole rows 4 % (B=3001 n=4 C=2560: 27.4 -> 28.5 us).
 template <typename TX, typename TY, int NP, int V, int CPT, bool RX = false, bool RAG = false>
-__global__ __launch_bounds__(256, (CPT == 2 && NP == 4 && !std::is_same<TX, float>::value) ? 4 : kMfmaMinWaves)
+__global__ __launch_bounds__(256, (CPT == (NP == 4 ? 2 : 1) && !std::is_same<TX, float>::value) ? 4 : kMfmaMinWaves)
 void layer_fwd_small_kernel(LayerFwdArgs a) {
     using SK = SkSmall<NP>;
     __shared__ float coef_s[NP * NP + 2 * NP];  // M | Hpre | Hpost
     __shared__ float red[4];
     const int b = blockIdx.x, n = a.n, C = a.C, tid = threadIdx.x;
-    const int nt = blockDim.x;  // whole waves, as few as hold the sample's chunks (256 for 8x8: the four waves share the split sums)
+    const int nt = blockDim.x;  // whole waves, as few as hold the sample's chunks (see launch_fused_small)
     const TX *__restrict__ xb = static_cast<const TX *>(a.x) + (size_t)b * n * C;
     TY *__restrict__ yb = static_cast<TY *>(a.y) + (size_t)b * n * C;
     const bool inject = a.f_inject != nullptr;
@@ -180,19 +186,20 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
     // the bulk data, so the Sinkhorn chain below runs while the tile is still streaming in),
     // then every thread issues the loads of the sample's whole tile. ------------------------------
     // Lane g of a group owns matrix element (r0, c0) and, for g < 2n, entry g of the vector (pre | post).
-    // The K-split sums are shared four ways: by the four groups of wave 0 (4x4 matrices, combined
-    // with lane swaps) or by the four waves (8x8 matrices, a whole wave per group, combined through
+    // The K-split sums are shared: by the four groups of wave 0 (4x4 matrices, combined with lane
+    // swaps) or by the waves of the workgroup (8x8 matrices, a whole wave per group, combined through
     // LDS); the coefficient step itself runs on the first group.
-    constexpr int kSplitWaves = SK::kPerWave == 1 ? 4 : 1;
+    constexpr int kSplitWaves = SK::kPerWave == 1 ? 4 : 1;  // at most
     __shared__ float psum_s[kSplitWaves == 4 ? 4 * 3 * 64 : 1];
-    const int g = tid % SK::kGroup, part = (tid / SK::kGroup) % 4;
+    const int g = tid % SK::kGroup, parts = kSplitWaves == 4 ? nt / kWave : 4, part = (tid / SK::kGroup) % parts;
     const int D = n * n + 2 * n;
     const int r0 = SK::row(g), c0 = SK::col0(g);
     const bool mv = r0 < n && c0 < n, vv = g < 2 * n;
     float al0 = 0.f, al1 = 0.f, al2 = 0.f, bvec = 0.f, bres = 0.f;
     // 4 * SU K-splits are summed from one round of loads (proj_fwd_ksplit caps the split count to
     // match; the two-chunk variant has no registers to spare for more)
-    constexpr int SU = (CPT == 1 ? 24 : 16) / 4;
+    constexpr int SU = fwd_splits_in_one_round(NP, CPT) / 4;
+    constexpr int SH = NP == 8 ? SU / 2 : SU;
     float t_ssq[SU], t_vec[SU], t_e[SU];
     const size_t ps = (size_t)a.B * a.DP;
     const float *Pb = dyn ? a.Ppart + (size_t)b * a.DP : nullptr;
@@ -203,13 +210,19 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
         bvec = g < n ? a.b_pre[g] : a.b_post[vv ? g - n : 0];
         bres = a.b_res[mv ? r0 * n + c0 : 0];
         if (dyn) {
-#pragma unroll
-            for (int u = 0; u < SU; u++) {  // first batch of K-split partials: ks = part*SU + u
-                const int ks = part * SU + u;
+            // first batch of K-split partials: ks = parts u + part, the upper half only where there are as many
+            auto split_sums = [&](int u) {
+                const int ks = parts * u + part;
                 const size_t ko = ks < a.KS ? ks : 0;
                 t_ssq[u] = a.ssqpart[ko * a.B + b];
                 t_vec[u] = Pb[ko * ps + (vv ? g : 0)];
                 t_e[u] = Pb[ko * ps + (mv ? 2 * n + r0 * n + c0 : 0)];
+            };
+#pragma unroll
+            for (int u = 0; u < SH; u++) split_sums(u);
+            if (a.KS > parts * SH) {
+#pragma unroll
+                for (int u = SH; u < SU; u++) split_sums(u);
             }
         }
     }
@@ -251,21 +264,15 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
     if (tid < 64 * kSplitWaves && dyn) {
 #pragma unroll
         for (int u = 0; u < SU; u++) {
-            const bool ok = part * SU + u < a.KS;
+            const bool ok = parts * u + part < a.KS;
             ssq += ok ? t_ssq[u] : 0.f;
             pvec += (ok && vv) ? t_vec[u] : 0.f;
             pe += (ok && mv) ? t_e[u] : 0.f;
         }
-        for (int ks0 = (4 + part) * SU; ks0 < a.KS; ks0 += 4 * SU) {  // never with proj_fwd_ksplit's cap
-#pragma unroll
-            for (int u = 0; u < SU; u++) {
-                const int ks = ks0 + u;
-                if (ks < a.KS) {
-                    ssq += a.ssqpart[(size_t)ks * a.B + b];
-                    if (vv) pvec += Pb[ks * ps + g];
-                    if (mv) pe += Pb[ks * ps + 2 * n + r0 * n + c0];
-                }
-            }
+        for (int ks = parts * SU + part; ks < a.KS; ks += parts) {  // never with proj_fwd_ksplit's cap
+            ssq += a.ssqpart[(size_t)ks * a.B + b];
+            if (vv) pvec += Pb[ks * ps + g];
+            if (mv) pe += Pb[ks * ps + 2 * n + r0 * n + c0];
         }
         if constexpr (kSplitWaves == 1) {  // the four groups of wave 0 hold a quarter of the splits each
             ssq = xor32_add(xor16_add(ssq));
@@ -281,9 +288,11 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
         if (dyn) {  // uniform over the workgroup
             __syncthreads();
             if (tid < 64) {
-                ssq = (psum_s[0 * 64 + g] + psum_s[3 * 64 + g]) + (psum_s[6 * 64 + g] + psum_s[9 * 64 + g]);
-                pvec = (psum_s[1 * 64 + g] + psum_s[4 * 64 + g]) + (psum_s[7 * 64 + g] + psum_s[10 * 64 + g]);
-                pe = (psum_s[2 * 64 + g] + psum_s[5 * 64 + g]) + (psum_s[8 * 64 + g] + psum_s[11 * 64 + g]);
+                for (int p = 1; p < parts; p++) {
+                    ssq += psum_s[(p * 3 + 0) * 64 + g];
+                    pvec += psum_s[(p * 3 + 1) * 64 + g];
+                    pe += psum_s[(p * 3 + 2) * 64 + g];
+                }
             }
         }
     }
@@ -624,9 +633,14 @@ static bool launch_fused_small(const LayerFwdArgs &a, hipStream_t stream, hipErr
     const int nch = (a.C + V - 1) / V;
     const int cpt = (nch + 255) / 256;
     // as few whole waves as hold the chunks: a thread without a chunk of its own still runs the loads
-    // and the arithmetic on an aliased one (320 chunks on 2 x 256 slots would waste 37 % of both)
+    // and the arithmetic on an aliased one (320 chunks on 2 x 256 slots would waste 37 % of both), and short
+    // rows leave room for more workgroups, whose serial coefficient steps then overlap.  8 x 8: the waves share
+    // the split sums, four take them where fewer would need a second round of loads
+    // Always 256 threads -> as few as needed, with 128 registers (kernel us): n=5 B=3000 C=1024 33.1 -> 20.0,
+    // n=8 B=6000 C=512 64.1 -> 22.5, n=6 B=2000 C=384 24.5 -> 10.2, n=8 B=789 C=1984 18.2 -> 14.0 (registers only).
     const int per = cpt == 3 ? 4 : cpt;  // chunks per thread of the instantiation that runs
-    const int nt = NP == 8 ? 256 : round_up((nch + per - 1) / per, kWave);
+    int nt = round_up((nch + per - 1) / per, kWave);
+    if (NP == 8 && a.KS > fwd_splits_in_one_round(8, per) / 4 * (nt / kWave)) nt = 256;
     if (cpt == 1) layer_fwd_small_kernel<TX, TY, NP, V, 1, RX, RAG><<<a.B, nt, 0, stream>>>(a);
     else if (cpt == 2) layer_fwd_small_kernel<TX, TY, NP, V, 2, RX, RAG><<<a.B, nt, 0, stream>>>(a);
     else if (cpt <= 4 && NP == 4) layer_fwd_small_kernel<TX, TY, 4, V, 4, RX, RAG><<<a.B, nt, 0, stream>>>(a);

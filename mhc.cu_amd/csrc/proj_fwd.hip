@@ -113,8 +113,10 @@ __device__ __forceinline__ void gather_small(const PhiSrc &g, int tid, int nthr,
 // accumulators) is the same.  With 32 samples per tile and D padded to 32 instead of 128 x 128 tiles the fp32
 // projection of B=2560 n=4 C=1280 went from 58 to 20 us.
 // RAG: rows of any length (nC no multiple of the pieces): the last piece is read from nC - EL on and shifted down.
-template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false, bool RAG = false>
-__global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
+// NW: waves per workgroup, four, or eight where four would leave a wave several chunks to walk one after the other
+// on a chip that is not full (narrow_waves below).
+template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false, bool RAG = false, int NW = 4>
+__global__ __launch_bounds__(64 * NW, kMfmaMinWaves) void proj_fwd_mfma_kernel(const void *__restrict__ x_,
                                                             const void *__restrict__ phi_,
                                                             float *__restrict__ Ppart,
                                                             float *__restrict__ ssqpart, int B,
@@ -144,7 +146,7 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
     const int row = lane & 31, kh = lane >> 5;
     const int b = st * 32 + row;
     const int dbase = blockIdx.y * NT * 32;
-    const int kbeg = (ks * 4 + wave) * sub;
+    const int kbeg = (ks * NW + wave) * sub;
     const int kend = min(kbeg + sub, nC);
     const bool bvalid = b < B;
 
@@ -278,7 +280,7 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
     int kc = kbeg + (nch ? st % nch : 0) * CH;  // first chunk
     if (nch) fetch(kc);
     if constexpr (PF32)
-        if (item == 0 && blockIdx.y == 0) gather_small(src, threadIdx.x, 256, D);
+        if (item == 0 && blockIdx.y == 0) gather_small(src, threadIdx.x, 64 * NW, D);
     MHC_PHASE_ADD(kPhaseProjFwd, pwg, 0, pclk);
     for (int it = 0; it < nch; it++) {
         park(kc);
@@ -325,8 +327,8 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
     __syncthreads();  // every wave is done with its chunk tile: the memory becomes the cross-wave buffer
     ssq = xor32_add(ssq);  // both K halves of the row
 
-    // cross-wave sum: every wave parks its tiles in LDS, then wave w adds and writes accumulator
-    // registers 4w .. 4w+3 of every tile (rows 8w + 4 kh .. +3 of the 32 x 32 tile), wave 0 also x^2
+    // cross-wave sum: every wave parks its tiles in LDS, then wave w adds and writes its 16 / NW accumulator
+    // registers of every tile, wave 0 also x^2
     constexpr int R = NT * 16 + 1;
     {
         float *dst = lds + (size_t)wave * R * 64;
@@ -344,19 +346,19 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void proj_fwd_mfma_kernel(const
     for (int t = 0; t < NT; t++) {
         const int d = dbase + t * 32 + row;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int i = 4 * wave + q;
+        for (int q = 0; q < 16 / NW; q++) {
+            const int i = 16 / NW * wave + q;
             float v = 0.f;
 #pragma unroll
-            for (int w = 0; w < 4; w++) v += lds[((size_t)w * R + t * 16 + i) * 64 + lane];
-            const int bs = st * 32 + 8 * wave + 4 * kh + q;
+            for (int w = 0; w < NW; w++) v += lds[((size_t)w * R + t * 16 + i) * 64 + lane];
+            const int bs = st * 32 + 8 * (i >> 2) + 4 * kh + (i & 3);
             if (bs < B && d < DP) out[(size_t)bs * DP + d] = d < D ? v : 0.f;  // padded rows stay zero
         }
     }
     if (wave == 0 && blockIdx.y == 0 && kh == 0 && bvalid) {
         float v = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) v += lds[((size_t)w * R + R - 1) * 64 + lane];
+        for (int w = 0; w < NW; w++) v += lds[((size_t)w * R + R - 1) * 64 + lane];
         ssqpart[(size_t)ks * B + b] = v;
     }
     MHC_PHASE_ADD(kPhaseProjFwd, pwg, 3, pclk);
@@ -628,11 +630,9 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
     const int cap_bytes = (int)(0.35 * (esize * B * nC + esize * DP * nC) / (4.0 * B * DP));
     if (ks > cap_slab) ks = cap_slab;
     if (ks > cap_bytes) ks = cap_bytes;
-    // the fused forward kernel (n <= 8) sums up to 24 splits (16 when a thread holds two chunks of
-    // the sample, C > 2048) with loads that it issues ahead of the sample's tile; more splits would
-    // queue behind the tile
-    const int fused_cap = C <= 2048 ? 24 : 16;
-    if (n <= 8 && ks > fused_cap) ks = fused_cap;
+    // the fused forward kernel (n <= 8) sums that many splits with loads that it issues ahead of the sample's
+    // tile; more splits would queue behind the tile
+    if (const int cap = fwd_splits_summed_at_once(n, C); n <= 8 && ks > cap) ks = cap;
     if (ks > 64) ks = 64;
     if (ks < 1) ks = 1;
     // splits with work when ks are asked for (see below)
@@ -666,7 +666,15 @@ static hipError_t launch_generic(const void *x, const void *phi, float *Ppart, f
     return hipGetLastError();
 }
 
-template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false, bool RAG = false>
+// Waves per workgroup of the narrow kernel.  Few samples and a long row (the split count is capped by what the
+// forward kernel sums in one round): a wave's chunks are one dependent round trip to memory each, so eight waves
+// share the slab where that shortens the walk and at most one workgroup falls to a CU anyway (147 KB of LDS at n = 8).
+// Kernel us, four -> eight: n=6 B=2 C=2752 11.3 -> 10.3, n=8 B=64 C=3072 17.0 -> 15.3, n=4 B=64 C=4096 7.2 -> 6.3.
+static int narrow_waves(int workgroups, int KS, int nC, int chunk) {
+    return workgroups <= 256 && (nC + KS * 4 - 1) / (KS * 4) > chunk ? 8 : 4;
+}
+
+template <int NT, bool XF32 = false, bool PF32 = false, bool EXACT = false, bool RAG = false, int NW = 4>
 static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, float *ssqpart, int KS,
                               int B, int D, int DP, int nC, hipStream_t stream, const PhiSrc &src = PhiSrc{}) {
     if constexpr (NT <= 3 && !RAG) {
@@ -677,13 +685,18 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
     }
     const int tiles_s = (B + 31) / 32;
     const int groups = (DP / 32 + NT - 1) / NT;
-    const int sub = round_up((nC + KS * 4 - 1) / (KS * 4), EXACT ? 32 : 64);  // whole chunks: 128-byte lines
+    constexpr int kChunk = EXACT ? 32 : 64;
+    if constexpr (NT <= 3 && !RAG && NW == 4) {
+        if (narrow_waves(tiles_s * KS * groups, KS, nC, kChunk) == 8)
+            return launch_mfma<NT, XF32, PF32, EXACT, RAG, 8>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
+    }
+    const int sub = round_up((nC + KS * NW - 1) / (KS * NW), kChunk);  // whole chunks: 128-byte lines
     dim3 grid(8 * ((tiles_s * KS + 7) / 8), groups);
-    const size_t smem_chunks = sizeof(bf16_t) * 4 * (1 + NT) * 32 * kNarrowPitch;
-    const size_t smem_sum = sizeof(float) * 4 * (NT * 16 + 1) * 64;
+    const size_t smem_chunks = sizeof(bf16_t) * NW * (1 + NT) * 32 * kNarrowPitch;
+    const size_t smem_sum = sizeof(float) * NW * (NT * 16 + 1) * 64;
     const size_t smem = smem_chunks > smem_sum ? smem_chunks : smem_sum;
-    if (hipError_t e = allow_dynamic_lds<&proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG>>(smem); e != hipSuccess) return e;
-    proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG><<<grid, 256, smem, stream>>>(x, phi, Ppart,
+    if (hipError_t e = allow_dynamic_lds<&proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG, NW>>(smem); e != hipSuccess) return e;
+    proj_fwd_mfma_kernel<NT, XF32, PF32, EXACT, RAG, NW><<<grid, 64 * NW, smem, stream>>>(x, phi, Ppart,
                                                                  ssqpart, B, D, DP, nC, tiles_s, KS, sub, src);
     return hipGetLastError();
 }
