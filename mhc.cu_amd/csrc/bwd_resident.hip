@@ -100,28 +100,15 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     constexpr int CW = STATIC ? 0 : 1;    // coefficient waves in front of the tile waves
     __shared__ float slot_s[K * TW * 4];  // one slot per 16-lane row of the tile waves
     __shared__ float tot_s[K + 1];        // the sums, then s1
-    __shared__ float park_s[STATIC ? 1 : SkSmall<NP>::kGroup];  // one value per coefficient lane, see below
     extern __shared__ float sc[];         // Sinkhorn denominators, SK::scaling_floats(T), then CB::kXch
     const int b = blockIdx.x, n = a.n, C = a.C;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pwg = blockIdx.x;
     (void)pwg;
     MHC_PHASE_ZERO(kPhaseGramSmall, pwg);
     MHC_PHASE_ZERO(kPhaseDxSmall, pwg);   // second timeline: the first tile wave (thread 64)
     MHC_PHASE_BEGIN(pclk);
     MHC_PHASE_BEGIN(tclk);
-    CB cb;
-    if (tid < SK::kGroup) {
-        // everything the coefficient backward needs besides the sums, requested at once
-        cb.prefetch(a, b, tid);
-        if constexpr (!STATIC) {
-            cb.forward_recompute(a, b, tid, tid, sc);
-            // The coefficient lanes share their register budget with the tile code below; the final
-            // iterate lived across it in scratch memory, and reading it back was a global round trip in
-            // front of the serial Sinkhorn sweep: it is parked in LDS instead.
-            park_s[tid] = cb.m_fin;
-        }
-    }
     // the NP^2 threads that will hold the sums of W1 (one DPP row of wave 0 for 4x4, wave 1 for 8x8) ask
     // for their factor of s1 = Hpost^T W1 Hpre now, not behind the barrier
     // (the two factors stay as loaded until then: for 8x8 these threads are a tile wave, and a product
@@ -134,10 +121,51 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
         hp_l = a.Hpre[(size_t)b * hs + (c < n ? c : 0)];
         hohp_ok = r < n && c < n;
     }
-    MHC_PHASE_ADD(kPhaseGramSmall, pwg, 0, pclk);
+    // K threads finish the sums; the NP^2 threads that hold W1 (one DPP row for 4x4, wave 1 for 8x8)
+    // also form s1 = Hpost^T W1 Hpre, which the tile waves need for da
+    auto finish_sums = [&]() {
+        __syncthreads();
+        MHC_PHASE_ADD(kPhaseGramSmall, pwg, 1, pclk);
+        if (tid < K) {
+            float v = 0.f;
+#pragma unroll
+            for (int sl = 0; sl < TW * 4; sl++) v += slot_s[tid * (TW * 4) + sl];
+            tot_s[tid] = v;
+            if (!inject && tid >= NP * NP && tid < 2 * NP * NP) {
+                float t = hohp_ok ? ho_l * hp_l * v : 0.f;
+                if constexpr (NP == 4) t = row16_allreduce(t);
+                else t = wave_allreduce_sum(t);
+                if (tid == NP * NP) tot_s[K] = t;
+            }
+        }
+        __syncthreads();
+        MHC_PHASE_ADD(kPhaseGramSmall, pwg, 2, pclk);
+    };
+    CB cb;
+    // ---- 2. the coefficient wave's whole life, a uniform branch of its own: it meets the tile waves at the two
+    // barriers of finish_sums() and shares no register with their code (in one body with it, its values lived
+    // across the Gram products: 130 -> 112 registers at n = 8 with one item) --------------------------------
+    if constexpr (!STATIC) {
+        if (wave == 0) {
+            if (tid < SK::kGroup) {
+                // everything the coefficient backward needs besides the sums, requested at once
+                cb.prefetch(a, b, tid);
+                cb.forward_recompute(a, b, tid, tid, sc);
+            }
+            MHC_PHASE_ADD(kPhaseGramSmall, pwg, 0, pclk);
+            finish_sums();
+            if (tid < SK::kGroup) {
+                cb.fetch_sums(tot_s, 1);
+                cb.run(a, b, tid, tid, sc, sc + SK::scaling_floats(a.T));
+            }
+            MHC_PHASE_ADD(kPhaseGramSmall, pwg, 3, pclk);
+            return;
+        }
+    } else if (tid < SK::kGroup) {
+        cb.prefetch(a, b, tid);
+    }
     const int blk = lane >> 2, i = lane & 3;
-    const int tw = wave - CW;             // tile wave index, -1 for the coefficient wave
-    const bool tile = tw >= 0;
+    const int tw = wave - CW;             // tile wave index
 
     // ---- tile waves: every load of the sample up front -----------------------------------------
     uint4 gr[ITEMS][NB], xr[ITEMS][NB], fr[ITEMS];
@@ -149,7 +177,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     RawVec<float, 8> wf[ITEMS];
     bool in[ITEMS], sv[NB];
     float hpre[NB], hpost[NB], Mc[NB][NB][4], qraw = 1.f;
-    if (tile) {
+    {
         size_t rowoff[NB];
 #pragma unroll
         for (int I = 0; I < NB; I++) {
@@ -172,26 +200,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
             else if constexpr (RAG) wf[it].load_any(static_cast<const float *>(a.w) + cc);
             else wf[it].load(static_cast<const float *>(a.w) + cc);
         }
-        // this lane's coefficients for step 3 (its own streams j = 4I + i), in flight with the tile
-        const float *Hp = a.Hpre + (size_t)b * hs, *Ho = a.Hpost + (size_t)b * hs, *Mb = a.M + (size_t)b * hs * n;
-#pragma unroll
-        for (int I = 0; I < NB; I++) {
-            hpre[I] = Hp[sv[I] ? 4 * I + i : 0];
-            hpost[I] = Ho[sv[I] ? 4 * I + i : 0];
-#pragma unroll
-            for (int J = 0; J < NB; J++)
-#pragma unroll
-                for (int ii = 0; ii < 4; ii++) {
-                    // Mc[I][J][ii] = M[source stream 4J + ii][target stream 4I + i]
-                    const bool ok = sv[I] && 4 * J + ii < n;
-                    const float m = Mb[ok ? (4 * J + ii) * n + 4 * I + i : 0];
-                    Mc[I][J][ii] = ok ? m : 0.f;
-                }
-        }
         if constexpr (!inject) qraw = a.q[b];
-#pragma unroll
-        for (int I = 0; I < NB; I++)
-            if (!sv[I]) { hpre[I] = 0.f; hpost[I] = 0.f; }
         // every load is requested: from here on the tile is four words of bf16 pairs per chunk
 #pragma unroll
         for (int it = 0; it < ITEMS; it++) {
@@ -212,10 +221,33 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
             }
         }
     }
+    auto load_coefs = [&]() {
+        // this lane's coefficients for step 3 (its own streams j = 4I + i), requested behind the Gram products (8 x 8:
+        // twenty registers less at their peak) and waited for behind the barrier
+        const float *Hp = a.Hpre + (size_t)b * hs, *Ho = a.Hpost + (size_t)b * hs, *Mb = a.M + (size_t)b * hs * n;
+#pragma unroll
+        for (int I = 0; I < NB; I++) {
+            hpre[I] = Hp[sv[I] ? 4 * I + i : 0];
+            hpost[I] = Ho[sv[I] ? 4 * I + i : 0];
+#pragma unroll
+            for (int J = 0; J < NB; J++)
+#pragma unroll
+                for (int ii = 0; ii < 4; ii++) {
+                    // Mc[I][J][ii] = M[source stream 4J + ii][target stream 4I + i]
+                    const bool ok = sv[I] && 4 * J + ii < n;
+                    const float m = Mb[ok ? (4 * J + ii) * n + 4 * I + i : 0];
+                    Mc[I][J][ii] = ok ? m : 0.f;
+                }
+        }
+#pragma unroll
+        for (int I = 0; I < NB; I++)
+            if (!sv[I]) { hpre[I] = 0.f; hpost[I] = 0.f; }
+    };
+    if constexpr (NP == 4) load_coefs();
 
     MHC_PHASE_ADD_BY(64, kPhaseDxSmall, pwg, 0, tclk);
     // ---- 1. Gram sums -------------------------------------------------------------------------------
-    if (tile) {
+    {
         f32x4_t acc[3][NB][NB];
 #pragma unroll
         for (int m = 0; m < 3; m++)
@@ -273,6 +305,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                 }
             }
         }
+        if constexpr (NP == 8) load_coefs();
         // Lane (block, j) holds column j of its block's products, register = row.  Sum over the four
         // blocks of a 16-lane row with DPP, one LDS slot per row.
         const int slot = (tid - 64 * CW) >> 4;
@@ -292,106 +325,120 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                     }
     }
     MHC_PHASE_ADD_BY(64, kPhaseDxSmall, pwg, 1, tclk);
-    __syncthreads();
-    MHC_PHASE_ADD(kPhaseGramSmall, pwg, 1, pclk);
-    // K threads finish the sums; the NP^2 threads that hold W1 (one DPP row for 4x4, wave 1 for 8x8)
-    // also form s1 = Hpost^T W1 Hpre, which the tile waves need for da
-    if (tid < K) {
-        float v = 0.f;
-#pragma unroll
-        for (int sl = 0; sl < TW * 4; sl++) v += slot_s[tid * (TW * 4) + sl];
-        tot_s[tid] = v;
-        if (!inject && tid >= NP * NP && tid < 2 * NP * NP) {
-            float t = hohp_ok ? ho_l * hp_l * v : 0.f;
-            if constexpr (NP == 4) t = row16_allreduce(t);
-            else t = wave_allreduce_sum(t);
-            if (tid == NP * NP) tot_s[K] = t;
-        }
-    }
-    __syncthreads();
-
-    MHC_PHASE_ADD(kPhaseGramSmall, pwg, 2, pclk);
+    finish_sums();
     MHC_PHASE_ADD_BY(64, kPhaseDxSmall, pwg, 2, tclk);
-    // ---- 2. coefficient backward on the first lanes of wave 0 -----------------------------------------
-    if (tid < SK::kGroup) {
-        if constexpr (!STATIC) {
-            cb.m_fin = park_s[tid];
+    if constexpr (STATIC) {
+        if (tid < SK::kGroup) {
+            cb.fetch_sums(tot_s, 1);
+            cb.run(a, b, tid, tid, sc, sc);
         }
-        cb.fetch_sums(tot_s, 1);
-        cb.run(a, b, tid, tid, sc, sc + (STATIC ? 0 : SK::scaling_floats(a.T)));
     }
-    MHC_PHASE_ADD(kPhaseGramSmall, pwg, 3, pclk);
-    if (!tile) return;  // the coefficient wave (none with STATIC) is done
 
     // ---- 3. tile waves: dxp, u, df ---------------------------------------------------------------------
-    auto put8 = [](auto *p, const float (&v)[8], int left) {  // left: elements up to the row's end
-        using T = typename std::remove_reference<decltype(*p)>::type;
-        if constexpr (RAG) store_vec_any<T, 8>(p, v, left);
-        else store_vec<T, 8>(p, v);
-    };
     float qinv = 0.f, k2 = 0.f;
     if constexpr (!inject) {
         qinv = 1.0f / qraw;
         k2 = tot_s[K] * qinv * qinv * qinv / (float)C;
     }
+    // eight results of a row in two halves, stored together (neighbouring 16-byte pieces at once)
+    constexpr int OW = F32 ? 8 : 4;  // words of a chunk as stored
+    auto put_half = [](TS *p, uint32_t (&w)[OW], const float (&v)[4], int h, int left) {
+        if constexpr (F32) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) w[4 * h + k] = __float_as_uint(v[k]);
+            if (h == 1) {
+                st16<false>(p, w[0], w[1], w[2], w[3]);
+                st16<false>(p + 4, w[4], w[5], w[6], w[7]);
+            }
+        } else {
+            w[2 * h] = pack_bf16x2(v[0], v[1]);
+            w[2 * h + 1] = pack_bf16x2(v[2], v[3]);
+            if (h == 1) {
+                if constexpr (!RAG) {
+                    st16<false>(p, w[0], w[1], w[2], w[3]);
+                } else if (left >= 8) {
+                    st16_any<false>(p, w[0], w[1], w[2], w[3]);
+                } else {  // left: elements up to the row's end
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if (e < left) p[e] = (TS)(w[e / 2] >> (16 * (e & 1)));
+                }
+            }
+        }
+    };
 #pragma unroll
     for (int it = 0; it < ITEMS; it++) {
         const int c = (tw + TW * it) * 128 + blk * 8;
         if (!in[it]) continue;  // quads are inside or outside together: the DPP exchanges stay within a quad
-        float gv[NB][8], xv[NB][8];
+        uint32_t ow[NB][OW], dfw[OW];
+        float u8[8];
+        // four channels at a time: the fp32 copies of eight cost the 8 x 8 case thirty registers
 #pragma unroll
-        for (int I = 0; I < NB; I++) {
-            const uint32_t gw[4] = {gr[it][I].x, gr[it][I].y, gr[it][I].z, gr[it][I].w};
-            const uint32_t xw[4] = {xr[it][I].x, xr[it][I].y, xr[it][I].z, xr[it][I].w};
+        for (int h = 0; h < 2; h++) {
+            float gv[NB][4], xv[NB][4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                gv[I][2 * k] = bf16lo_to_f32(gw[k]); gv[I][2 * k + 1] = bf16hi_to_f32(gw[k]);
-                xv[I][2 * k] = bf16lo_to_f32(xw[k]); xv[I][2 * k + 1] = bf16hi_to_f32(xw[k]);
-            }
-        }
-        float dfv[8], da[8];
+            for (int I = 0; I < NB; I++) {
+                const uint32_t gw[2] = {h ? gr[it][I].z : gr[it][I].x, h ? gr[it][I].w : gr[it][I].y};
+                const uint32_t xw[2] = {h ? xr[it][I].z : xr[it][I].x, h ? xr[it][I].w : xr[it][I].y};
 #pragma unroll
-        for (int v = 0; v < 8; v++) {
-            float pd = 0.f;
-#pragma unroll
-            for (int I = 0; I < NB; I++) pd += hpost[I] * gv[I][v];
-            dfv[v] = quad_allreduce(pd);
-        }
-        if constexpr (inject) {
-#pragma unroll
-            for (int v = 0; v < 8; v++) da[v] = 0.f;
-            if (ra.df && i == 0) put8(static_cast<TS *>(ra.df) + (size_t)b * C + c, dfv, C - c);
-        } else {
-            float wv[8], uv[8];
-            if constexpr (WMODE == kGramWBf16) wb[it].get(wv);
-            else wf[it].get(wv);
-#pragma unroll
-            for (int v = 0; v < 8; v++) {
-                float pa = 0.f;
-#pragma unroll
-                for (int I = 0; I < NB; I++) pa += hpre[I] * xv[I][v];
-                const float av = quad_allreduce(pa);
-                da[v] = dfv[v] * wv[v] * qinv - av * k2;
-                uv[v] = dfv[v] * av * qinv;
-            }
-            if (i == 0) put8(ra.u + (size_t)b * C + c, uv, C - c);
-        }
-#pragma unroll
-        for (int I = 0; I < NB; I++) {
-            float out[8];
-#pragma unroll
-            for (int v = 0; v < 8; v++) out[v] = hpre[I] * da[v];
-#pragma unroll
-            for (int J = 0; J < NB; J++)
-#pragma unroll
-                for (int v = 0; v < 8; v++) {
-                    out[v] += Mc[I][J][0] * quad_bcast<0>(gv[J][v]);
-                    out[v] += Mc[I][J][1] * quad_bcast<1>(gv[J][v]);
-                    out[v] += Mc[I][J][2] * quad_bcast<2>(gv[J][v]);
-                    out[v] += Mc[I][J][3] * quad_bcast<3>(gv[J][v]);
+                for (int k = 0; k < 2; k++) {
+                    gv[I][2 * k] = bf16lo_to_f32(gw[k]); gv[I][2 * k + 1] = bf16hi_to_f32(gw[k]);
+                    xv[I][2 * k] = bf16lo_to_f32(xw[k]); xv[I][2 * k + 1] = bf16hi_to_f32(xw[k]);
                 }
-            // plain stores: the projection-backward launch reads dxp back right away
-            if (sv[I]) put8(static_cast<TS *>(ra.dxp) + ((size_t)b * n + 4 * I + i) * C + c, out, C - c);
+            }
+            float dfv[4], da[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                float pd = 0.f;
+#pragma unroll
+                for (int I = 0; I < NB; I++) pd += hpost[I] * gv[I][v];
+                dfv[v] = quad_allreduce(pd);
+            }
+            if constexpr (inject) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) da[v] = 0.f;
+                if (ra.df && i == 0) put_half(static_cast<TS *>(ra.df) + (size_t)b * C + c, dfw, dfv, h, C - c);
+            } else {
+                float wv[4], uv[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    if constexpr (WMODE == kGramWBf16) wv[v] = v & 1 ? bf16hi_to_f32(wb[it].w[2 * h + v / 2]) : bf16lo_to_f32(wb[it].w[2 * h + v / 2]);
+                    else wv[v] = __uint_as_float(wf[it].w[4 * h + v]);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    float pa = 0.f;
+#pragma unroll
+                    for (int I = 0; I < NB; I++) pa += hpre[I] * xv[I][v];
+                    const float av = quad_allreduce(pa);
+                    da[v] = dfv[v] * wv[v] * qinv - av * k2;
+                    uv[v] = dfv[v] * av * qinv;
+                }
+#pragma unroll
+                for (int v = 0; v < 4; v++) u8[4 * h + v] = uv[v];
+                if (h == 1 && i == 0) {
+                    float *up = ra.u + (size_t)b * C + c;
+                    if constexpr (RAG) store_vec_any<float, 8>(up, u8, C - c);
+                    else store_vec<float, 8>(up, u8);
+                }
+            }
+#pragma unroll
+            for (int I = 0; I < NB; I++) {
+                float out[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) out[v] = hpre[I] * da[v];
+#pragma unroll
+                for (int J = 0; J < NB; J++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        out[v] += Mc[I][J][0] * quad_bcast<0>(gv[J][v]);
+                        out[v] += Mc[I][J][1] * quad_bcast<1>(gv[J][v]);
+                        out[v] += Mc[I][J][2] * quad_bcast<2>(gv[J][v]);
+                        out[v] += Mc[I][J][3] * quad_bcast<3>(gv[J][v]);
+                    }
+                // plain stores: the projection-backward launch reads dxp back right away
+                if (sv[I]) put_half(static_cast<TS *>(ra.dxp) + ((size_t)b * n + 4 * I + i) * C + c, ow[I], out, h, C - c);
+            }
         }
     }
     MHC_PHASE_ADD_BY(64, kPhaseDxSmall, pwg, 3, tclk);
@@ -414,8 +461,8 @@ static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream)
     const int threads = 64 * (TW + (STATIC ? 0 : 1));
     // five and ten tile waves are for rows that they hold in one or two items, seven for the longest rows;
     // ragged rows round the count up (fewer instantiations)
-    constexpr int kMinItems = TW == kResLongWaves ? (RAG ? 5 : 2) : 1;
-    constexpr int kMaxItems = TW == kResTileWaves || TW == kResLongWaves ? kResMaxItems : 2;
+    constexpr int kMinItems = TW == kResLongWaves ? (RAG ? 5 : (NP == 8 && !STATIC ? 1 : 3)) : 1;
+    constexpr int kMaxItems = TW == kResTileWaves ? (NP == 8 && !STATIC && !RAG ? 1 : kResMaxItems) : (TW == kResLongWaves ? kResMaxItems : 2);
     if (RAG && items == 4) items = 5;
     if (items < kMinItems) items = kMinItems;
 #define MHC_RES_ITEMS(N)                                                                              \
@@ -444,21 +491,16 @@ static hipError_t launch_items(const BwdResidentArgs &ra, hipStream_t stream) {
         else return launch_items_tw<NP, WMODE, F32, STATIC, kResTileWaves, true>(ra, stream);
     }
     if (ra.r.C > 128 * kResTileWaves * kResMaxItems) return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves>(ra, stream);
-    // Eight streams, rows of at most 1280 channels: ten tile waves hold the row in one item each
-    // instead of four in three - the Gram and mixing products of an 8 x 8 sample are most of such a
-    // workgroup's life, and one wave per SIMD has nobody to overlap them with.  Backward at B=256,
-    // C=1280, n=8, graphs of ten: 4 tile waves 21.3 us, 5 21.8, 8 21.4, 10 20.8 (n=4, B=320: 15.1 / 14.9 /
-    // 15.9 / 15.0: four stay).
-    if constexpr (NP == 8 && !F32 && !STATIC) {
-        if (ra.r.C <= 1280) return launch_items_tw<NP, WMODE, F32, STATIC, 10>(ra, stream);
-    }
-    // Longer rows of eight streams: as many tile waves as hold the row in two items (7 up to 1792 channels, 10 up to
-    // 2560).  One workgroup fits a CU at any of these register counts, so its waves are all the overlap there is
-    // (kernel us, four waves -> these: n=8 B=1300 C=1600 70.6 -> 54.4, B=2000 C=2048 106.0 -> 97.5, B=256 C=2560
-    // 16.8 -> 15.8; n=6 B=600 C=2304 38.8 -> 35.1).
-    if constexpr (NP == 8 && !F32 && !STATIC) {
-        if (ra.r.C > 128 * 2 * kResLongWaves) return launch_items_tw<NP, WMODE, F32, STATIC, 10>(ra, stream);
-        return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves>(ra, stream);
+    // Eight streams: the waves that hold the row in one item (512, 896, 1280 channels) or two (1792, 2560).  The Gram
+    // and mixing products of an 8 x 8 sample are most of such a workgroup's life, one wave per SIMD has nobody to
+    // overlap them with, and one workgroup fits a CU at the register counts of more items; waves without channels of
+    // their own only take room (kernel us): B=256 C=1280 four waves 12.1, ten 10.6; B=1300 C=1600 four 70.6, seven
+    // 53.1; B=2000 C=2048 four 106.0, ten 97.5; n=6 B=900 C=512 ten 33.0, four
+    // 22.3; n=8 B=600 C=768 ten 23.9, seven 18.0.
+    if constexpr (NP == 8 && !STATIC) {
+        const int C = ra.r.C;
+        if ((C > 896 && C <= 1280) || C > 1792) return launch_items_tw<NP, WMODE, F32, STATIC, 10>(ra, stream);
+        if (C > 512) return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves>(ra, stream);
     }
     // Four streams: a fifth tile wave where it saves every wave an item (rows of 513..640 and 1025..1280
     // channels: ten 128-channel chunks are 3 + 3 + 2 + 2 on four waves, 2 each on five).  B=320, C=1280,
