@@ -462,7 +462,7 @@ static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream)
     // five and ten tile waves are for rows that they hold in one or two items, seven for the longest rows;
     // ragged rows round the count up (fewer instantiations)
     constexpr int kMinItems = TW == kResLongWaves ? (RAG ? 5 : (NP == 8 && !STATIC ? 1 : 3)) : 1;
-    constexpr int kMaxItems = TW == kResTileWaves ? (NP == 8 && !STATIC && !RAG ? 1 : kResMaxItems) : (TW == kResLongWaves ? kResMaxItems : 2);
+    constexpr int kMaxItems = TW == 2 ? 1 : TW == kResTileWaves ? (NP == 8 && !STATIC && !RAG ? 1 : kResMaxItems) : (TW == kResLongWaves ? kResMaxItems : 2);
     if (RAG && items == 4) items = 5;
     if (items < kMinItems) items = kMinItems;
 #define MHC_RES_ITEMS(N)                                                                              \
@@ -499,8 +499,12 @@ static hipError_t launch_items(const BwdResidentArgs &ra, hipStream_t stream) {
     // 22.3; n=8 B=600 C=768 ten 23.9, seven 18.0.
     if constexpr (NP == 8 && !STATIC) {
         const int C = ra.r.C;
+        if (C <= 256) return launch_items_tw<NP, WMODE, F32, STATIC, 2>(ra, stream);
         if ((C > 896 && C <= 1280) || C > 1792) return launch_items_tw<NP, WMODE, F32, STATIC, 10>(ra, stream);
         if (C > 512) return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves>(ra, stream);
+    }
+    if constexpr (NP == 4) {
+        if (ra.r.C <= 256) return launch_items_tw<NP, WMODE, F32, STATIC, 2>(ra, stream);
     }
     // Four streams: a fifth tile wave where it saves every wave an item (rows of 513..640 and 1025..1280
     // channels: ten 128-channel chunks are 3 + 3 + 2 + 2 on four waves, 2 each on five).  B=320, C=1280,

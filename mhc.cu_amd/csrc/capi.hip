@@ -62,7 +62,7 @@ int ws_check(void *ws, size_t have, size_t need) {
 
 // ---- dynamic workspace layout ----------------------------------------------------------------
 struct DynFwdWs { float *Ppart, *ssqpart, *agg; size_t bytes; };
-struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *dtpart, *raw, *s1part, *dx_part, *dphi_part; unsigned short *dPb, *dPT; int BP; size_t bytes; };
+struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, *dx_part, *dphi_part; unsigned short *dPb, *dPT; int BP; size_t bytes; };
 
 // Whether the sample-resident backward (bwd_resident.hip + the column-slab kernel without batch split)
 // is taken where it is supported.  Its second launch walks all samples of a column slab in one
@@ -72,14 +72,12 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *dtpart, *raw, *s1part, *dx_part
 //               1024 29.8 -> 29.6, 1536 35.7 -> 39.4, 2560 46.2 -> 62.5;  n=4 C=2048: B=768 33.5 -> 30.3, 1024 35.1 -> 41.2
 //   n=4 C=2560: B=256 23.9 -> 17.8, 512 32.0 -> 26.9, 768 36.3 -> 35.9, 1280 42.4 -> 53.9;  n=2 C=1280: B=1024 23.7 -> 28.8
 //   n=8 C=1280: B=128 25.1 -> 16.9, 256 30.5 -> 22.0, 512 46.1 -> 36.1, 1024 77.3 -> 62.7
-// n = 5 .. 8 with short rows and a large batch: few column slabs walk many samples, and the tiled path, which splits
-// the batch, wins.  Backward kernels, tiled -> resident (us):
-//   n=8 C=256: B=2048 56.7 -> 63.0, 6000 118.5 -> 166.9;  C=512: B=1100 53.8 -> 45.3, 2048 70.5 -> 68.5, 6000 168.3 -> 188.8
-//   n=5 C=384: B=3000 75.3 -> 81.9;  n=6 C=320: B=6000 125.0 -> 153.1
+// n = 5 .. 8 at every batch size (backward kernels, tiled -> resident with the batch split of its second launch, us):
+//   n=8 C=256: B=6000 118 -> 105;  C=512: B=2048 71 -> 56, 6000 168 -> 149;  n=5 C=384: B=3000 76 -> 61
 // Experiment hook: 1 = never, 2 = always.
 bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;
-    if (n > 4) return !(C <= 512 && B >= 5 * C);
+    if (n > 4) return true;
     return B <= 768;
 }
 
@@ -143,6 +141,9 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     if (bs4 > bs) bs = bs4;
     const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1;
     if (bs5 > bs) bs = bs5;
+    const int bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
+    if (bs6 > bs) bs = bs6;
+    w.upart = c.floats(bs6 > 1 ? (size_t)proj_bwd_addx_sum_parts(B, bs6) * C : 0);
     w.dphi_part = c.floats(bs > 1 ? (size_t)bs * D * nC : 0);
     w.BP = (B + 31) / 32 * 32;
     w.dPb = reinterpret_cast<unsigned short *>(c.floats(((size_t)w.BP * padded_D(n) + 1) / 2));
@@ -629,13 +630,25 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         out2.dP = nullptr;  // the second launch takes dP as matrix-core operands only
         MHC_LAUNCH(launch_bwd_resident(dy, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, q, P, r, alpha, bias + 2 * n,
                                        sk_state, out2, dx, df, ws.u, B, n, C, iters, eps, st));
-        const BatchSumArgs sums = make_batch_sums(ws.u, B, C, f_inject ? DwOut{} : dw, ws.dt, B, D, dbias, dalpha);
+        const DwOut dwo = f_inject ? DwOut{} : dw;
+        const int S = proj_bwd_addx_splits(B, n, C), parts = proj_bwd_addx_sum_parts(B, S);
         bool tail_taken = false;
-        MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, dphi, dx, B, n, C,
+        if (S > 1) {
+            // partial sums of dphi, dw, dbias and dalpha, added up by one more launch
+            const BatchSumArgs sums = make_batch_sums(ws.u, B, C, dwo ? DwOut{ws.upart, false} : dwo, ws.dt, B, D, ws.dtpart,
+                                                      ws.dtpart + D);
+            MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, ws.dphi_part, S, dx, B, n, C, &sums,
+                                            &tail_taken, st));
+            if (!tail_taken) return MHC_ERR_LAUNCH;  // not reached: any number of workgroups can carry the parts
+            MHC_LAUNCH(launch_finalize(ws.upart, parts, C, dwo, ws.dtpart, parts, D, dbias, dalpha, ws.dphi_part, S,
+                                       (size_t)D * n * C, dphi, st));
+            return MHC_OK;
+        }
+        const BatchSumArgs sums = make_batch_sums(ws.u, B, C, dwo, ws.dt, B, D, dbias, dalpha);
+        MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, dphi, 1, dx, B, n, C,
                                         tuning_get(kTuneSeparateFinalize) == 1 ? nullptr : &sums, &tail_taken, st));
         if (!tail_taken)
-            MHC_LAUNCH(launch_finalize(ws.u, B, C, f_inject ? DwOut{} : dw, ws.dt, B, D, dbias, dalpha, nullptr, 1,
-                                       0, nullptr, st));
+            MHC_LAUNCH(launch_finalize(ws.u, B, C, dwo, ws.dt, B, D, dbias, dalpha, nullptr, 1, 0, nullptr, st));
         return MHC_OK;
     }
     if (x_dtype == kF32AsBF16) return MHC_ERR_BAD_DTYPE;  // not reached: accepted shapes take the path above

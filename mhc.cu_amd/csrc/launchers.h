@@ -248,8 +248,12 @@ hipError_t launch_bwd_resident_static(const void *dy, const void *x, const void 
 // dphi = dP^T x_flat without batch split, dx completed in place (dx = dxp + dP phi - cx x), and `tail`
 // (dw, dbias, dalpha) summed by extra workgroups when the grid has room (*tail_taken).
 bool proj_bwd_addx_supported(int n);
+// batch splits S: with more than one, dphi holds S planes [D, nC] and the outputs of `tail` (fp32) proj_bwd_addx_sum_parts()
+// rows ([C] and [D + 3]) of partial sums
+int proj_bwd_addx_splits(int B, int n, int C);
+int proj_bwd_addx_sum_parts(int B, int S);
 hipError_t launch_proj_bwd_addx(const void *x, int x_dtype, const void *phi, const void *dPb, const void *dPT, int BP,
-                                const float *cx, float *dphi, void *dx, int B, int n, int C, const BatchSumArgs *tail,
+                                const float *cx, float *dphi, int S, void *dx, int B, int n, int C, const BatchSumArgs *tail,
                                 bool *tail_taken, hipStream_t stream);
 // n <= 18: whether the two products are faster apart (measured: from D > 128 on)
 bool proj_bwd_products_apart(int n);

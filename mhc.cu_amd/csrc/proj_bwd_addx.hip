@@ -36,13 +36,20 @@ struct ProjAddxArgs {
     const bf16_t *dPb;   // dP, fragment-major (frag_dpb); columns >= D are zero
     const bf16_t *dPT;   // dP^T hi and lo bf16 planes, fragment-major (frag_dpt); rows >= D, columns >= B zero
     const float *cx;     // [B]
-    float *dphi;         // [D][nC]
+    float *dphi;         // [D][nC], one such plane per batch split
     void *dx;            // [B][nC]: in dxp, out dx; stored like x
     int B, BP, D, DP, nC;
-    int tail_row;        // blockIdx.y of the workgroups that compute `tail` (-1: none)
+    int per_split;       // samples of a batch split (whole blocks); blockIdx.y < splits
+    int tail_row;        // first blockIdx.y of the workgroups that compute `tail` (-1: none)
+    int tail_rows;       // samples per workgroup of the tail (all of them, or a part with partial sums as the result)
+    int tail_parts;
     BatchSumArgs tail;
 };
 
+// Columns per workgroup of the batch sums: 16 leave sixteen row groups in four waves (a walk of 1000 samples is 4
+// rounds of loads; with 64 columns and four groups it was 16, longer than the slabs': B=789 n=8 C=1984 30.1 -> 27.0 us)
+constexpr int kAxSumCols = 16;
+constexpr int kAxSumRows = 128;    // samples per part of the sums beside a split batch
 constexpr int kAxKW = 32;          // slab width (columns)
 constexpr int kAxLD = kAxKW + 8;   // LDS pitch of the bf16 tiles (elements): rows stay 16-byte aligned
 constexpr int kAxLDO = kAxKW + 4;  // LDS pitch of the fp32 tile of dP phi
@@ -56,7 +63,9 @@ constexpr int kAxLDR = 36;         // LDS pitch of the dphi tiles in the final c
 // the bf16 storage case; dxp is read and dx written as fp32).
 // NW: waves per workgroup (a block is NW * SPW samples).
 // RAG: rows of any length (nC % 8 != 0): the last chunk of a row is loaded from nC - 8 on and shifted down.
-template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false>
+// SPLIT: blockIdx.y is a batch split (a template argument: with a run-time first sample the compiler keeps fewer
+// loads in flight, B=1000 n=6 C=1024 17.2 -> 21.2 us without any split).
+template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel(ProjAddxArgs a) {
     constexpr int NT_ = 64 * NW;  // threads
     using TS = typename std::conditional<F32, float, bf16_t>::type;
@@ -70,9 +79,21 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
     float *o_s = reinterpret_cast<float *>(x_s + (size_t)SBR * kAxLD);    // [SBR][LDO]
     float *red_s = reinterpret_cast<float *>(ax_smem);                    // final sum: [NW][NTD][32][LDR], over everything
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if ((int)blockIdx.y == a.tail_row) {
-        // the extra row of the grid: its first workgroups do the batch sums, the others have nothing to do
-        if ((int)blockIdx.x < a.tail.nblk) batch_sum_block<NW>(a.tail, blockIdx.x, tid, reinterpret_cast<double *>(ax_smem));
+    if (a.tail_row >= 0 && (int)blockIdx.y >= a.tail_row) {
+        // the extra rows of the grid: the first workgroups do the batch sums, the others have nothing to do
+        const int id = ((int)blockIdx.y - a.tail_row) * (int)gridDim.x + (int)blockIdx.x, part = id / a.tail.nblk;
+        if (part >= a.tail_parts) return;
+        BatchSumArgs s = a.tail;
+        const int r0 = part * a.tail_rows, rows = min(a.tail_rows, a.B - r0);
+        s.rows_u = s.rows_dt = rows;
+        s.u += (size_t)r0 * s.C;
+        s.dt += (size_t)r0 * (s.D + 3);
+        if (a.tail_parts > 1) {  // fp32 rows, added up by the launch that follows
+            s.dw = s.dw ? static_cast<float *>(s.dw) + (size_t)part * s.C : nullptr;
+            s.dbias += (size_t)part * (s.D + 3);
+            s.dalpha += (size_t)part * (s.D + 3);
+        }
+        batch_sum_block<NT_ / kAxSumCols, kAxSumCols>(s, id % s.nblk, tid, reinterpret_cast<double *>(ax_smem));
         return;
     }
     // Workgroup ids go round robin over the 8 XCDs (each with its own L2, 128-byte lines).  A slab
@@ -82,7 +103,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
     const int k0 = slab * kAxKW;
     if (k0 >= a.nC) return;  // ids of the padded grid; the whole workgroup, before any barrier
     const int row = lane & 31, kg = lane >> 5;
-    const int D = a.D, nC = a.nC, B = a.B;
+    const int D = a.D, nC = a.nC, b_begin = SPLIT ? (int)blockIdx.y * a.per_split : 0, B = SPLIT ? min(a.B, b_begin + a.per_split) : a.B;  // the split's samples
     const int pwg = slab;
     (void)pwg;
     MHC_PHASE_ZERO(kPhaseColSlab, pwg);
@@ -183,11 +204,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         const uint4 v = ldg16<RAG>(a.phi + (ok ? (size_t)d * nC + kl - kls : 0));
         phir[u] = make_uint4(ok ? v.x : 0u, ok ? v.y : 0u, ok ? v.z : 0u, ok ? v.w : 0u);
     }
-    load_block(0, Slot0{});
-    load_ops(0, ops[0]);
-    if (SBR < B) {
-        load_block(SBR, Slot1{});
-        if constexpr (PFOP) load_ops(SBR, ops[1]);
+    load_block(b_begin, Slot0{});
+    load_ops(b_begin, ops[0]);
+    if (b_begin + SBR < B) {
+        load_block(b_begin + SBR, Slot1{});
+        if constexpr (PFOP) load_ops(b_begin + SBR, ops[1]);
     }
 #pragma unroll
     for (int u = 0; u < (PCH + NT_ - 1) / NT_; u++) {
@@ -208,7 +229,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         Ops &op = ops[PFOP ? S : 0];
         constexpr int P = PS == 2 ? S : 0;
         if constexpr (PS == 1) load_prev(sb);
-        if (sb != 0) {
+        if (sb != b_begin) {
             if constexpr (!PFOP) load_ops(sb, op);
             __syncthreads();  // every wave is done with the previous block's tile
         }
@@ -290,11 +311,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         }
         MHC_PHASE_ADD(kPhaseColSlab, pwg, 3, pclk);
     };
-    for (int sb = 0; sb < B; sb += 2 * SBR) {
+    for (int sb = b_begin; sb < B; sb += 2 * SBR) {
         process_block(sb, Slot0{});
         if (sb + SBR < B) process_block(sb + SBR, Slot1{});
     }
 
+    float *dphi = a.dphi + (SPLIT ? (size_t)blockIdx.y * D * nC : 0);
     // ---- dphi: sum the four waves' shares through LDS, store row-major --------------------------------
     __syncthreads();  // all tiles consumed; the memory becomes red_s
 #pragma unroll
@@ -314,9 +336,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         if (d < D && k0 + c < nC) {
             if constexpr (RAG) {
                 const float out[4] = {s.x, s.y, s.z, s.w};
-                store_vec_any<float, 4>(a.dphi + (size_t)d * nC + k0 + c, out, nC - (k0 + c));
+                store_vec_any<float, 4>(dphi + (size_t)d * nC + k0 + c, out, nC - (k0 + c));
             } else {  // k0 % 32 == 0: a quad of columns is inside or outside
-                *reinterpret_cast<float4 *>(a.dphi + (size_t)d * nC + k0 + c) = s;
+                *reinterpret_cast<float4 *>(dphi + (size_t)d * nC + k0 + c) = s;
             }
         }
     }
@@ -325,33 +347,62 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 
 bool proj_bwd_addx_supported(int n) { return padded_D(n) / 32 <= 3; }
 
-template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false>
+template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false, bool SPLIT = false>
 static hipError_t launch_addx(const ProjAddxArgs &a, hipStream_t stream) {
+    if constexpr (NW == 4 && !SPLIT) {
+        if (a.per_split < a.B) return launch_addx<NTD, SPW, PFOP, F32, NW, RAG, true>(a, stream);
+    }
     if constexpr (!F32 && !RAG) {
-        if (a.nC % 8 != 0) return launch_addx<NTD, SPW, PFOP, F32, NW, true>(a, stream);
+        if (a.nC % 8 != 0) return launch_addx<NTD, SPW, PFOP, F32, NW, true, SPLIT>(a, stream);
     }
     constexpr int SBR = NW * SPW;
     const size_t tiles = sizeof(bf16_t) * (size_t)kAxLD * (32 * NTD + SBR) + sizeof(float) * SBR * kAxLDO;
     const size_t red = sizeof(float) * NW * NTD * 32 * kAxLDR;  // the final cross-wave sum reuses the tiles' memory
     const size_t smem = tiles > red ? tiles : red;
-    hipError_t e = allow_dynamic_lds<&proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG>>(smem);
+    hipError_t e = allow_dynamic_lds<&proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG, SPLIT>>(smem);
     if (e != hipSuccess) return e;
     const int slabs = (a.nC + kAxKW - 1) / kAxKW;
-    dim3 grid(round_up(slabs, 16), 1 + (a.tail_row >= 0 ? 1 : 0));
-    proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG><<<grid, 64 * NW, smem, stream>>>(a);
+    dim3 grid(round_up(slabs, 16), (a.B + a.per_split - 1) / a.per_split + (a.tail_row >= 0 ? (a.tail.nblk * a.tail_parts + round_up(slabs, 16) - 1) / round_up(slabs, 16) : 0));
+    proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG, SPLIT><<<grid, 64 * NW, smem, stream>>>(a);
     return hipGetLastError();
 }
 
+// Short rows make few slabs, and one workgroup of each then walks a large batch by itself.  Where the walk is long
+// and the slabs leave room for it (two workgroups per CU), the batch is split and the finalize launch adds up the
+// partial dphi (kernels us, one workgroup per slab -> split with
+// its finalize launch: n=8 B=6000 C=256 94.9 -> 30.2, B=2048 C=512 36.0 -> 22.9; float32 storage n=4 B=6835 C=320
+// 91.2 -> 34.7, B=2560 C=1280 41.0 -> 38.6).
+int proj_bwd_addx_splits(int B, int n, int C) {
+    const int slabs = (n * C + kAxKW - 1) / kAxKW, D = n * n + 2 * n;
+    const int walk = padded_D(n) == 32 && slabs <= 256 ? (B + 383) / 384 : (B + 127) / 128;  // blocks without a split
+    int S = 512 / slabs, blocks = (B + 127) / 128;
+    if (S > blocks / 2) S = blocks / 2;
+    // the partial copies (written and read once) stay below half of the activation bytes of this launch
+    const int cap = (int)(0.375 * B / D);
+    if (S > cap) S = cap;
+    // (one launch more: B=2000 n=8 C=1024, walk 16, S = 2 40.2 -> 39.3; B=1000 n=6 C=1024, walk 8 17.9 -> 21.6)
+    if (S < 2 || walk < (S == 2 ? 20 : (padded_D(n) == 32 ? 5 : 10))) return 1;
+    const int per = (blocks + S - 1) / S;  // blocks of the longest split
+    return (blocks + per - 1) / per;
+}
+
+// Parts of the batch sums beside a split batch: a workgroup per 64 columns that walks thousands of samples would be
+// the longest of the launch (B=6835 n=4 C=320: 66 us, the split slabs 30).
+int proj_bwd_addx_sum_parts(int B, int S) { return S > 1 ? (B + kAxSumRows - 1) / kAxSumRows : 1; }
+
 hipError_t launch_proj_bwd_addx(const void *x, int x_dtype, const void *phi, const void *dPb, const void *dPT, int BP,
-                                const float *cx, float *dphi, void *dx, int B, int n, int C, const BatchSumArgs *tail,
-                                bool *tail_taken, hipStream_t stream) {
+                                const float *cx, float *dphi, int S, void *dx, int B, int n, int C,
+                                const BatchSumArgs *tail, bool *tail_taken, hipStream_t stream) {
     const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n), NTD = DP / 32;
     ProjAddxArgs a{x, static_cast<const bf16_t *>(phi), static_cast<const bf16_t *>(dPb),
-                   static_cast<const bf16_t *>(dPT), cx, dphi, dx, B, BP, D, DP, nC, -1, {}};
+                   static_cast<const bf16_t *>(dPT), cx, dphi, dx, B, BP, D, DP, nC, S > 1 ? ((B + 127) / 128 + S - 1) / S * 128 : B, -1, B, 1, {}};
     if (tail_taken) *tail_taken = false;
-    if (tail && tail->nblk <= round_up((nC + kAxKW - 1) / kAxKW, 16)) {
+    if (tail) {
         a.tail = *tail;
-        a.tail_row = 1;
+        a.tail.nblk = ((tail->dw ? C : 0) + D + 3 + kAxSumCols - 1) / kAxSumCols;
+        a.tail_row = S;
+        a.tail_parts = proj_bwd_addx_sum_parts(B, S);
+        if (a.tail_parts > 1) a.tail_rows = kAxSumRows;
         if (tail_taken) *tail_taken = true;
     }
     const bool f32 = x_dtype == kF32AsBF16;
@@ -363,7 +414,7 @@ hipError_t launch_proj_bwd_addx(const void *x, int x_dtype, const void *phi, con
     // More than 256 slabs: workgroups of four waves, of which three fit a CU, keep the grid in one round
     // (B=1280, C=2560, n=4: 24.4 us with 4 waves, 31.7 with 12).
     int nw = 4;
-    if (NTD == 1 && (nC + kAxKW - 1) / kAxKW <= 256) {
+    if (S == 1 && NTD == 1 && (nC + kAxKW - 1) / kAxKW <= 256) {
         int best = (B + 127) / 128;
         if ((B + 255) / 256 < best) { nw = 8; best = (B + 255) / 256; }
         if ((B + 383) / 384 < best) nw = 12;
