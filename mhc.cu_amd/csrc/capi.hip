@@ -730,7 +730,7 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
                                                  kProjPartDphi, tail, &tail_taken));
             if (tail_taken) return MHC_OK;
         }
-    } else if (gemm_f32_supported(x_dtype, phi_dtype, n, C)) {
+    } else if (dx_dphi_f32_supported(x_dtype, phi_dtype, n, C)) {
         // exact float32 tier, wide projection: both products on the fp32 matrix cores; the projection
         // term of dx is written into dx and completed in place
         MHC_LAUNCH(launch_gemm_f32_dxflat(ws.dP, static_cast<const float *>(phi), static_cast<float *>(dx), B, n, C, st));

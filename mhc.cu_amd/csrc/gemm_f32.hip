@@ -64,7 +64,9 @@ __device__ __forceinline__ void park_kc(const Slice &s, float *Xs, int tid) {
 
 // Row-contiguous operand, element (r, k) at P[k * ld + r]: thread = float4 (tid & 31) of k-rows
 // (tid >> 5) + 8 j.  float4s that start at or beyond R alias the tile's first one (never stored);
-// k-rows >= K are zeroed.  The k-row pitch must cover R rounded up to 4.
+// k-rows >= K are zeroed.  The k-row pitch must cover R rounded up to 4, except with RAG (rows of any length, R >= 4):
+// there the float4 that straddles the row's end is read from R - 4 on and shifted down.
+template <bool RAG>
 __device__ __forceinline__ void load_rc(Slice &s, const float *P, long long ld, int r0, int R, int k0,
                                         int K, int tid) {
     const int q = tid & 31;
@@ -72,7 +74,16 @@ __device__ __forceinline__ void load_rc(Slice &s, const float *P, long long ld, 
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int k = k0 + (tid >> 5) + 8 * j;
-        float4 t = *reinterpret_cast<const float4 *>(P + (size_t)(k < K ? k : 0) * ld + r);
+        float4 t;
+        if constexpr (RAG) {
+            const int rr = min(r, R - 4);
+            const uint4 u = ldg16_any(P + (size_t)(k < K ? k : 0) * ld + rr);
+            uint32_t w[4] = {u.x, u.y, u.z, u.w};
+            drop_elems<4>(w, r - rr);
+            t = make_float4(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]), __uint_as_float(w[3]));
+        } else {
+            t = *reinterpret_cast<const float4 *>(P + (size_t)(k < K ? k : 0) * ld + r);
+        }
         if (k >= K) t = make_float4(0.f, 0.f, 0.f, 0.f);
         s.v[j] = t;
     }
@@ -84,7 +95,7 @@ __device__ __forceinline__ void park_rc(const Slice &s, float *Xs, int tid) {
 }
 
 // AK / BK: the operand's contiguous index is k.  grid: (N tiles, M tiles, splits)
-template <bool AK, bool BK>
+template <bool AK, bool BK, bool RAG = false>
 __global__ __launch_bounds__(256, kMfmaMinWaves) void gemm_f32_kernel(GemmArgs a) {
     __shared__ __align__(16) float As[kGK * kGLD];
     __shared__ __align__(16) float Bs[kGK * kGLD];
@@ -107,9 +118,9 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void gemm_f32_kernel(GemmArgs a
     Slice sa, sb;
     auto fetch = [&](int k0) {
         if constexpr (AK) load_kc(sa, a.A, a.lda, m0, a.M, k0, kend, tid);
-        else load_rc(sa, a.A, a.lda, m0, a.M, k0, kend, tid);
+        else load_rc<false>(sa, a.A, a.lda, m0, a.M, k0, kend, tid);
         if constexpr (BK) load_kc(sb, a.B, a.ldb, n0, a.N, k0, kend, tid);
-        else load_rc(sb, a.B, a.ldb, n0, a.N, k0, kend, tid);
+        else load_rc<RAG>(sb, a.B, a.ldb, n0, a.N, k0, kend, tid);
     };
     fetch(kbeg);
     for (int k0 = kbeg; k0 < kend; k0 += kGK) {
@@ -181,10 +192,13 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void dphi_f32_kernel(const floa
                                                        int per_wave /* samples, even */) {
     extern __shared__ __align__(16) float lds[];  // [4 waves][NT * CPL * 16][64]
     constexpr int U = 8;                          // products (pairs of samples) in flight
-    typedef float vec_t __attribute__((ext_vector_type(CPL)));
+    typedef float vec_t __attribute__((ext_vector_type(CPL), aligned(4)));  // rows of any length start at any element
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 31, h = lane >> 5;
     const int col = blockIdx.x * 32 * CPL + CPL * l;
-    const float *xc = x + (col < nC ? col : 0);  // nC % 4 == 0: a lane's columns are all inside or all outside
+    // the lane at the end of a row that is no multiple of CPL takes the last CPL columns: some of them twice, with
+    // the same result
+    const int cl = col < nC ? min(col, nC - CPL) : 0;
+    const float *xc = x + cl;
     const float *pc = dP + l;
     const int b0 = (blockIdx.z * 4 + wave) * per_wave, b1 = min(B, b0 + per_wave);
 
@@ -234,7 +248,7 @@ __global__ __launch_bounds__(256, kMfmaMinWaves) void dphi_f32_kernel(const floa
 #pragma unroll
             for (int i = 0; i < 16; i++) lds[((size_t)wave * R + (t * CPL + c) * 16 + i) * 64 + lane] = acc[t][c][i];
     __syncthreads();
-    float *o = out + (size_t)blockIdx.z * D * nC + col;
+    float *o = out + (size_t)blockIdx.z * D * nC + cl;
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -282,10 +296,15 @@ hipError_t launch_dphi_f32(const float *dP, const float *x, float *out, int S, i
     return hipGetLastError();
 }
 
-template <bool AK, bool BK> static hipError_t launch_gemm(const GemmArgs &a, int splits, hipStream_t stream) {
+template <bool AK, bool BK, bool RAG = false> static hipError_t launch_gemm(const GemmArgs &a, int splits, hipStream_t stream) {
     dim3 grid((a.n_store + kGT - 1) / kGT, (a.M + kGT - 1) / kGT, splits);
-    gemm_f32_kernel<AK, BK><<<grid, 256, 0, stream>>>(a);
+    gemm_f32_kernel<AK, BK, RAG><<<grid, 256, 0, stream>>>(a);
     return hipGetLastError();
+}
+
+// n <= 8: the projection term of dx and dphi take rows of any length
+bool dx_dphi_f32_supported(int x_dtype, int phi_dtype, int n, int C) {
+    return x_dtype == kF32 && phi_dtype == kF32 && (n <= 8 || (n * C) % 4 == 0) && n * C >= 256;
 }
 
 bool gemm_f32_supported(int x_dtype, int phi_dtype, int n, int C) {
@@ -299,8 +318,6 @@ int gemm_f32_proj_ksplit(int B, int n, int C, int max_splits) {
     const int cap = nC / (8 * kGK);  // at least 8 slices per split
     if (ks > cap) ks = cap;
     if (ks > max_splits) ks = max_splits;
-    // n <= 8: the fused forward kernel sums at most 24 splits (16 for rows longer than 2048) in its one round of loads
-    if (n <= 8 && ks > (C <= 2048 ? 24 : 16)) ks = C <= 2048 ? 24 : 16;
     if (ks < 1) ks = 1;
     // whole slices per split; drop the splits that would get none
     const int kps = ((nC + ks - 1) / ks + kGK - 1) / kGK * kGK;
@@ -326,6 +343,7 @@ hipError_t launch_gemm_f32_dxflat(const float *dP, const float *phi, float *dxfl
                                   hipStream_t stream) {
     const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n);
     GemmArgs a{dP, phi, dxflat, B, nC, D, DP, nC, nC, nC, (D + kGK - 1) / kGK * kGK, 0, nullptr};
+    if (nC % 4 != 0) return launch_gemm<true, false, true>(a, 1, stream);
     return launch_gemm<true, false>(a, 1, stream);
 }
 

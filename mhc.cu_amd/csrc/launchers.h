@@ -114,6 +114,7 @@ hipError_t launch_layer_fwd_onepass(const void *x, const void *w, int w_dtype, c
                                     float *sk_state, int B, int n, int C, int T, float eps, hipStream_t stream);
 
 // fp32 matrix-core GEMMs of the exact float32 tier (wide projections): see gemm_f32.hip.
+bool dx_dphi_f32_supported(int x_dtype, int phi_dtype, int n, int C);
 bool gemm_f32_supported(int x_dtype, int phi_dtype, int n, int C);
 int gemm_f32_proj_ksplit(int B, int n, int C, int max_splits);
 hipError_t launch_gemm_f32_proj(const float *x, const float *phi, float *Ppart, float *ssqpart, int KS,
