@@ -167,11 +167,11 @@ constexpr int kFwdStaggerMinB = 512;  // two or more workgroups per CU
 // shifted down behind the barrier.  A template argument: as a run-time switch the clamps and compares cost the
 // whole rows 4 % (B=3001 n=4 C=2560: 27.4 -> 28.5 us).
 template <typename TX, typename TY, int NP, int V, int CPT, bool RX = false, bool RAG = false>
-__global__ __launch_bounds__(256, (CPT == (NP == 4 ? 2 : 1) && !std::is_same<TX, float>::value) ? 4 : kMfmaMinWaves)
+__global__ __launch_bounds__((NP == 8 && std::is_same<TX, float>::value) ? 512 : 256, (CPT == (NP == 4 ? 2 : 1) && !std::is_same<TX, float>::value) ? 4 : kMfmaMinWaves)
 void layer_fwd_small_kernel(LayerFwdArgs a) {
     using SK = SkSmall<NP>;
     __shared__ float coef_s[NP * NP + 2 * NP];  // M | Hpre | Hpost
-    __shared__ float red[4];
+    __shared__ float red[8];
     const int b = blockIdx.x, n = a.n, C = a.C, tid = threadIdx.x;
     const int nt = blockDim.x;  // whole waves, as few as hold the sample's chunks (see launch_fused_small)
     const TX *__restrict__ xb = static_cast<const TX *>(a.x) + (size_t)b * n * C;
@@ -191,7 +191,7 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
     // LDS); the coefficient step itself runs on the first group.
     constexpr int kSplitWaves = SK::kPerWave == 1 ? 4 : 1;  // at most
     __shared__ float psum_s[kSplitWaves == 4 ? 4 * 3 * 64 : 1];
-    const int g = tid % SK::kGroup, parts = kSplitWaves == 4 ? nt / kWave : 4, part = (tid / SK::kGroup) % parts;
+    const int g = tid % SK::kGroup, parts = kSplitWaves == 4 ? min(nt / kWave, kSplitWaves) : 4, part = (tid / SK::kGroup) % parts;
     const int D = n * n + 2 * n;
     const int r0 = SK::row(g), c0 = SK::col0(g);
     const bool mv = r0 < n && c0 < n, vv = g < 2 * n;
@@ -638,11 +638,13 @@ static bool launch_fused_small(const LayerFwdArgs &a, hipStream_t stream, hipErr
     // the split sums, four take them where fewer would need a second round of loads
     // Always 256 threads -> as few as needed, with 128 registers (kernel us): n=5 B=3000 C=1024 33.1 -> 20.0,
     // n=8 B=6000 C=512 64.1 -> 22.5, n=6 B=2000 C=384 24.5 -> 10.2, n=8 B=789 C=1984 18.2 -> 14.0 (registers only).
-    const int per = cpt == 3 ? 4 : cpt;  // chunks per thread of the instantiation that runs
+    // (fp32 rows of more than 2048 channels: 8 x 8 takes up to 512 threads, 4 x 4 four chunks per thread)
+    const int per = NP == 8 ? (cpt < 2 ? cpt : 2) : (cpt == 3 ? 4 : cpt);  // chunks per thread of the instantiation that runs
     int nt = round_up((nch + per - 1) / per, kWave);
     if (NP == 8 && a.KS > fwd_splits_in_one_round(8, per) / 4 * (nt / kWave)) nt = 256;
+    constexpr int kMost = NP == 8 && std::is_same<TX, float>::value ? 4 : 2;  // 256-thread rounds of chunks with two per thread
     if (cpt == 1) layer_fwd_small_kernel<TX, TY, NP, V, 1, RX, RAG><<<a.B, nt, 0, stream>>>(a);
-    else if (cpt == 2) layer_fwd_small_kernel<TX, TY, NP, V, 2, RX, RAG><<<a.B, nt, 0, stream>>>(a);
+    else if (cpt == 2 || (NP == 8 && cpt <= kMost)) layer_fwd_small_kernel<TX, TY, NP, V, 2, RX, RAG><<<a.B, nt, 0, stream>>>(a);
     else if (cpt <= 4 && NP == 4) layer_fwd_small_kernel<TX, TY, 4, V, 4, RX, RAG><<<a.B, nt, 0, stream>>>(a);
     else return false;
     *err = hipGetLastError();
@@ -654,7 +656,7 @@ bool layer_fwd_fused_supported(int n, int C, int x_dtype) {
     const int V = x_dtype == kBF16 ? 8 : 4;
     if (C < V) return false;
     const int cpt = ((C + V - 1) / V + 255) / 256;
-    return cpt <= 2 || (cpt <= 4 && n <= 4);
+    return cpt <= 2 || (cpt <= 4 && (n <= 4 || V == 4));
 }
 
 hipError_t launch_layer_fwd_fused(const void *x, int x_dtype, const void *w, int w_dtype,
