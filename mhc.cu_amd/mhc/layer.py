@@ -8,7 +8,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from .ops import _ext
+from .ops import _as_tensor, _ext
 
 # in the order of the operators' arguments
 _DYNAMIC_PARAMS = ("rmsnorm_weight", "phi_pre", "phi_post", "phi_res", "alpha_pre", "alpha_post", "alpha_res",
@@ -75,13 +75,16 @@ class MHCLayer(nn.Module):
         try:
             return [p[k] for k in names]
         except KeyError:
-            return [getattr(self, k) for k in names]
+            # (an alpha may also have been replaced by a plain number)
+            return [_as_tensor(getattr(self, k), self.phi_pre) if k.startswith("alpha") else getattr(self, k) for k in names]
 
     def forward(self, x_expanded: torch.Tensor) -> torch.Tensor:
         B, n, C = x_expanded.shape
         assert n == self.expansion_rate
         assert C == self.hidden_dim
         compute = self.compute_dtype
+        # (a configuration file hands over 20.0 or "1e-5")
+        iters, eps = int(self.sinkhorn_iters), float(self.eps)
         cast = compute is not None and x_expanded.dtype != compute
         if self.use_dynamic_h:
             # float32 activations with compute_dtype=bfloat16: the operator rounds them inside its kernels
@@ -89,11 +92,11 @@ class MHCLayer(nn.Module):
             in_op = cast and compute == torch.bfloat16 and x_expanded.dtype == torch.float32
             if cast and not in_op:
                 x_expanded = x_expanded.to(compute)
-            return _ext.mhc_layer_dynamic(x_expanded, *self._params(_DYNAMIC_PARAMS), self.sinkhorn_iters, self.eps,
+            return _ext.mhc_layer_dynamic(x_expanded, *self._params(_DYNAMIC_PARAMS), iters, eps,
                                           self.output_dtype, None, in_op)
         if cast:
             x_expanded = x_expanded.to(compute)
         params = self._params(_STATIC_PARAMS)
         if not self.training and not torch.is_grad_enabled():
-            return _ext.mhc_layer_inference(x_expanded, *params, self.sinkhorn_iters, self.eps, self.output_dtype)
-        return _ext.mhc_layer_static(x_expanded, *params, self.sinkhorn_iters, self.eps, self.output_dtype, None)
+            return _ext.mhc_layer_inference(x_expanded, *params, iters, eps, self.output_dtype)
+        return _ext.mhc_layer_static(x_expanded, *params, iters, eps, self.output_dtype, None)
