@@ -92,8 +92,8 @@ Tensor workspace(const Tensor &like, size_t nbytes) {
 // A forward + backward of a small layer is bound by the host, so the two layers are autograd nodes of
 // their own (torch::autograd::Node) instead of torch::autograd::Function: no string-keyed dictionary of
 // saved values, no generic argument extraction and output wrapping; everything a call keeps sits in ONE
-// byte buffer, all parameter gradients in another, and the gradients handed back are tensors built
-// directly over that buffer's storage (nine narrow / select / reshape calls through the dispatcher cost
+// byte buffer, dphi in another and the small parameter gradients in a third, and the gradients handed back are
+// tensors built directly over those buffers' storage (nine narrow / select / reshape calls through the dispatcher cost
 // more than the backward's kernel launches).  B=320 C=1280 n=4, same box: forward + backward 126 -> 105 us,
 // of which about 75 are the engine's own (the hand-over to its device thread and back, about 4 us per leaf);
 // B=7 forward without gradients 19.8 -> 14.3 us.
@@ -104,7 +104,7 @@ inline Tensor byte_buffer(const Tensor &like, size_t bytes) {
     return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
 }
 
-// A contiguous tensor over part of `base`'s storage (base: a byte buffer, byte_off a multiple of the element size).
+// A contiguous tensor over part of `base`'s storage (base at offset 0, byte_off a multiple of the element size).
 Tensor over(const Tensor &base, at::ScalarType st, size_t byte_off, at::IntArrayRef sizes) {
     Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(base.storage()), base.key_set(),
                                                         c10::scalarTypeToTypeMeta(st));
@@ -287,12 +287,14 @@ struct MHCDynamicBackward final : public torch::autograd::Node {
         const Tensor dy = incoming_gradient(grads[0], x, y_type);
         Tensor dx = at::empty(x.sizes(), x.options());
         Tensor df = has_f ? at::empty(f.sizes(), f.options()) : Tensor();
-        // dphi [D, nC] | dbias [D] dalpha [3], fp32 | dw [C] in the weight's type where the library writes it
+        // dphi [D, nC], fp32; in a buffer of their own, so that keeping one of them does not keep dphi, the small ones:
+        // dbias [D] dalpha [3], fp32 | dw [C] in the weight's type where the library writes it
         const at::ScalarType dw_type = w_type == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
-        const size_t off_ba = align256((size_t)D * nC * 4), off_w = off_ba + align256((size_t)(D + 3) * 4);
-        Tensor g = byte_buffer(x, off_w + (size_t)C * 4);
-        char *gp = static_cast<char *>(g.data_ptr());
-        float *dphi = reinterpret_cast<float *>(gp), *dba = reinterpret_cast<float *>(gp + off_ba);
+        Tensor g = at::empty({D, nC}, x.options().dtype(at::kFloat));
+        const size_t off_w = align256((size_t)(D + 3) * 4);
+        Tensor gs = byte_buffer(x, off_w + (size_t)C * 4);
+        char *gp = static_cast<char *>(gs.data_ptr());
+        float *dphi = g.data_ptr<float>(), *dba = reinterpret_cast<float *>(gp);
         Tensor ws = workspace(x, mhc_layer_dynamic_workspace_bytes(B, n, C));
         check("mhc_layer_bwd_dynamic",
               mhc_layer_bwd_dynamic_dw(ptr(dy), dt(dy), ptr(x), x_code, ptr(w), has_w ? dt(w) : 0, v.phi, cd, v.ba, v.ba + D, ptr(f),
@@ -301,16 +303,16 @@ struct MHCDynamicBackward final : public torch::autograd::Node {
                                     (float)eps, ws.data_ptr(), (size_t)ws.numel(), stream_of(x)));
         variable_list out(12);
         if (task_should_compute_output(0)) out[0] = cast_to(dx, x_type);
-        if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(g, dw_type, off_w, {C}), w_type);
+        if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(gs, dw_type, off_w, {C}), w_type);
         if (has_f && task_should_compute_output(2)) out[2] = cast_to(df, f_type);
         const int64_t rows[3] = {n, n, (int64_t)n * n}, row0[3] = {0, n, 2 * n};
         for (int i = 0; i < 3; i++) {
             if (task_should_compute_output(3 + i))
                 out[3 + i] = cast_to(over(g, at::kFloat, (size_t)row0[i] * nC * 4, {rows[i], nC}), p_type[i]);
-            if (task_should_compute_output(6 + i)) out[6 + i] = cast_to(over(g, at::kFloat, off_ba + (size_t)(D + i) * 4, {}), p_type[3 + i]);
+            if (task_should_compute_output(6 + i)) out[6 + i] = cast_to(over(gs, at::kFloat, (size_t)(D + i) * 4, {}), p_type[3 + i]);
             if (task_should_compute_output(9 + i)) {
                 const at::IntArrayRef sizes = i < 2 ? at::IntArrayRef(rows[i]) : at::IntArrayRef(b_res_sizes);
-                out[9 + i] = cast_to(over(g, at::kFloat, off_ba + (size_t)row0[i] * 4, sizes), p_type[6 + i]);
+                out[9 + i] = cast_to(over(gs, at::kFloat, (size_t)row0[i] * 4, sizes), p_type[6 + i]);
             }
         }
         return out;
