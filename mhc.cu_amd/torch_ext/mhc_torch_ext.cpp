@@ -6,6 +6,7 @@
 // every mhc_* call below is the C ABI of include/mhc_hip.h.
 #include <torch/extension.h>
 
+#include <ATen/FuncTorchTLS.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/forward_grad.h>
@@ -13,6 +14,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 
+#include <array>
 #include <mutex>
 #include <unordered_map>
 
@@ -43,7 +45,8 @@ inline int dt(const Tensor &t) {
     if (t.scalar_type() == at::kBFloat16) return MHC_BF16;
     TORCH_CHECK(false, "mhc: unsupported dtype ", t.scalar_type(), ": the HIP library takes float32 or bfloat16");
 }
-inline bool is_act_dtype(const Tensor &t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
+inline bool is_act(at::ScalarType st) { return st == at::kFloat || st == at::kBFloat16; }
+inline bool is_act_dtype(const Tensor &t) { return is_act(t.scalar_type()); }
 
 inline void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
@@ -116,7 +119,10 @@ Tensor over(const Tensor &base, at::ScalarType st, size_t byte_off, at::IntArray
 
 inline Tensor cast_to(Tensor t, at::ScalarType st) { return t.scalar_type() == st ? t : t.to(st); }
 
-inline void refuse_forward_mode(std::initializer_list<const Tensor *> inputs) {
+// What torch::autograd::Function refuses by itself and a node of one's own does not: the function transforms
+// (vmap, grad, jvp ... of torch.func), whose wrapped tensors no kernel can read, and forward mode.
+inline void refuse_transforms(std::initializer_list<const Tensor *> inputs) {
+    if (const auto &tls = at::functorch::functorchTLSAccessor()) tls->checkSupportsCppAutogradFunction();
     // outside a dual level no tensor has a tangent (asking all of them costs a lock each, 1.5 us a call)
     if (!torch::autograd::ForwardADLevel::try_get_by_idx(0)) return;
     for (const Tensor *t : inputs)
@@ -136,6 +142,15 @@ Tensor incoming_gradient(const Tensor &g, const Tensor &x, at::ScalarType y_type
     if (!g.defined()) return at::zeros(x.sizes(), x.options().dtype(x.scalar_type() == at::kBFloat16 ? at::kBFloat16 : y_type));
     const bool round_dy = x.scalar_type() == at::kBFloat16 && g.scalar_type() == at::kFloat;
     return act(round_dy ? g.to(g.options().dtype(at::kBFloat16), false, false, at::MemoryFormat::Contiguous) : g);
+}
+
+// A saved tensor as the backward takes it; what a hook of torch.autograd.graph.saved_tensors_hooks handed back has to be
+// of the type and size that was saved.
+inline Tensor unpacked(const SavedVariable &v, at::ScalarType st, int64_t numel) {
+    const Tensor t = act(v.unpack());
+    TORCH_CHECK(t.scalar_type() == st && t.numel() >= numel,
+                "mhc: a saved-tensor hook changed the type or the size of a tensor saved for the backward");
+    return t;
 }
 
 template <typename N> std::shared_ptr<N> make_node(torch::autograd::edge_list &&edges) {
@@ -257,7 +272,8 @@ struct DynViews {
 
 struct MHCDynamicBackward final : public torch::autograd::Node {
     SavedVariable x_, w_, f_, kept_, phi_, ba_;  // phi_, ba_: only with the parameter cache
-    bool has_w = false, has_f = false, cached = false, released = false, for_backward = true;
+    bool has_w = false, has_f = false, cached = false, released = false;
+    std::array<int64_t, 3> shape;  // of x
     int iters = 0, x_code = 0, cd = 0;
     double eps = 0.0;
     at::ScalarType x_type, w_type, f_type, y_type, p_type[9];
@@ -274,18 +290,21 @@ struct MHCDynamicBackward final : public torch::autograd::Node {
     variable_list apply(variable_list &&grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         TORCH_CHECK(!released, torch::autograd::ERR_BACKWARD_TWICE);
-        const Tensor x = x_.unpack(), kept = kept_.unpack();
-        const Tensor w = has_w ? w_.unpack() : Tensor(), f = has_f ? f_.unpack() : Tensor();
-        const Tensor phi_c = cached ? phi_.unpack() : Tensor(), ba_c = cached ? ba_.unpack() : Tensor();
-        at::AutoDispatchBelowADInplaceOrView below;
-        const int B = x.size(0), n = x.size(1), C = x.size(2), D = n * n + 2 * n;
+        const at::ScalarType act_type = x_code == MHC_BF16 ? at::kBFloat16 : at::kFloat;
+        const int B = (int)shape[0], n = (int)shape[1], C = (int)shape[2], D = n * n + 2 * n;
         const int64_t nC = (int64_t)n * C;
+        const DynLayout l(B, n, C, iters, true, cd, !cached);
+        const Tensor x = unpacked(x_, act_type, B * nC), kept = unpacked(kept_, at::kByte, (int64_t)l.bytes);
+        const Tensor w = has_w ? unpacked(w_, is_act(w_type) ? w_type : at::kFloat, C) : Tensor();
+        const Tensor f = has_f ? unpacked(f_, act_type, (int64_t)B * C) : Tensor();
+        const Tensor phi_c = cached ? unpacked(phi_, cd == MHC_BF16 ? at::kBFloat16 : at::kFloat, D * nC) : Tensor();
+        const Tensor ba_c = cached ? unpacked(ba_, at::kFloat, D + 3) : Tensor();
+        at::AutoDispatchBelowADInplaceOrView below;
         c10::DeviceGuard guard(x.device());
-        const DynLayout l(B, n, C, iters, for_backward, cd, !cached);
         DynViews v(static_cast<char *>(kept.data_ptr()), l);
         if (cached) { v.phi = phi_c.data_ptr(); v.ba = ba_c.data_ptr<float>(); }
         const Tensor dy = incoming_gradient(grads[0], x, y_type);
-        Tensor dx = at::empty(x.sizes(), x.options());
+        Tensor dx = at::empty(shape, x.options());
         Tensor df = has_f ? at::empty(f.sizes(), f.options()) : Tensor();
         // dphi [D, nC], fp32; in a buffer of their own, so that keeping one of them does not keep dphi, the small ones:
         // dbias [D] dalpha [3], fp32 | dw [C] in the weight's type where the library writes it
@@ -325,7 +344,7 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
                          c10::optional<at::ScalarType> out_dtype, const OptTensor &f_opt, bool compute_bf16) {
     TORCH_CHECK(x_in.dim() == 3, "mhc: x must be [B, n, C]");
     const Tensor &w_in = optional_tensor(w_opt), &f_in = optional_tensor(f_opt);
-    refuse_forward_mode({&x_in, &w_in, &f_in, &phi_pre, &phi_post, &phi_res, &alpha_pre, &alpha_post, &alpha_res, &b_pre, &b_post, &b_res});
+    refuse_transforms({&x_in, &w_in, &f_in, &phi_pre, &phi_post, &phi_res, &alpha_pre, &alpha_post, &alpha_res, &b_pre, &b_post, &b_res});
     const bool record = torch::autograd::compute_requires_grad(x_in, w_in, f_in, phi_pre, phi_post, phi_res, alpha_pre,
                                                                alpha_post, alpha_res, b_pre, b_post, b_res);
     std::shared_ptr<MHCDynamicBackward> node;
@@ -333,17 +352,20 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
         node = make_node<MHCDynamicBackward>(torch::autograd::collect_next_edges(
             x_in, w_in, f_in, phi_pre, phi_post, phi_res, alpha_pre, alpha_post, alpha_res, b_pre, b_post, b_res));
     const at::ScalarType y_type = out_dtype.value_or(at::kFloat);
-    Tensor y;
+    const bool cached = g_param_cache;
+    Tensor y, x, w, f, kept;
+    Packed pk;
+    int x_code = 0, cd = 0;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         // compute_bf16 with float32 activations (the reference's default contract: float32 in and out
         // around a bf16 kernel path): where the library's kernels load fp32 storage themselves, x is
         // handed over as it is and rounded in registers; elsewhere it is cast here, as the reference
         // casts it (bindings.cu:421-423)
-        Tensor x = act(is_act_dtype(x_in) ? x_in : x_in.to(at::kFloat));
+        x = act(is_act_dtype(x_in) ? x_in : x_in.to(at::kFloat));
         const int B = x.size(0), n = x.size(1), C = x.size(2), D = n * n + 2 * n;
         c10::DeviceGuard guard(x.device());
-        int x_code = dt(x);
+        x_code = dt(x);
         if (compute_bf16 && x_code == MHC_F32) {
             if (y_type == at::kFloat && mhc_layer_dynamic_accepts_f32_as_bf16(B, n, C, (int)iters))
                 x_code = MHC_F32_AS_BF16;
@@ -352,13 +374,10 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
                 x_code = MHC_BF16;
             }
         }
-        Tensor w, f;
         if (w_in.defined()) w = act(is_act_dtype(w_in) ? w_in : w_in.to(at::kFloat));
         if (f_in.defined()) f = act(f_in.to(x.scalar_type()));
-        const int cd = x_code == MHC_F32 ? MHC_F32 : MHC_BF16;
+        cd = x_code == MHC_F32 ? MHC_F32 : MHC_BF16;
         const DynParams params{{&phi_pre, &phi_post, &phi_res, &alpha_pre, &alpha_post, &alpha_res, &b_pre, &b_post, &b_res}};
-        const bool cached = g_param_cache;
-        Packed pk;
         if (cached) pk = cached_params(params, x, n, C, cd);
         y = at::empty({B, n, C}, x.options().dtype(y_type));
         const DynLayout l(B, n, C, (int)iters, record, cd, !cached);
@@ -367,7 +386,7 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
         const bool own = record || l.bytes > ((size_t)8 << 20);
         const size_t ws_bytes = align256(mhc_layer_dynamic_workspace_bytes(B, n, C));
         Tensor ws = workspace(x, ws_bytes + (own ? 0 : l.bytes));
-        Tensor kept = own ? byte_buffer(x, l.bytes) : Tensor();
+        if (own) kept = byte_buffer(x, l.bytes);
         DynViews v(own ? static_cast<char *>(kept.data_ptr()) : static_cast<char *>(ws.data_ptr()) + ws_bytes, l);
         const int w_dt = w.defined() ? dt(w) : 0;
         if (cached) {
@@ -385,28 +404,31 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
                                                v.Hp, v.Ho, v.M, v.P, v.r, v.q, v.sk, B, n, C, (int)iters, (float)eps,
                                                ws.data_ptr(), ws_bytes, stream_of(x)));
         }
-        if (record) {
-            node->x_ = SavedVariable(x, false);
-            node->kept_ = SavedVariable(kept, false);
-            if ((node->has_w = w.defined())) node->w_ = SavedVariable(w, false);
-            if ((node->has_f = f.defined())) node->f_ = SavedVariable(f, false);
-            if ((node->cached = cached)) {
-                node->phi_ = SavedVariable(pk.phi, false);
-                node->ba_ = SavedVariable(pk.ba, false);
-            }
-            node->iters = (int)iters;
-            node->eps = eps;
-            node->x_code = x_code;
-            node->cd = cd;
-            node->x_type = x_in.scalar_type();
-            node->y_type = y_type;
-            node->w_type = w_in.defined() ? w_in.scalar_type() : at::kFloat;
-            node->f_type = f_in.defined() ? f_in.scalar_type() : at::kFloat;
-            for (int i = 0; i < 9; i++) node->p_type[i] = params.src[i]->scalar_type();
-            node->b_res_sizes = b_res.sizes().vec();
-        }
     }
-    if (record) torch::autograd::set_history(y, node);
+    if (record) {
+        // outside the guard: the hooks of torch.autograd.graph.saved_tensors_hooks run here and are user code
+        node->x_ = SavedVariable(x, false);
+        node->kept_ = SavedVariable(kept, false);
+        if ((node->has_w = w.defined())) node->w_ = SavedVariable(w, false);
+        if ((node->has_f = f.defined())) node->f_ = SavedVariable(f, false);
+        if ((node->cached = cached)) {
+            node->phi_ = SavedVariable(pk.phi, false);
+            node->ba_ = SavedVariable(pk.ba, false);
+        }
+        node->iters = (int)iters;
+        node->eps = eps;
+        node->x_code = x_code;
+        node->cd = cd;
+        node->shape = {x.size(0), x.size(1), x.size(2)};
+        node->x_type = x_in.scalar_type();
+        node->y_type = y_type;
+        node->w_type = w_in.defined() ? w_in.scalar_type() : at::kFloat;
+        node->f_type = f_in.defined() ? f_in.scalar_type() : at::kFloat;
+        const Tensor *src[9] = {&phi_pre, &phi_post, &phi_res, &alpha_pre, &alpha_post, &alpha_res, &b_pre, &b_post, &b_res};
+        for (int i = 0; i < 9; i++) node->p_type[i] = src[i]->scalar_type();
+        node->b_res_sizes = b_res.sizes().vec();
+        torch::autograd::set_history(y, node);
+    }
     return y;
 }
 
@@ -418,7 +440,8 @@ struct MHCStaticBackward final : public torch::autograd::Node {
     bool has_w = false, has_f = false, released = false;
     int iters = 0;
     double eps = 0.0;
-    at::ScalarType x_type, w_type, f_type, y_type, h_type[3];
+    at::ScalarType x_type, act_type, w_type, f_type, y_type, h_type[3];  // act_type: of the saved x
+    std::array<int64_t, 3> shape;                                         // of x
     std::vector<int64_t> h_res_sizes;
 
     std::string name() const override { return "MHCLayerStaticBackward"; }
@@ -432,13 +455,15 @@ struct MHCStaticBackward final : public torch::autograd::Node {
     variable_list apply(variable_list &&grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         TORCH_CHECK(!released, torch::autograd::ERR_BACKWARD_TWICE);
-        const Tensor x = x_.unpack(), hp = hp_.unpack(), ho = ho_.unpack(), hr = hr_.unpack(), kept = kept_.unpack();
-        const Tensor w = has_w ? w_.unpack() : Tensor(), f = has_f ? f_.unpack() : Tensor();
+        const int B = (int)shape[0], n = (int)shape[1], C = (int)shape[2];
+        const Tensor x = unpacked(x_, act_type, (int64_t)B * n * C), kept = unpacked(kept_, at::kFloat, 2 * n + n * n + B);
+        const Tensor hp = unpacked(hp_, at::kFloat, n), ho = unpacked(ho_, at::kFloat, n), hr = unpacked(hr_, at::kFloat, n * n);
+        const Tensor w = has_w ? unpacked(w_, is_act(w_type) ? w_type : at::kFloat, C) : Tensor();
+        const Tensor f = has_f ? unpacked(f_, act_type, (int64_t)B * C) : Tensor();
         at::AutoDispatchBelowADInplaceOrView below;
-        const int B = x.size(0), n = x.size(1), C = x.size(2);
         c10::DeviceGuard guard(x.device());
         const Tensor dy = incoming_gradient(grads[0], x, y_type);
-        Tensor dx = at::empty(x.sizes(), x.options());
+        Tensor dx = at::empty(shape, x.options());
         Tensor df = has_f ? at::empty(f.sizes(), f.options()) : Tensor();
         // dH_pre | dH_post | dH_res, fp32 | dw [C] in the weight's type where the library writes it
         const at::ScalarType dw_type = w_type == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
@@ -467,52 +492,53 @@ Tensor mhc_layer_static(const Tensor &x_in, const OptTensor &w_opt, const Tensor
                         const OptTensor &f_opt) {
     TORCH_CHECK(x_in.dim() == 3, "mhc: x must be [B, n, C]");
     const Tensor &w_in = optional_tensor(w_opt), &f_in = optional_tensor(f_opt);
-    refuse_forward_mode({&x_in, &w_in, &f_in, &H_pre, &H_post, &H_res});
+    refuse_transforms({&x_in, &w_in, &f_in, &H_pre, &H_post, &H_res});
     const bool record = torch::autograd::compute_requires_grad(x_in, w_in, f_in, H_pre, H_post, H_res);
     std::shared_ptr<MHCStaticBackward> node;
     if (record)
         node = make_node<MHCStaticBackward>(torch::autograd::collect_next_edges(x_in, w_in, f_in, H_pre, H_post, H_res));
     const at::ScalarType y_type = out_dtype.value_or(at::kFloat);
-    Tensor y;
+    Tensor y, x, w, f, hp, ho, hr, kept;
     {
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor x = act(is_act_dtype(x_in) ? x_in : x_in.to(at::kFloat));
+        x = act(is_act_dtype(x_in) ? x_in : x_in.to(at::kFloat));
         const int B = x.size(0), n = x.size(1), C = x.size(2);
         c10::DeviceGuard guard(x.device());
-        Tensor w, f;
         if (w_in.defined()) w = act(is_act_dtype(w_in) ? w_in : w_in.to(at::kFloat));
         if (f_in.defined()) f = act(f_in.to(x.scalar_type()));
-        const Tensor hp = f32c(H_pre), ho = f32c(H_post), hr = f32c(H_res);
+        hp = f32c(H_pre); ho = f32c(H_post); hr = f32c(H_res);
         TORCH_CHECK(hp.numel() == n && ho.numel() == n && hr.numel() == n * n, "mhc: H shapes do not match n = ", n);
         y = at::empty({B, n, C}, x.options().dtype(y_type));
-        Tensor kept = at::empty({2 * n + n * n + B}, x.options().dtype(at::kFloat));
+        kept = at::empty({2 * n + n * n + B}, x.options().dtype(at::kFloat));
         float *s = kept.data_ptr<float>();
         Tensor ws = workspace(x, mhc_layer_static_workspace_bytes(B, n, C));
         check("mhc_layer_fwd",
               mhc_layer_fwd(ptr(x), dt(x), ptr(w), w.defined() ? dt(w) : 0, hp.data_ptr<float>(), ho.data_ptr<float>(),
                             hr.data_ptr<float>(), ptr(f), ptr(y), dt(y), s, s + n, s + 2 * n, s + 2 * n + n * n, B, n, C,
                             (int)iters, (float)eps, ws.data_ptr(), (size_t)ws.numel(), stream_of(x)));
-        if (record) {
-            node->x_ = SavedVariable(x, false);
-            node->kept_ = SavedVariable(kept, false);
-            node->hp_ = SavedVariable(hp, false);
-            node->ho_ = SavedVariable(ho, false);
-            node->hr_ = SavedVariable(hr, false);
-            if ((node->has_w = w.defined())) node->w_ = SavedVariable(w, false);
-            if ((node->has_f = f.defined())) node->f_ = SavedVariable(f, false);
-            node->iters = (int)iters;
-            node->eps = eps;
-            node->x_type = x_in.scalar_type();
-            node->y_type = y_type;
-            node->w_type = w_in.defined() ? w_in.scalar_type() : at::kFloat;
-            node->f_type = f_in.defined() ? f_in.scalar_type() : at::kFloat;
-            node->h_type[0] = H_pre.scalar_type();
-            node->h_type[1] = H_post.scalar_type();
-            node->h_type[2] = H_res.scalar_type();
-            node->h_res_sizes = H_res.sizes().vec();
-        }
     }
-    if (record) torch::autograd::set_history(y, node);
+    if (record) {
+        node->x_ = SavedVariable(x, false);
+        node->kept_ = SavedVariable(kept, false);
+        node->hp_ = SavedVariable(hp, false);
+        node->ho_ = SavedVariable(ho, false);
+        node->hr_ = SavedVariable(hr, false);
+        if ((node->has_w = w.defined())) node->w_ = SavedVariable(w, false);
+        if ((node->has_f = f.defined())) node->f_ = SavedVariable(f, false);
+        node->iters = (int)iters;
+        node->eps = eps;
+        node->shape = {x.size(0), x.size(1), x.size(2)};
+        node->x_type = x_in.scalar_type();
+        node->act_type = x.scalar_type();
+        node->y_type = y_type;
+        node->w_type = w_in.defined() ? w_in.scalar_type() : at::kFloat;
+        node->f_type = f_in.defined() ? f_in.scalar_type() : at::kFloat;
+        node->h_type[0] = H_pre.scalar_type();
+        node->h_type[1] = H_post.scalar_type();
+        node->h_type[2] = H_res.scalar_type();
+        node->h_res_sizes = H_res.sizes().vec();
+        torch::autograd::set_history(y, node);
+    }
     return y;
 }
 
