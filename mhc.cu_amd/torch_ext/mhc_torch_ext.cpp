@@ -71,22 +71,44 @@ inline void *stream_of(const Tensor &t) {
     return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-// Scratch buffer per (device, stream), grown on demand.  Kernels that use it are ordered on that
-// stream, so reuse across calls is safe.
-Tensor workspace(const Tensor &like, size_t nbytes) {
+// Scratch memory per (device, stream), grown on demand and held while a call enqueues its launches: on the stream
+// the calls are then ordered one after the other, each with the memory to itself.  Two host threads that use one
+// stream (a forward beside the backward of another thread, which the engine runs on the forward's stream) would
+// otherwise enqueue their launches in between each other's.
+struct Scratch {
+    Tensor retired;  // a smaller buffer that this call replaced; released after the lock
+    std::unique_lock<std::mutex> held;
+    char *ptr;
+    size_t bytes;
+};
+
+Scratch scratch(const Tensor &like, size_t nbytes) {
+    struct Slot {
+        std::mutex mu;
+        Tensor buf;
+    };
     static std::mutex mu;
-    static std::unordered_map<uint64_t, Tensor> cache;
+    static std::unordered_map<uint64_t, Slot> slots;  // (references to its elements stay valid)
     const uint64_t key = (static_cast<uint64_t>(like.device().index()) << 56) ^
                          reinterpret_cast<uint64_t>(stream_of(like));
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = cache.find(key);
-    if (it == cache.end() || static_cast<size_t>(it->second.numel()) < nbytes) {
-        const int64_t want = static_cast<int64_t>(std::max<size_t>(nbytes, 1 << 20));
-        Tensor buf = at::empty({want}, like.options().dtype(at::kByte));
-        cache[key] = buf;
-        return buf;
+    Slot *slot;
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        slot = &slots[key];
     }
-    return it->second;
+    // While a slot is held nothing but library calls may run (no tensor is made, converted or freed): torch may ask
+    // for the interpreter's lock there, which a thread that waits for the slot holds.
+    Tensor buf;
+    std::unique_lock<std::mutex> held(slot->mu);
+    while (!slot->buf.defined() || static_cast<size_t>(slot->buf.numel()) < nbytes) {
+        held.unlock();
+        buf = at::empty({static_cast<int64_t>(std::max<size_t>(nbytes, 1 << 20))}, like.options().dtype(at::kByte));
+        held.lock();
+        if (!slot->buf.defined() || slot->buf.numel() < buf.numel()) std::swap(slot->buf, buf);
+    }
+    char *p = static_cast<char *>(slot->buf.data_ptr());
+    const size_t n = static_cast<size_t>(slot->buf.numel());
+    return Scratch{std::move(buf), std::move(held), p, n};
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -314,12 +336,13 @@ struct MHCDynamicBackward final : public torch::autograd::Node {
         Tensor gs = byte_buffer(x, off_w + (size_t)C * 4);
         char *gp = static_cast<char *>(gs.data_ptr());
         float *dphi = g.data_ptr<float>(), *dba = reinterpret_cast<float *>(gp);
-        Tensor ws = workspace(x, mhc_layer_dynamic_workspace_bytes(B, n, C));
+        Scratch ws = scratch(x, mhc_layer_dynamic_workspace_bytes(B, n, C));
         check("mhc_layer_bwd_dynamic",
               mhc_layer_bwd_dynamic_dw(ptr(dy), dt(dy), ptr(x), x_code, ptr(w), has_w ? dt(w) : 0, v.phi, cd, v.ba, v.ba + D, ptr(f),
                                     v.Hp, v.Ho, v.M, v.P, v.r, v.q, v.sk, ptr(dx), ptr(df),
                                     has_f ? nullptr : gp + off_w, dw_type == at::kBFloat16 ? MHC_BF16 : MHC_F32, dphi, dba, dba + D, B, n, C, iters,
-                                    (float)eps, ws.data_ptr(), (size_t)ws.numel(), stream_of(x)));
+                                    (float)eps, ws.ptr, ws.bytes, stream_of(x)));
+        ws.held.unlock();
         variable_list out(12);
         if (task_should_compute_output(0)) out[0] = cast_to(dx, x_type);
         if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(gs, dw_type, off_w, {C}), w_type);
@@ -385,24 +408,25 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
         // allocation less, 1.5 us; larger ones are not worth the memory that the workspace would hold on to)
         const bool own = record || l.bytes > ((size_t)8 << 20);
         const size_t ws_bytes = align256(mhc_layer_dynamic_workspace_bytes(B, n, C));
-        Tensor ws = workspace(x, ws_bytes + (own ? 0 : l.bytes));
         if (own) kept = byte_buffer(x, l.bytes);
-        DynViews v(own ? static_cast<char *>(kept.data_ptr()) : static_cast<char *>(ws.data_ptr()) + ws_bytes, l);
-        const int w_dt = w.defined() ? dt(w) : 0;
+        Tensor m[9];
+        struct mhc_dynamic_params lp;
+        if (!cached) lp = library_params(params, n, C, m);
+        const int w_dt = w.defined() ? dt(w) : 0, y_dt = dt(y);
+        const Scratch ws = scratch(x, ws_bytes + (own ? 0 : l.bytes));
+        DynViews v(own ? static_cast<char *>(kept.data_ptr()) : ws.ptr + ws_bytes, l);
         if (cached) {
             v.phi = pk.phi.data_ptr();
             v.ba = pk.ba.data_ptr<float>();
             check("mhc_layer_fwd_dynamic",
-                  mhc_layer_fwd_dynamic(ptr(x), x_code, ptr(w), w_dt, v.phi, cd, v.ba, v.ba + D, ptr(f), ptr(y), dt(y), v.Hp, v.Ho,
-                                        v.M, v.P, v.r, v.q, v.sk, B, n, C, (int)iters, (float)eps, ws.data_ptr(),
-                                        ws_bytes, stream_of(x)));
+                  mhc_layer_fwd_dynamic(ptr(x), x_code, ptr(w), w_dt, v.phi, cd, v.ba, v.ba + D, ptr(f), ptr(y), y_dt, v.Hp, v.Ho,
+                                        v.M, v.P, v.r, v.q, v.sk, B, n, C, (int)iters, (float)eps, ws.ptr, ws_bytes,
+                                        stream_of(x)));
         } else {
-            Tensor m[9];
-            const struct mhc_dynamic_params lp = library_params(params, n, C, m);
             check("mhc_layer_fwd_dynamic",
-                  mhc_layer_fwd_dynamic_params(ptr(x), x_code, ptr(w), w_dt, &lp, v.phi, cd, v.ba, v.ba + D, ptr(f), ptr(y), dt(y),
+                  mhc_layer_fwd_dynamic_params(ptr(x), x_code, ptr(w), w_dt, &lp, v.phi, cd, v.ba, v.ba + D, ptr(f), ptr(y), y_dt,
                                                v.Hp, v.Ho, v.M, v.P, v.r, v.q, v.sk, B, n, C, (int)iters, (float)eps,
-                                               ws.data_ptr(), ws_bytes, stream_of(x)));
+                                               ws.ptr, ws_bytes, stream_of(x)));
         }
     }
     if (record) {
@@ -470,12 +494,13 @@ struct MHCStaticBackward final : public torch::autograd::Node {
         const size_t off_w = align256((size_t)(2 * n + n * n) * 4);
         Tensor g = byte_buffer(x, off_w + (size_t)C * 4);
         float *d = static_cast<float *>(g.data_ptr()), *s = kept.data_ptr<float>();
-        Tensor ws = workspace(x, mhc_layer_static_workspace_bytes(B, n, C));
+        Scratch ws = scratch(x, mhc_layer_static_workspace_bytes(B, n, C));
         check("mhc_layer_bwd",
               mhc_layer_bwd_dw(ptr(dy), dt(dy), ptr(x), dt(x), ptr(w), has_w ? dt(w) : 0, hp.data_ptr<float>(), ho.data_ptr<float>(),
                             hr.data_ptr<float>(), ptr(f), s, s + n, s + 2 * n, s + 2 * n + n * n, ptr(dx), ptr(df),
-                            has_f ? nullptr : d + off_w / 4, dw_type == at::kBFloat16 ? MHC_BF16 : MHC_F32, d, d + n, d + 2 * n, B, n, C, iters, (float)eps, ws.data_ptr(),
-                            (size_t)ws.numel(), stream_of(x)));
+                            has_f ? nullptr : d + off_w / 4, dw_type == at::kBFloat16 ? MHC_BF16 : MHC_F32, d, d + n, d + 2 * n, B, n, C, iters, (float)eps, ws.ptr,
+                            ws.bytes, stream_of(x)));
+        ws.held.unlock();
         variable_list out(6);
         if (task_should_compute_output(0)) out[0] = cast_to(dx, x_type);
         if (has_w && !has_f && task_should_compute_output(1)) out[1] = cast_to(over(g, dw_type, off_w, {C}), w_type);
@@ -511,11 +536,11 @@ Tensor mhc_layer_static(const Tensor &x_in, const OptTensor &w_opt, const Tensor
         y = at::empty({B, n, C}, x.options().dtype(y_type));
         kept = at::empty({2 * n + n * n + B}, x.options().dtype(at::kFloat));
         float *s = kept.data_ptr<float>();
-        Tensor ws = workspace(x, mhc_layer_static_workspace_bytes(B, n, C));
+        const Scratch ws = scratch(x, mhc_layer_static_workspace_bytes(B, n, C));
         check("mhc_layer_fwd",
               mhc_layer_fwd(ptr(x), dt(x), ptr(w), w.defined() ? dt(w) : 0, hp.data_ptr<float>(), ho.data_ptr<float>(),
                             hr.data_ptr<float>(), ptr(f), ptr(y), dt(y), s, s + n, s + 2 * n, s + 2 * n + n * n, B, n, C,
-                            (int)iters, (float)eps, ws.data_ptr(), (size_t)ws.numel(), stream_of(x)));
+                            (int)iters, (float)eps, ws.ptr, ws.bytes, stream_of(x)));
     }
     if (record) {
         node->x_ = SavedVariable(x, false);
@@ -551,11 +576,11 @@ Tensor mhc_layer_inference(const Tensor &x_in, const Tensor &w_in, const Tensor 
     c10::DeviceGuard guard(x.device());
     const Tensor hp = f32c(H_pre), ho = f32c(H_post), hr = f32c(H_res);
     Tensor y = at::empty({B, n, C}, x.options().dtype(out_dtype.value_or(at::kFloat)));
-    Tensor ws = workspace(x, mhc_layer_static_workspace_bytes(B, n, C));
+    const Scratch ws = scratch(x, mhc_layer_static_workspace_bytes(B, n, C));
     check("mhc_layer_fwd",
           mhc_layer_fwd(ptr(x), dt(x), ptr(w), dt(w), hp.data_ptr<float>(), ho.data_ptr<float>(), hr.data_ptr<float>(),
                         nullptr, ptr(y), dt(y), nullptr, nullptr, nullptr, nullptr, B, n, C, (int)iters, (float)eps,
-                        ws.data_ptr(), (size_t)ws.numel(), stream_of(x)));
+                        ws.ptr, ws.bytes, stream_of(x)));
     return y;
 }
 
@@ -585,13 +610,14 @@ struct SinkhornFn : public torch::autograd::Function<SinkhornFn> {
         const int rows = inp.size(-2), cols = inp.size(-1);
         const int batch = (int)(inp.numel() / ((int64_t)rows * cols));
         const int iters = (int)ctx->saved_data["iters"].toInt();
+        const double eps = ctx->saved_data["eps"].toDouble();
+        const auto sd = (at::ScalarType)ctx->saved_data["dtype"].toInt();
         Tensor d_inp = at::empty_like(inp);
-        Tensor ws = workspace(inp, mhc_sinkhorn_knopp_bwd_workspace_bytes(batch, rows, cols, iters));
+        Scratch ws = scratch(inp, mhc_sinkhorn_knopp_bwd_workspace_bytes(batch, rows, cols, iters));
         check("mhc_sinkhorn_knopp_bwd",
               mhc_sinkhorn_knopp_bwd(go.data_ptr<float>(), inp.data_ptr<float>(), d_inp.data_ptr<float>(), batch, rows, cols,
-                                     iters, (float)ctx->saved_data["eps"].toDouble(), ws.data_ptr(), (size_t)ws.numel(),
-                                     stream_of(inp)));
-        const auto sd = (at::ScalarType)ctx->saved_data["dtype"].toInt();
+                                     iters, (float)eps, ws.ptr, ws.bytes, stream_of(inp)));
+        ws.held.unlock();
         return {d_inp.scalar_type() == sd ? d_inp : d_inp.to(sd), Tensor(), Tensor()};
     }
 };
@@ -619,10 +645,11 @@ struct RMSNormFn : public torch::autograd::Function<RMSNormFn> {
         const int rows = (int)(inp.numel() / C);
         Tensor d_inp = at::empty_like(inp);
         Tensor d_w = at::empty({C}, inp.options().dtype(at::kFloat));
-        Tensor ws = workspace(inp, mhc_rmsnorm_bwd_workspace_bytes(rows, C));
+        Scratch ws = scratch(inp, mhc_rmsnorm_bwd_workspace_bytes(rows, C));
         check("mhc_rmsnorm_bwd",
               mhc_rmsnorm_bwd(ptr(go), ptr(inp), dt(inp), ptr(w), dt(w), rms.data_ptr<float>(), ptr(d_inp),
-                              d_w.data_ptr<float>(), rows, C, ws.data_ptr(), (size_t)ws.numel(), stream_of(inp)));
+                              d_w.data_ptr<float>(), rows, C, ws.ptr, ws.bytes, stream_of(inp)));
+        ws.held.unlock();
         return {d_inp, d_w.scalar_type() == w.scalar_type() ? d_w : d_w.to(w.scalar_type()), Tensor()};
     }
 };
