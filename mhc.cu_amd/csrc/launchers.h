@@ -5,9 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
-#include <atomic>
-
 #include "batch_sums.h"
+#include "raised_limit.h"
 
 namespace mhc {
 
@@ -22,20 +21,15 @@ inline size_t dtype_size(int dt) { return dt == kBF16 ? 2 : 4; }
 inline int max_layer_sinkhorn_iters(int) { return 256; }
 
 // Dynamic LDS above 64 KB has to be enabled per kernel and device before the launch: asked for once, not on every
-// call (the attribute only ever grows; two threads that ask at the same time set the same or the larger value).
+// call, and only ever raised (kernels whose LDS depends on the iteration count ask for different sizes).
 template <auto Kernel> inline hipError_t allow_dynamic_lds(size_t bytes) {
     if (bytes <= 64 * 1024) return hipSuccess;
-    constexpr int kDevices = 64;
-    static std::atomic<int> allowed[kDevices];
+    static RaisedLimit allowed;
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-    const bool known = dev >= 0 && dev < kDevices;
-    int have = known ? allowed[dev].load(std::memory_order_relaxed) : 0;
-    if (have >= (int)bytes) return hipSuccess;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e == hipSuccess && known)
-        while (have < (int)bytes && !allowed[dev].compare_exchange_weak(have, (int)bytes, std::memory_order_relaxed)) {}
-    return e;
+    return allowed.raise(dev, (int)bytes, [](int value) {
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, value);
+    });
 }
 
 // Projection row count padded to whole 32-wide MFMA tiles.

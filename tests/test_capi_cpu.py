@@ -165,3 +165,13 @@ def test_torch_extension_is_built_and_bound_to_the_same_library():
     with open("/proc/self/maps") as f:
         libs = {line.split()[-1] for line in f if "libmhc_hip" in line}
     assert len(libs) == 1, libs
+
+
+def test_raised_limit_of_two_threads_is_the_larger_one(tmp_path):
+    """The launchers raise a kernel's dynamic LDS limit once per size and device (csrc/raised_limit.h)."""
+    import subprocess
+    exe = tmp_path / "test_raised_limit"
+    src = os.path.join(ROOT, "tests", "native", "test_raised_limit.cpp")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-pthread", src, "-o", str(exe)])
+    p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert p.returncode == 0, p.stdout
