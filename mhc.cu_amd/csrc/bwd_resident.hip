@@ -30,7 +30,7 @@ namespace mhc {
 
 struct BwdResidentArgs {
     BwdReduceArgs r;   // inputs and the outputs of the coefficient backward
-    void *dxp;         // [B, n, C], stored like x (bf16, or fp32 with F32)
+    void *dxp;         // [B, n, C], stored like x (bf16, or fp32 with F32), or fp32 (bwd_resident_dxp_f32())
     void *df;          // [B, C] or nullptr (only with r.f_inject), stored like x
     float *u;          // [B, C] (unused with r.f_inject)
 };
@@ -39,7 +39,8 @@ constexpr int kResTileWaves = 4;                         // waves that hold the 
 constexpr int kResMaxItems = 5;                          // 128-channel steps per tile wave
 // rows of more than 4 * 5 * 128 channels: seven tile waves (eight with the coefficient wave are two per SIMD and
 // leave 256 registers; one wave more would leave 168, which 8 x 8 samples do not fit)
-constexpr int kResLongWaves = 7, kResMaxC = 4096;
+constexpr int kResLongWaves = 7;
+static_assert(kResWholeMaxC == 128 * kResTileWaves * kResMaxItems && kResShortMaxC == 128 * kResTileWaves, "bwd_resident_dxp_f32()");
 
 template <int SEL> __device__ __forceinline__ float quad_bcast(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), SEL * 0x55, 0xF, 0xF, true));
@@ -77,6 +78,11 @@ template <bool ANY> struct Act8<true, ANY> {
     }
 };
 
+// bwd_resident_dxp_f32() in terms of the instantiation that serves a shape (launch_items below)
+template <int NP, int ITEMS, bool F32, bool STATIC, int TWV, bool RAG> constexpr bool res_dxp_f32() {
+    return !F32 && !STATIC && (RAG || (TWV == kResLongWaves && ITEMS >= 3) || (NP == 8 && TWV <= kResTileWaves));
+}
+
 // F32: dy, x (and an injected f) are stored as fp32 and rounded to bf16 as they are loaded; dxp and df
 // are written as fp32.  The arithmetic is the same either way.
 // STATIC: shared coefficients ([n] / [n, n] instead of per sample).  There is no projection, so dxp is
@@ -86,6 +92,8 @@ template <bool ANY> struct Act8<true, ANY> {
 template <int NP, int WMODE, int ITEMS, bool F32, bool STATIC = false, int TWV = kResTileWaves, bool RAG = false>
 __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void bwd_resident_kernel(BwdResidentArgs ra) {
     using TS = typename std::conditional<F32, float, bf16_t>::type;  // storage type of the activations
+    constexpr bool X32 = res_dxp_f32<NP, ITEMS, F32, STATIC, TWV, RAG>();
+    using TD = typename std::conditional<X32, float, TS>::type;      // of dxp
     static_assert(NP == 4 || NP == 8, "stream groups of four");
     using SK = SkSmall<NP>;
     using CB = CoefBwdSmall<NP, false, true, STATIC>;
@@ -341,36 +349,38 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
         k2 = tot_s[K] * qinv * qinv * qinv / (float)C;
     }
     // eight results of a row in two halves, stored together (neighbouring 16-byte pieces at once)
-    constexpr int OW = F32 ? 8 : 4;  // words of a chunk as stored
-    auto put_half = [](TS *p, uint32_t (&w)[OW], const float (&v)[4], int h, int left) {
-        if constexpr (F32) {
+    constexpr int OWD = sizeof(TD) * 2, OWS = sizeof(TS) * 2;  // words of a chunk as stored: of dxp, of df
+    auto put_half = [](auto *p, auto &w, const float (&v)[4], int h, int left) {
+        using T = typename std::remove_pointer<decltype(p)>::type;
+        constexpr bool W32 = sizeof(T) == 4;
+        if constexpr (W32) {
 #pragma unroll
             for (int k = 0; k < 4; k++) w[4 * h + k] = __float_as_uint(v[k]);
-            if (h == 1) {
-                st16<false>(p, w[0], w[1], w[2], w[3]);
-                st16<false>(p + 4, w[4], w[5], w[6], w[7]);
-            }
         } else {
             w[2 * h] = pack_bf16x2(v[0], v[1]);
             w[2 * h + 1] = pack_bf16x2(v[2], v[3]);
-            if (h == 1) {
-                if constexpr (!RAG) {
-                    st16<false>(p, w[0], w[1], w[2], w[3]);
-                } else if (left >= 8) {
-                    st16_any<false>(p, w[0], w[1], w[2], w[3]);
-                } else {  // left: elements up to the row's end
+        }
+        if (h == 0) return;
+        if constexpr (!RAG) {
 #pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        if (e < left) p[e] = (TS)(w[e / 2] >> (16 * (e & 1)));
+            for (int k = 0; k < (W32 ? 2 : 1); k++) st16<false>(p + 4 * k, w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+        } else if (left >= 8) {
+#pragma unroll
+            for (int k = 0; k < (W32 ? 2 : 1); k++) st16_any<false>(p + 4 * k, w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+        } else {  // left: elements up to the row's end
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (e < left) {
+                    if constexpr (W32) p[e] = __uint_as_float(w[e]);
+                    else p[e] = (T)(w[e / 2] >> (16 * (e & 1)));
                 }
-            }
         }
     };
 #pragma unroll
     for (int it = 0; it < ITEMS; it++) {
         const int c = (tw + TW * it) * 128 + blk * 8;
         if (!in[it]) continue;  // quads are inside or outside together: the DPP exchanges stay within a quad
-        uint32_t ow[NB][OW], dfw[OW];
+        uint32_t ow[NB][OWD], dfw[OWS];
         float u8[8];
         // four channels at a time: the fp32 copies of eight cost the 8 x 8 case thirty registers
 #pragma unroll
@@ -437,7 +447,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                         out[v] += Mc[I][J][3] * quad_bcast<3>(gv[J][v]);
                     }
                 // plain stores: the projection-backward launch reads dxp back right away
-                if (sv[I]) put_half(static_cast<TS *>(ra.dxp) + ((size_t)b * n + 4 * I + i) * C + c, ow[I], out, h, C - c);
+                if (sv[I]) put_half(static_cast<TD *>(ra.dxp) + ((size_t)b * n + 4 * I + i) * C + c, ow[I], out, h, C - c);
             }
         }
     }
@@ -468,6 +478,8 @@ static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream)
 #define MHC_RES_ITEMS(N)                                                                              \
     case N:                                                                                           \
         if constexpr (N >= kMinItems && N <= kMaxItems && !(RAG && N == 4)) {                         \
+            if (!F32 && !STATIC && res_dxp_f32<NP, N, F32, STATIC, TW, RAG>() != bwd_resident_dxp_f32(ra.r.n, ra.r.C)) \
+                return hipErrorInvalidValue; /* not reached */                                        \
             bwd_resident_kernel<NP, WMODE, N, F32, STATIC, TW, RAG><<<grid, threads, smem, stream>>>(ra); \
             return hipGetLastError();                                                                 \
         }                                                                                             \

@@ -62,7 +62,7 @@ int ws_check(void *ws, size_t have, size_t need) {
 
 // ---- dynamic workspace layout ----------------------------------------------------------------
 struct DynFwdWs { float *Ppart, *ssqpart, *agg; size_t bytes; };
-struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, *dx_part, *dphi_part; unsigned short *dPb, *dPT; int BP; size_t bytes; };
+struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, *dx_part, *dxp, *dphi_part; unsigned short *dPb, *dPT; int BP; size_t bytes; };
 
 // Whether the sample-resident backward (bwd_resident.hip + the column-slab kernel without batch split)
 // is taken where it is supported.  Its second launch walks all samples of a column slab in one
@@ -132,6 +132,9 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     w.s1part = c.floats(n > 8 ? (size_t)B * bwd_reduce_parts(B, n, C) : 0);
     // wide projections: the part of dx that is formed beside the coefficient backward, fp32
     w.dx_part = c.floats(wide_dx_beside(B, n, C) ? (size_t)B * nC : 0);
+    // n <= 8, sample-resident backward: dxp where it is handed over in fp32
+    const bool resident = n <= 8 && C <= kResMaxC && (bwd_resident_preferred(B, n, C) || C % 8 != 0);
+    w.dxp = c.floats(resident && bwd_resident_dxp_f32(n, C) ? (size_t)B * nC : 0);
     int bs = dphi_batch_splits(B, n, C);
     const int bs2 = proj_bwd_batch_splits(B, n, C);
     if (bs2 > bs) bs = bs2;
@@ -628,8 +631,9 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         BwdCoefOut out2 = out;
         out2.dPb = ws.dPb;
         out2.dP = nullptr;  // the second launch takes dP as matrix-core operands only
+        float *dxp = x_dtype == kBF16 && bwd_resident_dxp_f32(n, C) ? ws.dxp : nullptr;
         MHC_LAUNCH(launch_bwd_resident(dy, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, q, P, r, alpha, bias + 2 * n,
-                                       sk_state, out2, dx, df, ws.u, B, n, C, iters, eps, st));
+                                       sk_state, out2, dxp ? dxp : dx, df, ws.u, B, n, C, iters, eps, st));
         const DwOut dwo = f_inject ? DwOut{} : dw;
         const int S = proj_bwd_addx_splits(B, n, C), parts = proj_bwd_addx_sum_parts(B, S);
         bool tail_taken = false;
@@ -637,7 +641,7 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
             // partial sums of dphi, dw, dbias and dalpha, added up by one more launch
             const BatchSumArgs sums = make_batch_sums(ws.u, B, C, dwo ? DwOut{ws.upart, false} : dwo, ws.dt, B, D, ws.dtpart,
                                                       ws.dtpart + D);
-            MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, ws.dphi_part, S, dx, B, n, C, &sums,
+            MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, ws.dphi_part, S, dxp, dx, B, n, C, &sums,
                                             &tail_taken, st));
             if (!tail_taken) return MHC_ERR_LAUNCH;  // not reached: any number of workgroups can carry the parts
             MHC_LAUNCH(launch_finalize(ws.upart, parts, C, dwo, ws.dtpart, parts, D, dbias, dalpha, ws.dphi_part, S,
@@ -645,7 +649,7 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
             return MHC_OK;
         }
         const BatchSumArgs sums = make_batch_sums(ws.u, B, C, dwo, ws.dt, B, D, dbias, dalpha);
-        MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, dphi, 1, dx, B, n, C,
+        MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, dphi, 1, dxp, dx, B, n, C,
                                         tuning_get(kTuneSeparateFinalize) == 1 ? nullptr : &sums, &tail_taken, st));
         if (!tail_taken)
             MHC_LAUNCH(launch_finalize(ws.u, B, C, dwo, ws.dt, B, D, dbias, dalpha, nullptr, 1, 0, nullptr, st));

@@ -228,6 +228,14 @@ hipError_t launch_proj_bwd_mfma(const void *x, const void *phi, const void *dPb,
 // outputs of launch_mix_bwd_reduce) and dxp = M^T dy + Hpre (x) da from ONE pass over dy and x, one
 // workgroup per sample; u [B, C] = the samples' summands of dw, df with an injected f.
 bool bwd_resident_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C, int T);
+constexpr int kResShortMaxC = 512, kResWholeMaxC = 2560, kResMaxC = 4096;
+// bf16 storage: whether dxp goes to the second launch in fp32 (a buffer [B, n, C] of its own) instead of bf16 in dx.
+// dx is then rounded once and its error against float64 is that of the tiled kernels, which would serve these
+// shapes otherwise (1.66e-3 relative); handed over in bf16 it is rounded twice (2.35e-3).
+// The price is 4 bytes per element (backward us, tiled | handed over in bf16 | in fp32): n=4 C=2880 B=256 27.6 | 19.2 |
+// 21.5; n=8 C=4096 B=100 45.5 | 32.7 | 33.3; n=8 C=3072 B=1000 128.6 | 102.7 | 107.2; n=8 C=256 B=6000 113.3 | 66.9 |
+// 70.4, B=600 29.9 | 22.7 | 24.6.  Rows of 513 .. 2560 channels (n <= 4: up to 2560) keep the bf16 hand-over.
+inline bool bwd_resident_dxp_f32(int n, int C) { return C % 8 != 0 || C > kResWholeMaxC || (n > 4 && C <= kResShortMaxC); }
 hipError_t launch_bwd_resident(const void *dy, const void *x, int x_dtype, const void *w, int w_dtype, const void *f_inject,
                                const float *Hpre, const float *Hpost, const float *M, const float *q,
                                const float *P, const float *r, const float *alpha, const float *b_res,
@@ -247,9 +255,10 @@ bool proj_bwd_addx_supported(int n);
 // rows ([C] and [D + 3]) of partial sums
 int proj_bwd_addx_splits(int B, int n, int C);
 int proj_bwd_addx_sum_parts(int B, int S);
+// dxp: nullptr (in dx, stored like it), or fp32 where bwd_resident_dxp_f32() holds
 hipError_t launch_proj_bwd_addx(const void *x, int x_dtype, const void *phi, const void *dPb, const void *dPT, int BP,
-                                const float *cx, float *dphi, int S, void *dx, int B, int n, int C, const BatchSumArgs *tail,
-                                bool *tail_taken, hipStream_t stream);
+                                const float *cx, float *dphi, int S, const float *dxp, void *dx, int B, int n, int C,
+                                const BatchSumArgs *tail, bool *tail_taken, hipStream_t stream);
 // n <= 18: whether the two products are faster apart (measured: from D > 128 on)
 bool proj_bwd_products_apart(int n);
 // Wide projections (more than 12 row tiles of 32, n > 18) always run the two products as two GEMM

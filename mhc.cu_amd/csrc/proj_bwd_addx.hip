@@ -3,11 +3,11 @@
 //
 //   dphi[d, k] = sum_b dP[b, d] x_flat[b, k]                      (reference ops.py:332-334)
 //
-// is finished here without batch-split partial sums, and completes dx in place,
+// is finished here without batch-split partial sums, and completes dx,
 //
 //   dx[b, k] = dxp[b, k] + sum_d dP[b, d] phi[d, k] - cx[b] x_flat[b, k]      (reference ops.py:336-351)
 //
-// where dxp = M^T dy + Hpre (x) da was left in the dx buffer by the first launch.  A few extra
+// where dxp = M^T dy + Hpre (x) da was left by the first launch, in the dx buffer or in fp32 beside it.  A few extra
 // workgroups (one more grid row) add up dw, dbias and dalpha (batch_sums.h), so the backward needs no
 // third launch.
 //
@@ -37,7 +37,8 @@ struct ProjAddxArgs {
     const bf16_t *dPT;   // dP^T hi and lo bf16 planes, fragment-major (frag_dpt); rows >= D, columns >= B zero
     const float *cx;     // [B]
     float *dphi;         // [D][nC], one such plane per batch split
-    void *dx;            // [B][nC]: in dxp, out dx; stored like x
+    const void *dxp;     // [B][nC]: dx itself, or fp32 (kAxFine, kAxRagged)
+    void *dx;            // [B][nC], stored like x
     int B, BP, D, DP, nC;
     int per_split;       // samples of a batch split (whole blocks); blockIdx.y < splits
     int tail_row;        // first blockIdx.y of the workgroups that compute `tail` (-1: none)
@@ -59,17 +60,25 @@ constexpr int kAxLDR = 36;         // LDS pitch of the dphi tiles in the final c
 // 4 SPW samples).  PFOP: the dP operands of the next block are requested a block ahead like x and dxp.
 // Measured at B=320, C=1280, n=4 (backward, graphs of ten): SPW 32 without / with PFOP 16.1 / 16.1 us,
 // SPW 64 without PFOP 19.1 us, with PFOP 23.0 us (registers spill).
-// F32: x and dx are stored as fp32 (x is rounded to bf16 for the products and for the -cx x term, as in
-// the bf16 storage case; dxp is read and dx written as fp32).
+// ST: how the activations are stored and dxp is handed over
+//   kAxBf16    bf16, dxp in place (dx is rounded twice)
+//   kAxF32     fp32, dxp in place (x is rounded to bf16 for the products and for the -cx x term, as in the bf16
+//              storage case; dxp is read and dx written as fp32)
+//   kAxFine    bf16, dxp fp32 in a buffer of its own (dx is rounded once)
+//   kAxRagged  the same for rows of any length (C % 8 != 0): the last chunk of a row is loaded from nC - 8 on and
+//              shifted down
 // NW: waves per workgroup (a block is NW * SPW samples).
-// RAG: rows of any length (nC % 8 != 0): the last chunk of a row is loaded from nC - 8 on and shifted down.
 // SPLIT: blockIdx.y is a batch split (a template argument: with a run-time first sample the compiler keeps fewer
 // loads in flight, B=1000 n=6 C=1024 17.2 -> 21.2 us without any split).
-template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false, bool SPLIT = false>
+enum { kAxBf16 = 0, kAxF32 = 1, kAxFine = 2, kAxRagged = 3 };
+
+template <int NTD, int SPW, bool PFOP, int ST, int NW = 4, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel(ProjAddxArgs a) {
     constexpr int NT_ = 64 * NW;  // threads
+    constexpr bool F32 = ST == kAxF32, RAG = ST == kAxRagged, P32 = ST != kAxBf16;  // P32: dxp is fp32
     using TS = typename std::conditional<F32, float, bf16_t>::type;
-    constexpr int AW = F32 ? 8 : 4;  // words of an 8-element chunk as stored
+    using TP = typename std::conditional<P32, float, bf16_t>::type;
+    constexpr int AW = F32 ? 8 : 4, PW = P32 ? 8 : 4;  // words of an 8-element chunk as stored: of x, of dxp
     constexpr int SBR = NW * SPW;  // samples per block
     constexpr int KS = SPW / 16;   // k-steps (16 samples) of a wave per block = its 16-byte chunks of x and of dxp
     constexpr int TT = SPW / 32;   // 32-sample tiles of a wave per block
@@ -119,17 +128,18 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
     const int kl = k0 + (tid & 3) * 8;  // the chunk of x and phi
     const int kls = RAG && kl < nC && kl + 8 > nC ? kl + 8 - nC : 0, kcs = RAG && kok && kc + 8 > nC ? kc + 8 - nC : 0;
     // dxp of the next block is requested a block ahead like x, except where that costs the registers that
-    // keep two workgroups on a CU (fp32 storage with a wide projection): there it is requested at the top
+    // keep two workgroups on a CU (fp32 dxp with a wide projection): there it is requested at the top
     // of its own block and arrives under the matrix-core phase
-    constexpr int PS = (F32 && NTD >= 2) ? 1 : 2;
-    uint32_t xr[2][KS][AW], pr[PS][KS][AW];
+    constexpr int PS = (P32 && NTD >= 2) ? 1 : 2;
+    uint32_t xr[2][KS][AW], pr[PS][KS][PW];
     float cxr[PS][KS];
     const TS *xg = static_cast<const TS *>(a.x);
     TS *dxg = static_cast<TS *>(a.dx);
-    auto load_chunk = [&](const TS *p, uint32_t (&q)[AW], bool ok) {
+    const TP *dxpg = static_cast<const TP *>(a.dxp);
+    auto load_chunk = [&](const auto *p, auto &q, bool ok) {
         const uint4 v = ldg16<RAG>(p);
         q[0] = ok ? v.x : 0u; q[1] = ok ? v.y : 0u; q[2] = ok ? v.z : 0u; q[3] = ok ? v.w : 0u;
-        if constexpr (F32) {
+        if constexpr (sizeof(*p) == 4) {
             const uint4 v2 = ldg16<RAG>(p + 4);
             q[4] = ok ? v2.x : 0u; q[5] = ok ? v2.y : 0u; q[6] = ok ? v2.z : 0u; q[7] = ok ? v2.w : 0u;
         }
@@ -148,7 +158,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
             for (int t = 0; t < KS; t++) {
                 const int b = sb + erow + 16 * t;
                 const bool ok = b < B && kok;
-                load_chunk(dxg + (ok ? (size_t)b * nC + kc - kcs : 0), pr[S][t], ok);
+                load_chunk(dxpg + (ok ? (size_t)b * nC + kc - kcs : 0), pr[S][t], ok);
                 cxr[S][t] = a.cx[b < B ? b : 0];
             }
         }
@@ -158,37 +168,40 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         for (int t = 0; t < KS; t++) {
             const int b = sb + erow + 16 * t;
             const bool ok = b < B && kok;
-            load_chunk(dxg + (ok ? (size_t)b * nC + kc - kcs : 0), pr[0][t], ok);
+            load_chunk(dxpg + (ok ? (size_t)b * nC + kc - kcs : 0), pr[0][t], ok);
             cxr[0][t] = a.cx[b < B ? b : 0];
         }
     };
     // Operands that come straight from global memory in fragment order: dP^T (rounded value and
     // remainder) of this wave's samples for every dphi tile, and dP of its sample tiles.  Steps and
     // tiles beyond the padded batch read zeros.
+    constexpr int TPL = 2, BPL = 1, HELD = 2;  // planes of dP^T and of dP, planes of dP^T requested here
+    const size_t plane = (size_t)a.DP * a.BP;
+    auto load_at = [&](int sb, int p, int m, int ks) {
+        const int nsteps = a.BP >> 4, step = (sb >> 4) + KS * wave + ks;
+        const bool ok = step < nsteps;
+        return load16_masked(reinterpret_cast<const uint4 *>(a.dPT + p * plane + (ok ? frag_base(m, nsteps, step) : 0) + lane * 8), ok);
+    };
+    auto load_av = [&](int sb, int p, int t, int ks) {
+        const int tile = (sb >> 5) + TT * wave + t;
+        const bool ok = tile < (a.BP >> 5);
+        return load16_masked(reinterpret_cast<const uint4 *>(a.dPb + p * plane + (ok ? frag_base(tile, a.DP >> 4, ks) : 0) + lane * 8), ok);
+    };
     struct Ops {
-        uint4 ah[NTD][KS], al[NTD][KS], av[TT][2 * NTD];
+        uint4 at[HELD][NTD][KS], av[TT][2 * NTD];
     };
     Ops ops[PFOP ? 2 : 1];
     auto load_ops = [&](int sb, Ops &o) {
-        const int step0 = (sb >> 4) + KS * wave, nsteps = a.BP >> 4;
 #pragma unroll
         for (int m = 0; m < NTD; m++)
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const bool ok = step0 + ks < nsteps;
-                const bf16_t *ap = a.dPT + (ok ? frag_base(m, nsteps, step0 + ks) : 0) + lane * 8;
-                o.ah[m][ks] = load16_masked(reinterpret_cast<const uint4 *>(ap), ok);
-                o.al[m][ks] = load16_masked(reinterpret_cast<const uint4 *>(ap + (size_t)a.DP * a.BP), ok);
-            }
+            for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const int tile = (sb >> 5) + TT * wave + t;
-            const bool ok = tile < (a.BP >> 5);
+                for (int p = 0; p < HELD; p++) o.at[p][m][ks] = load_at(sb, p, m, ks);
 #pragma unroll
-            for (int ks = 0; ks < 2 * NTD; ks++)
-                o.av[t][ks] = load16_masked(
-                    reinterpret_cast<const uint4 *>(a.dPb + (ok ? frag_base(tile, a.DP >> 4, ks) : 0) + lane * 8), ok);
-        }
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int ks = 0; ks < 2 * NTD; ks++) o.av[t][ks] = load_av(sb, 0, t, ks);
     };
     using Slot0 = std::integral_constant<int, 0>;
     using Slot1 = std::integral_constant<int, 1>;
@@ -258,10 +271,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 #pragma unroll
             for (int m = 0; m < NTD; m++)
 #pragma unroll
-                for (int ks = 0; ks < KS; ks++) {
-                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op.ah[m][ks]), xf[ks], acc[m], 0, 0, 0);
-                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op.al[m][ks]), xf[ks], acc[m], 0, 0, 0);
-                }
+                for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+                    for (int p = 0; p < TPL; p++)
+                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(bf16x8_t, p < HELD ? op.at[p < HELD ? p : 0][m][ks] : load_at(sb, p, m, ks)), xf[ks], acc[m], 0, 0, 0);
         }
         // ---- dP phi of this wave's sample tiles -> its own rows of o_s (phi fragments from the slab) -----
 #pragma unroll
@@ -272,7 +286,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 #pragma unroll
             for (int ks = 0; ks < 2 * NTD; ks++) {
                 const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, lds_frag_tr(phi_s, kAxLD, ks * 16, 0, lane));
-                o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op.av[t][ks]), pf, o, 0, 0, 0);
+#pragma unroll
+                for (int p = 0; p < BPL; p++)
+                    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, p < 1 ? op.av[t][ks] : load_av(sb, p, t, ks)), pf, o, 0, 0, 0);
             }
             // accumulator layout: column = lane & 31, register i -> row 8*(i/4) + 4*(lane/32) + i%4
 #pragma unroll
@@ -289,14 +305,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
             const float4 o1 = *reinterpret_cast<const float4 *>(o_s + (size_t)r * kAxLDO + ech * 8 + 4);
             const uint4 xv = *reinterpret_cast<const uint4 *>(x_s + (size_t)r * kAxLD + ech * 8);
             const float cxv = cxr[P][t];
-            if constexpr (RAG) drop_elems<(int)sizeof(TS)>(pr[P][t], kcs);
+            if constexpr (RAG) drop_elems<(int)sizeof(TP)>(pr[P][t], kcs);
             const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
             const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
             float res[8];
 #pragma unroll
             for (int p = 0; p < 4; p++) {
-                const float plo = F32 ? __uint_as_float(pr[P][t][F32 ? 2 * p : p]) : bf16lo_to_f32(pr[P][t][p]);
-                const float phi_ = F32 ? __uint_as_float(pr[P][t][F32 ? 2 * p + 1 : p]) : bf16hi_to_f32(pr[P][t][p]);
+                const float plo = P32 ? __uint_as_float(pr[P][t][P32 ? 2 * p : p]) : bf16lo_to_f32(pr[P][t][p]);
+                const float phi_ = P32 ? __uint_as_float(pr[P][t][P32 ? 2 * p + 1 : p]) : bf16hi_to_f32(pr[P][t][p]);
                 res[2 * p] = plo + ov[2 * p] - cxv * bf16lo_to_f32(xw[p]);
                 res[2 * p + 1] = phi_ + ov[2 * p + 1] - cxv * bf16hi_to_f32(xw[p]);
             }
@@ -347,23 +363,20 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 
 bool proj_bwd_addx_supported(int n) { return padded_D(n) / 32 <= 3; }
 
-template <int NTD, int SPW, bool PFOP, bool F32, int NW = 4, bool RAG = false, bool SPLIT = false>
+template <int NTD, int SPW, bool PFOP, int ST, int NW = 4, bool SPLIT = false>
 static hipError_t launch_addx(const ProjAddxArgs &a, hipStream_t stream) {
     if constexpr (NW == 4 && !SPLIT) {
-        if (a.per_split < a.B) return launch_addx<NTD, SPW, PFOP, F32, NW, RAG, true>(a, stream);
-    }
-    if constexpr (!F32 && !RAG) {
-        if (a.nC % 8 != 0) return launch_addx<NTD, SPW, PFOP, F32, NW, true, SPLIT>(a, stream);
+        if (a.per_split < a.B) return launch_addx<NTD, SPW, PFOP, ST, NW, true>(a, stream);
     }
     constexpr int SBR = NW * SPW;
     const size_t tiles = sizeof(bf16_t) * (size_t)kAxLD * (32 * NTD + SBR) + sizeof(float) * SBR * kAxLDO;
     const size_t red = sizeof(float) * NW * NTD * 32 * kAxLDR;  // the final cross-wave sum reuses the tiles' memory
     const size_t smem = tiles > red ? tiles : red;
-    hipError_t e = allow_dynamic_lds<&proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG, SPLIT>>(smem);
+    hipError_t e = allow_dynamic_lds<&proj_bwd_addx_kernel<NTD, SPW, PFOP, ST, NW, SPLIT>>(smem);
     if (e != hipSuccess) return e;
     const int slabs = (a.nC + kAxKW - 1) / kAxKW;
     dim3 grid(round_up(slabs, 16), (a.B + a.per_split - 1) / a.per_split + (a.tail_row >= 0 ? (a.tail.nblk * a.tail_parts + round_up(slabs, 16) - 1) / round_up(slabs, 16) : 0));
-    proj_bwd_addx_kernel<NTD, SPW, PFOP, F32, NW, RAG, SPLIT><<<grid, 64 * NW, smem, stream>>>(a);
+    proj_bwd_addx_kernel<NTD, SPW, PFOP, ST, NW, SPLIT><<<grid, 64 * NW, smem, stream>>>(a);
     return hipGetLastError();
 }
 
@@ -391,11 +404,11 @@ int proj_bwd_addx_splits(int B, int n, int C) {
 int proj_bwd_addx_sum_parts(int B, int S) { return S > 1 ? (B + kAxSumRows - 1) / kAxSumRows : 1; }
 
 hipError_t launch_proj_bwd_addx(const void *x, int x_dtype, const void *phi, const void *dPb, const void *dPT, int BP,
-                                const float *cx, float *dphi, int S, void *dx, int B, int n, int C,
+                                const float *cx, float *dphi, int S, const float *dxp, void *dx, int B, int n, int C,
                                 const BatchSumArgs *tail, bool *tail_taken, hipStream_t stream) {
     const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n), NTD = DP / 32;
     ProjAddxArgs a{x, static_cast<const bf16_t *>(phi), static_cast<const bf16_t *>(dPb),
-                   static_cast<const bf16_t *>(dPT), cx, dphi, dx, B, BP, D, DP, nC, S > 1 ? ((B + 127) / 128 + S - 1) / S * 128 : B, -1, B, 1, {}};
+                   static_cast<const bf16_t *>(dPT), cx, dphi, dxp ? dxp : dx, dx, B, BP, D, DP, nC, S > 1 ? ((B + 127) / 128 + S - 1) / S * 128 : B, -1, B, 1, {}};
     if (tail_taken) *tail_taken = false;
     if (tail) {
         a.tail = *tail;
@@ -405,7 +418,8 @@ hipError_t launch_proj_bwd_addx(const void *x, int x_dtype, const void *phi, con
         if (a.tail_parts > 1) a.tail_rows = kAxSumRows;
         if (tail_taken) *tail_taken = true;
     }
-    const bool f32 = x_dtype == kF32AsBF16;
+    const int st = x_dtype == kF32AsBF16 ? kAxF32 : (!dxp ? kAxBf16 : (C % 8 == 0 ? kAxFine : kAxRagged));
+    if (C % 8 != 0 && st != kAxRagged) return hipErrorInvalidValue;
     // D <= 32: the workgroup is sized so that it walks its samples in as few blocks as possible (4, 8 or
     // 12 waves of 32 samples; every block costs two barriers and a round of dependent LDS traffic).
     // Backward at B=320, C=1280, n=4, graphs of ten: 4 waves (three blocks) 16.5 us, 8 waves 16.0, 12 waves
@@ -419,17 +433,22 @@ hipError_t launch_proj_bwd_addx(const void *x, int x_dtype, const void *phi, con
         if ((B + 255) / 256 < best) { nw = 8; best = (B + 255) / 256; }
         if ((B + 383) / 384 < best) nw = 12;
     }
+#define MHC_ADDX(NTD, NW)                                                                                            \
+    return st == kAxBf16 ? launch_addx<NTD, 32, false, kAxBf16, NW>(a, stream)                                       \
+                         : (st == kAxFine ? launch_addx<NTD, 32, false, kAxFine, NW>(a, stream)                      \
+                                          : (st == kAxRagged ? launch_addx<NTD, 32, false, kAxRagged, NW>(a, stream) \
+                                                             : launch_addx<NTD, 32, false, kAxF32, NW>(a, stream)))
     switch (NTD) {
         case 1:
-            // (fp32 storage needs more registers per wave: eight waves at most)
-            if (nw == 12 && !f32) return launch_addx<1, 32, false, false, 12>(a, stream);
-            if (nw == 12) return launch_addx<1, 32, false, true, 8>(a, stream);
-            if (nw == 8) return f32 ? launch_addx<1, 32, false, true, 8>(a, stream) : launch_addx<1, 32, false, false, 8>(a, stream);
-            return f32 ? launch_addx<1, 32, false, true>(a, stream) : launch_addx<1, 32, false, false>(a, stream);
-        case 2: return f32 ? launch_addx<2, 32, false, true>(a, stream) : launch_addx<2, 32, false, false>(a, stream);
-        case 3: return f32 ? launch_addx<3, 32, false, true>(a, stream) : launch_addx<3, 32, false, false>(a, stream);
+            // (fp32 dxp needs more registers per wave: eight waves at most)
+            if (nw == 12 && st == kAxBf16) return launch_addx<1, 32, false, kAxBf16, 12>(a, stream);
+            if (nw >= 8) MHC_ADDX(1, 8);
+            MHC_ADDX(1, 4);
+        case 2: MHC_ADDX(2, 4);
+        case 3: MHC_ADDX(3, 4);
         default: return hipErrorInvalidValue;
     }
+#undef MHC_ADDX
 }
 
 }  // namespace mhc
