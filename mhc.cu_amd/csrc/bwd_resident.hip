@@ -96,7 +96,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     using TD = typename std::conditional<X32, float, TS>::type;      // of dxp
     static_assert(NP == 4 || NP == 8, "stream groups of four");
     using SK = SkSmall<NP>;
-    using CB = CoefBwdSmall<NP, false, true, STATIC>;
+    using CB = CoefBwdSmall<NP, false, true, STATIC, RAG>;
     constexpr int NB = NP / 4;            // stream groups
     constexpr int K = 3 * NP * NP;
     constexpr int TW = TWV;
@@ -294,12 +294,17 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                     // dy * w as a bf16 pair (rounded value + remainder): dHpre is a difference of two
                     // sums built on W1, a single rounding of the products is not enough for it
                     const uint32_t gw[4] = {gr[it][I].x, gr[it][I].y, gr[it][I].z, gr[it][I].w};
-                    uint32_t hw[4], lw[4];
+                    // (the product with a bf16 weight has 16 bits, which the pair holds exactly; with an fp32
+                    // weight ragged rows take the rest of its 24 bits too)
+                    constexpr bool REST = RAG && WMODE == kGramWF32;
+                    uint32_t hw[4], lw[4], rw[4];
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
                         const float p0 = bf16lo_to_f32(gw[k]) * wv[2 * k], p1 = bf16hi_to_f32(gw[k]) * wv[2 * k + 1];
                         hw[k] = pack_bf16x2(p0, p1);
-                        lw[k] = pack_bf16x2(p0 - bf16lo_to_f32(hw[k]), p1 - bf16hi_to_f32(hw[k]));
+                        const float q0 = p0 - bf16lo_to_f32(hw[k]), q1 = p1 - bf16hi_to_f32(hw[k]);
+                        lw[k] = pack_bf16x2(q0, q1);
+                        if constexpr (REST) rw[k] = pack_bf16x2(q0 - bf16lo_to_f32(lw[k]), q1 - bf16hi_to_f32(lw[k]));
                     }
 #pragma unroll
                     for (int J = 0; J < NB; J++) {
@@ -307,6 +312,10 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                         acc[1][I][J] = mfma4(bf16x4_of(hw[2], hw[3]), x1[J], acc[1][I][J]);
                         acc[1][I][J] = mfma4(bf16x4_of(lw[0], lw[1]), x0[J], acc[1][I][J]);
                         acc[1][I][J] = mfma4(bf16x4_of(lw[2], lw[3]), x1[J], acc[1][I][J]);
+                        if constexpr (REST) {
+                            acc[1][I][J] = mfma4(bf16x4_of(rw[0], rw[1]), x0[J], acc[1][I][J]);
+                            acc[1][I][J] = mfma4(bf16x4_of(rw[2], rw[3]), x1[J], acc[1][I][J]);
+                        }
                         acc[2][I][J] = mfma4(x0[I], x0[J], acc[2][I][J]);
                         acc[2][I][J] = mfma4(x1[I], x1[J], acc[2][I][J]);
                     }
@@ -464,7 +473,7 @@ bool bwd_resident_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int 
 template <int NP, int WMODE, bool F32, bool STATIC, int TW, bool RAG = false>
 static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream) {
     using SK = SkSmall<NP>;
-    using CB = CoefBwdSmall<NP, false, true, STATIC>;
+    using CB = CoefBwdSmall<NP, false, true, STATIC, RAG>;
     const size_t smem = sizeof(float) * ((STATIC ? 0 : SK::scaling_floats(ra.r.T)) + CB::kXch);
     int items = (ra.r.C + 128 * TW - 1) / (128 * TW);
     const dim3 grid(ra.r.B);

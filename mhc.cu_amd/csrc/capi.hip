@@ -149,8 +149,10 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     w.upart = c.floats(bs6 > 1 ? (size_t)proj_bwd_addx_sum_parts(B, bs6) * C : 0);
     w.dphi_part = c.floats(bs > 1 ? (size_t)bs * D * nC : 0);
     w.BP = (B + 31) / 32 * 32;
-    w.dPb = reinterpret_cast<unsigned short *>(c.floats(((size_t)w.BP * padded_D(n) + 1) / 2));
-    w.dPT = reinterpret_cast<unsigned short *>(c.floats((size_t)padded_D(n) * w.BP));  // two bf16 planes
+    // planes of bf16: one of dP and two of dP^T, one more each for ragged rows (BP is even)
+    const size_t half_plane = (size_t)w.BP / 2 * padded_D(n);
+    w.dPb = reinterpret_cast<unsigned short *>(c.floats((C % 8 != 0 ? 2 : 1) * half_plane));
+    w.dPT = reinterpret_cast<unsigned short *>(c.floats((C % 8 != 0 ? 3 : 2) * half_plane));
     w.bytes = c.off;
     return w;
 }

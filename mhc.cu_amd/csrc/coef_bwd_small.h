@@ -47,22 +47,25 @@ __device__ __forceinline__ float row16_allreduce(float v) {
 // transpose, plane 0 = value rounded to bf16, plane 1 = the rounding remainder, so that dphi
 // keeps ~16 mantissa bits of dP).  Padded
 // rows d >= D and, from the last sample's workgroup, padded columns b >= B are zeroed.
-struct DPWriter {
+// FINE: one more plane each, the remainder of what the others hold (dphi keeps all 24 bits of dP, dP phi 16).
+template <bool FINE> struct DPWriterT {
     BwdCoefOut o;
     int b, B, DP;
     __device__ __forceinline__ void put(int d, float v) const {
         if (o.dP) o.dP[(size_t)b * DP + d] = v;  // fp32 copy: only the kernels without matrix-core operands read it
         if (o.dPb) {
-            const bf16_t h = f32_to_bf16(v);
             const size_t plane = (size_t)DP * o.BP;
+            const bf16_t h = f32_to_bf16(v);
+            const float rest = v - bf16_to_f32(h);
+            const bf16_t m = f32_to_bf16(rest);
             o.dPb[frag_dpb(b, d, DP)] = h;
             o.dPT[frag_dpt(d, b, o.BP)] = h;
-            o.dPT[plane + frag_dpt(d, b, o.BP)] = f32_to_bf16(v - bf16_to_f32(h));
-            if (b == B - 1)
-                for (int bb = B; bb < o.BP; bb++) {
-                    o.dPT[frag_dpt(d, bb, o.BP)] = 0;
-                    o.dPT[plane + frag_dpt(d, bb, o.BP)] = 0;
-                }
+            o.dPT[plane + frag_dpt(d, b, o.BP)] = m;
+            if constexpr (FINE) {
+                o.dPb[plane + frag_dpb(b, d, DP)] = m;
+                o.dPT[2 * plane + frag_dpt(d, b, o.BP)] = f32_to_bf16(rest - bf16_to_f32(m));
+            }
+            if (b == B - 1) zero_columns(d, plane);
         }
     }
     __device__ __forceinline__ void pad(int D, int first, int step) const {
@@ -70,18 +73,21 @@ struct DPWriter {
             if (o.dP) o.dP[(size_t)b * DP + d] = 0.f;
             if (o.dPb) {
                 const size_t plane = (size_t)DP * o.BP;
-                o.dPb[frag_dpb(b, d, DP)] = 0;
-                o.dPT[frag_dpt(d, b, o.BP)] = 0;
-                o.dPT[plane + frag_dpt(d, b, o.BP)] = 0;
-                if (b == B - 1)
-                    for (int bb = B; bb < o.BP; bb++) {
-                        o.dPT[frag_dpt(d, bb, o.BP)] = 0;
-                        o.dPT[plane + frag_dpt(d, bb, o.BP)] = 0;
-                    }
+#pragma unroll
+                for (int k = 0; k < (FINE ? 2 : 1); k++) o.dPb[k * plane + frag_dpb(b, d, DP)] = 0;
+#pragma unroll
+                for (int k = 0; k < (FINE ? 3 : 2); k++) o.dPT[k * plane + frag_dpt(d, b, o.BP)] = 0;
+                if (b == B - 1) zero_columns(d, plane);
             }
         }
     }
+    __device__ __forceinline__ void zero_columns(int d, size_t plane) const {
+        for (int bb = B; bb < o.BP; bb++)
+#pragma unroll
+            for (int k = 0; k < (FINE ? 3 : 2); k++) o.dPT[k * plane + frag_dpt(d, bb, o.BP)] = 0;
+    }
 };
+using DPWriter = DPWriterT<false>;
 
 // =============================================================================================
 // n <= 8, dynamic H: coefficient backward of one sample on the lanes of one SkSmall group (16 lanes
@@ -96,7 +102,8 @@ struct DPWriter {
 // STATIC (with GRAM): shared coefficients - prefetch() takes H from the [n] vectors and nothing else, and
 // run() stops after the channel-sum vectors: it writes the sample's raw gradients (dM | dHpre | dHpost)
 // as a row of `red` for the batch-sum launch; the Sinkhorn backward then runs once on the batch total.
-template <int NP, bool PRECISE, bool GRAM, bool STATIC = false> struct CoefBwdSmall {
+// FINE: dP in the planes of DPWriterT<true>.
+template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = false> struct CoefBwdSmall {
     using SK = SkSmall<NP>;
     static constexpr int K = GRAM ? 3 * NP * NP : NP * NP + 3 * NP + 1;
     // LDS floats next to the Sinkhorn denominators, per group: the column results of the Gram sums
@@ -215,7 +222,7 @@ template <int NP, bool PRECISE, bool GRAM, bool STATIC = false> struct CoefBwdSm
             return;
         }
         float *dt = a.out.dt + (size_t)b * (D + 3);
-        const DPWriter dpw{a.out, b, a.B, a.DP};
+        const DPWriterT<FINE> dpw{a.out, b, a.B, a.DP};
         float S0 = 0.f, S1 = 0.f, S2 = 0.f;  // sum_d dt_d p_d per alpha group
         if (g < n) {
             const float dHpost = tpost;

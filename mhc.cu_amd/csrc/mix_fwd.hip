@@ -300,7 +300,8 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
         MHC_PHASE(kPhaseFwdFused, b, 2);
         if (tid < SK::kGroup) {
             // bf16 tier: hardware exp2 / reciprocal / square root (1 ulp) instead of the library routines
-            constexpr bool kFast = !std::is_same<TX, float>::value;
+            // (ragged rows: the library routines, as the general kernels for them use)
+            constexpr bool kFastSk = !std::is_same<TX, float>::value, kFast = kFastSk && !RAG;
             float rinv = 0.f;
             if (dyn) {
                 const float ms = ssq * (1.0f / (float)(n * C)) + a.eps;
@@ -339,8 +340,8 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
             // scalings (m * s * rho) without a bias that grows with the iteration count
             // (the same arithmetic with and without the state: the dynamic forward result does not depend
             // on whether the caller keeps it; static H has no state to undo and takes the reciprocals)
-            if (dyn && a.sk_state) SK::template forward_save<!kFast>(m, g, n, a.T, a.eps, a.sk_state + (size_t)b * SK::state_floats(a.T));
-            else if (dyn) SK::template forward<!kFast, false>(m, g, n, a.T, a.eps, nullptr, tid);
+            if (dyn && a.sk_state) SK::template forward_save<!kFastSk>(m, g, n, a.T, a.eps, a.sk_state + (size_t)b * SK::state_floats(a.T));
+            else if (dyn) SK::template forward<!kFastSk, false>(m, g, n, a.T, a.eps, nullptr, tid);
             else SK::template forward<false, false>(m, g, n, a.T, a.eps, nullptr, tid);
             coef_s[r0 * NP + c0] = m[0];
             if (wr && a.M && mv) a.M[ms + r0 * n + c0] = m[0];
@@ -375,7 +376,9 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
     // + remainder), the lane receives four output streams of its own channel; for n > 4 the streams
     // form two groups of four and M is 2 x 2 such blocks.  With the products on the VALU this kernel
     // is bound by VALU issue once several workgroups share a CU.
-    constexpr bool kMixMfma = std::is_same<TX, bf16_t>::value && V == 8;
+    // Ragged rows stay on the VALU, where the coefficients keep their 24 bits: y (fp32 from bf16 x) and q are off by
+    // 1e-7 instead of 2e-6.
+    constexpr bool kMixMfma = std::is_same<TX, bf16_t>::value && V == 8 && !RAG;
     if constexpr (kMixMfma) {
         constexpr int NB = NP / 4;  // stream groups
         const int jq = tid & 3;
@@ -452,11 +455,7 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
             if (inject) {
                 get_act<RX>(fr[k], f);
             } else {
-                if (RAG && c + V > C) {  // the row's last chunk: behind its end any finite value will do
-#pragma unroll
-                    for (int v = 0; v < V; v++) f[v] = load_w(a.w, a.w_bf16, min(c + v, C - 1));
-                }
-                else if (a.w_bf16) load_vec<bf16_t, V>(static_cast<const bf16_t *>(a.w) + c, f);
+                if (a.w_bf16) load_vec<bf16_t, V>(static_cast<const bf16_t *>(a.w) + c, f);
                 else load_vec<float, V>(static_cast<const float *>(a.w) + c, f);
             }
             uint32_t yw[NP][2];  // packed first half (bf16 output), stored with the second
@@ -502,24 +501,14 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
                             yw[i][0] = pack_bf16x2(o0, o1); yw[i][1] = pack_bf16x2(o2, o3);
                         } else if (i < n && ch < nch) {
                             TY *yp = yb + (size_t)i * C + c;
-                            const uint32_t w4[4] = {yw[i][0], yw[i][1], pack_bf16x2(o0, o1), pack_bf16x2(o2, o3)};
-                            if constexpr (!RAG) {
-                                st16<true>(yp, w4[0], w4[1], w4[2], w4[3]);
-                            } else if (c + V <= C) {
-                                st16_any<true>(yp, w4[0], w4[1], w4[2], w4[3]);
-                            } else {
-#pragma unroll
-                                for (int v = 0; v < V; v++)
-                                    if (c + v < C) yp[v] = (bf16_t)(v & 1 ? w4[v / 2] >> 16 : w4[v / 2] & 0xffffu);
-                            }
+                            st16<true>(yp, yw[i][0], yw[i][1], pack_bf16x2(o0, o1), pack_bf16x2(o2, o3));
                         }
                     } else {
                         if (h == 0) {
                             yf[i][0] = o0; yf[i][1] = o1; yf[i][2] = o2; yf[i][3] = o3;
                         } else if (i < n && ch < nch) {
                             const float out[V] = {yf[i][0], yf[i][1], yf[i][2], yf[i][3], o0, o1, o2, o3};
-                            if constexpr (RAG) store_vec_any<TY, V, true>(yb + (size_t)i * C + c, out, C - c);
-                            else store_vec<TY, V, true>(yb + (size_t)i * C + c, out);
+                            store_vec<TY, V, true>(yb + (size_t)i * C + c, out);
                         }
                     }
                 }
@@ -527,11 +516,11 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
         }
     } else {
         // ---- 3. aggregate + RMS ------------------------------------------------------------------
-        // (VALU path: fp32 x.)  The tile stays in registers as raw
-        // words; LEAN (two chunks per thread) widens a stream at the point of use instead of holding
+        // (VALU path: fp32 x, ragged rows.)  The tile stays in registers as raw
+        // words; LEAN (two chunks per thread, bf16) widens a stream at the point of use instead of holding
         // the fp32 copy of the whole tile, which keeps the register count down; the extra
         // conversions are cheaper than a second round of the grid.
-        constexpr bool LEAN = CPT >= 2 && NP <= 4 && !std::is_same<TX, float>::value;
+        constexpr bool LEAN = (RAG || (CPT >= 2 && NP <= 4)) && !std::is_same<TX, float>::value;
         float xv[LEAN ? 1 : CPT][NP][V];
         if constexpr (!LEAN) {
 #pragma unroll

@@ -66,7 +66,10 @@ constexpr int kAxLDR = 36;         // LDS pitch of the dphi tiles in the final c
 //              storage case; dxp is read and dx written as fp32)
 //   kAxFine    bf16, dxp fp32 in a buffer of its own (dx is rounded once)
 //   kAxRagged  the same for rows of any length (C % 8 != 0): the last chunk of a row is loaded from nC - 8 on and
-//              shifted down
+//              shifted down; dP in one more bf16 plane each (dphi: three, 24 bits; dP phi: two), so that the
+//              gradients are as good as from the fp32 arithmetic of the general kernels (dphi off by 2e-7, with
+//              two planes 3e-6; B=333 n=3 C=1230 backward 19.7 us with two planes and dxp in bf16, 22.6 with
+//              three and dxp in fp32, 46.6 in the general kernels; B=130 n=8 C=643 20.7, 30.1, 160.9)
 // NW: waves per workgroup (a block is NW * SPW samples).
 // SPLIT: blockIdx.y is a batch split (a template argument: with a run-time first sample the compiler keeps fewer
 // loads in flight, B=1000 n=6 C=1024 17.2 -> 21.2 us without any split).
@@ -175,7 +178,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
     // Operands that come straight from global memory in fragment order: dP^T (rounded value and
     // remainder) of this wave's samples for every dphi tile, and dP of its sample tiles.  Steps and
     // tiles beyond the padded batch read zeros.
-    constexpr int TPL = 2, BPL = 1, HELD = 2;  // planes of dP^T and of dP, planes of dP^T requested here
+    // (the planes that only ragged rows have are fetched where they are used: held from here they spill)
+    constexpr int TPL = RAG ? 3 : 2, BPL = RAG ? 2 : 1;  // planes of dP^T and of dP
+    constexpr int HELD = RAG && NTD == 3 ? 1 : 2;        // planes of dP^T requested here
     const size_t plane = (size_t)a.DP * a.BP;
     auto load_at = [&](int sb, int p, int m, int ks) {
         const int nsteps = a.BP >> 4, step = (sb >> 4) + KS * wave + ks;
