@@ -6,7 +6,9 @@
 // workgroups of a large kernel that comes last in the stream anyway.  One block = 64 columns x RG
 // row groups; float64 accumulation: dalpha is a sum of B * n^2 terms of mixed sign whose total can be a
 // hundred times smaller than the terms, and a float32 running sum loses what the 1e-5 parity tier
-// needs.  The terms themselves stay float32.
+// needs.  The terms themselves (a sample's row, or the row of a few samples that one workgroup added up) are
+// float32; where a split batch makes the sums in two launches, the parts in between are float64 too
+// (rows of the same layout, BatchSumArgs::rows64 / OUT64).
 #pragma once
 #include "mhc_common.h"
 
@@ -21,22 +23,48 @@ struct DwOut {
 };
 
 struct BatchSumArgs {
-    const float *u; int rows_u, C; void *dw;
-    const float *dt; int rows_dt, D; float *dbias, *dalpha;
+    const void *u; int rows_u, C; void *dw;
+    const void *dt; int rows_dt, D; float *dbias, *dalpha;
     int nblk;  // blocks of 64 columns
     bool dw_bf16;
+    bool rows64;  // u and dt are rows of float64 (else float32)
 };
 
-inline BatchSumArgs make_batch_sums(const float *u, int rows_u, int C, DwOut dw, const float *dt, int rows_dt,
-                                    int D, float *dbias, float *dalpha) {
+inline BatchSumArgs make_batch_sums(const void *u, int rows_u, int C, DwOut dw, const void *dt, int rows_dt,
+                                    int D, float *dbias, float *dalpha, bool rows64 = false) {
     const int ncols = (dw ? C : 0) + (dt ? D + 3 : 0);  // dt == nullptr: the u columns only
-    return BatchSumArgs{u, rows_u, C, dw.p, dt, rows_dt, D, dbias, dalpha, (ncols + 63) / 64, dw.bf16};
+    return BatchSumArgs{u, rows_u, C, dw.p, dt, rows_dt, D, dbias, dalpha, (ncols + 63) / 64, dw.bf16, rows64};
+}
+
+// Sum of src[r * ld] over r = first, first + RG, ... < rows.
+template <int RG, typename T> __device__ __forceinline__ double batch_sum_column(const T *src, int ld, int first, int rows) {
+    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+    int r = first;
+    // many rows (per-sample rows of a large batch): sixteen loads in flight, the round trips decide
+    for (; r + 15 * RG < rows; r += 16 * RG) {
+        T t[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) t[k] = src[(size_t)(r + k * RG) * ld];
+#pragma unroll
+        for (int k = 0; k < 16; k += 4) {
+            a0 += (double)t[k]; a1 += (double)t[k + 1]; a2 += (double)t[k + 2]; a3 += (double)t[k + 3];
+        }
+    }
+    for (; r + 3 * RG < rows; r += 4 * RG) {
+        const T t0 = src[(size_t)r * ld], t1 = src[(size_t)(r + RG) * ld];
+        const T t2 = src[(size_t)(r + 2 * RG) * ld], t3 = src[(size_t)(r + 3 * RG) * ld];
+        a0 += (double)t0; a1 += (double)t1; a2 += (double)t2; a3 += (double)t3;
+    }
+    for (; r < rows; r += RG) a0 += (double)src[(size_t)r * ld];
+    return (a0 + a1) + (a2 + a3);
 }
 
 // red: RG * (CW + 1) doubles of LDS; called by all CW * RG threads of the workgroup (contains a barrier).
-// CW = columns per block: 64, or 32 (still whole 128-byte lines per row) where twice the blocks are
+// CW = columns per block: 64, or fewer (down to 16, half a 128-byte line per row) where more blocks are
 // wanted; a.nblk must count blocks of CW columns.
-template <int RG, int CW = 64>
+// IN64: a.rows64 is looked at (otherwise the rows are float32).  OUT64: the results are parts of sums, one row of
+// float64 in dw ([C]) and in dbias ([D + 3], dalpha unused).
+template <int RG, int CW = 64, bool IN64 = false, bool OUT64 = false>
 __device__ __forceinline__ void batch_sum_block(const BatchSumArgs &a, int blk, int tid, double *red) {
     const int cl = tid % CW, rg = tid / CW;
     const int col = blk * CW + cl;
@@ -45,28 +73,10 @@ __device__ __forceinline__ void batch_sum_block(const BatchSumArgs &a, int blk, 
     double acc = 0.0;
     if (col < ncols) {
         const bool is_u = col < ncol_u;
-        const float *src = is_u ? a.u + col : a.dt + (col - ncol_u);
-        const int ld = is_u ? a.C : a.D + 3;
-        const int rows = is_u ? a.rows_u : a.rows_dt;
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-        int r = rg;
-        // many rows (per-sample rows of a large batch): sixteen loads in flight, the round trips decide
-        for (; r + 15 * RG < rows; r += 16 * RG) {
-            float t[16];
-#pragma unroll
-            for (int k = 0; k < 16; k++) t[k] = src[(size_t)(r + k * RG) * ld];
-#pragma unroll
-            for (int k = 0; k < 16; k += 4) {
-                a0 += (double)t[k]; a1 += (double)t[k + 1]; a2 += (double)t[k + 2]; a3 += (double)t[k + 3];
-            }
-        }
-        for (; r + 3 * RG < rows; r += 4 * RG) {
-            const float t0 = src[(size_t)r * ld], t1 = src[(size_t)(r + RG) * ld];
-            const float t2 = src[(size_t)(r + 2 * RG) * ld], t3 = src[(size_t)(r + 3 * RG) * ld];
-            a0 += (double)t0; a1 += (double)t1; a2 += (double)t2; a3 += (double)t3;
-        }
-        for (; r < rows; r += RG) a0 += (double)src[(size_t)r * ld];
-        acc = (a0 + a1) + (a2 + a3);
+        const void *base = is_u ? a.u : a.dt;
+        const int at = is_u ? col : col - ncol_u, ld = is_u ? a.C : a.D + 3, rows = is_u ? a.rows_u : a.rows_dt;
+        if (IN64 && a.rows64) acc = batch_sum_column<RG>(static_cast<const double *>(base) + at, ld, rg, rows);
+        else acc = batch_sum_column<RG>(static_cast<const float *>(base) + at, ld, rg, rows);
     }
     red[rg * (CW + 1) + cl] = acc;
     __syncthreads();
@@ -74,7 +84,10 @@ __device__ __forceinline__ void batch_sum_block(const BatchSumArgs &a, int blk, 
         double v = 0.0;
 #pragma unroll
         for (int i = 0; i < RG; i++) v += red[i * (CW + 1) + cl];
-        if (col < ncol_u) {
+        if constexpr (OUT64) {
+            if (col < ncol_u) static_cast<double *>(a.dw)[col] = v;
+            else reinterpret_cast<double *>(a.dbias)[col - ncol_u] = v;
+        } else if (col < ncol_u) {
             if (a.dw_bf16) static_cast<unsigned short *>(a.dw)[col] = f32_to_bf16((float)v);
             else static_cast<float *>(a.dw)[col] = (float)v;
         }

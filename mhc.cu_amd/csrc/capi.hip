@@ -9,6 +9,7 @@
 #include "phase_profiler.h"
 #include "tuning.h"
 
+#include <algorithm>
 #include <mutex>
 #include <stdint.h>
 
@@ -127,7 +128,6 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     w.cx = c.floats(B);
     w.s1 = c.floats(B);
     w.u = c.floats((size_t)B * C);
-    w.dtpart = c.floats((size_t)B * (D + 3));
     w.raw = c.floats(bwd_reduce_raw_floats(B, n, C));
     w.s1part = c.floats(n > 8 ? (size_t)B * bwd_reduce_parts(B, n, C) : 0);
     // wide projections: the part of dx that is formed beside the coefficient backward, fp32
@@ -146,7 +146,10 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     if (bs5 > bs) bs = bs5;
     const int bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
     if (bs6 > bs) bs = bs6;
-    w.upart = c.floats(bs6 > 1 ? (size_t)proj_bwd_addx_sum_parts(B, bs6) * C : 0);
+    // partial sums of a split batch: float32 rows of at most B, float64 rows of the resident backward's second launch
+    const size_t parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
+    w.upart = c.floats(2 * parts64 * C);
+    w.dtpart = c.floats(std::max((size_t)B, 2 * parts64) * (D + 3));
     w.dphi_part = c.floats(bs > 1 ? (size_t)bs * D * nC : 0);
     w.BP = (B + 31) / 32 * 32;
     // planes of bf16: one of dP and two of dP^T, one more each for ragged rows (BP is even)
@@ -642,12 +645,12 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         if (S > 1) {
             // partial sums of dphi, dw, dbias and dalpha, added up by one more launch
             const BatchSumArgs sums = make_batch_sums(ws.u, B, C, dwo ? DwOut{ws.upart, false} : dwo, ws.dt, B, D, ws.dtpart,
-                                                      ws.dtpart + D);
+                                                      nullptr);
             MHC_LAUNCH(launch_proj_bwd_addx(x, x_dtype, phi, ws.dPb, ws.dPT, ws.BP, ws.cx, ws.dphi_part, S, dxp, dx, B, n, C, &sums,
                                             &tail_taken, st));
             if (!tail_taken) return MHC_ERR_LAUNCH;  // not reached: any number of workgroups can carry the parts
             MHC_LAUNCH(launch_finalize(ws.upart, parts, C, dwo, ws.dtpart, parts, D, dbias, dalpha, ws.dphi_part, S,
-                                       (size_t)D * n * C, dphi, st));
+                                       (size_t)D * n * C, dphi, st, true));
             return MHC_OK;
         }
         const BatchSumArgs sums = make_batch_sums(ws.u, B, C, dwo, ws.dt, B, D, dbias, dalpha);

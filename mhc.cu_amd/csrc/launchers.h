@@ -203,10 +203,11 @@ hipError_t launch_bwd_slab_f32(const float *dy, const float *x, const void *w, i
 int bwd_dx_samples_per_group(int B, int n);
 
 // One launch for all remaining batch sums: u [rows_u, C] -> dw (skipped when dw == nullptr),
-// dt [rows_dt, D+3] -> dbias, dalpha, and (S > 1) dphi_part [S, dphi_elems] -> dphi.
-hipError_t launch_finalize(const float *u, int rows_u, int C, DwOut dw, const float *dt, int rows_dt,
+// dt [rows_dt, D+3] -> dbias, dalpha, and (S > 1) dphi_part [S, dphi_elems] -> dphi.  rows64: u and dt are float64
+// (parts of sums), otherwise float32.
+hipError_t launch_finalize(const void *u, int rows_u, int C, DwOut dw, const void *dt, int rows_dt,
                            int D, float *dbias, float *dalpha, const float *dphi_part, int S,
-                           size_t dphi_elems, float *dphi, hipStream_t stream);
+                           size_t dphi_elems, float *dphi, hipStream_t stream, bool rows64 = false);
 
 // Matrix-core projection backward (x and phi bf16, C % 8 == 0): dphi = dP^T x_flat and
 // dxflat = dP phi (bf16 [B, nC]) in one pass over x and phi.  With S = proj_bwd_batch_splits() > 1
@@ -251,8 +252,8 @@ hipError_t launch_bwd_resident_static(const void *dy, const void *x, const void 
 // dphi = dP^T x_flat without batch split, dx completed in place (dx = dxp + dP phi - cx x), and `tail`
 // (dw, dbias, dalpha) summed by extra workgroups when the grid has room (*tail_taken).
 bool proj_bwd_addx_supported(int n);
-// batch splits S: with more than one, dphi holds S planes [D, nC] and the outputs of `tail` (fp32) proj_bwd_addx_sum_parts()
-// rows ([C] and [D + 3]) of partial sums
+// batch splits S: with more than one, dphi holds S planes [D, nC] and the outputs dw and dbias of `tail`
+// proj_bwd_addx_sum_parts() rows ([C] and [D + 3]) of partial sums in float64
 int proj_bwd_addx_splits(int B, int n, int C);
 int proj_bwd_addx_sum_parts(int B, int S);
 // dxp: nullptr (in dx, stored like it), or fp32 where bwd_resident_dxp_f32() holds

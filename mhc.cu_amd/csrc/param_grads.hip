@@ -149,7 +149,7 @@ __global__ __launch_bounds__(1024) void finalize_kernel(FinalizeArgs a) {
     __shared__ double red[16 * 65];
     const int tid = threadIdx.x;
     if ((int)blockIdx.x < a.sums.nblk) {
-        batch_sum_block<16>(a.sums, blockIdx.x, tid, red);
+        batch_sum_block<16, 64, true>(a.sums, blockIdx.x, tid, red);
         return;
     }
     // dphi partial sums: one float per thread per 1024-column block (coalesced)
@@ -172,10 +172,10 @@ __global__ __launch_bounds__(1024) void finalize_kernel(FinalizeArgs a) {
     }
 }
 
-hipError_t launch_finalize(const float *u, int rows_u, int C, DwOut dw, const float *dt, int rows_dt,
+hipError_t launch_finalize(const void *u, int rows_u, int C, DwOut dw, const void *dt, int rows_dt,
                            int D, float *dbias, float *dalpha, const float *dphi_part, int S,
-                           size_t dphi_elems, float *dphi, hipStream_t stream) {
-    const BatchSumArgs sums = make_batch_sums(u, rows_u, C, dw, dt, rows_dt, D, dbias, dalpha);
+                           size_t dphi_elems, float *dphi, hipStream_t stream, bool rows64) {
+    const BatchSumArgs sums = make_batch_sums(u, rows_u, C, dw, dt, rows_dt, D, dbias, dalpha, rows64);
     const int nblk_a = sums.nblk;
     const int nblk_b = S > 1 ? (int)((dphi_elems + 1023) / 1024) : 0;
     FinalizeArgs a{sums, dphi_part, S, dphi_elems, dphi};

@@ -98,14 +98,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         BatchSumArgs s = a.tail;
         const int r0 = part * a.tail_rows, rows = min(a.tail_rows, a.B - r0);
         s.rows_u = s.rows_dt = rows;
-        s.u += (size_t)r0 * s.C;
-        s.dt += (size_t)r0 * (s.D + 3);
-        if (a.tail_parts > 1) {  // fp32 rows, added up by the launch that follows
-            s.dw = s.dw ? static_cast<float *>(s.dw) + (size_t)part * s.C : nullptr;
-            s.dbias += (size_t)part * (s.D + 3);
-            s.dalpha += (size_t)part * (s.D + 3);
+        s.u = static_cast<const float *>(s.u) + (size_t)r0 * s.C;
+        s.dt = static_cast<const float *>(s.dt) + (size_t)r0 * (s.D + 3);
+        double *red = reinterpret_cast<double *>(ax_smem);
+        if constexpr (SPLIT) {  // rows of float64, added up by the launch that follows
+            if (s.dw) s.dw = static_cast<double *>(s.dw) + (size_t)part * s.C;
+            s.dbias = reinterpret_cast<float *>(reinterpret_cast<double *>(s.dbias) + (size_t)part * (s.D + 3));
+            batch_sum_block<NT_ / kAxSumCols, kAxSumCols, false, true>(s, id % s.nblk, tid, red);
+        } else {
+            batch_sum_block<NT_ / kAxSumCols, kAxSumCols>(s, id % s.nblk, tid, red);
         }
-        batch_sum_block<NT_ / kAxSumCols, kAxSumCols>(s, id % s.nblk, tid, reinterpret_cast<double *>(ax_smem));
         return;
     }
     // Workgroup ids go round robin over the 8 XCDs (each with its own L2, 128-byte lines).  A slab

@@ -60,3 +60,56 @@ def test_ragged_rows_of_shared_coefficients_keep_float32_results(B, n, C):
     y_ref, ref = nm.mhc_static_fwd_bwd(x, p, dy, T, EPS, dtype=torch.float64)
     y, got = hip_static(x, p, dy, T, EPS, act_dtype=torch.bfloat16)
     assert rel2(y, y_ref) <= 5e-7 and rel2(got["w"], ref["w"]) <= 1e-6
+
+
+
+def _batch_and_single_sums(B, n, C, act):
+    """dw, dbias and dalpha of one backward call over B samples, and of B calls over one sample each on the same saved
+    state, whose results are the terms of those sums; every sample comes twice, with dy and with -dy, in random order,
+    so that the sums are far smaller than what is added up on the way."""
+    from mhc import _lib
+    lib, D, dev = _lib.lib, n * n + 2 * n, "cuda"
+    x, dy, p = _dynamic(B // 2, n, C)
+    order = torch.randperm(B, generator=torch.Generator().manual_seed(6))
+    x, dy = torch.cat([x, x])[order].to(dev, act), torch.cat([dy, -dy])[order].to(dev, act)
+    phi = torch.cat([p["phi_pre"], p["phi_post"], p["phi_res"]]).to(dev, act)
+    bias = torch.cat([p["b_pre"], p["b_post"], p["b_res"].reshape(-1)]).to(dev)
+    alpha, w = torch.full((3,), 0.1, device=dev), p["w"].to(dev)
+    code = _lib.dtype_code(x)
+    empty = lambda *s: torch.full(s, float("nan"), device=dev)
+    H_pre, H_post, M, P, r, q = empty(B, n), empty(B, n), empty(B, n, n), empty(B, D), empty(B), empty(B)
+    sk = empty(B, lib.mhc_layer_sinkhorn_state_floats(1, n, T))
+    y, dx = torch.empty_like(x), torch.empty_like(x)
+    size = lib.mhc_layer_dynamic_workspace_bytes(B, n, C)
+    ws, stream = _lib.workspace(x.device, size), _lib.stream_ptr(x.device)
+    at = _lib.ptr
+    _lib.check("fwd", lib.mhc_layer_fwd_dynamic(at(x), code, at(w), 0, at(phi), code, at(bias), at(alpha), None, at(y), code,
+                                                at(H_pre), at(H_post), at(M), at(P), at(r), at(q), at(sk), B, n, C, T, EPS,
+                                                at(ws), ws.numel(), stream))
+
+    def backward(i, count, out):
+        dw, db = out[:C], out[C:]
+        _lib.check("bwd", lib.mhc_layer_bwd_dynamic(
+            at(dy[i]), code, at(x[i]), code, at(w), 0, at(phi), code, at(bias), at(alpha), None, at(H_pre[i]), at(H_post[i]),
+            at(M[i]), at(P[i]), at(r[i:]), at(q[i:]), at(sk[i]), at(dx[i]), None, at(dw), at(dphi), at(db), at(db[D:]), count,
+            n, C, T, EPS, at(ws), ws.numel(), stream))
+
+    dphi, whole, terms = empty(D, n * C), empty(C + D + 3), empty(B, C + D + 3)
+    backward(0, B, whole)
+    for i in range(B):
+        backward(i, 1, terms[i])
+    torch.cuda.synchronize()
+    return whole.double(), terms.double()
+
+
+# The sums are float64 and rounded to float32 at the end; parts of 128 samples in float32 would be off by 1e-7 of the
+# parts, thousands of times this bound.
+def _close_to_float64(whole, terms):
+    total = terms.sum(0)
+    off, bound = (whole - total).abs(), 2.0 ** -23 * total.abs() + 2.0 ** -45 * terms.abs().sum(0)
+    assert torch.isfinite(whole).all() and (off <= bound).all(), float((off / bound.clamp_min(1e-300)).max())
+
+
+@pytest.mark.parametrize("B,n,C", [(1536, 8, 64), (2050, 6, 16), (1794, 2, 44), (1600, 7, 48), (1922, 4, 42)])
+def test_split_batch_sums_stay_in_float64(B, n, C):
+    _close_to_float64(*_batch_and_single_sums(B, n, C, torch.bfloat16))
