@@ -13,14 +13,15 @@
 // 16.  The products run on v_mfma_f32_16x16x4_f32 (IEEE fp32): the tile is 16 samples x 16 channels, a lane holds
 // the two channels 2 l, 2 l + 1 (l = lane & 15; one per product column tile) of the four samples 4 g .. 4 g + 3
 // (g = lane / 16), which is at once
-//   * the layout of an accumulator (dx: rows = samples), so the mixing is lane-local arithmetic that
-//     initialises the accumulator of dP phi, and
+//   * the layout of an accumulator (dx: rows = samples), so the mixing is lane-local arithmetic on the
+//     accumulator of dP phi, and
 //   * the layout of the right-hand operand of dphi (contraction over samples: product i takes sample 4 g + i),
 // so x and dy go from memory into registers in 128-byte pieces and nothing but the samples' coefficients and dP
 // passes through LDS (wave-private, no barrier).  D <= 24 rows of phi are 6 products of depth 4 (row 6 g + s in
 // product s) and stay in LDS.  dphi stays in registers for the whole range of samples and is added up over
-// the four waves at the end; with the batch split S ways the copies are summed by the finalize launch.
-// About 200 registers: two workgroups per CU, which hide each other's loads.
+// the four waves at the end; with the batch split S ways the copies are summed by the finalize launch.  The sums over
+// samples of dw and dt are float64 from the first sample on (batch_sums.h).
+// 206 (n = 3) and 249 (n = 4) registers: two workgroups per CU, which hide each other's loads.
 #include "launchers.h"
 #include "mhc_common.h"
 
@@ -39,7 +40,8 @@ constexpr int sf_phi_pitch(int n) { return (n * 32 + 16) / 32 * 32 + 16; }
 struct SlabF32Args {
     const float *dy, *x, *w_f32; const bf16_t *w_bf16;
     const float *phi, *Hpre, *Hpost, *M, *q, *s1, *cx, *dP, *dt;
-    float *dx, *df, *dphi, *dw_part, *dt_part;
+    float *dx, *df, *dphi;
+    double *dw_part, *dt_part;
     int B, C, D, slabs, per_split, per_wave;  // samples
 };
 
@@ -65,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32_kernel(SlabF32Args a) {
             double v = 0.0;
 #pragma unroll
             for (int i = 0; i < 8; i++) v += red[i * 32 + tid];
-            a.dt_part[(size_t)blockIdx.y * (D + 3) + tid] = (float)v;
+            a.dt_part[(size_t)blockIdx.y * (D + 3) + tid] = v;
         }
         return;
     }
@@ -94,7 +96,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32_kernel(SlabF32Args a) {
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int v = 0; v < 2; v++) dphi[j][t][v] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float usum[2] = {0.f, 0.f};
+    double usum[2] = {0.0, 0.0};
 
     const uint32_t off0 = 4u * (uint32_t)cl, row_bytes = 4u * (uint32_t)nC;  // 15 rows of at most 4 * 32768 floats
     const int w0 = s0 + __builtin_amdgcn_readfirstlane(wave) * a.per_wave, w1 = min(s1, w0 + a.per_wave);
@@ -140,33 +142,48 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32_kernel(SlabF32Args a) {
         // (a wave's LDS accesses complete in order; the fence keeps the compiler from reordering them)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        auto ld4 = [](float *d, const float *s) {
+            const float4 t = *reinterpret_cast<const float4 *>(s);
+            d[0] = t.x; d[1] = t.y; d[2] = t.z; d[3] = t.w;
+        };
+        if (INJECT && a.df) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float hpost[4];
+                ld4(hpost, co + (4 * g + i) * kSfCo + 20);
+                float2 d = make_float2(0.f, 0.f);
+#pragma unroll
+                for (int j = 0; j < N; j++) { d.x += hpost[j] * gv[j][i].x; d.y += hpost[j] * gv[j][i].y; }
+                if (cok && b0 + 4 * g + i < w1)
+                    *reinterpret_cast<float2 *>(reinterpret_cast<char *>(a.df + (size_t)b0 * C) + off0 + (4 * g + i) * 4u * (uint32_t)C) = d;
+            }
+        }
         // mixing part of dx, lane-local
         f32x4_t out[N][2];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const float *cb = co + (4 * g + i) * kSfCo;
             float m[4 * N], hpre[4], hpost[4], k3[4];
-            auto ld4 = [](float *d, const float *s) {
-                const float4 t = *reinterpret_cast<const float4 *>(s);
-                d[0] = t.x; d[1] = t.y; d[2] = t.z; d[3] = t.w;
-            };
 #pragma unroll
             for (int k = 0; k < N; k++) ld4(m + 4 * k, cb + 4 * k);
-            ld4(hpre, cb + 16); ld4(hpost, cb + 20); ld4(k3, cb + 24);
+            if (!INJECT) { ld4(hpre, cb + 16); ld4(hpost, cb + 20); }
+            ld4(k3, cb + 24);
 #pragma unroll
             for (int v = 0; v < 2; v++) {
-                float s_a = 0.f, s_df = 0.f;
+                float da = 0.f;
+                if constexpr (!INJECT) {
+                    float s_a = 0.f, s_df = 0.f;
 #pragma unroll
-                for (int j = 0; j < N; j++) {
-                    s_a += hpre[j] * (v ? xv[j][i].y : xv[j][i].x);
-                    s_df += hpost[j] * (v ? gv[j][i].y : gv[j][i].x);
+                    for (int j = 0; j < N; j++) {
+                        s_a += hpre[j] * (v ? xv[j][i].y : xv[j][i].x);
+                        s_df += hpost[j] * (v ? gv[j][i].y : gv[j][i].x);
+                    }
+                    da = s_df * w[v] * k3[0] - s_a * k3[1];
+                    usum[v] += (double)(s_df * s_a * k3[0]);
                 }
-                const float da = s_df * w[v] * k3[0] - s_a * k3[1];
-                usum[v] += s_df * s_a * k3[0];
-                if (INJECT && a.df && cok && b0 + 4 * g + i < w1) a.df[(size_t)(b0 + 4 * g + i) * C + c + v] = s_df;
 #pragma unroll
                 for (int j = 0; j < N; j++) {
-                    float o = hpre[j] * da - k3[2] * (v ? xv[j][i].y : xv[j][i].x);
+                    float o = (INJECT ? 0.f : hpre[j] * da) - k3[2] * (v ? xv[j][i].y : xv[j][i].x);
 #pragma unroll
                     for (int k = 0; k < N; k++) o += m[4 * k + j] * (v ? gv[k][i].y : gv[k][i].x);
                     out[j][v][i] = o;
@@ -174,16 +191,23 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32_kernel(SlabF32Args a) {
             }
             __builtin_amdgcn_sched_barrier(0);  // one sample's coefficients at a time: registers
         }
-        // + dP phi: product s, left operand lane (sample l, rows 6 g + s of dP)
+        // + dP phi: product s, left operand lane (sample l, rows 6 g + s of dP).  Summed up by itself and added once: in the
+        // accumulator of the mixing part each of the 24 steps would be rounded at the size of dx (error of dx 1.5e-7
+        // instead of 9e-8).
+        float av[nDp];
 #pragma unroll
-        for (int s = 0; s < nDp; s++) {
-            const float av = dp[l * kSfDp + nDp * g + s];
+        for (int s = 0; s < nDp; s++) av[s] = dp[l * kSfDp + nDp * g + s];
 #pragma unroll
-            for (int j = 0; j < N; j++) {
+        for (int j = 0; j < N; j++) {
+            f32x4_t t[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int s = 0; s < nDp; s++) {
                 const float2 ph = *reinterpret_cast<const float2 *>(phi_s + (nDp * g + s) * PP + j * 32 + 2 * l);
-                out[j][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, ph.x, out[j][0], 0, 0, 0);
-                out[j][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, ph.y, out[j][1], 0, 0, 0);
+                t[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], ph.x, t[0], 0, 0, 0);
+                t[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], ph.y, t[1], 0, 0, 0);
             }
+            out[j][0] += t[0];
+            out[j][1] += t[1];
             __builtin_amdgcn_sched_barrier(0);
         }
         // dphi: product i contracts samples 4 g + i, left operand lane (row l of the tile of 16, same samples)
@@ -221,7 +245,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32_kernel(SlabF32Args a) {
 #pragma unroll
             for (int v = 0; v < 2; v++)
                 *reinterpret_cast<f32x4_t *>(lds + ((size_t)(wave * R + (j * 2 + t) * 2 + v) * 64 + lane) * 4) = dphi[j][t][v];
-    float *us = lds + (size_t)4 * R * 64 * 4;  // [4 waves][32]
+    double *us = reinterpret_cast<double *>(lds + (size_t)4 * R * 64 * 4);  // [4 waves][32]
     if (!INJECT) {
 #pragma unroll
         for (int v = 0; v < 2; v++) {
@@ -276,7 +300,7 @@ int bwd_slab_f32_splits(int B, int C) {
 
 hipError_t launch_bwd_slab_f32(const float *dy, const float *x, const void *w, int w_dtype, const void *f_inject,
                                const float *phi, const float *Hpre, const float *Hpost, const float *M, const float *q,
-                               const BwdCoefOut &co, float *dx, float *df, float *dphi, float *dw_part, float *dt_part,
+                               const BwdCoefOut &co, float *dx, float *df, float *dphi, double *dw_part, double *dt_part,
                                int B, int n, int C, hipStream_t stream) {
     int S;
     const int tiles = slab_f32_tiles(B, C, &S);
@@ -291,7 +315,7 @@ hipError_t launch_bwd_slab_f32(const float *dy, const float *x, const void *w, i
     a.per_wave = tiles * kSfTile;
     a.per_split = 4 * a.per_wave;
     const dim3 grid(a.slabs + 1, S);
-    const size_t sum = sizeof(float) * ((size_t)4 * n * 4 * 64 * 4 + 128), tile = sizeof(float) * (4 * kSfWave + 24 * sf_phi_pitch(n));
+    const size_t sum = sizeof(float) * ((size_t)4 * n * 4 * 64 * 4 + 256), tile = sizeof(float) * (4 * kSfWave + 24 * sf_phi_pitch(n));
     const size_t smem = sum > tile ? sum : tile;
 #define MHC_SLAB_F32(N)                                                                                    \
     do {                                                                                                   \

@@ -127,7 +127,13 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     w.dP = c.floats((size_t)B * padded_D(n));
     w.cx = c.floats(B);
     w.s1 = c.floats(B);
-    w.u = c.floats((size_t)B * C);
+    // partial sums of dw and dt: float32 rows of at most B, float64 rows of the fp32 slab kernel or of the resident
+    // backward's second launch with a split batch
+    const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1, bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
+    const size_t slab64 = n <= 4 ? bs5 : 0, parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
+    w.u = c.floats(std::max((size_t)B, 2 * slab64) * C);
+    w.upart = c.floats(2 * parts64 * C);
+    w.dtpart = c.floats(std::max((size_t)B, 2 * std::max(slab64, parts64)) * (D + 3));
     w.raw = c.floats(bwd_reduce_raw_floats(B, n, C));
     w.s1part = c.floats(n > 8 ? (size_t)B * bwd_reduce_parts(B, n, C) : 0);
     // wide projections: the part of dx that is formed beside the coefficient backward, fp32
@@ -142,14 +148,8 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     if (bs3 > bs) bs = bs3;
     const int bs4 = dphi_f32_splits(B, n, C);
     if (bs4 > bs) bs = bs4;
-    const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1;
     if (bs5 > bs) bs = bs5;
-    const int bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
     if (bs6 > bs) bs = bs6;
-    // partial sums of a split batch: float32 rows of at most B, float64 rows of the resident backward's second launch
-    const size_t parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
-    w.upart = c.floats(2 * parts64 * C);
-    w.dtpart = c.floats(std::max((size_t)B, 2 * parts64) * (D + 3));
     w.dphi_part = c.floats(bs > 1 ? (size_t)bs * D * nC : 0);
     w.BP = (B + 31) / 32 * 32;
     // planes of bf16: one of dP and two of dP^T, one more each for ragged rows (BP is even)
@@ -698,9 +698,10 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         const int S = bwd_slab_f32_splits(B, C);
         MHC_LAUNCH(launch_bwd_slab_f32(static_cast<const float *>(dy), static_cast<const float *>(x), w, w_dtype, f_inject,
                                        static_cast<const float *>(phi), H_pre, H_post, M, q, out, static_cast<float *>(dx),
-                                       static_cast<float *>(df), S > 1 ? ws.dphi_part : dphi, ws.u, ws.dtpart, B, n, C, st));
+                                       static_cast<float *>(df), S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
+                                       reinterpret_cast<double *>(ws.dtpart), B, n, C, st));
         MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S, D, dbias, dalpha, ws.dphi_part, S,
-                                   (size_t)D * n * C, dphi, st));
+                                   (size_t)D * n * C, dphi, st, true));
         return MHC_OK;
     }
     const int spg = bwd_dx_samples_per_group(B, n);

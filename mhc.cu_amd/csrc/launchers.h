@@ -191,12 +191,13 @@ hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const voi
                            int B, int n, int C, hipStream_t stream);
 
 // The same for the fp32 tier (n <= 4, even C), behind launch_mix_bwd_reduce (dP [B, 32], cx, s1, dt of `co`):
-// dx, df and the batch-split partial sums of dphi [S][D][nC], dw [S][C] and dt [S][D+3], S = bwd_slab_f32_splits().
+// dx, df and the batch-split partial sums of dphi [S][D][nC] and, in float64, dw [S][C] and dt [S][D+3],
+// S = bwd_slab_f32_splits().
 bool bwd_slab_f32_supported(int x_dtype, int phi_dtype, int n, int C);
 int bwd_slab_f32_splits(int B, int C);
 hipError_t launch_bwd_slab_f32(const float *dy, const float *x, const void *w, int w_dtype, const void *f_inject,
                                const float *phi, const float *Hpre, const float *Hpost, const float *M, const float *q,
-                               const BwdCoefOut &co, float *dx, float *df, float *dphi, float *dw_part, float *dt_part,
+                               const BwdCoefOut &co, float *dx, float *df, float *dphi, double *dw_part, double *dt_part,
                                int B, int n, int C, hipStream_t stream);
 
 // Samples per workgroup of launch_mix_bwd_dx and the resulting row count of u / dtpart.

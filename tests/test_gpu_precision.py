@@ -113,3 +113,18 @@ def _close_to_float64(whole, terms):
 @pytest.mark.parametrize("B,n,C", [(1536, 8, 64), (2050, 6, 16), (1794, 2, 44), (1600, 7, 48), (1922, 4, 42)])
 def test_split_batch_sums_stay_in_float64(B, n, C):
     _close_to_float64(*_batch_and_single_sums(B, n, C, torch.bfloat16))
+
+
+@pytest.mark.parametrize("B,n,C", [(640, 4, 64), (770, 3, 36), (300, 1, 96), (1030, 2, 130), (2, 4, 8), (18, 4, 512)])
+def test_float32_slab_sums_stay_in_float64(B, n, C):
+    _close_to_float64(*_batch_and_single_sums(B, n, C, torch.float32))
+
+
+# n = 4: a sum of six terms and a product of depth 24, about 9e-8; with every step of the product rounded at the size of
+# dx 1.5e-7
+@pytest.mark.parametrize("B,n,C", [(65, 4, 128), (40, 4, 514), (100, 3, 66)])
+def test_float32_dx_adds_the_projection_term_once(B, n, C):
+    x, dy, p = _dynamic(B, n, C, bf16_weight=False)
+    _, ref = nm.mhc_dynamic_fwd_bwd(x, p, dy, T, EPS, dtype=torch.float64)
+    _, got = hip_dynamic(x, p, dy, T, EPS)
+    assert rel2(got["x"], ref["x"]) <= 1.15e-7, rel2(got["x"], ref["x"])
