@@ -58,16 +58,16 @@ __device__ __forceinline__ float quad_allreduce(float v) {
 template <bool F32, bool ANY> struct Act8;
 template <bool ANY> struct Act8<false, ANY> {
     uint32_t w[4];
-    __device__ __forceinline__ void load(const void *base, size_t elem, bool ok) {
-        const uint4 t = ldg16<ANY>(static_cast<const bf16_t *>(base) + elem);
+    __device__ __forceinline__ void load(const void *base, uint32_t elem, bool ok) {
+        const uint4 t = ldg16<ANY>(reinterpret_cast<const bf16_t *>(static_cast<const char *>(base) + elem * 2u));
         w[0] = ok ? t.x : 0u; w[1] = ok ? t.y : 0u; w[2] = ok ? t.z : 0u; w[3] = ok ? t.w : 0u;
     }
     __device__ __forceinline__ uint4 get() const { return make_uint4(w[0], w[1], w[2], w[3]); }
 };
 template <bool ANY> struct Act8<true, ANY> {
     uint32_t w[8];
-    __device__ __forceinline__ void load(const void *base, size_t elem, bool ok) {
-        const float *p = static_cast<const float *>(base) + elem;
+    __device__ __forceinline__ void load(const void *base, uint32_t elem, bool ok) {
+        const float *p = reinterpret_cast<const float *>(static_cast<const char *>(base) + elem * 4u);
         const uint4 t = ldg16<ANY>(p), u = ldg16<ANY>(p + 4);
         w[0] = ok ? t.x : 0u; w[1] = ok ? t.y : 0u; w[2] = ok ? t.z : 0u; w[3] = ok ? t.w : 0u;
         w[4] = ok ? u.x : 0u; w[5] = ok ? u.y : 0u; w[6] = ok ? u.z : 0u; w[7] = ok ? u.w : 0u;
@@ -183,15 +183,27 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     // and forcing four workgroups per CU made the compiler spill: 50.1 us)
     RawVec<bf16_t, 8> wb[ITEMS];
     RawVec<float, 8> wf[ITEMS];
+    auto load_w = [&](int it, int cc) {
+        if constexpr (WMODE == kGramWBf16 && RAG) wb[it].load_any(static_cast<const bf16_t *>(a.w) + cc);
+        else if constexpr (WMODE == kGramWBf16) wb[it].load(static_cast<const bf16_t *>(a.w) + cc);
+        else if constexpr (RAG) wf[it].load_any(static_cast<const float *>(a.w) + cc);
+        else wf[it].load(static_cast<const float *>(a.w) + cc);
+    };
+    // The largest tile in fp32 storage is 160 registers as loaded: the weights are fetched where they are used (all of it
+    // at once spilled 29 registers, this 6 with a bf16 weight and none with an fp32 one; backward n=8 C=4096 B=500
+    // 107.8 -> 89.5 us, n=5 B=1000 177.8 -> 132.7).
+    constexpr bool kRereadW = F32 && NB * ITEMS >= 10 && !inject;
     bool in[ITEMS], sv[NB];
     float hpre[NB], hpost[NB], Mc[NB][NB][4], qraw = 1.f;
     {
-        size_t rowoff[NB];
+        // the sample's base is uniform and the offset in it has 32 bits: one address register per chunk
+        uint32_t rowoff[NB];
 #pragma unroll
         for (int I = 0; I < NB; I++) {
             sv[I] = 4 * I + i < n;  // streams >= n: masked, they alias stream 0
-            rowoff[I] = (size_t)b * n * C + (size_t)(sv[I] ? 4 * I + i : 0) * C;
+            rowoff[I] = (uint32_t)(sv[I] ? 4 * I + i : 0) * (uint32_t)C;
         }
+        const TS *dyb = static_cast<const TS *>(a.dy) + (size_t)b * n * C, *xb = static_cast<const TS *>(a.x) + (size_t)b * n * C;
 #pragma unroll
         for (int it = 0; it < ITEMS; it++) {
             const int c = (tw + TW * it) * 128 + blk * 8;
@@ -199,14 +211,11 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
             const int cc = in[it] ? (RAG ? min(c, C - 8) : c) : 0;
 #pragma unroll
             for (int I = 0; I < NB; I++) {
-                graw[it][I].load(a.dy, rowoff[I] + cc, in[it] && sv[I]);
-                xraw[it][I].load(a.x, rowoff[I] + cc, in[it] && sv[I]);
+                graw[it][I].load(dyb, rowoff[I] + cc, in[it] && sv[I]);
+                xraw[it][I].load(xb, rowoff[I] + cc, in[it] && sv[I]);
             }
-            if constexpr (inject) fraw[it].load(a.f_inject, (size_t)b * C + cc, in[it] && i == 0);
-            else if constexpr (WMODE == kGramWBf16 && RAG) wb[it].load_any(static_cast<const bf16_t *>(a.w) + cc);
-            else if constexpr (WMODE == kGramWBf16) wb[it].load(static_cast<const bf16_t *>(a.w) + cc);
-            else if constexpr (RAG) wf[it].load_any(static_cast<const float *>(a.w) + cc);
-            else wf[it].load(static_cast<const float *>(a.w) + cc);
+            if constexpr (inject) fraw[it].load(static_cast<const TS *>(a.f_inject) + (size_t)b * C, cc, in[it] && i == 0);
+            else if constexpr (!kRereadW) load_w(it, cc);
         }
         if constexpr (!inject) qraw = a.q[b];
         // every load is requested: from here on the tile is four words of bf16 pairs per chunk
@@ -287,6 +296,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                 }
             } else {
                 float wv[8];
+                if constexpr (kRereadW) load_w(it, in[it] ? (tw + TW * it) * 128 + blk * 8 : 0);
                 if constexpr (WMODE == kGramWBf16) wb[it].get(wv);
                 else wf[it].get(wv);
 #pragma unroll
@@ -389,6 +399,10 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     for (int it = 0; it < ITEMS; it++) {
         const int c = (tw + TW * it) * 128 + blk * 8;
         if (!in[it]) continue;  // quads are inside or outside together: the DPP exchanges stay within a quad
+        if constexpr (kRereadW) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_w(it, c);
+        }
         uint32_t ow[NB][OWD], dfw[OWS];
         float u8[8];
         // four channels at a time: the fp32 copies of eight cost the 8 x 8 case thirty registers

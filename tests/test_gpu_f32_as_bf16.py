@@ -108,3 +108,10 @@ def test_shapes_without_an_fp32_storage_path_are_refused(B, n, C):
     assert lib.mhc_layer_dynamic_accepts_f32_as_bf16(B, n, C, T) == 0
     st, got, _ = _run(B, n, C, "f32_as_bf16", False)
     assert st[0] == MHC_ERR_BAD_DTYPE and got is None
+
+
+# rows that seven tile waves hold in three, four and five items; five items of eight streams fetch the weight twice
+@pytest.mark.parametrize("B,n,C", [(2, 8, 2568), (3, 8, 3000), (2, 6, 3592), (3, 8, 4096), (5, 4, 4088)])
+@pytest.mark.parametrize("inject", [False, True])
+def test_the_longest_rows(B, n, C, inject):
+    test_f32_storage_consumed_as_bf16(B, n, C, inject)
