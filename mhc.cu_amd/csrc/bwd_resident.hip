@@ -58,16 +58,16 @@ __device__ __forceinline__ float quad_allreduce(float v) {
 template <bool F32, bool ANY> struct Act8;
 template <bool ANY> struct Act8<false, ANY> {
     uint32_t w[4];
-    __device__ __forceinline__ void load(const void *base, uint32_t elem, bool ok) {
-        const uint4 t = ldg16<ANY>(reinterpret_cast<const bf16_t *>(static_cast<const char *>(base) + elem * 2u));
+    __device__ __forceinline__ void load(const void *base, size_t elem, bool ok) {
+        const uint4 t = ldg16<ANY>(static_cast<const bf16_t *>(base) + elem);
         w[0] = ok ? t.x : 0u; w[1] = ok ? t.y : 0u; w[2] = ok ? t.z : 0u; w[3] = ok ? t.w : 0u;
     }
     __device__ __forceinline__ uint4 get() const { return make_uint4(w[0], w[1], w[2], w[3]); }
 };
 template <bool ANY> struct Act8<true, ANY> {
     uint32_t w[8];
-    __device__ __forceinline__ void load(const void *base, uint32_t elem, bool ok) {
-        const float *p = reinterpret_cast<const float *>(static_cast<const char *>(base) + elem * 4u);
+    template <typename O> __device__ __forceinline__ void load(const void *base, O elem, bool ok) {
+        const float *p = reinterpret_cast<const float *>(static_cast<const char *>(base) + elem * (O)sizeof(float));
         const uint4 t = ldg16<ANY>(p), u = ldg16<ANY>(p + 4);
         w[0] = ok ? t.x : 0u; w[1] = ok ? t.y : 0u; w[2] = ok ? t.z : 0u; w[3] = ok ? t.w : 0u;
         w[4] = ok ? u.x : 0u; w[5] = ok ? u.y : 0u; w[6] = ok ? u.z : 0u; w[7] = ok ? u.w : 0u;
@@ -196,14 +196,17 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     bool in[ITEMS], sv[NB];
     float hpre[NB], hpost[NB], Mc[NB][NB][4], qraw = 1.f;
     {
-        // the sample's base is uniform and the offset in it has 32 bits: one address register per chunk
-        uint32_t rowoff[NB];
+        // (kRereadW: a uniform base per sample and offsets of 32 bits, half the address registers; where registers
+        // are not short that was slower, n=8 C=768 B=1000 fp32 storage 26.8 -> 32.6 us)
+        using Off = typename std::conditional<kRereadW, uint32_t, size_t>::type;
+        const size_t sample = (size_t)b * n * C;
+        const TS *dyb = static_cast<const TS *>(a.dy) + (kRereadW ? sample : 0), *xb = static_cast<const TS *>(a.x) + (kRereadW ? sample : 0);
+        Off rowoff[NB];
 #pragma unroll
         for (int I = 0; I < NB; I++) {
             sv[I] = 4 * I + i < n;  // streams >= n: masked, they alias stream 0
-            rowoff[I] = (uint32_t)(sv[I] ? 4 * I + i : 0) * (uint32_t)C;
+            rowoff[I] = (Off)(kRereadW ? 0 : sample) + (Off)(sv[I] ? 4 * I + i : 0) * C;
         }
-        const TS *dyb = static_cast<const TS *>(a.dy) + (size_t)b * n * C, *xb = static_cast<const TS *>(a.x) + (size_t)b * n * C;
 #pragma unroll
         for (int it = 0; it < ITEMS; it++) {
             const int c = (tw + TW * it) * 128 + blk * 8;
@@ -214,7 +217,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
                 graw[it][I].load(dyb, rowoff[I] + cc, in[it] && sv[I]);
                 xraw[it][I].load(xb, rowoff[I] + cc, in[it] && sv[I]);
             }
-            if constexpr (inject) fraw[it].load(static_cast<const TS *>(a.f_inject) + (size_t)b * C, cc, in[it] && i == 0);
+            if constexpr (inject) fraw[it].load(a.f_inject, (size_t)b * C + cc, in[it] && i == 0);
             else if constexpr (!kRereadW) load_w(it, cc);
         }
         if constexpr (!inject) qraw = a.q[b];

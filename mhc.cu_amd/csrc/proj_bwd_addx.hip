@@ -180,9 +180,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
     // Operands that come straight from global memory in fragment order: dP^T (rounded value and
     // remainder) of this wave's samples for every dphi tile, and dP of its sample tiles.  Steps and
     // tiles beyond the padded batch read zeros.
-    // (the planes that only ragged rows have are fetched where they are used: held from here they spill)
-    constexpr int TPL = RAG ? 3 : 2, BPL = RAG ? 2 : 1;  // planes of dP^T and of dP
-    constexpr int HELD = RAG && NTD == 3 ? 1 : 2;        // planes of dP^T requested here
+    // (the planes that only ragged rows have - the third of dP^T, the second of dP - are fetched where they are used: held
+    // from here they spill)
+    constexpr int HELD = RAG && NTD == 3 ? 1 : 2;  // planes of dP^T requested here
     const size_t plane = (size_t)a.DP * a.BP;
     auto load_at = [&](int sb, int p, int m, int ks) {
         const int nsteps = a.BP >> 4, step = (sb >> 4) + KS * wave + ks;
@@ -195,20 +195,30 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
         return load16_masked(reinterpret_cast<const uint4 *>(a.dPb + p * plane + (ok ? frag_base(tile, a.DP >> 4, ks) : 0) + lane * 8), ok);
     };
     struct Ops {
-        uint4 at[HELD][NTD][KS], av[TT][2 * NTD];
+        uint4 ah[NTD][KS], al[NTD][KS], av[TT][2 * NTD];
     };
     Ops ops[PFOP ? 2 : 1];
     auto load_ops = [&](int sb, Ops &o) {
+        const int step0 = (sb >> 4) + KS * wave, nsteps = a.BP >> 4;
 #pragma unroll
         for (int m = 0; m < NTD; m++)
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++)
+            for (int ks = 0; ks < KS; ks++) {
+                const bool ok = step0 + ks < nsteps;
+                const bf16_t *ap = a.dPT + (ok ? frag_base(m, nsteps, step0 + ks) : 0) + lane * 8;
+                o.ah[m][ks] = load16_masked(reinterpret_cast<const uint4 *>(ap), ok);
+                if constexpr (HELD == 2)
+                    o.al[m][ks] = load16_masked(reinterpret_cast<const uint4 *>(ap + (size_t)a.DP * a.BP), ok);
+            }
 #pragma unroll
-                for (int p = 0; p < HELD; p++) o.at[p][m][ks] = load_at(sb, p, m, ks);
+        for (int t = 0; t < TT; t++) {
+            const int tile = (sb >> 5) + TT * wave + t;
+            const bool ok = tile < (a.BP >> 5);
 #pragma unroll
-        for (int t = 0; t < TT; t++)
-#pragma unroll
-            for (int ks = 0; ks < 2 * NTD; ks++) o.av[t][ks] = load_av(sb, 0, t, ks);
+            for (int ks = 0; ks < 2 * NTD; ks++)
+                o.av[t][ks] = load16_masked(
+                    reinterpret_cast<const uint4 *>(a.dPb + (ok ? frag_base(tile, a.DP >> 4, ks) : 0) + lane * 8), ok);
+        }
     };
     using Slot0 = std::integral_constant<int, 0>;
     using Slot1 = std::integral_constant<int, 1>;
@@ -278,11 +288,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 #pragma unroll
             for (int m = 0; m < NTD; m++)
 #pragma unroll
-                for (int ks = 0; ks < KS; ks++)
+                for (int ks = 0; ks < KS; ks++) {
+                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op.ah[m][ks]), xf[ks], acc[m], 0, 0, 0);
+                    if constexpr (HELD == 2)
+                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op.al[m][ks]), xf[ks], acc[m], 0, 0, 0);
+                    if constexpr (RAG) {
 #pragma unroll
-                    for (int p = 0; p < TPL; p++)
-                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8_t, p < HELD ? op.at[p < HELD ? p : 0][m][ks] : load_at(sb, p, m, ks)), xf[ks], acc[m], 0, 0, 0);
+                        for (int p = HELD; p < 3; p++)
+                            acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, load_at(sb, p, m, ks)), xf[ks], acc[m], 0, 0, 0);
+                    }
+                }
         }
         // ---- dP phi of this wave's sample tiles -> its own rows of o_s (phi fragments from the slab) -----
 #pragma unroll
@@ -293,9 +308,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void proj_bwd_addx_kernel
 #pragma unroll
             for (int ks = 0; ks < 2 * NTD; ks++) {
                 const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, lds_frag_tr(phi_s, kAxLD, ks * 16, 0, lane));
-#pragma unroll
-                for (int p = 0; p < BPL; p++)
-                    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, p < 1 ? op.av[t][ks] : load_av(sb, p, t, ks)), pf, o, 0, 0, 0);
+                o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op.av[t][ks]), pf, o, 0, 0, 0);
+                if constexpr (RAG)
+                    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, load_av(sb, 1, t, ks)), pf, o, 0, 0, 0);
             }
             // accumulator layout: column = lane & 31, register i -> row 8*(i/4) + 4*(lane/32) + i%4
 #pragma unroll
