@@ -197,7 +197,7 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
     const bool mv = r0 < n && c0 < n, vv = g < 2 * n;
     float al0 = 0.f, al1 = 0.f, al2 = 0.f, bvec = 0.f, bres = 0.f;
     // 4 * SU K-splits are summed from one round of loads (proj_fwd_ksplit caps the split count to
-    // match; the two-chunk variant has no registers to spare for more)
+    // match bf16 rows; the two-chunk variant has no registers to spare for more)
     constexpr int SU = fwd_splits_in_one_round(NP, CPT) / 4;
     constexpr int SH = NP == 8 ? SU / 2 : SU;
     float t_ssq[SU], t_vec[SU], t_e[SU];
@@ -269,7 +269,7 @@ void layer_fwd_small_kernel(LayerFwdArgs a) {
             pvec += (ok && vv) ? t_vec[u] : 0.f;
             pe += (ok && mv) ? t_e[u] : 0.f;
         }
-        for (int ks = parts * SU + part; ks < a.KS; ks += parts) {  // never with proj_fwd_ksplit's cap
+        for (int ks = parts * SU + part; ks < a.KS; ks += parts) {  // 4-byte x, C = 1025 .. 2048, n <= 4 (proj_fwd_ksplit's cap)
             ssq += a.ssqpart[(size_t)ks * a.B + b];
             if (vv) pvec += Pb[ks * ps + g];
             if (mv) pe += Pb[ks * ps + 2 * n + r0 * n + c0];

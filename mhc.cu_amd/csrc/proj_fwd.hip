@@ -631,7 +631,9 @@ int proj_fwd_ksplit(int x_dtype, int phi_dtype, int B, int n, int C) {
     if (ks > cap_slab) ks = cap_slab;
     if (ks > cap_bytes) ks = cap_bytes;
     // the fused forward kernel (n <= 8) sums that many splits with loads that it issues ahead of the sample's
-    // tile; more splits would queue behind the tile
+    // tile; more splits would queue behind the tile.  (The cap is that of bf16 rows: with 4-byte x a thread has two
+    // chunks from C = 1025 on and sums 16 at once, the rest in a second round.  Capped at 16 instead: float32 storage of
+    // bf16 arithmetic n=4 C=1280 B=512 14.0 -> 13.2 us, but float32 B=200 12.2 -> 13.5, 320 13.4 -> 14.4.)
     if (const int cap = fwd_splits_summed_at_once(n, C); n <= 8 && ks > cap) ks = cap;
     if (ks > 64) ks = 64;
     if (ks < 1) ks = 1;
@@ -709,6 +711,10 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
 //   n=6 C=1280: B=1024 27.2 -> 26.7, 2048 41.2 -> 42.5
 //   n=8 C=1280: B=256 17.9 -> 18.3, 512 23.0 -> 23.5, 1024 34.0 -> 36.5  (and one launch less on the host)
 //   n=32 C=1280: B=64 89.0 -> 66.5, 128 91.5 -> 75.0, 256 112.5 -> 109.5, 384 137.9 -> 140.2;  n=16: B=128 39.2 -> 30.6
+// The wide case is decided on whole steps, forward + backward in graphs of ten: each row of 128 samples reads the fp32
+// phi again, and in a step dphi (as many bytes) has gone through the memory-side cache (256 MB) since the last one.
+//   n=32 C=1280 (178 MB of phi): B=32 170 -> 150, 64 176 -> 154, 128 188 -> 175, 192 261 -> 253, 256 272 -> 275, 320 350 -> 367
+//   n=24 C=1280 (77 MB): B=128 120 -> 106, 320 209 -> 195;  n=16 (24 MB): B=128 87 -> 80, 320 139 -> 128
 bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     if (g.phi_dtype != kF32 || !al16(g.phi[0]) || !al16(g.phi[1]) || !al16(g.phi[2])) return false;
@@ -718,7 +724,8 @@ bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
     // whole 64-element chunks keep the packing launch
     if (!use_wide(n, C) && n > 8) return false;
     if (const int hook = tuning_get(kTuneGather)) return hook == 2;
-    if (use_wide(n, C)) return B <= 320;
+    // (128 MB: phi and dphi together fit that cache)
+    if (use_wide(n, C)) return B <= ((size_t)padded_D(n) * n * C * 4 > (128u << 20) ? 192 : 320);
     const int nt = mfma_nt(n);
     return B <= (nt == 1 ? 4096 : (nt == 2 ? 1024 : 512));
 }
