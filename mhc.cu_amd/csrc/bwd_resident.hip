@@ -1,7 +1,8 @@
 // Backward, first launch for n <= 8 in the bf16 tier when a sample's rows fit in the registers of one
 // workgroup: dy and x cross HBM ONCE for everything that depends only on the sample itself.
 //
-// One workgroup per sample: wave 0 runs the coefficient backward, waves 1..4 each keep their share of
+// One workgroup per sample: wave 0 runs the coefficient backward, the tile waves behind it (two to ten, as the row needs:
+// launch_items) each keep their share of
 // the sample's [n, C] rows of dy and x in registers (a lane holds 8 consecutive channels of one stream,
 // four neighbouring lanes hold the four streams of a stream group - the words as they lie in memory,
 // which is the operand layout of v_mfma_f32_4x4x4_16b_bf16).
@@ -10,15 +11,15 @@
 //        dM = dy x^T     W1 = dy diag(w) x^T     XX = x x^T          reference stream_ops.cuh:852-927
 //   2. wave 0: dHpre / dHpost from the sums, sigmoid derivatives, exact Sinkhorn backward, dP in the
 //      layouts of the projection backward, cx (CoefBwdSmall)          reference ops.py:297-349
-//   3. waves 1..4, meanwhile, from the registers they already hold:
+//   3. the tile waves, meanwhile, from the registers they already hold:
 //        dxp[j,c] = sum_i M[i,j] dy[i,c] + Hpre[j] da[c]               reference stream_ops.cuh:761-850, :646-663
 //        da = df w / q - a s1 / (C q^3),  df = Hpost . dy, a = Hpre . x   reference rmsnorm.cuh:255-294
 //        u[c] = df a / q   (the sample's summand of dw),  df (kernel-level view)
 //      s1 = Hpost^T W1 Hpre follows from the Gram sums, so this step does not wait for the serial
 //      Sinkhorn chain of step 2: the stores of dxp run under it.
 // The terms of dx that need dP (dP phi, reference ops.py:336-338) or cx (-cx x, ops.py:340-349) are
-// added by the projection-backward launch that follows (proj_bwd.hip, which owns a column slab for all
-// samples and therefore also finishes dphi without batch-split partial sums).
+// added by the launch that follows (proj_bwd_addx.hip, whose workgroups own a column slab for all samples and
+// therefore also finish dphi without batch-split partial sums, unless slabs are few).
 // The mixing uses the VALU with DPP quad broadcasts: the contraction runs over streams, which lie
 // across the four lanes of a quad.
 #include "coef_bwd_small.h"

@@ -9,10 +9,10 @@ Differences that a caller can observe are limited to these:
   (fp32 accumulation) instead of being up-cast first;
 * no host synchronisation (the alphas are read on the device) and no Python loop over samples.
 
-The dynamic layer gathers its parameters (three phi matrices, biases, alphas) into the library's
-layout with one small launch per forward call, as the reference re-concatenates them on every call
-(ops.py:172-177).  `set_param_cache(True)` reuses the gathered copy while the parameters' storage
-addresses and in-place version counters are unchanged; writes through `.data` do not bump those
+The dynamic layer reads its parameters (three phi matrices, biases, alphas) on every call, in the projection
+itself or through one small launch that brings them into the library's layout, as the reference re-concatenates
+them on every call (ops.py:172-177).  `set_param_cache(True)` reuses that gathered copy while the parameters'
+storage addresses and in-place version counters are unchanged; writes through `.data` do not bump those
 counters, so the cache is off unless asked for.
 """
 from __future__ import annotations
