@@ -192,7 +192,7 @@ __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void 
     };
     // The largest tile in fp32 storage is 160 registers as loaded: the weights are fetched where they are used (all of it
     // at once spilled 29 registers, this 6 with a bf16 weight and none with an fp32 one; backward n=8 C=4096 B=500
-    // 107.8 -> 89.5 us, n=5 B=1000 177.8 -> 132.7).
+    // 106.4 -> 87.5 us, n=5 B=1000 179 -> 133).
     constexpr bool kRereadW = F32 && NB * ITEMS >= 10 && !inject;
     bool in[ITEMS], sv[NB];
     float hpre[NB], hpost[NB], Mc[NB][NB][4], qraw = 1.f;

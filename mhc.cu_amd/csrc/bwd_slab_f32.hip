@@ -6,8 +6,8 @@
 //   (reference stream_ops.cuh:646-663, :761-850, rmsnorm.cuh:255-294, ops.py:332-351)
 //
 // Bound by bytes: x and dy in, dx out (157 MB at B=2560 n=4 C=1280).  The three launches it replaces (dP phi
-// into dx, the dx kernel, dphi) moved 367 MB and took 84 us there; this one takes 39 us (4.1 TB/s)
-// and leaves the finalize launch fewer rows (10 -> 4 us).
+// into dx, the dx kernel, dphi) moved 367 MB and took 84 us there; this one takes 39 us (4.0 TB/s, 1.2 us of it for the
+// float64 sums and for adding dP phi in one piece) and leaves the finalize launch fewer rows (10 -> 4 us).
 //
 // A workgroup owns 32 channels of all streams and a range of samples that its four waves share out in tiles of
 // 16.  The products run on v_mfma_f32_16x16x4_f32 (IEEE fp32): the tile is 16 samples x 16 channels, a lane holds

@@ -69,20 +69,20 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 // supported.  Its second launch walks all samples of a column slab in one workgroup, which stops paying once the batch is
 // large enough to fill the chip with batch splits; the fewer streams, the fewer slabs.
 // Measured, backward in graphs of ten, tiled (slab / Gram) path -> resident path (us):
-//   n=4 C=256:  B=768 19.5 -> 15.8, 2048 28.6 -> 21.4, 6000 46.0 -> 38.7;  C=640: B=768 21.5 -> 18.9, 1024 23.8 -> 25.9
-//   n=4 C=1280: B=64 17.1 -> 9.2, 320 19.1 -> 14.9, 512 23.0 -> 19.2, 768 25.1 -> 24.1, 1024 28.6 -> 29.1, 1536 34.5 -> 38.9
-//   n=4 C=2048: B=512 27.0 -> 24.0, 768 30.6 -> 29.2, 1024 34.0 -> 38.8;  C=2560: B=256 23.9 -> 17.8, 512 30.9 -> 28.6,
-//               640 32.9 -> 35.0, 768 35.0 -> 37.7
-//   n=3 C=1920: B=768 26.8 -> 25.2, 1024 28.6 -> 33.3;  n=2 C=512: B=768 18.6 -> 16.4, 2048 26.6 -> 27.0;  n=2 C=1280:
-//               B=768 20.5 -> 21.8, 1024 23.8 -> 28.6
+//   n=4 C=256:  B=768 19.2 -> 16.3, 2048 28.5 -> 22.2, 6000 45.8 -> 38.8;  C=640: B=768 21.4 -> 19.3, 1024 23.8 -> 26.3
+//   n=4 C=1280: B=64 17.1 -> 9.2, 320 19.1 -> 14.6, 512 23.0 -> 19.3, 768 25.2 -> 24.7, 1024 28.5 -> 29.5, 1536 34.6 -> 39.1
+//   n=4 C=2048: B=512 26.9 -> 23.9, 768 30.6 -> 28.8, 1024 33.8 -> 38.4;  C=2560: B=256 23.9 -> 18.2, 512 30.7 -> 27.9,
+//               640 32.8 -> 34.7, 768 34.7 -> 37.6
+//   n=3 C=1920: B=768 26.6 -> 24.7, 1024 28.5 -> 32.6;  n=2 C=512: B=768 18.6 -> 16.8, 2048 26.5 -> 28.2;  n=2 C=1280:
+//               B=768 20.3 -> 21.9, 1024 23.7 -> 29.0
 // (the line is one number, B <= 768: at its ends, C <= 256 and C >= 2500, it is off by a few us)
 // Rows of more than 2560 channels hand dxp over in fp32 (bwd_resident_dxp_f32), and the line lies lower:
-//   n=4 C=2688: B=512 32.6 -> 27.6, 768 35.0 -> 37.2;  C=4096: B=256 31.4 -> 23.7, 512 38.7 -> 37.9, 768 41.7 -> 52.4
-//   n=3 C=3072: B=256 21.0 -> 20.2, 512 28.5 -> 28.6, 768 32.7 -> 36.0;  n=2 C=4096: B=256 20.5 -> 21.8, 768 33.8 -> 39.2
+//   n=4 C=2688: B=512 32.4 -> 28.0, 768 34.8 -> 38.0;  C=4096: B=256 31.2 -> 23.8, 512 38.6 -> 38.7, 768 41.7 -> 53.4
+//   n=3 C=3072: B=256 20.9 -> 20.2, 512 28.5 -> 28.8, 768 32.8 -> 37.0;  n=2 C=4096: B=256 20.3 -> 22.0, 768 33.8 -> 39.5
 // n = 5 .. 8 at every batch size:
-//   n=8 C=1280: B=128 25.1 -> 16.9, 256 30.5 -> 22.0, 512 46.1 -> 36.1, 1024 77.3 -> 62.7;  C=3072: B=1000 128.6 -> 107.2
-//   n=8 C=256: B=600 29.9 -> 24.6, 6000 113.3 -> 70.4;  C=512: B=2048 74.3 -> 54.7, 6000 181.2 -> 135.4;  n=5 C=384:
-//               B=3000 86.2 -> 55.0
+//   n=8 C=1280: B=128 25.1 -> 16.0, 256 30.5 -> 21.2, 512 46.1 -> 34.1, 1024 77.3 -> 59.3;  C=3072: B=1000 128.9 -> 105.7
+//   n=8 C=256: B=600 29.9 -> 23.3, 6000 113.4 -> 69.3;  C=512: B=2048 74.1 -> 55.0, 6000 181.0 -> 135.1;  n=5 C=384:
+//               B=3000 86.1 -> 57.9
 // Experiment hook: 1 = never, 2 = always.
 bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;

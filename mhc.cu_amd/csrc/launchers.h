@@ -235,8 +235,8 @@ constexpr int kResShortMaxC = 512, kResWholeMaxC = 2560, kResMaxC = 4096;
 // dx is then rounded once and its error against float64 is that of the tiled kernels, which would serve these
 // shapes otherwise (1.66e-3 relative); handed over in bf16 it is rounded twice (2.35e-3).
 // The price is 4 bytes per element (backward us, tiled | handed over in bf16 | in fp32): n=4 C=2880 B=256 27.6 | 19.2 |
-// 21.5; n=8 C=4096 B=100 45.5 | 32.7 | 33.3; n=8 C=3072 B=1000 128.6 | 102.7 | 107.2; n=8 C=256 B=6000 113.3 | 66.9 |
-// 70.4, B=600 29.9 | 22.7 | 24.6.  Rows of 513 .. 2560 channels (n <= 4: up to 2560) keep the bf16 hand-over.
+// 21.6; n=8 C=4096 B=100 45.5 | 32.1 | 32.9; n=8 C=3072 B=1000 128.9 | 102.9 | 105.7; n=8 C=256 B=6000 113.4 | 66.8 |
+// 69.2, B=600 29.9 | 22.6 | 23.3.  Rows of 513 .. 2560 channels (n <= 4: up to 2560) keep the bf16 hand-over.
 inline bool bwd_resident_dxp_f32(int n, int C) { return C % 8 != 0 || C > kResWholeMaxC || (n > 4 && C <= kResShortMaxC); }
 hipError_t launch_bwd_resident(const void *dy, const void *x, int x_dtype, const void *w, int w_dtype, const void *f_inject,
                                const float *Hpre, const float *Hpost, const float *M, const float *q,

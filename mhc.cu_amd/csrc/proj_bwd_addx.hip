@@ -68,8 +68,8 @@ constexpr int kAxLDR = 36;         // LDS pitch of the dphi tiles in the final c
 //   kAxRagged  the same for rows of any length (C % 8 != 0): the last chunk of a row is loaded from nC - 8 on and
 //              shifted down; dP in one more bf16 plane each (dphi: three, 24 bits; dP phi: two), so that the
 //              gradients are as good as from the fp32 arithmetic of the general kernels (dphi off by 2e-7, with
-//              two planes 3e-6; B=333 n=3 C=1230 backward 19.7 us with two planes and dxp in bf16, 22.6 with
-//              three and dxp in fp32, 46.6 in the general kernels; B=130 n=8 C=643 20.7, 30.1, 160.9)
+//              two planes 3e-6; B=333 n=3 C=1230 backward 19.7 us with two planes and dxp in bf16, 21.9 with
+//              three and dxp in fp32, 46.1 in the general kernels; B=130 n=8 C=643 21.1, 33.4, 160.7)
 // NW: waves per workgroup (a block is NW * SPW samples).
 // SPLIT: blockIdx.y is a batch split (a template argument: with a run-time first sample the compiler keeps fewer
 // loads in flight, B=1000 n=6 C=1024 17.2 -> 21.2 us without any split).
