@@ -11,7 +11,7 @@ for p in (ROOT, PKG_ROOT):
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
 def pytest_collection_modifyitems(config, items):
