@@ -405,9 +405,11 @@ Tensor mhc_layer_dynamic(const Tensor &x_in, const OptTensor &w_opt, const Tenso
         if (cached) pk = cached_params(params, x, n, C, cd);
         y = at::empty({B, n, C}, x.options().dtype(y_type));
         const DynLayout l(B, n, C, (int)iters, record, cd, !cached);
-        // without a backward nothing of it outlives the call: a small one lies behind the workspace then (one
-        // allocation less, 1.5 us; larger ones are not worth the memory that the workspace would hold on to)
-        const bool own = record || l.bytes > ((size_t)8 << 20);
+        // Without a backward nothing of it outlives the call: a small one lies behind the workspace then, one allocation
+        // less.  It pays where the host bounds the call (n=4 C=1280, phi 0.25 MB: B=7 10.72 us against 11.17 with a buffer
+        // of its own, B=200 10.76 against 11.15); from 0.8 MB of phi on the device does (n=4 C=4096 12.68 against 12.56,
+        // n=8 C=1280 14.94 against 14.91), and the workspace, which is held on to, need not grow for it.
+        const bool own = record || l.bytes > ((size_t)512 << 10);
         const size_t ws_bytes = align256(mhc_layer_dynamic_workspace_bytes(B, n, C));
         if (own) kept = byte_buffer(x, l.bytes);
         Tensor m[9];
