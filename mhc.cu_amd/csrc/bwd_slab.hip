@@ -1,6 +1,6 @@
 // Backward, second launch for n <= 4 in the bf16 tier: everything that needs dP, in ONE pass over
-// dy and x.  A workgroup owns a slab of 64 channels (all n streams) and walks the samples of its
-// batch split in tiles of 32:
+// dy and x.  A workgroup owns a slab of channels (all n streams) and walks the samples of its batch
+// split in tiles:
 //
 //   dx[b,j,c]  = sum_i M_b[i,j] dy[b,i,c] + Hpre_b[j] da[b,c] - cx_b x[b,j,c] + sum_d dP[b,d] phi[d, jC+c]
 //   df[b,c]    (kernel-level view)                                   reference stream_ops.cuh:761-850,
@@ -8,16 +8,16 @@
 //   dw[c]     += sum_b df[b,c] a[b,c] / q_b                          reference rmsnorm.cuh:282-294
 //   dbias / dalpha partial sums of dt over the split's samples       reference ops.py:319-325
 //
-// The two projection products run on the matrix cores (v_mfma_f32_32x32x16_bf16): their
-// contraction index (b for dphi, d for the dx term) is not the contiguous one in memory, so the
-// x tile and the phi slab are staged row-major in LDS and read back transposed; dP arrives from
-// the reduce kernel as bf16 [B, DP] and as a transposed hi/lo pair [2][DP][BP].  The projection
-// term of dx goes from the accumulators through LDS to the thread that owns (sample, 8 channels)
-// of all streams, which finishes dx on the VALU and stores 16 bytes per stream.
-// Per tile: two barriers, x and dy read once from HBM, dx written once; no atomics.
+// The two projection products run on the matrix cores: their contraction index (b for dphi, d for the
+// dx term) is not the contiguous one in memory, so the x tile and the phi slab are staged row-major in LDS
+// and read back transposed; dP arrives from the reduce kernel as bf16 [B, DP] and as a transposed hi/lo
+// pair [2][DP][BP].  x and dy are read once from HBM, dx is written once; no atomics.
+//
+// Two kernels: bwd_slab_stage_kernel for bf16 dy, bwd_slab_f32dy_kernel for fp32 dy beside bf16 x.
 #include "launchers.h"
 
-#include <type_traits>
+#include <algorithm>
+
 #include "mhc_common.h"
 #include "phase_profiler.h"
 #include "tuning.h"
@@ -34,7 +34,7 @@ constexpr int kSlabLDX = kSlabKW + 8;       // LDS pitch of the bf16 tiles (elem
 constexpr int kSlabLDF = kSlabKW + 4;       // LDS pitch of the fp32 projection-term tile
 
 struct BwdSlabArgs {
-    const void *dy;          // TG [B, n, C]
+    const void *dy;          // [B, n, C]
     const bf16_t *x;         // [B, n, C]
     const void *w;           // [C]
     const void *f_inject;    // bf16 [B, C] or nullptr
@@ -46,9 +46,9 @@ struct BwdSlabArgs {
     bf16_t *dx;              // [B, n, C]
     bf16_t *df;              // [B, C] or nullptr
     float *dphi_part;        // [S][D][nC]
-    float *dw_part;          // [S][C]
-    float *dt_part;          // [S][D+3]
-    int w_bf16, B, BP, n, C, tiles;  // tiles = 32-sample tiles of the batch; split y takes tiles [y T / S, (y + 1) T / S)
+    double *dw_part;         // [S][C]
+    double *dt_part;         // [S][D+3]
+    int w_bf16, B, BP, n, C, tiles;  // tiles of the batch (32 samples, bf16 dy: 16); split y takes tiles [y T / S, (y + 1) T / S)
 };
 
 __device__ __forceinline__ bf16x8_t slab_frag_t(const bf16_t *tile, int k0, int col0, int lane) {
@@ -63,14 +63,8 @@ __device__ __forceinline__ void unpack8(const uint4 &r, float (&v)[8]) {
     v[6] = bf16lo_to_f32(r.w); v[7] = bf16hi_to_f32(r.w);
 }
 
-// Eight consecutive values of dy kept as loaded (16 bytes for bf16, 32 for fp32) until they are used.
-template <typename T> struct Raw8;
-template <> struct Raw8<bf16_t> {
-    uint4 r;
-    __device__ __forceinline__ void load(const bf16_t *p) { r = *reinterpret_cast<const uint4 *>(p); }
-    __device__ __forceinline__ void get(float (&v)[8]) const { unpack8(r, v); }
-};
-template <> struct Raw8<float> {
+// Eight consecutive values of dy kept as loaded until they are used.
+struct Raw8 {
     float4 r0, r1;
     __device__ __forceinline__ void load(const float *p) {
         r0 = reinterpret_cast<const float4 *>(p)[0];
@@ -81,10 +75,10 @@ template <> struct Raw8<float> {
     }
 };
 
-template <typename TG>
-__global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
-    // bf16 dy: the per-sample 4x4 mixing of phase C runs on v_mfma_f32_4x4x4_16b_bf16 (below)
-    constexpr bool kMixMfma = std::is_same<TG, bf16_t>::value;
+// fp32 dy.  Tiles of 32 samples; the projection term of dx goes from the accumulators through LDS to the thread that
+// owns (sample, 8 channels) of all streams, which finishes dx on the VALU and stores 16 bytes per stream.  Two barriers
+// per tile.
+__global__ __launch_bounds__(256, 2) void bwd_slab_f32dy_kernel(BwdSlabArgs a) {
     extern __shared__ float smem_f[];
     float *dxf_s = smem_f;                                                  // [32][LDF] fp32
     bf16_t *x_s = reinterpret_cast<bf16_t *>(dxf_s + 32 * kSlabLDF);         // [32][LDX] bf16
@@ -98,9 +92,8 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
     // whole tiles per split, the counts of two splits differing by at most one: any split count up to the
     // tile count can be used, so the grid can be sized to the chip instead of to a divisor of the batch
     const unsigned nsplit = gridDim.y;
-    // (tiles <= 2^26 and at most 512 splits: the products fit 32 bits)
-    const int b_begin = (int)(blockIdx.y * (unsigned)a.tiles / nsplit) * 32;
-    const int b_end = min(a.B, (int)((blockIdx.y + 1) * (unsigned)a.tiles / nsplit) * 32);
+    const int b_begin = (int)((uint64_t)blockIdx.y * (unsigned)a.tiles / nsplit) * 32;
+    const int b_end = min(a.B, (int)((uint64_t)(blockIdx.y + 1) * (unsigned)a.tiles / nsplit) * 32);
     const bool inject = a.f_inject != nullptr;
     const int row = lane & 31, kg = lane >> 5;
     // VALU ownership: sample bl of the tile, channels c0 + ch*8 .. +8 of every stream
@@ -113,7 +106,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
     // that come straight from global memory (dP^T hi/lo rows d, dP rows b)
     struct TileRegs {
         uint4 xr[kSlabNS];
-        Raw8<TG> gr[kSlabNS];
+        Raw8 gr[kSlabNS];
     };
     // Loads carry no predicate (a predicate would be applied right behind the load and make the
     // prefetch wait): slots beyond the batch, streams >= n and channel chunks >= C alias valid
@@ -125,7 +118,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
         const bool bok = b < b_end && cok;
         const size_t base = bok ? (size_t)b * nC + cth : 0;
         const bf16_t *xb = a.x + base;
-        const TG *gb = static_cast<const TG *>(a.dy) + base;
+        const float *gb = static_cast<const float *>(a.dy) + base;
 #pragma unroll
         for (int j = 0; j < kSlabNS; j++) {
             const size_t so = j < n ? (size_t)j * C : 0;
@@ -174,7 +167,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
     float usum[8];
 #pragma unroll
     for (int v = 0; v < 8; v++) usum[v] = 0.f;
-    float dtsum = 0.f;  // slab 0 only: thread (col = tid & 31, row group = tid >> 5)
+    double dtsum = 0.0;  // slab 0 only: thread (col = tid & 31, row group = tid >> 5)
 
     float wv[8];
 #pragma unroll
@@ -206,23 +199,15 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
         // this thread's sample coefficients for phase C: asked for here so that they arrive behind
         // the barriers and the matrix-core phase (slots beyond the split alias sample 0, streams
         // >= n alias stream 0; both are discarded below)
-        // (matrix-core mixing: a lane only needs column lane & 3 of M)
-        constexpr int MC = kMixMfma ? 1 : kSlabNS;
-        const int jq = tid & 3;
-        float hpre[kSlabNS], hpost[kSlabNS], Mr[kSlabNS][MC], cxv, qv = 1.f, s1v = 0.f;
+        float hpre[kSlabNS], hpost[kSlabNS], Mr[kSlabNS][kSlabNS], cxv, qv = 1.f, s1v = 0.f;
         {
-            // by sample only, whatever the lane's channel chunk: in the matrix-core mixing the four
-            // lanes of a block supply each other's coefficient rows
             const size_t bc = b < b_end ? b : 0;
 #pragma unroll
             for (int i = 0; i < kSlabNS; i++) {
                 hpre[i] = a.Hpre[bc * n + (i < n ? i : 0)];
                 hpost[i] = a.Hpost[bc * n + (i < n ? i : 0)];
 #pragma unroll
-                for (int j = 0; j < MC; j++) {
-                    const int jj = kMixMfma ? jq : j;
-                    Mr[i][j] = a.M[bc * n * n + ((i < n && jj < n) ? i * n + jj : 0)];
-                }
+                for (int j = 0; j < kSlabNS; j++) Mr[i][j] = a.M[bc * n * n + ((i < n && j < n) ? i * n + j : 0)];
             }
             cxv = a.cx[bc];
             if (!inject) { qv = a.q[bc]; s1v = a.s1[bc]; }
@@ -274,100 +259,6 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
         MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 2, pclk);
 
         // ---- phase C: finish dx ------------------------------------------------------------------
-        if constexpr (kMixMfma) {
-            // One v_mfma_f32_4x4x4_16b_bf16 is 16 independent 4x4x4 products; a block is four
-            // consecutive lanes, here four channel chunks of ONE sample.  With B = the four streams of
-            // a lane's channel (column = lane) and A = a coefficient matrix of the sample (row r from
-            // lane r of the block), lane l receives column l: the four output streams of its own channel.
-            //   D1 = G (M^T dy) + X (-(Hpre Hpre^T k2 + cx I) x)        rows: dx streams (without the
-            //   D2 = [Hpost; 0; 0; 0] dy + [0; Hpre; 0; 0] x             projection and da terms)
-            //                                                            rows 0, 1: df and the aggregate a
-            // Coefficients enter as bf16 value + remainder (two instructions each).  Every lane runs
-            // the instructions (lanes beyond the split or the channel range compute on aliased data
-            // that is never stored).
-            float qinv = 0.f, k2 = 0.f;
-            if (!inject) {
-                qinv = 1.0f / qv;
-                k2 = s1v * qinv * qinv * qinv / (float)C;
-            }
-#pragma unroll
-            for (int i = 0; i < kSlabNS; i++)
-                if (i >= n) { hpre[i] = 0.f; hpost[i] = 0.f; }
-            float mcol[kSlabNS], xrow[kSlabNS];
-            const float hq = jq == 0 ? hpre[0] : (jq == 1 ? hpre[1] : (jq == 2 ? hpre[2] : hpre[3]));  // Hpre[lane & 3]
-#pragma unroll
-            for (int i = 0; i < kSlabNS; i++) {
-                mcol[i] = (i < n && jq < n) ? Mr[i][0] : 0.f;
-                xrow[i] = -(hq * hpre[i] * k2 + (i == jq ? cxv : 0.f));
-            }
-            CoefRow cg, cxr, cdf, caa;
-            cg.set(mcol[0], mcol[1], mcol[2], mcol[3]);
-            cxr.set(xrow[0], xrow[1], xrow[2], xrow[3]);
-            const bool r0 = jq == 0, r1 = jq == 1;
-            cdf.set(r0 ? hpost[0] : 0.f, r0 ? hpost[1] : 0.f, r0 ? hpost[2] : 0.f, r0 ? hpost[3] : 0.f);
-            caa.set(r1 ? hpre[0] : 0.f, r1 ? hpre[1] : 0.f, r1 ? hpre[2] : 0.f, r1 ? hpre[3] : 0.f);
-            const uint32_t gw[kSlabNS][4] = {{cur.gr[0].r.x, cur.gr[0].r.y, cur.gr[0].r.z, cur.gr[0].r.w},
-                                             {cur.gr[1].r.x, cur.gr[1].r.y, cur.gr[1].r.z, cur.gr[1].r.w},
-                                             {cur.gr[2].r.x, cur.gr[2].r.y, cur.gr[2].r.z, cur.gr[2].r.w},
-                                             {cur.gr[3].r.x, cur.gr[3].r.y, cur.gr[3].r.z, cur.gr[3].r.w}};
-            const uint32_t xw[kSlabNS][4] = {{cur.xr[0].x, cur.xr[0].y, cur.xr[0].z, cur.xr[0].w},
-                                             {cur.xr[1].x, cur.xr[1].y, cur.xr[1].z, cur.xr[1].w},
-                                             {cur.xr[2].x, cur.xr[2].y, cur.xr[2].z, cur.xr[2].w},
-                                             {cur.xr[3].x, cur.xr[3].y, cur.xr[3].z, cur.xr[3].w}};
-            float dfv[8];
-            uint32_t dxw[kSlabNS][2];  // packed dx of the first half, stored with the second (16 bytes per stream)
-#pragma unroll
-            for (int h = 0; h < 2; h++) {  // two halves of four channels keep the accumulators small
-                f32x4_t d1[4], d2[4];
-                bf16x4_t bg[4], bx[4];
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int p = 2 * h + (v >> 1);  // word of the channel pair
-                    if (v & 1) {
-                        bg[v] = streams_of_channel<true>(gw[0][p], gw[1][p], gw[2][p], gw[3][p]);
-                        bx[v] = streams_of_channel<true>(xw[0][p], xw[1][p], xw[2][p], xw[3][p]);
-                    } else {
-                        bg[v] = streams_of_channel<false>(gw[0][p], gw[1][p], gw[2][p], gw[3][p]);
-                        bx[v] = streams_of_channel<false>(xw[0][p], xw[1][p], xw[2][p], xw[3][p]);
-                    }
-                }
-                const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int v = 0; v < 4; v++) { d1[v] = mfma4(cg.hi, bg[v], zero); d2[v] = mfma4(cdf.hi, bg[v], zero); }
-#pragma unroll
-                for (int v = 0; v < 4; v++) { d1[v] = mfma4(cg.lo, bg[v], d1[v]); d2[v] = mfma4(cdf.lo, bg[v], d2[v]); }
-#pragma unroll
-                for (int v = 0; v < 4; v++) { d1[v] = mfma4(cxr.hi, bx[v], d1[v]); d2[v] = mfma4(caa.hi, bx[v], d2[v]); }
-#pragma unroll
-                for (int v = 0; v < 4; v++) { d1[v] = mfma4(cxr.lo, bx[v], d1[v]); d2[v] = mfma4(caa.lo, bx[v], d2[v]); }
-                float dw4[4];  // df * w / q per channel: the da term of dx is Hpre[j] times this
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const float s_df = d2[v][0], s_a = d2[v][1];
-                    dfv[4 * h + v] = s_df;
-                    dw4[v] = s_df * wv[4 * h + v] * qinv;
-                    usum[4 * h + v] += bok ? s_df * s_a * qinv : 0.f;
-                }
-                if (bok) {
-#pragma unroll
-                    for (int j = 0; j < kSlabNS; j++) {
-                        if (j < n) {
-                            const float4 p0 = *reinterpret_cast<const float4 *>(dxf_s + (size_t)bl * kSlabLDF + j * kSlabCW + ch * 8 + 4 * h);
-                            const float out[4] = {p0.x + d1[0][j] + hpre[j] * dw4[0], p0.y + d1[1][j] + hpre[j] * dw4[1],
-                                                  p0.z + d1[2][j] + hpre[j] * dw4[2], p0.w + d1[3][j] + hpre[j] * dw4[3]};
-                            if (h == 0) {
-                                dxw[j][0] = pack_bf16x2(out[0], out[1]);
-                                dxw[j][1] = pack_bf16x2(out[2], out[3]);
-                            } else {
-                                st16<true>(a.dx + (size_t)b * nC + (size_t)j * C + cth, dxw[j][0], dxw[j][1],
-                                           pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]));
-                            }
-                        }
-                    }
-                }
-            }
-            if (bok && inject && a.df) store_vec<bf16_t, 8>(a.df + (size_t)b * C + cth, dfv);
-        } else
         if (bok) {
             float qinv = 0.f, k2 = 0.f;
 #pragma unroll
@@ -463,7 +354,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
         for (int v = 0; v < 8; v++) red[bl * 65 + ch * 8 + v] = usum[v];
         __syncthreads();
         if (tid < 64) {
-            float s = 0.f;
+            double s = 0.0;
 #pragma unroll
             for (int r = 0; r < 32; r++) s += red[r * 65 + tid];
             if (c0 + tid < C) a.dw_part[(size_t)blockIdx.y * C + c0 + tid] = s;
@@ -471,11 +362,11 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
         __syncthreads();
     }
     if (blockIdx.x == 0) {
-        float *red = dxf_s;  // [8][32]
+        double *red = reinterpret_cast<double *>(dxf_s);  // [8][32]
         red[tid] = dtsum;
         __syncthreads();
         if (tid < D + 3 && tid < 32) {
-            float s = 0.f;
+            double s = 0.0;
 #pragma unroll
             for (int r = 0; r < 8; r++) s += red[r * 32 + tid];
             a.dt_part[(size_t)blockIdx.y * (D + 3) + tid] = s;
@@ -484,53 +375,501 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_kernel(BwdSlabArgs a) {
     MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 5, pclk);
 }
 
+
+// ---------------------------------------------------------------------------------------------
+// The same pass for bf16 dy.
+//
+// What bounds it is bytes - x and dy once in, dx once out - and how they are asked for.  Plain copies of two arrays into a
+// third in this access pattern reach 5.7 TB/s with 256-byte pieces of a row and some 130 KB per CU on their way, 4.8 with
+// 128-byte pieces, and the kernel above, used for both types before, reached 3.9: two tiles in 248 registers, phases
+// that run one after the other between barriers while the memory waits.  Here
+//   - every operand goes from global memory straight into LDS (global_load_lds, no registers in between), 16 samples
+//     at a time, x three and dy two tiles ahead (95 KB);
+//   - dP phi is formed transposed (phi^T as the A operand, dP as B, 16x16x32): a lane of the accumulators
+//     then holds four consecutive channels of ONE sample for every stream, which is what the mixing needs,
+//     so the projection term never leaves the registers;
+//   - dx replaces dy in LDS and leaves one tile later, row by row in 256-byte pieces: written as the lanes hold it, in
+//     pieces of 64 bytes, the stores alone cost 20 us at B=8192 C=2560;
+//   - the waves are of two kinds.  Loaders (a wave per 32 channels) request the tiles and do nothing else: one that
+//     also accumulated dphi held the barrier up (109 us).  Mixers (a wave per 16 channels) accumulate dphi, form dx and
+//     store it.
+// A period is one tile: one barrier, and nothing else between the waves.  CW channels per workgroup, one workgroup per CU.
+// Measured, n=4 B=8192 C=2560: 130 -> 98 us (503 MB, 5.1 TB/s); backward in graphs of ten: B=8192 C=2560 209 -> 174 us,
+// B=1280 C=2560 42.4 -> 37.4, B=2048 C=1280 41.0 -> 37.0, n=3 B=5000 C=1920 85.5 -> 71.0, n=2 B=3000 C=1024 37.8 -> 31.7.
+// Tried and slower at B=8192 C=2560 (backward): tiles of 32 samples in two stages with eight waves of one kind 193 us; dy
+// in the mixers' registers, dx stored from them, 214 us.
+//
+// LDS: a ring of x [N][16][CW] with the tile's dP^T hi, lo and dP in operand order (1 KiB each) and its samples'
+// coefficients, dense arrays copied as they are; a ring of dy, then dx, [N][16][CW].  The 16-byte chunks of a
+// row are permuted (slab_swizzle) so that neither the transposed reads (dphi) nor the row reads (dx) meet in a bank.
+// ---------------------------------------------------------------------------------------------
+
+// global -> LDS without registers in between: lane i's BYTES from base + off to lds + i * BYTES.  As assembly because the
+// compiler would wait for ALL of them before the next LDS access of any kind; the loaders wait by count (wait_vmem).
+// M0 is used by nothing else here (LDS instructions of this architecture do not read it).
+template <int BYTES> __device__ __forceinline__ void load_to_lds(const void *base, uint32_t off, uint32_t lds) {
+    static_assert(BYTES == 4 || BYTES == 16, "one or four words per lane");
+    const uint64_t p = (uint64_t)(uintptr_t)base;
+    if constexpr (BYTES == 16) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(p), "s"(lds) : "memory");
+    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(p), "s"(lds) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
+}
+template <int K> __device__ __forceinline__ void wait_vmem() {  // at most K younger vector memory operations in flight
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(K) : "memory");
+}
+// Barrier of the whole workgroup that waits for this wave's LDS accesses but not for its global ones (__syncthreads
+// is free to wait for both).
+__device__ __forceinline__ void stage_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// K floats from LDS, 16 bytes at a time where they are whole 16-byte pieces (and then aligned to them).
+template <int K> __device__ __forceinline__ void lds_floats(const float *p, float *v) {
+    if constexpr (K % 4 == 0) {
+#pragma unroll
+        for (int i = 0; i < K / 4; i++) {
+            const float4 t = reinterpret_cast<const float4 *>(p)[i];
+            v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < K; i++) v[i] = p[i];
+    }
+}
+
+// Where chunk 0 of sample row b lands within its row (chunk c: at c ^ this).  Four consecutive rows differ
+// in the chunk bits above a 32-channel group (transposed reads: 4 rows x 64 bytes at a time), sixteen rows in
+// all chunk bits (row reads: the same chunk of 16 rows).
+template <int CW> __device__ __forceinline__ int slab_swizzle(int b) {
+    if constexpr (CW == 128) return ((b & 3) << 2) | ((b >> 2) & 3);
+    else return ((b >> 3) & 1) | ((b >> 1) & 2) | ((b << 1) & 4);  // bits 1, 2, 3 of b, reversed (two rows per 256 bytes)
+}
+
+template <int N, int CW> struct SlabStage {
+    static constexpr int TB = 16, kLoaders = CW / 32, kMixers = CW / 16, kThreads = 64 * (kLoaders + kMixers);  // 6 CW
+    static constexpr int kXAhead = 3, kGAhead = 2;        // tiles requested ahead
+    static constexpr int kXRing = kXAhead + 1, kGRing = kGAhead + 2;
+    static constexpr int kTile = N * TB * CW * 2;         // bytes of x or dy
+    static constexpr int kP = kTile, kCoef = kP + 3 * 1024;
+    // coefficient blocks of 64 floats: M | Hpre | Hpost | cx | q | s1 | dt (slab 0 only)
+    static constexpr int kSegM = (TB * N * N + 63) / 64, kSegs = kSegM + 5, kSegDt = (TB * (N * N + 2 * N + 3) + 63) / 64;
+    static constexpr int kXBytes = kCoef + (kSegs + kSegDt) * 256;
+    // a loader's share of the dP and coefficient blocks (the last ones twice where they do not come out even, so that
+    // every loader has the same number of instructions in flight)
+    static constexpr int kShare = (3 + kSegs + kLoaders - 1) / kLoaders, kShareDt = (3 + kSegs + kSegDt + kLoaders - 1) / kLoaders;
+    static constexpr int kG = kXRing * kXBytes;           // the dy / dx ring
+    static constexpr int kW = kG + kGRing * kTile;        // the slab's w in fp32
+    static constexpr int kLds = kW + CW * 4;
+    static constexpr int kPhi = 32 * N * CW * 2;          // prologue: the phi slab, in the part of the dy ring not yet requested
+    static_assert(kPhi <= (kGRing - kGAhead) * kTile && kLds <= 160 * 1024, "the rings fit the LDS of a CU");
+};
+
+template <int N, int CW, bool INJECT>
+__global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a) {
+    using ST = SlabStage<N, CW>;
+    constexpr int kChunks = CW / 8, kRows = 512 / CW;  // 16-byte chunks per row, rows per KiB
+    constexpr int D = N * N + 2 * N, TB = ST::TB;
+    extern __shared__ float smem_f[];
+    char *const smem = reinterpret_cast<char *>(smem_f);
+    const uint32_t smem_at = lds_address(smem);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int C = a.C, nC = N * C;
+    const int slab = blockIdx.x, c0 = slab * CW;
+    const unsigned nsplit = gridDim.y;
+    const int b_begin = (int)((uint64_t)blockIdx.y * (unsigned)a.tiles / nsplit) * TB;
+    const int b_end = min(a.B, (int)((uint64_t)(blockIdx.y + 1) * (unsigned)a.tiles / nsplit) * TB);
+    const int T = (b_end - b_begin + TB - 1) / TB;
+    const int pwg = blockIdx.y * gridDim.x + blockIdx.x;
+    (void)pwg;
+    MHC_PHASE_ZERO(kPhaseBwdSlab, pwg);
+    MHC_PHASE_BEGIN(pclk);
+    const bool loader = wave >= ST::kMixers;
+    const int lw = wave - ST::kMixers;  // loader index
+
+    // One KiB of a tile of x, dy or dx is kRows sample rows of one stream: where lane's 16 bytes belong, for the rows from row0
+    const auto lane_row = [&](int row0) { return row0 + lane / kChunks; };
+    const auto lane_col = [&](int row) { return c0 + ((lane % kChunks) ^ slab_swizzle<CW>(row)) * 8; };
+
+    // ---- loads of a tile (loaders); loader l brings rows l kRows .. of every stream --------------------
+    // slots beyond the batch alias its last sample, columns beyond C the last ones: they only meet zero columns of
+    // dP^T or land in rows and columns that are not stored
+    const int ld_row = lane_row(lw * kRows), ld_col = min(lane_col(ld_row), C - 8);
+    auto load_tile = [&](const bf16_t *src, int t, uint32_t dst) {
+        const int sb = b_begin + t * TB;
+        const bf16_t *base = src + (size_t)sb * nC;
+        const uint32_t off = (uint32_t)(min(ld_row, b_end - sb - 1) * nC + ld_col) * 2;
+#pragma unroll
+        for (int j = 0; j < N; j++) load_to_lds<16>(base + (size_t)j * C, off, dst + (j * TB + lw * kRows) * CW * 2);
+    };
+    auto load_dy = [&](int t) { load_tile(static_cast<const bf16_t *>(a.dy), t, smem_at + ST::kG + t % ST::kGRing * ST::kTile); };
+    // The dP operands and the blocks of 64 coefficients of a tile are dealt out to the loaders: what this one brings is
+    // settled once, so that a tile costs it no more than the instructions.
+    struct Block {
+        const char *src;          // for the first sample of the batch
+        uint32_t step, at, dst;   // bytes per sample; this lane's bytes behind the tile's first; place behind the tile's x
+        int words;                // coefficients: floats per sample; 0: a KiB of dP operands
+    };
+    const int blocks = 3 + ST::kSegs + (slab == 0 ? ST::kSegDt : 0);
+    auto block_of = [&](int k) {
+        k = min(k, blocks - 1);
+        if (k < 2) return Block{reinterpret_cast<const char *>(a.dPT + (size_t)k * 32 * a.BP), 64u, lane * 16u, ST::kP + k * 1024u, 0};
+        // dP: [d / 8][16 samples][8] out of the fragments of 32 samples
+        if (k == 2) return Block{reinterpret_cast<const char *>(a.dPb), 64u, (lane >> 5) * 1024u + ((lane >> 4) & 1) * 512u + (lane & 15) * 16u, ST::kP + 2048u, 0};
+        const int s = k - 3;
+        const float *src;
+        int words = 1, i = lane;
+        if (s < ST::kSegM) { src = a.M; words = N * N; i += s * 64; }
+        else if (s == ST::kSegM) { src = a.Hpre; words = N; }
+        else if (s == ST::kSegM + 1) { src = a.Hpost; words = N; }
+        else if (s == ST::kSegM + 2 || (INJECT && s < ST::kSegs)) src = a.cx;
+        else if (s == ST::kSegM + 3) src = a.q;
+        else if (s == ST::kSegM + 4) src = a.s1;
+        else { src = a.dt; words = D + 3; i += (s - ST::kSegs) * 64; }
+        return Block{reinterpret_cast<const char *>(src), words * 4u, i * 4u, ST::kCoef + s * 256u, words};
+    };
+    Block mine[ST::kShareDt];
+#pragma unroll
+    for (int i = 0; i < ST::kShareDt; i++) mine[i] = block_of(lw + i * ST::kLoaders);
+    auto load_x = [&](int t) {
+        const uint32_t st = smem_at + t % ST::kXRing * ST::kXBytes;
+        const int sb = b_begin + t * TB, left = min(b_end - sb, TB);
+        load_tile(a.x, t, st);
+#pragma unroll
+        for (int i = 0; i < ST::kShareDt; i++) {
+            const Block &m = mine[i];
+            if (i >= ST::kShare && slab != 0) break;
+            if (m.words == 0) {  // (the second half of a 32-sample fragment of dP lies 256 bytes behind the first)
+                const bool half = m.dst == ST::kP + 2048u && (sb & 16);
+                load_to_lds<16>(m.src + (size_t)(half ? sb - 16 : sb) * m.step + (half ? 256 : 0), m.at, st + m.dst);
+            } else {
+                load_to_lds<4>(m.src + (size_t)sb * m.step, min(m.at, left * m.step - 4), st + m.dst);
+            }
+        }
+    };
+
+    // ---- prologue: phi slab -> LDS, row-major [32 d][N][CW] -> the mixers' transposed fragments -----
+    constexpr int kPhiChunks = N * 32 * kChunks, kPhiIters = (kPhiChunks + ST::kThreads - 1) / ST::kThreads;
+    uint4 phir[kPhiIters];
+#pragma unroll
+    for (int i = 0; i < kPhiIters; i++) {
+        const int e = tid + i * ST::kThreads;
+        const int d = e / (N * kChunks), j = e / kChunks % N, c = c0 + e % kChunks * 8;
+        const bool ok = d < D && c < C;
+        phir[i] = load16_masked(reinterpret_cast<const uint4 *>(a.phi + (ok ? (size_t)d * nC + (size_t)j * C + c : 0)), ok);
+    }
+    if (loader) {
+        // in the order in which the loop below counts them: what period p - 1 would have requested before what period p would
+        load_x(0);
+        if (T > 1) load_x(1);
+        load_dy(0);
+        if (T > 2) load_x(2);
+        if (T > 1) load_dy(1);
+    }
+    char *const phi_s = smem + ST::kG + ST::kGAhead * ST::kTile;
+#pragma unroll
+    for (int i = 0; i < kPhiIters; i++)
+        if (tid + i * ST::kThreads < kPhiChunks) *reinterpret_cast<uint4 *>(phi_s + (tid + i * ST::kThreads) * 16) = phir[i];
+    if (tid < CW)
+        reinterpret_cast<float *>(smem + ST::kW)[tid] =
+            (c0 + tid < C && !INJECT) ? (a.w_bf16 ? bf16_to_f32(static_cast<const bf16_t *>(a.w)[c0 + tid])
+                                                  : static_cast<const float *>(a.w)[c0 + tid]) : 0.f;
+    __syncthreads();
+
+    float usum[4] = {0.f, 0.f, 0.f, 0.f};  // mixers
+    double dtsum = 0.0;                    // loaders of slab 0: column tid & 31, row group
+    // mixer lane (l16, kq): the four channels from c0 + cl of sample l16
+    const int l16 = lane & 15, kq = lane >> 4, cl = 16 * wave + 4 * kq;
+
+    if (loader) {
+        // ---- requests the tiles --------------------------------------------------------------------------
+        __syncthreads();  // the mixers hold their fragments of phi
+        for (int p = 0; p < T; p++) {
+            // Tile p has landed, for everybody behind the barrier: its dy is the last of it, requested in period p - 2, and
+            // behind that are the x of tile p + 2 and the dy of tile p + 1 (period p - 1).  Towards the end there are fewer.
+            if (p + 2 >= T) wait_vmem<0>();
+            else if (slab == 0) wait_vmem<2 * N + ST::kShareDt>();
+            else wait_vmem<2 * N + ST::kShare>();
+            stage_barrier();
+            // everybody is done with x of tile p - 1 and with dx of tile p - 2, whose places these take
+            if (p + ST::kXAhead < T) load_x(p + ST::kXAhead);
+            if (p + ST::kGAhead < T) load_dy(p + ST::kGAhead);
+            if (slab == 0) {  // dt column sums: 32 columns x 2 kLoaders row groups
+                const char *st = smem + p % ST::kXRing * ST::kXBytes;
+                const int col = tid & 31, rg = (tid >> 5) - 2 * ST::kMixers, left = b_end - (b_begin + p * TB);
+                const float *dts = reinterpret_cast<const float *>(st + ST::kCoef) + ST::kSegs * 64;
+                if (col < D + 3) {
+#pragma unroll
+                    for (int rr = 0; rr < TB / (2 * ST::kLoaders); rr++) {
+                        const int bb = rg * (TB / (2 * ST::kLoaders)) + rr;
+                        if (bb < left) dtsum += dts[bb * (D + 3) + col];
+                    }
+                }
+            }
+        }
+        stage_barrier();  // the mixers' last dx
+    } else {
+        // ---- dphi and dx of a tile, stores dx of the one before -------------------------------------------
+        bf16x8_t phif[N];  // A operand: rows = this wave's 16 channels of a stream, contraction over d
+        {
+            const int q = lane & 3, jj = (lane >> 2) & 3;
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                const char *p = phi_s + ((kq * 8 + jj) * N + j) * CW * 2 + (16 * wave + 4 * q) * 2;
+                typedef __attribute__((address_space(3))) lds_tr_v4i16 *lds_ptr;
+                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p));
+                const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 4 * N * CW * 2)));
+                phif[j] = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+            }
+        }
+        const float4 w4 = *reinterpret_cast<const float4 *>(smem + ST::kW + cl * 4);
+        const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
+        const float inv_c = 1.0f / (float)C;
+        __syncthreads();  // the loaders may fill the places that hold phi
+        const int row_at = l16 * CW * 2 + (((cl >> 3) ^ slab_swizzle<CW>(l16)) * 16) + (kq & 1) * 8;  // this lane's 8 bytes of its sample's row
+        // a tile of dx leaves in pieces of one KiB, kOut for every mixer
+        constexpr int kPieces = N * TB / kRows, kOut = (kPieces + ST::kMixers - 1) / ST::kMixers;
+        auto store_dx = [&](int t) {
+            const int sb = b_begin + t * TB;
+            const char *g = smem + ST::kG + t % ST::kGRing * ST::kTile;
+#pragma unroll
+            for (int i = 0; i < kOut; i++) {
+                const int at = wave + i * ST::kMixers, piece = min(at, kPieces - 1), j = piece / (TB / kRows), row = lane_row(piece % (TB / kRows) * kRows);
+                const int c = lane_col(row);
+                const uint4 v = *reinterpret_cast<const uint4 *>(g + piece * 1024 + lane * 16);
+                if (at < kPieces && sb + row < b_end && c < C)  // C % 8 == 0: eight channels are inside or outside
+                    st16<true>(a.dx + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+            }
+        };
+        // dphi: 32-column tiles wave, wave + kMixers (stream, 32-channel group)
+        constexpr int kCols = N * CW / 32, kAcc = (kCols + ST::kMixers - 1) / ST::kMixers;
+        f32x16_t acc[kAcc];
+#pragma unroll
+        for (int k = 0; k < kAcc; k++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[k][i] = 0.f;
+        // transposed reads of x: this lane's row (lo; hi: + 4) and its 8 bytes of a 32-channel group
+        const int tr_q = lane & 3, tr_row = (lane >> 5) * 8 + ((lane >> 2) & 3), tr_c = ((lane >> 4) & 1) * 2 + (tr_q >> 1);
+        for (int t = 0; t < T; t++) {
+            const char *st = smem + t % ST::kXRing * ST::kXBytes;
+            char *const gs = smem + ST::kG + t % ST::kGRing * ST::kTile;
+            const int sb = b_begin + t * TB;
+            const float *co = reinterpret_cast<const float *>(st + ST::kCoef);
+            MHC_PHASE_ADD(kPhaseBwdSlab, pwg, t > 0 ? 2 : 0, pclk);
+            stage_barrier();
+            MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 1, pclk);
+            if (t > 0) store_dx(t - 1);
+            const bf16x8_t ah = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + lane * 16);
+            const bf16x8_t al = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + 1024 + lane * 16);
+#pragma unroll
+            for (int k = 0; k < kAcc; k++) {
+                const int tile = wave + k * ST::kMixers, c = (tile % (CW / 32)) * 4 + tr_c;
+                if (kCols % ST::kMixers != 0 && tile >= kCols) break;
+                typedef __attribute__((address_space(3))) lds_tr_v4i16 *lds_ptr;
+                const char *xs = st + (tile / (CW / 32) * TB + tr_row) * CW * 2 + (tr_q & 1) * 8;
+                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(xs + (c ^ slab_swizzle<CW>(tr_row)) * 16)));
+                const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds_ptr)(xs + 4 * CW * 2 + (c ^ slab_swizzle<CW>(tr_row + 4)) * 16)));
+                const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+                acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, xf, acc[k], 0, 0, 0);
+                acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, xf, acc[k], 0, 0, 0);
+            }
+            // projection term: columns = samples, rows = this lane's channels
+            const bf16x8_t pf = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + 2048 + lane * 16);
+            f32x4_t o[N];
+            uint2 xr[N], gr[N];
+            float Mr[N][N], hpre[N], hpost[N];
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(phif[j], pf, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * CW * 2 + row_at);
+                gr[j] = *reinterpret_cast<const uint2 *>(gs + j * TB * CW * 2 + row_at);
+            }
+            lds_floats<N * N>(co + l16 * N * N, &Mr[0][0]);
+            lds_floats<N>(co + ST::kSegM * 64 + l16 * N, hpre);
+            lds_floats<N>(co + (ST::kSegM + 1) * 64 + l16 * N, hpost);
+            const float *sc = co + (ST::kSegM + 2) * 64 + l16;
+            const float cxv = sc[0];
+            float qinv = 0.f, k2 = 0.f;
+            if constexpr (!INJECT) {
+                qinv = 1.0f / sc[64];
+                k2 = sc[128] * qinv * qinv * qinv * inv_c;
+                qinv = sb + l16 < b_end ? qinv : 0.f;  // a slot beyond the batch adds nothing to usum
+            }
+            float dfv[4];
+            uint32_t out[N][2];
+#pragma unroll
+            for (int p = 0; p < 2; p++) {  // channel pairs
+                float r[N][2];
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int c = 2 * p + e;
+                    float xv[N], gv[N];
+#pragma unroll
+                    for (int j = 0; j < N; j++) {
+                        const uint32_t xw = p ? xr[j].y : xr[j].x, gw = p ? gr[j].y : gr[j].x;
+                        xv[j] = e ? bf16hi_to_f32(xw) : bf16lo_to_f32(xw);
+                        gv[j] = e ? bf16hi_to_f32(gw) : bf16lo_to_f32(gw);
+                    }
+                    float s_a = 0.f, s_df = 0.f;
+#pragma unroll
+                    for (int j = 0; j < N; j++) { s_a += hpre[j] * xv[j]; s_df += hpost[j] * gv[j]; }
+                    dfv[c] = s_df;
+                    const float dq = s_df * qinv;
+                    const float da = INJECT ? 0.f : dq * wv[c] - s_a * k2;
+                    if constexpr (!INJECT) usum[c] += dq * s_a;
+#pragma unroll
+                    for (int j = 0; j < N; j++) {
+                        float v = o[j][c] + hpre[j] * da - cxv * xv[j];
+#pragma unroll
+                        for (int i = 0; i < N; i++) v += Mr[i][j] * gv[i];
+                        r[j][e] = v;
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < N; j++) out[j][p] = pack_bf16x2(r[j][0], r[j][1]);
+            }
+#pragma unroll
+            for (int j = 0; j < N; j++) *reinterpret_cast<uint2 *>(gs + j * TB * CW * 2 + row_at) = make_uint2(out[j][0], out[j][1]);
+            if (INJECT && a.df && sb + l16 < b_end && c0 + cl < C)
+                store_vec<bf16_t, 4>(a.df + (size_t)sb * C + (uint32_t)(l16 * C + c0 + cl), dfv);
+        }
+        MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 2, pclk);
+        stage_barrier();
+        store_dx(T - 1);
+        float *dphi_out = a.dphi_part + (size_t)blockIdx.y * D * nC;
+#pragma unroll
+        for (int k = 0; k < kAcc; k++) {
+            const int tile = wave + k * ST::kMixers, c = c0 + tile % (CW / 32) * 32 + (lane & 31);
+            if (tile < kCols && c < C) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int d = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                    if (d < D) dphi_out[(size_t)d * nC + (size_t)(tile / (CW / 32)) * C + c] = acc[k][i];
+                }
+            }
+        }
+    }
+
+    // ---- small outputs of the split -------------------------------------------------------------------
+    MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 3, pclk);
+    __syncthreads();  // everyone is done with the rings; reuse them for the two small reductions
+    if constexpr (!INJECT) {
+        float *red = smem_f;  // [16][CW + 1]
+        if (!loader) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) red[l16 * (CW + 1) + cl + v] = usum[v];
+        }
+        __syncthreads();
+        if (tid < CW) {
+            double s = 0.0;
+#pragma unroll
+            for (int r = 0; r < 16; r++) s += red[r * (CW + 1) + tid];
+            if (c0 + tid < C) a.dw_part[(size_t)blockIdx.y * C + c0 + tid] = s;
+        }
+        __syncthreads();
+    }
+    if (slab == 0) {
+        double *red = reinterpret_cast<double *>(smem);  // [2 kLoaders][32]
+        if (loader) red[tid - 64 * ST::kMixers] = dtsum;
+        __syncthreads();
+        if (tid < 32 && tid < D + 3) {
+            double s = 0.0;
+#pragma unroll
+            for (int r = 0; r < 2 * ST::kLoaders; r++) s += red[r * 32 + tid];
+            a.dt_part[(size_t)blockIdx.y * (D + 3) + tid] = s;
+        }
+    }
+    MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 4, pclk);
+}
+
 bool bwd_slab_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) {
     (void)y_dtype;
     return x_dtype == kBF16 && phi_dtype == kBF16 && n <= 4 && C % 8 == 0;
 }
 
-int bwd_slab_batch_splits(int B, int n, int C) {
-    const int slabs = (C + kSlabCW - 1) / kSlabCW;
-    const int tiles = (B + 31) / 32;
+// Channels per workgroup of the bf16 kernel.  A CU carries one workgroup of either width, so the narrow one leaves half as
+// many partial sums of dphi behind (C / 64 slabs in half as many splits) but has half the waves to hide its latencies
+// and loads half as wide pieces of a row.  Backward, 64 | 128 channels (us, the better split count of each):
+//   n=4  B=800 C=1280 23.5 | 25.0   1024 x 1024 22.4 | 24.9   2048 x 512 27.0 | 29.4   6000 x 256 40.8 | 43.8
+//        1024 x 2048 29.0 | 29.8   2048 x 1280 37.0 | 38.2   4096 x 640 39.5 | 40.7   8192 x 320 51.5 | 54.0
+//        1280 x 2560 39.2 | 37.4   900 x 4096 47.3 | 45.5   8192 x 768 66.3 | 64.9   3000 x 4096 101 | 91
+//   n=3  1500 x 1920 31.3 | 30.1   n=2  4000 x 1024 35.6 | 35.7   1000 x 2560 29.7 | 29.3
+// The lines: n = 4 below 12 M activation elements.
+static int slab_width(int B, int n, int C) {
+    if (const int forced = tuning_get(kTuneSlabWidth)) return forced == 1 ? 64 : 128;
+    return n == 4 && (long long)B * n * C < 12'000'000 ? 64 : 128;
+}
+
+int bwd_slab_batch_splits(int B, int n, int C, int y_dtype) {
+    const bool staged = y_dtype == kBF16;
+    const int width = staged ? slab_width(B, n, C) : kSlabCW, slabs = (C + width - 1) / width;
+    const int tiles = (B - 1) / (staged ? 16 : 32) + 1;
     if (const int forced = tuning_get(kTuneSlabSplits); forced > 0) {  // experiment hook
         return forced < tiles ? forced : tiles;
     }
-    // Two workgroups per CU, all resident at once (one split more than that costs a second round:
-    // B=1280 C=2560, 12 splits 42.5 us, 13 splits 48.5).
-    int S = 512 / slabs;
+    // All workgroups resident at once: one per CU (bf16 dy) or two (fp32 dy).  One split more than that costs a second
+    // round (B=1280 C=2560, 12 splits of 20 slabs 37.4 us, 20 splits 45.1), fewer leave CUs idle (8 splits 40.2).
+    int S = std::max(1, (staged ? 256 : 512) / slabs);
     if (S > tiles) S = tiles;
-    // the dphi partial copies (written here, read once by the finalize launch) stay below 16 MB or
-    // 0.4 of the activation bytes this kernel moves, whichever is larger
-    const int D = n * n + 2 * n;
-    const double part = 2.0 * 4.0 * D * n * C;  // bytes written + read per split
-    double budget = 0.4 * (3.0 * 2.0 * B * n * C);
-    if (budget < 16e6) budget = 16e6;
-    if (S > (int)(budget / part)) S = (int)(budget / part);
-    if (S < 1) S = 1;
+    if (!staged) {
+        // the dphi partial copies (written here, read once by the finalize launch) stay below 16 MB or
+        // 0.4 of the activation bytes this kernel moves, whichever is larger
+        const int D = n * n + 2 * n;
+        const double part = 2.0 * 4.0 * D * n * C;  // bytes written + read per split
+        double budget = 0.4 * (3.0 * 2.0 * B * n * C);
+        if (budget < 16e6) budget = 16e6;
+        if (S > (int)(budget / part)) S = std::max(1, (int)(budget / part));
+    }
     // the longest split decides: the fewest splits that keep its tile count
-    // (backward us: B=1024 C=2560  11 splits of 3 tiles 37 | 8 of 4: 40.0;  B=1536 C=1920  16 of 3: 39.4 | 12 of 4: 41.7;
-    //  B=800 C=1280  13 of 2: 25.5 | 12 of 2 or 3: 28.8)
     const int tps = (tiles + S - 1) / S;
-    S = (tiles + tps - 1) / tps;
-    return S;  // <= tiles: every split has at least one tile
+    return (tiles + tps - 1) / tps;  // <= tiles: every split has at least one tile
 }
 
 hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const void *w, int w_dtype,
                            const void *f_inject, const void *phi, const float *Hpre,
                            const float *Hpost, const float *M, const float *q, const float *s1,
                            const float *cx, const void *dPb, const void *dPT, int BP, const float *dt,
-                           void *dx, void *df, float *dphi_part, float *dw_part, float *dt_part, int S,
+                           void *dx, void *df, float *dphi_part, double *dw_part, double *dt_part, int S,
                            int B, int n, int C, hipStream_t stream) {
-    const int tiles = (B + 31) / 32;
+    const int tiles = y_dtype == kBF16 ? (B - 1) / 16 + 1 : (B + 31) / 32;
     if (S < 1 || S > tiles) return hipErrorInvalidValue;
     BwdSlabArgs a{dy, static_cast<const bf16_t *>(x), w, f_inject, static_cast<const bf16_t *>(phi),
                   Hpre, Hpost, M, q, s1, cx, static_cast<const bf16_t *>(dPb),
                   static_cast<const bf16_t *>(dPT), dt, static_cast<bf16_t *>(dx),
                   static_cast<bf16_t *>(df), dphi_part, dw_part, dt_part, w_dtype == kBF16, B, BP, n, C, tiles};
+    if (y_dtype == kBF16) {
+        const int cw = slab_width(B, n, C);
+        dim3 grid((C + cw - 1) / cw, S);
+#define MHC_SLAB(N, CW, INJ)                                                                                      \
+    do {                                                                                                          \
+        constexpr size_t lds = SlabStage<N, CW>::kLds;                                                            \
+        if (hipError_t e = allow_dynamic_lds<&bwd_slab_stage_kernel<N, CW, INJ>>(lds); e != hipSuccess) return e; \
+        bwd_slab_stage_kernel<N, CW, INJ><<<grid, SlabStage<N, CW>::kThreads, lds, stream>>>(a);                                      \
+    } while (0)
+#define MHC_SLAB_N(N)                                                                       \
+    do {                                                                                    \
+        if (cw == 64) { if (f_inject) MHC_SLAB(N, 64, true); else MHC_SLAB(N, 64, false); } \
+        else { if (f_inject) MHC_SLAB(N, 128, true); else MHC_SLAB(N, 128, false); }        \
+    } while (0)
+        switch (n) {
+            case 1: MHC_SLAB_N(1); break;
+            case 2: MHC_SLAB_N(2); break;
+            case 3: MHC_SLAB_N(3); break;
+            default: MHC_SLAB_N(4); break;
+        }
+#undef MHC_SLAB_N
+#undef MHC_SLAB
+        return hipGetLastError();
+    }
     const size_t smem = sizeof(float) * 32 * kSlabLDF + sizeof(bf16_t) * 32 * kSlabLDX;
     dim3 grid((C + kSlabCW - 1) / kSlabCW, S);
-    if (y_dtype == kBF16) bwd_slab_kernel<bf16_t><<<grid, 256, smem, stream>>>(a);
-    else bwd_slab_kernel<float><<<grid, 256, smem, stream>>>(a);
+    bwd_slab_f32dy_kernel<<<grid, 256, smem, stream>>>(a);
     return hipGetLastError();
 }
 

@@ -135,10 +135,11 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     w.dP = c.floats((size_t)B * padded_D(n));
     w.cx = c.floats(B);
     w.s1 = c.floats(B);
-    // partial sums of dw and dt: float32 rows of at most B, float64 rows of the fp32 slab kernel or of the resident
+    // partial sums of dw and dt: float32 rows of at most B, float64 rows of the slab kernels or of the resident
     // backward's second launch with a split batch
+    const int bs3 = n <= 4 ? std::max(bwd_slab_batch_splits(B, n, C, kBF16), bwd_slab_batch_splits(B, n, C, kF32)) : 1;
     const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1, bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
-    const size_t slab64 = n <= 4 ? bs5 : 0, parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
+    const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : 0, parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
     w.u = c.floats(std::max((size_t)B, 2 * slab64) * C);
     w.upart = c.floats(2 * parts64 * C);
     w.dtpart = c.floats(std::max((size_t)B, 2 * std::max(slab64, parts64)) * (D + 3));
@@ -152,7 +153,6 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     int bs = dphi_batch_splits(B, n, C);
     const int bs2 = proj_bwd_batch_splits(B, n, C);
     if (bs2 > bs) bs = bs2;
-    const int bs3 = n <= 4 ? bwd_slab_batch_splits(B, n, C) : 1;
     if (bs3 > bs) bs = bs3;
     const int bs4 = dphi_f32_splits(B, n, C);
     if (bs4 > bs) bs = bs4;
@@ -694,12 +694,13 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
                                      st));
     if (mfma && bwd_slab_supported(x_dtype, y_dtype, phi_dtype, n, C)) {
         // n <= 4: one slab kernel finishes dx and produces every batch-split partial sum
-        const int S = bwd_slab_batch_splits(B, n, C);
+        const int S = bwd_slab_batch_splits(B, n, C, y_dtype);
         MHC_LAUNCH(launch_bwd_slab(dy, y_dtype, x, w, w_dtype, f_inject, phi, H_pre, H_post, M, q, ws.s1,
                                    ws.cx, ws.dPb, ws.dPT, ws.BP, ws.dt, dx, df,
-                                   S > 1 ? ws.dphi_part : dphi, ws.u, ws.dtpart, S, B, n, C, st));
+                                   S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
+                                   reinterpret_cast<double *>(ws.dtpart), S, B, n, C, st));
         MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S, D, dbias, dalpha,
-                                   ws.dphi_part, S, (size_t)D * n * C, dphi, st));
+                                   ws.dphi_part, S, (size_t)D * n * C, dphi, st, true));
         return MHC_OK;
     }
     if (bwd_slab_f32_supported(x_dtype, phi_dtype, n, C)) {

@@ -179,15 +179,15 @@ hipError_t launch_mix_bwd_dx(const void *dy, int y_dtype, const void *x, int x_d
                              hipStream_t stream);
 
 // Slab kernel for n <= 4 in the bf16 tier: dx (complete), df, and the batch-split partial sums of
-// dphi [S][D][nC], dw [S][C] and dt [S][D+3] in one pass over dy and x.  With S == 1 pass the final
+// dphi [S][D][nC], dw [S][C] and dt [S][D+3] (the last two in float64) in one pass over dy and x.  With S == 1 pass the final
 // dphi as dphi_part.
 bool bwd_slab_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C);
-int bwd_slab_batch_splits(int B, int n, int C);
+int bwd_slab_batch_splits(int B, int n, int C, int y_dtype);
 hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const void *w, int w_dtype,
                            const void *f_inject, const void *phi, const float *Hpre,
                            const float *Hpost, const float *M, const float *q, const float *s1,
                            const float *cx, const void *dPb, const void *dPT, int BP, const float *dt,
-                           void *dx, void *df, float *dphi_part, float *dw_part, float *dt_part, int S,
+                           void *dx, void *df, float *dphi_part, double *dw_part, double *dt_part, int S,
                            int B, int n, int C, hipStream_t stream);
 
 // The same for the fp32 tier (n <= 4, even C), behind launch_mix_bwd_reduce (dP [B, 32], cx, s1, dt of `co`):

@@ -19,7 +19,8 @@ enum TuneKey {
     kTuneWideDxBeside = 8,  // wide projections (n > 18): dx workgroups beside the coefficient launch: 1 = never, 2 = always
     kTuneSpareB = 9,        // projection forward (matrix-core kernels): K splits, 0 = by heuristic
     kTuneGather = 10,       // projection reads the caller's fp32 parameters itself: 1 = never, 2 = whenever the shape allows
-    kTuneCount = 11
+    kTuneSlabWidth = 11,    // slab backward (n <= 4, bf16): channels per workgroup, 1 = 64, 2 = 128, 0 = by size
+    kTuneCount = 12
 };
 
 #ifdef MHC_TUNING

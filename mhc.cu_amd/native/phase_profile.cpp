@@ -164,9 +164,9 @@ int main(int argc, char **argv) {
                  "fragments, dphi on the matrix cores (all)", "dxflat on the matrix cores, stores (all)", "dphi stores"}, false);
         return 0;
     }
-    const int slabs = (C + 63) / 64;
-    summary("slab backward kernel, one workgroup per (64 channels, batch split)", 1, std::min(slabs * 4, 4096),
-            {"prologue (phi slab, first loads)", "tile loads, LDS, barrier (all tiles)", "matrix cores, barrier (all tiles)",
-             "coefficients, mixing, stores (all)", "epilogue: dphi partial stores", "epilogue: dw / dbias partial sums"}, false);
+    const int width = n == 4 && (long long)B * n * C < 12000000 ? 64 : 128, slabs = (C + width - 1) / width;
+    summary("slab backward kernel, one workgroup per (64 or 128 channels, batch split), its first mixer", 1, std::min(slabs * 4, 4096),
+            {"prologue (phi slab, first loads)", "barriers: tile on its way, other waves (all)",
+             "dphi, dx, stores of the tile before (all)", "last dx, dphi partial stores", "epilogue: dw / dbias partial sums"}, false);
     return 0;
 }
