@@ -23,6 +23,7 @@ struct BwdReduceArgs {
     // backward, which then has half its chain left (SkWg::save_state layout, (2 T + 2) * NP floats)
     const float *static_logits = nullptr;
     float *static_state = nullptr;
+    int per_wg = 1;  // gram_quad_kernel: samples per workgroup, up to four
 };
 
 // Where the weight of the W1 = dy diag(w) x^T Gram matrix comes from: an injected f [B, C] (W1 = dy [f; 0 ..]^T),
@@ -147,11 +148,13 @@ template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = fals
     // still on their way.  g: lane within the group; lane: lane within the wave (indexes sc).
     // With the denominators saved by the forward call there is nothing to iterate: they are copied
     // into sc and the final iterate is the saved M.
+    // kBatch: iterations of the saved state requested together (two registers each).
+    template <int kBatch = 24>
     __device__ __forceinline__ void forward_recompute(const BwdReduceArgs &a, int b, int g, int lane, float *sc) {
         if (a.sk_state) {
             // every load is requested before the first value (of prefetch() too) is used
             m_fin = a.M[(size_t)b * a.n * a.n + (mv ? r0 * a.n + c0 : 0)];
-            SK::load_state(a.sk_state + (size_t)b * SK::state_floats(a.T), g, a.T, sc, lane);
+            SK::template load_state<kBatch>(a.sk_state + (size_t)b * SK::state_floats(a.T), g, a.T, sc, lane);
             m_fin = mv ? m_fin : 0.f;
             return;
         }

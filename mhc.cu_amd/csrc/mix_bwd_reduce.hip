@@ -393,6 +393,135 @@ __global__ __launch_bounds__(256, NP == 4 ? 4 : kMfmaMinWaves) void gram_small_k
     }
 }
 
+// The same launch (n <= 4, dynamic H, coefficient backward inside) for large batches: a workgroup takes three or four
+// samples.  Its streaming waves hold a sample's rows together (U <= 3 steps each, every load of the sample requested at
+// once) and go through them; then wave 0 runs the coefficient backward of all, one per 16 lanes, in the time and with the
+// instructions of one.  In gram_small_kernel, one sample per workgroup, that tail is a fifth of all instructions and
+// over a quarter of a workgroup's life, and three of four lanes of its wave are empty; more loads in flight alone gained
+// nothing there.  Registers decide how many workgroups a CU holds: w comes from LDS, the saved Sinkhorn state in batches of
+// eight iterations, and four steps per wave (80 registers and spills) lost to gram_small_kernel.
+// B=8192 n=4 C=2560: 72 -> 65 us (336 MB, 5.2 TB/s).
+constexpr int kGramQuadSteps = 33;
+template <int WMODE, int U>
+__global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduceArgs a) {
+    using SK = SkSmall<4>;
+    using CB = CoefBwdSmall<4, false, true>;
+    constexpr int K = CB::K, Q = SK::kPerWave;
+    constexpr bool inject = WMODE == kGramInject;
+    extern __shared__ float smem[];  // slots [Q][K][SW] | sums [Q][K] | Sinkhorn denominators, SK::scaling_floats(T) | Q CB::kXch | w, 16-byte aligned
+    const int b0 = blockIdx.x * a.per_wg, n = a.n, C = a.C, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), SW = (blockDim.x >> 6) - 1;
+    const int nb = min(a.per_wg, a.B - b0);
+    float *slot_s = smem, *tot_s = slot_s + Q * K * SW, *sc = tot_s + Q * K;
+    MHC_PHASE_ZERO(kPhaseGramSmall, blockIdx.x);
+    MHC_PHASE_BEGIN(pclk);
+    if (wave == 0) {
+        CB cb;
+        const int k = lane / SK::kGroup, g = lane % SK::kGroup;
+        const bool live = k < nb;  // whole groups: the reductions never cross them
+        if (live) {
+            cb.prefetch(a, b0 + k, g);
+            cb.forward_recompute<8>(a, b0 + k, g, lane, sc);
+        }
+        MHC_PHASE_ADD(kPhaseGramSmall, blockIdx.x, 0, pclk);
+        __syncthreads();
+        MHC_PHASE_ADD(kPhaseGramSmall, blockIdx.x, 1, pclk);
+        for (int e = lane; e < nb * K; e += 64) {
+            float v = 0.f;
+            for (int r = 0; r < SW; r++) v += slot_s[e * SW + r];
+            tot_s[e] = v;
+        }
+        MHC_PHASE_ADD(kPhaseGramSmall, blockIdx.x, 2, pclk);
+        if (live) {  // (same wave: no barrier)
+            cb.fetch_sums(tot_s + k * K, 1);
+            cb.run(a, b0 + k, g, lane, sc, sc + SK::scaling_floats(a.T) + k * CB::kXch);
+        }
+        MHC_PHASE_ADD(kPhaseGramSmall, blockIdx.x, 3, pclk);
+        return;
+    }
+    const int blk = lane >> 2, i = lane & 3, nsteps = (C + 127) / 128;
+    const int s_first = wave - 1;  // this wave's steps: s_first, s_first + SW ..
+    // w of the streaming waves' steps, each wave's own chunks: from LDS, since registers decide how many workgroups a CU holds
+    typedef typename std::conditional<WMODE == kGramWF32, float, bf16_t>::type TW;
+    TW *w_s = reinterpret_cast<TW *>(smem + (Q * (K * (SW + 1) + CB::kXch) + SK::scaling_floats(a.T) + 3) / 4 * 4);
+    if constexpr (!inject) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int c = (s_first + u * SW) * 128 + lane * 2;
+            if (c < C) { w_s[c] = static_cast<const TW *>(a.w)[c]; w_s[c + 1] = static_cast<const TW *>(a.w)[c + 1]; }
+        }
+    }
+    for (int k = 0; k < nb; k++) {
+        const bf16_t *gb = static_cast<const bf16_t *>(a.dy) + (size_t)(b0 + k) * n * C;
+        const bf16_t *xb = static_cast<const bf16_t *>(a.x) + (size_t)(b0 + k) * n * C;
+        uint4 gr[U], xr[U], fr[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            // beyond the row: any valid chunk (dropped or masked below); streams >= n alias stream 0: their entries of the
+            // sums are read by nobody
+            const int st = s_first + u * SW < nsteps ? s_first + u * SW : 0;
+            const uint32_t at = (uint32_t)((i < n ? i : 0) * C + st * 128 + min(blk * 8, C - 8 - st * 128));
+            gr[u] = *reinterpret_cast<const uint4 *>(gb + at);
+            xr[u] = *reinterpret_cast<const uint4 *>(xb + at);
+            if constexpr (inject)
+                fr[u] = load16_masked(reinterpret_cast<const uint4 *>(static_cast<const bf16_t *>(a.f_inject) + (size_t)(b0 + k) * C +
+                                                                      st * 128 + min(blk * 8, C - 8 - st * 128)), i == 0);
+        }
+        f32x4_t acc[3];
+#pragma unroll
+        for (int m = 0; m < 3; m++) acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int st = s_first + u * SW;
+            if (st >= nsteps) break;
+            if ((st + 1) * 128 > C) {  // the row ends within this step
+                const bool in = st * 128 + blk * 8 < C;
+                gr[u].x = in ? gr[u].x : 0u; gr[u].y = in ? gr[u].y : 0u; gr[u].z = in ? gr[u].z : 0u; gr[u].w = in ? gr[u].w : 0u;
+                xr[u].x = in ? xr[u].x : 0u; xr[u].y = in ? xr[u].y : 0u; xr[u].z = in ? xr[u].z : 0u; xr[u].w = in ? xr[u].w : 0u;
+            }
+            const bf16x4_t x0 = bf16x4_of(xr[u].x, xr[u].y), x1 = bf16x4_of(xr[u].z, xr[u].w);
+            const bf16x4_t g0 = bf16x4_of(gr[u].x, gr[u].y), g1 = bf16x4_of(gr[u].z, gr[u].w);
+            acc[0] = mfma4(g0, x0, acc[0]);
+            acc[0] = mfma4(g1, x1, acc[0]);
+            if constexpr (inject) {
+                acc[1] = mfma4(g0, bf16x4_of(fr[u].x, fr[u].y), acc[1]);
+                acc[1] = mfma4(g1, bf16x4_of(fr[u].z, fr[u].w), acc[1]);
+            } else {
+                float wv[8];
+                load_vec<TW, 8>(w_s + st * 128 + min(blk * 8, C - 8 - st * 128), wv);
+                // dy * w as a bf16 pair (rounded value + remainder), see gram_small_kernel
+                const uint32_t gw[4] = {gr[u].x, gr[u].y, gr[u].z, gr[u].w};
+                uint32_t hw[4], lw[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float p0 = bf16lo_to_f32(gw[e]) * wv[2 * e], p1 = bf16hi_to_f32(gw[e]) * wv[2 * e + 1];
+                    hw[e] = pack_bf16x2(p0, p1);
+                    lw[e] = pack_bf16x2(p0 - bf16lo_to_f32(hw[e]), p1 - bf16hi_to_f32(hw[e]));
+                }
+                acc[1] = mfma4(bf16x4_of(hw[0], hw[1]), x0, acc[1]);
+                acc[1] = mfma4(bf16x4_of(hw[2], hw[3]), x1, acc[1]);
+                acc[1] = mfma4(bf16x4_of(lw[0], lw[1]), x0, acc[1]);
+                acc[1] = mfma4(bf16x4_of(lw[2], lw[3]), x1, acc[1]);
+                acc[2] = mfma4(x0, x0, acc[2]);
+                acc[2] = mfma4(x1, x1, acc[2]);
+            }
+        }
+        // lane (block, j) holds column j of its block's products, register = row: sum over the sixteen blocks
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float v = acc[m][r];
+                v += dpp_mov<kDppRowRor4>(v);
+                v += dpp_mov<kDppRowRor8>(v);
+                v = xor16_add(v);
+                v = xor32_add(v);
+                if (lane < 4) slot_s[(k * K + m * 16 + 4 * r + lane) * SW + wave - 1] = v;
+            }
+    }
+    __syncthreads();
+}
+
 // =============================================================================================
 // n > 8: the channel sums as three 32x32 Gram matrices on the matrix cores
 //
@@ -940,16 +1069,29 @@ static bool gram_small_supported(const BwdReduceArgs &a) { return a.raw != nullp
 // Column parts of gram_small_kernel: never more than bwd_reduce_parts(), which sizes `raw`.
 static int gram_small_parts(int B, int C) { return C >= 1024 && B < 1024 ? 2 : 1; }
 
-// One launch (channel sums, then the coefficient backward at the tail of every workgroup) unless the
+// gram_small_kernel: one launch (channel sums, then the coefficient backward at the tail of every workgroup) unless the
 // Sinkhorn state would take the LDS that keeps several workgroups per CU resident, or the batch is
 // too small to do without column parts.
 static bool gram_small_fused(const BwdReduceArgs &a) {
     if (const int hook = tuning_get(kTuneGramFused); hook && a.T <= 32) return hook == 2;  // experiment hook
-    // very short rows in a very large batch: the tail of a workgroup (one wave, 2.6 us) outweighs its
-    // streaming, and a separate launch packs the chains of four samples into a wave
-    // (backward us, one launch | two: B=8192 n=4 C=128 50.3 | 45.2, 6000 C=256 46.7 | 45.4, 4096 C=512 42.4 | 45.5)
+    // (n <= 4: the tail of a workgroup outweighs the streaming of very short rows, but such batches of those take
+    // gram_quad_kernel; n > 4 has no rows to pack four samples of into a wave)
     if (a.B >= 6000 && a.C <= 256) return false;
     return a.T <= 32 && (a.B >= 128 || a.C <= 2048);
+}
+
+// Samples per workgroup of gram_quad_kernel, 0 = not taken.  Backward us, gram_small_kernel | four | three | two per workgroup:
+//   C=1280 n=4  B=1280 (C=2560) 37.7 | 42.1 | 39.4 | 39.8   1600 32.3 | 33.2 | 32.9 | 32.5   1800 39.5 | 37.9 | 37.9 | 37.1
+//               2048 37.4 | 35.7 | 35.5 | 35.2   2500 45.3 | 44.8 | 41.5 | 43.5   4000 54.7 | 51.0 | 53.6 | 54.0
+//               5300 67.1 | 65.3 | 63.9 | 65.7   7000 80.7 | 77.9 | 78.9 | 79.6   8192 (C=2560) 171 | 165 | 168 | 169
+//   C=512       1600 25.2 | 25.7 | 25.6 | 24.9   3500 37.0 | 35.6 | 33.9 | 35.9   5000 44.5 | 41.0 | 41.4 | 43.5
+//   (the second launch that very short rows took instead: B=8192 C=128 42.7 -> 35.4, C=256 45.5 -> 37.4)
+// So from 1700 samples on, four where that gives the busiest CU less to do than three.
+static int gram_quad_samples(const BwdReduceArgs &a) {
+    const int hook = tuning_get(kTuneGramFused);  // experiment hook
+    if ((a.C + 127) / 128 > kGramQuadSteps || a.T > 32 || (hook ? hook != 2 : a.B < 1700)) return 0;
+    const auto busiest = [&](int q) { return ((a.B - 1) / q / 256 + 1) * q; };
+    return hook || busiest(4) < busiest(3) ? 4 : 3;
 }
 
 template <int NP, bool FUSED>
@@ -965,6 +1107,31 @@ template <int NP>
 static hipError_t launch_gram_small(BwdReduceArgs a, hipStream_t stream) {
     using SK = SkSmall<NP>;
     using CB = CoefBwdSmall<NP, false, true>;
+    if constexpr (NP == 4) {
+        if (const int per_wg = gram_quad_samples(a)) {
+            // streaming waves: as many as give the fewest steps per wave, up to seven, eleven for rows beyond 21 steps
+            const int nsteps = (a.C + 127) / 128, most = nsteps <= 21 ? 7 : 11;
+            const int U = (nsteps + most - 1) / most, SW = (nsteps + U - 1) / U, Q = SK::kPerWave;
+            a.parts = 1;
+            a.per_wg = per_wg;
+            const size_t smem = sizeof(float) * ((Q * (CB::K * (SW + 1) + CB::kXch) + SK::scaling_floats(a.T) + 3) / 4 * 4 +
+                                                 (a.f_inject ? 0 : (a.w_bf16 ? (a.C + 1) / 2 : a.C)));  // at most 43 KB
+            const unsigned block = 64 * (SW + 1), grid = (a.B - 1) / per_wg + 1;
+#define MHC_GRAM(UU)                                                                                        \
+    do {                                                                                                    \
+        if (a.f_inject) gram_quad_kernel<kGramInject, UU><<<grid, block, smem, stream>>>(a);                \
+        else if (a.w_bf16) gram_quad_kernel<kGramWBf16, UU><<<grid, block, smem, stream>>>(a);              \
+        else gram_quad_kernel<kGramWF32, UU><<<grid, block, smem, stream>>>(a);                             \
+    } while (0)
+            switch (U) {
+                case 1: MHC_GRAM(1); break;
+                case 2: MHC_GRAM(2); break;
+                default: MHC_GRAM(3); break;
+            }
+#undef MHC_GRAM
+            return hipGetLastError();
+        }
+    }
     if (gram_small_fused(a)) {
         a.parts = 1;
         const size_t smem = sizeof(float) * (SK::scaling_floats(a.T) + CB::kXch);  // at most 16 KB + 96 B

@@ -121,9 +121,9 @@ template <int NP> struct SkSmall {
         sk_chain_end();
     }
     // Denominators saved by forward_save() -> the per-lane LDS layout that backward() reads.  The
-    // loads of 24 iterations are requested together (one round trip for the usual 20).
+    // loads of kBatch iterations are requested together (24: one round trip for the usual 20).
+    template <int kBatch = 24>
     __device__ static __forceinline__ void load_state(const float *st, int g, int T, float *sc, int lane) {
-        constexpr int kBatch = 24;
         const float *pr = st + row(g), *pc = st + NP + col0(g);
         for (int t0 = 0; t0 < T; t0 += kBatch) {
             float rs[kBatch], cs[kBatch];

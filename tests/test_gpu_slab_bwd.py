@@ -1,12 +1,13 @@
-"""The slab backward of n <= 4 (csrc/bwd_slab.hip): both channel widths at the edges of its tiles (16 samples, 64 / 128
+"""The tiled backward of n <= 4.  The slab kernel (csrc/bwd_slab.hip): both channel widths at the edges of its tiles (16 samples, 64 / 128
 channels), of its ring of tiles in flight (1 .. 5 tiles per batch split) and of its splits, against the oracle and
-each other.  Reference backward: src/python/mhc/ops.py:276-361."""
+each other.  The channel sums with the coefficient backward of several samples per workgroup (gram_quad_kernel,
+csrc/mix_bwd_reduce.hip): against the two launches.  Reference backward: src/python/mhc/ops.py:276-361."""
 import pytest
 
 from test_gpu_resident_bwd import K_RESIDENT, _both_paths
 
 pytestmark = pytest.mark.gpu
-K_SLAB_SPLITS, K_SLAB_WIDTH = 3, 11
+K_GRAM, K_SLAB_SPLITS, K_SLAB_WIDTH = 2, 3, 11
 
 # (B, n, C, splits; 0 = as the library chooses)
 SHAPES = [(1, 4, 8, 0), (16, 4, 128, 1), (17, 4, 136, 1), (33, 3, 64, 1), (50, 4, 72, 1), (65, 2, 200, 1), (80, 1, 40, 1),
@@ -25,3 +26,18 @@ def test_slab_backward_widths(B, n, C, splits, inject, w_f32):
     finally:
         lib.mhc_tuning_set(K_RESIDENT, 0)
         lib.mhc_tuning_set(K_SLAB_SPLITS, 0)
+
+
+# one to four samples in the last workgroup; rows of one step, of whole and cut steps, of one to three steps per wave
+@pytest.mark.parametrize("B,n,C", [(1, 4, 8), (2, 4, 128), (3, 2, 136), (5, 4, 904), (9, 3, 1032), (6, 4, 2560), (7, 1, 2688),
+                                   (4, 4, 4096), (10, 2, 4224)])
+@pytest.mark.parametrize("inject,w_f32", [(False, False), (False, True), (True, False)])
+def test_channel_sums_of_several_samples_per_workgroup(B, n, C, inject, w_f32):
+    from mhc._lib import tuning_lib
+
+    lib = tuning_lib()
+    try:
+        assert lib.mhc_tuning_set(K_RESIDENT, 1) == 0
+        _both_paths(K_GRAM, ("two launches", "several samples"), B, n, C, inject, w_f32)
+    finally:
+        lib.mhc_tuning_set(K_RESIDENT, 0)
