@@ -68,17 +68,19 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 // Whether the sample-resident backward (bwd_resident.hip + the column-slab kernel) is taken where it is
 // supported.  Its second launch walks all samples of a column slab in one workgroup, which stops paying once the batch is
 // large enough to fill the chip with batch splits; the fewer streams, the fewer slabs.
-// Measured, backward in graphs of ten, tiled (slab / Gram) path -> resident path (us):
-//   n=4 C=256:  B=768 19.2 -> 16.3, 2048 28.5 -> 22.2, 6000 45.8 -> 38.8;  C=640: B=768 21.4 -> 19.3, 1024 23.8 -> 26.3
-//   n=4 C=1280: B=64 17.1 -> 9.2, 320 19.1 -> 14.6, 512 23.0 -> 19.3, 768 25.2 -> 24.7, 1024 28.5 -> 29.5, 1536 34.6 -> 39.1
-//   n=4 C=2048: B=512 26.9 -> 23.9, 768 30.6 -> 28.8, 1024 33.8 -> 38.4;  C=2560: B=256 23.9 -> 18.2, 512 30.7 -> 27.9,
-//               640 32.8 -> 34.7, 768 34.7 -> 37.6
-//   n=3 C=1920: B=768 26.6 -> 24.7, 1024 28.5 -> 32.6;  n=2 C=512: B=768 18.6 -> 16.8, 2048 26.5 -> 28.2;  n=2 C=1280:
-//               B=768 20.3 -> 21.9, 1024 23.7 -> 29.0
-// (the line is one number, B <= 768: at its ends, C <= 256 and C >= 2500, it is off by a few us)
-// Rows of more than 2560 channels hand dxp over in fp32 (bwd_resident_dxp_f32), and the line lies lower:
-//   n=4 C=2688: B=512 32.4 -> 28.0, 768 34.8 -> 38.0;  C=4096: B=256 31.2 -> 23.8, 512 38.6 -> 38.7, 768 41.7 -> 53.4
-//   n=3 C=3072: B=256 20.9 -> 20.2, 512 28.5 -> 28.8, 768 32.8 -> 37.0;  n=2 C=4096: B=256 20.3 -> 22.0, 768 33.8 -> 39.5
+// Measured, backward in graphs of ten, tiled (Gram + slab) path | resident path (us):
+//   n=4 C=256:  B=768 19.8 | 16.1, 2048 26.7 | 22.2, 3000 27.5 | 27.5, 6000 34.9 | 39.3;  C=512: 768 19.7 | 17.5, 1024 21.5 | 22.0
+//   n=4 C=1024: B=640 21.4 | 20.2, 768 21.9 | 22.3, 1024 23.0 | 27.0;  C=1280: 320 18.8 | 14.8, 512 21.6 | 19.3, 640 22.4 | 23.1,
+//               768 22.5 | 24.9, 1024 25.0 | 29.3;  C=1920: 512 23.7 | 23.6, 640 25.2 | 28.4
+//   n=4 C=2560: B=192 20.9 | 16.4, 320 25.3 | 25.3, 512 27.7 | 27.2, 640 29.1 | 34.5;  C=3200: 512 31.1 | 30.5, 640 33.2 | 37.7
+//               C=4096: 192 27.5 | 22.1, 320 30.3 | 32.2, 512 34.1 | 38.0, 768 38.0 | 53.0
+//   n=3 C=512:  B=1024 22.9 | 21.5, 1536 23.8 | 31.5;  C=1280: 768 22.4 | 23.0;  C=1920: 384 20.7 | 17.9, 576 22.9 | 24.8;
+//               C=3200: 192 20.1 | 18.3, 384 25.5 | 26.2, 576 27.8 | 33.7
+//   n=2 C=512:  B=768 17.9 | 16.5, 1024 19.9 | 20.5;  C=1280: 512 16.2 | 16.6, 768 19.2 | 21.6;  C=1920: 384 17.0 | 15.9, 576 19.5 | 23.7;
+//               C=3200: 192 17.5 | 16.5, 384 20.8 | 25.4
+//   n=1 C=256:  B=768 15.8 | 15.1, 1024 17.2 | 18.0;  C=960: 576 16.3 | 16.1, 768 16.5 | 17.4;  C=3200: 192 16.1 | 13.9, 384 17.9 | 21.6
+// The tiled path is one launch more, so the lines lie a little above the crossings: about 1.0 M / C samples, within bounds,
+// and 768 n samples of at most 256 channels (n=4 C=128: B=4096 31.9 | 27.1, 6000 35.0 | 33.9).
 // n = 5 .. 8 at every batch size:
 //   n=8 C=1280: B=128 25.1 -> 16.0, 256 30.5 -> 21.2, 512 46.1 -> 34.1, 1024 77.3 -> 59.3;  C=3072: B=1000 128.9 -> 105.7
 //   n=8 C=256: B=600 29.9 -> 23.3, 6000 113.4 -> 69.3;  C=512: B=2048 74.1 -> 55.0, 6000 181.0 -> 135.1;  n=5 C=384:
@@ -87,7 +89,9 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;
     if (n > 4) return true;
-    return B <= (C <= kResWholeMaxC ? 768 : 32 * n * n);
+    if (C <= 256) return B <= (C <= 128 ? 1536 : 768) * n;
+    const int per_row[4] = {640'000, 800'000, 1'040'000, 900'000};
+    return B <= std::min(960, std::max(n >= 3 ? 320 : 224, per_row[n - 1] / C));
 }
 
 // Shapes for which the dynamic entry points take fp32 activations that are consumed as bf16
