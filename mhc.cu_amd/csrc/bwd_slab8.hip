@@ -1,0 +1,459 @@
+// Slab backward for n = 5 .. 8 in the bf16 tier, behind the channel sums (gram_small_kernel): dx, df and the batch-split
+// partial sums of dphi, dw and dt in one pass over dy and x, as bwd_slab.hip does it for n <= 4:
+//
+//   dx[b,j,c]  = sum_i M_b[i,j] dy[b,i,c] + Hpre_b[j] da[b,c] - cx_b x[b,j,c] + sum_d dP[b,d] phi[d, jC+c]
+//   dphi[d,k] += sum_b dP[b,d] x_flat[b,k]            dw[c] += sum_b df[b,c] a[b,c] / q_b
+//   (reference stream_ops.cuh:761-850, :646-663, ops.py:319-351, rmsnorm.cuh:282-294)
+//
+// A workgroup owns 64 channels of every stream, walks the samples of its batch split 16 at a time and has a CU to
+// itself.  Everything goes from global memory straight into LDS, two tiles ahead; dP phi is formed transposed, so that
+// it stays with the lane that mixes the sample; dx replaces dy in LDS and leaves a tile later in whole 128-byte rows.
+// What differs from n <= 4 is what the registers hold: the projection has up to 96 rows here (80 at n = 8), so phi takes
+// 12 registers per stream and dphi 48 per 32 columns.  Four waves mix (phi in their registers, the rows of M fetched from
+// LDS one at a time), four others hold dphi and request the tiles; eight waves of 256 registers fill the CU.
+//
+// What bounds it: bytes (x, dy in, dx out) and the partial sums of dphi, 256 * 64 columns of every stream and D rows in
+// fp32 whatever the shape (42 MB at n = 8), written here and added up by the finalize launch.  n=8 B=2000 C=2560: 56 us for
+// 246 MB and the 42 MB of partial sums; the whole backward 182 us (resident path) -> 106, n=5 B=2000 C=1280 89 -> 54,
+// n=6 B=3000 C=768 79 -> 59.  One walk of the batch per 64 channels took the resident path's second launch 120 us there.
+#include "launchers.h"
+
+#include <algorithm>
+
+#include "lds_stage.h"
+#include "phase_profiler.h"
+#include "tuning.h"
+
+namespace mhc {
+
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
+
+struct BwdSlab8Args {
+    const bf16_t *dy, *x;    // [B, N, C]
+    const void *w;           // [C]
+    const bf16_t *phi;       // [D, N C]
+    const float *Hpre, *Hpost, *M, *q, *s1, *cx;  // per sample
+    const bf16_t *dPb, *dPT; // dP and dP^T hi / lo, fragment-major (frag_dpb, frag_dpt)
+    const float *dt;         // [B, D+3]
+    bf16_t *dx;              // [B, N, C]
+    bf16_t *df;              // [B, C] or nullptr
+    float *dphi_part;        // [S][D][N C]
+    double *dw_part;         // [S][C]
+    double *dt_part;         // [S slabs][D+3]
+    int w_bf16, B, BP, C, tiles;  // tiles of 16 samples; split y takes tiles [y T / S, (y + 1) T / S)
+};
+
+template <int N> struct Slab8Stage {
+    static constexpr int CW = 64, TB = 16, kMixers = 4, kHolders = 4;  // waves
+    static constexpr int D = N * N + 2 * N, NTD = (D + 31) / 32, DP = 32 * NTD;
+    static constexpr int kXRing = 3, kGRing = 4;                       // two tiles ahead
+    static constexpr int kTile = N * TB * CW * 2;                      // bytes of x or dy
+    // behind x: dP^T hi and lo of every 32 rows, dP of every 32 columns (1 KiB each), then blocks of 64 floats: M (a block
+    // per sample, rows of 8), Hpre and Hpost (8 samples a block, 8 floats each), cx | q | s1
+    static constexpr int kP = kTile, kPBlocks = 3 * NTD, kCoef = kP + kPBlocks * 1024, kCoefBlocks = TB + 2 + 2 + 3;
+    static constexpr int kXBytes = kCoef + kCoefBlocks * 256;
+    static constexpr int kG = kXRing * kXBytes, kW = kG + kGRing * kTile, kLds = kW + CW * 4;
+    static constexpr int kStreams = (N + 1) / 2;                       // KiB of x (and of dy) per holder
+    static constexpr int kShare = (kPBlocks + kCoefBlocks + kHolders - 1) / kHolders;
+    static constexpr int kCols = N * CW / 32, kAcc = (kCols + kHolders - 1) / kHolders;  // 32-column tiles of dphi, per holder
+    static_assert(32 * N * CW * 2 <= 2 * kTile && kLds <= 160 * 1024, "32 rows of phi fit two places of the dy ring");
+};
+
+template <int N, bool INJECT>
+__global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
+    using ST = Slab8Stage<N>;
+    constexpr int CW = ST::CW, TB = ST::TB, D = ST::D, NTD = ST::NTD;
+    constexpr int kChunks = CW / 8, kRows = 512 / CW;  // 16-byte chunks per row, rows per KiB
+    typedef __attribute__((address_space(3))) lds_tr_v4i16 *lds_tr_ptr;
+    extern __shared__ float smem_f[];
+    char *const smem = reinterpret_cast<char *>(smem_f);
+    const uint32_t smem_at = lds_address(smem);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int C = a.C, nC = N * C;
+    const int slab = blockIdx.x, slabs = gridDim.x, c0 = slab * CW;
+    const unsigned nsplit = gridDim.y;
+    const int b_begin = (int)((uint64_t)blockIdx.y * (unsigned)a.tiles / nsplit) * TB;
+    const int b_end = min(a.B, (int)((uint64_t)(blockIdx.y + 1) * (unsigned)a.tiles / nsplit) * TB);
+    const int T = (b_end - b_begin + TB - 1) / TB;
+    const int pwg = blockIdx.y * gridDim.x + blockIdx.x;
+    (void)pwg;
+    MHC_PHASE_ZERO(kPhaseBwdSlab, pwg);
+    MHC_PHASE_BEGIN(pclk);
+    const bool holder = wave >= ST::kMixers;
+    const int hw = wave - ST::kMixers;  // holder index
+
+    const auto lane_row = [&](int row0) { return row0 + lane / kChunks; };
+    const auto lane_col = [&](int row) { return c0 + ((lane % kChunks) ^ slab_swizzle<CW>(row)) * 8; };
+
+    // ---- loads of a tile (holders) -------------------------------------------------------------------
+    // holder h brings eight rows (h % 2) of the streams h / 2, h / 2 + 2 .. (the last one twice where they do not come out
+    // even: every holder has the same number of instructions in flight) and its share of the blocks behind x
+    const int ld_row = lane_row((hw & 1) * kRows), ld_col = min(lane_col(ld_row), C - 8);
+    auto load_tile = [&](const bf16_t *src, int t, uint32_t dst) {
+        const int sb = b_begin + t * TB;
+        const bf16_t *base = src + (size_t)sb * nC;
+        // slots beyond the batch alias its last sample, columns beyond C the last ones: they only meet zero columns of
+        // dP^T or land in rows and columns that are not stored
+        const uint32_t off = (uint32_t)(min(ld_row, b_end - sb - 1) * nC + ld_col) * 2;
+#pragma unroll
+        for (int i = 0; i < ST::kStreams; i++) {
+            const int j = min((hw >> 1) + 2 * i, N - 1);
+            load_to_lds<16>(base + (size_t)j * C, off, dst + (j * TB + (hw & 1) * kRows) * CW * 2);
+        }
+    };
+    struct Block {
+        const char *src;          // for the first sample of the batch
+        uint32_t step, at, dst;   // bytes per sample; this lane's bytes behind the tile's first; place behind the tile's x
+        bool wide;                // a KiB of dP operands; otherwise 64 floats of the coefficients
+    };
+    auto block_of = [&](int k) {
+        k = min(k, ST::kPBlocks + ST::kCoefBlocks - 1);
+        const size_t plane = (size_t)ST::DP * a.BP;
+        if (k < 2 * NTD)  // rows 32 (k / 2) ..: value (k even) or remainder
+            return Block{reinterpret_cast<const char *>(a.dPT + (k & 1) * plane + frag_base(k >> 1, a.BP >> 4, 0)), 64u, lane * 16u,
+                         ST::kP + k * 1024u, true};
+        if (k < ST::kPBlocks) {  // columns 32 kk ..: [d / 8][16 samples][8] out of the fragments of 32 samples
+            const int kk = k - 2 * NTD;
+            return Block{reinterpret_cast<const char *>(a.dPb + frag_base(0, ST::DP >> 4, 2 * kk)), ST::DP * 2u,
+                         (lane >> 5) * 1024u + ((lane >> 4) & 1) * 512u + (lane & 15) * 16u, ST::kP + k * 1024u, true};
+        }
+        const int s = k - ST::kPBlocks;
+        const uint32_t dst = ST::kCoef + s * 256u;
+        if (s < TB) {
+            // sample s: element (i, j) of M at (8 i + j + 4 s) mod 64, so that sixteen samples' rows lie in different banks
+            const int e = (lane - 4 * s) & 63, i = min(e >> 3, N - 1), j = min(e & 7, N - 1);
+            return Block{reinterpret_cast<const char *>(a.M), N * N * 4u, (uint32_t)(s * N * N + i * N + j) * 4u, dst, false};
+        }
+        const int v = s - TB;
+        if (v < 4) {
+            const int row = (v & 1) * 8 + (lane >> 3);
+            return Block{reinterpret_cast<const char *>(v < 2 ? a.Hpre : a.Hpost), N * 4u, (uint32_t)(row * N + min(lane & 7, N - 1)) * 4u, dst, false};
+        }
+        return Block{reinterpret_cast<const char *>(INJECT || v == 4 ? a.cx : (v == 5 ? a.q : a.s1)), 4u, (lane & 15) * 4u, dst, false};
+    };
+    auto load_all = [&](int t, const Block (&mine)[ST::kShare]) {
+        const uint32_t st = smem_at + t % ST::kXRing * ST::kXBytes;
+        const int sb = b_begin + t * TB;
+        const uint32_t left = min(b_end - sb, TB);
+        load_tile(a.x, t, st);
+#pragma unroll
+        for (int i = 0; i < ST::kShare; i++) {
+            const Block &m = mine[i];
+            if (m.wide) {  // (the second half of a 32-sample fragment of dP lies 256 bytes behind the first)
+                const bool half = m.dst >= ST::kP + 2 * NTD * 1024u && (sb & 16);
+                load_to_lds<16>(m.src + (size_t)(half ? sb - 16 : sb) * m.step + (half ? 256 : 0), m.at, st + m.dst);
+            } else {
+                // slots beyond the batch: the last float of the batch, whatever it is
+                load_to_lds<4>(m.src + (size_t)sb * m.step, min(m.at, left * m.step - 4), st + m.dst);
+            }
+        }
+        load_tile(a.dy, t, smem_at + ST::kG + t % ST::kGRing * ST::kTile);
+    };
+
+    // ---- prologue: the first tiles requested; phi -> LDS, 32 rows at a time, row-major [32 d][N][CW] -> the mixers' fragments
+    if (holder) {
+        Block mine[ST::kShare];
+#pragma unroll
+        for (int i = 0; i < ST::kShare; i++) mine[i] = block_of(hw + i * ST::kHolders);
+        load_all(0, mine);
+        if (T > 1) load_all(1, mine);
+    }
+    char *const phi_s = smem + ST::kG + 2 * ST::kTile;
+    if (tid < CW)
+        reinterpret_cast<float *>(smem + ST::kW)[tid] =
+            (c0 + tid < C && !INJECT) ? (a.w_bf16 ? bf16_to_f32(static_cast<const bf16_t *>(a.w)[c0 + tid])
+                                                  : static_cast<const float *>(a.w)[c0 + tid]) : 0.f;
+    // mixer lane (l16, kq): the four channels from c0 + cl of sample l16
+    const int l16 = lane & 15, kq = lane >> 4, cl = 16 * (wave & 3) + 4 * kq;
+    bf16x8_t phif[N][NTD];  // mixers: A operand, rows = this wave's 16 channels of a stream, contraction over 32 d
+#pragma unroll
+    for (int kk = 0; kk < NTD; kk++) {
+        constexpr int kPhiIters = (N * 32 * kChunks + 511) / 512;
+        uint4 phir[kPhiIters];
+#pragma unroll
+        for (int i = 0; i < kPhiIters; i++) {
+            const int e = tid + i * 512;
+            const int d = 32 * kk + e / (N * kChunks), j = e / kChunks % N, c = c0 + e % kChunks * 8;
+            const bool ok = e < N * 32 * kChunks && d < D && c < C;
+            phir[i] = load16_masked(reinterpret_cast<const uint4 *>(a.phi + (ok ? (size_t)d * nC + (size_t)j * C + c : 0)), ok);
+        }
+        __syncthreads();  // the rows before have been read
+#pragma unroll
+        for (int i = 0; i < kPhiIters; i++)
+            if (tid + i * 512 < N * 32 * kChunks) *reinterpret_cast<uint4 *>(phi_s + (tid + i * 512) * 16) = phir[i];
+        __syncthreads();
+        if (!holder) {
+            const int q = lane & 3, jj = (lane >> 2) & 3;
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                const char *p = phi_s + ((kq * 8 + jj) * N + j) * CW * 2 + (16 * wave + 4 * q) * 2;
+                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)p));
+                const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(p + 4 * N * CW * 2)));
+                phif[j][kk] = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+            }
+        }
+    }
+    __syncthreads();  // the places that held phi may be filled
+
+    float *const red_w = smem_f;                                                       // at the end: [16][CW + 1]
+    double *const red_dt = reinterpret_cast<double *>(smem + 16 * (CW + 2) * 4);       // and [mixers][128]
+    if (holder) {
+        // ---- requests the tiles, accumulates dphi: 32-column tiles hw, hw + 4 .. (stream, channel half) ----------
+        Block mine[ST::kShare];  // (formed again: kept across the prologue they spill)
+#pragma unroll
+        for (int i = 0; i < ST::kShare; i++) {
+            int k = hw + i * ST::kHolders;
+            asm volatile("" : "+s"(k));
+            mine[i] = block_of(k);
+        }
+        f32x16_t acc[ST::kAcc][NTD];
+#pragma unroll
+        for (int k = 0; k < ST::kAcc; k++)
+#pragma unroll
+            for (int m = 0; m < NTD; m++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[k][m][i] = 0.f;
+        // transposed reads of x: this lane's row (lo; hi: + 4) and its 8 bytes of the 32-channel group
+        const int q = lane & 3, row = (lane >> 5) * 8 + ((lane >> 2) & 3), ch = 4 * (hw & 1) + ((lane >> 4) & 1) * 2 + (q >> 1);
+        const int at_lo = row * CW * 2 + (ch ^ slab_swizzle<CW>(row)) * 16 + (q & 1) * 8;
+        const int at_hi = (row + 4) * CW * 2 + (ch ^ slab_swizzle<CW>(row + 4)) * 16 + (q & 1) * 8;
+        for (int p = 0; p < T; p++) {
+            // tile p has landed: all but the next tile's instructions; for everybody behind the barrier, where everybody is
+            // done with x of tile p - 1 and with dx of tile p - 2 as well, whose places tile p + 2 takes
+            if (p + 1 < T) wait_vmem<2 * ST::kStreams + ST::kShare>();
+            else wait_vmem<0>();
+            stage_barrier();
+            if (p + 2 < T) load_all(p + 2, mine);
+            const char *st = smem + p % ST::kXRing * ST::kXBytes;
+            bf16x8_t xf[ST::kAcc];
+#pragma unroll
+            for (int k = 0; k < ST::kAcc; k++) {
+                const int tile = min(hw + 4 * k, ST::kCols - 1);  // (both have the channel half hw & 1: kCols is even)
+                const char *xs = st + (tile >> 1) * TB * CW * 2;
+                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(xs + at_lo)));
+                const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(xs + at_hi)));
+                xf[k] = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+            }
+#pragma unroll
+            for (int m = 0; m < NTD; m++) {
+                const bf16x8_t ah = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + 2 * m * 1024 + lane * 16);
+                const bf16x8_t al = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + (2 * m + 1) * 1024 + lane * 16);
+#pragma unroll
+                for (int k = 0; k < ST::kAcc; k++) {
+                    acc[k][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, xf[k], acc[k][m], 0, 0, 0);
+                    acc[k][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, xf[k], acc[k][m], 0, 0, 0);
+                }
+            }
+        }
+        stage_barrier();  // the mixers' last dx
+        float *dphi_out = a.dphi_part + (size_t)blockIdx.y * D * nC;
+#pragma unroll
+        for (int k = 0; k < ST::kAcc; k++) {
+            const int tile = hw + 4 * k, c = c0 + (tile & 1) * 32 + (lane & 31);
+            if (tile < ST::kCols && c < C) {
+#pragma unroll
+                for (int m = 0; m < NTD; m++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const int d = 32 * m + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                        if (d < D) dphi_out[(size_t)d * nC + (size_t)(tile >> 1) * C + c] = acc[k][m][i];
+                    }
+            }
+        }
+        __syncthreads();
+        __syncthreads();
+    } else {
+        // ---- forms dx, stores the tile before ---------------------------------------------------------------------
+        const float4 w4 = *reinterpret_cast<const float4 *>(smem + ST::kW + cl * 4);
+        const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
+        const float inv_c = 1.0f / (float)C;
+        float usum[4] = {0.f, 0.f, 0.f, 0.f};
+        double dtsum[2] = {0.0, 0.0};  // columns lane, lane + 64 of dt
+        const int row_at = l16 * CW * 2 + (((cl >> 3) ^ slab_swizzle<CW>(l16)) * 16) + (kq & 1) * 8;  // this lane's 8 bytes of its sample's row
+        constexpr int kPieces = N * TB / kRows, kOut = (kPieces + ST::kMixers - 1) / ST::kMixers;
+        auto store_dx = [&](int t) {
+            const int sb = b_begin + t * TB;
+            const char *g = smem + ST::kG + t % ST::kGRing * ST::kTile;
+#pragma unroll
+            for (int i = 0; i < kOut; i++) {
+                const int at = wave + i * ST::kMixers, piece = min(at, kPieces - 1), j = piece / (TB / kRows);
+                const int row = lane_row(piece % (TB / kRows) * kRows), c = lane_col(row);
+                const uint4 v = *reinterpret_cast<const uint4 *>(g + piece * 1024 + lane * 16);
+                if (at < kPieces && sb + row < b_end && c < C)  // C % 8 == 0: eight channels are inside or outside
+                    st16<true>(a.dx + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+            }
+        };
+        for (int t = 0; t < T; t++) {
+            const char *st = smem + t % ST::kXRing * ST::kXBytes;
+            char *const gs = smem + ST::kG + t % ST::kGRing * ST::kTile;
+            const int sb = b_begin + t * TB;
+            const float *co = reinterpret_cast<const float *>(st + ST::kCoef);
+            MHC_PHASE_ADD(kPhaseBwdSlab, pwg, t > 0 ? 2 : 0, pclk);
+            stage_barrier();
+            MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 1, pclk);
+            if (t > 0) store_dx(t - 1);
+            // dt is summed by the slabs in turn: this tile's rows by slab t % slabs, four rows per mixer
+            const bool my_dt = t % slabs == slab;
+            float dtv[4][2];
+            if (my_dt) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int b = min(sb + 4 * wave + r, b_end - 1);
+                    const float *p = a.dt + (size_t)b * (D + 3);
+                    dtv[r][0] = p[min(lane, D + 2)];
+                    dtv[r][1] = p[min(lane + 64, D + 2)];
+                }
+            }
+            // projection term: columns = samples, rows = this lane's channels
+            f32x4_t o[N];
+            {
+                bf16x8_t pf[NTD];
+#pragma unroll
+                for (int kk = 0; kk < NTD; kk++) pf[kk] = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + (2 * NTD + kk) * 1024 + lane * 16);
+#pragma unroll
+                for (int j = 0; j < N; j++) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(phif[j][0], pf[0], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int kk = 1; kk < NTD; kk++)
+#pragma unroll
+                    for (int j = 0; j < N; j++) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(phif[j][kk], pf[kk], o[j], 0, 0, 0);
+            }
+            float hpre[8], hpost[8];
+            lds_floats<8>(co + (TB + (l16 >> 3)) * 64 + (l16 & 7) * 8, hpre);
+            lds_floats<8>(co + (TB + 2 + (l16 >> 3)) * 64 + (l16 & 7) * 8, hpost);
+            const float *sc = co + (TB + 4) * 64 + l16;
+            const float cxv = sc[0];
+            float qinv = 0.f, k2 = 0.f;
+            if constexpr (!INJECT) {
+                qinv = 1.0f / sc[64];
+                k2 = sc[128] * qinv * qinv * qinv * inv_c;
+                qinv = sb + l16 < b_end ? qinv : 0.f;  // a slot beyond the batch adds nothing to usum
+            }
+            // streams of dy one after the other: df, and the rows of M^T dy added into the accumulators
+            float s_df[4] = {0.f, 0.f, 0.f, 0.f};
+            const float *Mb = co + l16 * 64;
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                const uint2 g = *reinterpret_cast<const uint2 *>(gs + i * TB * CW * 2 + row_at);
+                const float gv[4] = {bf16lo_to_f32(g.x), bf16hi_to_f32(g.x), bf16lo_to_f32(g.y), bf16hi_to_f32(g.y)};
+                const float4 m0 = *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 * l16) & 63));
+                const float4 m1 = *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 + 4 * l16) & 63));
+                const float mr[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    s_df[c] += hpost[i] * gv[c];
+#pragma unroll
+                    for (int j = 0; j < N; j++) o[j][c] += mr[j] * gv[c];
+                }
+            }
+            uint2 xr[N];
+            float s_a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * CW * 2 + row_at);
+                s_a[0] += hpre[j] * bf16lo_to_f32(xr[j].x); s_a[1] += hpre[j] * bf16hi_to_f32(xr[j].x);
+                s_a[2] += hpre[j] * bf16lo_to_f32(xr[j].y); s_a[3] += hpre[j] * bf16hi_to_f32(xr[j].y);
+            }
+            float da[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float dq = s_df[c] * qinv;
+                da[c] = INJECT ? 0.f : dq * wv[c] - s_a[c] * k2;
+                if constexpr (!INJECT) usum[c] += dq * s_a[c];
+            }
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                const float xv[4] = {bf16lo_to_f32(xr[j].x), bf16hi_to_f32(xr[j].x), bf16lo_to_f32(xr[j].y), bf16hi_to_f32(xr[j].y)};
+                float r[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) r[c] = o[j][c] + hpre[j] * da[c] - cxv * xv[c];
+                *reinterpret_cast<uint2 *>(gs + j * TB * CW * 2 + row_at) = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
+            }
+            if (my_dt) {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (sb + 4 * wave + r < b_end) { dtsum[0] += dtv[r][0]; dtsum[1] += dtv[r][1]; }
+            }
+            if (INJECT && a.df && sb + l16 < b_end && c0 + cl < C)
+                store_vec<bf16_t, 4>(a.df + (size_t)sb * C + (uint32_t)(l16 * C + c0 + cl), s_df);
+        }
+        MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 2, pclk);
+        stage_barrier();
+        store_dx(T - 1);
+        // vmcnt(0), for the compiler: it sees the loads of dt above as pending on every path out of here, and would wait for
+        // them - and with them for all that the holders have requested - in the holders' loop
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 3, pclk);
+        __syncthreads();  // everyone is done with the rings
+        if constexpr (!INJECT) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) red_w[l16 * (CW + 1) + cl + v] = usum[v];
+        }
+        red_dt[wave * 128 + lane] = dtsum[0];
+        red_dt[wave * 128 + 64 + lane] = dtsum[1];
+        __syncthreads();
+    }
+
+    // ---- small outputs of the split -------------------------------------------------------------------
+    if (!INJECT && tid < CW && c0 + tid < C) {
+        double s = 0.0;
+#pragma unroll
+        for (int r = 0; r < 16; r++) s += red_w[r * (CW + 1) + tid];
+        a.dw_part[(size_t)blockIdx.y * C + c0 + tid] = s;
+    }
+    if (tid < D + 3) {
+        double s = 0.0;
+#pragma unroll
+        for (int r = 0; r < ST::kMixers; r++) s += red_dt[r * 128 + tid];
+        a.dt_part[((size_t)blockIdx.y * slabs + slab) * (D + 3) + tid] = s;
+    }
+    MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 4, pclk);
+}
+
+bool bwd_slab8_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) {
+    return x_dtype == kBF16 && y_dtype == kBF16 && phi_dtype == kBF16 && n >= 5 && n <= 8 && C % 8 == 0;
+}
+
+int bwd_slab8_slabs(int C) { return (C + 63) / 64; }
+
+int bwd_slab8_batch_splits(int B, int C) {
+    const int slabs = bwd_slab8_slabs(C), tiles = (B - 1) / 16 + 1;
+    int S = tuning_get(kTuneSlabSplits);  // experiment hook
+    // one workgroup per CU, but at least three tiles each: a workgroup leaves its partial dphi behind however short its walk
+    // (backward us: B=2000 n=8 C=256 two tiles 50.3, three 47.3, four 47.1, seven 51.4)
+    if (S <= 0) S = std::max(1, std::min(256 / slabs, tiles / 3));
+    if (S > tiles) S = tiles;
+    // the longest split decides: the fewest splits that keep its tile count
+    const int tps = (tiles + S - 1) / S;
+    return (tiles + tps - 1) / tps;
+}
+
+hipError_t launch_bwd_slab8(const void *dy, const void *x, const void *w, int w_dtype, const void *f_inject, const void *phi,
+                            const float *Hpre, const float *Hpost, const float *M, const float *q, const BwdCoefOut &co,
+                            void *dx, void *df, float *dphi_part, double *dw_part, double *dt_part, int S, int B, int n, int C,
+                            hipStream_t stream) {
+    const int tiles = (B - 1) / 16 + 1;
+    if (S < 1 || S > tiles) return hipErrorInvalidValue;
+    const BwdSlab8Args a{static_cast<const bf16_t *>(dy), static_cast<const bf16_t *>(x), w, static_cast<const bf16_t *>(phi),
+                         Hpre, Hpost, M, q, co.s1, co.cx, co.dPb, co.dPT, co.dt, static_cast<bf16_t *>(dx),
+                         static_cast<bf16_t *>(df), dphi_part, dw_part, dt_part, w_dtype == kBF16, B, co.BP, C, tiles};
+    const dim3 grid(bwd_slab8_slabs(C), S);
+#define MHC_SLAB8(N, INJ)                                                                                     \
+    do {                                                                                                      \
+        constexpr size_t lds = Slab8Stage<N>::kLds;                                                           \
+        if (hipError_t e = allow_dynamic_lds<&bwd_slab8_kernel<N, INJ>>(lds); e != hipSuccess) return e;      \
+        bwd_slab8_kernel<N, INJ><<<grid, 512, lds, stream>>>(a);                                              \
+    } while (0)
+#define MHC_SLAB8_N(N) do { if (f_inject) MHC_SLAB8(N, true); else MHC_SLAB8(N, false); } while (0)
+    switch (n) {
+        case 5: MHC_SLAB8_N(5); break;
+        case 6: MHC_SLAB8_N(6); break;
+        case 7: MHC_SLAB8_N(7); break;
+        default: MHC_SLAB8_N(8); break;
+    }
+#undef MHC_SLAB8_N
+#undef MHC_SLAB8
+    return hipGetLastError();
+}
+
+}  // namespace mhc

@@ -81,14 +81,24 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 //   n=1 C=256:  B=768 15.8 | 15.1, 1024 17.2 | 18.0;  C=960: 576 16.3 | 16.1, 768 16.5 | 17.4;  C=3200: 192 16.1 | 13.9, 384 17.9 | 21.6
 // The tiled path is one launch more, so the lines lie a little above the crossings: about 1.0 M / C samples, within bounds,
 // and 768 n samples of at most 256 channels (n=4 C=128: B=4096 31.9 | 27.1, 6000 35.0 | 33.9).
-// n = 5 .. 8 at every batch size:
-//   n=8 C=1280: B=128 25.1 -> 16.0, 256 30.5 -> 21.2, 512 46.1 -> 34.1, 1024 77.3 -> 59.3;  C=3072: B=1000 128.9 -> 105.7
-//   n=8 C=256: B=600 29.9 -> 23.3, 6000 113.4 -> 69.3;  C=512: B=2048 74.1 -> 55.0, 6000 181.0 -> 135.1;  n=5 C=384:
-//               B=3000 86.1 -> 57.9
+// n = 5 .. 8, where the slab is bwd_slab8.hip (n=8 C=2560 B=2000: 106 | 182):
+//   n=5 C=256:  B=1024 27.1 | 28.2, 1536 32.5 | 30.2, 4000 53.7 | 47.8;  C=320: 768 24.8 | 27.7;  C=640: 512 24.1 | 21.2,
+//               768 26.5 | 30.0;  C=1280: 384 26.4 | 26.1, 512 27.0 | 28.0;  C=2560: 256 29.4 | 24.4, 384 32.1 | 35.4
+//   n=6 C=320:  B=768 27.6 | 28.5, 1100 36.7 | 39.0;  C=384: 512 25.9 | 19.4;  C=512: 768 29.3 | 29.1, 1100 36.9 | 40.2;
+//               C=1280: 512 30.8 | 28.6, 1024 41.6 | 49.0;  C=2560: 256 33.3 | 25.6, 512 39.1 | 39.8
+//   n=7 C=384:  B=768 31.6 | 29.9, 1100 38.5 | 39.7;  C=512: 768 31.2 | 29.5, 1100 39.7 | 40.4;  C=1280: 512 34.7 | 31.0,
+//               1024 46.4 | 53.3;  C=2560: 256 38.4 | 29.5, 512 44.5 | 48.3
+//   n=8 C=256:  B=1536 40.2 | 30.0, 6000 82.8 | 68.9;  C=320: 3000 60.6 | 58.7, 4500 75.9 | 81.4;  C=512: 2048 54.9 | 54.5,
+//               3000 65.7 | 74.9;  C=1280: 512 39.5 | 34.0, 768 47.0 | 46.7, 1024 52.6 | 59.5;  C=2560: 384 48.9 | 44.7,
+//               512 51.8 | 52.4;  C=4096: 384 62.2 | 60.4, 512 66.8 | 68.5
 // Experiment hook: 1 = never, 2 = always.
 bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;
-    if (n > 4) return true;
+    if (n > 4) {
+        if (C <= 256) return true;
+        const int per_row[4] = {500'000, 740'000, 880'000, 1'020'000}, least[4] = {320, 448, 448, 480}, most[4] = {704, 896, 1024, 4096};
+        return B <= std::min(most[n - 5], std::max(least[n - 5], per_row[n - 5] / C));
+    }
     if (C <= 256) return B <= (C <= 128 ? 1536 : 768) * n;
     const int per_row[4] = {640'000, 800'000, 1'040'000, 900'000};
     return B <= std::min(960, std::max(n >= 3 ? 320 : 224, per_row[n - 1] / C));
@@ -143,21 +153,24 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     // backward's second launch with a split batch
     const int bs3 = n <= 4 ? std::max(bwd_slab_batch_splits(B, n, C, kBF16), bwd_slab_batch_splits(B, n, C, kF32)) : 1;
     const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1, bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
-    const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : 0, parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
-    w.u = c.floats(std::max((size_t)B, 2 * slab64) * C);
+    const int bs7 = n >= 5 && n <= 8 ? bwd_slab8_batch_splits(B, C) : 1;
+    const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : (n <= 8 ? (size_t)bs7 * bwd_slab8_slabs(C) : 0), parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
+    w.u = c.floats(std::max((size_t)B, 2 * (n <= 4 ? slab64 : (size_t)bs7)) * C);
     w.upart = c.floats(2 * parts64 * C);
     w.dtpart = c.floats(std::max((size_t)B, 2 * std::max(slab64, parts64)) * (D + 3));
     w.raw = c.floats(bwd_reduce_raw_floats(B, n, C));
     w.s1part = c.floats(n > 8 ? (size_t)B * bwd_reduce_parts(B, n, C) : 0);
     // wide projections: the part of dx that is formed beside the coefficient backward, fp32
     w.dx_part = c.floats(wide_dx_beside(B, n, C) ? (size_t)B * nC : 0);
-    // n <= 8, sample-resident backward: dxp where it is handed over in fp32
-    const bool resident = n <= 8 && C <= kResMaxC && (bwd_resident_preferred(B, n, C) || C % 8 != 0);
+    // n <= 8, sample-resident backward: dxp where it is handed over in fp32 (n = 5 .. 8: on either side of the line, for
+    // the experiment hook)
+    const bool resident = n <= 8 && C <= kResMaxC && (n > 4 || bwd_resident_preferred(B, n, C) || C % 8 != 0);
     w.dxp = c.floats(resident && bwd_resident_dxp_f32(n, C) ? (size_t)B * nC : 0);
     int bs = dphi_batch_splits(B, n, C);
     const int bs2 = proj_bwd_batch_splits(B, n, C);
     if (bs2 > bs) bs = bs2;
     if (bs3 > bs) bs = bs3;
+    if (bs7 > bs) bs = bs7;
     const int bs4 = dphi_f32_splits(B, n, C);
     if (bs4 > bs) bs = bs4;
     if (bs5 > bs) bs = bs5;
@@ -704,6 +717,15 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
                                    S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
                                    reinterpret_cast<double *>(ws.dtpart), S, B, n, C, st));
         MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S, D, dbias, dalpha,
+                                   ws.dphi_part, S, (size_t)D * n * C, dphi, st, true));
+        return MHC_OK;
+    }
+    if (mfma && bwd_slab8_supported(x_dtype, y_dtype, phi_dtype, n, C) && tuning_get(kTuneSlab8) != 1) {
+        const int S = bwd_slab8_batch_splits(B, C);
+        MHC_LAUNCH(launch_bwd_slab8(dy, x, w, w_dtype, f_inject, phi, H_pre, H_post, M, q, out, dx, df,
+                                    S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
+                                    reinterpret_cast<double *>(ws.dtpart), S, B, n, C, st));
+        MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S * bwd_slab8_slabs(C), D, dbias, dalpha,
                                    ws.dphi_part, S, (size_t)D * n * C, dphi, st, true));
         return MHC_OK;
     }

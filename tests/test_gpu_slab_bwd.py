@@ -1,13 +1,14 @@
 """The tiled backward of n <= 4.  The slab kernel (csrc/bwd_slab.hip): both channel widths at the edges of its tiles (16 samples, 64 / 128
 channels), of its ring of tiles in flight (1 .. 5 tiles per batch split) and of its splits, against the oracle and
 each other.  The channel sums with the coefficient backward of several samples per workgroup (gram_quad_kernel,
-csrc/mix_bwd_reduce.hip): against the two launches.  Reference backward: src/python/mhc/ops.py:276-361."""
+csrc/mix_bwd_reduce.hip): against the two launches.  The slab
+kernel of five to eight streams: against the general kernels.  Reference backward: src/python/mhc/ops.py:276-361."""
 import pytest
 
 from test_gpu_resident_bwd import K_RESIDENT, _both_paths
 
 pytestmark = pytest.mark.gpu
-K_GRAM, K_SLAB_SPLITS, K_SLAB_WIDTH = 2, 3, 11
+K_GRAM, K_SLAB_SPLITS, K_SLAB_WIDTH, K_SLAB8 = 2, 3, 11, 12
 
 # (B, n, C, splits; 0 = as the library chooses)
 SHAPES = [(1, 4, 8, 0), (16, 4, 128, 1), (17, 4, 136, 1), (33, 3, 64, 1), (50, 4, 72, 1), (65, 2, 200, 1), (80, 1, 40, 1),
@@ -41,3 +42,19 @@ def test_channel_sums_of_several_samples_per_workgroup(B, n, C, inject, w_f32):
         _both_paths(K_GRAM, ("two launches", "several samples"), B, n, C, inject, w_f32)
     finally:
         lib.mhc_tuning_set(K_RESIDENT, 0)
+
+
+# n = 5 .. 8 (csrc/bwd_slab8.hip): one to four tiles of 16 samples per split, cut tiles, channels beyond the row, several slabs
+@pytest.mark.parametrize("B,n,C,splits", [(1, 5, 8, 1), (16, 8, 64, 1), (17, 8, 72, 1), (33, 6, 136, 1), (50, 7, 64, 1), (49, 8, 200, 2),
+                                          (130, 5, 264, 3), (65, 7, 320, 0), (200, 8, 1280, 0), (300, 6, 1928, 0)])
+@pytest.mark.parametrize("inject,w_f32", [(False, False), (False, True), (True, False)])
+def test_slab_backward_of_five_to_eight_streams(B, n, C, splits, inject, w_f32):
+    from mhc._lib import tuning_lib
+
+    lib = tuning_lib()
+    try:
+        assert lib.mhc_tuning_set(K_RESIDENT, 1) == 0 and lib.mhc_tuning_set(K_SLAB_SPLITS, splits) == 0
+        _both_paths(K_SLAB8, ("general kernels", "slab"), B, n, C, inject, w_f32)
+    finally:
+        lib.mhc_tuning_set(K_RESIDENT, 0)
+        lib.mhc_tuning_set(K_SLAB_SPLITS, 0)
