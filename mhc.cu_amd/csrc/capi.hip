@@ -202,9 +202,10 @@ StaBwdWs carve_sta_bwd(void *ws, int B, int n, int C) {
     Carver c(ws);
     const int D = n * n + 2 * n;
     StaBwdWs w;
-    w.red = c.floats((size_t)B * (D + 3));
+    // a row per sample in float32, or (n <= 8) one of at least two samples in float64: (B + 1) / 2 rows at most
+    w.red = c.floats(((size_t)B + 1) * (D + 3));
     w.s1 = c.floats(B);
-    w.u = c.floats((size_t)B * C);
+    w.u = c.floats(((size_t)B + 1) * C);
     w.red_sum = c.floats(D + 3);
     w.raw = c.floats(n > 8 ? bwd_reduce_raw_floats(B, n, C) : 0);
     w.sk = c.floats(n > 8 ? (size_t)(2 * max_layer_sinkhorn_iters(n) + 2) * 32 : 0);
@@ -819,12 +820,15 @@ int bwd_static(const void *dy, int y_dtype, const void *x, int x_dtype, const vo
     BwdCoefOut out{nullptr, nullptr, nullptr, ws.s1, ws.red, nullptr, nullptr, 0};
     if (bwd_resident_supported(x_dtype, y_dtype, kBF16, n, C, 0) && tuning_get(kTuneResident) != 1) {
         // bf16 activations, n <= 8: with shared coefficients nothing of dx depends on a batch-wide
-        // result, so ONE pass over dy and x (a workgroup keeps its sample's rows in registers) forms
-        // the channel sums, the sample's raw coefficient gradients and the complete dx
-        MHC_LAUNCH(launch_bwd_resident_static(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, q, out, dx, df, ws.u,
-                                              B, n, C, st));
-        MHC_LAUNCH(launch_finalize_static(ws.u, B, C, f_inject ? DwOut{} : dw, ws.red, B, ws.red_sum, H_pre, H_post,
-                                          H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st));
+        // result, so ONE pass over dy and x (a workgroup keeps a sample's rows in registers) forms
+        // the channel sums, the raw coefficient gradients and the complete dx; large batches several samples per workgroup
+        const bool walk = bwd_static_preferred(B, n, C);
+        const int rows = walk ? bwd_static_rows(B, n, C) : B;
+        if (walk) MHC_LAUNCH(launch_bwd_static(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, q, dx, df, ws.u, ws.red, B, n, C, st));
+        else MHC_LAUNCH(launch_bwd_resident_static(dy, x, w, w_dtype, f_inject, H_pre, H_post, M, q, out, dx, df, ws.u,
+                                                   B, n, C, st));
+        MHC_LAUNCH(launch_finalize_static(ws.u, rows, C, f_inject ? DwOut{} : dw, ws.red, rows, ws.red_sum, H_pre, H_post,
+                                          H_res_logits, dH_pre, dH_post, dH_res, n, iters, eps, st, nullptr, walk));
         return MHC_OK;
     }
     if (n > 16 && x_dtype == kBF16 && y_dtype == kBF16 && C % 8 == 0) {

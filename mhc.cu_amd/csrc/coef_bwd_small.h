@@ -181,6 +181,36 @@ template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = fals
         }
     }
 
+    // GRAM: the vectors that the coefficient gradients are made of, from this lane's entries of the Gram sums (fetch_sums);
+    // lane g < n gets entry g.  xch: kXch floats of LDS private to the group.
+    __device__ __forceinline__ void gram_vectors(int n, int g, float *xch, float &tpost, float &tA1, float &tA2, float &s1) const {
+        // lane (r0, c0) takes its element of each matrix and the mirrored element of W1, so that
+        // every sum below runs down a column:
+        //   dHpost[c] = sum_r Hpre[r] W1[c][r] / q        A1[c] = sum_r Hpost[r] W1[r][c]
+        //   A2[c] = sum_r Hpre[r] XX[r][c]                s1 = sum_c Hpost[c] (sum_r Hpre[r] W1[c][r])
+        // The column results are handed to lanes 0 .. n-1 through LDS (same wave: no barrier).
+        const float w1 = s_a, w1t = s_b, xx = s_c;
+        const float hr = r0 < n ? hpre_r : 0.f, hor = r0 < n ? hpost_r : 0.f;
+        // with an injected f, W1 = dy [f; 0; ...]^T and dHpost is its column 0
+        const float sel = inject ? (r0 == 0 ? 1.f : 0.f) : hr;
+        const float x0 = SK::col_allreduce(sel * w1t);
+        const float x1 = SK::col_allreduce(hor * w1);
+        const float x2 = SK::col_allreduce(hr * xx);
+        if (r0 == 0) { xch[c0] = x0; xch[NP + c0] = x1; xch[2 * NP + c0] = x2; }
+        const float hw = xch[gc];
+        if (inject) {
+            tpost = hw;
+        } else {
+            tpost = hw * qinv;
+            tA1 = xch[NP + gc];
+            tA2 = xch[2 * NP + gc];
+            s1 = SK::group_allreduce(g < n ? ho * hw : 0.f);
+        }
+    }
+    __device__ __forceinline__ float dhpre_of(float tA1, float tA2, float s1) const {
+        return inject ? 0.f : tA1 * qinv - s1 * tA2 * qinv * qinv * qinv * inv_c;
+    }
+
     // after fetch_sums() and forward_recompute(); xch: kXch floats of LDS private to the group
     __device__ __forceinline__ void run(const BwdReduceArgs &a, int b, int g, int lane, float *sc, float *xch) {
         const int n = a.n, D = n * n + 2 * n;
@@ -189,28 +219,7 @@ template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = fals
         MHC_PHASE_BEGIN(rclk);
         float tpost = 0.f, tA1 = 0.f, tA2 = 0.f, s1 = 0.f;
         if constexpr (GRAM) {
-            // lane (r0, c0) takes its element of each matrix and the mirrored element of W1, so that
-            // every sum below runs down a column:
-            //   dHpost[c] = sum_r Hpre[r] W1[c][r] / q        A1[c] = sum_r Hpost[r] W1[r][c]
-            //   A2[c] = sum_r Hpre[r] XX[r][c]                s1 = sum_c Hpost[c] (sum_r Hpre[r] W1[c][r])
-            // The column results are handed to lanes 0 .. n-1 through LDS (same wave: no barrier).
-            const float w1 = s_a, w1t = s_b, xx = s_c;
-            const float hr = r0 < n ? hpre_r : 0.f, hor = r0 < n ? hpost_r : 0.f;
-            // with an injected f, W1 = dy [f; 0; ...]^T and dHpost is its column 0
-            const float sel = inject ? (r0 == 0 ? 1.f : 0.f) : hr;
-            const float x0 = SK::col_allreduce(sel * w1t);
-            const float x1 = SK::col_allreduce(hor * w1);
-            const float x2 = SK::col_allreduce(hr * xx);
-            if (r0 == 0) { xch[c0] = x0; xch[NP + c0] = x1; xch[2 * NP + c0] = x2; }
-            const float hw = xch[gc];
-            if (inject) {
-                tpost = hw;
-            } else {
-                tpost = hw * qinv;
-                tA1 = xch[NP + gc];
-                tA2 = xch[2 * NP + gc];
-                s1 = SK::group_allreduce(g < n ? ho * hw : 0.f);
-            }
+            gram_vectors(n, g, xch, tpost, tA1, tA2, s1);
         } else {
             tpost = s_a; tA1 = s_b; tA2 = s_c; s1 = s_d;
         }
@@ -219,7 +228,7 @@ template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = fals
             float *red = a.out.red + (size_t)b * (D + 3);  // rows padded like dt, for the batch-sum launch
             if (mv) red[r0 * n + c0] = dMe;
             if (g < n) {
-                red[n * n + g] = inject ? 0.f : tA1 * qinv - s1 * tA2 * qinv * qinv * qinv * inv_c;
+                red[n * n + g] = dhpre_of(tA1, tA2, s1);
                 red[n * n + n + g] = tpost;
             }
             return;
@@ -229,7 +238,7 @@ template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = fals
         float S0 = 0.f, S1 = 0.f, S2 = 0.f;  // sum_d dt_d p_d per alpha group
         if (g < n) {
             const float dHpost = tpost;
-            const float dHpre = inject ? 0.f : tA1 * qinv - s1 * tA2 * qinv * qinv * qinv * inv_c;
+            const float dHpre = dhpre_of(tA1, tA2, s1);
             const float dtp = dHpre * hp * (1.0f - hp);
             const float dto = dHpost * ho * (1.0f - 0.5f * ho);
             dt[g] = dtp; dt[n + g] = dto;

@@ -259,6 +259,13 @@ hipError_t launch_bwd_resident_static(const void *dy, const void *x, const void 
                                       const float *Hpre, const float *Hpost, const float *M, const float *q,
                                       BwdCoefOut out, void *dx, void *df, float *u, int B, int n, int C,
                                       hipStream_t stream);
+// The same for large batches (bwd_static_preferred), where a workgroup walks several samples: u [rows][C] and red [rows][D + 3] (raw dM | dHpre | dHpost),
+// summed over a workgroup's samples in float64.
+bool bwd_static_preferred(int B, int n, int C);
+int bwd_static_rows(int B, int n, int C);
+hipError_t launch_bwd_static(const void *dy, const void *x, const void *w, int w_dtype, const void *f_inject, const float *Hpre,
+                             const float *Hpost, const float *M, const float *q, void *dx, void *df, void *u, void *red, int B, int n,
+                             int C, hipStream_t stream);
 // Second and last launch of that backward (D <= 96): a column slab for all samples per workgroup;
 // dphi = dP^T x_flat without batch split, dx completed in place (dx = dxp + dP phi - cx x), and `tail`
 // (dw, dbias, dalpha) summed by extra workgroups when the grid has room (*tail_taken).
@@ -301,10 +308,11 @@ hipError_t launch_colsum_split(const float *in, int rows, int cols, int ld, floa
 hipError_t launch_coef_bwd_static(const float *red_sum, const float *Hpre, const float *Hpost,
                                   const float *H_res_logits, float *dH_pre, float *dH_post,
                                   float *dH_res, int n, int T, float eps, hipStream_t stream, const float *state = nullptr);
-hipError_t launch_finalize_static(const float *u, int rows_u, int C, DwOut dw, const float *red, int rows,
+// rows64 (n <= 8): u and red are rows of float64.
+hipError_t launch_finalize_static(const void *u, int rows_u, int C, DwOut dw, const void *red, int rows,
                                   float *red_sum, const float *Hpre, const float *Hpost,
                                   const float *H_res_logits, float *dH_pre, float *dH_post, float *dH_res, int n,
-                                  int T, float eps, hipStream_t stream, const float *static_state = nullptr);
+                                  int T, float eps, hipStream_t stream, const float *static_state = nullptr, bool rows64 = false);
 
 // phi [D, nC] (out_dtype) = rows [pre | post | res] of the three parameter matrices (src_dtype),
 // bias [D] and alpha [3] likewise, in one launch.

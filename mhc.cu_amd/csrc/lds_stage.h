@@ -1,4 +1,4 @@
-// Pieces of the slab backward kernels (bwd_slab.hip, bwd_slab8.hip): loads from global memory straight into LDS, waits and
+// Pieces of the kernels that keep global memory busy across barriers (bwd_slab.hip, bwd_slab8.hip, bwd_static.hip): loads from global memory straight into LDS, waits and
 // barriers that count them, and the order of the chunks of a row there.
 #pragma once
 #include "mhc_common.h"

@@ -5,6 +5,8 @@
 #include "launchers.h"
 #include "sinkhorn_device.h"
 
+#include <type_traits>
+
 namespace mhc {
 
 // --------------------------------------------------------------------------------------------
@@ -286,7 +288,7 @@ hipError_t launch_coef_bwd_static(const float *red_sum, const float *Hpre, const
 //       never leave the workgroup.
 struct FinalizeStaticArgs {
     BatchSumArgs sums;  // u -> dw only
-    const float *red; int rows, n, T; float eps;
+    const void *red; int rows, n, T; float eps;  // rows of float64 where sums.rows64
     const float *Hpre, *Hpost, *H_res_logits;
     float *dH_pre, *dH_post, *dH_res;
 };
@@ -299,7 +301,7 @@ __global__ __launch_bounds__(1024) void finalize_static_kernel(FinalizeStaticArg
     extern __shared__ float sc[];  // SK::scaling_floats(T)
     const int tid = threadIdx.x;
     if ((int)blockIdx.x < a.sums.nblk) {
-        batch_sum_block<32, 32>(a.sums, blockIdx.x, tid, red);
+        batch_sum_block<32, 32, true>(a.sums, blockIdx.x, tid, red);
         return;
     }
     const int n = a.n, D = n * n + 2 * n, ld = D + 3;
@@ -317,14 +319,12 @@ __global__ __launch_bounds__(1024) void finalize_static_kernel(FinalizeStaticArg
         // `red` as one flat array: thread t of the 960 takes element t of every pass of RP whole rows, so a
         // pass is one contiguous piece of memory and a thread stays on its column
         const int t = tid - 64, RP = 896 / ld;  // ld <= 83: at least 10 rows per pass
-        if (t < RP * ld) {
-            const float *src = a.red + t;
+        auto column = [&](auto *src) {
             const size_t step = (size_t)RP * ld;
-            const int rs = t / ld;
             double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-            int r = rs;
+            int r = t / ld;
             for (; r + 15 * RP < a.rows; r += 16 * RP, src += 16 * step) {  // sixteen loads in flight
-                float v[16];
+                typename std::remove_const<typename std::remove_pointer<decltype(src)>::type>::type v[16];
 #pragma unroll
                 for (int k = 0; k < 16; k++) v[k] = src[k * step];
 #pragma unroll
@@ -333,8 +333,10 @@ __global__ __launch_bounds__(1024) void finalize_static_kernel(FinalizeStaticArg
                 }
             }
             for (; r < a.rows; r += RP, src += step) a0 += (double)*src;
-            red[t] = (a0 + a1) + (a2 + a3);  // [row slot][column]
-        }
+            return (a0 + a1) + (a2 + a3);
+        };
+        if (t < RP * ld)
+            red[t] = a.sums.rows64 ? column(static_cast<const double *>(a.red) + t) : column(static_cast<const float *>(a.red) + t);  // [row slot][column]
     }
     __syncthreads();
     if (tid >= 64 && tid < 64 + D) {
@@ -357,19 +359,20 @@ __global__ __launch_bounds__(1024) void finalize_static_kernel(FinalizeStaticArg
 
 // Batch sums + coefficient backward of the static path.  n <= 8: one launch (above); wider matrices: the
 // finalize launch writes the sums to red_sum [D + 3] and the workgroup-wide Sinkhorn kernel follows.
-hipError_t launch_finalize_static(const float *u, int rows_u, int C, DwOut dw, const float *red, int rows,
+hipError_t launch_finalize_static(const void *u, int rows_u, int C, DwOut dw, const void *red, int rows,
                                   float *red_sum, const float *Hpre, const float *Hpost,
                                   const float *H_res_logits, float *dH_pre, float *dH_post, float *dH_res, int n,
-                                  int T, float eps, hipStream_t stream, const float *static_state) {
+                                  int T, float eps, hipStream_t stream, const float *static_state, bool rows64) {
     const int D = n * n + 2 * n;
     if (n > 8) {
-        if (hipError_t e = launch_finalize(u, rows_u, C, dw, red, rows, D, red_sum, red_sum + D, nullptr, 1, 0,
+        if (rows64) return hipErrorInvalidValue;
+        if (hipError_t e = launch_finalize(static_cast<const float *>(u), rows_u, C, dw, static_cast<const float *>(red), rows, D, red_sum, red_sum + D, nullptr, 1, 0,
                                            nullptr, stream); e != hipSuccess)
             return e;
         return launch_coef_bwd_static(red_sum, Hpre, Hpost, H_res_logits, dH_pre, dH_post, dH_res, n, T, eps, stream,
                                       static_state);
     }
-    FinalizeStaticArgs a{make_batch_sums(u, rows_u, C, dw, nullptr, 0, 0, nullptr, nullptr), red, rows, n, T, eps,
+    FinalizeStaticArgs a{make_batch_sums(u, rows_u, C, dw, nullptr, 0, 0, nullptr, nullptr, rows64), red, rows, n, T, eps,
                          Hpre, Hpost, H_res_logits, dH_pre, dH_post, dH_res};
     a.sums.nblk = dw ? (C + 31) / 32 : 0;  // blocks of 32 columns
     if (n <= 4) {

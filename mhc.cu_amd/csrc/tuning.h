@@ -14,7 +14,7 @@ enum TuneKey {
     kTuneSlabSplits = 3,    // batch splits of the slab backward (n <= 4) and of the projection backward (n = 5 .. 18)
     kTuneSeparateFinalize = 4,  // 1 = batch sums always as a launch of their own, never inside the dphi launch
     kTuneProjApart = 5,     // n <= 18 projection backward: 1 = both products in one launch, 2 = two launches
-    kTuneStaticSpg = 6,     // static backward: samples per workgroup of the dx kernel (n <= 8)
+    kTuneStaticSpg = 6,     // static backward (n <= 8): samples per workgroup (bf16: 1 = the sample-resident kernel)
     kTuneResident = 7,      // n <= 8 sample-resident backward: 0 = by heuristic, 1 = never, 2 = whenever the shape allows
     kTuneWideDxBeside = 8,  // wide projections (n > 18): dx workgroups beside the coefficient launch: 1 = never, 2 = always
     kTuneSpareB = 9,        // projection forward (matrix-core kernels): K splits, 0 = by heuristic
