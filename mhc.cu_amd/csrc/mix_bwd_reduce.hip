@@ -231,8 +231,11 @@ __global__ __launch_bounds__(64) void coef_bwd_small_kernel(BwdReduceArgs a) {
 // and the launch of the coefficient kernel is saved.
 // STATIC (with FUSED): shared coefficients; the tail only converts the sums into the sample's row of raw
 // gradients (see CoefBwdSmall).
+// 128 registers, four workgroups per CU: their coefficient steps, serial chains on one wave each, hide behind each other (8 x 8 with
+// as many registers as it likes, 138, has three; backward us: n=8 B=2000 C=2560 102.9 -> 100.1, B=3000 C=512 65.3 -> 63.1, n=6
+// B=3000 C=768 57.6 -> 55.1, n=5 B=2000 C=1280 51.5 -> 49.6; five workgroups spill: 122.7, 76.9).
 template <int NP, int WMODE, bool FUSED, bool STATIC = false>
-__global__ __launch_bounds__(256, NP == 4 ? 4 : kMfmaMinWaves) void gram_small_kernel(BwdReduceArgs a) {
+__global__ __launch_bounds__(256, 4) void gram_small_kernel(BwdReduceArgs a) {
     static_assert(NP == 4 || NP == 8, "stream groups of four");
     static_assert(FUSED || !STATIC, "the static tail runs inside the launch");
     using SK = SkSmall<NP>;
