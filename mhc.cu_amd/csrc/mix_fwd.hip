@@ -166,8 +166,11 @@ constexpr int kFwdStaggerMinB = 512;  // two or more workgroups per CU
 // RAG: rows of any length (C % V != 0): the last chunk of a row is loaded V elements wide from C - V on and
 // shifted down behind the barrier.  A template argument: as a run-time switch the clamps and compares cost the
 // whole rows 4 % (B=3001 n=4 C=2560: 27.4 -> 28.5 us).
+// Registers: 8 x 8 in bf16 with two chunks per thread is held at 168, three waves per SIMD (twenty of 176 go to scratch memory, and
+// still: n=8 B=4000 C=2560 forward 116.7 -> 101.3 us, B=600 C=2304 28.4 -> 23.5, n=6 B=2000 C=3072 57.4 -> 49.7; with fp32
+// storage 32 go and it loses: n=8 B=1300 C=2560 87.2 -> 96.4).
 template <typename TX, typename TY, int NP, int V, int CPT, bool RX = false, bool RAG = false>
-__global__ __launch_bounds__((NP == 8 && std::is_same<TX, float>::value) ? 512 : 256, (CPT == (NP == 4 ? 2 : 1) && !std::is_same<TX, float>::value) ? 4 : kMfmaMinWaves)
+__global__ __launch_bounds__((NP == 8 && std::is_same<TX, float>::value) ? 512 : 256, (CPT == (NP == 4 ? 2 : 1) && !std::is_same<TX, float>::value) ? 4 : (NP == 8 && CPT == 2 && !std::is_same<TX, float>::value) ? 3 : kMfmaMinWaves)
 void layer_fwd_small_kernel(LayerFwdArgs a) {
     using SK = SkSmall<NP>;
     __shared__ float coef_s[NP * NP + 2 * NP];  // M | Hpre | Hpost
