@@ -730,10 +730,21 @@ bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
     return B <= (nt == 1 ? 4096 : (nt == 2 ? 1024 : 512));
 }
 
+// Row tiles of phi per workgroup of the narrow kernel, n = 5 .. 8: one, in as many groups, where all of them (two or three) would
+// leave the chip few workgroups that each walk three times the bytes, and while reading x once per group costs less than that.
+// Forward us, all tiles -> one: n=8 B=1 C=4096 14.8 -> 12.3, 16 2560 15.2 -> 12.8, 64 1280 12.7 -> 11.1, 100 2560 16.0 -> 14.0, 1000 1280
+// (20 MB of x) 23.2 -> 22.4; n=6 B=32 C=1024 11.4 -> 10.7; n=5 B=10 C=777 13.7 -> 12.8; float32 n=8 B=16 C=2560 23.6 -> 16.2, 500 1280
+// (20 MB) 28.1 -> 25.8.  Beyond: n=6 B=2000 C=1024 (25 MB) 20.6 -> 21.3, n=8 B=700 C=2560 (29 MB) 26.3 -> 27.7, 2000 2560 54.9 -> 70.2.
+static int narrow_nt(int x_dtype, int B, int n, int C, int KS) {
+    const int tiles = mfma_nt(n);
+    const bool few = (B + 31) / 32 * KS * tiles <= 1024 && (size_t)B * n * C * (x_dtype == kBF16 ? 2 : 4) <= (22u << 20);
+    return n <= 8 && few ? 1 : tiles;
+}
+
 hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_dtype, float *Ppart,
                            float *ssqpart, int KS, int B, int n, int C, hipStream_t stream,
                            const ParamGather *gather) {
-    const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n);
+    const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n), nt = narrow_nt(x_dtype, B, n, C, KS);
     if (gather) {
         PhiSrc src;
         for (int i = 0; i < 3; i++) {
@@ -746,7 +757,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
         src.alpha_out = gather->alpha_out;
         src.n = n;
         if (x_dtype == kF32) {
-            switch (mfma_nt(n)) {
+            switch (nt) {
                 case 1: return launch_mfma<1, false, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
                 case 2: return launch_mfma<2, false, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
                 case 3: return launch_mfma<3, false, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
@@ -756,7 +767,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
         if (use_wide(n, C)) return launch_wide<1, 2, 4, 2, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
         if (n > 8) return hipErrorInvalidValue;  // see proj_fwd_gathers
         const bool xf32 = x_dtype == kF32AsBF16;
-        switch (mfma_nt(n)) {
+        switch (nt) {
             case 1: return xf32 ? launch_mfma<1, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src)
                                 : launch_mfma<1, false, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
             case 2: return xf32 ? launch_mfma<2, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src)
@@ -768,7 +779,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
     }
     if (use_mfma(x_dtype, phi_dtype, n, C)) {
         if (x_dtype == kF32AsBF16) {  // fp32 storage, rounded on load: the narrow kernel only (n <= 8)
-            switch (use_wide(n, C) ? 0 : mfma_nt(n)) {
+            switch (use_wide(n, C) ? 0 : nt) {
                 case 1: return launch_mfma<1, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
                 case 2: return launch_mfma<2, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
                 case 3: return launch_mfma<3, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
@@ -776,7 +787,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
             }
         }
         if (use_wide(n, C)) return launch_wide<1, 2, 4>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
-        switch (mfma_nt(n)) {
+        switch (nt) {
             case 1: return launch_mfma<1>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
             case 2: return launch_mfma<2>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
             case 3: return launch_mfma<3>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
@@ -784,7 +795,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
         }
     }
     if (use_exact(x_dtype, phi_dtype, n, C)) {
-        switch (mfma_nt(n)) {
+        switch (nt) {
             case 1: return launch_mfma<1, false, false, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
             case 2: return launch_mfma<2, false, false, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
             case 3: return launch_mfma<3, false, false, true>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream);
