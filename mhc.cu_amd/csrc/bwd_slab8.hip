@@ -160,29 +160,38 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
         if (T > 1) load_all(1, mine);
     }
     char *const phi_s = smem + ST::kG + 2 * ST::kTile;
-    if (tid < CW)
-        reinterpret_cast<float *>(smem + ST::kW)[tid] =
-            (c0 + tid < C && !INJECT) ? (a.w_bf16 ? bf16_to_f32(static_cast<const bf16_t *>(a.w)[c0 + tid])
-                                                  : static_cast<const float *>(a.w)[c0 + tid]) : 0.f;
     // mixer lane (l16, kq): the four channels from c0 + cl of sample l16
     const int l16 = lane & 15, kq = lane >> 4, cl = 16 * (wave & 3) + 4 * kq;
     bf16x8_t phif[N][NTD];  // mixers: A operand, rows = this wave's 16 channels of a stream, contraction over 32 d
+    // The mixers alone bring phi and w, all of it asked for at once, and none of these barriers waits for global memory: holders
+    // that brought a part of it waited for their first tiles before they could hand it on.  Backward in graphs of ten: n=5 B=3000
+    // C=1024 55.4 -> 54.3 us, n=7 B=700 C=2552 56.1 -> 55.1, n=8 B=2048 C=2560 99.5 -> 99.2.
+    constexpr int kPhiThreads = 64 * ST::kMixers, kPhiIters = N * 32 * kChunks / kPhiThreads;
+    static_assert(kPhiIters * kPhiThreads == N * 32 * kChunks, "whole chunks of phi for every mixer");
+    uint4 phir[NTD][kPhiIters];
+    if (!holder) {
+#pragma unroll
+        for (int kk = 0; kk < NTD; kk++)
+#pragma unroll
+            for (int i = 0; i < kPhiIters; i++) {
+                const int e = tid + i * kPhiThreads;
+                const int d = 32 * kk + e / (N * kChunks), j = e / kChunks % N, c = c0 + e % kChunks * 8;
+                const bool ok = d < D && c < C;
+                phir[kk][i] = load16_masked(reinterpret_cast<const uint4 *>(a.phi + (ok ? (size_t)d * nC + (size_t)j * C + c : 0)), ok);
+            }
+        if (tid < CW)
+            reinterpret_cast<float *>(smem + ST::kW)[tid] =
+                (c0 + tid < C && !INJECT) ? (a.w_bf16 ? bf16_to_f32(static_cast<const bf16_t *>(a.w)[c0 + tid])
+                                                      : static_cast<const float *>(a.w)[c0 + tid]) : 0.f;
+    }
 #pragma unroll
     for (int kk = 0; kk < NTD; kk++) {
-        constexpr int kPhiIters = (N * 32 * kChunks + 511) / 512;
-        uint4 phir[kPhiIters];
+        if (kk > 0) stage_barrier();  // the rows before have been read
+        if (!holder) {
 #pragma unroll
-        for (int i = 0; i < kPhiIters; i++) {
-            const int e = tid + i * 512;
-            const int d = 32 * kk + e / (N * kChunks), j = e / kChunks % N, c = c0 + e % kChunks * 8;
-            const bool ok = e < N * 32 * kChunks && d < D && c < C;
-            phir[i] = load16_masked(reinterpret_cast<const uint4 *>(a.phi + (ok ? (size_t)d * nC + (size_t)j * C + c : 0)), ok);
+            for (int i = 0; i < kPhiIters; i++) *reinterpret_cast<uint4 *>(phi_s + (tid + i * kPhiThreads) * 16) = phir[kk][i];
         }
-        __syncthreads();  // the rows before have been read
-#pragma unroll
-        for (int i = 0; i < kPhiIters; i++)
-            if (tid + i * 512 < N * 32 * kChunks) *reinterpret_cast<uint4 *>(phi_s + (tid + i * 512) * 16) = phir[i];
-        __syncthreads();
+        stage_barrier();
         if (!holder) {
             const int q = lane & 3, jj = (lane >> 2) & 3;
 #pragma unroll
@@ -194,7 +203,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             }
         }
     }
-    __syncthreads();  // the places that held phi may be filled
+    stage_barrier();  // the places that held phi may be filled
 
     float *const red_w = smem_f;                                                       // at the end: [16][CW + 1]
     double *const red_dt = reinterpret_cast<double *>(smem + 16 * (CW + 2) * 4);       // and [mixers][128]
