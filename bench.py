@@ -36,22 +36,22 @@ HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 # `--copy-calibration` (a 64 MiB copy).  Filled from the committed counter summary
 # (profiles/hbm_traffic_counters.txt); `commit` is the revision of the kernels the counters ran on.
 MEASURED_TRAFFIC = {
-    "commit": "f150377",
-    "bytes": {"c1": 13286270, "c2": 39643066, "c3": 251141433, "c4": 66398090, "c5": 577632535},
+    "commit": "32aec46",
+    "bytes": {"c1": 13286270, "c2": 39643076, "c3": 251122787, "c4": 66398218, "c5": 577670210},
 }
 
 # The kernel with the largest share of a step's device time, from the committed kernel-trace summaries
 # (profiles/layer_step_<config>.txt): average duration per dispatch and the HBM bytes the algorithm
 # needs that kernel to move (its own inputs and outputs once; for the split projections the partial
 # sums are not counted).
-PROFILED_AT = "f150377"
+PROFILED_AT = "32aec46"
 PROFILED_DOMINANT = {
-    "c1": dict(kernel="layer_fwd_small_kernel<float,float,4,4,2>", us=6.62, bytes=2 * 4 * 320 * 4 * 1280),
+    "c1": dict(kernel="layer_fwd_small_kernel<float,float,4,4,2>", us=6.65, bytes=2 * 4 * 320 * 4 * 1280),
     # sample-resident backward kernel: reads dy and x, writes the partial dx and the fp32 rows the batch sums are made of
-    "c2": dict(kernel="bwd_resident_kernel<4,bf16 w,2 items,5 tile waves>", us=9.06, bytes=3 * 2 * 320 * 4 * 1280 + 4 * 320 * 1280),
-    "c3": dict(kernel="bwd_slab_stage_kernel<4,128 channels>", us=18.86, bytes=3 * 2 * 1280 * 4 * 2560 + 2 * 24 * 10240 + 4 * 24 * 10240),
-    "c4": dict(kernel="bwd_resident_kernel<8,bf16 w,1 item,10 tile waves>", us=11.24, bytes=3 * 2 * 256 * 8 * 1280 + 4 * 256 * 1280),
-    "c5": dict(kernel="dphi_large_kernel<9,true>", us=36.94, bytes=2 * 128 * 40960 + 4 * 1088 * 40960),
+    "c2": dict(kernel="bwd_resident_kernel<4,bf16 w,2 items,5 tile waves>", us=9.08, bytes=3 * 2 * 320 * 4 * 1280 + 4 * 320 * 1280),
+    "c3": dict(kernel="bwd_slab_stage_kernel<4,128 channels>", us=18.04, bytes=3 * 2 * 1280 * 4 * 2560 + 2 * 24 * 10240 + 4 * 24 * 10240),
+    "c4": dict(kernel="bwd_resident_kernel<8,bf16 w,1 item,10 tile waves>", us=11.30, bytes=3 * 2 * 256 * 8 * 1280 + 4 * 256 * 1280),
+    "c5": dict(kernel="dphi_large_kernel<9,true>", us=36.02, bytes=2 * 128 * 40960 + 4 * 1088 * 40960),
 }
 
 CONFIGS = {
