@@ -540,8 +540,8 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
     }
     stage_barrier();
 
-    float usum[4] = {0.f, 0.f, 0.f, 0.f};  // mixers
-    double dtsum = 0.0;                    // loaders of slab 0: column tid & 31, row group
+    double usum[4] = {0.0, 0.0, 0.0, 0.0};  // mixers: float32 terms, a sample each (the walk may be hundreds of tiles long)
+    double dtsum = 0.0;                     // loaders of slab 0: column tid & 31, row group
     // mixer lane (l16, kq): the four channels from c0 + cl of sample l16
     const int l16 = lane & 15, kq = lane >> 4, cl = 16 * wave + 4 * kq;
 
@@ -624,6 +624,19 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
             MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 1, pclk);
             if (t > 0) store_dx(t - 1);
             const bf16x8_t ah = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + lane * 16);
+            // what the mixing needs, requested ahead of the products, under which it arrives (n=4 B=1605 C=1728, whole backward:
+            // 40.0 -> 39.1 us)
+            float Mr[N][N], hpre[N], hpost[N];
+            uint2 xr[N], gr[N];
+            lds_floats<N>(co + ST::kSegM * 64 + l16 * N, hpre);
+            lds_floats<N>(co + (ST::kSegM + 1) * 64 + l16 * N, hpost);
+            lds_floats<N * N>(co + l16 * N * N, &Mr[0][0]);
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * CW * 2 + row_at);
+                gr[j] = *reinterpret_cast<const uint2 *>(gs + j * TB * CW * 2 + row_at);
+            }
+            __builtin_amdgcn_sched_barrier(0);
             const bf16x8_t al = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + 1024 + lane * 16);
 #pragma unroll
             for (int k = 0; k < kAcc; k++) {
@@ -641,17 +654,9 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
             // projection term: columns = samples, rows = this lane's channels
             const bf16x8_t pf = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + 2048 + lane * 16);
             f32x4_t o[N];
-            uint2 xr[N], gr[N];
-            float Mr[N][N], hpre[N], hpost[N];
 #pragma unroll
-            for (int j = 0; j < N; j++) {
+            for (int j = 0; j < N; j++)
                 o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(phif[j], pf, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * CW * 2 + row_at);
-                gr[j] = *reinterpret_cast<const uint2 *>(gs + j * TB * CW * 2 + row_at);
-            }
-            lds_floats<N * N>(co + l16 * N * N, &Mr[0][0]);
-            lds_floats<N>(co + ST::kSegM * 64 + l16 * N, hpre);
-            lds_floats<N>(co + (ST::kSegM + 1) * 64 + l16 * N, hpost);
             const float *sc = co + (ST::kSegM + 2) * 64 + l16;
             const float cxv = sc[0];
             float qinv = 0.f, k2 = 0.f;
@@ -681,7 +686,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
                     dfv[c] = s_df;
                     const float dq = s_df * qinv;
                     const float da = INJECT ? 0.f : dq * wv[c] - s_a * k2;
-                    if constexpr (!INJECT) usum[c] += dq * s_a;
+                    if constexpr (!INJECT) usum[c] += (double)(dq * s_a);
 #pragma unroll
                     for (int j = 0; j < N; j++) {
                         float v = o[j][c] + hpre[j] * da - cxv * xv[j];
@@ -719,7 +724,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
     MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 3, pclk);
     __syncthreads();  // everyone is done with the rings; reuse them for the two small reductions
     if constexpr (!INJECT) {
-        float *red = smem_f;  // [16][CW + 1]
+        double *red = reinterpret_cast<double *>(smem);  // [16][CW + 1]
         if (!loader) {
 #pragma unroll
             for (int v = 0; v < 4; v++) red[l16 * (CW + 1) + cl + v] = usum[v];

@@ -205,8 +205,8 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
     }
     stage_barrier();  // the places that held phi may be filled
 
-    float *const red_w = smem_f;                                                       // at the end: [16][CW + 1]
-    double *const red_dt = reinterpret_cast<double *>(smem + 16 * (CW + 2) * 4);       // and [mixers][128]
+    double *const red_w = reinterpret_cast<double *>(smem);  // at the end: [16][CW + 1]
+    double *const red_dt = red_w + 16 * (CW + 1);            // and [mixers][128]
     if (holder) {
         // ---- requests the tiles, accumulates dphi: 32-column tiles hw, hw + 4 .. (stream, channel half) ----------
         Block mine[ST::kShare];  // (formed again: kept across the prologue they spill)
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
         const float4 w4 = *reinterpret_cast<const float4 *>(smem + ST::kW + cl * 4);
         const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
         const float inv_c = 1.0f / (float)C;
-        float usum[4] = {0.f, 0.f, 0.f, 0.f};
+        double usum[4] = {0.0, 0.0, 0.0, 0.0};  // float32 terms, a sample each: the walk may be hundreds of tiles long
         double dtsum[2] = {0.0, 0.0};  // columns lane, lane + 64 of dt
         const int row_at = l16 * CW * 2 + (((cl >> 3) ^ slab_swizzle<CW>(l16)) * 16) + (kq & 1) * 8;  // this lane's 8 bytes of its sample's row
         constexpr int kPieces = N * TB / kRows, kOut = (kPieces + ST::kMixers - 1) / ST::kMixers;
@@ -314,12 +314,27 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
                     dtv[r][1] = p[min(lane + 64, D + 2)];
                 }
             }
-            // projection term: columns = samples, rows = this lane's channels
+            // projection term: columns = samples, rows = this lane's channels.  What the mixing needs first is requested before
+            // it, and below every stream of dy with its row of M one stream ahead: left to itself the scheduler puts the reads
+            // where their waits are not hidden as soon as registers get short (n=8 B=2000 C=2560, whole backward: 105.6 -> 101.5 us)
             f32x4_t o[N];
+            float hpre[8], hpost[8];
+            const float *const Mb = co + l16 * 64;
+            struct Row { uint2 g; float4 m0, m1; };
+            auto row_of = [&](int i) {
+                return Row{*reinterpret_cast<const uint2 *>(gs + i * TB * CW * 2 + row_at),
+                           *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 * l16) & 63)),
+                           *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 + 4 * l16) & 63))};
+            };
+            Row row;
             {
                 bf16x8_t pf[NTD];
 #pragma unroll
                 for (int kk = 0; kk < NTD; kk++) pf[kk] = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + (2 * NTD + kk) * 1024 + lane * 16);
+                lds_floats<8>(co + (TB + (l16 >> 3)) * 64 + (l16 & 7) * 8, hpre);
+                lds_floats<8>(co + (TB + 2 + (l16 >> 3)) * 64 + (l16 & 7) * 8, hpost);
+                row = row_of(0);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int j = 0; j < N; j++) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(phif[j][0], pf[0], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
@@ -327,9 +342,6 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
 #pragma unroll
                     for (int j = 0; j < N; j++) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(phif[j][kk], pf[kk], o[j], 0, 0, 0);
             }
-            float hpre[8], hpost[8];
-            lds_floats<8>(co + (TB + (l16 >> 3)) * 64 + (l16 & 7) * 8, hpre);
-            lds_floats<8>(co + (TB + 2 + (l16 >> 3)) * 64 + (l16 & 7) * 8, hpost);
             const float *sc = co + (TB + 4) * 64 + l16;
             const float cxv = sc[0];
             float qinv = 0.f, k2 = 0.f;
@@ -340,20 +352,20 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             }
             // streams of dy one after the other: df, and the rows of M^T dy added into the accumulators
             float s_df[4] = {0.f, 0.f, 0.f, 0.f};
-            const float *Mb = co + l16 * 64;
 #pragma unroll
             for (int i = 0; i < N; i++) {
-                const uint2 g = *reinterpret_cast<const uint2 *>(gs + i * TB * CW * 2 + row_at);
+                const Row next = row_of(min(i + 1, N - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                const uint2 g = row.g;
                 const float gv[4] = {bf16lo_to_f32(g.x), bf16hi_to_f32(g.x), bf16lo_to_f32(g.y), bf16hi_to_f32(g.y)};
-                const float4 m0 = *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 * l16) & 63));
-                const float4 m1 = *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 + 4 * l16) & 63));
-                const float mr[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+                const float mr[8] = {row.m0.x, row.m0.y, row.m0.z, row.m0.w, row.m1.x, row.m1.y, row.m1.z, row.m1.w};
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
                     s_df[c] += hpost[i] * gv[c];
 #pragma unroll
                     for (int j = 0; j < N; j++) o[j][c] += mr[j] * gv[c];
                 }
+                row = next;
             }
             uint2 xr[N];
             float s_a[4] = {0.f, 0.f, 0.f, 0.f};
@@ -368,7 +380,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             for (int c = 0; c < 4; c++) {
                 const float dq = s_df[c] * qinv;
                 da[c] = INJECT ? 0.f : dq * wv[c] - s_a[c] * k2;
-                if constexpr (!INJECT) usum[c] += dq * s_a[c];
+                if constexpr (!INJECT) usum[c] += (double)(dq * s_a[c]);
             }
 #pragma unroll
             for (int j = 0; j < N; j++) {

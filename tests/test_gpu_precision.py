@@ -63,12 +63,12 @@ def test_ragged_rows_of_shared_coefficients_keep_float32_results(B, n, C):
 
 
 
-def _batch_and_single_sums(B, n, C, act):
+def _batch_and_single_sums(B, n, C, act, lib=None):
     """dw, dbias and dalpha of one backward call over B samples, and of B calls over one sample each on the same saved
     state, whose results are the terms of those sums; every sample comes twice, with dy and with -dy, in random order,
     so that the sums are far smaller than what is added up on the way."""
     from mhc import _lib
-    lib, D, dev = _lib.lib, n * n + 2 * n, "cuda"
+    lib, D, dev = _lib.lib if lib is None else lib, n * n + 2 * n, "cuda"
     x, dy, p = _dynamic(B // 2, n, C)
     order = torch.randperm(B, generator=torch.Generator().manual_seed(6))
     x, dy = torch.cat([x, x])[order].to(dev, act), torch.cat([dy, -dy])[order].to(dev, act)
@@ -113,6 +113,25 @@ def _close_to_float64(whole, terms):
 @pytest.mark.parametrize("B,n,C", [(1536, 8, 64), (2050, 6, 16), (1794, 2, 44), (1600, 7, 48), (1922, 4, 42)])
 def test_split_batch_sums_stay_in_float64(B, n, C):
     _close_to_float64(*_batch_and_single_sums(B, n, C, torch.bfloat16))
+
+
+# The bf16 slab kernels (n <= 4 with 64 and 128 channels per workgroup, n = 5 .. 8): up to 128 tiles of 16 samples per batch split,
+# so that a float32 sum over the tiles of a lane would be off by some 2^-24 of what is added up on the way, a million times the bound.
+@pytest.mark.parametrize("B,n,C,width,splits", [(2050, 4, 264, 1, 1), (1100, 4, 136, 2, 2), (1500, 3, 64, 2, 1), (1026, 1, 72, 1, 2),
+                                                (1100, 8, 264, 0, 1), (1500, 5, 72, 0, 2), (700, 7, 64, 0, 1)])
+def test_slab_sums_stay_in_float64(B, n, C, width, splits):
+    from mhc._lib import tuning_lib
+
+    lib = tuning_lib()
+    # the tiled path; one launch of channel sums and coefficient backward, as for one sample; slab width and splits
+    hooks = {7: 1, 2: 2, 11: width, 3: splits}
+    try:
+        for k, v in hooks.items():
+            assert lib.mhc_tuning_set(k, v) == 0
+        _close_to_float64(*_batch_and_single_sums(B, n, C, torch.bfloat16, lib))
+    finally:
+        for k in hooks:
+            lib.mhc_tuning_set(k, 0)
 
 
 @pytest.mark.parametrize("B,n,C", [(640, 4, 64), (770, 3, 36), (300, 1, 96), (1030, 2, 130), (2, 4, 8), (18, 4, 512)])
