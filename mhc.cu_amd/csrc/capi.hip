@@ -68,40 +68,44 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 // Whether the sample-resident backward (bwd_resident.hip + the column-slab kernel) is taken where it is
 // supported.  Its second launch walks all samples of a column slab in one workgroup, which stops paying once the batch is
 // large enough to fill the chip with batch splits; the fewer streams, the fewer slabs.
-// Measured, backward in graphs of ten, tiled (Gram + slab) path | resident path (us):
-//   n=4 C=256:  B=768 19.8 | 16.1, 2048 26.7 | 22.2, 3000 27.5 | 27.5, 6000 34.9 | 39.3;  C=512: 768 19.7 | 17.5, 1024 21.5 | 22.0
-//   n=4 C=1024: B=640 21.4 | 20.2, 768 21.9 | 22.3, 1024 23.0 | 27.0;  C=1280: 320 18.8 | 14.8, 512 21.6 | 19.3, 640 22.4 | 23.1,
-//               768 22.5 | 24.9, 1024 25.0 | 29.3;  C=1920: 512 23.7 | 23.6, 640 25.2 | 28.4
-//   n=4 C=2560: B=192 20.9 | 16.4, 320 25.3 | 25.3, 512 27.7 | 27.2, 640 29.1 | 34.5;  C=3200: 512 31.1 | 30.5, 640 33.2 | 37.7
-//               C=4096: 192 27.5 | 22.1, 320 30.3 | 32.2, 512 34.1 | 38.0, 768 38.0 | 53.0
-//   n=3 C=512:  B=1024 22.9 | 21.5, 1536 23.8 | 31.5;  C=1280: 768 22.4 | 23.0;  C=1920: 384 20.7 | 17.9, 576 22.9 | 24.8;
-//               C=3200: 192 20.1 | 18.3, 384 25.5 | 26.2, 576 27.8 | 33.7
-//   n=2 C=512:  B=768 17.9 | 16.5, 1024 19.9 | 20.5;  C=1280: 512 16.2 | 16.6, 768 19.2 | 21.6;  C=1920: 384 17.0 | 15.9, 576 19.5 | 23.7;
-//               C=3200: 192 17.5 | 16.5, 384 20.8 | 25.4
-//   n=1 C=256:  B=768 15.8 | 15.1, 1024 17.2 | 18.0;  C=960: 576 16.3 | 16.1, 768 16.5 | 17.4;  C=3200: 192 16.1 | 13.9, 384 17.9 | 21.6
-// The tiled path is one launch more, so the lines lie a little above the crossings: about 1.0 M / C samples, within bounds,
-// and 768 n samples of at most 256 channels (n=4 C=128: B=4096 31.9 | 27.1, 6000 35.0 | 33.9).
-// n = 5 .. 8, where the slab is bwd_slab8.hip (n=8 C=2560 B=2000: 106 | 182):
-//   n=5 C=256:  B=1024 27.1 | 28.2, 1536 32.5 | 30.2, 4000 53.7 | 47.8;  C=320: 768 24.8 | 27.7;  C=640: 512 24.1 | 21.2,
-//               768 26.5 | 30.0;  C=1280: 384 26.4 | 26.1, 512 27.0 | 28.0;  C=2560: 256 29.4 | 24.4, 384 32.1 | 35.4
-//   n=6 C=320:  B=768 27.6 | 28.5, 1100 36.7 | 39.0;  C=384: 512 25.9 | 19.4;  C=512: 768 29.3 | 29.1, 1100 36.9 | 40.2;
-//               C=1280: 512 30.8 | 28.6, 1024 41.6 | 49.0;  C=2560: 256 33.3 | 25.6, 512 39.1 | 39.8
-//   n=7 C=384:  B=768 31.6 | 29.9, 1100 38.5 | 39.7;  C=512: 768 31.2 | 29.5, 1100 39.7 | 40.4;  C=1280: 512 34.7 | 31.0,
-//               1024 46.4 | 53.3;  C=2560: 256 38.4 | 29.5, 512 44.5 | 48.3
-//   n=8 C=256:  B=1536 40.2 | 30.0, 6000 82.8 | 68.9;  C=320: 3000 60.6 | 58.7, 4500 75.9 | 81.4;  C=512: 2048 54.9 | 54.5,
-//               3000 65.7 | 74.9;  C=1280: 512 39.5 | 34.0, 768 47.0 | 46.7, 1024 52.6 | 59.5;  C=2560: 384 48.9 | 44.7,
-//               512 51.8 | 52.4;  C=4096: 384 62.2 | 60.4, 512 66.8 | 68.5
+// Measured, backward in graphs of ten, tiled (Gram + slab) path | resident path (us), in each row from below the line to above it
+// (a step of the tiled path's tile counts moves single rows by a few us either way):
+//   n=1 C=128:  B=844 18.0 | 19.8, 1304 17.5 | 21.1;  C=256: 652 18.8 | 17.8, 920 16.4 | 17.8;  C=384: 672 15.4 | 14.9, 816 18.6 | 19.9
+//       C=1024: 528 18.9 | 17.5, 904 20.8 | 23.9;  C=1920: 332 18.3 | 15.7, 480 15.0 | 16.2;  C=3200: 188 14.7 | 13.9, 268 19.1 | 19.5
+//   n=2 C=128:  2148 25.6 | 25.3, 2608 22.3 | 24.3;  C=256: 844 20.7 | 20.7, 1304 20.5 | 23.0, 1840 23.2 | 22.4, 2764 24.2 | 25.5
+//       C=384:  672 16.8 | 15.4, 960 17.2 | 19.0;  C=1280: 528 20.6 | 19.2, 624 20.8 | 21.4;  C=1920: 352 16.0 | 14.8, 416 16.4 | 17.0
+//       C=3200: 212 17.8 | 17.0, 248 17.0 | 18.4;  C=4096: 120 18.6 | 13.7, 188 16.7 | 19.2
+//   n=3 C=128:  3224 25.5 | 23.9, 4608 27.5 | 29.5;  C=256: 1956 28.4 | 24.8, 2764 26.7 | 27.8;  C=384: 816 22.3 | 20.3, 1152 22.0 | 22.6
+//       C=1280: 568 21.8 | 21.1, 812 25.6 | 27.9;  C=1920: 376 20.4 | 18.2, 540 22.9 | 24.2;  C=3200: 224 19.0 | 18.6, 276 22.7 | 24.6
+//       C=4096: 176 22.0 | 20.2, 320 22.2 | 29.8
+//   n=4 C=128:  3376 26.4 | 26.5, 4300 29.4 | 31.1;  C=256: 2148 28.6 | 27.5, 2608 26.2 | 27.2, 4452 33.5 | 35.7;  C=264: 816 22.0 | 19.5,
+//               1152 22.9 | 22.0, 1392 25.3 | 26.1;  C=320: 816 21.9 | 19.9, 960 19.8 | 19.8, 1392 25.9 | 27.5;  C=384: 816 21.7 | 20.4,
+//               960 19.7 | 20.6, 1392 25.6 | 29.0 (the step at 256 channels: up to there a workgroup of the resident path has
+//               two tile waves instead of four, and more workgroups fit a CU)
+//       C=1024: 744 25.0 | 22.4, 876 24.6 | 25.9;  C=1280: 596 23.2 | 22.8, 700 21.7 | 24.0;  C=1920: 396 24.3 | 22.1, 468 22.9 | 23.7
+//       C=2560: 296 26.4 | 24.9, 348 22.7 | 24.8;  C=3200: 224 22.7 | 21.5, 320 24.0 | 26.6;  C=4096: 176 25.5 | 22.0, 272 27.8 | 31.9
+// n = 5 .. 8, where the slab is bwd_slab8.hip:
+//   n=5 C=256:  4000 48.7 | 47.3, 5800 63.4 | 67.8;  C=384: 596 25.7 | 24.2, 704 24.7 | 27.3;  C=768: 552 29.5 | 29.1, 780 30.0 | 35.5
+//       C=1280: 388 30.6 | 29.2, 564 29.7 | 34.7;  C=2560: 224 29.0 | 23.3, 320 29.6 | 35.2;  C=4096: 224 32.4 | 30.6, 272 37.4 | 46.2
+//   n=6 C=256:  5800 66.7 | 61.7;  C=384: 624 28.2 | 25.4, 760 27.9 | 29.0;  C=768: 624 30.1 | 29.1, 760 29.5 | 31.0;  C=1280: 488 33.2 |
+//               30.2, 576 31.4 | 35.2;  C=2560: 244 33.3 | 26.4, 312 34.9 | 36.6;  C=4096: 244 38.4 | 33.7, 312 41.4 | 48.3
+//   n=7 C=256:  6000 71.1 | 67.1, 8700 88.8 | 90.7;  C=384: 868 35.9 | 32.9, 1024 31.8 | 32.9, 1484 39.9 | 42.8;  C=768: 868 38.4 | 38.4,
+//               1228 44.1 | 48.0;  C=1280: 480 32.9 | 29.8, 684 39.6 | 42.6;  C=2560: 244 38.5 | 28.8, 312 40.0 | 41.0, 536 47.0 | 59.2
+//   n=8 C=256:  8000 91.2 | 84.7, 11600 118.4 | 117.5;  C=320: 2228 49.5 | 49.1, 2708 54.4 | 56.5;  C=512: 1392 46.9 | 45.6, 1692 48.7 |
+//               50.9;  C=1280: 556 43.7 | 43.4, 676 46.9 | 48.3;  C=2560: 408 49.1 | 47.8, 480 49.5 | 50.6;  C=4096: 336 61.1 | 57.0,
+//               408 62.0 | 64.2
 // Experiment hook: 1 = never, 2 = always.
 bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;
     if (n > 4) {
         if (C <= 256) return true;
-        const int per_row[4] = {500'000, 740'000, 880'000, 1'020'000}, least[4] = {320, 448, 448, 480}, most[4] = {704, 896, 1024, 4096};
+        const int per_row[4] = {520'000, 640'000, 760'000, 720'000}, least[4] = {224, 256, 256, 448}, most[4] = {640, 640, 896, 3000};
         return B <= std::min(most[n - 5], std::max(least[n - 5], per_row[n - 5] / C));
     }
-    if (C <= 256) return B <= (C <= 128 ? 1536 : 768) * n;
-    const int per_row[4] = {640'000, 800'000, 1'040'000, 900'000};
-    return B <= std::min(960, std::max(n >= 3 ? 320 : 224, per_row[n - 1] / C));
+    const int upto128[4] = {768, 2176, 3968, 3840}, upto256[4] = {768, 1088, 2304, 2304};
+    if (C <= 256) return B <= (C <= 128 ? upto128 : upto256)[n - 1];
+    const int per_row[4] = {640'000, 680'000, 760'000, 780'000}, most[4] = {768, 704, 832, 832};
+    return B <= std::min(most[n - 1], per_row[n - 1] / C);
 }
 
 // Shapes for which the dynamic entry points take fp32 activations that are consumed as bf16
