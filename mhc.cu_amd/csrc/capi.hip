@@ -157,18 +157,23 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     // backward's second launch with a split batch
     const int bs3 = n <= 4 ? std::max(bwd_slab_batch_splits(B, n, C, kBF16), bwd_slab_batch_splits(B, n, C, kF32)) : 1;
     const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1, bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
-    const int bs7 = n >= 5 && n <= 8 ? bwd_slab8_batch_splits(B, C) : 1;
-    const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : (n <= 8 ? (size_t)bs7 * bwd_slab8_slabs(C) : 0), parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
-    w.u = c.floats(std::max((size_t)B, 2 * (n <= 4 ? slab64 : (size_t)bs7)) * C);
+    // (also where the resident path is preferred: it does not take more than 32 Sinkhorn iterations)
+    const bool slab8 = n >= 5 && n <= 8 && C % 8 == 0;
+    const int bs7 = slab8 ? bwd_slab8_batch_splits(B, C) : 1;
+    const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : (slab8 ? (size_t)bs7 * bwd_slab8_slabs(C) : 0), parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
+    w.u = c.floats(std::max((size_t)B, 2 * (n <= 4 ? slab64 : (size_t)(slab8 ? bs7 : 0))) * C);
     w.upart = c.floats(2 * parts64 * C);
     w.dtpart = c.floats(std::max((size_t)B, 2 * std::max(slab64, parts64)) * (D + 3));
     w.raw = c.floats(bwd_reduce_raw_floats(B, n, C));
     w.s1part = c.floats(n > 8 ? (size_t)B * bwd_reduce_parts(B, n, C) : 0);
     // wide projections: the part of dx that is formed beside the coefficient backward, fp32
     w.dx_part = c.floats(wide_dx_beside(B, n, C) ? (size_t)B * nC : 0);
-    // n <= 8, sample-resident backward: dxp where it is handed over in fp32 (n = 5 .. 8: on either side of the line, for
-    // the experiment hook)
-    const bool resident = n <= 8 && C <= kResMaxC && (n > 4 || bwd_resident_preferred(B, n, C) || C % 8 != 0);
+    // n <= 8, sample-resident backward: dxp where it is handed over in fp32
+#ifdef MHC_TUNING
+    const bool resident = n <= 8 && C <= kResMaxC;  // on either side of the line: the experiment hook may be set later
+#else
+    const bool resident = n <= 8 && C <= kResMaxC && (bwd_resident_preferred(B, n, C) || C % 8 != 0);
+#endif
     w.dxp = c.floats(resident && bwd_resident_dxp_f32(n, C) ? (size_t)B * nC : 0);
     int bs = dphi_batch_splits(B, n, C);
     const int bs2 = proj_bwd_batch_splits(B, n, C);

@@ -66,6 +66,15 @@ def test_workspace_queries():
     assert L.mhc_sinkhorn_knopp_bwd_workspace_bytes(1, 200, 4, 5) == 0
 
 
+# above the line between the two backward paths: no fp32 copy of dx for the path that is not taken; ragged rows: no partial
+# sums for a kernel that does not take them
+@pytest.mark.parametrize("B,n,C,most", [(8192, 8, 4096, 0.3), (4000, 5, 2816, 0.4), (3000, 6, 384, 1.5), (8192, 4, 4096, 0.4), (4000, 8, 257, 1.9)])
+def test_workspace_holds_only_what_the_path_uses(B, n, C, most):
+    from mhc import _lib
+
+    assert _lib.lib.mhc_layer_dynamic_workspace_bytes(B, n, C) <= most * 4 * B * n * C
+
+
 def test_argument_validation_happens_before_any_launch():
     """Bad arguments are rejected with distinct codes; nothing is launched, so this runs without a GPU."""
     from mhc import _lib
