@@ -444,7 +444,7 @@ __global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduc
         for (int e = lane; e < nb * K; e += 64) {
             float v = 0.f;
             for (int r = 0; r < SW; r++) v += slot_s[e * SW + r];
-            tot_s[e] = v;
+            tot_s[e] = (e >> 2 & 3) < n && (e & 3) < n ? v : 0.f;  // row and column of a product: streams >= n count for nothing
         }
         MHC_PHASE_ADD(kPhaseGramSmall, blockIdx.x, 2, pclk);
         if (live) {  // (same wave: no barrier)
@@ -472,8 +472,8 @@ __global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduc
         uint4 gr[U], xr[U], fr[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            // beyond the row: any valid chunk (dropped or masked below); streams >= n alias stream 0: their entries of the
-            // sums are read by nobody
+            // beyond the row: any valid chunk (dropped or masked below); streams >= n alias stream 0: their entries are
+            // dropped where the sums are finished
             const int st = s_first + u * SW < nsteps ? s_first + u * SW : 0;
             const uint32_t at = (uint32_t)((i < n ? i : 0) * C + st * 128 + min(blk * 8, C - 8 - st * 128));
             gr[u] = *reinterpret_cast<const uint4 *>(gb + at);

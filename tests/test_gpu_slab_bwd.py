@@ -44,6 +44,32 @@ def test_channel_sums_of_several_samples_per_workgroup(B, n, C, inject, w_f32):
         lib.mhc_tuning_set(K_RESIDENT, 0)
 
 
+# fewer than four streams, whose sums share a 4 x 4 product with nobody's: a sum of stream 0 that overflows stays infinite where the
+# two launches have infinity (NaN comes from an infinity times the zero coefficient of a stream that is not there)
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_overflow_of_one_sum_stays_where_it_is(n):
+    from mhc._lib import tuning_lib
+    from test_gpu_resident_bwd import _step
+
+    lib, got = tuning_lib(), []
+    st = _step(6, n, 136, False, False)
+    st.forward()
+    st.dy.zero_()
+    st.x[4, :, 7] = 0
+    st.x[4, 0, 7], st.dy[4, n - 1, 7] = 8.0, 1e38  # dy x^T of streams (n - 1, 0) only
+    try:
+        assert lib.mhc_tuning_set(K_RESIDENT, 1) == 0
+        for mode in (1, 2):
+            assert lib.mhc_tuning_set(K_GRAM, mode) == 0
+            st.backward()
+            got.append(st.dbias[n:2 * n].cpu())  # of H_post
+    finally:
+        lib.mhc_tuning_set(K_RESIDENT, 0)
+        lib.mhc_tuning_set(K_GRAM, 0)
+    for g in got:
+        assert g[n - 1] == float("inf") and not g[:n - 1].any(), got
+
+
 # n = 5 .. 8 (csrc/bwd_slab8.hip): one to four tiles of 16 samples per split, cut tiles, channels beyond the row, several slabs
 @pytest.mark.parametrize("B,n,C,splits", [(1, 5, 8, 1), (16, 8, 64, 1), (17, 8, 72, 1), (33, 6, 136, 1), (50, 7, 64, 1), (49, 8, 200, 2),
                                           (130, 5, 264, 3), (65, 7, 320, 0), (200, 8, 1280, 0), (300, 6, 1928, 0)])
