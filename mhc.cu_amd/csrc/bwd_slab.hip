@@ -660,10 +660,10 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
             const float *sc = co + (ST::kSegM + 2) * 64 + l16;
             const float cxv = sc[0];
             float qinv = 0.f, k2 = 0.f;
+            const bool real = sb + l16 < b_end;  // a slot beyond the batch adds nothing to usum, whatever its sample holds
             if constexpr (!INJECT) {
                 qinv = 1.0f / sc[64];
                 k2 = sc[128] * qinv * qinv * qinv * inv_c;
-                qinv = sb + l16 < b_end ? qinv : 0.f;  // a slot beyond the batch adds nothing to usum
             }
             float dfv[4];
             uint32_t out[N][2];
@@ -686,7 +686,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
                     dfv[c] = s_df;
                     const float dq = s_df * qinv;
                     const float da = INJECT ? 0.f : dq * wv[c] - s_a * k2;
-                    if constexpr (!INJECT) usum[c] += (double)(dq * s_a);
+                    if constexpr (!INJECT) usum[c] += (double)(real ? dq * s_a : 0.f);
 #pragma unroll
                     for (int j = 0; j < N; j++) {
                         float v = o[j][c] + hpre[j] * da - cxv * xv[j];

@@ -345,10 +345,10 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             const float *sc = co + (TB + 4) * 64 + l16;
             const float cxv = sc[0];
             float qinv = 0.f, k2 = 0.f;
+            const bool real = sb + l16 < b_end;  // a slot beyond the batch adds nothing to usum, whatever its sample holds
             if constexpr (!INJECT) {
                 qinv = 1.0f / sc[64];
                 k2 = sc[128] * qinv * qinv * qinv * inv_c;
-                qinv = sb + l16 < b_end ? qinv : 0.f;  // a slot beyond the batch adds nothing to usum
             }
             // streams of dy one after the other: df, and the rows of M^T dy added into the accumulators
             float s_df[4] = {0.f, 0.f, 0.f, 0.f};
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             for (int c = 0; c < 4; c++) {
                 const float dq = s_df[c] * qinv;
                 da[c] = INJECT ? 0.f : dq * wv[c] - s_a[c] * k2;
-                if constexpr (!INJECT) usum[c] += (double)(dq * s_a[c]);
+                if constexpr (!INJECT) usum[c] += (double)(real ? dq * s_a[c] : 0.f);
             }
 #pragma unroll
             for (int j = 0; j < N; j++) {

@@ -4,6 +4,7 @@ each other.  The channel sums with the coefficient backward of several samples p
 csrc/mix_bwd_reduce.hip): against the two launches.  The slab
 kernel of five to eight streams: against the general kernels.  Reference backward: src/python/mhc/ops.py:276-361."""
 import pytest
+import torch
 
 from test_gpu_resident_bwd import K_RESIDENT, _both_paths
 
@@ -68,6 +69,28 @@ def test_overflow_of_one_sum_stays_where_it_is(n):
         lib.mhc_tuning_set(K_GRAM, 0)
     for g in got:
         assert g[n - 1] == float("inf") and not g[:n - 1].any(), got
+
+
+# slots of a tile beyond the batch repeat its last sample: one whose df overflows adds its infinity to dw and the slots nothing
+@pytest.mark.parametrize("n", [2, 4, 5, 8])
+def test_slots_beyond_the_batch_add_nothing(n):
+    from mhc._lib import tuning_lib
+    from test_gpu_resident_bwd import _step
+
+    lib, got = tuning_lib(), []
+    st = _step(17, n, 72, False, False)
+    st.forward()
+    st.dy[16, :, 7] = 3e38
+    st.x[16, :, 7] = 1.0
+    try:
+        for mode in (1, 2):
+            assert lib.mhc_tuning_set(K_RESIDENT, mode) == 0
+            st.backward()
+            got.append(st.dw.cpu())
+    finally:
+        lib.mhc_tuning_set(K_RESIDENT, 0)
+    for g in got:
+        assert g[7] == float("inf") and torch.isfinite(g[:7]).all() and torch.isfinite(g[8:]).all(), g
 
 
 # n = 5 .. 8 (csrc/bwd_slab8.hip): one to four tiles of 16 samples per split, cut tiles, channels beyond the row, several slabs
