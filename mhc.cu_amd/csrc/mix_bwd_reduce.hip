@@ -446,6 +446,10 @@ __global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduc
             for (int r = 0; r < SW; r++) v += slot_s[e * SW + r];
             tot_s[e] = (e >> 2 & 3) < n && (e & 3) < n ? v : 0.f;  // row and column of a product: streams >= n count for nothing
         }
+        // (here and for w_s below: a wave's LDS accesses complete in order, the fence keeps the compiler from moving reads of
+        // another lane's values above the writes)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         MHC_PHASE_ADD(kPhaseGramSmall, blockIdx.x, 2, pclk);
         if (live) {  // (same wave: no barrier)
             cb.fetch_sums(tot_s + k * K, 1);
@@ -481,6 +485,10 @@ __global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduc
             if constexpr (inject)
                 fr[u] = load16_masked(reinterpret_cast<const uint4 *>(static_cast<const bf16_t *>(a.f_inject) + (size_t)(b0 + k) * C +
                                                                       st * 128 + min(blk * 8, C - 8 - st * 128)), i == 0);
+        }
+        if constexpr (!inject) {  // (behind the loads: they need not wait for w)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
         f32x4_t acc[3];
 #pragma unroll
