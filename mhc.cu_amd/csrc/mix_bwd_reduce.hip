@@ -1097,9 +1097,6 @@ static int gram_small_parts(int B, int C) { return C >= 1024 && B < 1024 ? 2 : 1
 // too small to do without column parts.
 static bool gram_small_fused(const BwdReduceArgs &a) {
     if (const int hook = tuning_get(kTuneGramFused); hook && a.T <= 32) return hook == 2;  // experiment hook
-    // (n <= 4: the tail of a workgroup outweighs the streaming of very short rows, but such batches of those take
-    // gram_quad_kernel; n > 4 has no rows to pack four samples of into a wave)
-    if (a.B >= 6000 && a.C <= 256) return false;
     return a.T <= 32 && (a.B >= 128 || a.C <= 2048);
 }
 
