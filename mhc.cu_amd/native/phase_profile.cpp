@@ -1,7 +1,6 @@
-// Prints the in-kernel phase timeline of the fused forward kernel and of the slab backward kernel.
+// Prints the in-kernel phase timelines of the forward kernels and of the backward kernels that ran.
 //
 //   phase_profile [--batch B] [--hidden C] [--expansion n]          (C % 8 == 0, bf16;
-//                                                                    n > 4: projection backward instead of the slab kernel;
 //                                                                    n > 8: the two coefficient kernels only)
 //
 // Links libmhc_hip_profile.so (python mhc.cu_amd/build.py --profile), the build of the library with
@@ -44,6 +43,15 @@ static bool phase_slot_used(int kernel) {
     std::vector<unsigned long long> t(8 * 8);
     if (mhc_phase_read(kernel, t.data(), 8) != 0) return false;
     return std::any_of(t.begin(), t.end(), [](unsigned long long v) { return v != 0; });
+}
+
+// Workgroups of a kernel's grid that left stamps (how many a launch has is the library's choice).
+static int phase_workgroups(int kernel) {
+    std::vector<unsigned long long> t(4096 * 8);
+    if (mhc_phase_read(kernel, t.data(), 4096) != 0) return 1;
+    int w = 0;
+    while (w < 4096 && std::any_of(t.begin() + w * 8, t.begin() + w * 8 + 8, [](unsigned long long v) { return v != 0; })) w++;
+    return std::max(w, 1);
 }
 
 static void summary(const char *title, int kernel, int wgs, const std::vector<const char *> &names, bool stamps) {
@@ -133,11 +141,11 @@ int main(int argc, char **argv) {
                 {"start, first chunk requested", "waits for chunks, parks (all chunks)", "fragments, matrix cores (all chunks)",
                  "cross-wave sum, partial stores"}, false);
     }
-    // Which backward ran shows in the stamps: the tiled path leaves the slab (n <= 4) or the projection-backward
+    // Which backward ran shows in the stamps: the tiled path leaves the slab or the projection-backward
     // table, the two-launch path neither.  Both use slots 4 and 5, for different kernels.
-    const bool tiled = phase_slot_used(n > 4 ? 2 : 1);
+    const bool slab = phase_slot_used(1), tiled = slab || phase_slot_used(2);
     if (tiled) {
-        summary("channel sums + coefficient backward kernel, one workgroup per sample", 4, std::min(B, 4096),
+        summary("channel sums + coefficient backward kernel, one workgroup per sample (n <= 4, large batches: per three or four)", 4, phase_workgroups(4),
                 {"start: coefficient inputs, Sinkhorn state (wave 0)", "streaming loop (wave 0's steps)",
                  "workgroup sums", "coefficient backward (all of it: the three lines below)",
                  "  channel-sum vectors, dHpre / dHpost", "  Sinkhorn reverse sweep", "  dt / dP stores, alpha sums"}, false);
@@ -156,7 +164,7 @@ int main(int argc, char **argv) {
                  "epilogue: dx completed and stored, next loads requested (all)", "dphi summed over the waves and stored"}, false);
         return 0;
     }
-    if (n > 4) {
+    if (!slab) {
         summary("dx kernel (generic, one wave per workgroup)", 5, std::min(B * ((C / 4 + 63) / 64), 4096),
                 {"start: coefficients and all loads requested", "data arrives, df / a / da", "mixing, dx stores issued", "dw / dt partial sums"}, false);
         summary("projection backward kernel, one workgroup per 32 columns of x_flat", 2, std::min((int)(nC / 32), 4096),
@@ -164,8 +172,7 @@ int main(int argc, char **argv) {
                  "fragments, dphi on the matrix cores (all)", "dxflat on the matrix cores, stores (all)", "dphi stores"}, false);
         return 0;
     }
-    const int width = n == 4 && (long long)B * n * C < 12000000 ? 64 : 128, slabs = (C + width - 1) / width;
-    summary("slab backward kernel, one workgroup per (64 or 128 channels, batch split), its first mixer", 1, std::min(slabs * 4, 4096),
+    summary("slab backward kernel, one workgroup per (64 or 128 channels, batch split), its first mixer", 1, phase_workgroups(1),
             {"prologue (phi slab, first loads)", "barriers: tile on its way, other waves (all)",
              "dphi, dx, stores of the tile before (all)", "last dx, dphi partial stores", "epilogue: dw / dbias partial sums"}, false);
     return 0;

@@ -31,3 +31,13 @@ def test_native_parity_executable():
     print(p.stdout[-3000:])
     assert p.returncode == 0, p.stdout[-3000:] + p.stderr[-2000:]
     assert "all comparisons passed" in p.stdout
+
+
+# the tables follow the kernels that ran: the tiled backward of four and of eight streams, and the two-launch one
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,n,C,tiled", [(1280, 4, 512, True), (2000, 8, 1024, True), (64, 8, 512, False)])
+def test_phase_profile_names_the_kernels_that_ran(B, n, C, tiled):
+    exe = os.path.join(os.path.dirname(HERE), "mhc.cu_amd", "native", "phase_profile")
+    p = subprocess.run([exe, "--batch", str(B), "--hidden", str(C), "--expansion", str(n)], capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-2000:]
+    assert ("slab backward kernel" in p.stdout) == tiled and ("sample-resident backward kernel" in p.stdout) != tiled, p.stdout
