@@ -28,7 +28,7 @@ def _run(dyn, x, dy, p, T, eps, out_dtype):
 
 @pytest.mark.parametrize("B,n,C,dyn,bf16", [
     (220000, 4, 2560, True, True),     # fused forward, channel-sum and slab kernels
-    (110000, 8, 2560, True, True),     # 8 x 8 coefficients, matrix-core projection backward + dx kernel
+    (110000, 8, 2560, True, True),     # 8 x 8 coefficients: channel sums and the slab kernel of five to eight streams
     (40000, 32, 2048, True, True),     # workgroup-wide Sinkhorn, wide projection kernels
     (140000, 4, 4096, False, False),   # static H, float32
 ])

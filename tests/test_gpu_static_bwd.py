@@ -16,11 +16,13 @@ pytestmark = pytest.mark.gpu
 K_SPG, T_ITERS, EPS = 6, 20, 1e-6
 
 
+# (rounds 0: as the library chooses, above its lines, cut workgroups and chunks among them.)
 # waves per workgroup: 2 (n <= 4, C <= 256), 4, 8 (C > 2560; n > 4: C > 1024); 3 samples make a last round that is not full
 @pytest.mark.parametrize("B,n,C,rounds", [(2, 4, 8, 2), (7, 3, 256, 3), (5, 1, 264, 2), (9, 2, 513, 4), (33, 4, 1024, 5), (20, 4, 1288, 3),
                                           (11, 4, 2048, 4), (13, 4, 2560, 6), (10, 3, 2555, 3), (7, 4, 2568, 2), (6, 2, 4096, 5),
                                           (5, 4, 3333, 2), (9, 8, 64, 3), (12, 5, 520, 4), (10, 7, 1023, 3), (7, 8, 1032, 2),
-                                          (9, 6, 2048, 4), (5, 8, 2056, 2), (6, 5, 3080, 3), (5, 8, 4093, 2), (4, 8, 4096, 4)])
+                                          (9, 6, 2048, 4), (5, 8, 2056, 2), (6, 5, 3080, 3), (5, 8, 4093, 2), (4, 8, 4096, 4),
+                                          (4101, 2, 72, 0), (3073, 4, 264, 0), (515, 4, 2568, 0), (2051, 8, 520, 0), (769, 5, 3080, 0)])
 @pytest.mark.parametrize("inject", [False, True])
 @pytest.mark.parametrize("w_f32", [False, True])
 def test_one_and_several_samples_per_workgroup(B, n, C, rounds, inject, w_f32):
