@@ -689,7 +689,9 @@ static hipError_t launch_mfma(const void *x, const void *phi, float *Ppart, floa
     const int groups = (DP / 32 + NT - 1) / NT;
     constexpr int kChunk = EXACT ? 32 : 64;
     if constexpr (NT <= 3 && !RAG && NW == 4) {
-        if (narrow_waves(tiles_s * KS * groups, KS, nC, kChunk) == 8)
+        // (n <= 8: counted without the groups.  Row tiles in workgroups of their own (narrow_nt) add up in the same order as all
+        // in one; four waves, whose chains are twice as long, are off by 14 to 28 % more in float32 and 2 to 8 % in bf16, for 0 to 10 % of time)
+        if (narrow_waves(tiles_s * KS * (DP <= 96 ? 1 : groups), KS, nC, kChunk) == 8)
             return launch_mfma<NT, XF32, PF32, EXACT, RAG, 8>(x, phi, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);
     }
     const int sub = round_up((nC + KS * NW - 1) / (KS * NW), kChunk);  // whole chunks: 128-byte lines
@@ -732,12 +734,16 @@ bool proj_fwd_gathers(const ParamGather &g, int x_dtype, int B, int n, int C) {
 
 // Row tiles of phi per workgroup of the narrow kernel, n = 5 .. 8: one, in as many groups, where all of them (two or three) would
 // leave the chip few workgroups that each walk three times the bytes, and while reading x once per group costs less than that.
-// Forward us, all tiles -> one: n=8 B=1 C=4096 14.8 -> 12.3, 16 2560 15.2 -> 12.8, 64 1280 12.7 -> 11.1, 100 2560 16.0 -> 14.0, 1000 1280
-// (20 MB of x) 23.2 -> 22.4; n=6 B=32 C=1024 11.4 -> 10.7; n=5 B=10 C=777 13.7 -> 12.8; float32 n=8 B=16 C=2560 23.6 -> 16.2, 500 1280
-// (20 MB) 28.1 -> 25.8.  Beyond: n=6 B=2000 C=1024 (25 MB) 20.6 -> 21.3, n=8 B=700 C=2560 (29 MB) 26.3 -> 27.7, 2000 2560 54.9 -> 70.2.
+// Forward us, all tiles -> one: n=8 B=1 C=4096 14.8 -> 12.3, 16 2560 15.2 -> 12.8, 100 1280 12.9 -> 11.4, 100 2560 15.9 -> 14.5, 150 4096
+// 17.1 -> 15.9, 600 512 13.7 -> 12.9; n=6 B=32 C=1024 11.4 -> 10.7; n=5 B=10 C=777 13.7 -> 12.8; float32 n=8 B=16 C=2560 23.6 -> 16.2,
+// 100 1280 20.1 -> 17.3, 100 2560 25.1 -> 21.0, 150 4096 30.5 -> 26.1.  Beyond: n=6 B=2000 C=1024 (25 MB) 20.6 -> 21.3, n=8 B=700 C=2560
+// (29 MB) 26.3 -> 27.7, 2000 2560 54.9 -> 70.2.
 static int narrow_nt(int x_dtype, int B, int n, int C, int KS) {
-    const int tiles = mfma_nt(n);
-    const bool few = (B + 31) / 32 * KS * tiles <= 1024 && (size_t)B * n * C * (x_dtype == kBF16 ? 2 : 4) <= (22u << 20);
+    const int tiles = mfma_nt(n), wgs = (B + 31) / 32 * KS;
+    // (eight waves: 74 KB of LDS, two workgroups per CU; n=8, all tiles -> one: float32 B=600 C=512 20.6 -> 21.5, B=512 C=1024
+    // 22.2 -> 24.3, bf16 B=800 C=512 14.0 -> 15.3)
+    const int most = narrow_waves(wgs, KS, n * C, x_dtype == kF32 ? 32 : 64) == 8 ? 512 : 1024;
+    const bool few = wgs * tiles <= most && (size_t)B * n * C * (x_dtype == kBF16 ? 2 : 4) <= (22u << 20);
     return n <= 8 && few ? 1 : tiles;
 }
 

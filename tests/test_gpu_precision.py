@@ -141,6 +141,20 @@ def test_float32_slab_sums_stay_in_float64(B, n, C):
     _close_to_float64(*_batch_and_single_sums(B, n, C, torch.float32))
 
 
+# Row tiles of phi in workgroups of their own: the sums that eight waves form.  Four waves with chains twice as long were off by
+# 2.2e-7 and 2.0e-7 in these shapes, eight are by 1.73e-7 and 1.74e-7 (seeds scatter by 1e-9).
+@pytest.mark.parametrize("B,n,C,most", [(600, 6, 1024, 1.95e-7), (100, 8, 1280, 1.86e-7)])
+def test_float32_projection_in_row_groups(B, n, C, most):
+    import bench
+
+    st = bench.Step(dict(kind="dynamic", B=B, n=n, C=C, dtype="f32", bwd=False), "L", torch)
+    st.forward()
+    x, p = st.host["x"].double().reshape(B, -1), st.host["p"]
+    phi = torch.cat([p["phi_pre"], p["phi_post"], p["phi_res"]]).double()
+    want = x @ phi.T / (x.square().mean(1, keepdim=True) + bench.EPS).sqrt()
+    assert rel2(st.P.cpu(), want) <= most, rel2(st.P.cpu(), want)
+
+
 # n = 4: a sum of six terms and a product of depth 24, about 9e-8; with every step of the product rounded at the size of
 # dx 1.5e-7
 @pytest.mark.parametrize("B,n,C", [(65, 4, 128), (40, 4, 514), (100, 3, 66)])
