@@ -80,8 +80,8 @@ template <bool ANY> struct Act8<true, ANY> {
 };
 
 // bwd_resident_dxp_f32() in terms of the instantiation that serves a shape (launch_items below)
-template <int NP, int ITEMS, bool F32, bool STATIC, int TWV, bool RAG> constexpr bool res_dxp_f32() {
-    return !F32 && !STATIC && (RAG || (TWV == kResLongWaves && ITEMS >= 3) || (NP == 8 && TWV <= kResTileWaves));
+template <int NP, int ITEMS, bool F32, bool STATIC, int TWV, bool RAG, bool FINE> constexpr bool res_dxp_f32() {
+    return !F32 && !STATIC && (RAG || FINE || (TWV == kResLongWaves && ITEMS >= 3) || (NP == 8 && TWV <= kResTileWaves));
 }
 
 // F32: dy, x (and an injected f) are stored as fp32 and rounded to bf16 as they are loaded; dxp and df
@@ -90,10 +90,11 @@ template <int NP, int ITEMS, bool F32, bool STATIC, int TWV, bool RAG> constexpr
 // the complete dx; wave 0 only turns the sums into the sample's row of raw coefficient gradients
 // (dM | dHpre | dHpost), whose batch sum feeds the one Sinkhorn backward of the static layer.
 // RAG: rows of any length (C % 8 != 0): the last chunk of a row is loaded from C - 8 on and shifted down.
-template <int NP, int WMODE, int ITEMS, bool F32, bool STATIC = false, int TWV = kResTileWaves, bool RAG = false>
+// FINE: dxp in fp32 where the other instantiation of the shape leaves it in bf16.
+template <int NP, int WMODE, int ITEMS, bool F32, bool STATIC = false, int TWV = kResTileWaves, bool RAG = false, bool FINE = false>
 __global__ __launch_bounds__(64 * (TWV + (STATIC ? 0 : 1)), kMfmaMinWaves) void bwd_resident_kernel(BwdResidentArgs ra) {
     using TS = typename std::conditional<F32, float, bf16_t>::type;  // storage type of the activations
-    constexpr bool X32 = res_dxp_f32<NP, ITEMS, F32, STATIC, TWV, RAG>();
+    constexpr bool X32 = res_dxp_f32<NP, ITEMS, F32, STATIC, TWV, RAG, FINE>();
     using TD = typename std::conditional<X32, float, TS>::type;      // of dxp
     static_assert(NP == 4 || NP == 8, "stream groups of four");
     using SK = SkSmall<NP>;
@@ -488,7 +489,7 @@ bool bwd_resident_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int 
     return io && phi_dtype == kBF16 && n <= 8 && C <= kResMaxC && (C % 8 == 0 || (C > 8 && x_dtype == kBF16)) && T <= 32;
 }
 
-template <int NP, int WMODE, bool F32, bool STATIC, int TW, bool RAG = false>
+template <int NP, int WMODE, bool F32, bool STATIC, int TW, bool RAG = false, bool FINE = false>
 static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream) {
     using SK = SkSmall<NP>;
     using CB = CoefBwdSmall<NP, false, true, STATIC, RAG>;
@@ -505,9 +506,9 @@ static hipError_t launch_items_tw(const BwdResidentArgs &ra, hipStream_t stream)
 #define MHC_RES_ITEMS(N)                                                                              \
     case N:                                                                                           \
         if constexpr (N >= kMinItems && N <= kMaxItems && !(RAG && N == 4)) {                         \
-            if (!F32 && !STATIC && res_dxp_f32<NP, N, F32, STATIC, TW, RAG>() != bwd_resident_dxp_f32(ra.r.n, ra.r.C)) \
+            if (!F32 && !STATIC && res_dxp_f32<NP, N, F32, STATIC, TW, RAG, FINE>() != bwd_resident_dxp_f32(ra.r.B, ra.r.n, ra.r.C)) \
                 return hipErrorInvalidValue; /* not reached */                                        \
-            bwd_resident_kernel<NP, WMODE, N, F32, STATIC, TW, RAG><<<grid, threads, smem, stream>>>(ra); \
+            bwd_resident_kernel<NP, WMODE, N, F32, STATIC, TW, RAG, FINE><<<grid, threads, smem, stream>>>(ra); \
             return hipGetLastError();                                                                 \
         }                                                                                             \
         return hipErrorInvalidValue
@@ -543,7 +544,11 @@ static hipError_t launch_items(const BwdResidentArgs &ra, hipStream_t stream) {
         if (C > 512) return launch_items_tw<NP, WMODE, F32, STATIC, kResLongWaves>(ra, stream);
     }
     if constexpr (NP == 4) {
-        if (ra.r.C <= 256) return launch_items_tw<NP, WMODE, F32, STATIC, 2>(ra, stream);
+        if (ra.r.C <= 256) {
+            if constexpr (!F32 && !STATIC)
+                if (bwd_resident_dxp_f32(ra.r.B, ra.r.n, ra.r.C)) return launch_items_tw<NP, WMODE, F32, STATIC, 2, false, true>(ra, stream);
+            return launch_items_tw<NP, WMODE, F32, STATIC, 2>(ra, stream);
+        }
     }
     // Four streams: a fifth tile wave where it saves every wave an item (rows of 513..640 and 1025..1280
     // channels: ten 128-channel chunks are 3 + 3 + 2 + 2 on four waves, 2 each on five).  B=320, C=1280,

@@ -70,18 +70,21 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 // large enough to fill the chip with batch splits; the fewer streams, the fewer slabs.
 // Measured, backward in graphs of ten, tiled (Gram + slab) path | resident path (us), in each row from below the line to above it
 // (a step of the tiled path's tile counts moves single rows by a few us either way):
-//   n=1 C=128:  B=844 18.0 | 19.8, 1304 17.5 | 21.1;  C=256: 652 18.8 | 17.8, 920 16.4 | 17.8;  C=384: 672 15.4 | 14.9, 816 18.6 | 19.9
+//   n=1 C=128:  B=850 17.1 | 18.4, 1500 16.7 | 23.2, 2000 19.5 | 17.5, 2800 18.9 | 20.4;  C=256: 652 18.8 | 17.8, 850 17.8 | 19.0,
+//               1500 17.8 | 24.9, 2000 21.2 | 19.0, 2800 20.8 | 22.6;  C=384: 672 15.4 | 14.9, 816 18.6 | 19.9
 //       C=1024: 528 18.9 | 17.5, 904 20.8 | 23.9;  C=1920: 332 18.3 | 15.7, 480 15.0 | 16.2;  C=3200: 188 14.7 | 13.9, 268 19.1 | 19.5
-//   n=2 C=128:  2148 25.6 | 25.3, 2608 22.3 | 24.3;  C=256: 844 20.7 | 20.7, 1304 20.5 | 23.0, 1840 23.2 | 22.4, 2764 24.2 | 25.5
-//       C=384:  672 16.8 | 15.4, 960 17.2 | 19.0;  C=1280: 528 20.6 | 19.2, 624 20.8 | 21.4;  C=1920: 352 16.0 | 14.8, 416 16.4 | 17.0
-//       C=3200: 212 17.8 | 17.0, 248 17.0 | 18.4;  C=4096: 120 18.6 | 13.7, 188 16.7 | 19.2
-//   n=3 C=128:  3224 25.5 | 23.9, 4608 27.5 | 29.5;  C=256: 1956 28.4 | 24.8, 2764 26.7 | 27.8;  C=384: 816 22.3 | 20.3, 1152 22.0 | 22.6
+//   n=2 C=128:  850 19.2 | 19.0, 1000 21.3 | 21.7, 1500 19.5 | 24.2, 2800 22.5 | 21.7, 3700 23.7 | 25.1;  C=256: 850 19.6 | 19.6,
+//               1000 21.6 | 22.3, 1500 19.8 | 25.7, 2000 23.2 | 20.0, 2800 23.3 | 24.7;  C=384: 672 16.8 | 15.4, 960 17.2 | 19.0
+//       C=1280: 528 20.6 | 19.2, 624 20.8 | 21.4;  C=1920: 352 16.0 | 14.8, 416 16.4 | 17.0;  C=3200: 212 17.8 | 17.0, 248
+//               17.0 | 18.4;  C=4096: 120 18.6 | 13.7, 188 16.7 | 19.2
+//   n=3 C=128:  1000 23.4 | 22.2, 1500 21.7 | 24.8, 2800 24.8 | 22.9, 3700 26.1 | 26.5;  C=256: 1200 24.0 | 24.2, 1500 21.9 | 27.2,
+//               2000 25.5 | 22.0, 2800 26.2 | 27.1;  C=384: 672 19.1 | 15.7, 816 22.3 | 20.3 (rounded twice), 1152 22.0 | 22.6
 //       C=1280: 568 21.8 | 21.1, 812 25.6 | 27.9;  C=1920: 376 20.4 | 18.2, 540 22.9 | 24.2;  C=3200: 224 19.0 | 18.6, 276 22.7 | 24.6
 //       C=4096: 176 22.0 | 20.2, 320 22.2 | 29.8
-//   n=4 C=128:  3376 26.4 | 26.5, 4300 29.4 | 31.1;  C=256: 2148 28.6 | 27.5, 2608 26.2 | 27.2, 4452 33.5 | 35.7;  C=264: 816 22.0 | 19.5,
-//               1152 22.9 | 22.0, 1392 25.3 | 26.1;  C=320: 816 21.9 | 19.9, 960 19.8 | 19.8, 1392 25.9 | 27.5;  C=384: 816 21.7 | 20.4,
-//               960 19.7 | 20.6, 1392 25.6 | 29.0 (the step at 256 channels: up to there a workgroup of the resident path has
-//               two tile waves instead of four, and more workgroups fit a CU)
+//   n=4 C=128:  1000 22.1 | 21.2, 1500 21.1 | 24.9, 2800 24.1 | 23.2, 3700 26.6 | 26.6, 4300 29.4 | 31.1;  C=256: 1200 23.5 | 24.0, 1500
+//               21.9 | 27.4, 2000 25.5 | 23.1, 2800 26.2 | 26.8;  C=264: 672 19.2 | 15.4, 816 22.0 | 19.5 (rounded twice), 1152
+//               22.9 | 22.0, 1392 25.3 | 26.1;  C=384: 816 21.7 | 20.4, 960 19.7 | 20.6 (the step at 256 channels: up to there a
+//               workgroup of the resident path has two tile waves instead of four, and more workgroups fit a CU)
 //       C=1024: 744 25.0 | 22.4, 876 24.6 | 25.9;  C=1280: 596 23.2 | 22.8, 700 21.7 | 24.0;  C=1920: 396 24.3 | 22.1, 468 22.9 | 23.7
 //       C=2560: 296 26.4 | 24.9, 348 22.7 | 24.8;  C=3200: 224 22.7 | 21.5, 320 24.0 | 26.6;  C=4096: 176 25.5 | 22.0, 272 27.8 | 31.9
 // n = 5 .. 8, where the slab is bwd_slab8.hip:
@@ -102,9 +105,13 @@ bool bwd_resident_preferred(int B, int n, int C) {
         const int per_row[4] = {520'000, 640'000, 760'000, 720'000}, least[4] = {224, 256, 256, 448}, most[4] = {640, 640, 896, 3000};
         return B <= std::min(most[n - 5], std::max(least[n - 5], per_row[n - 5] / C));
     }
-    const int upto128[4] = {768, 2176, 3968, 3840}, upto256[4] = {768, 1088, 2304, 2304};
-    if (C <= 256) return B <= (C <= 128 ? upto128 : upto256)[n - 1];
-    const int per_row[4] = {640'000, 680'000, 760'000, 780'000}, most[4] = {768, 704, 832, 832};
+    if (C <= 256) {
+        // up to 1536 samples one workgroup of the second launch walks all of them, beyond the batch is split
+        const int walk[4] = {768, 896, 1216, 1216}, upto128[4] = {2432, 3200, 3968, 3840}, upto256[4] = {2432, 2432, 2432, 2432};
+        return B <= (B <= 1536 ? walk : (C <= 128 ? upto128 : upto256))[n - 1];
+    }
+    // (never beyond kResTwiceMaxB samples where dxp is handed over in bf16: dx would be rounded twice, on the tiled path once)
+    const int per_row[4] = {640'000, 680'000, 760'000, 780'000}, most[4] = {768, 704, 768, 768};
     return B <= std::min(most[n - 1], per_row[n - 1] / C);
 }
 
@@ -174,7 +181,7 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
 #else
     const bool resident = n <= 8 && C <= kResMaxC && (bwd_resident_preferred(B, n, C) || C % 8 != 0);
 #endif
-    w.dxp = c.floats(resident && bwd_resident_dxp_f32(n, C) ? (size_t)B * nC : 0);
+    w.dxp = c.floats(resident && bwd_resident_dxp_f32(B, n, C) ? (size_t)B * nC : 0);
     int bs = dphi_batch_splits(B, n, C);
     const int bs2 = proj_bwd_batch_splits(B, n, C);
     if (bs2 > bs) bs = bs2;
@@ -671,7 +678,7 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         BwdCoefOut out2 = out;
         out2.dPb = ws.dPb;
         out2.dP = nullptr;  // the second launch takes dP as matrix-core operands only
-        float *dxp = x_dtype == kBF16 && bwd_resident_dxp_f32(n, C) ? ws.dxp : nullptr;
+        float *dxp = x_dtype == kBF16 && bwd_resident_dxp_f32(B, n, C) ? ws.dxp : nullptr;
         MHC_LAUNCH(launch_bwd_resident(dy, x, x_dtype, w, w_dtype, f_inject, H_pre, H_post, M, q, P, r, alpha, bias + 2 * n,
                                        sk_state, out2, dxp ? dxp : dx, df, ws.u, B, n, C, iters, eps, st));
         const DwOut dwo = f_inject ? DwOut{} : dw;

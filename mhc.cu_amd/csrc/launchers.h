@@ -240,14 +240,18 @@ hipError_t launch_proj_bwd_mfma(const void *x, const void *phi, const void *dPb,
 // outputs of launch_mix_bwd_reduce) and dxp = M^T dy + Hpre (x) da from ONE pass over dy and x, one
 // workgroup per sample; u [B, C] = the samples' summands of dw, df with an injected f.
 bool bwd_resident_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C, int T);
-constexpr int kResShortMaxC = 512, kResWholeMaxC = 2560, kResMaxC = 4096;
+constexpr int kResTwiceMaxB = 768, kResShortMaxC = 512, kResWholeMaxC = 2560, kResMaxC = 4096;
 // bf16 storage: whether dxp goes to the second launch in fp32 (a buffer [B, n, C] of its own) instead of bf16 in dx.
 // dx is then rounded once and its error against float64 is that of the tiled kernels, which would serve these
 // shapes otherwise (1.66e-3 relative); handed over in bf16 it is rounded twice (2.35e-3).
 // The price is 4 bytes per element (backward us, tiled | handed over in bf16 | in fp32): n=4 C=2880 B=256 27.6 | 19.2 |
 // 21.6; n=8 C=4096 B=100 45.5 | 32.1 | 32.9; n=8 C=3072 B=1000 128.9 | 102.9 | 105.7; n=8 C=256 B=6000 113.4 | 66.8 |
-// 69.2, B=600 29.9 | 22.6 | 23.3.  Rows of 513 .. 2560 channels (n <= 4: up to 2560) keep the bf16 hand-over.
-inline bool bwd_resident_dxp_f32(int n, int C) { return C % 8 != 0 || C > kResWholeMaxC || (n > 4 && C <= kResShortMaxC); }
+// 69.2, B=600 29.9 | 22.6 | 23.3; n=4 C=128 B=1000 22.1 | 21.5 | 21.2, B=2800 24.1 | 23.3 | 23.2; n=4 C=256 B=2000 25.5 | 22.5 | 23.1.
+// Rows of 513 .. 2560 channels keep the bf16 hand-over, n <= 4 up to 2560 channels and 768 samples (bwd_resident_preferred()
+// sends no larger batch of them there).
+inline bool bwd_resident_dxp_f32(int B, int n, int C) {
+    return C % 8 != 0 || C > kResWholeMaxC || (n > 4 ? C <= kResShortMaxC : C <= 256 && B > kResTwiceMaxB);
+}
 hipError_t launch_bwd_resident(const void *dy, const void *x, int x_dtype, const void *w, int w_dtype, const void *f_inject,
                                const float *Hpre, const float *Hpost, const float *M, const float *q,
                                const float *P, const float *r, const float *alpha, const float *b_res,
