@@ -68,41 +68,42 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 // Whether the sample-resident backward (bwd_resident.hip + the column-slab kernel) is taken where it is
 // supported.  Its second launch walks all samples of a column slab in one workgroup, which stops paying once the batch is
 // large enough to fill the chip with batch splits; the fewer streams, the fewer slabs.
-// Measured, backward in graphs of ten, tiled (Gram + slab) path | resident path (us), in each row from below the line to above it
-// (a step of the tiled path's tile counts moves single rows by a few us either way):
+// Measured, backward in graphs of ten, tiled (Gram + slab) path | resident path (us), in each row from below the line to above it.
+// Single rows jump by a few us with B mod 32 and the tiles per split; the lines are fitted to 1500 shapes of all remainders.
 //   n=1 C=128:  B=850 17.1 | 18.4, 1500 16.7 | 23.2, 2000 19.5 | 17.5, 2800 18.9 | 20.4;  C=256: 652 18.8 | 17.8, 850 17.8 | 19.0,
-//               1500 17.8 | 24.9, 2000 21.2 | 19.0, 2800 20.8 | 22.6;  C=384: 672 15.4 | 14.9, 816 18.6 | 19.9
-//       C=1024: 528 18.9 | 17.5, 904 20.8 | 23.9;  C=1920: 332 18.3 | 15.7, 480 15.0 | 16.2;  C=3200: 188 14.7 | 13.9, 268 19.1 | 19.5
+//               1500 17.8 | 24.9, 2000 21.2 | 19.0, 2800 20.8 | 22.6;  C=640: 559 18.9 | 17.5, 671 15.7 | 16.0
+//       C=1280: 437 17.3 | 15.6, 614 20.9 | 22.4;  C=1920: 354 20.6 | 18.0, 543 17.2 | 20.2;  C=3200: 206 17.9 | 15.7, 300 19.3 | 19.8
 //   n=2 C=128:  850 19.2 | 19.0, 1000 21.3 | 21.7, 1500 19.5 | 24.2, 2800 22.5 | 21.7, 3700 23.7 | 25.1;  C=256: 850 19.6 | 19.6,
-//               1000 21.6 | 22.3, 1500 19.8 | 25.7, 2000 23.2 | 20.0, 2800 23.3 | 24.7;  C=384: 672 16.8 | 15.4, 960 17.2 | 19.0
-//       C=1280: 528 20.6 | 19.2, 624 20.8 | 21.4;  C=1920: 352 16.0 | 14.8, 416 16.4 | 17.0;  C=3200: 212 17.8 | 17.0, 248
-//               17.0 | 18.4;  C=4096: 120 18.6 | 13.7, 188 16.7 | 19.2
+//               1000 21.6 | 22.3, 1500 19.8 | 25.7, 2000 23.2 | 20.0, 2800 23.3 | 24.7;  C=384: 676 22.5 | 19.9, 960 17.2 | 19.0
+//       C=1280: 495 19.9 | 17.3, 659 19.9 | 21.3;  C=1920: 354 21.9 | 18.2, 447 16.5 | 17.4;  C=3200: 212 17.9 | 16.9, 265 21.3 | 23.0
+//       C=4096: 172 20.0 | 19.0, 212 18.5 | 20.1
 //   n=3 C=128:  1000 23.4 | 22.2, 1500 21.7 | 24.8, 2800 24.8 | 22.9, 3700 26.1 | 26.5;  C=256: 1200 24.0 | 24.2, 1500 21.9 | 27.2,
-//               2000 25.5 | 22.0, 2800 26.2 | 27.1;  C=384: 672 19.1 | 15.7, 816 22.3 | 20.3 (rounded twice), 1152 22.0 | 22.6
-//       C=1280: 568 21.8 | 21.1, 812 25.6 | 27.9;  C=1920: 376 20.4 | 18.2, 540 22.9 | 24.2;  C=3200: 224 19.0 | 18.6, 276 22.7 | 24.6
-//       C=4096: 176 22.0 | 20.2, 320 22.2 | 29.8
+//               2000 25.5 | 22.0, 2800 26.2 | 27.1;  C=384: 721 22.0 | 17.7, 816 22.3 | 20.3 (rounded twice), 1152 22.0 | 22.6
+//       C=1280: 593 23.5 | 21.7, 764 21.7 | 23.2;  C=1920: 472 21.0 | 19.7, 577 27.6 | 27.3, 700 22.2 | 24.5;  C=2560: 310 21.3 | 22.7,
+//               444 21.6 | 25.1;  C=4096: 242 23.4 | 22.3, 266 27.0 | 30.4
 //   n=4 C=128:  1000 22.1 | 21.2, 1500 21.1 | 24.9, 2800 24.1 | 23.2, 3700 26.6 | 26.6, 4300 29.4 | 31.1;  C=256: 1200 23.5 | 24.0, 1500
-//               21.9 | 27.4, 2000 25.5 | 23.1, 2800 26.2 | 26.8;  C=264: 672 19.2 | 15.4, 816 22.0 | 19.5 (rounded twice), 1152
+//               21.9 | 27.4, 2000 25.5 | 23.1, 2800 26.2 | 26.8;  C=264: 687 21.9 | 17.2, 816 22.0 | 19.5 (rounded twice), 1152
 //               22.9 | 22.0, 1392 25.3 | 26.1;  C=384: 816 21.7 | 20.4, 960 19.7 | 20.6 (the step at 256 channels: up to there a
 //               workgroup of the resident path has two tile waves instead of four, and more workgroups fit a CU)
-//       C=1024: 744 25.0 | 22.4, 876 24.6 | 25.9;  C=1280: 596 23.2 | 22.8, 700 21.7 | 24.0;  C=1920: 396 24.3 | 22.1, 468 22.9 | 23.7
-//       C=2560: 296 26.4 | 24.9, 348 22.7 | 24.8;  C=3200: 224 22.7 | 21.5, 320 24.0 | 26.6;  C=4096: 176 25.5 | 22.0, 272 27.8 | 31.9
+//       C=1280: 473 21.0 | 18.1, 624 24.2 | 23.6, 729 22.3 | 24.1;  C=1920: 424 25.0 | 22.9, 489 24.6 | 24.4, 611 28.2 | 30.7
+//       C=2560: 331 25.8 | 24.7, 450 27.9 | 29.2;  C=3200: 247 23.6 | 22.4, 364 27.7 | 28.4;  C=4096: 235 26.6 | 23.9, 270 28.0 | 31.8
+// (from about 2000 channels and five streams on, and 4096 and three, one workgroup of the resident path fills a CU: the step at 256)
 // n = 5 .. 8, where the slab is bwd_slab8.hip:
-//   n=5 C=256:  4000 48.7 | 47.3, 5800 63.4 | 67.8;  C=384: 596 25.7 | 24.2, 704 24.7 | 27.3;  C=768: 552 29.5 | 29.1, 780 30.0 | 35.5
-//       C=1280: 388 30.6 | 29.2, 564 29.7 | 34.7;  C=2560: 224 29.0 | 23.3, 320 29.6 | 35.2;  C=4096: 224 32.4 | 30.6, 272 37.4 | 46.2
-//   n=6 C=256:  5800 66.7 | 61.7;  C=384: 624 28.2 | 25.4, 760 27.9 | 29.0;  C=768: 624 30.1 | 29.1, 760 29.5 | 31.0;  C=1280: 488 33.2 |
-//               30.2, 576 31.4 | 35.2;  C=2560: 244 33.3 | 26.4, 312 34.9 | 36.6;  C=4096: 244 38.4 | 33.7, 312 41.4 | 48.3
-//   n=7 C=256:  6000 71.1 | 67.1, 8700 88.8 | 90.7;  C=384: 868 35.9 | 32.9, 1024 31.8 | 32.9, 1484 39.9 | 42.8;  C=768: 868 38.4 | 38.4,
-//               1228 44.1 | 48.0;  C=1280: 480 32.9 | 29.8, 684 39.6 | 42.6;  C=2560: 244 38.5 | 28.8, 312 40.0 | 41.0, 536 47.0 | 59.2
-//   n=8 C=256:  8000 91.2 | 84.7, 11600 118.4 | 117.5;  C=320: 2228 49.5 | 49.1, 2708 54.4 | 56.5;  C=512: 1392 46.9 | 45.6, 1692 48.7 |
-//               50.9;  C=1280: 556 43.7 | 43.4, 676 46.9 | 48.3;  C=2560: 408 49.1 | 47.8, 480 49.5 | 50.6;  C=4096: 336 61.1 | 57.0,
-//               408 62.0 | 64.2
+//   n=5 C=256:  4000 48.7 | 47.3, 5800 63.4 | 67.8;  C=384: 565 24.7 | 23.7, 655 26.8 | 26.9, 829 26.0 | 30.0;  C=1280: 382 25.9 | 25.1,
+//               518 31.4 | 36.7;  C=2560: 245 30.3 | 25.1, 273 30.8 | 35.0;  C=4096: 225 36.7 | 30.9, 291 39.6 | 46.9
+//   n=6 C=256:  5800 66.7 | 61.7;  C=384: 655 29.3 | 27.2, 765 27.3 | 29.0;  C=768: 647 32.8 | 32.0, 790 30.8 | 35.0;  C=1280: 472 29.9 |
+//               27.8, 527 33.5 | 36.1;  C=2560: 256 31.8 | 25.1, 307 35.4 | 36.4;  C=4096: 227 41.3 | 33.3, 291 44.7 | 48.9
+//   n=7 C=256:  6000 71.1 | 67.1, 8700 88.8 | 90.7;  C=384: 777 35.6 | 31.4, 1024 31.8 | 32.9, 1163 39.3 | 36.9;  C=768: 680 36.0 | 32.7,
+//               832 34.2 | 35.2, 1087 40.4 | 41.4;  C=1280: 455 37.4 | 32.3, 705 42.0 | 44.9;  C=2560: 361 42.7 | 41.7, 448 41.5 | 45.1
+//   n=8 C=256:  8000 91.2 | 84.7, 11600 118.4 | 117.5;  C=320: 2386 54.6 | 52.4, 2728 56.9 | 59.2;  C=512: 1406 46.0 | 44.1, 2095 55.2 |
+//               59.6;  C=1280: 569 43.5 | 42.0, 815 49.3 | 55.7;  C=2560: 387 52.5 | 49.6, 532 56.4 | 64.1;  C=4096: 344 60.8 | 58.2,
+//               539 73.1 | 85.6
 // Experiment hook: 1 = never, 2 = always.
 bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;
     if (n > 4) {
         if (C <= 256) return true;
-        const int per_row[4] = {520'000, 640'000, 760'000, 720'000}, least[4] = {224, 256, 256, 448}, most[4] = {640, 640, 896, 3000};
+        const int per_row[4] = {500'000, 680'000, 880'000, 940'000}, least[4] = {256, 256, 256, 448}, most[4] = {640, 704, 832, 2560};
         return B <= std::min(most[n - 5], std::max(least[n - 5], per_row[n - 5] / C));
     }
     if (C <= 256) {
@@ -111,8 +112,8 @@ bool bwd_resident_preferred(int B, int n, int C) {
         return B <= (B <= 1536 ? walk : (C <= 128 ? upto128 : upto256))[n - 1];
     }
     // (never beyond kResTwiceMaxB samples where dxp is handed over in bf16: dx would be rounded twice, on the tiled path once)
-    const int per_row[4] = {640'000, 680'000, 760'000, 780'000}, most[4] = {768, 704, 768, 768};
-    return B <= std::min(most[n - 1], per_row[n - 1] / C);
+    const int per_row[4] = {640'000, 740'000, 900'000, 860'000}, least[4] = {0, 0, 256, 256};
+    return B <= std::min(kResTwiceMaxB, std::max(least[n - 1], per_row[n - 1] / C));
 }
 
 // Shapes for which the dynamic entry points take fp32 activations that are consumed as bf16
