@@ -415,8 +415,19 @@ int bwd_static_rows(int B, int n, int C) {
 //               14.8 | 59.0 + 7.4, 3072 81.3 + 19.2 | 84.8 + 7.7;  C=2560: 2048 69.2 + 15.6 | 77.2 + 7.8, 3072 109.5 + 22.5 | 109.9 + 7.9;
 //               C=4096: 512 34.6 + 6.4 | 32.1 + 7.7, 1024 69.0 + 10.2 | 57.0 + 7.7
 //   n=6 C=1280 (ten chunks on eight waves): B=4096 71.6 + 15.6 | 87.3 + 8.0;  n=5 C=256: B=4096 27.4 + 12.4 | 33.4 + 8.7
+// Ragged rows are held in more chunks than they have (launch_static_items) and shifted down sample by sample; whole backward, one
+// sample per workgroup | this:
+//   n=4 C=333:  B=4150 31.2 | 36.9, 7000 47.1 | 48.9;  n=2 C=333: 4150 28.1 | 28.6, 7000 41.7 | 36.3;  n=4 C=777: 4150 45.9 | 45.6
+//   n=4 C=1283: 3080 55.1 | 86.1, 7000 110.7 | 161.8;  C=1789: 4150 97.6 | 100.9, 6000 137.9 | 127.6;  C=2555: 4150 113.0 | 116.4, 6000
+//               160.7 | 152.6;  C=2811: 520 41.0 | 31.2;  n=8 C=777: 2060 54.6 | 52.2;  C=2045: 3080 158.7 | 143.1;  C=2051: 3080 163.9 |
+//               177.8, 4000 202.5 | 218.5;  C=2555: 4000 232.1 | 244.9;  C=3069: 3080 293.6 | 215.9
 bool bwd_static_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneStaticSpg); hook > 0) return hook > 1 && B > 1;
+    if (C % 8 != 0) {
+        if (n <= 4 && C > 256 && C <= 512 && B < (n <= 2 ? 5000 : 9000)) return false;
+        if (n <= 4 && C > 1024 && C <= 2560) return C > 1536 && B >= 6000;
+        if (n > 4 && C > 2048 && C <= 2560) return false;
+    }
     if (n <= 4) return B >= (C > 2560 ? 512 : (C > 256 && C <= 1536 ? 3072 : 4096));
     if (C > 3072) return B >= 768;
     if (C > 1536) return B >= 3072;
