@@ -437,16 +437,29 @@ bool bwd_slab8_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) 
 
 int bwd_slab8_slabs(int C) { return (C + 63) / 64; }
 
-int bwd_slab8_batch_splits(int B, int C) {
+// At most one workgroup per CU and at least three tiles each, and within that the splits that cost least: a tile is some 0.2 n us
+// of a walk, and from two splits on their partial dphi are written, read and added up, D n C elements each, while a single one
+// leaves the result.  Backward us, one split | two | as many as the CUs (and tiles) allow:
+//   n=8 C=256  B=100 36.6 | 32.3 | 32.3 (2), 300 58.0 | 42.7 | 32.7 (6), 2000 two tiles each 50.3, three 47.3, four 47.1, seven 51.4
+//   n=8 C=2560 B=100 41.8 | 50.8 | 50.8 (2), 200 52.3 | 52.5 | 47.9 (4);  C=4104 100 46.2 | 57.7, 200 55.5 | 62.3 | 61.2 (3), 300 67.4 |
+//              69.0 | 66.6 (3);  C=8192 100 50.2 | 74.9, 300 77.0 | 92.5
+//   n=5 C=2560 B=100 33.6 | 32.3, 200 36.8 | 34.1 | 32.1 (4);  C=6144 100 35.2 | 40.9, 200 42.9 | 43.7, 300 51.7 | 48.4
+int bwd_slab8_batch_splits(int B, int n, int C) {
     const int slabs = bwd_slab8_slabs(C), tiles = (B - 1) / 16 + 1;
-    int S = tuning_get(kTuneSlabSplits);  // experiment hook
-    // one workgroup per CU, but at least three tiles each: a workgroup leaves its partial dphi behind however short its walk
-    // (backward us: B=2000 n=8 C=256 two tiles 50.3, three 47.3, four 47.1, seven 51.4)
-    if (S <= 0) S = std::max(1, std::min(256 / slabs, tiles / 3));
-    if (S > tiles) S = tiles;
+    const auto per_split = [&](int s) { return (tiles + s - 1) / s; };
+    int S = 1;
+    if (const int hook = tuning_get(kTuneSlabSplits); hook > 0) {  // experiment hook
+        S = std::min(hook, tiles);
+    } else {
+        const double part = 6.4e-6 * (n * n + 2 * n) * n * C;
+        double least = 0.2 * n * tiles;
+        for (int s = 2; s <= std::min(256 / slabs, tiles / 3); s++) {
+            const double us = 0.2 * n * per_split(s) + part * (0.7 + 0.15 * s);
+            if (us < least) { least = us; S = s; }
+        }
+    }
     // the longest split decides: the fewest splits that keep its tile count
-    const int tps = (tiles + S - 1) / S;
-    return (tiles + tps - 1) / tps;
+    return (tiles + per_split(S) - 1) / per_split(S);
 }
 
 hipError_t launch_bwd_slab8(const void *dy, const void *x, const void *w, int w_dtype, const void *f_inject, const void *phi,

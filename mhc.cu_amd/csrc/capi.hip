@@ -167,7 +167,7 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1, bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
     // (also where the resident path is preferred: it does not take more than 32 Sinkhorn iterations)
     const bool slab8 = n >= 5 && n <= 8 && C % 8 == 0;
-    const int bs7 = slab8 ? bwd_slab8_batch_splits(B, C) : 1;
+    const int bs7 = slab8 ? bwd_slab8_batch_splits(B, n, C) : 1;
     const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : (slab8 ? (size_t)bs7 * bwd_slab8_slabs(C) : 0), parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
     w.u = c.floats(std::max((size_t)B, 2 * (n <= 4 ? slab64 : (size_t)(slab8 ? bs7 : 0))) * C);
     w.upart = c.floats(2 * parts64 * C);
@@ -739,7 +739,7 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         return MHC_OK;
     }
     if (mfma && bwd_slab8_supported(x_dtype, y_dtype, phi_dtype, n, C) && tuning_get(kTuneSlab8) != 1) {
-        const int S = bwd_slab8_batch_splits(B, C);
+        const int S = bwd_slab8_batch_splits(B, n, C);
         MHC_LAUNCH(launch_bwd_slab8(dy, x, w, w_dtype, f_inject, phi, H_pre, H_post, M, q, out, dx, df,
                                     S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
                                     reinterpret_cast<double *>(ws.dtpart), S, B, n, C, st));

@@ -194,7 +194,7 @@ hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const voi
 // dt_part [S bwd_slab8_slabs()][D+3].
 bool bwd_slab8_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C);
 int bwd_slab8_slabs(int C);
-int bwd_slab8_batch_splits(int B, int C);
+int bwd_slab8_batch_splits(int B, int n, int C);
 hipError_t launch_bwd_slab8(const void *dy, const void *x, const void *w, int w_dtype, const void *f_inject, const void *phi,
                             const float *Hpre, const float *Hpost, const float *M, const float *q, const BwdCoefOut &co,
                             void *dx, void *df, float *dphi_part, double *dw_part, double *dt_part, int S, int B, int n, int C,
