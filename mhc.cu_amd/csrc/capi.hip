@@ -116,6 +116,18 @@ bool bwd_resident_preferred(int B, int n, int C) {
     return B <= std::min(kResTwiceMaxB, std::max(least[n - 1], per_row[n - 1] / C));
 }
 
+// Whether the tiled path of n = 5 .. 8 ends in the slab kernel or in the general ones.  Small batches of rows that the resident
+// path would hold get here with more than 32 Sinkhorn iterations only (backward us, general kernels | slab):
+//   n=5 C=1280 B=100 26.2 | 27.0, 170 28.8 | 26.6;  n=6 C=1280 100 26.5 | 30.1, 170 29.3 | 29.9, 300 34.4 | 32.8;  n=7 C=512 170 27.4 | 29.0,
+//   300 30.9 | 30.5, C=2560 100 36.4 | 37.2, 170 42.4 | 40.9;  n=8 C=512 300 31.8 | 36.1, 500 36.0 | 37.2, 700 36.7 | 36.1, C=1280
+//   170 32.9 | 41.6, 300 39.8 | 41.9, 500 47.9 | 41.5, C=2560 170 44.3 | 48.3, 300 56.3 |
+//   49.7, C=4096 100 43.1 | 44.5;  C=4608 64 40.0 | 35.7, 100 48.3 | 45.9
+bool bwd_slab8_preferred(int B, int n, int C) {
+    if (const int hook = tuning_get(kTuneSlab8)) return hook == 2;
+    const int least[4] = {112, 176, 208, C <= 1280 ? 400 : 208};
+    return C > kResWholeMaxC || B > least[n - 5];
+}
+
 // Shapes for which the dynamic entry points take fp32 activations that are consumed as bf16
 // (MHC_F32_AS_BF16): the kernels that load fp32 storage directly are the narrow projection, the fused
 // n <= 8 forward and the two launches of the sample-resident backward.  That backward is taken for fp32
@@ -738,7 +750,7 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
                                    ws.dphi_part, S, (size_t)D * n * C, dphi, st, true));
         return MHC_OK;
     }
-    if (mfma && bwd_slab8_supported(x_dtype, y_dtype, phi_dtype, n, C) && tuning_get(kTuneSlab8) != 1) {
+    if (mfma && bwd_slab8_supported(x_dtype, y_dtype, phi_dtype, n, C) && bwd_slab8_preferred(B, n, C)) {
         const int S = bwd_slab8_batch_splits(B, n, C);
         MHC_LAUNCH(launch_bwd_slab8(dy, x, w, w_dtype, f_inject, phi, H_pre, H_post, M, q, out, dx, df,
                                     S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),

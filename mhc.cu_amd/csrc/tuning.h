@@ -20,7 +20,7 @@ enum TuneKey {
     kTuneSpareB = 9,        // projection forward (matrix-core kernels): K splits, 0 = by heuristic
     kTuneGather = 10,       // projection reads the caller's fp32 parameters itself: 1 = never, 2 = whenever the shape allows
     kTuneSlabWidth = 11,    // slab backward (n <= 4, bf16): channels per workgroup, 1 = 64, 2 = 128, 0 = by size
-    kTuneSlab8 = 12,        // slab backward of n = 5 .. 8 behind the channel sums: 1 = never (general kernels)
+    kTuneSlab8 = 12,        // slab backward of n = 5 .. 8 behind the channel sums: 1 = never (general kernels), 2 = always
     kTuneCount = 13
 };
 

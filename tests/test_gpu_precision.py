@@ -126,8 +126,9 @@ def test_slab_sums_stay_in_float64(B, n, C, width, splits):
     from mhc._lib import tuning_lib
 
     lib = tuning_lib()
-    # the tiled path; one launch of channel sums and coefficient backward, as for one sample; slab width and splits
-    hooks = {7: 1, 2: 2, 11: width, 3: splits}
+    # the tiled path; one launch of channel sums and coefficient backward, as for one sample; the slab kernel (n = 5 .. 8) for one
+    # sample too; slab width and splits
+    hooks = {7: 1, 2: 2, 12: 2, 11: width, 3: splits}
     try:
         for k, v in hooks.items():
             assert lib.mhc_tuning_set(k, v) == 0
