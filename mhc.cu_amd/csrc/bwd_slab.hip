@@ -781,12 +781,18 @@ int bwd_slab_batch_splits(int B, int n, int C, int y_dtype) {
     // round (B=1280 C=2560, 12 splits of 20 slabs 37.4 us, 20 splits 45.1), fewer leave CUs idle (8 splits 40.2).
     int S = std::max(1, (staged ? 256 : 512) / slabs);
     if (S > tiles) S = tiles;
-    // Short rows: at least four tiles per split.  A split leaves its partial dphi behind however short its walk, and of few
-    // columns the finalize launch adds hundreds of copies up one after the other.  Backward us, as many splits as fit (one to
-    // three tiles each) | four tiles each: n=2 B=3300 C=64 39.0 | 28.2, n=4 B=6200 C=64 39.5 | 32.6, n=1 B=2000 C=256 26.7 | 21.3,
-    // n=3 B=1000 C=384 26.5 | 23.8, n=3 B=1300 C=384 29.0 | 24.5, n=4 B=1400 C=264 24.4 | 24.0, n=2 B=650 C=1280 22.2 | 21.9.
-    // Longer rows walk two tiles as well: n=2 B=450 C=1920 22.0 | 23.4, n=1 B=240 C=3200 17.4 | 18.5.
-    if (staged && slabs <= 10) S = std::min(S, (tiles + 3) / 4);
+    // Short rows: the splits that cost least, a tile being some 0.65 us of a walk and a copy of the partial dphi 0.09 us of the
+    // finalize launch, which adds up hundreds of copies of few columns one after the other.  Backward us, as many splits as fit
+    // (one to three tiles each) | four tiles each: n=2 B=3300 C=64 39.0 | 28.2, n=4 B=6200 C=64 39.5 | 32.6 (six: 31.3), n=1 B=2000 C=256
+    // 26.7 | 21.3, n=3 B=1000 C=384 26.5 | 23.8, n=3 B=1300 C=384 29.0 | 24.5, n=4 B=100 C=64 21.8 | 25.4, n=2 B=650 C=1280 22.2 | 21.9.
+    // Longer rows have few splits: n=2 B=450 C=1920 (two tiles each) 22.0 | 23.4, n=1 B=240 C=3200 17.4 | 18.5.
+    if (staged && slabs <= 10) {
+        const auto us = [&](int s) { return 0.65 * ((tiles + s - 1) / s) + 0.09 * s; };
+        int best = S;
+        for (int s = 1; s < S; s++)
+            if (us(s) < us(best)) best = s;
+        S = best;
+    }
     if (!staged) {
         // the dphi partial copies (written here, read once by the finalize launch) stay below 16 MB or
         // 0.4 of the activation bytes this kernel moves, whichever is larger
