@@ -394,8 +394,9 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32dy_kernel(BwdSlabArgs a) {
 //     also accumulated dphi held the barrier up (109 us).  Mixers (a wave per 16 channels) accumulate dphi, form dx and
 //     store it.
 // A period is one tile: one barrier, and nothing else between the waves.  CW channels per workgroup, one workgroup per CU.
-// Measured, n=4 B=8192 C=2560: 130 -> 98 us (503 MB, 5.1 TB/s); backward in graphs of ten: B=8192 C=2560 209 -> 174 us,
-// B=1280 C=2560 42.4 -> 37.4, B=2048 C=1280 41.0 -> 37.0, n=3 B=5000 C=1920 85.5 -> 71.0, n=2 B=3000 C=1024 37.8 -> 31.7.
+// Measured, n=4 B=8192 C=2560: 130 -> 94 us (503 MB, 5.3 TB/s); backward in graphs of ten, with the former kernel and channel
+// sums -> now: B=8192 C=2560 209 -> 164 us, B=1280 C=2560 42.4 -> 36.9, B=2048 C=1280 41.0 -> 33.1, n=3 B=5000 C=1920 86.7 ->
+// 68.4, n=2 B=3000 C=1024 37.6 -> 28.8.
 // Tried and slower at B=8192 C=2560 (backward): tiles of 32 samples in two stages with eight waves of one kind 193 us; dy
 // in the mixers' registers, dx stored from them, 214 us.
 //
@@ -760,14 +761,15 @@ bool bwd_slab_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) {
 // Channels per workgroup of the bf16 kernel.  A CU carries one workgroup of either width, so the narrow one leaves half as
 // many partial sums of dphi behind (C / 64 slabs in half as many splits) but has half the waves to hide its latencies
 // and loads half as wide pieces of a row.  Backward, 64 | 128 channels (us, the better split count of each):
-//   n=4  B=800 C=1280 23.5 | 25.0   1024 x 1024 22.4 | 24.9   2048 x 512 27.0 | 29.4   6000 x 256 40.8 | 43.8
-//        1024 x 2048 29.0 | 29.8   2048 x 1280 37.0 | 38.2   4096 x 640 39.5 | 40.7   8192 x 320 51.5 | 54.0
-//        1280 x 2560 39.2 | 37.4   900 x 4096 47.3 | 45.5   8192 x 768 66.3 | 64.9   3000 x 4096 101 | 91
-//   n=3  1500 x 1920 31.3 | 30.1   n=2  4000 x 1024 35.6 | 35.7   1000 x 2560 29.7 | 29.3
-// The lines: n = 4 below 12 M activation elements.
+//   n=4  B=800 C=1280 23.1 | 25.8   1024 x 1024 22.2 | 25.6   2048 x 512 24.8 | 27.3   6000 x 256 34.5 | 37.8
+//        1024 x 2048 28.3 | 29.9   2048 x 1280 33.1 | 35.2   4096 x 640 36.0 | 37.9   8192 x 320 39.8 | 43.1
+//        8192 x 768 64.9 | 67.3   8192 x 1024 70.8 | 73.0   8192 x 1280 84.9 | 86.7   5000 x 1920 79.9 | 80.7
+//        1280 x 2560 37.1 | 37.0   1000 x 3712 43.5 | 42.6   4000 x 2560 80.4 | 79.2   8192 x 2560 185 | 164
+//   n=3  1500 x 1920 31.6 | 29.5   n=2  4000 x 1024 34.4 | 32.1   1000 x 2560 29.6 | 27.2
+// The lines: n = 4 up to 1280 channels, or below 12 M activation elements.
 static int slab_width(int B, int n, int C) {
     if (const int forced = tuning_get(kTuneSlabWidth)) return forced == 1 ? 64 : 128;
-    return n == 4 && (long long)B * n * C < 12'000'000 ? 64 : 128;
+    return n == 4 && (C <= 1280 || (long long)B * n * C < 12'000'000) ? 64 : 128;
 }
 
 int bwd_slab_batch_splits(int B, int n, int C, int y_dtype) {
@@ -778,7 +780,7 @@ int bwd_slab_batch_splits(int B, int n, int C, int y_dtype) {
         return forced < tiles ? forced : tiles;
     }
     // All workgroups resident at once: one per CU (bf16 dy) or two (fp32 dy).  One split more than that costs a second
-    // round (B=1280 C=2560, 12 splits of 20 slabs 37.4 us, 20 splits 45.1), fewer leave CUs idle (8 splits 40.2).
+    // round (B=1280 C=2560, 12 splits of 20 slabs 37.1 us, 20 splits 44.8), fewer leave CUs idle (8 splits 39.4).
     int S = std::max(1, (staged ? 256 : 512) / slabs);
     if (S > tiles) S = tiles;
     // Short rows: the splits that cost least, a tile being some 0.65 us of a walk and a copy of the partial dphi 0.09 us of the

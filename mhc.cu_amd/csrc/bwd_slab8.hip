@@ -12,10 +12,10 @@
 // 12 registers per stream and dphi 48 per 32 columns.  Four waves mix (phi in their registers, the rows of M fetched from
 // LDS one at a time), four others hold dphi and request the tiles; eight waves of 256 registers fill the CU.
 //
-// What bounds it: bytes (x, dy in, dx out) and the partial sums of dphi, 256 * 64 columns of every stream and D rows in
-// fp32 whatever the shape (42 MB at n = 8), written here and added up by the finalize launch.  n=8 B=2000 C=2560: 56 us for
-// 246 MB and the 42 MB of partial sums; the whole backward 182 us (resident path) -> 106, n=5 B=2000 C=1280 89 -> 54,
-// n=6 B=3000 C=768 79 -> 59.  One walk of the batch per 64 channels took the resident path's second launch 120 us there.
+// What bounds it: bytes (x, dy in, dx out) and the partial sums of dphi, up to 256 * 64 columns of every stream and D rows in
+// fp32 (up to 42 MB at n = 8), written here and added up by the finalize launch.  n=8 B=2000 C=2560: 62 us for 246 MB and
+// 39 MB of partial sums (4.6 TB/s); the whole backward 182 us (resident path) -> 102, n=5 B=2000 C=1280 89 -> 50, n=6 B=3000
+// C=768 80 -> 54.  One walk of the batch per 64 channels took the resident path's second launch 120 us there.
 #include "launchers.h"
 
 #include <algorithm>
