@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "mhc", "libmhc_hip.so")
 
-SOURCES = ["capi.hip", "proj_fwd.hip", "gemm_f32.hip", "proj_bwd.hip", "proj_bwd_addx.hip", "proj_bwd_large.hip", "bwd_slab.hip", "bwd_slab8.hip", "bwd_slab_f32.hip", "bwd_static.hip", "coef_fwd.hip", "mix_fwd.hip", "layer_fwd_onepass.hip", "mix_bwd_reduce.hip",
+SOURCES = ["capi.hip", "proj_fwd.hip", "gemm_f32.hip", "proj_bwd.hip", "proj_bwd_addx.hip", "proj_bwd_large.hip", "bwd_slab.hip", "bwd_slab8.hip", "bwd_slab_f32.hip", "bwd_static.hip", "coef_fwd.hip", "mix_fwd.hip", "layer_fwd_onepass.hip", "layer_fwd_held.hip", "mix_bwd_reduce.hip",
            "bwd_resident.hip", "mix_bwd_dx.hip", "param_grads.hip", "pack_params.hip", "ops.hip"]
 
 # -packed-fp32-ops off: v_pk_*_f32 forms are not trusted on this hardware pool.

@@ -62,7 +62,7 @@ int ws_check(void *ws, size_t have, size_t need) {
     } while (0)
 
 // ---- dynamic workspace layout ----------------------------------------------------------------
-struct DynFwdWs { float *Ppart, *ssqpart, *agg; size_t bytes; };
+struct DynFwdWs { float *Ppart, *ssqpart, *agg; size_t part_bytes, bytes; };  // Ppart (part_bytes): partial sums, or phi for the held forward
 struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, *dx_part, *dxp, *dphi_part; unsigned short *dPb, *dPT; int BP; size_t bytes; };
 
 // Whether the sample-resident backward (bwd_resident.hip + the column-slab kernel) is taken where it is
@@ -148,7 +148,11 @@ DynFwdWs carve_dyn_fwd(void *ws, int B, int n, int C) {
     Carver c(ws);
     const int ks = max_ksplit(B, n, C);
     DynFwdWs w;
-    w.Ppart = c.floats((size_t)ks * B * padded_D(n));
+    w.part_bytes = (size_t)ks * B * padded_D(n) * sizeof(float);
+#ifdef MHC_TUNING  // batches below the line of the held forward, whose partial sums are smaller than phi
+    if (n >= 2 && n <= 4) w.part_bytes = std::max({w.part_bytes, layer_fwd_held_bytes(kBF16, n, C), layer_fwd_held_bytes(kF32, n, C)});
+#endif
+    w.Ppart = c.floats(w.part_bytes / sizeof(float));
     w.ssqpart = c.floats((size_t)ks * B);
     w.agg = c.floats(n > 8 ? (size_t)B * C : 0);  // stream aggregate of the matrix-core mix
     w.bytes = c.off;
@@ -628,6 +632,15 @@ int fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype, const Pa
     const DynFwdWs ws = carve_dyn_fwd(workspace, B, n, C);
     if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!f_inject && layer_fwd_held_supported(x_dtype, y_dtype, phi_dtype, B, n, C) &&
+        layer_fwd_held_bytes(x_dtype, n, C) <= ws.part_bytes) {
+        // (parameters that are not whole 16-byte pieces are packed by a launch of their own)
+        const bool direct = gather && aligned16(gather->phi[0]) && aligned16(gather->phi[1]) && aligned16(gather->phi[2]);
+        if (gather && !direct) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
+        MHC_LAUNCH(launch_layer_fwd_held(x, x_dtype, w, w_dtype, y, direct ? gather : nullptr, phi, alpha, bias, ws.Ppart, H_pre, H_post,
+                                         M, P, r, q, sk_state, B, n, C, iters, eps, st));
+        return MHC_OK;
+    }
     // the caller's own parameters: read by the projection where it can, otherwise packed by a launch of their own
     const bool in_proj = gather && !layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C) &&
                          proj_fwd_gathers(*gather, x_dtype, B, n, C);

@@ -102,10 +102,19 @@ hipError_t launch_layer_fwd_fused(const void *x, int x_dtype, const void *w, int
 // Whole dynamic-H forward in one launch (bf16 x and phi, n <= 4, n*C % 64 == 0): projection,
 // coefficients and mix with the samples' rows resident in LDS.  bias = [pre | post | res].
 bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C);
+int layer_fwd_onepass_most_samples(int n, int C);  // per workgroup
 hipError_t launch_layer_fwd_onepass(const void *x, const void *w, int w_dtype, const void *f_inject, void *y,
                                     int y_dtype, const void *phi, const float *alpha, const float *bias,
                                     float *Hpre, float *Hpost, float *M, float *P, float *r, float *q,
                                     float *sk_state, int B, int n, int C, int T, float eps, hipStream_t stream);
+
+// The same for large batches: sixteen samples per workgroup, their rows in registers (layer_fwd_held.hip).  frag: scratch
+// of layer_fwd_held_bytes(), phi in operand layout.  gather: the caller's own parameters, packed on the way.
+bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C);
+size_t layer_fwd_held_bytes(int x_dtype, int n, int C);
+hipError_t launch_layer_fwd_held(const void *x, int x_dtype, const void *w, int w_dtype, void *y, const ParamGather *gather, const void *phi,
+                                 const float *alpha, const float *bias, void *frag, float *Hpre, float *Hpost, float *M, float *P,
+                                 float *r, float *q, float *sk_state, int B, int n, int C, int T, float eps, hipStream_t stream);
 
 // fp32 matrix-core GEMMs of the exact float32 tier (wide projections): see gemm_f32.hip.
 bool dx_dphi_f32_supported(int x_dtype, int phi_dtype, int n, int C);

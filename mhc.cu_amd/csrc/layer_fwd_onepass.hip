@@ -23,6 +23,8 @@
 #include "sinkhorn_device.h"
 #include "tuning.h"
 
+#include <algorithm>
+
 namespace mhc {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
@@ -440,13 +442,14 @@ __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
 
 // Samples per workgroup: about one workgroup per CU (phi is re-read by every workgroup), bounded by
 // the 16 columns of the product tile and by LDS.
-static int onepass_group(int B, int n, int C) {
-    const int t = tuning_get(kTuneOnepassG);
-    int G = t > 0 ? t : (B + 255) / 256;
-    if (G > kOpMaxG) G = kOpMaxG;
-    if (G < 1) G = 1;
+int layer_fwd_onepass_most_samples(int n, int C) {
+    int G = kOpMaxG;
     while (G > 1 && OnePassLds(G, n * C, round_up(C / 8, 4), 8).total > 158 * 1024) G--;
     return G;
+}
+static int onepass_group(int B, int n, int C) {
+    const int t = tuning_get(kTuneOnepassG), G = t > 0 ? t : (B + 255) / 256;
+    return std::max(1, std::min(G, layer_fwd_onepass_most_samples(n, C)));
 }
 
 // Every workgroup streams all of phi out of the L2 (about 90 GB/s per CU in this access pattern, measured

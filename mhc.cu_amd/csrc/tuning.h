@@ -8,7 +8,7 @@
 namespace mhc {
 
 enum TuneKey {
-    kTuneOnepassOff = 0,    // one-launch forward: 0 = by cost model, 1 = never, 2 = whenever the shape allows
+    kTuneOnepassOff = 0,    // one-pass forwards: 0 = by size, 1 = neither, 2 = the one-launch forward, 3 = the held one, whenever the shape allows
     kTuneOnepassG = 1,      // samples per workgroup of the one-launch forward
     kTuneGramFused = 2,     // n <= 8 channel sums and coefficient backward: 1 = two launches, 2 = one launch (n <= 4: four samples per workgroup)
     kTuneSlabSplits = 3,    // batch splits of the slab backward (n <= 8) and of the projection backward (n = 5 .. 18)
