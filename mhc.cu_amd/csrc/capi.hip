@@ -641,14 +641,16 @@ int fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype, const Pa
                                          M, P, r, q, sk_state, B, n, C, iters, eps, st));
         return MHC_OK;
     }
-    // the caller's own parameters: read by the projection where it can, otherwise packed by a launch of their own
-    const bool in_proj = gather && !layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C) &&
-                         proj_fwd_gathers(*gather, x_dtype, B, n, C);
-    if (gather && !in_proj) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
-    if (layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C)) {
+    // the caller's own parameters: read by the kernel that multiplies with them where it can, otherwise packed by a launch
+    // of their own
+    const bool can_gather = gather && layer_fwd_onepass_gathers(*gather);
+    const bool one = layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C, can_gather), in_one = one && can_gather;
+    const bool in_proj = gather && !one && proj_fwd_gathers(*gather, x_dtype, B, n, C);
+    if (gather && !in_one && !in_proj) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
+    if (one) {
         // projection, coefficients and mix in one launch; x crosses HBM once
         MHC_LAUNCH(launch_layer_fwd_onepass(x, w, w_dtype, f_inject, y, y_dtype, phi, alpha, bias, H_pre, H_post,
-                                            M, P, r, q, sk_state, B, n, C, iters, eps, st));
+                                            M, P, r, q, sk_state, B, n, C, iters, eps, st, in_one ? gather : nullptr));
         return MHC_OK;
     }
     const int KS = proj_fwd_ksplit(x_dtype, phi_dtype, B, n, C);

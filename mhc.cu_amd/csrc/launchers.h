@@ -101,12 +101,14 @@ hipError_t launch_layer_fwd_fused(const void *x, int x_dtype, const void *w, int
 
 // Whole dynamic-H forward in one launch (bf16 x and phi, n <= 4, n*C % 64 == 0): projection,
 // coefficients and mix with the samples' rows resident in LDS.  bias = [pre | post | res].
-bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C);
+bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C, bool from_params = false);
 int layer_fwd_onepass_most_samples(int n, int C);  // per workgroup
+bool layer_fwd_onepass_gathers(const ParamGather &g);  // it reads the caller's own parameters itself
 hipError_t launch_layer_fwd_onepass(const void *x, const void *w, int w_dtype, const void *f_inject, void *y,
                                     int y_dtype, const void *phi, const float *alpha, const float *bias,
                                     float *Hpre, float *Hpost, float *M, float *P, float *r, float *q,
-                                    float *sk_state, int B, int n, int C, int T, float eps, hipStream_t stream);
+                                    float *sk_state, int B, int n, int C, int T, float eps, hipStream_t stream,
+                                    const ParamGather *gather = nullptr);
 
 // The same for large batches: sixteen samples per workgroup, their rows in registers (layer_fwd_held.hip).  frag: scratch
 // of layer_fwd_held_bytes(), phi in operand layout.  gather: the caller's own parameters, packed on the way.

@@ -20,6 +20,7 @@
 #include "launchers.h"
 #include "mhc_common.h"
 #include "phase_profiler.h"
+#include "phi_src.h"
 #include "sinkhorn_device.h"
 #include "tuning.h"
 
@@ -41,6 +42,7 @@ struct OnePassArgs {
     int w_bf16, B, n, C, T, G;
     float eps;
     float *sk_state;  // [B][T + 1][2][NP] Sinkhorn denominators kept for the backward, or nullptr
+    PhiSrc src;       // PF32: phi, alpha and bias as the caller stores them
 };
 
 constexpr int kOpMaxG = 16;      // samples per workgroup: the columns of one 16-wide tile
@@ -71,7 +73,9 @@ struct OnePassLds {
 constexpr int kOnePassWaves = 8;  // waves per workgroup (4..7 measured slower at every shape of the sweep)
 constexpr int kDppQuadBcast0 = 0x00, kDppQuadBcast1 = 0x55, kDppQuadBcast2 = 0xAA, kDppQuadBcast3 = 0xFF;
 
-template <typename TY, int GH>
+// PF32: phi comes from the caller's fp32 matrices; the steps of K go round the workgroups, each of which leaves its steps of the
+// packed phi behind.
+template <typename TY, int GH, bool PF32>
 __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
     constexpr int NP = 4, DT = 2;
     using SK = SkSmall<NP>;
@@ -101,12 +105,21 @@ __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
     {
         const int g = lane & 15, r0 = SK::row(g), c0 = SK::col0(g);
         const bool mv = r0 < n && c0 < n, vv = g < 2 * n;
-        c_al = a.alpha[vv ? (g < n ? 0 : 1) : 2];
-        c_al2 = a.alpha[2];
-        c_bvec = a.bias[vv ? g : 0];
-        c_bres = a.bias[mv ? 2 * n + r0 * n + c0 : 0];
+        if constexpr (PF32) {
+            c_al = *a.src.alpha[vv ? (g < n ? 0 : 1) : 2];
+            c_al2 = *a.src.alpha[2];
+            c_bvec = *(!vv || g < n ? a.src.b[0] + (vv ? g : 0) : a.src.b[1] + (g - n));
+            c_bres = a.src.b[2][mv ? r0 * n + c0 : 0];
+        } else {
+            c_al = a.alpha[vv ? (g < n ? 0 : 1) : 2];
+            c_al2 = a.alpha[2];
+            c_bvec = a.bias[vv ? g : 0];
+            c_bres = a.bias[mv ? 2 * n + r0 * n + c0 : 0];
+        }
     }
 
+    if constexpr (PF32)
+        if (blockIdx.x == 0) gather_small(a.src, tid, NT, D);
     // ---- phase A: stream x and phi, project ---------------------------------------------------
     {
         const int steps = nC >> 6;  // 64 contraction elements (128 bytes of every row) per step
@@ -124,7 +137,9 @@ __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
         // alias the last valid one and are not parked; phi rows beyond D alias row 0.
         const int r8 = lane >> 3, seg = lane & 7;
         const int dj = (D + 7) >> 3;  // 8-row pieces of phi: 1..3
-        const bf16_t *xrow[GH], *prow[3];
+        constexpr int PW = PF32 ? 8 : 4;  // words per piece of phi
+        const bf16_t *xrow[GH];
+        const uint32_t *prow[3];
         bool xv[GH];
 #pragma unroll
         for (int h = 0; h < GH; h++) {
@@ -135,7 +150,8 @@ __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             const int d = j * 8 + r8;
-            prow[j] = a.phi + (size_t)(d < D ? d : 0) * nC + seg * 8;
+            if constexpr (PF32) prow[j] = reinterpret_cast<const uint32_t *>(phi_src_row(a.src, d < D ? d : 0, nC) + seg * 8);
+            else prow[j] = reinterpret_cast<const uint32_t *>(a.phi + (size_t)(d < D ? d : 0) * nC + seg * 8);
         }
         // operand layout: lane (row, kg) holds k = 16 kg .. 16 kg + 15 of its row; the first 8 feed the
         // first product of the step, the other 8 the second (x follows the same order)
@@ -144,7 +160,7 @@ __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
         const bf16_t *pfrag = ps + row * kOpStagePitch + kg * 16;
 
         // kOpDepth steps in flight per wave (scalar words: whole-uint4 array elements can end up in scratch)
-        uint32_t xq[kOpDepth][GH][4], pq[kOpDepth][3][4];
+        uint32_t xq[kOpDepth][GH][4], pq[kOpDepth][3][PW];
         auto fetch = [&](int slot, int st) {
             const int k0 = k_of(st);
 #pragma unroll
@@ -155,8 +171,11 @@ __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
 #pragma unroll
             for (int j = 0; j < 3; j++) {
                 if (j < dj) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(prow[j] + k0);
-                    pq[slot][j][0] = v.x; pq[slot][j][1] = v.y; pq[slot][j][2] = v.z; pq[slot][j][3] = v.w;
+#pragma unroll
+                    for (int i = 0; i < PW; i += 4) {
+                        const uint4 v = *reinterpret_cast<const uint4 *>(prow[j] + (PF32 ? k0 : k0 / 2) + i);
+                        pq[slot][j][i] = v.x; pq[slot][j][i + 1] = v.y; pq[slot][j][i + 2] = v.z; pq[slot][j][i + 3] = v.w;
+                    }
                 }
             }
         };
@@ -181,9 +200,18 @@ __global__ __launch_bounds__(512) void layer_fwd_onepass_kernel(OnePassArgs a) {
             }
 #pragma unroll
             for (int j = 0; j < 3; j++) {
-                if (j < dj)
-                    *reinterpret_cast<uint4 *>(ps + (j * 8 + r8) * kOpStagePitch + seg * 8) =
-                        make_uint4(pq[slot][j][0], pq[slot][j][1], pq[slot][j][2], pq[slot][j][3]);
+                if (j < dj) {
+                    const uint32_t(&w)[PW] = pq[slot][j];
+                    uint4 v = make_uint4(w[0], w[1], w[2], w[3]);
+                    if constexpr (PF32) {
+                        auto pair = [&](int i) { return pack_bf16x2(__uint_as_float(w[i]), __uint_as_float(w[i + 1])); };
+                        v = make_uint4(pair(0), pair(2), pair(4), pair(6));
+                        const int d = j * 8 + r8;
+                        if ((k0 >> 6) % (int)gridDim.x == (int)blockIdx.x && d < D)
+                            *reinterpret_cast<uint4 *>(static_cast<bf16_t *>(a.src.phi_out) + (size_t)d * nC + k0 + seg * 8) = v;
+                    }
+                    *reinterpret_cast<uint4 *>(ps + (j * 8 + r8) * kOpStagePitch + seg * 8) = v;
+                }
             }
             // both come back in operand layout from the lines this wave has just written (a wave's LDS
             // accesses complete in order; the fence keeps the compiler from moving the reads up)
@@ -461,39 +489,53 @@ static int onepass_group(int B, int n, int C) {
 // (B=320 C=1280 n=4, 240 KB: 31.4 against 30.3 us); beyond 256 KB it loses everywhere (B=1280 C=2560
 // n=4: 64.1 against 62.2 us).  Elsewhere the two-launch forward (split-K projection, then the fused mix
 // kernel) stays.
-bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C) {
+// From the caller's own fp32 parameters (read by the kernel itself, twice the bytes of phi; the two-launch forward reads them in
+// its projection) the window between 120 and 256 KB starts at 1280 samples: n=4 C=1280 B=1024 14.8 against 13.4 us, 1600 16.4 | 16.6;
+// n=2 C=4096 1024 17.5 | 15.2; n=3 C=1920 1024 13.6 | 13.7, 1600 16.2 | 20.2.  Below 120 KB it saves the packing launch (forward
+// us from parameters, packed by a launch -> read here: n=4 C=256 B=7 8.8 -> 7.3, 2048 9.8 -> 8.5, C=512 7 9.9 -> 8.7, n=3 C=640 320 9.4 ->
+// 8.4, n=2 C=1024 7 8.9 -> 7.4).
+bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C, bool from_params) {
     const int mode = tuning_get(kTuneOnepassOff);  // 0 = by cost, 1 = never, 2 = whenever the shape allows
     if (mode == 1) return false;
     if (x_dtype != kBF16 || phi_dtype != kBF16 || n > 4 || C % 8 != 0 || (n * C) % 64 != 0) return false;
     if (OnePassLds(1, n * C, round_up(C / 8, 4), kOnePassWaves).total > 158 * 1024) return false;
     if (mode == 2) return true;
     const long long phi_bytes = 2ll * (n * n + 2 * n) * n * C;
-    return phi_bytes <= 120 * 1024 || (phi_bytes <= 256 * 1024 && B >= 1024 && B <= 2048);
+    return phi_bytes <= 120 * 1024 || (phi_bytes <= 256 * 1024 && B >= (from_params ? 1280 : 1024) && B <= 2048);
+}
+
+bool layer_fwd_onepass_gathers(const ParamGather &g) {
+    auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    return g.phi_dtype == kF32 && al16(g.phi[0]) && al16(g.phi[1]) && al16(g.phi[2]) && tuning_get(kTuneGather) != 1;
 }
 
 hipError_t launch_layer_fwd_onepass(const void *x, const void *w, int w_dtype, const void *f_inject, void *y,
                                     int y_dtype, const void *phi, const float *alpha, const float *bias,
                                     float *Hpre, float *Hpost, float *M, float *P, float *r, float *q,
-                                    float *sk_state, int B, int n, int C, int T, float eps, hipStream_t stream) {
+                                    float *sk_state, int B, int n, int C, int T, float eps, hipStream_t stream,
+                                    const ParamGather *gather) {
     const int G = onepass_group(B, n, C);
     constexpr int NW = kOnePassWaves;
     OnePassArgs a{static_cast<const bf16_t *>(x), w, static_cast<const bf16_t *>(f_inject), y,
                   static_cast<const bf16_t *>(phi), alpha, bias, Hpre, Hpost, M, P, r, q,
-                  w_dtype == kBF16, B, n, C, T, G, eps, sk_state};
+                  w_dtype == kBF16, B, n, C, T, G, eps, sk_state, gather ? phi_src_of(*gather, n) : PhiSrc{}};
     const size_t smem = OnePassLds(G, n * C, round_up(C / 8, 4), NW).total;
     const int grid = (B + G - 1) / G;
     hipError_t e = hipSuccess;
-#define MHC_ONEPASS(TY, GH)                                                                  \
+#define MHC_ONEPASS(TY, GH, PF32)                                                            \
     do {                                                                                     \
-        e = allow_dynamic_lds<&layer_fwd_onepass_kernel<TY, GH>>(smem);                      \
+        e = allow_dynamic_lds<&layer_fwd_onepass_kernel<TY, GH, PF32>>(smem);                \
         if (e != hipSuccess) return e;                                                       \
-        layer_fwd_onepass_kernel<TY, GH><<<grid, NW * 64, smem, stream>>>(a);                \
+        layer_fwd_onepass_kernel<TY, GH, PF32><<<grid, NW * 64, smem, stream>>>(a);          \
     } while (0)
-    if (y_dtype == kBF16) {
-        if (G <= 8) MHC_ONEPASS(bf16_t, 1); else MHC_ONEPASS(bf16_t, 2);
-    } else {
-        if (G <= 8) MHC_ONEPASS(float, 1); else MHC_ONEPASS(float, 2);
-    }
+#define MHC_ONEPASS_TY(TY)                                                                   \
+    do {                                                                                     \
+        if (gather) { if (G <= 8) MHC_ONEPASS(TY, 1, true); else MHC_ONEPASS(TY, 2, true); } \
+        else { if (G <= 8) MHC_ONEPASS(TY, 1, false); else MHC_ONEPASS(TY, 2, false); }      \
+    } while (0)
+    if (y_dtype == kBF16) MHC_ONEPASS_TY(bf16_t);
+    else MHC_ONEPASS_TY(float);
+#undef MHC_ONEPASS_TY
 #undef MHC_ONEPASS
     return hipGetLastError();
 }

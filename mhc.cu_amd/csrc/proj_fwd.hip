@@ -17,6 +17,7 @@
 #include <type_traits>
 #include "mhc_common.h"
 #include "phase_profiler.h"
+#include "phi_src.h"
 #include "tuning.h"
 
 namespace mhc {
@@ -82,29 +83,6 @@ __global__ __launch_bounds__(256) void proj_fwd_generic_kernel(const TX *__restr
 // --------------------------------------------------------------------------------------------
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2_t;
 constexpr int kNarrowPitch = 72;  // LDS row of a 64-element chunk: 128 data bytes + 16 pad (bf16 elements)
-
-// The caller's fp32 parameters, read by the projection itself (PF32 of the two kernels below): projection row d
-// is a row of one of the three matrices, rounded to bf16 on its way into the LDS tile; the workgroups of the
-// first sample tile also store the rounded rows, [bias] and [alpha] for the kernels that follow and for the
-// backward call.  Saves a packing launch (about 3 us of device and 5 us of host time per call, and for n = 32
-// a read of the 89 MB that it wrote).
-struct PhiSrc {
-    const float *phi[3];
-    const float *b[3], *alpha[3];
-    void *phi_out;  // in the compute type: bf16, or fp32 in the exact tier
-    float *bias_out, *alpha_out;
-    int n;
-};
-__device__ __forceinline__ const float *phi_src_row(const PhiSrc &g, int d, int nC) {
-    const float *base = d < g.n ? g.phi[0] : (d < 2 * g.n ? g.phi[1] : g.phi[2]);
-    const int r = d < g.n ? d : (d < 2 * g.n ? d - g.n : d - 2 * g.n);
-    return base + (size_t)r * nC;
-}
-__device__ __forceinline__ void gather_small(const PhiSrc &g, int tid, int nthr, int D) {
-    if (tid < 3) g.alpha_out[tid] = g.alpha[tid][0];
-    for (int i = tid; i < D; i += nthr)
-        g.bias_out[i] = i < g.n ? g.b[0][i] : (i < 2 * g.n ? g.b[1][i - g.n] : g.b[2][i - 2 * g.n]);
-}
 
 // XF32: x is stored as fp32 and rounded to bf16 (nearest even) on its way into the LDS tile; everything
 // behind the tile, the sum of squares included, sees the rounded values.
@@ -752,16 +730,7 @@ hipError_t launch_proj_fwd(const void *x, int x_dtype, const void *phi, int phi_
                            const ParamGather *gather) {
     const int nC = n * C, D = n * n + 2 * n, DP = padded_D(n), nt = narrow_nt(x_dtype, B, n, C, KS);
     if (gather) {
-        PhiSrc src;
-        for (int i = 0; i < 3; i++) {
-            src.phi[i] = static_cast<const float *>(gather->phi[i]);
-            src.b[i] = gather->b[i];
-            src.alpha[i] = gather->alpha[i];
-        }
-        src.phi_out = gather->phi_out;
-        src.bias_out = gather->bias_out;
-        src.alpha_out = gather->alpha_out;
-        src.n = n;
+        const PhiSrc src = phi_src_of(*gather, n);
         if (x_dtype == kF32) {
             switch (nt) {
                 case 1: return launch_mfma<1, false, true, true>(x, nullptr, Ppart, ssqpart, KS, B, D, DP, nC, stream, src);

@@ -58,6 +58,15 @@ def test_parameters_read_by_the_projection_match_the_packing_launch(B, n, C, mix
         assert torch.equal(a.nan_to_num(1e30), b.nan_to_num(1e30)), k
 
 
+@pytest.mark.parametrize("B,n,C,mixed", [
+    (1, 4, 64, False), (37, 4, 64, False), (300, 4, 128, False), (3000, 2, 64, False), (9, 3, 640, False), (40, 1, 128, False),
+    (1500, 4, 832, False),                              # one launch: one workgroup, fewer steps than workgroups, two row pieces, steps from each workgroup's own starting point
+    (4112, 4, 384, False), (1700, 3, 192, True),        # sixteen samples per workgroup
+])
+def test_parameters_read_by_the_one_pass_forwards(B, n, C, mixed):
+    test_parameters_read_by_the_projection_match_the_packing_launch(B, n, C, mixed)
+
+
 @pytest.mark.parametrize("dynamic", [True, False])
 @pytest.mark.parametrize("B,n,C", [(5, 4, 64), (900, 4, 72), (9, 8, 136), (6, 32, 64), (4, 3, 37)])
 def test_weight_gradient_in_bfloat16_is_the_rounded_float32_one(dynamic, B, n, C):
