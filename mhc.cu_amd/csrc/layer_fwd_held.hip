@@ -119,7 +119,7 @@ __global__ __launch_bounds__(NW * 64, held_waves(N * CB)) void layer_fwd_held_ke
     constexpr bool kExact = std::is_same<TX, float>::value;
     constexpr bool kRound = sizeof(TS) > sizeof(TX);            // fp32 storage, rounded to bf16 behind the load
     constexpr bool kFine = std::is_same<TS, float>::value;      // fp32 results: library functions, IEEE divisions, mix in fp32
-    constexpr int kFold = kExact ? 1 : 2;
+    constexpr int kFold = kExact ? 1 : 2, kSums = kRound || N < 4 ? 2 : 1;
     constexpr int LP = kRound ? 2 : 1;                          // loads per piece: 16 bytes of either half of the chunk's channels
     constexpr int kCoef = 28;                  // floats of a sample's coefficients (pitch)
     constexpr int kPitch = 144;                // bytes of a staged row
@@ -249,11 +249,14 @@ __global__ __launch_bounds__(NW * 64, held_waves(N * CB)) void layer_fwd_held_ke
         // ---- projection and sum of squares -------------------------------------------------------
 #pragma unroll
         for (int u = 0; u < WP; u++) load_phi(u);
-        // The products of kFold units are summed on the matrix cores and then added to the wave's sums: a chain over all units
-        // loses bits
-        f32x4_t sum[H::kTiles], acc[N == 4 ? 3 : (N == 2 ? 2 : 1)];
+        // The products of kFold units are summed on the matrix cores and then added to the wave's sums, to each of kSums in turn: a
+        // chain over all units loses bits (error of P against float64, one chain | this | the two-launch forward: bf16 n=4 B=3001 C=2560
+        // 2.0e-7 | 1.1e-7 | 1.4e-7, float32 2560 1280 4.2e-7 | 1.5e-7 | 2.4e-7)
+        f32x4_t sum[kSums][H::kTiles], acc[N == 4 ? 3 : (N == 2 ? 2 : 1)];
 #pragma unroll
-        for (auto &t : sum) t = zero;
+        for (auto &k : sum)
+#pragma unroll
+            for (auto &t : k) t = zero;
         float ssx[2] = {0.f, 0.f};
         stage(0);
         operands(0);
@@ -278,11 +281,12 @@ __global__ __launch_bounds__(NW * 64, held_waves(N * CB)) void layer_fwd_held_ke
                 acc[1] = product(p[0], xf[1], acc[1]);
             }
             if (u % kFold == kFold - 1 || u == U - 1) {
-                if constexpr (N != 2) sum[0] += acc[0];
+                auto &to = sum[u / kFold % kSums];
+                if constexpr (N != 2) to[0] += acc[0];
                 if constexpr (N != 3) {  // paired rows: one half of the lanes holds either product
                     const f32x4_t &lo = acc[N == 4 ? 1 : 0], &hi = acc[N == 4 ? 2 : 1];
 #pragma unroll
-                    for (int r = 0; r < 4; r++) sum[H::kTiles - 1][r] += lane < 32 ? lo[r] : hi[r];
+                    for (int r = 0; r < 4; r++) to[H::kTiles - 1][r] += lane < 32 ? lo[r] : hi[r];
                 }
             }
 #pragma unroll
@@ -311,7 +315,7 @@ __global__ __launch_bounds__(NW * 64, held_waves(N * CB)) void layer_fwd_held_ke
 #pragma unroll
         for (int t = 0; t < H::kTiles; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) red(wave, t, r, lane) = sum[t][r];
+            for (int r = 0; r < 4; r++) red(wave, t, r, lane) = kSums == 2 ? sum[0][t][r] + sum[kSums - 1][t][r] : sum[0][t][r];
         auto row_sum = [&](float v) {  // over the eight lanes that hold a row
             v += dpp_mov<kDppQuadXor1>(v);
             v += dpp_mov<kDppQuadXor2>(v);
