@@ -13,7 +13,7 @@
 // and read back transposed; dP arrives from the reduce kernel as bf16 [B, DP] and as a transposed hi/lo
 // pair [2][DP][BP].  x and dy are read once from HBM, dx is written once; no atomics.
 //
-// Two kernels: bwd_slab_stage_kernel for bf16 dy, bwd_slab_f32dy_kernel for fp32 dy beside bf16 x.
+// Two kernels: bwd_slab_stage_kernel for bf16 dy (and for fp32 storage of both), bwd_slab_f32dy_kernel for fp32 dy beside bf16 x.
 #include "launchers.h"
 
 #include <algorithm>
@@ -43,7 +43,7 @@ struct BwdSlabArgs {
     const bf16_t *dPb;       // dP, fragment-major (frag_dpb, DP = 32)
     const bf16_t *dPT;       // dP^T hi/lo planes, fragment-major (frag_dpt), plane stride 32 * BP
     const float *dt;         // [B, D+3]
-    bf16_t *dx;              // [B, n, C]
+    void *dx;                // [B, n, C], in the type of x's storage
     bf16_t *df;              // [B, C] or nullptr
     float *dphi_part;        // [S][D][nC]
     double *dw_part;         // [S][C]
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32dy_kernel(BwdSlabArgs a) {
                             dxw[j][0] = pack_bf16x2(out[0], out[1]);
                             dxw[j][1] = pack_bf16x2(out[2], out[3]);
                         } else {
-                            st16<true>(a.dx + (size_t)b * nC + (size_t)j * C + cth, dxw[j][0], dxw[j][1],
+                            st16<true>(static_cast<bf16_t *>(a.dx) + (size_t)b * nC + (size_t)j * C + cth, dxw[j][0], dxw[j][1],
                                        pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]));
                         }
                     }
@@ -405,11 +405,18 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32dy_kernel(BwdSlabArgs a) {
 // row are permuted (slab_swizzle) so that neither the transposed reads (dphi) nor the row reads (dx) meet in a bank.
 // ---------------------------------------------------------------------------------------------
 
-template <int N, int CW> struct SlabStage {
+// F32: float32 storage.  The channel sums have left x and dy in bf16 where dx will be (mix_bwd_reduce.hip): the 256 bytes of 64
+// channels hold 128 of x, then 128 of dy, and this kernel's slab of 64 reads such a piece and later puts 64 values of dx in its
+// place.  x and dy are then one tile, three tiles ahead, a row of 16 chunks like those of a slab of 128; dx, twice as wide as dy, leaves
+// through two places of its own.  Backward in graphs of ten, resident path -> channel sums and this: n=4 B=4369 C=1280 142 -> 113 us,
+// 2000 2560 133 -> 90, n=3 3000 3136 199 -> 124, n=2 4369 2560 185 -> 105.
+template <int N, int CW, bool F32> struct SlabStage {
+    static_assert(!F32 || CW == 64, "the pieces of a row are 64 channels wide");
     static constexpr int TB = 16, kLoaders = CW / 32, kMixers = CW / 16, kThreads = 64 * (kLoaders + kMixers);  // 6 CW
-    static constexpr int kXAhead = 3, kGAhead = 2;        // tiles requested ahead
+    static constexpr int kXAhead = 3, kGAhead = F32 ? 0 : 2;  // tiles requested ahead
     static constexpr int kXRing = kXAhead + 1, kGRing = kGAhead + 2;
-    static constexpr int kTile = N * TB * CW * 2;         // bytes of x or dy
+    static constexpr int kRowBytes = CW * (F32 ? 4 : 2), kChunks = kRowBytes / 16, kRows = 1024 / kRowBytes;  // of a tile's row; rows per KiB
+    static constexpr int kTile = N * TB * kRowBytes;      // bytes of x or dy, or of both; of dx
     static constexpr int kP = kTile, kCoef = kP + 3 * 1024;
     // coefficient blocks of 64 floats: M | Hpre | Hpost | cx | q | s1 | dt (slab 0 only)
     static constexpr int kSegM = (TB * N * N + 63) / 64, kSegs = kSegM + 5, kSegDt = (TB * (N * N + 2 * N + 3) + 63) / 64;
@@ -421,13 +428,15 @@ template <int N, int CW> struct SlabStage {
     static constexpr int kW = kG + kGRing * kTile;        // the slab's w in fp32
     static constexpr int kLds = kW + CW * 4;
     static constexpr int kPhi = 32 * N * CW * 2;          // prologue: the phi slab, in the part of the dy ring not yet requested
+    static constexpr int kRing = kChunks * 8;             // what slab_swizzle() goes by
     static_assert(kPhi <= (kGRing - kGAhead) * kTile && kLds <= 160 * 1024, "the rings fit the LDS of a CU");
 };
 
-template <int N, int CW, bool INJECT>
+template <int N, int CW, bool INJECT, bool F32>
 __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a) {
-    using ST = SlabStage<N, CW>;
-    constexpr int kChunks = CW / 8, kRows = 512 / CW;  // 16-byte chunks per row, rows per KiB
+    static_assert(!(INJECT && F32), "an injected f takes the other kernels");
+    using ST = SlabStage<N, CW, F32>;
+    constexpr int kChunks = ST::kChunks, kRows = ST::kRows, kRowBytes = ST::kRowBytes;
     constexpr int D = N * N + 2 * N, TB = ST::TB;
     extern __shared__ float smem_f[];
     char *const smem = reinterpret_cast<char *>(smem_f);
@@ -448,20 +457,37 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
 
     // One KiB of a tile of x, dy or dx is kRows sample rows of one stream: where lane's 16 bytes belong, for the rows from row0
     const auto lane_row = [&](int row0) { return row0 + lane / kChunks; };
-    const auto lane_col = [&](int row) { return c0 + ((lane % kChunks) ^ slab_swizzle<CW>(row)) * 8; };
+    const auto lane_chunk = [&](int row) { return (lane % kChunks) ^ slab_swizzle<ST::kRing>(row); };
+    const auto lane_col = [&](int row) { return c0 + lane_chunk(row) * (F32 ? 4 : 8); };  // of x or dy; F32: of dx
 
     // ---- loads of a tile (loaders); loader l brings rows l kRows .. of every stream --------------------
     // slots beyond the batch alias its last sample, columns beyond C the last ones: they only meet zero columns of
     // dP^T or land in rows and columns that are not stored
+    // (F32: C is a multiple of 64; a loader brings every kLoaders-th group of rows)
     const int ld_row = lane_row(lw * kRows), ld_col = min(lane_col(ld_row), C - 8);
-    auto load_tile = [&](const bf16_t *src, int t, uint32_t dst) {
+    constexpr int kLoads = F32 ? N * TB / kRows / ST::kLoaders : N;  // instructions per loader for a tile of x, or of both
+    auto load_tile = [&](const void *src, int t, uint32_t dst) {
         const int sb = b_begin + t * TB;
-        const bf16_t *base = src + (size_t)sb * nC;
-        const uint32_t off = (uint32_t)(min(ld_row, b_end - sb - 1) * nC + ld_col) * 2;
+        if constexpr (F32) {
+            const char *base = static_cast<const char *>(src) + ((size_t)sb * nC + c0) * 4;
 #pragma unroll
-        for (int j = 0; j < N; j++) load_to_lds<16>(base + (size_t)j * C, off, dst + (j * TB + lw * kRows) * CW * 2);
+            for (int j = 0; j < N; j++)
+#pragma unroll
+                for (int i = 0; i < TB / kRows / ST::kLoaders; i++) {
+                    const int row0 = (lw + i * ST::kLoaders) * kRows, row = lane_row(row0);
+                    load_to_lds<16>(base + (size_t)j * C * 4, (uint32_t)min(row, b_end - sb - 1) * nC * 4 + lane_chunk(row) * 16,
+                                    dst + (j * TB + row0) * kRowBytes);
+                }
+        } else {
+            const bf16_t *base = static_cast<const bf16_t *>(src) + (size_t)sb * nC;
+            const uint32_t off = (uint32_t)(min(ld_row, b_end - sb - 1) * nC + ld_col) * 2;
+#pragma unroll
+            for (int j = 0; j < N; j++) load_to_lds<16>(base + (size_t)j * C, off, dst + (j * TB + lw * kRows) * kRowBytes);
+        }
     };
-    auto load_dy = [&](int t) { load_tile(static_cast<const bf16_t *>(a.dy), t, smem_at + ST::kG + t % ST::kGRing * ST::kTile); };
+    auto load_dy = [&](int t) {
+        if constexpr (!F32) load_tile(a.dy, t, smem_at + ST::kG + t % ST::kGRing * ST::kTile);
+    };
     // The dP operands and the blocks of 64 coefficients of a tile are dealt out to the loaders: what this one brings is
     // settled once, so that a tile costs it no more than the instructions.
     struct Block {
@@ -493,7 +519,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
     auto load_x = [&](int t) {
         const uint32_t st = smem_at + t % ST::kXRing * ST::kXBytes;
         const int sb = b_begin + t * TB, left = min(b_end - sb, TB);
-        load_tile(a.x, t, st);
+        load_tile(F32 ? a.dx : static_cast<const void *>(a.x), t, st);
 #pragma unroll
         for (int i = 0; i < ST::kShareDt; i++) {
             const Block &m = mine[i];
@@ -522,13 +548,13 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
     }
     char *const phi_s = smem + ST::kG + ST::kGAhead * ST::kTile;
     if (!loader) {
-        constexpr int kThreads = 64 * ST::kMixers, kPhiIters = N * 32 * kChunks / kThreads;
-        static_assert(kPhiIters * kThreads == N * 32 * kChunks, "whole chunks of phi for every mixer");
+        constexpr int kThreads = 64 * ST::kMixers, kPc = CW / 8, kPhiIters = N * 32 * kPc / kThreads;
+        static_assert(kPhiIters * kThreads == N * 32 * kPc, "whole chunks of phi for every mixer");
         uint4 phir[kPhiIters];
 #pragma unroll
         for (int i = 0; i < kPhiIters; i++) {
             const int e = tid + i * kThreads;
-            const int d = e / (N * kChunks), j = e / kChunks % N, c = c0 + e % kChunks * 8;
+            const int d = e / (N * kPc), j = e / kPc % N, c = c0 + e % kPc * 8;
             const bool ok = d < D && c < C;
             phir[i] = load16_masked(reinterpret_cast<const uint4 *>(a.phi + (ok ? (size_t)d * nC + (size_t)j * C + c : 0)), ok);
         }
@@ -552,9 +578,17 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
         for (int p = 0; p < T; p++) {
             // Tile p has landed, for everybody behind the barrier: its dy is the last of it, requested in period p - 2, and
             // behind that are the x of tile p + 2 and the dy of tile p + 1 (period p - 1).  Towards the end there are fewer.
-            if (p + 2 >= T) wait_vmem<0>();
-            else if (slab == 0) wait_vmem<2 * N + ST::kShareDt>();
-            else wait_vmem<2 * N + ST::kShare>();
+            // (F32: behind it are the tiles p + 1 and p + 2)
+            if constexpr (F32) {
+                if (p + 1 >= T) wait_vmem<0>();
+                else if (p + 2 >= T) { if (slab == 0) wait_vmem<kLoads + ST::kShareDt>(); else wait_vmem<kLoads + ST::kShare>(); }
+                else if (slab == 0) wait_vmem<2 * (kLoads + ST::kShareDt)>();
+                else wait_vmem<2 * (kLoads + ST::kShare)>();
+            } else {
+                if (p + 2 >= T) wait_vmem<0>();
+                else if (slab == 0) wait_vmem<2 * N + ST::kShareDt>();
+                else wait_vmem<2 * N + ST::kShare>();
+            }
             stage_barrier();
             // everybody is done with x of tile p - 1 and with dx of tile p - 2, whose places these take
             if (p + ST::kXAhead < T) load_x(p + ST::kXAhead);
@@ -591,7 +625,9 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
         const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
         const float inv_c = 1.0f / (float)C;
         stage_barrier();  // the loaders may fill the places that hold phi
-        const int row_at = l16 * CW * 2 + (((cl >> 3) ^ slab_swizzle<CW>(l16)) * 16) + (kq & 1) * 8;  // this lane's 8 bytes of its sample's row
+        // this lane's 8 bytes of its sample's row of x, of dy (F32: 8 chunks behind), and what it writes of dx
+        const auto row_place = [&](int chunk) { return l16 * kRowBytes + ((chunk ^ slab_swizzle<ST::kRing>(l16)) * 16); };
+        const int row_at = row_place(cl >> 3) + (kq & 1) * 8, row_dy = F32 ? row_place(8 + (cl >> 3)) + (kq & 1) * 8 : row_at;
         // a tile of dx leaves in pieces of one KiB, kOut for every mixer
         constexpr int kPieces = N * TB / kRows, kOut = (kPieces + ST::kMixers - 1) / ST::kMixers;
         auto store_dx = [&](int t) {
@@ -602,8 +638,10 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
                 const int at = wave + i * ST::kMixers, piece = min(at, kPieces - 1), j = piece / (TB / kRows), row = lane_row(piece % (TB / kRows) * kRows);
                 const int c = lane_col(row);
                 const uint4 v = *reinterpret_cast<const uint4 *>(g + piece * 1024 + lane * 16);
-                if (at < kPieces && sb + row < b_end && c < C)  // C % 8 == 0: eight channels are inside or outside
-                    st16<true>(a.dx + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+                if (at < kPieces && sb + row < b_end && c < C) {  // C % 8 == 0: eight channels are inside or outside
+                    if constexpr (F32) st16<true>(static_cast<float *>(a.dx) + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+                    else st16<true>(static_cast<bf16_t *>(a.dx) + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+                }
             }
         };
         // dphi: 32-column tiles wave, wave + kMixers (stream, 32-channel group)
@@ -634,8 +672,8 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
             lds_floats<N * N>(co + l16 * N * N, &Mr[0][0]);
 #pragma unroll
             for (int j = 0; j < N; j++) {
-                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * CW * 2 + row_at);
-                gr[j] = *reinterpret_cast<const uint2 *>(gs + j * TB * CW * 2 + row_at);
+                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * kRowBytes + row_at);
+                gr[j] = *reinterpret_cast<const uint2 *>((F32 ? st : gs) + j * TB * kRowBytes + row_dy);
             }
             __builtin_amdgcn_sched_barrier(0);
             const bf16x8_t al = *reinterpret_cast<const bf16x8_t *>(st + ST::kP + 1024 + lane * 16);
@@ -644,10 +682,10 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
                 const int tile = wave + k * ST::kMixers, c = (tile % (CW / 32)) * 4 + tr_c;
                 if (kCols % ST::kMixers != 0 && tile >= kCols) break;
                 typedef __attribute__((address_space(3))) lds_tr_v4i16 *lds_ptr;
-                const char *xs = st + (tile / (CW / 32) * TB + tr_row) * CW * 2 + (tr_q & 1) * 8;
-                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(xs + (c ^ slab_swizzle<CW>(tr_row)) * 16)));
+                const char *xs = st + (tile / (CW / 32) * TB + tr_row) * kRowBytes + (tr_q & 1) * 8;
+                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(xs + (c ^ slab_swizzle<ST::kRing>(tr_row)) * 16)));
                 const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (lds_ptr)(xs + 4 * CW * 2 + (c ^ slab_swizzle<CW>(tr_row + 4)) * 16)));
+                    (lds_ptr)(xs + 4 * kRowBytes + (c ^ slab_swizzle<ST::kRing>(tr_row + 4)) * 16)));
                 const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
                 acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, xf, acc[k], 0, 0, 0);
                 acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, xf, acc[k], 0, 0, 0);
@@ -667,7 +705,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
                 k2 = sc[128] * qinv * qinv * qinv * inv_c;
             }
             float dfv[4];
-            uint32_t out[N][2];
+            uint32_t out[N][F32 ? 4 : 2];
 #pragma unroll
             for (int p = 0; p < 2; p++) {  // channel pairs
                 float r[N][2];
@@ -697,10 +735,20 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
                     }
                 }
 #pragma unroll
-                for (int j = 0; j < N; j++) out[j][p] = pack_bf16x2(r[j][0], r[j][1]);
+                for (int j = 0; j < N; j++) {
+                    if constexpr (F32) {
+                        out[j][2 * p] = __float_as_uint(r[j][0]);
+                        out[j][2 * p + 1] = __float_as_uint(r[j][1]);
+                    } else {
+                        out[j][p] = pack_bf16x2(r[j][0], r[j][1]);
+                    }
+                }
             }
 #pragma unroll
-            for (int j = 0; j < N; j++) *reinterpret_cast<uint2 *>(gs + j * TB * CW * 2 + row_at) = make_uint2(out[j][0], out[j][1]);
+            for (int j = 0; j < N; j++) {
+                if constexpr (F32) *reinterpret_cast<uint4 *>(gs + j * TB * kRowBytes + row_place(cl >> 2)) = make_uint4(out[j][0], out[j][1], out[j][2], out[j][3]);
+                else *reinterpret_cast<uint2 *>(gs + j * TB * kRowBytes + row_at) = make_uint2(out[j][0], out[j][1]);
+            }
             if (INJECT && a.df && sb + l16 < b_end && c0 + cl < C)
                 store_vec<bf16_t, 4>(a.df + (size_t)sb * C + (uint32_t)(l16 * C + c0 + cl), dfv);
         }
@@ -767,14 +815,15 @@ bool bwd_slab_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) {
 //        1280 x 2560 37.1 | 37.0   1000 x 3712 43.5 | 42.6   4000 x 2560 80.4 | 79.2   8192 x 2560 185 | 164
 //   n=3  1500 x 1920 31.6 | 29.5   n=2  4000 x 1024 34.4 | 32.1   1000 x 2560 29.6 | 27.2
 // The lines: n = 4 up to 1280 channels, or below 12 M activation elements.
-static int slab_width(int B, int n, int C) {
+static int slab_width(int B, int n, int C, bool f32 = false) {
+    if (f32) return 64;
     if (const int forced = tuning_get(kTuneSlabWidth)) return forced == 1 ? 64 : 128;
     return n == 4 && (C <= 1280 || (long long)B * n * C < 12'000'000) ? 64 : 128;
 }
 
 int bwd_slab_batch_splits(int B, int n, int C, int y_dtype) {
-    const bool staged = y_dtype == kBF16;
-    const int width = staged ? slab_width(B, n, C) : kSlabCW, slabs = (C + width - 1) / width;
+    const bool staged = y_dtype != kF32;
+    const int width = staged ? slab_width(B, n, C, y_dtype == kF32AsBF16) : kSlabCW, slabs = (C + width - 1) / width;
     const int tiles = (B - 1) / (staged ? 16 : 32) + 1;
     if (const int forced = tuning_get(kTuneSlabSplits); forced > 0) {  // experiment hook
         return forced < tiles ? forced : tiles;
@@ -815,25 +864,28 @@ hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const voi
                            const float *cx, const void *dPb, const void *dPT, int BP, const float *dt,
                            void *dx, void *df, float *dphi_part, double *dw_part, double *dt_part, int S,
                            int B, int n, int C, hipStream_t stream) {
-    const int tiles = y_dtype == kBF16 ? (B - 1) / 16 + 1 : (B + 31) / 32;
+    const int tiles = y_dtype != kF32 ? (B - 1) / 16 + 1 : (B + 31) / 32;
     if (S < 1 || S > tiles) return hipErrorInvalidValue;
     BwdSlabArgs a{dy, static_cast<const bf16_t *>(x), w, f_inject, static_cast<const bf16_t *>(phi),
                   Hpre, Hpost, M, q, s1, cx, static_cast<const bf16_t *>(dPb),
-                  static_cast<const bf16_t *>(dPT), dt, static_cast<bf16_t *>(dx),
+                  static_cast<const bf16_t *>(dPT), dt, dx,
                   static_cast<bf16_t *>(df), dphi_part, dw_part, dt_part, w_dtype == kBF16, B, BP, n, C, tiles};
-    if (y_dtype == kBF16) {
-        const int cw = slab_width(B, n, C);
+    if (y_dtype != kF32) {
+        const bool f32 = y_dtype == kF32AsBF16;
+        if (f32 && (f_inject || C % 64 != 0)) return hipErrorInvalidValue;
+        const int cw = slab_width(B, n, C, f32);
         dim3 grid((C + cw - 1) / cw, S);
-#define MHC_SLAB(N, CW, INJ)                                                                                      \
+#define MHC_SLAB(N, CW, INJ, F32)                                                                                  \
     do {                                                                                                          \
-        constexpr size_t lds = SlabStage<N, CW>::kLds;                                                            \
-        if (hipError_t e = allow_dynamic_lds<&bwd_slab_stage_kernel<N, CW, INJ>>(lds); e != hipSuccess) return e; \
-        bwd_slab_stage_kernel<N, CW, INJ><<<grid, SlabStage<N, CW>::kThreads, lds, stream>>>(a);                                      \
+        constexpr size_t lds = SlabStage<N, CW, F32>::kLds;                                                          \
+        if (hipError_t e = allow_dynamic_lds<&bwd_slab_stage_kernel<N, CW, INJ, F32>>(lds); e != hipSuccess) return e; \
+        bwd_slab_stage_kernel<N, CW, INJ, F32><<<grid, SlabStage<N, CW, F32>::kThreads, lds, stream>>>(a);                                     \
     } while (0)
 #define MHC_SLAB_N(N)                                                                       \
     do {                                                                                    \
-        if (cw == 64) { if (f_inject) MHC_SLAB(N, 64, true); else MHC_SLAB(N, 64, false); } \
-        else { if (f_inject) MHC_SLAB(N, 128, true); else MHC_SLAB(N, 128, false); }        \
+        if (f32) MHC_SLAB(N, 64, false, true);                                              \
+        else if (cw == 64) { if (f_inject) MHC_SLAB(N, 64, true, false); else MHC_SLAB(N, 64, false, false); } \
+        else { if (f_inject) MHC_SLAB(N, 128, true, false); else MHC_SLAB(N, 128, false, false); }        \
     } while (0)
         switch (n) {
             case 1: MHC_SLAB_N(1); break;

@@ -139,6 +139,25 @@ bool f32_as_bf16_accepted(int B, int n, int C, int iters) {
            bwd_resident_supported(kF32AsBF16, kF32, kBF16, n, C, iters) && proj_bwd_addx_supported(n);
 }
 
+// Whether the backward of float32 storage takes the tiled path (channel sums that leave x and dy in bf16, slab) instead of the
+// resident one.  Backward us, tiled | resident, on either side of the line and beyond:
+//   n=1 C=256 B=600 17 | 17, 1300 20 | 27;  C=1280 510 20 | 20, 580 20 | 24;  C=4096 260 20 | 21, 4369 118 | 192
+//   n=2 C=512 600 18 | 17, 800 19 | 20;  C=1280 510 21 | 20, 580 23 | 25;  C=4096 300 27 | 32, 3000 108 | 177
+//   n=3 C=512 760 20 | 20, 1000 24 | 26;  C=1280 510 25 | 23, 580 25 | 26;  C=2560 330 26 | 27;  C=3136 3000 124 | 199
+//   n=4 C=640 720 25 | 24, 1000 27 | 29, 8000 98 | 131;  C=1280 510 28 | 24, 760 30 | 31, 4369 113 | 142;  C=2560 330 33 | 32, 513 39 | 46,
+//       2000 90 | 133;  C=4096 400 42 | 43
+//   at most 256 channels the resident path splits the batch beyond 1536 samples: n=4 C=256 1536 28 | 30, 2000 28 | 26, 4369 37 | 39
+bool bwd_f32_tiled(int B, int n, int C) {
+    if (n > 4 || C % 64 != 0) return false;
+    if (const int hook = tuning_get(kTuneResident)) return hook == 1;
+    if (C <= 256) {
+        const int from[4] = {700, 850, 1000, 1150}, again[4] = {2000, 2000, 2000, 4000};
+        return B > 1536 ? B >= again[n - 1] : B >= from[n - 1];
+    }
+    const int least[4] = {280, 280, 320, 420}, most[4] = {620, 740, 950, 1000}, per_row[4] = {720'000, 720'000, 730'000, 880'000};
+    return B >= std::max(least[n - 1], std::min(most[n - 1], per_row[n - 1] / C));
+}
+
 int max_ksplit(int B, int n, int C) {
     const int a = proj_fwd_ksplit(kBF16, kBF16, B, n, C), b = proj_fwd_ksplit(kF32, kF32, B, n, C);
     return a > b ? a : b;
@@ -179,7 +198,7 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     w.s1 = c.floats(B);
     // partial sums of dw and dt: float32 rows of at most B, float64 rows of the slab kernels or of the resident
     // backward's second launch with a split batch
-    const int bs3 = n <= 4 ? std::max(bwd_slab_batch_splits(B, n, C, kBF16), bwd_slab_batch_splits(B, n, C, kF32)) : 1;
+    const int bs3 = n <= 4 ? std::max({bwd_slab_batch_splits(B, n, C, kBF16), bwd_slab_batch_splits(B, n, C, kF32), bwd_slab_batch_splits(B, n, C, kF32AsBF16)}) : 1;
     const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1, bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
     // (also where the resident path is preferred: it does not take more than 32 Sinkhorn iterations)
     const bool slab8 = n >= 5 && n <= 8 && C % 8 == 0;
@@ -696,6 +715,18 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
     const int D = n * n + 2 * n, DP = padded_D(n);
     const bool mfma = proj_bwd_mfma_supported(x_dtype == kF32AsBF16 ? kBF16 : x_dtype, phi_dtype, C);
     BwdCoefOut out{ws.dt, ws.dP, ws.cx, ws.s1, nullptr, mfma ? ws.dPb : nullptr, ws.dPT, ws.BP};
+    if (x_dtype == kF32AsBF16 && !f_inject && bwd_f32_tiled(B, n, C)) {
+        // float32 storage, large batches: the channel sums round x and dy once and leave both where dx will be; the slab kernel
+        // reads them there, half the bytes, and puts dx in their place
+        MHC_LAUNCH(launch_mix_bwd_reduce_f32_as_bf16(static_cast<const float *>(dy), static_cast<const float *>(x), w, w_dtype, H_pre, H_post, M,
+                                                     q, P, r, alpha, bias + 2 * n, sk_state, out, dx, B, n, C, iters, eps, st));
+        const int S = bwd_slab_batch_splits(B, n, C, kF32AsBF16);
+        MHC_LAUNCH(launch_bwd_slab(dx, kF32AsBF16, nullptr, w, w_dtype, nullptr, phi, H_pre, H_post, M, q, ws.s1, ws.cx, ws.dPb, ws.dPT, ws.BP,
+                                   ws.dt, dx, nullptr, S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
+                                   reinterpret_cast<double *>(ws.dtpart), S, B, n, C, st));
+        MHC_LAUNCH(launch_finalize(ws.u, S, C, dw, ws.dtpart, S, D, dbias, dalpha, ws.dphi_part, S, (size_t)D * n * C, dphi, st, true));
+        return MHC_OK;
+    }
     // (rows that are no multiple of 8 elements: these two launches are the only matrix-core ones that take them)
     if (bwd_resident_supported(x_dtype, y_dtype, phi_dtype, n, C, iters) && proj_bwd_addx_supported(n) &&
         (bwd_resident_preferred(B, n, C) || x_dtype == kF32AsBF16 || C % 8 != 0)) {

@@ -23,6 +23,8 @@ struct BwdReduceArgs {
     // backward, which then has half its chain left (SkWg::save_state layout, (2 T + 2) * NP floats)
     const float *static_logits = nullptr;
     float *static_state = nullptr;
+    // float32 storage of bf16 arithmetic: x and dy in bf16 go here, 128 bytes of x and 128 of dy for every 64 channels of a row
+    void *copy = nullptr;
     int per_wg = 1;  // gram_quad_kernel: samples per workgroup, up to four
 };
 

@@ -145,6 +145,11 @@ struct BwdCoefOut {
     int BP;               // row pitch of dPT, a multiple of 32 that is >= B
 };
 
+hipError_t launch_mix_bwd_reduce_f32_as_bf16(const float *dy, const float *x, const void *w, int w_dtype, const float *Hpre, const float *Hpost,
+                                             const float *M, const float *q, const float *P, const float *r, const float *alpha,
+                                             const float *b_res, const float *sk_state, BwdCoefOut out, void *copy, int B, int n, int C,
+                                             int T, float eps, hipStream_t stream);
+
 // Per-sample reductions over c (dM, dHpost, dHpre, s1) and, for dynamic H, the coefficient
 // backward (activation derivatives + exact Sinkhorn backward) in the same launch.
 hipError_t launch_mix_bwd_reduce(const void *dy, int y_dtype, const void *x, int x_dtype,

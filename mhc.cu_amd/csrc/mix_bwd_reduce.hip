@@ -225,6 +225,56 @@ __global__ __launch_bounds__(64) void coef_bwd_small_kernel(BwdReduceArgs a) {
 // Output: raw[b][part][m][i][j] (NP x NP each), m = dM | W1 | XX.
 // =============================================================================================
 
+// The same from float32 storage: of a step of 128 channels a lane holds four of either half of 64, so that every load is one run
+// of 256 bytes per stream (which channels of a step meet is the same for dy, x and w, and that is all the sums ask for).
+template <int NB> struct GramF32 {
+    float4 g[NB][2], x[NB][2];
+    uint32_t w[8];
+    bool w16;
+    __device__ __forceinline__ void load(const float *const (&gb)[NB], const float *const (&xb)[NB], int c, int c2) {
+#pragma unroll
+        for (int I = 0; I < NB; I++) {
+            g[I][0] = *reinterpret_cast<const float4 *>(gb[I] + c);
+            x[I][0] = *reinterpret_cast<const float4 *>(xb[I] + c);
+            g[I][1] = *reinterpret_cast<const float4 *>(gb[I] + c2);
+            x[I][1] = *reinterpret_cast<const float4 *>(xb[I] + c2);
+        }
+    }
+    __device__ __forceinline__ void load_w(const bf16_t *p, int c, int c2) {
+        w16 = true;
+        const uint2 a = *reinterpret_cast<const uint2 *>(p + c), b = *reinterpret_cast<const uint2 *>(p + c2);
+        w[0] = a.x; w[1] = a.y; w[2] = b.x; w[3] = b.y;
+    }
+    __device__ __forceinline__ void load_w(const float *p, int c, int c2) {
+        w16 = false;
+        const uint4 a = *reinterpret_cast<const uint4 *>(p + c), b = *reinterpret_cast<const uint4 *>(p + c2);
+        w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w; w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
+    }
+    __device__ __forceinline__ void get_w(float (&v)[8]) const {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            v[2 * k] = w16 ? bf16lo_to_f32(w[k]) : __uint_as_float(w[2 * k]);
+            v[2 * k + 1] = w16 ? bf16hi_to_f32(w[k]) : __uint_as_float(w[2 * k + 1]);
+        }
+    }
+    __device__ __forceinline__ void round(int I, uint4 &gr, uint4 &xr) const { gr = pack8(g[I][0], g[I][1]); xr = pack8(x[I][0], x[I][1]); }
+    __device__ static __forceinline__ uint4 pack8(const float4 &a, const float4 &b) {
+        return make_uint4(pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w));
+    }
+};
+// to: this lane's 8 bytes of the step's first block (128 bytes of x, 128 of dy); the second block lies 256 bytes behind
+__device__ __forceinline__ void gram_copy(char *to, const uint4 &g, const uint4 &x, bool second) {
+    st8<false>(to, x.x, x.y);
+    st8<false>(to + 128, g.x, g.y);
+    if (second) {
+        st8<false>(to + 256, x.z, x.w);
+        st8<false>(to + 384, g.z, g.w);
+    }
+}
+__device__ __forceinline__ uint4 masked_halves(uint4 v, bool first, bool second) {
+    return make_uint4(first ? v.x : 0u, first ? v.y : 0u, second ? v.z : 0u, second ? v.w : 0u);
+}
+
 // FUSED (one column part per sample): the first lanes of wave 0 go on with the sample's coefficient
 // backward (CoefBwdSmall) as soon as the sums are complete, its other inputs requested at the start;
 // with several workgroups per CU the serial Sinkhorn chain of one runs under the loads of the others,
@@ -234,8 +284,11 @@ __global__ __launch_bounds__(64) void coef_bwd_small_kernel(BwdReduceArgs a) {
 // 128 registers, four workgroups per CU: their coefficient steps, serial chains on one wave each, hide behind each other (8 x 8 with
 // as many registers as it likes, 138, has three; backward us: n=8 B=2000 C=2560 102.9 -> 100.1, B=3000 C=512 65.3 -> 63.1, n=6
 // B=3000 C=768 57.6 -> 55.1, n=5 B=2000 C=1280 51.5 -> 49.6; five workgroups spill: 122.7, 76.9).
-template <int NP, int WMODE, bool FUSED, bool STATIC = false>
-__global__ __launch_bounds__(256, 4) void gram_small_kernel(BwdReduceArgs a) {
+// F32 (with FUSED): x and dy in float32, rounded to bf16 as they arrive; a.copy takes what they became, for the slab kernel behind.
+template <int NP, int WMODE, bool FUSED, bool STATIC = false, bool F32 = false>
+__global__ __launch_bounds__(256, F32 ? 3 : 4) void gram_small_kernel(BwdReduceArgs a) {
+    static_assert(!F32 || (FUSED && !STATIC && WMODE != kGramInject), "the float32 form of the dynamic layer");
+    using TS = typename std::conditional<F32, float, bf16_t>::type;
     static_assert(NP == 4 || NP == 8, "stream groups of four");
     static_assert(FUSED || !STATIC, "the static tail runs inside the launch");
     using SK = SkSmall<NP>;
@@ -265,14 +318,14 @@ __global__ __launch_bounds__(256, 4) void gram_small_kernel(BwdReduceArgs a) {
     const int blk = lane >> 2, i = lane & 3;
     const int nsteps = (C + 127) / 128, spp = (nsteps + a.parts - 1) / a.parts;
     const int s_begin = part * spp, s_end = min(nsteps, s_begin + spp);
-    const bf16_t *gb[NB], *xb[NB];
+    const TS *gb[NB], *xb[NB];
     bool sv[NB];
 #pragma unroll
     for (int I = 0; I < NB; I++) {
         sv[I] = 4 * I + i < n;  // streams >= n: masked below
         const size_t row = (size_t)b * n * C + (size_t)(sv[I] ? 4 * I + i : 0) * C;
-        gb[I] = static_cast<const bf16_t *>(a.dy) + row;
-        xb[I] = static_cast<const bf16_t *>(a.x) + row;
+        gb[I] = static_cast<const TS *>(a.dy) + row;
+        xb[I] = static_cast<const TS *>(a.x) + row;
     }
     const bf16_t *fb = inject ? static_cast<const bf16_t *>(a.f_inject) + (size_t)b * C : nullptr;
 
@@ -293,15 +346,25 @@ __global__ __launch_bounds__(256, 4) void gram_small_kernel(BwdReduceArgs a) {
         uint4 gr[U][NB], xr[U][NB], fr[U];
         RawVec<bf16_t, 8> wb[U];
         RawVec<float, 8> wf[U];
+        GramF32<NB> fl[F32 ? U : 1];
 #pragma unroll
         for (int u = 0; u < U; u++) {
+            if constexpr (F32) {
+                const int st = s0 + SW * u < s_end ? s0 + SW * u : s_begin, c = st * 128 + blk * 4, c2 = min(c + 64, C - 4);
+                fl[u].load(gb, xb, c, c2);
+                if constexpr (WMODE == kGramWBf16) fl[u].load_w(static_cast<const bf16_t *>(a.w), c, c2);
+                else fl[u].load_w(static_cast<const float *>(a.w), c, c2);
+                continue;
+            }
             const int c = (s0 + SW * u) * 128 + blk * 8;
             const bool in = s0 + SW * u < s_end && c < C;  // C % 8 == 0: a chunk is inside or outside
             const int cc = in ? c : 0;
 #pragma unroll
             for (int I = 0; I < NB; I++) {
-                gr[u][I] = *reinterpret_cast<const uint4 *>(gb[I] + cc);
-                xr[u][I] = *reinterpret_cast<const uint4 *>(xb[I] + cc);
+                if constexpr (!F32) {
+                    gr[u][I] = *reinterpret_cast<const uint4 *>(gb[I] + cc);
+                    xr[u][I] = *reinterpret_cast<const uint4 *>(xb[I] + cc);
+                }
             }
             if constexpr (inject) fr[u] = *reinterpret_cast<const uint4 *>(fb + cc);
             else if constexpr (WMODE == kGramWBf16) wb[u].load(static_cast<const bf16_t *>(a.w) + cc);
@@ -312,7 +375,19 @@ __global__ __launch_bounds__(256, 4) void gram_small_kernel(BwdReduceArgs a) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            {
+            if constexpr (F32) {
+                // the row may end with the first half of a step
+                const int st = s0 + SW * u;
+                const bool in = st < s_end, in2 = in && st * 128 + 64 < C;
+#pragma unroll
+                for (int I = 0; I < NB; I++) {
+                    fl[u].round(I, gr[u][I], xr[u][I]);
+                    if (in && sv[I])
+                        gram_copy(static_cast<char *>(a.copy) + (((size_t)b * n + 4 * I + i) * C + st * 128) * 4 + blk * 8, gr[u][I], xr[u][I], in2);
+                    gr[u][I] = masked_halves(gr[u][I], in && sv[I], in2 && sv[I]);
+                    xr[u][I] = masked_halves(xr[u][I], in && sv[I], in2 && sv[I]);
+                }
+            } else {
                 const bool in = s0 + SW * u < s_end && (s0 + SW * u) * 128 + blk * 8 < C;
 #pragma unroll
                 for (int I = 0; I < NB; I++) {
@@ -343,7 +418,8 @@ __global__ __launch_bounds__(256, 4) void gram_small_kernel(BwdReduceArgs a) {
                 }
             } else {
                 float wv[8];
-                if constexpr (WMODE == kGramWBf16) wb[u].get(wv);
+                if constexpr (F32) fl[u].get_w(wv);
+                else if constexpr (WMODE == kGramWBf16) wb[u].get(wv);
                 else wf[u].get(wv);
 #pragma unroll
                 for (int I = 0; I < NB; I++) {
@@ -417,8 +493,11 @@ __global__ __launch_bounds__(256, 4) void gram_small_kernel(BwdReduceArgs a) {
 // eight iterations, and four steps per wave (80 registers and spills) lost to gram_small_kernel.
 // B=8192 n=4 C=2560: 72 -> 65 us (336 MB, 5.2 TB/s).
 constexpr int kGramQuadSteps = 33;
-template <int WMODE, int U>
-__global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduceArgs a) {
+// F32: as in gram_small_kernel.
+template <int WMODE, int U, bool F32 = false>
+__global__ __launch_bounds__(768, F32 ? (U <= 2 ? 6 : 4) : (U <= 2 ? 8 : 7)) void gram_quad_kernel(BwdReduceArgs a) {
+    static_assert(!F32 || WMODE != kGramInject, "an injected f takes the other kernels");
+    using TS = typename std::conditional<F32, float, bf16_t>::type;
     using SK = SkSmall<4>;
     using CB = CoefBwdSmall<4, false, true>;
     constexpr int K = CB::K, Q = SK::kPerWave;
@@ -471,17 +550,26 @@ __global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduc
         }
     }
     for (int k = 0; k < nb; k++) {
-        const bf16_t *gb = static_cast<const bf16_t *>(a.dy) + (size_t)(b0 + k) * n * C;
-        const bf16_t *xb = static_cast<const bf16_t *>(a.x) + (size_t)(b0 + k) * n * C;
+        const TS *gb = static_cast<const TS *>(a.dy) + (size_t)(b0 + k) * n * C;
+        const TS *xb = static_cast<const TS *>(a.x) + (size_t)(b0 + k) * n * C;
         uint4 gr[U], xr[U], fr[U];
+        GramF32<1> fl[F32 ? U : 1];
 #pragma unroll
         for (int u = 0; u < U; u++) {
+            if constexpr (F32) {
+                const int st = s_first + u * SW < nsteps ? s_first + u * SW : 0, c = st * 128 + blk * 4;
+                const float *const gi[1] = {gb + (size_t)(i < n ? i : 0) * C}, *const xi[1] = {xb + (size_t)(i < n ? i : 0) * C};
+                fl[u].load(gi, xi, c, min(c + 64, C - 4));
+                continue;
+            }
             // beyond the row: any valid chunk (dropped or masked below); streams >= n alias stream 0: their entries are
             // dropped where the sums are finished
             const int st = s_first + u * SW < nsteps ? s_first + u * SW : 0;
             const uint32_t at = (uint32_t)((i < n ? i : 0) * C + st * 128 + min(blk * 8, C - 8 - st * 128));
-            gr[u] = *reinterpret_cast<const uint4 *>(gb + at);
-            xr[u] = *reinterpret_cast<const uint4 *>(xb + at);
+            if constexpr (!F32) {
+                gr[u] = *reinterpret_cast<const uint4 *>(gb + at);
+                xr[u] = *reinterpret_cast<const uint4 *>(xb + at);
+            }
             if constexpr (inject)
                 fr[u] = load16_masked(reinterpret_cast<const uint4 *>(static_cast<const bf16_t *>(a.f_inject) + (size_t)(b0 + k) * C +
                                                                       st * 128 + min(blk * 8, C - 8 - st * 128)), i == 0);
@@ -497,7 +585,13 @@ __global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduc
         for (int u = 0; u < U; u++) {
             const int st = s_first + u * SW;
             if (st >= nsteps) break;
-            if ((st + 1) * 128 > C) {  // the row ends within this step
+            if constexpr (F32) {
+                const bool in2 = st * 128 + 64 < C;
+                fl[u].round(0, gr[u], xr[u]);
+                if (i < n) gram_copy(static_cast<char *>(a.copy) + (((size_t)(b0 + k) * n + i) * C + st * 128) * 4 + blk * 8, gr[u], xr[u], in2);
+                gr[u] = masked_halves(gr[u], true, in2);
+                xr[u] = masked_halves(xr[u], true, in2);
+            } else if ((st + 1) * 128 > C) {  // the row ends within this step
                 const bool in = st * 128 + blk * 8 < C;
                 gr[u].x = in ? gr[u].x : 0u; gr[u].y = in ? gr[u].y : 0u; gr[u].z = in ? gr[u].z : 0u; gr[u].w = in ? gr[u].w : 0u;
                 xr[u].x = in ? xr[u].x : 0u; xr[u].y = in ? xr[u].y : 0u; xr[u].z = in ? xr[u].z : 0u; xr[u].w = in ? xr[u].w : 0u;
@@ -511,7 +605,15 @@ __global__ __launch_bounds__(768, U <= 2 ? 8 : 7) void gram_quad_kernel(BwdReduc
                 acc[1] = mfma4(g1, bf16x4_of(fr[u].z, fr[u].w), acc[1]);
             } else {
                 float wv[8];
-                load_vec<TW, 8>(w_s + st * 128 + min(blk * 8, C - 8 - st * 128), wv);
+                if constexpr (F32) {
+                    float lo[4], hi[4];
+                    load_vec<TW, 4>(w_s + st * 128 + blk * 4, lo);
+                    load_vec<TW, 4>(w_s + min(st * 128 + blk * 4 + 64, C - 4), hi);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) { wv[e] = lo[e]; wv[4 + e] = hi[e]; }
+                } else {
+                    load_vec<TW, 8>(w_s + st * 128 + min(blk * 8, C - 8 - st * 128), wv);
+                }
                 // dy * w as a bf16 pair (rounded value + remainder), see gram_small_kernel
                 const uint32_t gw[4] = {gr[u].x, gr[u].y, gr[u].z, gr[u].w};
                 uint32_t hw[4], lw[4];
@@ -1139,7 +1241,10 @@ static hipError_t launch_gram_small(BwdReduceArgs a, hipStream_t stream) {
             const unsigned block = 64 * (SW + 1), grid = (a.B - 1) / per_wg + 1;
 #define MHC_GRAM(UU)                                                                                        \
     do {                                                                                                    \
-        if (a.f_inject) gram_quad_kernel<kGramInject, UU><<<grid, block, smem, stream>>>(a);                \
+        if (a.copy) {                                                                                       \
+            if (a.w_bf16) gram_quad_kernel<kGramWBf16, UU, true><<<grid, block, smem, stream>>>(a);         \
+            else gram_quad_kernel<kGramWF32, UU, true><<<grid, block, smem, stream>>>(a);                   \
+        } else if (a.f_inject) gram_quad_kernel<kGramInject, UU><<<grid, block, smem, stream>>>(a);         \
         else if (a.w_bf16) gram_quad_kernel<kGramWBf16, UU><<<grid, block, smem, stream>>>(a);              \
         else gram_quad_kernel<kGramWF32, UU><<<grid, block, smem, stream>>>(a);                             \
     } while (0)
@@ -1152,9 +1257,14 @@ static hipError_t launch_gram_small(BwdReduceArgs a, hipStream_t stream) {
             return hipGetLastError();
         }
     }
-    if (gram_small_fused(a)) {
+    if (a.copy || gram_small_fused(a)) {
         a.parts = 1;
         const size_t smem = sizeof(float) * (SK::scaling_floats(a.T) + CB::kXch);  // at most 16 KB + 96 B
+        if (a.copy) {
+            if (a.w_bf16) gram_small_kernel<NP, kGramWBf16, true, false, true><<<a.B, 256, smem, stream>>>(a);
+            else gram_small_kernel<NP, kGramWF32, true, false, true><<<a.B, 256, smem, stream>>>(a);
+            return hipGetLastError();
+        }
         return launch_gram_small_kernel<NP, true>(a, smem, stream);
     }
     a.parts = gram_small_parts(a.B, a.C);
@@ -1318,6 +1428,19 @@ hipError_t launch_mix_bwd_reduce(const void *dy, int y_dtype, const void *x, int
     if (y_dtype == kBF16 && x_dtype == kBF16) return launch_large<bf16_t, bf16_t>(a, stream);
     if (y_dtype == kF32 && x_dtype == kBF16) return launch_large<float, bf16_t>(a, stream);
     return hipErrorInvalidValue;
+}
+
+// float32 storage of bf16 arithmetic (n <= 8, dynamic H, C % 64 == 0): the same sums from dy and x as they are stored, rounded on the
+// way in; copy [B, n, C] floats: both in bf16, where the slab kernel behind reads them (BwdReduceArgs::copy).
+hipError_t launch_mix_bwd_reduce_f32_as_bf16(const float *dy, const float *x, const void *w, int w_dtype, const float *Hpre, const float *Hpost,
+                                             const float *M, const float *q, const float *P, const float *r, const float *alpha,
+                                             const float *b_res, const float *sk_state, BwdCoefOut out, void *copy, int B, int n, int C,
+                                             int T, float eps, hipStream_t stream) {
+    if (n > 8 || C % 64 != 0 || T > 32 || !copy) return hipErrorInvalidValue;
+    BwdReduceArgs a{dy, x, w, nullptr, Hpre, Hpost, M, q, P, r, alpha, b_res, sk_state, out,
+                    n, w_dtype == kBF16, B, n, C, T, padded_D(n), eps, nullptr, 1};
+    a.copy = copy;
+    return n <= 4 ? launch_gram_small<4>(a, stream) : launch_gram_small<8>(a, stream);
 }
 
 // n > 16, dynamic H, bf16 dy and x: the channel sums, then ONE launch that holds the coefficient
