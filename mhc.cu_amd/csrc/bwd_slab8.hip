@@ -36,7 +36,7 @@ struct BwdSlab8Args {
     const float *Hpre, *Hpost, *M, *q, *s1, *cx;  // per sample
     const bf16_t *dPb, *dPT; // dP and dP^T hi / lo, fragment-major (frag_dpb, frag_dpt)
     const float *dt;         // [B, D+3]
-    bf16_t *dx;              // [B, N, C]
+    void *dx;                // [B, N, C], in the type of x's storage
     bf16_t *df;              // [B, C] or nullptr
     float *dphi_part;        // [S][D][N C]
     double *dw_part;         // [S][C]
@@ -44,27 +44,36 @@ struct BwdSlab8Args {
     int w_bf16, B, BP, C, tiles;  // tiles of 16 samples; split y takes tiles [y T / S, (y + 1) T / S)
 };
 
-template <int N> struct Slab8Stage {
-    static constexpr int CW = 64, TB = 16, kMixers = 4, kHolders = 4;  // waves
+// F32: float32 storage, as in bwd_slab.hip: the channel sums have left x and dy in bf16 where dx will be, and the bytes of CW channels
+// of dx hold CW of x, then CW of dy.  x and dy are one tile, two ahead, and dx leaves through two places of its own; at n = 7 and 8
+// the LDS holds that for 32 channels (two mixers).  Whole backward, resident path -> this: n=5 B=2000 C=2560 198 -> 116 us, n=6 B=3000
+// C=1024 146 -> 83, n=7 B=3000 C=1024 160 -> 109, n=8 B=4369 C=1024 269 -> 211.
+template <int N, bool F32> struct Slab8Stage {
+    static constexpr int CW = F32 && N > 6 ? 32 : 64, TB = 16, kMixers = CW / 16, kHolders = 4, kThreads = 64 * (kMixers + kHolders);  // waves
+    static constexpr int kRowBytes = CW * (F32 ? 4 : 2), kChunks = kRowBytes / 16, kRows = 1024 / kRowBytes;  // of a tile's row; rows per KiB
+    static constexpr int kRing8 = kChunks * 8;                         // what slab_swizzle() goes by
     static constexpr int D = N * N + 2 * N, NTD = (D + 31) / 32, DP = 32 * NTD;
-    static constexpr int kXRing = 3, kGRing = 4;                       // two tiles ahead
-    static constexpr int kTile = N * TB * CW * 2;                      // bytes of x or dy
+    static constexpr int kXRing = 3, kGRing = F32 ? 2 : 4;             // two tiles ahead
+    static constexpr int kTile = N * TB * kRowBytes;                   // bytes of x or dy, or of both; of dx
     // behind x: dP^T hi and lo of every 32 rows, dP of every 32 columns (1 KiB each), then blocks of 64 floats: M (a block
     // per sample, rows of 8), Hpre and Hpost (8 samples a block, 8 floats each), cx | q | s1
     static constexpr int kP = kTile, kPBlocks = 3 * NTD, kCoef = kP + kPBlocks * 1024, kCoefBlocks = TB + 2 + 2 + 3;
     static constexpr int kXBytes = kCoef + kCoefBlocks * 256;
     static constexpr int kG = kXRing * kXBytes, kW = kG + kGRing * kTile, kLds = kW + CW * 4;
-    static constexpr int kStreams = (N + 1) / 2;                       // KiB of x (and of dy) per holder
+    // KiB of x (and of dy), or of both, per holder: eight rows of every second stream, or (256-byte rows) four rows of every stream
+    static constexpr int kStreams = kRows == 8 ? (N + 1) / 2 : N, kLoads = kStreams * (F32 ? 1 : 2);
     static constexpr int kShare = (kPBlocks + kCoefBlocks + kHolders - 1) / kHolders;
     static constexpr int kCols = N * CW / 32, kAcc = (kCols + kHolders - 1) / kHolders;  // 32-column tiles of dphi, per holder
-    static_assert(32 * N * CW * 2 <= 2 * kTile && kLds <= 160 * 1024, "32 rows of phi fit two places of the dy ring");
+    static constexpr int kPhiAt = kG + (kGRing - 2) * kTile;           // prologue: 32 rows of phi, in two places of the dy / dx ring
+    static_assert(32 * N * CW * 2 <= 2 * kTile && kLds <= 160 * 1024, "32 rows of phi fit two places of the ring");
 };
 
-template <int N, bool INJECT>
-__global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
-    using ST = Slab8Stage<N>;
+template <int N, bool INJECT, bool F32>
+__global__ __launch_bounds__((Slab8Stage<N, F32>::kThreads), 2) void bwd_slab8_kernel(BwdSlab8Args a) {
+    static_assert(!(INJECT && F32), "an injected f takes the other kernels");
+    using ST = Slab8Stage<N, F32>;
     constexpr int CW = ST::CW, TB = ST::TB, D = ST::D, NTD = ST::NTD;
-    constexpr int kChunks = CW / 8, kRows = 512 / CW;  // 16-byte chunks per row, rows per KiB
+    constexpr int kChunks = ST::kChunks, kRows = ST::kRows, kRowBytes = ST::kRowBytes;
     typedef __attribute__((address_space(3))) lds_tr_v4i16 *lds_tr_ptr;
     extern __shared__ float smem_f[];
     char *const smem = reinterpret_cast<char *>(smem_f);
@@ -84,22 +93,25 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
     const int hw = wave - ST::kMixers;  // holder index
 
     const auto lane_row = [&](int row0) { return row0 + lane / kChunks; };
-    const auto lane_col = [&](int row) { return c0 + ((lane % kChunks) ^ slab_swizzle<CW>(row)) * 8; };
+    const auto lane_chunk = [&](int row) { return (lane % kChunks) ^ slab_swizzle<ST::kRing8>(row); };
+    const auto lane_col = [&](int row) { return c0 + lane_chunk(row) * (F32 ? 4 : 8); };  // of x or dy; F32: of dx
 
     // ---- loads of a tile (holders) -------------------------------------------------------------------
     // holder h brings eight rows (h % 2) of the streams h / 2, h / 2 + 2 .. (the last one twice where they do not come out
     // even: every holder has the same number of instructions in flight) and its share of the blocks behind x
-    const int ld_row = lane_row((hw & 1) * kRows), ld_col = min(lane_col(ld_row), C - 8);
-    auto load_tile = [&](const bf16_t *src, int t, uint32_t dst) {
+    const int ld_row0 = kRows == 8 ? (hw & 1) * 8 : hw * 4, ld_row = lane_row(ld_row0);
+    const int ld_at = F32 ? c0 * 4 + lane_chunk(ld_row) * 16 : min(lane_col(ld_row), C - 8) * 2;  // bytes behind the row's first
+    auto load_tile = [&](const void *src, int t, uint32_t dst) {
+        constexpr int ES = F32 ? 4 : 2;
         const int sb = b_begin + t * TB;
-        const bf16_t *base = src + (size_t)sb * nC;
+        const char *base = static_cast<const char *>(src) + (size_t)sb * nC * ES;
         // slots beyond the batch alias its last sample, columns beyond C the last ones: they only meet zero columns of
-        // dP^T or land in rows and columns that are not stored
-        const uint32_t off = (uint32_t)(min(ld_row, b_end - sb - 1) * nC + ld_col) * 2;
+        // dP^T or land in rows and columns that are not stored (F32: C is a multiple of 64)
+        const uint32_t off = (uint32_t)min(ld_row, b_end - sb - 1) * nC * ES + ld_at;
 #pragma unroll
         for (int i = 0; i < ST::kStreams; i++) {
-            const int j = min((hw >> 1) + 2 * i, N - 1);
-            load_to_lds<16>(base + (size_t)j * C, off, dst + (j * TB + (hw & 1) * kRows) * CW * 2);
+            const int j = kRows == 8 ? min((hw >> 1) + 2 * i, N - 1) : i;
+            load_to_lds<16>(base + (size_t)j * C * ES, off, dst + (j * TB + ld_row0) * kRowBytes);
         }
     };
     struct Block {
@@ -136,7 +148,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
         const uint32_t st = smem_at + t % ST::kXRing * ST::kXBytes;
         const int sb = b_begin + t * TB;
         const uint32_t left = min(b_end - sb, TB);
-        load_tile(a.x, t, st);
+        load_tile(F32 ? a.dx : static_cast<const void *>(a.x), t, st);
 #pragma unroll
         for (int i = 0; i < ST::kShare; i++) {
             const Block &m = mine[i];
@@ -148,7 +160,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
                 load_to_lds<4>(m.src + (size_t)sb * m.step, min(m.at, left * m.step - 4), st + m.dst);
             }
         }
-        load_tile(a.dy, t, smem_at + ST::kG + t % ST::kGRing * ST::kTile);
+        if constexpr (!F32) load_tile(a.dy, t, smem_at + ST::kG + t % ST::kGRing * ST::kTile);
     };
 
     // ---- prologue: the first tiles requested; phi -> LDS, 32 rows at a time, row-major [32 d][N][CW] -> the mixers' fragments
@@ -159,15 +171,15 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
         load_all(0, mine);
         if (T > 1) load_all(1, mine);
     }
-    char *const phi_s = smem + ST::kG + 2 * ST::kTile;
+    char *const phi_s = smem + ST::kPhiAt;
     // mixer lane (l16, kq): the four channels from c0 + cl of sample l16
-    const int l16 = lane & 15, kq = lane >> 4, cl = 16 * (wave & 3) + 4 * kq;
+    const int l16 = lane & 15, kq = lane >> 4, cl = 16 * (wave % ST::kMixers) + 4 * kq;
     bf16x8_t phif[N][NTD];  // mixers: A operand, rows = this wave's 16 channels of a stream, contraction over 32 d
     // The mixers alone bring phi and w, all of it asked for at once, and none of these barriers waits for global memory: holders
     // that brought a part of it waited for their first tiles before they could hand it on.  Backward in graphs of ten: n=5 B=3000
     // C=1024 55.4 -> 54.3 us, n=7 B=700 C=2552 56.1 -> 55.1, n=8 B=2048 C=2560 99.5 -> 99.2.
-    constexpr int kPhiThreads = 64 * ST::kMixers, kPhiIters = N * 32 * kChunks / kPhiThreads;
-    static_assert(kPhiIters * kPhiThreads == N * 32 * kChunks, "whole chunks of phi for every mixer");
+    constexpr int kPhiThreads = 64 * ST::kMixers, kPc = CW / 8, kPhiIters = N * 32 * kPc / kPhiThreads;
+    static_assert(kPhiIters * kPhiThreads == N * 32 * kPc, "whole chunks of phi for every mixer");
     uint4 phir[NTD][kPhiIters];
     if (!holder) {
 #pragma unroll
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
 #pragma unroll
             for (int i = 0; i < kPhiIters; i++) {
                 const int e = tid + i * kPhiThreads;
-                const int d = 32 * kk + e / (N * kChunks), j = e / kChunks % N, c = c0 + e % kChunks * 8;
+                const int d = 32 * kk + e / (N * kPc), j = e / kPc % N, c = c0 + e % kPc * 8;
                 const bool ok = d < D && c < C;
                 phir[kk][i] = load16_masked(reinterpret_cast<const uint4 *>(a.phi + (ok ? (size_t)d * nC + (size_t)j * C + c : 0)), ok);
             }
@@ -224,13 +236,14 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) acc[k][m][i] = 0.f;
         // transposed reads of x: this lane's row (lo; hi: + 4) and its 8 bytes of the 32-channel group
-        const int q = lane & 3, row = (lane >> 5) * 8 + ((lane >> 2) & 3), ch = 4 * (hw & 1) + ((lane >> 4) & 1) * 2 + (q >> 1);
-        const int at_lo = row * CW * 2 + (ch ^ slab_swizzle<CW>(row)) * 16 + (q & 1) * 8;
-        const int at_hi = (row + 4) * CW * 2 + (ch ^ slab_swizzle<CW>(row + 4)) * 16 + (q & 1) * 8;
+        constexpr int kHalves = CW / 32;  // 32-column tiles of a stream
+        const int q = lane & 3, row = (lane >> 5) * 8 + ((lane >> 2) & 3), ch = 4 * (hw % kHalves) + ((lane >> 4) & 1) * 2 + (q >> 1);
+        const int at_lo = row * kRowBytes + (ch ^ slab_swizzle<ST::kRing8>(row)) * 16 + (q & 1) * 8;
+        const int at_hi = (row + 4) * kRowBytes + (ch ^ slab_swizzle<ST::kRing8>(row + 4)) * 16 + (q & 1) * 8;
         for (int p = 0; p < T; p++) {
             // tile p has landed: all but the next tile's instructions; for everybody behind the barrier, where everybody is
             // done with x of tile p - 1 and with dx of tile p - 2 as well, whose places tile p + 2 takes
-            if (p + 1 < T) wait_vmem<2 * ST::kStreams + ST::kShare>();
+            if (p + 1 < T) wait_vmem<ST::kLoads + ST::kShare>();
             else wait_vmem<0>();
             stage_barrier();
             if (p + 2 < T) load_all(p + 2, mine);
@@ -238,8 +251,8 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             bf16x8_t xf[ST::kAcc];
 #pragma unroll
             for (int k = 0; k < ST::kAcc; k++) {
-                const int tile = min(hw + 4 * k, ST::kCols - 1);  // (both have the channel half hw & 1: kCols is even)
-                const char *xs = st + (tile >> 1) * TB * CW * 2;
+                const int tile = min(hw + 4 * k, ST::kCols - 1);  // (64 channels: both have the half hw & 1, kCols is even)
+                const char *xs = st + tile / kHalves * TB * kRowBytes;
                 const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(xs + at_lo)));
                 const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(xs + at_hi)));
                 xf[k] = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
@@ -259,14 +272,14 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
         float *dphi_out = a.dphi_part + (size_t)blockIdx.y * D * nC;
 #pragma unroll
         for (int k = 0; k < ST::kAcc; k++) {
-            const int tile = hw + 4 * k, c = c0 + (tile & 1) * 32 + (lane & 31);
+            const int tile = hw + 4 * k, c = c0 + tile % kHalves * 32 + (lane & 31);
             if (tile < ST::kCols && c < C) {
 #pragma unroll
                 for (int m = 0; m < NTD; m++)
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
                         const int d = 32 * m + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-                        if (d < D) dphi_out[(size_t)d * nC + (size_t)(tile >> 1) * C + c] = acc[k][m][i];
+                        if (d < D) dphi_out[(size_t)d * nC + (size_t)(tile / kHalves) * C + c] = acc[k][m][i];
                     }
             }
         }
@@ -279,7 +292,9 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
         const float inv_c = 1.0f / (float)C;
         double usum[4] = {0.0, 0.0, 0.0, 0.0};  // float32 terms, a sample each: the walk may be hundreds of tiles long
         double dtsum[2] = {0.0, 0.0};  // columns lane, lane + 64 of dt
-        const int row_at = l16 * CW * 2 + (((cl >> 3) ^ slab_swizzle<CW>(l16)) * 16) + (kq & 1) * 8;  // this lane's 8 bytes of its sample's row
+        // this lane's 8 bytes of its sample's row of x, of dy (F32: behind x), and what it writes of dx
+        const auto row_place = [&](int chunk) { return l16 * kRowBytes + ((chunk ^ slab_swizzle<ST::kRing8>(l16)) * 16); };
+        const int row_at = row_place(cl >> 3) + (kq & 1) * 8, row_dy = F32 ? row_place(kChunks / 2 + (cl >> 3)) + (kq & 1) * 8 : row_at;
         constexpr int kPieces = N * TB / kRows, kOut = (kPieces + ST::kMixers - 1) / ST::kMixers;
         auto store_dx = [&](int t) {
             const int sb = b_begin + t * TB;
@@ -289,8 +304,10 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
                 const int at = wave + i * ST::kMixers, piece = min(at, kPieces - 1), j = piece / (TB / kRows);
                 const int row = lane_row(piece % (TB / kRows) * kRows), c = lane_col(row);
                 const uint4 v = *reinterpret_cast<const uint4 *>(g + piece * 1024 + lane * 16);
-                if (at < kPieces && sb + row < b_end && c < C)  // C % 8 == 0: eight channels are inside or outside
-                    st16<true>(a.dx + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+                if (at < kPieces && sb + row < b_end && c < C) {  // C % 8 == 0: eight channels are inside or outside
+                    if constexpr (F32) st16<true>(static_cast<float *>(a.dx) + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+                    else st16<true>(static_cast<bf16_t *>(a.dx) + (size_t)sb * nC + (uint32_t)(row * nC + j * C + c), v.x, v.y, v.z, v.w);
+                }
             }
         };
         for (int t = 0; t < T; t++) {
@@ -302,13 +319,14 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             stage_barrier();
             MHC_PHASE_ADD(kPhaseBwdSlab, pwg, 1, pclk);
             if (t > 0) store_dx(t - 1);
-            // dt is summed by the slabs in turn: this tile's rows by slab t % slabs, four rows per mixer
+            // dt is summed by the slabs in turn: this tile's rows by slab t % slabs, as many rows per mixer
+            constexpr int kDtRows = TB / ST::kMixers;
             const bool my_dt = t % slabs == slab;
-            float dtv[4][2];
+            float dtv[kDtRows][2];
             if (my_dt) {
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int b = min(sb + 4 * wave + r, b_end - 1);
+                for (int r = 0; r < kDtRows; r++) {
+                    const int b = min(sb + kDtRows * wave + r, b_end - 1);
                     const float *p = a.dt + (size_t)b * (D + 3);
                     dtv[r][0] = p[min(lane, D + 2)];
                     dtv[r][1] = p[min(lane + 64, D + 2)];
@@ -322,7 +340,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             const float *const Mb = co + l16 * 64;
             struct Row { uint2 g; float4 m0, m1; };
             auto row_of = [&](int i) {
-                return Row{*reinterpret_cast<const uint2 *>(gs + i * TB * CW * 2 + row_at),
+                return Row{*reinterpret_cast<const uint2 *>((F32 ? st : gs) + i * TB * kRowBytes + row_dy),
                            *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 * l16) & 63)),
                            *reinterpret_cast<const float4 *>(Mb + ((8 * i + 4 + 4 * l16) & 63))};
             };
@@ -371,7 +389,7 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
             float s_a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j = 0; j < N; j++) {
-                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * CW * 2 + row_at);
+                xr[j] = *reinterpret_cast<const uint2 *>(st + j * TB * kRowBytes + row_at);
                 s_a[0] += hpre[j] * bf16lo_to_f32(xr[j].x); s_a[1] += hpre[j] * bf16hi_to_f32(xr[j].x);
                 s_a[2] += hpre[j] * bf16lo_to_f32(xr[j].y); s_a[3] += hpre[j] * bf16hi_to_f32(xr[j].y);
             }
@@ -388,12 +406,13 @@ __global__ __launch_bounds__(512, 2) void bwd_slab8_kernel(BwdSlab8Args a) {
                 float r[4];
 #pragma unroll
                 for (int c = 0; c < 4; c++) r[c] = o[j][c] + hpre[j] * da[c] - cxv * xv[c];
-                *reinterpret_cast<uint2 *>(gs + j * TB * CW * 2 + row_at) = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
+                if constexpr (F32) *reinterpret_cast<float4 *>(gs + j * TB * kRowBytes + row_place(cl >> 2)) = make_float4(r[0], r[1], r[2], r[3]);
+                else *reinterpret_cast<uint2 *>(gs + j * TB * kRowBytes + row_at) = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
             }
             if (my_dt) {
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-                    if (sb + 4 * wave + r < b_end) { dtsum[0] += dtv[r][0]; dtsum[1] += dtv[r][1]; }
+                for (int r = 0; r < kDtRows; r++)
+                    if (sb + kDtRows * wave + r < b_end) { dtsum[0] += dtv[r][0]; dtsum[1] += dtv[r][1]; }
             }
             if (INJECT && a.df && sb + l16 < b_end && c0 + cl < C)
                 store_vec<bf16_t, 4>(a.df + (size_t)sb * C + (uint32_t)(l16 * C + c0 + cl), s_df);
@@ -435,7 +454,8 @@ bool bwd_slab8_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) 
     return x_dtype == kBF16 && y_dtype == kBF16 && phi_dtype == kBF16 && n >= 5 && n <= 8 && C % 8 == 0;
 }
 
-int bwd_slab8_slabs(int C) { return (C + 63) / 64; }
+static int slab8_width(int n, bool f32) { return f32 && n > 6 ? 32 : 64; }
+int bwd_slab8_slabs(int n, int C, bool f32) { return (C + slab8_width(n, f32) - 1) / slab8_width(n, f32); }
 
 // At most one workgroup per CU and at least three tiles each, and within that the splits that cost least: a tile is some 0.2 n us
 // of a walk, and from two splits on their partial dphi are written, read and added up, D n C elements each, while a single one
@@ -444,8 +464,8 @@ int bwd_slab8_slabs(int C) { return (C + 63) / 64; }
 //   n=8 C=2560 B=100 41.8 | 50.8 | 50.8 (2), 200 52.3 | 52.5 | 47.9 (4);  C=4104 100 46.2 | 57.7, 200 55.5 | 62.3 | 61.2 (3), 300 67.4 |
 //              69.0 | 66.6 (3);  C=8192 100 50.2 | 74.9, 300 77.0 | 92.5
 //   n=5 C=2560 B=100 33.6 | 32.3, 200 36.8 | 34.1 | 32.1 (4);  C=6144 100 35.2 | 40.9, 200 42.9 | 43.7, 300 51.7 | 48.4
-int bwd_slab8_batch_splits(int B, int n, int C) {
-    const int slabs = bwd_slab8_slabs(C), tiles = (B - 1) / 16 + 1;
+int bwd_slab8_batch_splits(int B, int n, int C, bool f32) {
+    const int slabs = bwd_slab8_slabs(n, C, f32), tiles = (B - 1) / 16 + 1;
     const auto per_split = [&](int s) { return (tiles + s - 1) / s; };
     int S = 1;
     if (const int hook = tuning_get(kTuneSlabSplits); hook > 0) {  // experiment hook
@@ -465,20 +485,25 @@ int bwd_slab8_batch_splits(int B, int n, int C) {
 hipError_t launch_bwd_slab8(const void *dy, const void *x, const void *w, int w_dtype, const void *f_inject, const void *phi,
                             const float *Hpre, const float *Hpost, const float *M, const float *q, const BwdCoefOut &co,
                             void *dx, void *df, float *dphi_part, double *dw_part, double *dt_part, int S, int B, int n, int C,
-                            hipStream_t stream) {
+                            hipStream_t stream, bool f32) {
     const int tiles = (B - 1) / 16 + 1;
-    if (S < 1 || S > tiles) return hipErrorInvalidValue;
+    if (S < 1 || S > tiles || (f32 && (f_inject || C % 64 != 0))) return hipErrorInvalidValue;
     const BwdSlab8Args a{static_cast<const bf16_t *>(dy), static_cast<const bf16_t *>(x), w, static_cast<const bf16_t *>(phi),
-                         Hpre, Hpost, M, q, co.s1, co.cx, co.dPb, co.dPT, co.dt, static_cast<bf16_t *>(dx),
+                         Hpre, Hpost, M, q, co.s1, co.cx, co.dPb, co.dPT, co.dt, dx,
                          static_cast<bf16_t *>(df), dphi_part, dw_part, dt_part, w_dtype == kBF16, B, co.BP, C, tiles};
-    const dim3 grid(bwd_slab8_slabs(C), S);
-#define MHC_SLAB8(N, INJ)                                                                                     \
+    const dim3 grid(bwd_slab8_slabs(n, C, f32), S);
+#define MHC_SLAB8(N, INJ, F32)                                                                                \
     do {                                                                                                      \
-        constexpr size_t lds = Slab8Stage<N>::kLds;                                                           \
-        if (hipError_t e = allow_dynamic_lds<&bwd_slab8_kernel<N, INJ>>(lds); e != hipSuccess) return e;      \
-        bwd_slab8_kernel<N, INJ><<<grid, 512, lds, stream>>>(a);                                              \
+        constexpr size_t lds = Slab8Stage<N, F32>::kLds;                                                      \
+        if (hipError_t e = allow_dynamic_lds<&bwd_slab8_kernel<N, INJ, F32>>(lds); e != hipSuccess) return e; \
+        bwd_slab8_kernel<N, INJ, F32><<<grid, Slab8Stage<N, F32>::kThreads, lds, stream>>>(a);                \
     } while (0)
-#define MHC_SLAB8_N(N) do { if (f_inject) MHC_SLAB8(N, true); else MHC_SLAB8(N, false); } while (0)
+#define MHC_SLAB8_N(N)                                                                                        \
+    do {                                                                                                      \
+        if (f32) MHC_SLAB8(N, false, true);                                                                   \
+        else if (f_inject) MHC_SLAB8(N, true, false);                                                         \
+        else MHC_SLAB8(N, false, false);                                                                      \
+    } while (0)
     switch (n) {
         case 5: MHC_SLAB8_N(5); break;
         case 6: MHC_SLAB8_N(6); break;

@@ -130,10 +130,8 @@ bool bwd_slab8_preferred(int B, int n, int C) {
 
 // Shapes for which the dynamic entry points take fp32 activations that are consumed as bf16
 // (MHC_F32_AS_BF16): the kernels that load fp32 storage directly are the narrow projection, the fused
-// n <= 8 forward and the two launches of the sample-resident backward.  That backward is taken for fp32
-// storage at every batch size, also where the tiled path is faster on bf16 storage: the alternative is
-// a cast pass over x on top of the tiled path (through the module, fp32 tensors, forward + backward:
-// B=1280 C=2560 n=4 186 -> 184 us, B=2560 C=1280 184 -> 176, B=1024 C=1280 111 -> 100).
+// n <= 8 forward, the two launches of the sample-resident backward and, for large batches of whole lines, the tiled backward
+// (bwd_f32_tiled).  Every batch size is taken: the alternative is a cast pass over x and dy.
 bool f32_as_bf16_accepted(int B, int n, int C, int iters) {
     return n <= 8 && C % 8 == 0 && layer_fwd_fused_supported(n, C, kF32) &&
            bwd_resident_supported(kF32AsBF16, kF32, kBF16, n, C, iters) && proj_bwd_addx_supported(n);
@@ -147,9 +145,24 @@ bool f32_as_bf16_accepted(int B, int n, int C, int iters) {
 //   n=4 C=640 720 25 | 24, 1000 27 | 29, 8000 98 | 131;  C=1280 510 28 | 24, 760 30 | 31, 4369 113 | 142;  C=2560 330 33 | 32, 513 39 | 46,
 //       2000 90 | 133;  C=4096 400 42 | 43
 //   at most 256 channels the resident path splits the batch beyond 1536 samples: n=4 C=256 1536 28 | 30, 2000 28 | 26, 4369 37 | 39
+//   n=5 C=320 925 30 | 34;  C=512 650 30 | 30, 850 32 | 36;  C=1024 450 31 | 30, 650 35 | 40, 4400 110 | 198;  C=2560 300 41 | 40, 450 43 | 46,
+//       2000 115 | 196
+//   n=6 C=512 650 32 | 31, 850 34 | 35;  C=1024 450 34 | 30, 650 38 | 41, 4400 126 | 239;  C=1536 399 37 | 37, 563 44 | 50;  C=2560 300
+//       45 | 42, 450 48 | 49, 2000 143 | 229
+//   n=7 C=512 650 33 | 31, 850 36 | 36, 1100 40 | 43;  C=1024 450 36 | 32, 650 42 | 44, 4400 156 | 273;  C=2560 450 59 | 57, 650 75 | 81, 2000
+//       192 | 282;  C=3136 568 88 | 85, 1183 150 | 164
+//   n=8 (slabs of 32 channels: shorter runs of a row, more partial sums) C=512 2000 63 | 62, 4400 114 | 118;  C=768 1700 75 | 71, 2600
+//       104 | 104;  C=1024 850 58 | 57, 1100 67 | 69, 4400 212 | 273;  C=1920 1100 113 | 112, 1700 164 | 184;  C=2560 1100 149 | 144, 1500
+//       198 | 222;  C=3072 1700 296 | 295
+//   at most 256 channels: n=5 C=64 3000 40 | 32, C=256 1100 32 | 34, 1500 34 | 31, 4400 54 | 55;  n=8 C=256 4400 74 | 63
 bool bwd_f32_tiled(int B, int n, int C) {
-    if (n > 4 || C % 64 != 0) return false;
+    if (n > 8 || C % 64 != 0) return false;
     if (const int hook = tuning_get(kTuneResident)) return hook == 1;
+    if (n == 8) return C >= 1024 && B >= std::max(1000, 5 * C / 8);
+    if (n > 4) {
+        const int least[3] = {340, 330, 450}, over_row[3] = {200'000, 215'000, 230'000};
+        return C > 256 && B >= std::max(least[n - 5] + over_row[n - 5] / C, n == 7 ? C / 4 : 0);
+    }
     if (C <= 256) {
         const int from[4] = {700, 850, 1000, 1150}, again[4] = {2000, 2000, 2000, 4000};
         return B > 1536 ? B >= again[n - 1] : B >= from[n - 1];
@@ -202,8 +215,10 @@ DynBwdWs carve_dyn_bwd(void *ws, int B, int n, int C) {
     const int bs5 = n <= 4 ? bwd_slab_f32_splits(B, C) : 1, bs6 = proj_bwd_addx_supported(n) ? proj_bwd_addx_splits(B, n, C) : 1;
     // (also where the resident path is preferred: it does not take more than 32 Sinkhorn iterations)
     const bool slab8 = n >= 5 && n <= 8 && C % 8 == 0;
-    const int bs7 = slab8 ? bwd_slab8_batch_splits(B, n, C) : 1;
-    const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : (slab8 ? (size_t)bs7 * bwd_slab8_slabs(C) : 0), parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
+    const bool slab8_f32 = slab8 && C % 64 == 0;  // float32 storage
+    const int bs7a = slab8 ? bwd_slab8_batch_splits(B, n, C, false) : 1, bs7b = slab8_f32 ? bwd_slab8_batch_splits(B, n, C, true) : 1;
+    const int bs7 = std::max(bs7a, bs7b);
+    const size_t slab64 = n <= 4 ? std::max(bs3, bs5) : (slab8 ? std::max((size_t)bs7a * bwd_slab8_slabs(n, C, false), slab8_f32 ? (size_t)bs7b * bwd_slab8_slabs(n, C, true) : 0) : 0), parts64 = bs6 > 1 ? proj_bwd_addx_sum_parts(B, bs6) : 0;
     w.u = c.floats(std::max((size_t)B, 2 * (n <= 4 ? slab64 : (size_t)(slab8 ? bs7 : 0))) * C);
     w.upart = c.floats(2 * parts64 * C);
     w.dtpart = c.floats(std::max((size_t)B, 2 * std::max(slab64, parts64)) * (D + 3));
@@ -720,6 +735,15 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         // reads them there, half the bytes, and puts dx in their place
         MHC_LAUNCH(launch_mix_bwd_reduce_f32_as_bf16(static_cast<const float *>(dy), static_cast<const float *>(x), w, w_dtype, H_pre, H_post, M,
                                                      q, P, r, alpha, bias + 2 * n, sk_state, out, dx, B, n, C, iters, eps, st));
+        if (n > 4) {
+            const int S = bwd_slab8_batch_splits(B, n, C, true);
+            MHC_LAUNCH(launch_bwd_slab8(nullptr, nullptr, w, w_dtype, nullptr, phi, H_pre, H_post, M, q, out, dx, nullptr,
+                                        S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u), reinterpret_cast<double *>(ws.dtpart),
+                                        S, B, n, C, st, true));
+            MHC_LAUNCH(launch_finalize(ws.u, S, C, dw, ws.dtpart, S * bwd_slab8_slabs(n, C, true), D, dbias, dalpha, ws.dphi_part, S,
+                                       (size_t)D * n * C, dphi, st, true));
+            return MHC_OK;
+        }
         const int S = bwd_slab_batch_splits(B, n, C, kF32AsBF16);
         MHC_LAUNCH(launch_bwd_slab(dx, kF32AsBF16, nullptr, w, w_dtype, nullptr, phi, H_pre, H_post, M, q, ws.s1, ws.cx, ws.dPb, ws.dPT, ws.BP,
                                    ws.dt, dx, nullptr, S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
@@ -797,11 +821,11 @@ int bwd_dynamic(const void *dy, int y_dtype, const void *x, int x_dtype, const v
         return MHC_OK;
     }
     if (mfma && bwd_slab8_supported(x_dtype, y_dtype, phi_dtype, n, C) && bwd_slab8_preferred(B, n, C)) {
-        const int S = bwd_slab8_batch_splits(B, n, C);
+        const int S = bwd_slab8_batch_splits(B, n, C, false);
         MHC_LAUNCH(launch_bwd_slab8(dy, x, w, w_dtype, f_inject, phi, H_pre, H_post, M, q, out, dx, df,
                                     S > 1 ? ws.dphi_part : dphi, reinterpret_cast<double *>(ws.u),
                                     reinterpret_cast<double *>(ws.dtpart), S, B, n, C, st));
-        MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S * bwd_slab8_slabs(C), D, dbias, dalpha,
+        MHC_LAUNCH(launch_finalize(ws.u, S, C, f_inject ? DwOut{} : dw, ws.dtpart, S * bwd_slab8_slabs(n, C, false), D, dbias, dalpha,
                                    ws.dphi_part, S, (size_t)D * n * C, dphi, st, true));
         return MHC_OK;
     }

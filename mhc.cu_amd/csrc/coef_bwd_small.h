@@ -23,8 +23,10 @@ struct BwdReduceArgs {
     // backward, which then has half its chain left (SkWg::save_state layout, (2 T + 2) * NP floats)
     const float *static_logits = nullptr;
     float *static_state = nullptr;
-    // float32 storage of bf16 arithmetic: x and dy in bf16 go here, 128 bytes of x and 128 of dy for every 64 channels of a row
+    // float32 storage of bf16 arithmetic: x and dy in bf16 go here, for every copy_block (64 or 32) channels of a row as many of x,
+    // then of dy
     void *copy = nullptr;
+    int copy_block = 64;
     int per_wg = 1;  // gram_quad_kernel: samples per workgroup, up to four
 };
 

@@ -209,12 +209,12 @@ hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const voi
 // The same for n = 5 .. 8 (bf16 dy and x), behind launch_mix_bwd_reduce (dP fragments, cx, s1, dt of `co`): dw_part [S][C],
 // dt_part [S bwd_slab8_slabs()][D+3].
 bool bwd_slab8_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C);
-int bwd_slab8_slabs(int C);
-int bwd_slab8_batch_splits(int B, int n, int C);
+int bwd_slab8_slabs(int n, int C, bool f32);  // f32: float32 storage of bf16 arithmetic, see launch_bwd_slab8
+int bwd_slab8_batch_splits(int B, int n, int C, bool f32);
 hipError_t launch_bwd_slab8(const void *dy, const void *x, const void *w, int w_dtype, const void *f_inject, const void *phi,
                             const float *Hpre, const float *Hpost, const float *M, const float *q, const BwdCoefOut &co,
                             void *dx, void *df, float *dphi_part, double *dw_part, double *dt_part, int S, int B, int n, int C,
-                            hipStream_t stream);
+                            hipStream_t stream, bool f32 = false);
 
 // The same for the fp32 tier (n <= 4, even C), behind launch_mix_bwd_reduce (dP [B, 32], cx, s1, dt of `co`):
 // dx, df and the batch-split partial sums of dphi [S][D][nC] and, in float64, dw [S][C] and dt [S][D+3],

@@ -262,13 +262,15 @@ template <int NB> struct GramF32 {
         return make_uint4(pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w));
     }
 };
-// to: this lane's 8 bytes of the step's first block (128 bytes of x, 128 of dy); the second block lies 256 bytes behind
-__device__ __forceinline__ void gram_copy(char *to, const uint4 &g, const uint4 &x, bool second) {
+// row: where dx of the step's 128 channels will be; blk: the lane's four channels of either half (BwdReduceArgs::copy)
+__device__ __forceinline__ void gram_copy(char *row, int blk, int block, const uint4 &g, const uint4 &x, bool second) {
+    const int dy = block * 2;
+    char *to = row + (block == 64 ? blk * 8 : (blk >> 3) * 128 + (blk & 7) * 8);
     st8<false>(to, x.x, x.y);
-    st8<false>(to + 128, g.x, g.y);
+    st8<false>(to + dy, g.x, g.y);
     if (second) {
         st8<false>(to + 256, x.z, x.w);
-        st8<false>(to + 384, g.z, g.w);
+        st8<false>(to + 256 + dy, g.z, g.w);
     }
 }
 __device__ __forceinline__ uint4 masked_halves(uint4 v, bool first, bool second) {
@@ -285,8 +287,10 @@ __device__ __forceinline__ uint4 masked_halves(uint4 v, bool first, bool second)
 // as many registers as it likes, 138, has three; backward us: n=8 B=2000 C=2560 102.9 -> 100.1, B=3000 C=512 65.3 -> 63.1, n=6
 // B=3000 C=768 57.6 -> 55.1, n=5 B=2000 C=1280 51.5 -> 49.6; five workgroups spill: 122.7, 76.9).
 // F32 (with FUSED): x and dy in float32, rounded to bf16 as they arrive; a.copy takes what they became, for the slab kernel behind.
+// One step in flight at 8 x 8, which leaves four workgroups per CU as well (backward us, two steps and two workgroups | two steps, three
+// workgroups and spills | one step: n=5 B=4369 C=1024 135 | 132 | 110, n=6 B=3000 C=1024 101 | 103 | 83, n=8 B=2000 C=1024 110 | 113 | 100).
 template <int NP, int WMODE, bool FUSED, bool STATIC = false, bool F32 = false>
-__global__ __launch_bounds__(256, F32 ? 3 : 4) void gram_small_kernel(BwdReduceArgs a) {
+__global__ __launch_bounds__(256, F32 && NP == 4 ? 3 : 4) void gram_small_kernel(BwdReduceArgs a) {
     static_assert(!F32 || (FUSED && !STATIC && WMODE != kGramInject), "the float32 form of the dynamic layer");
     using TS = typename std::conditional<F32, float, bf16_t>::type;
     static_assert(NP == 4 || NP == 8, "stream groups of four");
@@ -294,7 +298,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void gram_small_kernel(BwdReduceA
     using SK = SkSmall<NP>;
     using CB = CoefBwdSmall<NP, false, true, STATIC>;
     constexpr int NB = NP / 4;            // stream groups
-    constexpr int U = 2;                  // steps of a wave in flight
+    constexpr int U = F32 && NP == 8 ? 1 : 2;  // steps of a wave in flight
     constexpr int K = 3 * NP * NP;
     constexpr bool inject = WMODE == kGramInject;
     __shared__ float slot_s[K * 16];  // one slot per 16-lane row of the workgroup
@@ -336,12 +340,16 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void gram_small_kernel(BwdReduceA
         for (int I = 0; I < NB; I++)
 #pragma unroll
             for (int J = 0; J < NB; J++) acc[m][I][J] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // F32: the products of a step in sums of their own.  One chain over the row makes the mean error of dbias 1.4 times that of the
+    // resident path (n = 5 .. 8, C = 320 .. 1344), one over two steps 1.2 times, this 0.73 times.
+    const auto first_of = [](f32x4_t acc) { return F32 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc; };
+    const auto sum_of = [](f32x4_t acc, f32x4_t s) { return F32 ? acc + s : s; };
     MHC_PHASE_ADD(kPhaseGramSmall, pwg, 0, pclk);
 
     // FUSED: wave 0 is busy with the forward recompute while the others stream, so the steps are
     // shared by waves 1 .. 3 only
     constexpr int SW = FUSED ? 3 : 4;  // streaming waves
-    const int sw = FUSED ? wave - 1 : wave;
+    const int sw = F32 ? __builtin_amdgcn_readfirstlane(wave) - 1 : (FUSED ? wave - 1 : wave);
     for (int s0 = sw >= 0 ? s_begin + sw : s_end; s0 < s_end; s0 += SW * U) {
         uint4 gr[U][NB], xr[U][NB], fr[U];
         RawVec<bf16_t, 8> wb[U];
@@ -378,14 +386,15 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void gram_small_kernel(BwdReduceA
             if constexpr (F32) {
                 // the row may end with the first half of a step
                 const int st = s0 + SW * u;
-                const bool in = st < s_end, in2 = in && st * 128 + 64 < C;
+                if (st >= s_end) break;
+                const bool in2 = st * 128 + 64 < C;
 #pragma unroll
                 for (int I = 0; I < NB; I++) {
                     fl[u].round(I, gr[u][I], xr[u][I]);
-                    if (in && sv[I])
-                        gram_copy(static_cast<char *>(a.copy) + (((size_t)b * n + 4 * I + i) * C + st * 128) * 4 + blk * 8, gr[u][I], xr[u][I], in2);
-                    gr[u][I] = masked_halves(gr[u][I], in && sv[I], in2 && sv[I]);
-                    xr[u][I] = masked_halves(xr[u][I], in && sv[I], in2 && sv[I]);
+                    if (sv[I])
+                        gram_copy(static_cast<char *>(a.copy) + (((size_t)b * n + 4 * I + i) * C + st * 128) * 4, blk, a.copy_block, gr[u][I], xr[u][I], in2);
+                    gr[u][I] = masked_halves(gr[u][I], sv[I], in2 && sv[I]);
+                    xr[u][I] = masked_halves(xr[u][I], sv[I], in2 && sv[I]);
                 }
             } else {
                 const bool in = s0 + SW * u < s_end && (s0 + SW * u) * 128 + blk * 8 < C;
@@ -406,8 +415,10 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void gram_small_kernel(BwdReduceA
             for (int I = 0; I < NB; I++)
 #pragma unroll
                 for (int J = 0; J < NB; J++) {
-                    acc[0][I][J] = mfma4(g0[I], x0[J], acc[0][I][J]);
-                    acc[0][I][J] = mfma4(g1[I], x1[J], acc[0][I][J]);
+                    f32x4_t s = first_of(acc[0][I][J]);
+                    s = mfma4(g0[I], x0[J], s);
+                    s = mfma4(g1[I], x1[J], s);
+                    acc[0][I][J] = sum_of(acc[0][I][J], s);
                 }
             if constexpr (inject) {
                 const bf16x4_t f0 = bf16x4_of(fr[u].x, fr[u].y), f1 = bf16x4_of(fr[u].z, fr[u].w);
@@ -435,12 +446,15 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void gram_small_kernel(BwdReduceA
                     }
 #pragma unroll
                     for (int J = 0; J < NB; J++) {
-                        acc[1][I][J] = mfma4(bf16x4_of(hw[0], hw[1]), x0[J], acc[1][I][J]);
-                        acc[1][I][J] = mfma4(bf16x4_of(hw[2], hw[3]), x1[J], acc[1][I][J]);
-                        acc[1][I][J] = mfma4(bf16x4_of(lw[0], lw[1]), x0[J], acc[1][I][J]);
-                        acc[1][I][J] = mfma4(bf16x4_of(lw[2], lw[3]), x1[J], acc[1][I][J]);
-                        acc[2][I][J] = mfma4(x0[I], x0[J], acc[2][I][J]);
-                        acc[2][I][J] = mfma4(x1[I], x1[J], acc[2][I][J]);
+                        f32x4_t s = first_of(acc[1][I][J]), v = first_of(acc[2][I][J]);
+                        s = mfma4(bf16x4_of(hw[0], hw[1]), x0[J], s);
+                        s = mfma4(bf16x4_of(hw[2], hw[3]), x1[J], s);
+                        s = mfma4(bf16x4_of(lw[0], lw[1]), x0[J], s);
+                        s = mfma4(bf16x4_of(lw[2], lw[3]), x1[J], s);
+                        v = mfma4(x0[I], x0[J], v);
+                        v = mfma4(x1[I], x1[J], v);
+                        acc[1][I][J] = sum_of(acc[1][I][J], s);
+                        acc[2][I][J] = sum_of(acc[2][I][J], v);
                     }
                 }
             }
@@ -588,7 +602,7 @@ __global__ __launch_bounds__(768, F32 ? (U <= 2 ? 6 : 4) : (U <= 2 ? 8 : 7)) voi
             if constexpr (F32) {
                 const bool in2 = st * 128 + 64 < C;
                 fl[u].round(0, gr[u], xr[u]);
-                if (i < n) gram_copy(static_cast<char *>(a.copy) + (((size_t)(b0 + k) * n + i) * C + st * 128) * 4 + blk * 8, gr[u], xr[u], in2);
+                if (i < n) gram_copy(static_cast<char *>(a.copy) + (((size_t)(b0 + k) * n + i) * C + st * 128) * 4, blk, 64, gr[u], xr[u], in2);
                 gr[u] = masked_halves(gr[u], true, in2);
                 xr[u] = masked_halves(xr[u], true, in2);
             } else if ((st + 1) * 128 > C) {  // the row ends within this step
@@ -1440,6 +1454,7 @@ hipError_t launch_mix_bwd_reduce_f32_as_bf16(const float *dy, const float *x, co
     BwdReduceArgs a{dy, x, w, nullptr, Hpre, Hpost, M, q, P, r, alpha, b_res, sk_state, out,
                     n, w_dtype == kBF16, B, n, C, T, padded_D(n), eps, nullptr, 1};
     a.copy = copy;
+    a.copy_block = n > 6 ? 32 : 64;  // the widths of the slab kernels
     return n <= 4 ? launch_gram_small<4>(a, stream) : launch_gram_small<8>(a, stream);
 }
 
