@@ -95,8 +95,8 @@ template <int NP> __global__ __launch_bounds__(64) void coef_fwd_small_kernel(Co
 }
 
 // One workgroup (4 waves) per sample.  All 256 threads finish the split-K sums (D = n^2 + 2n
-// logits, KS partial sums each, eight loads in flight per thread), then run Sinkhorn with the
-// matrix spread over their registers (SkWg).
+// logits, KS partial sums each, eight loads in flight per thread), then Sinkhorn runs on the first
+// wave (SkWg).
 template <int NP, bool PRECISE, bool AGG = false>
 __global__ __launch_bounds__(256) void coef_fwd_lds_kernel(CoefArgs a) {
     using SK = SkWg<NP>;
@@ -233,7 +233,6 @@ __global__ __launch_bounds__(256) void coef_fwd_lds_kernel(CoefArgs a) {
     if (a.sk_state) SK::save_state(sk_s, a.T, a.sk_state + (size_t)b * SK::state_floats(a.T), tid, u, v);
     MHC_PHASE(kPhaseCoefFwdWide, b, 4);
     if constexpr (AGG) {
-        __syncthreads();  // hp_s (with zero iterations the Sinkhorn step has no barrier of its own)
         float acc[8], ssq = 0.f;
 #pragma unroll
         for (int k = 0; k < 8; k++) acc[k] = 0.f;

@@ -682,7 +682,7 @@ constexpr int kGramFloats = kGramMats * 1024;  // per (sample, part), row-major 
 // Static H: one workgroup behind the samples' (blockIdx.x == B) recomputes the Sinkhorn forward of the shared
 // logits with IEEE divisions and leaves the denominators of its iterations in a.static_state for the
 // static coefficient backward, the last launch of the call, which then has only the reverse sweep left.
-// The chain (about 6 us for 20 iterations of a 32 x 32 matrix) runs in the shadow of the channel sums.
+// The chain (about 3 us for 20 iterations of a 32 x 32 matrix) runs in the shadow of the channel sums.
 template <int NP>
 __device__ __forceinline__ void static_sinkhorn_forward_block(const BwdReduceArgs &a, float *smem) {
     using SK = SkWg<NP>;

@@ -195,13 +195,15 @@ template <int NP> struct SkSmall {
 
 // =============================================================================================
 // SkWg: one 256-thread workgroup per matrix, NP = 16 or 32, iterate kept in scaling form
-// diag(u) E diag(v) with E constant in registers: thread t owns E[a][b0 .. b0+EPL) with
+// diag(u) E diag(v) with E constant in registers: thread t brings E[a][b0 .. b0+EPL) with
 // (a, b0) = (t / LPR, (t % LPR) * EPL), and the running gradient there.
 //
-// forward(): every thread also holds the transposed elements E[b0 .. b0+EPL)[a] (copied once
-// through LDS), so both the row sums and the column sums are an in-register dot product plus a
-// reduction over the LPR lanes of a DPP row; only the vectors u and v travel through LDS (one
-// barrier per half-step).  The denominators rho/s of every iteration stay in LDS.
+// forward(): the first wave alone.  It holds E twice, by rows and by columns, 16 elements a lane (32 x 32: half a row, half a
+// column; 16 x 16: the 16-lane rows repeat each other), so that u and v stay one register each: a half-step is 16 products with
+// the vector broadcast inside a 16-lane row (DPP, in the instruction) and one v_permlane swap, 46 instructions an iteration and no
+// LDS round trip.  Spread over all four waves, u and v travelled through LDS with a barrier per half-step: 620 clocks an iteration
+// of 32 x 32.  Forward us, four waves -> one: n=32 B=128 C=1280 43.6 -> 41.8, n=16 B=64 C=1024 22.5 -> 20.1, B=3000 C=256 74.3 ->
+// 65.3, n=24 B=1000 C=256 54.4 -> 48.6.  The denominators rho/s of every iteration stay in LDS.
 // backward(): one copy of the product gradient x iterate; row sums inside a DPP row, column sums inside the wave
 // (DPP, v_permlane*_swap) and then across the 4 waves through a double-buffered LDS slot (one
 // barrier per iteration; keeping a transposed copy of the gradient as well needs two barriers and
@@ -216,7 +218,7 @@ template <int NP> struct SkWg {
     static constexpr int EPL = NP * NP / 256;  // 1 or 4
     static constexpr int LPR = NP / EPL;       // lanes per row: 16 or 8
     static constexpr int kTile = NP * (NP + 1);
-    // LDS floats: transpose tile (later the column slots [2][4][NP]) | u | v | rho [T][NP] | s [T][NP]
+    // LDS floats: tile of E (later the column slots [2][4][NP]) | u | v | rho [T][NP] | s [T][NP]
     __host__ __device__ static constexpr int lds_floats(int T) { return kTile + 2 * NP + 2 * T * NP; }
     __device__ static __forceinline__ int row(int tid) { return tid / LPR; }
     __device__ static __forceinline__ int col0(int tid) { return (tid % LPR) * EPL; }
@@ -262,18 +264,32 @@ template <int NP> struct SkWg {
             for (int e = 0; e < EPL; e++) x[e] = p[e];
         }
     }
-    // a[e] = A[a][b0+e]  ->  at[e] = A[b0+e][a]
-    __device__ static __forceinline__ void transpose(const float (&a)[EPL], float (&at)[EPL], float *tile,
-                                                     int tid) {
-        const int r = row(tid), c0 = col0(tid);
-#pragma unroll
-        for (int e = 0; e < EPL; e++) tile[r * (NP + 1) + c0 + e] = a[e];
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < EPL; e++) at[e] = tile[(c0 + e) * (NP + 1) + r];
-        __syncthreads();
+    // sum over k of x[lane k of this 16-lane row] * m[k], in four chains.  The compiler folds the broadcast into products but not
+    // into fused multiply-adds: half the instructions this way.  (s_nop: two wait states between the write of x and DPP reads)
+    static __forceinline__ __device__ float row_dot(float x, const float (&m)[16]) {
+        float a0, a1, a2, a3;
+        asm("s_nop 1\n"
+            "v_mul_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+            "v_mul_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+            "v_mul_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+            "v_mul_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %0, %4, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %1, %4, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %2, %4, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %3, %4, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %0, %4, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %1, %4, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %2, %4, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %3, %4, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %0, %4, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %1, %4, %18 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %2, %4, %19 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %3, %4, %20 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
+            : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3)
+            : "v"(x), "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]), "v"(m[7]), "v"(m[8]), "v"(m[9]),
+              "v"(m[10]), "v"(m[11]), "v"(m[12]), "v"(m[13]), "v"(m[14]), "v"(m[15]));
+        return (a0 + a1) + (a2 + a3);
     }
-
     // E: exp(logits), 0 outside n x n.  On return M = u * E[e] * v[e]; rho/s hold the denominators.
     // PRECISE selects IEEE divisions (fp32 parity tier) instead of v_rcp_f32 (1 ulp).
     template <bool PRECISE = true>
@@ -281,37 +297,43 @@ template <int NP> struct SkWg {
                                                    int T, float eps, float *lds, int tid) {
         float *ub = lds + kTile, *vb = ub + NP, *rho = vb + NP, *s = rho + T * NP;
         const int a = row(tid), b0 = col0(tid);
-        const bool head = (tid % LPR) == 0, live = a < n;
-        float ET[EPL];
-        transpose(E, ET, lds, tid);
-        u = 1.0f;
-        float vc = 1.0f;  // v[a]: this thread's column in the transposed role
 #pragma unroll
-        for (int e = 0; e < EPL; e++) v[e] = 1.0f;
-        for (int t = 0; t < T; t++) {
-            float p = 0.f;
+        for (int e = 0; e < EPL; e++) lds[a * (NP + 1) + b0 + e] = E[e];
+        __syncthreads();
+        if (tid < 64) {
+            // row 16 rb + l and columns 16 cb ..; column 16 cb + l and rows 16 rb ..: u[16 rb + l] and v[16 cb + l] are this lane's
+            const int l = tid & 15, rb = NP == 32 ? tid >> 5 : 0, cb = NP == 32 ? (tid >> 4) & 1 : 0;
+            const int r = 16 * rb + l, c = 16 * cb + l;
+            float er[16], ec[16];
 #pragma unroll
-            for (int e = 0; e < EPL; e++) p += E[e] * v[e];
-            p = seg_allreduce(p);
-            // fp32 tier: product and sum rounded separately.  With a fused multiply-add the converged
-            // denominators settle one ulp off 1 on some rows and columns (u and v keep drifting against
-            // each other), and the reverse sweep, which divides by them in every iteration, drifts away
-            // from the float64 result by ~2e-8 per iteration; rounded separately they settle at exactly 1.
-            const float rr = live ? (PRECISE ? mul_add_unfused(u, p, eps) : u * p + eps) : 1.0f;
-            u = PRECISE ? u / rr : u * fast_rcp(rr);
-            if (head) { rho[t * NP + a] = rr; ub[a] = u; }
-            __syncthreads();
-            float uc[EPL], q = 0.f;
-            ld_vec(ub + b0, uc);
-#pragma unroll
-            for (int e = 0; e < EPL; e++) q += ET[e] * uc[e];
-            q = seg_allreduce(q);
-            const float sc = live ? (PRECISE ? mul_add_unfused(vc, q, eps) : vc * q + eps) : 1.0f;
-            vc = PRECISE ? vc / sc : vc * fast_rcp(sc);
-            if (head) { s[t * NP + a] = sc; vb[a] = vc; }
-            __syncthreads();
-            ld_vec(vb + b0, v);
+            for (int k = 0; k < 16; k++) {
+                er[k] = lds[r * (NP + 1) + 16 * cb + k];
+                ec[k] = lds[(16 * rb + k) * (NP + 1) + c];
+            }
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0), here: not in the loop, behind its stores
+            float uu = 1.0f, vv = 1.0f;
+            for (int t = 0; t < T; t++) {
+                float p = row_dot(vv, er);
+                if constexpr (NP == 32) p = xor16_add(p);
+                // fp32 tier: product and sum rounded separately.  With a fused multiply-add the converged
+                // denominators settle one ulp off 1 on some rows and columns (u and v keep drifting against
+                // each other), and the reverse sweep, which divides by them in every iteration, drifts away
+                // from the float64 result by ~2e-8 per iteration; rounded separately they settle at exactly 1.
+                const float rr = r < n ? (PRECISE ? mul_add_unfused(uu, p, eps) : uu * p + eps) : 1.0f;
+                uu = PRECISE ? uu / rr : uu * fast_rcp(rr);
+                float q = row_dot(uu, ec);
+                if constexpr (NP == 32) q = xor32_add(q);
+                const float sc = c < n ? (PRECISE ? mul_add_unfused(vv, q, eps) : vv * q + eps) : 1.0f;
+                vv = PRECISE ? vv / sc : vv * fast_rcp(sc);
+                rho[t * NP + r] = rr;  // (every lane: those that share a row or column hold the same)
+                s[t * NP + c] = sc;
+            }
+            ub[r] = uu;
+            vb[c] = vv;
         }
+        __syncthreads();
+        u = ub[a];
+        ld_vec(vb + b0, v);
     }
 
     // Copies what forward() left behind to global memory for the backward call:
@@ -368,7 +390,7 @@ template <int NP> struct SkWg {
     template <bool PRECISE = true>
     __device__ static __forceinline__ void backward(const float (&E)[EPL], float (&d)[EPL], float u,
                                                     float (&v)[EPL], int T, float *lds, int tid) {
-        float *cw = lds;  // the transpose tile is dead after forward()
+        float *cw = lds;  // the tile of E is dead after forward()
         const float *rho = lds + kTile + 2 * NP, *s = rho + T * NP;
         const int r = row(tid), c0 = col0(tid);
         float p[EPL], W[EPL];  // W = E v: the iterate without its row scaling
