@@ -27,14 +27,16 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 // =============================================================================================
 // n <= 8
 // =============================================================================================
-template <typename TG, typename TX, int NP, int V>
+template <typename TG, typename TX, int NP, int V, bool FUSED>
 __global__ __launch_bounds__(256) void mix_bwd_reduce_small_kernel(BwdReduceArgs a) {
     using SK = SkSmall<NP>;
-    constexpr int K = NP * NP + 3 * NP + 1;  // dM | dHpost | A1 | A2 | s1
+    constexpr int kSlots = FUSED ? 32 : 16;  // FUSED: up to two column parts
+    using CB = CoefBwdSmall<NP, std::is_same<TX, float>::value, false>;
+    constexpr int K = CB::K;  // dM | dHpost | A1 | A2 | s1
     extern __shared__ float smem[];
-    float *slot_s = smem;          // [K][16]  one slot per 16-lane row of the workgroup
-    float *tot = slot_s + K * 16;  // [K]
-    float *sc = tot + K;           // Sinkhorn denominators, SK::scaling_floats(T)
+    float *slot_s = smem;              // [K][kSlots]  one slot per 16-lane row of the workgroup
+    float *tot = slot_s + K * kSlots;  // [K]
+    float *sc = tot + K;               // Sinkhorn denominators, SK::scaling_floats(T)
     const int b = blockIdx.x, n = a.n, C = a.C, tid = threadIdx.x, nt = blockDim.x;
     const TG *__restrict__ gb = static_cast<const TG *>(a.dy) + (size_t)b * n * C;
     const TX *__restrict__ xb = static_cast<const TX *>(a.x) + (size_t)b * n * C;
@@ -44,6 +46,15 @@ __global__ __launch_bounds__(256) void mix_bwd_reduce_small_kernel(BwdReduceArgs
     // q is only requested here: a division in front of the loop would make the wave wait for this
     // round trip before it asks for its data; 1/q is applied to the sums behind the loop instead
     const float qraw = inject ? 1.0f : a.q[b];
+    // FUSED: the lanes of the sample's coefficient backward (4 x 4: the last 16-lane row, 8 x 8: the first wave)
+    const int g = tid - (NP == 4 ? nt - SK::kGroup : 0);
+    CB cb;  // everything but the sums is asked for in front of the loop (behind it: 1 us more at n=4 B=1280 C=1280)
+    if constexpr (FUSED) {
+        if (g >= 0 && g < SK::kGroup) {
+            cb.prefetch(a, b, g);
+            cb.forward_recompute(a, b, g, g, sc);
+        }
+    }
 
     float hpre[NP], hpost[NP];
 #pragma unroll
@@ -51,146 +62,109 @@ __global__ __launch_bounds__(256) void mix_bwd_reduce_small_kernel(BwdReduceArgs
         hpre[i] = i < n ? Hpre[i] : 0.f;
         hpost[i] = i < n ? Hpost[i] : 0.f;
     }
-    float acc[K];
+    const int nch = C / V, cpp = (nch + a.parts - 1) / a.parts;  // chunks per part
+    float qinv = 0.f;
+    // FUSED: the parts one after the other, each with sums of its own: the chains of the launch that has a workgroup per part, bit for
+    // bit (one chain over the row made the errors of dphi and dbias 1.01 and 1.06 times those; more threads instead lost: n=4 B=1280
+    // C=1280 49.4 us | 46.6 two launches)
+    const int part_end = FUSED ? a.parts : (int)blockIdx.y + 1;
+    for (int part = FUSED ? 0 : blockIdx.y; part < part_end; part++) {
+        float acc[K];
 #pragma unroll
-    for (int k = 0; k < K; k++) acc[k] = 0.f;
+        for (int k = 0; k < K; k++) acc[k] = 0.f;
 
-    const int nch = C / V;
-    const int part = blockIdx.y, cpp = (nch + a.parts - 1) / a.parts;  // chunks per part
-    const int ch_end = min(nch, (part + 1) * cpp);
-    for (int ch = part * cpp + tid; ch < ch_end; ch += nt) {
-        const int c = ch * V;
-        float gv[NP][V], xv[NP][V];
+        const int ch_end = min(nch, (part + 1) * cpp);
+        for (int ch = part * cpp + tid; ch < ch_end; ch += nt) {
+            const int c = ch * V;
+            float gv[NP][V], xv[NP][V];
 #pragma unroll
-        for (int i = 0; i < NP; i++) {
-            // streams >= n alias stream 0 (no branch around the loads): their sums land in entries
-            // of acc that nobody reads, and they meet zero coefficients everywhere else
-            const size_t so = (size_t)(i < n ? i : 0) * C + c;
-            load_vec<TG, V>(gb + so, gv[i]);
-            load_vec<TX, V>(xb + so, xv[i]);
-        }
-        float av[V], fv[V], dfw[V];
-        if (inject) load_vec<TX, V>(static_cast<const TX *>(a.f_inject) + (size_t)b * C + c, fv);
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-            float s_a = 0.f, s_df = 0.f;
-#pragma unroll
-            for (int i = 0; i < NP; i++) { s_a += hpre[i] * xv[i][v]; s_df += hpost[i] * gv[i][v]; }
-            av[v] = s_a;
-            if (inject) {
-                dfw[v] = 0.f;
-            } else {
-                const float wv = load_w_(a.w, a.w_bf16, c + v);
-                fv[v] = s_a * wv;  // f * q
-                dfw[v] = s_df * wv;
+            for (int i = 0; i < NP; i++) {
+                // streams >= n alias stream 0 (no branch around the loads): their sums land in entries
+                // of acc that nobody reads, and they meet zero coefficients everywhere else
+                const size_t so = (size_t)(i < n ? i : 0) * C + c;
+                load_vec<TG, V>(gb + so, gv[i]);
+                load_vec<TX, V>(xb + so, xv[i]);
             }
-            acc[K - 1] += dfw[v] * s_a;
-        }
-#pragma unroll
-        for (int i = 0; i < NP; i++) {
+            float av[V], fv[V], dfw[V];
+            if (inject) load_vec<TX, V>(static_cast<const TX *>(a.f_inject) + (size_t)b * C + c, fv);
 #pragma unroll
             for (int v = 0; v < V; v++) {
-                acc[NP * NP + i] += gv[i][v] * fv[v];
-                acc[NP * NP + NP + i] += dfw[v] * xv[i][v];
-                acc[NP * NP + 2 * NP + i] += av[v] * xv[i][v];
+                float s_a = 0.f, s_df = 0.f;
+#pragma unroll
+                for (int i = 0; i < NP; i++) { s_a += hpre[i] * xv[i][v]; s_df += hpost[i] * gv[i][v]; }
+                av[v] = s_a;
+                if (inject) {
+                    dfw[v] = 0.f;
+                } else {
+                    const float wv = load_w_(a.w, a.w_bf16, c + v);
+                    fv[v] = s_a * wv;  // f * q
+                    dfw[v] = s_df * wv;
+                }
+                acc[K - 1] += dfw[v] * s_a;
             }
 #pragma unroll
-            for (int j = 0; j < NP; j++)
+            for (int i = 0; i < NP; i++) {
 #pragma unroll
-                for (int v = 0; v < V; v++) acc[i * NP + j] += gv[i][v] * xv[j][v];
+                for (int v = 0; v < V; v++) {
+                    acc[NP * NP + i] += gv[i][v] * fv[v];
+                    acc[NP * NP + NP + i] += dfw[v] * xv[i][v];
+                    acc[NP * NP + 2 * NP + i] += av[v] * xv[i][v];
+                }
+#pragma unroll
+                for (int j = 0; j < NP; j++)
+#pragma unroll
+                    for (int v = 0; v < V; v++) acc[i * NP + j] += gv[i][v] * xv[j][v];
+            }
+        }
+
+        qinv = inject ? 0.f : 1.0f / qraw;
+        if (!inject) {
+#pragma unroll
+            for (int i = 0; i < NP; i++) acc[NP * NP + i] *= qinv;  // dHpost was summed against f * q
+        }
+        // workgroup sum: DPP within each 16-lane row, one LDS slot per row, then K lanes finish
+        const int at = (FUSED ? part * 16 : 0) + (tid >> 4);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const float v = row16_allreduce(acc[k]);
+            if ((tid & 15) == 0) slot_s[k * kSlots + at] = v;
         }
     }
-
-    const float qinv = inject ? 0.f : 1.0f / qraw;
-    if (!inject) {
-#pragma unroll
-        for (int i = 0; i < NP; i++) acc[NP * NP + i] *= qinv;  // dHpost was summed against f * q
-    }
-    // workgroup sum: DPP within each 16-lane row, one LDS slot per row, then K lanes finish
-    const int slot = tid >> 4, nslots = nt >> 4;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const float v = row16_allreduce(acc[k]);
-        if ((tid & 15) == 0) slot_s[k * 16 + slot] = v;
-    }
     __syncthreads();
+    const int nslots = nt >> 4;
     for (int k = tid; k < K; k += nt) {
         float v = 0.f;
-        for (int s = 0; s < nslots; s++) v += slot_s[k * 16 + s];
+        for (int p = 0; p < (FUSED ? a.parts : 1); p++) {
+            float t = 0.f;
+            for (int s = 0; s < nslots; s++) t += slot_s[k * kSlots + p * 16 + s];
+            v += t;
+        }
         tot[k] = v;
         if (a.raw) a.raw[((size_t)b * a.parts + blockIdx.y) * K + k] = v;
     }
     if (a.raw) return;  // the coefficient backward runs as its own small launch
     __syncthreads();
-    if (tid >= SK::kGroup) return;
-
-    // ---- epilogue on the lanes of one matrix (SkSmall layout) -------------------------------
-    const int g = tid;
-    const float s1 = tot[K - 1];
-    const int D = n * n + 2 * n;
-    float dHpre = 0.f, dHpost = 0.f;
-    if (g < n) {
-        dHpost = tot[NP * NP + g];
-        dHpre = inject ? 0.f
-                       : tot[NP * NP + NP + g] * qinv -
-                             s1 * tot[NP * NP + 2 * NP + g] * qinv * qinv * qinv / (float)C;
-    }
-    if (g == 0) a.out.s1[b] = s1;
-    const int r0 = SK::row(g), c0 = SK::col0(g);
-    if (a.hstride == 0) {
-        // static H: raw sums only; the coefficient backward runs once on the batch total
-        float *red = a.out.red + (size_t)b * (D + 3);  // rows padded like dt, for the batch-sum launch
-#pragma unroll
-        for (int e = 0; e < SK::EPL; e++)
-            if (r0 < n && c0 + e < n) red[r0 * n + c0 + e] = tot[r0 * NP + c0 + e];
-        if (g < n) { red[n * n + g] = dHpre; red[n * n + n + g] = dHpost; }
+    if constexpr (FUSED) {
+        if (g >= 0 && g < SK::kGroup) {
+            cb.fetch_sums(tot, 1);
+            cb.run(a, b, g, g, sc, nullptr);
+        }
         return;
     }
-    const float *Pb = a.P + (size_t)b * D;
-    const float al0 = a.alpha[0], al1 = a.alpha[1], al2 = a.alpha[2];
-    const float rinv = 1.0f / a.r[b];
-    float *dt = a.out.dt + (size_t)b * (D + 3);
-    const DPWriter dpw{a.out, b, a.B, a.DP};
-    float S0 = 0.f, S1 = 0.f, S2 = 0.f;  // sum_d dt_d p_d per alpha group
-    if (g < n) {
-        const float hp = Hpre[g], ho = Hpost[g];
-        const float dtp = dHpre * hp * (1.0f - hp);
-        const float dto = dHpost * ho * (1.0f - 0.5f * ho);
-        dt[g] = dtp; dt[n + g] = dto;
-        dpw.put(g, dtp * al0 * rinv); dpw.put(n + g, dto * al1 * rinv);
-        S0 = dtp * Pb[g]; S1 = dto * Pb[n + g];
-    }
-    float E[SK::EPL], m[SK::EPL], d[SK::EPL];
+    if (tid >= SK::kGroup) return;
+    // static H: raw sums only; the coefficient backward runs once on the batch total
+    const float s1 = tot[K - 1];
+    const int D = n * n + 2 * n, r0 = SK::row(tid), c0 = SK::col0(tid);
+    float *red = a.out.red + (size_t)b * (D + 3);  // rows padded like dt, for the batch-sum launch
 #pragma unroll
-    for (int e = 0; e < SK::EPL; e++) {
-        const int c = c0 + e;
-        const bool ok = r0 < n && c < n;
-        E[e] = ok ? expf(al2 * Pb[2 * n + r0 * n + c] + a.b_res[r0 * n + c]) : 0.f;
-        m[e] = E[e];
-        d[e] = ok ? tot[r0 * NP + c] : 0.f;
+    for (int e = 0; e < SK::EPL; e++)
+        if (r0 < n && c0 + e < n) red[r0 * n + c0 + e] = tot[r0 * NP + c0 + e];
+    if (tid < n) {
+        red[n * n + tid] = inject ? 0.f : tot[NP * NP + NP + tid] * qinv - s1 * tot[NP * NP + 2 * NP + tid] * qinv * qinv * qinv / (float)C;
+        red[n * n + n + tid] = tot[NP * NP + tid];
     }
-    SK::template forward<false>(m, g, n, a.T, a.eps, sc, tid);
-    SK::template backward<false>(d, m, a.T, sc, tid);
-#pragma unroll
-    for (int e = 0; e < SK::EPL; e++) {
-        const int c = c0 + e;
-        if (r0 < n && c < n) {
-            const int di = 2 * n + r0 * n + c;
-            const float dtr = d[e];  // the Sinkhorn backward hands back the gradient of the logits
-            dt[di] = dtr;
-            dpw.put(di, dtr * al2 * rinv);
-            S2 += dtr * Pb[di];
-        }
-    }
-    S0 = SK::group_allreduce(S0); S1 = SK::group_allreduce(S1); S2 = SK::group_allreduce(S2);
-    if (g == 0) {
-        dt[D] = S0; dt[D + 1] = S1; dt[D + 2] = S2;
-        a.out.cx[b] = (al0 * S0 + al1 * S1 + al2 * S2) * rinv * rinv / (float)(n * C);
-    }
-    dpw.pad(D, g, SK::kGroup);
+    if (tid == 0) a.out.s1[b] = s1;
 }
-
-
 
 // The coefficient backward as its own launch: every sample's serial Sinkhorn chain runs concurrently
 // (four 4x4 samples or one 8x8 sample per wave) instead of at the tail of a bandwidth-bound workgroup.
@@ -1304,31 +1278,48 @@ static hipError_t launch_gram_small_static(BwdReduceArgs a, hipStream_t stream) 
     return hipGetLastError();
 }
 
+// mix_bwd_reduce_small_kernel, dynamic H: the coefficient backward at the end of every sample's workgroup (which then goes through the
+// column parts one after the other) instead of a second launch.  Backward us in the fp32 tier, two launches | one:
+//   one part   n=1 C=512 B=300 16.7 | 15.1, 1900 21.4 | 19.3;  n=4 C=128 64 18.9 | 17.3;  C=512 900 25.8 | 23.1;  n=8 C=256 700 52 | 50
+//              C=640 1700 n=1 23.9 | 25.7, n=4 40.8 | 42.4;  C=256 2300 35.4 | 34.0, 8000 66.4 | 73.7;  n=8 C=640 1700 125 | 124
+//   two parts  n=1 C=1920 300 18.9 | 19.7, 1000 28.2 | 27.3, 1300 33.6 | 38.6;  n=2 C=4096 300 30.2 | 31.2, 600 38.8 | 38.2, 1000 51.9 |
+//              50.1, 1300 63.3 | 69.6;  n=4 C=1920 400 33.4 | 33.4, 600 40.9 | 40.3, 1000 47.8 | 45.5, 1300 59.3 | 63.1
+//              n=6 C=1920 300 66.6 | 69.4, 400 80.6 | 76.6, 600 93.8 | 90.5, 1000 133 | 134;  n=8 C=1024 300 60.6 | 62.6, 600 86.1 |
+//              83.4, 1000 109 | 112
+// The one launch has fewer workgroups and, with 104 registers (n <= 4), four waves per SIMD instead of six: it is the faster one while
+// its workgroups are resident together, and with two parts once there are enough of them to fill the chip.  Not with a Sinkhorn state
+// that would take the LDS of the workgroups beside it.
+static bool reduce_small_fused(const BwdReduceArgs &a) {
+    if (const int hook = tuning_get(kTuneGramFused); hook && a.T <= 32) return hook == 2;  // experiment hook
+    if (a.T > 32) return false;
+    if (a.parts == 1) return a.B <= (a.C <= 512 ? 2047 : 1024);
+    return a.n <= 4 ? a.B > 512 && a.B <= 1024 : a.B >= 384 && a.B <= 768;
+}
+
 template <typename TG, typename TX, int NP, int V>
-static hipError_t launch_small(const BwdReduceArgs &a, hipStream_t stream) {
+static hipError_t launch_small(BwdReduceArgs a, hipStream_t stream) {
     if constexpr (std::is_same<TG, bf16_t>::value && std::is_same<TX, bf16_t>::value) {
         if (gram_small_supported(a)) return launch_gram_small<NP>(a, stream);
         // static H: worth it once the batch fills the chip (one workgroup per sample)
         if (a.hstride == 0 && a.C % 8 == 0 && a.B >= 128) return launch_gram_small_static<NP>(a, stream);
     }
+    if (a.raw && reduce_small_fused(a)) a.raw = nullptr;  // at most two parts
     const int nch = (a.C / V + a.parts - 1) / a.parts;  // chunks per column part
     // every thread gets the same number of chunks (whole 16-lane rows: the reduction works on them)
+    const bool fused = a.hstride != 0 && !a.raw;
     const int rounds = (nch + 255) / 256;
     int nt = round_up((nch + rounds - 1) / rounds, 16);
     if (nt > 256) nt = 256;
     if (nt < SkSmall<NP>::kGroup) nt = SkSmall<NP>::kGroup;  // the epilogue runs on the lanes of one matrix
     constexpr int K = NP * NP + 3 * NP + 1;
-    // the Sinkhorn area is only needed when the coefficient backward runs in the same launch
-    const size_t smem = sizeof(float) * (K * 16 + K + (a.raw ? 0 : SkSmall<NP>::scaling_floats(a.T)));
-    hipError_t e = allow_dynamic_lds<&mix_bwd_reduce_small_kernel<TG, TX, NP, V>>(smem);
-    if (e != hipSuccess) return e;
-    mix_bwd_reduce_small_kernel<TG, TX, NP, V><<<dim3(a.B, a.parts), nt, smem, stream>>>(a);
-    e = hipGetLastError();
-    if (e != hipSuccess || !a.raw) return e;
+    const size_t smem = sizeof(float) * (K * (fused ? 33 : 17) + (fused ? SkSmall<NP>::scaling_floats(a.T) : 0));  // at most 28 KB (T <= 32)
+    if (fused) mix_bwd_reduce_small_kernel<TG, TX, NP, V, true><<<a.B, nt, smem, stream>>>(a);
+    else mix_bwd_reduce_small_kernel<TG, TX, NP, V, false><<<dim3(a.B, a.parts), nt, smem, stream>>>(a);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess || !a.raw) return e;
     // fp32 activations: the parity tier, IEEE divisions in the Sinkhorn chain
     constexpr bool kPrecise = std::is_same<TX, float>::value;
     const size_t smem2 = sizeof(float) * SkSmall<NP>::scaling_floats(a.T);
-    e = allow_dynamic_lds<&coef_bwd_small_kernel<NP, kPrecise>>(smem2);
+    hipError_t e = allow_dynamic_lds<&coef_bwd_small_kernel<NP, kPrecise>>(smem2);
     if (e != hipSuccess) return e;
     coef_bwd_small_kernel<NP, kPrecise><<<(a.B + SkSmall<NP>::kPerWave - 1) / SkSmall<NP>::kPerWave, 64, smem2, stream>>>(a);
     return hipGetLastError();
@@ -1418,8 +1409,8 @@ hipError_t launch_mix_bwd_reduce(const void *dy, int y_dtype, const void *x, int
                                  const float *b_res, const float *sk_state, BwdCoefOut out, float *raw, int B,
                                  int n, int C, int T, float eps, hipStream_t stream, const float *static_logits,
                                  float *static_state) {
-    // n <= 8, dynamic H: channel sums per (sample, column part), coefficient backward as a second
-    // small launch (static H: everything in the per-sample workgroup).  n > 8: always two launches.
+    // n <= 8, dynamic H: channel sums and coefficient backward in one launch, or per (sample, column part) with the coefficient
+    // backward as a second small launch (static H: everything in the per-sample workgroup).  n > 8: always two launches.
     if (n > 8 && raw == nullptr) return hipErrorInvalidValue;
     const bool split = raw != nullptr && (n > 8 || hstride != 0);
     BwdReduceArgs a{dy, x, w, f_inject, Hpre, Hpost, M, q, P, r, alpha, b_res, sk_state, out,
