@@ -118,9 +118,9 @@ using DPWriter = DPWriterT<false>;
 // STATIC (with GRAM): shared coefficients - prefetch() takes H from the [n] vectors and nothing else, and
 // run() stops after the channel-sum vectors: it writes the sample's raw gradients (dM | dHpre | dHpost)
 // as a row of `red` for the batch-sum launch; the Sinkhorn backward then runs once on the batch total.
-// FINE: dP in the planes of DPWriterT<true>.
-template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = false> struct CoefBwdSmall {
-    using SK = SkSmall<NP>;
+// FINE: dP in the planes of DPWriterT<true>.  COMPACT: see SkSmall.
+template <int NP, bool PRECISE, bool GRAM, bool STATIC = false, bool FINE = false, bool COMPACT = false> struct CoefBwdSmall {
+    using SK = SkSmall<NP, COMPACT>;
     static constexpr int K = GRAM ? 3 * NP * NP : NP * NP + 3 * NP + 1;
     // LDS floats next to the Sinkhorn denominators, per group: the column results of the Gram sums
     static constexpr int kXch = GRAM ? 3 * NP : 0;

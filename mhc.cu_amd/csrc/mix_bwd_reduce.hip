@@ -472,6 +472,158 @@ __global__ __launch_bounds__(256, F32 && NP == 4 ? 3 : 4) void gram_small_kernel
     }
 }
 
+// The same launch (n = 5 .. 8, dynamic H, coefficient backward inside) for large batches: a wave takes a sample, from its rows to its dP,
+// and shares nothing with the others.  In gram_small_kernel the sums of a sample wait for three waves and its coefficient backward
+// leaves those three idle; with short rows it is most of a workgroup's life.  Channel sums of n=5 B=8192 C=512 54 us there (84 MB: 17).
+// A step's products have sums of their own: one chain over a row would be three times as long as there.
+// F32: as in gram_small_kernel.
+constexpr int kGramWaves = 4;
+template <int WMODE, bool F32>
+__global__ __launch_bounds__(64 * kGramWaves, 4) void gram_wave_kernel(BwdReduceArgs a) {
+    static_assert(!F32 || WMODE != kGramInject, "an injected f takes the other kernels");
+    using TS = typename std::conditional<F32, float, bf16_t>::type;
+    using CB = CoefBwdSmall<8, false, true, false, false, true>;
+    constexpr int NP = 8, NB = 2, K = CB::K, U = F32 ? 1 : 2;
+    constexpr bool inject = WMODE == kGramInject;
+    extern __shared__ float smem[];  // per wave: slots [K][4] | sums [K] | CB::kXch | Sinkhorn denominators
+    const int n = a.n, C = a.C, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b = blockIdx.x * kGramWaves + wave;
+    MHC_PHASE_ZERO(kPhaseGramSmall, blockIdx.x);
+    if (b >= a.B) return;
+    float *slot_s = smem + wave * (5 * K + CB::kXch + CB::SK::scaling_floats(a.T)), *tot_s = slot_s + 4 * K, *xch = tot_s + K, *sc = xch + CB::kXch;
+    const int blk = lane >> 2, i = lane & 3, nsteps = (C + 127) / 128;
+    const TS *gb[NB], *xb[NB];
+    bool sv[NB];
+#pragma unroll
+    for (int I = 0; I < NB; I++) {
+        sv[I] = 4 * I + i < n;  // streams >= n: masked below
+        const size_t row = (size_t)b * n * C + (size_t)(sv[I] ? 4 * I + i : 0) * C;
+        gb[I] = static_cast<const TS *>(a.dy) + row;
+        xb[I] = static_cast<const TS *>(a.x) + row;
+    }
+    f32x4_t acc[3][NB][NB];
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+#pragma unroll
+        for (int I = 0; I < NB; I++)
+#pragma unroll
+            for (int J = 0; J < NB; J++) acc[m][I][J] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < nsteps; s0 += U) {
+        uint4 gr[U][NB], xr[U][NB], fr[U];
+        RawVec<bf16_t, 8> wb[U];
+        RawVec<float, 8> wf[U];
+        GramF32<NB> fl[F32 ? U : 1];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int st = min(s0 + u, nsteps - 1);
+            if constexpr (F32) {
+                const int c = st * 128 + blk * 4, c2 = min(c + 64, C - 4);
+                fl[u].load(gb, xb, c, c2);
+                if constexpr (WMODE == kGramWBf16) fl[u].load_w(static_cast<const bf16_t *>(a.w), c, c2);
+                else fl[u].load_w(static_cast<const float *>(a.w), c, c2);
+            } else {
+                const int c = min(st * 128 + blk * 8, C - 8);  // C % 8 == 0: a chunk is inside or outside
+#pragma unroll
+                for (int I = 0; I < NB; I++) {
+                    gr[u][I] = *reinterpret_cast<const uint4 *>(gb[I] + c);
+                    xr[u][I] = *reinterpret_cast<const uint4 *>(xb[I] + c);
+                }
+                if constexpr (inject) fr[u] = *reinterpret_cast<const uint4 *>(static_cast<const bf16_t *>(a.f_inject) + (size_t)b * C + c);
+                else if constexpr (WMODE == kGramWBf16) wb[u].load(static_cast<const bf16_t *>(a.w) + c);
+                else wf[u].load(static_cast<const float *>(a.w) + c);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int st = s0 + u;
+            if (st >= nsteps) break;
+            if constexpr (F32) {
+                const bool in2 = st * 128 + 64 < C;
+#pragma unroll
+                for (int I = 0; I < NB; I++) {
+                    fl[u].round(I, gr[u][I], xr[u][I]);
+                    if (sv[I])
+                        gram_copy(static_cast<char *>(a.copy) + (((size_t)b * n + 4 * I + i) * C + st * 128) * 4, blk, a.copy_block, gr[u][I], xr[u][I], in2);
+                    gr[u][I] = masked_halves(gr[u][I], sv[I], in2 && sv[I]);
+                    xr[u][I] = masked_halves(xr[u][I], sv[I], in2 && sv[I]);
+                }
+            } else {
+                const bool in = st * 128 + blk * 8 < C;
+#pragma unroll
+                for (int I = 0; I < NB; I++) {
+                    gr[u][I] = masked16(gr[u][I], in && sv[I]);
+                    xr[u][I] = masked16(xr[u][I], in && sv[I]);
+                }
+                if constexpr (inject) fr[u] = masked16(fr[u], in && i == 0);
+            }
+            bf16x4_t x0[NB], x1[NB];  // first / second group of four channels
+#pragma unroll
+            for (int I = 0; I < NB; I++) { x0[I] = bf16x4_of(xr[u][I].x, xr[u][I].y); x1[I] = bf16x4_of(xr[u][I].z, xr[u][I].w); }
+            float wv[8];
+            if constexpr (F32) fl[u].get_w(wv);
+            else if constexpr (!inject && WMODE == kGramWBf16) wb[u].get(wv);
+            else if constexpr (!inject) wf[u].get(wv);
+#pragma unroll
+            for (int I = 0; I < NB; I++) {
+                const bf16x4_t g0 = bf16x4_of(gr[u][I].x, gr[u][I].y), g1 = bf16x4_of(gr[u][I].z, gr[u][I].w);
+                const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int J = 0; J < NB; J++) acc[0][I][J] += mfma4(g1, x1[J], mfma4(g0, x0[J], zero));
+                if constexpr (inject) {
+                    acc[1][I][0] += mfma4(g1, bf16x4_of(fr[u].z, fr[u].w), mfma4(g0, bf16x4_of(fr[u].x, fr[u].y), zero));
+                } else {
+                    // dy * w as a bf16 pair (rounded value + remainder), see gram_small_kernel
+                    const uint32_t gw[4] = {gr[u][I].x, gr[u][I].y, gr[u][I].z, gr[u][I].w};
+                    uint32_t hw[4], lw[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const float p0 = bf16lo_to_f32(gw[k]) * wv[2 * k], p1 = bf16hi_to_f32(gw[k]) * wv[2 * k + 1];
+                        hw[k] = pack_bf16x2(p0, p1);
+                        lw[k] = pack_bf16x2(p0 - bf16lo_to_f32(hw[k]), p1 - bf16hi_to_f32(hw[k]));
+                    }
+#pragma unroll
+                    for (int J = 0; J < NB; J++) {
+                        f32x4_t s = mfma4(bf16x4_of(hw[2], hw[3]), x1[J], mfma4(bf16x4_of(hw[0], hw[1]), x0[J], zero));
+                        s = mfma4(bf16x4_of(lw[2], lw[3]), x1[J], mfma4(bf16x4_of(lw[0], lw[1]), x0[J], s));
+                        acc[1][I][J] += s;
+                        acc[2][I][J] += mfma4(x1[I], x1[J], mfma4(x0[I], x0[J], zero));
+                    }
+                }
+            }
+        }
+    }
+    CB cb;
+    cb.prefetch(a, b, lane);
+    cb.forward_recompute(a, b, lane, lane, sc);
+    // lane (block, j) holds column j of its block's products, register = row: the four blocks of a 16-lane row by DPP, then three of the
+    // sums per lane
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+#pragma unroll
+        for (int I = 0; I < NB; I++)
+#pragma unroll
+            for (int J = 0; J < NB; J++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float v = acc[m][I][J][r];
+                    v += dpp_mov<kDppRowRor4>(v);
+                    v += dpp_mov<kDppRowRor8>(v);
+                    if ((lane & 15) < 4) slot_s[(m * NP * NP + (4 * I + r) * NP + 4 * J + i) * 4 + (lane >> 4)] = v;
+                }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < K / 64; k++) {
+        const float4 v = *reinterpret_cast<const float4 *>(slot_s + (lane + 64 * k) * 4);
+        tot_s[lane + 64 * k] = (v.x + v.y) + (v.z + v.w);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    cb.fetch_sums(tot_s, 1);
+    cb.run(a, b, lane, lane, sc, xch);
+}
+
 // The same launch (n <= 4, dynamic H, coefficient backward inside) for large batches: a workgroup takes three or four
 // samples.  Its streaming waves hold a sample's rows together (U <= 3 steps each, every load of the sample requested at
 // once) and go through them; then wave 0 runs the coefficient backward of all, one per 16 lanes, in the time and with the
@@ -1213,10 +1365,40 @@ static hipError_t launch_gram_small_kernel(const BwdReduceArgs &a, size_t smem, 
     return hipGetLastError();
 }
 
+// Whether the channel sums of n = 5 .. 8 are gram_wave_kernel.  Backward us, gram_small_kernel | this:
+//   n=5 C=384 B=800 25.9 | 24.9, 8192 84.3 | 60.9;  C=512 1000 28.8 | 27.8, 8192 88.2 | 67.5;  C=1024 800 29.2 | 30.4, 1200 37.8 | 35.1,
+//       8192 115 | 97;  C=1536 1200 41.2 | 41.4, 8192 149 | 136;  C=2048 1600 52.2 | 51.3, 4000 95.9 | 90.9;  C=2560 1000 44.4 | 47.1
+//   n=6 C=1536 1200 45.3 | 45.5, 4000 87.7 | 84.9;  C=2560 2500 87.9 | 88.6;  n=7 C=1024 800 36.9 | 37.4, 8192 157 | 126;  C=1536 1600 56.4 |
+//       55.8;  n=8 C=512 1600 49.0 | 43.7, 8192 118 | 99;  C=1024 2200 66.9 | 64.7, 4000 93.1 | 86.0;  C=1536 2200 78.4 | 80.9, 4000 117 | 113
+//   float32 storage: n=5 C=512 1000 32.0 | 33.6, 1800 41.4 | 39.2, 3500 57.5 | 53.7;  n=8 C=1024 1800 95.9 | 95.3;  n=6 C=2560 1800 131 | 134
+// Long rows of few samples want a sample's loads spread over three waves.  Not with a Sinkhorn state that would take the LDS of the
+// workgroups beside it.
+static bool gram_wave_preferred(const BwdReduceArgs &a) {
+    if (a.T > 32) return false;
+    if (const int hook = tuning_get(kTuneGramFused)) return hook == 2;  // experiment hook
+    if (a.C > 1024) return !a.copy && a.n < 8 && a.C <= 2048 && a.B >= 1500;
+    return a.B >= (a.copy ? 1700 : 1000);
+}
+
 template <int NP>
 static hipError_t launch_gram_small(BwdReduceArgs a, hipStream_t stream) {
     using SK = SkSmall<NP>;
     using CB = CoefBwdSmall<NP, false, true>;
+    if constexpr (NP == 8) {
+        if (gram_wave_preferred(a)) {
+            using CW = CoefBwdSmall<8, false, true, false, false, true>;
+            a.parts = 1;
+            const size_t smem = sizeof(float) * kGramWaves * (5 * CW::K + CW::kXch + CW::SK::scaling_floats(a.T));  // at most 24 KB
+            const unsigned grid = (a.B - 1) / kGramWaves + 1;
+            if (a.copy) {
+                if (a.w_bf16) gram_wave_kernel<kGramWBf16, true><<<grid, 64 * kGramWaves, smem, stream>>>(a);
+                else gram_wave_kernel<kGramWF32, true><<<grid, 64 * kGramWaves, smem, stream>>>(a);
+            } else if (a.f_inject) gram_wave_kernel<kGramInject, false><<<grid, 64 * kGramWaves, smem, stream>>>(a);
+            else if (a.w_bf16) gram_wave_kernel<kGramWBf16, false><<<grid, 64 * kGramWaves, smem, stream>>>(a);
+            else gram_wave_kernel<kGramWF32, false><<<grid, 64 * kGramWaves, smem, stream>>>(a);
+            return hipGetLastError();
+        }
+    }
     if constexpr (NP == 4) {
         if (const int per_wg = gram_quad_samples(a)) {
             // streaming waves: as many as give the fewest steps per wave, up to seven, eleven for rows beyond 21 steps

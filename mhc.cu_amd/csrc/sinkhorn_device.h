@@ -36,8 +36,11 @@ __device__ __forceinline__ float mul_add_unfused(float a, float b, float c) {
 __device__ __forceinline__ void sk_chain_begin() { __builtin_amdgcn_s_setprio(3); }
 __device__ __forceinline__ void sk_chain_end() { __builtin_amdgcn_s_setprio(0); }
 
-template <int NP> struct SkSmall {
+// COMPACT (8 x 8): the denominators in LDS as they are saved, 16 floats an iteration instead of one of each per lane: where every wave
+// of a workgroup has a matrix of its own.
+template <int NP, bool COMPACT = false> struct SkSmall {
     static_assert(NP == 4 || NP == 8, "SkSmall handles 4x4 and 8x8 tiles");
+    static_assert(!COMPACT || NP == 8, "one matrix per wave");
     static constexpr int EPL = 1;               // elements per lane
     static constexpr int kGroup = NP * NP;      // lanes per matrix: 16 or the whole wave
     static constexpr int kPerWave = kWave / kGroup;  // matrices per wave
@@ -67,6 +70,9 @@ template <int NP> struct SkSmall {
     // sum over all lanes of the matrix
     __device__ static __forceinline__ float group_allreduce(float v) { return col_allreduce(row_allreduce(v)); }
 
+    __device__ static __forceinline__ int rho_at(int t, int lane) { return COMPACT ? t * 2 * NP + row(lane) : (t * kRec) * kWave + lane; }
+    __device__ static __forceinline__ int s_at(int t, int lane) { return COMPACT ? (t * 2 + 1) * NP + col0(lane) : (t * kRec + 1) * kWave + lane; }
+
     // m: in = exp(logits) (0 outside n x n), out = final iterate.
     // RECORD: keep, per iteration t and lane, the row denominator and per element the column
     // denominator:  sc[(t * kRec + k) * 64 + lane], k = 0: rho | 1..EPL: s  (a compile-time switch:
@@ -89,12 +95,12 @@ template <int NP> struct SkSmall {
             for (int e = 0; e < EPL; e++) rs += m[e];
             rs = row_allreduce(rs) + eps_r;
             const float rinv = PRECISE ? 1.0f / rs : fast_rcp(rs);
-            if constexpr (RECORD) sc[(t * kRec) * kWave + lane] = rs;
+            if constexpr (RECORD) sc[rho_at(t, lane)] = rs;
 #pragma unroll
             for (int e = 0; e < EPL; e++) {
                 m[e] = PRECISE ? m[e] / rs : m[e] * rinv;
                 const float cs = col_allreduce(m[e]) + eps_c[e];
-                if constexpr (RECORD) sc[(t * kRec + 1 + e) * kWave + lane] = cs;
+                if constexpr (RECORD) sc[s_at(t, lane)] = cs;
                 m[e] = PRECISE ? m[e] / cs : m[e] * fast_rcp(cs);
             }
         }
@@ -124,6 +130,19 @@ template <int NP> struct SkSmall {
     // loads of kBatch iterations are requested together (24: one round trip for the usual 20).
     template <int kBatch = 24>
     __device__ static __forceinline__ void load_state(const float *st, int g, int T, float *sc, int lane) {
+        if constexpr (COMPACT) {
+            for (int e0 = g; e0 < 2 * NP * T; e0 += 8 * kWave) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = st[min(e0 + u * kWave, 2 * NP * T - 1)];
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (e0 + u * kWave < 2 * NP * T) sc[e0 + u * kWave] = v[u];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // other lanes read them
+            __builtin_amdgcn_wave_barrier();
+            return;
+        }
         const float *pr = st + row(g), *pc = st + NP + col0(g);
         for (int t0 = 0; t0 < T; t0 += kBatch) {
             float rs[kBatch], cs[kBatch];
@@ -136,8 +155,8 @@ template <int NP> struct SkSmall {
 #pragma unroll
             for (int u = 0; u < kBatch; u++) {
                 if (t0 + u < T) {
-                    sc[((t0 + u) * kRec) * kWave + lane] = rs[u];
-                    sc[((t0 + u) * kRec + 1) * kWave + lane] = cs[u];
+                    sc[rho_at(t0 + u, lane)] = rs[u];
+                    sc[s_at(t0 + u, lane)] = cs[u];
                 }
             }
         }
@@ -163,8 +182,8 @@ template <int NP> struct SkSmall {
         // register pairs, alternating), so that the LDS round trip stays off the dependent chain.
         auto fetch = [&](int t, float &rs, float &cs) {
             t = t < 0 ? 0 : t;
-            rs = sc[(t * kRec) * kWave + lane];
-            cs = sc[(t * kRec + 1) * kWave + lane];
+            rs = sc[rho_at(t, lane)];
+            cs = sc[s_at(t, lane)];
         };
         float p = d[0] * m[0];
         auto step = [&](float rs, float cs) {
@@ -190,7 +209,7 @@ template <int NP> struct SkSmall {
         sk_chain_end();
         d[0] = p;
     }
-    __host__ __device__ static constexpr int scaling_floats(int T) { return T * kRec * kWave; }
+    __host__ __device__ static constexpr int scaling_floats(int T) { return COMPACT ? 2 * NP * T : T * kRec * kWave; }
 };
 
 // =============================================================================================
