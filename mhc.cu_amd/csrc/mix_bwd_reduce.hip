@@ -27,11 +27,16 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 // =============================================================================================
 // n <= 8
 // =============================================================================================
-template <typename TG, typename TX, int NP, int V, bool FUSED>
-__global__ __launch_bounds__(256) void mix_bwd_reduce_small_kernel(BwdReduceArgs a) {
-    using SK = SkSmall<NP>;
-    constexpr int kSlots = FUSED ? 32 : 16;  // FUSED: up to two column parts
-    using CB = CoefBwdSmall<NP, std::is_same<TX, float>::value, false>;
+// FORM: kSumsOnly; kSumsCoef, the coefficient backward at the end of the workgroup; kWaveCoef, the same with a workgroup of one wave.
+// Bound by the bytes of dy and x and, where a launch follows, by that launch's 5 us: B=2560 n=4 C=1280 in fp32, 105 MB, 21 us (4.9
+// TB/s) + 5 in two launches, 22 with a wave per sample (reduce_small_form() has more).
+enum ReduceForm { kSumsOnly, kSumsCoef, kWaveCoef };
+template <typename TG, typename TX, int NP, int V, int FORM>
+__global__ __launch_bounds__(FORM == kWaveCoef ? 64 : 256) void mix_bwd_reduce_small_kernel(BwdReduceArgs a) {
+    constexpr bool FUSED = FORM != kSumsOnly;
+    constexpr int kSlots = FORM == kWaveCoef ? 4 : FUSED ? 32 : 16;  // kSumsCoef: up to two column parts
+    using CB = CoefBwdSmall<NP, std::is_same<TX, float>::value, false, false, false, FORM == kWaveCoef>;
+    using SK = typename CB::SK;
     constexpr int K = CB::K;  // dM | dHpost | A1 | A2 | s1
     extern __shared__ float smem[];
     float *slot_s = smem;              // [K][kSlots]  one slot per 16-lane row of the workgroup
@@ -69,9 +74,12 @@ __global__ __launch_bounds__(256) void mix_bwd_reduce_small_kernel(BwdReduceArgs
     // C=1280 49.4 us | 46.6 two launches)
     const int part_end = FUSED ? a.parts : (int)blockIdx.y + 1;
     for (int part = FUSED ? 0 : blockIdx.y; part < part_end; part++) {
-        float acc[K];
+        float acc[K], chunks[FORM == kWaveCoef ? K : 1];  // kWaveCoef: a chunk in sums of its own (a lane has the most of them)
 #pragma unroll
-        for (int k = 0; k < K; k++) acc[k] = 0.f;
+        for (int k = 0; k < K; k++) {
+            acc[k] = 0.f;
+            if constexpr (FORM == kWaveCoef) chunks[k] = 0.f;
+        }
 
         const int ch_end = min(nch, (part + 1) * cpp);
         for (int ch = part * cpp + tid; ch < ch_end; ch += nt) {
@@ -115,6 +123,17 @@ __global__ __launch_bounds__(256) void mix_bwd_reduce_small_kernel(BwdReduceArgs
 #pragma unroll
                     for (int v = 0; v < V; v++) acc[i * NP + j] += gv[i][v] * xv[j][v];
             }
+            if constexpr (FORM == kWaveCoef) {
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+                    chunks[k] += acc[k];
+                    acc[k] = 0.f;
+                }
+            }
+        }
+        if constexpr (FORM == kWaveCoef) {
+#pragma unroll
+            for (int k = 0; k < K; k++) acc[k] = chunks[k];
         }
 
         qinv = inject ? 0.f : 1.0f / qraw;
@@ -1460,22 +1479,31 @@ static hipError_t launch_gram_small_static(BwdReduceArgs a, hipStream_t stream) 
     return hipGetLastError();
 }
 
-// mix_bwd_reduce_small_kernel, dynamic H: the coefficient backward at the end of every sample's workgroup (which then goes through the
-// column parts one after the other) instead of a second launch.  Backward us in the fp32 tier, two launches | one:
-//   one part   n=1 C=512 B=300 16.7 | 15.1, 1900 21.4 | 19.3;  n=4 C=128 64 18.9 | 17.3;  C=512 900 25.8 | 23.1;  n=8 C=256 700 52 | 50
-//              C=640 1700 n=1 23.9 | 25.7, n=4 40.8 | 42.4;  C=256 2300 35.4 | 34.0, 8000 66.4 | 73.7;  n=8 C=640 1700 125 | 124
-//   two parts  n=1 C=1920 300 18.9 | 19.7, 1000 28.2 | 27.3, 1300 33.6 | 38.6;  n=2 C=4096 300 30.2 | 31.2, 600 38.8 | 38.2, 1000 51.9 |
-//              50.1, 1300 63.3 | 69.6;  n=4 C=1920 400 33.4 | 33.4, 600 40.9 | 40.3, 1000 47.8 | 45.5, 1300 59.3 | 63.1
-//              n=6 C=1920 300 66.6 | 69.4, 400 80.6 | 76.6, 600 93.8 | 90.5, 1000 133 | 134;  n=8 C=1024 300 60.6 | 62.6, 600 86.1 |
-//              83.4, 1000 109 | 112
-// The one launch has fewer workgroups and, with 104 registers (n <= 4), four waves per SIMD instead of six: it is the faster one while
-// its workgroups are resident together, and with two parts once there are enough of them to fill the chip.  Not with a Sinkhorn state
-// that would take the LDS of the workgroups beside it.
-static bool reduce_small_fused(const BwdReduceArgs &a) {
-    if (const int hook = tuning_get(kTuneGramFused); hook && a.T <= 32) return hook == 2;  // experiment hook
-    if (a.T > 32) return false;
-    if (a.parts == 1) return a.B <= (a.C <= 512 ? 2047 : 1024);
-    return a.n <= 4 ? a.B > 512 && a.B <= 1024 : a.B >= 384 && a.B <= 768;
+// mix_bwd_reduce_small_kernel, dynamic H: the coefficient backward at the end of every sample's workgroup (kSumsCoef: it goes through
+// the column parts one after the other; kWaveCoef: a wave takes the sample) instead of a second launch.  Backward us in the fp32 tier,
+// two launches | kSumsCoef | kWaveCoef:
+//   n=1 C=256 800 16.5 | 15.0 | 14.8, 8000 42.6 | 51.6 | 45.7;  C=512 400 16.8 | 15.7 | 16.3, 1800 21.8 | 19.6 | 19.3, 4000 34.9 | 36.4 | 31.9,
+//       8000 52.4 | 61.9 | 53.1;  C=1280 400 18.7 | 18.8 | 19.5, 800 22.8 | 22.4 | 22.2, 2560 39.2 | 41.9 | 35.0;  C=4096 800 37.2 | 36.7 | 44.1,
+//       2560 73.0 | 78.7 | 73.8
+//   n=2 C=1280 1200 33.7 | 32.1 | 31.0, 4000 61.4 | 68.5 | 57.6;  C=2560 800 37.6 | 37.0 | 39.9, 1200 47.0 | 43.9 | 45.4, 1800 55.3 | 59.9 | 53.0
+//   n=4 C=256 100 20.1 | 18.8 | 18.5, 4000 42.5 | 47.0 | 41.3;  C=512 800 25.1 | 23.2 | 23.7, 2560 42.2 | 42.4 | 40.0;  C=1280 100 21.1 | 22.1 |
+//       22.5, 800 39.5 | 38.8 | 38.5, 1800 58.0 | 60.9 | 54.0, 2560 70.0 | 72.5 | 65.8;  C=2560 400 37.7 | 37.0 | 42.1, 1200 67.6 | 64.1 | 65.6
+//   n=6 C=1920 300 66.6 | 69.4, 400 80.6 | 76.6, 600 93.8 | 90.5, 1000 133 | 134;  n=8 C=256 700 52 | 50, 2300 93.8 | 94.0;  C=640 1700 125 |
+//       124;  C=1024 300 60.6 | 62.6, 600 86.1 | 83.4, 1000 109 | 112   (kWaveCoef would hold 219 registers)
+// kSumsCoef has fewer workgroups and, with 104 registers (n <= 4), four waves per SIMD instead of six: it pays while its workgroups are
+// resident together, and with two parts once there are enough of them to fill the chip.  A wave per sample has nobody wait for the
+// coefficient backward, but a long row's loads come one after the other, and those of single elements (!wide) most of all: n=4 C=515
+// B=1500 56.1 | | 57.3, n=2 C=1283 B=1200 57.3 | | 63.6.  Not with a Sinkhorn state that would take the LDS of the
+// workgroups beside it.
+static ReduceForm reduce_small_form(const BwdReduceArgs &a, bool wide) {
+    const int B = a.B, C = a.C;
+    if (a.T > 32) return kSumsOnly;
+    if (const int hook = tuning_get(kTuneGramFused)) return hook == 3 && a.n <= 4 ? kWaveCoef : hook >= 2 ? kSumsCoef : kSumsOnly;  // experiment hook
+    if (a.n > 4) return (a.parts == 1 ? B <= (C <= 512 ? 2047 : 1024) : B >= 384 && B <= 768) ? kSumsCoef : kSumsOnly;
+    if (C <= 256) return B <= 4500 ? kWaveCoef : kSumsOnly;
+    if (C <= 512 && wide) return B <= 1700 ? kSumsCoef : B <= 6000 ? kWaveCoef : kSumsOnly;
+    if (C <= 3072 && wide && B > 1024) return kWaveCoef;
+    return B <= 1024 && (a.parts == 1 || B > 512) ? kSumsCoef : kSumsOnly;
 }
 
 template <typename TG, typename TX, int NP, int V>
@@ -1485,18 +1513,28 @@ static hipError_t launch_small(BwdReduceArgs a, hipStream_t stream) {
         // static H: worth it once the batch fills the chip (one workgroup per sample)
         if (a.hstride == 0 && a.C % 8 == 0 && a.B >= 128) return launch_gram_small_static<NP>(a, stream);
     }
-    if (a.raw && reduce_small_fused(a)) a.raw = nullptr;  // at most two parts
+    const ReduceForm form = a.hstride != 0 ? reduce_small_form(a, V > 1) : kSumsOnly;
+    if (form != kSumsOnly) a.raw = nullptr;  // (kSumsCoef: at most two parts)
+    if (form == kWaveCoef) a.parts = 1;
     const int nch = (a.C / V + a.parts - 1) / a.parts;  // chunks per column part
     // every thread gets the same number of chunks (whole 16-lane rows: the reduction works on them)
-    const bool fused = a.hstride != 0 && !a.raw;
     const int rounds = (nch + 255) / 256;
     int nt = round_up((nch + rounds - 1) / rounds, 16);
     if (nt > 256) nt = 256;
     if (nt < SkSmall<NP>::kGroup) nt = SkSmall<NP>::kGroup;  // the epilogue runs on the lanes of one matrix
     constexpr int K = NP * NP + 3 * NP + 1;
-    const size_t smem = sizeof(float) * (K * (fused ? 33 : 17) + (fused ? SkSmall<NP>::scaling_floats(a.T) : 0));  // at most 28 KB (T <= 32)
-    if (fused) mix_bwd_reduce_small_kernel<TG, TX, NP, V, true><<<a.B, nt, smem, stream>>>(a);
-    else mix_bwd_reduce_small_kernel<TG, TX, NP, V, false><<<dim3(a.B, a.parts), nt, smem, stream>>>(a);
+    // at most 28 KB (T <= 32 with the coefficient backward)
+    if (form == kWaveCoef) {
+        if constexpr (NP == 4) {
+            const size_t smem = sizeof(float) * (K * 5 + SkSmall<NP, true>::scaling_floats(a.T));
+            mix_bwd_reduce_small_kernel<TG, TX, NP, V, kWaveCoef><<<a.B, 64, smem, stream>>>(a);
+        }
+    } else if (form == kSumsCoef) {
+        const size_t smem = sizeof(float) * (K * 33 + SkSmall<NP>::scaling_floats(a.T));
+        mix_bwd_reduce_small_kernel<TG, TX, NP, V, kSumsCoef><<<a.B, nt, smem, stream>>>(a);
+    } else {
+        mix_bwd_reduce_small_kernel<TG, TX, NP, V, kSumsOnly><<<dim3(a.B, a.parts), nt, sizeof(float) * K * 17, stream>>>(a);
+    }
     if (hipError_t e = hipGetLastError(); e != hipSuccess || !a.raw) return e;
     // fp32 activations: the parity tier, IEEE divisions in the Sinkhorn chain
     constexpr bool kPrecise = std::is_same<TX, float>::value;
@@ -1593,8 +1631,8 @@ hipError_t launch_mix_bwd_reduce(const void *dy, int y_dtype, const void *x, int
                                  float *static_state) {
     // n <= 8, dynamic H: channel sums and coefficient backward in one launch, or per (sample, column part) with the coefficient
     // backward as a second small launch (static H: everything in the per-sample workgroup).  n > 8: always two launches.
-    if (n > 8 && raw == nullptr) return hipErrorInvalidValue;
-    const bool split = raw != nullptr && (n > 8 || hstride != 0);
+    if ((n > 8 || hstride != 0) && raw == nullptr) return hipErrorInvalidValue;
+    const bool split = n > 8 || hstride != 0;
     BwdReduceArgs a{dy, x, w, f_inject, Hpre, Hpost, M, q, P, r, alpha, b_res, sk_state, out,
                     hstride, w_dtype == kBF16, B, n, C, T, padded_D(n), eps,
                     split ? raw : nullptr, split ? bwd_reduce_parts(B, n, C) : 1};

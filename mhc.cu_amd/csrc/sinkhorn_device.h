@@ -36,11 +36,10 @@ __device__ __forceinline__ float mul_add_unfused(float a, float b, float c) {
 __device__ __forceinline__ void sk_chain_begin() { __builtin_amdgcn_s_setprio(3); }
 __device__ __forceinline__ void sk_chain_end() { __builtin_amdgcn_s_setprio(0); }
 
-// COMPACT (8 x 8): the denominators in LDS as they are saved, 16 floats an iteration instead of one of each per lane: where every wave
-// of a workgroup has a matrix of its own.
+// COMPACT: the denominators of one matrix in LDS as they are saved, 2 NP floats an iteration instead of one of each per lane of the
+// wave: where every wave of a workgroup has a matrix of its own (lane: within the matrix's group).
 template <int NP, bool COMPACT = false> struct SkSmall {
     static_assert(NP == 4 || NP == 8, "SkSmall handles 4x4 and 8x8 tiles");
-    static_assert(!COMPACT || NP == 8, "one matrix per wave");
     static constexpr int EPL = 1;               // elements per lane
     static constexpr int kGroup = NP * NP;      // lanes per matrix: 16 or the whole wave
     static constexpr int kPerWave = kWave / kGroup;  // matrices per wave
@@ -131,13 +130,14 @@ template <int NP, bool COMPACT = false> struct SkSmall {
     template <int kBatch = 24>
     __device__ static __forceinline__ void load_state(const float *st, int g, int T, float *sc, int lane) {
         if constexpr (COMPACT) {
-            for (int e0 = g; e0 < 2 * NP * T; e0 += 8 * kWave) {
-                float v[8];
+            constexpr int kU = NP == 8 ? 8 : 12;  // T = 24 and more in one round
+            for (int e0 = g; e0 < 2 * NP * T; e0 += kU * kGroup) {
+                float v[kU];
 #pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = st[min(e0 + u * kWave, 2 * NP * T - 1)];
+                for (int u = 0; u < kU; u++) v[u] = st[min(e0 + u * kGroup, 2 * NP * T - 1)];
 #pragma unroll
-                for (int u = 0; u < 8; u++)
-                    if (e0 + u * kWave < 2 * NP * T) sc[e0 + u * kWave] = v[u];
+                for (int u = 0; u < kU; u++)
+                    if (e0 + u * kGroup < 2 * NP * T) sc[e0 + u * kGroup] = v[u];
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // other lanes read them
             __builtin_amdgcn_wave_barrier();

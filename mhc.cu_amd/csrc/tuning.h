@@ -10,7 +10,7 @@ namespace mhc {
 enum TuneKey {
     kTuneOnepassOff = 0,    // one-pass forwards: 0 = by size, 1 = neither, 2 = the one-launch forward, 3 = the held one, whenever the shape allows
     kTuneOnepassG = 1,      // samples per workgroup of the one-launch forward
-    kTuneGramFused = 2,     // n <= 8 channel sums and coefficient backward: 1 = two launches, 2 = one launch (n <= 4: four samples per workgroup, n = 5 .. 8: one per wave)
+    kTuneGramFused = 2,     // n <= 8 channel sums and coefficient backward: 1 = two launches, 2 = one launch (n <= 4: four samples per workgroup, n = 5 .. 8: one per wave), 3 = VALU sums of n <= 4: one sample per wave
     kTuneSlabSplits = 3,    // batch splits of the slab backward (n <= 8) and of the projection backward (n = 5 .. 18)
     kTuneSeparateFinalize = 4,  // 1 = batch sums always as a launch of their own, never inside the dphi launch
     kTuneProjApart = 5,     // n <= 18 projection backward: 1 = both products in one launch, 2 = two launches
