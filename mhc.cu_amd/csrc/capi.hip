@@ -668,10 +668,10 @@ int fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype, const Pa
     const DynFwdWs ws = carve_dyn_fwd(workspace, B, n, C);
     if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (!f_inject && layer_fwd_held_supported(x_dtype, y_dtype, phi_dtype, B, n, C) &&
+    // (parameters that are not whole 16-byte pieces are packed by a launch of their own)
+    const bool direct = gather && aligned16(gather->phi[0]) && aligned16(gather->phi[1]) && aligned16(gather->phi[2]);
+    if (!f_inject && layer_fwd_held_supported(x_dtype, y_dtype, phi_dtype, B, n, C, direct && gather->phi_dtype == kF32) &&
         layer_fwd_held_bytes(x_dtype, n, C) <= ws.part_bytes) {
-        // (parameters that are not whole 16-byte pieces are packed by a launch of their own)
-        const bool direct = gather && aligned16(gather->phi[0]) && aligned16(gather->phi[1]) && aligned16(gather->phi[2]);
         if (gather && !direct) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
         MHC_LAUNCH(launch_layer_fwd_held(x, x_dtype, w, w_dtype, y, direct ? gather : nullptr, phi, alpha, bias, ws.Ppart, H_pre, H_post,
                                          M, P, r, q, sk_state, B, n, C, iters, eps, st));
@@ -680,7 +680,7 @@ int fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype, const Pa
     // the caller's own parameters: read by the kernel that multiplies with them where it can, otherwise packed by a launch
     // of their own
     const bool can_gather = gather && layer_fwd_onepass_gathers(*gather);
-    const bool one = layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C, can_gather), in_one = one && can_gather;
+    const bool one = layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C, can_gather), in_one = one && can_gather && layer_fwd_onepass_reads_params(B, n, C);
     const bool in_proj = gather && !one && proj_fwd_gathers(*gather, x_dtype, B, n, C);
     if (gather && !in_one && !in_proj) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
     if (one) {

@@ -104,6 +104,7 @@ hipError_t launch_layer_fwd_fused(const void *x, int x_dtype, const void *w, int
 bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C, bool from_params = false);
 int layer_fwd_onepass_most_samples(int n, int C);  // per workgroup
 bool layer_fwd_onepass_gathers(const ParamGather &g);  // it reads the caller's own parameters itself
+bool layer_fwd_onepass_reads_params(int B, int n, int C);
 hipError_t launch_layer_fwd_onepass(const void *x, const void *w, int w_dtype, const void *f_inject, void *y,
                                     int y_dtype, const void *phi, const float *alpha, const float *bias,
                                     float *Hpre, float *Hpost, float *M, float *P, float *r, float *q,
@@ -112,7 +113,7 @@ hipError_t launch_layer_fwd_onepass(const void *x, const void *w, int w_dtype, c
 
 // The same for large batches: sixteen samples per workgroup, their rows in registers (layer_fwd_held.hip).  frag: scratch
 // of layer_fwd_held_bytes(), phi in operand layout.  gather: the caller's own parameters, packed on the way.
-bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C);
+bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C, bool from_params);  // the caller's fp32 ones
 size_t layer_fwd_held_bytes(int x_dtype, int n, int C);
 hipError_t launch_layer_fwd_held(const void *x, int x_dtype, const void *w, int w_dtype, void *y, const ParamGather *gather, const void *phi,
                                  const float *alpha, const float *bias, void *frag, float *Hpre, float *Hpost, float *M, float *P,

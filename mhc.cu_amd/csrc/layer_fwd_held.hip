@@ -553,12 +553,14 @@ size_t layer_fwd_held_bytes(int x_dtype, int n, int C) { return (size_t)held_uni
 //            18 | 22, 1613 23 | 22;  2560 1333 25 | 26, 1613 27 | 26;  n=3 1664 2047 14 | 17, 2160 22 | 17;  3072 1333 23 | 23;  n=2 5120
 //            1333 38 | 26  (the two-launch forward has a step where x outgrows the L2)
 //            beside the one-launch forward: n=4 512 4000 12 | 13, 4400 21 | 16;  n=3 1280 3500 17 | 17, 4000 31 | 19;  n=2 2560 2450
-//            18 | 22, 2700 34 | 22;  shorter rows n=4 256 8192 12 | 13, 12000 19 | 16, 20000 28 | 28
+//            18 | 22, 2700 34 | 22;  shorter rows n=4 256 8192 12 | 13, 12000 19 | 16, 20000 28 | 28;  from the caller's fp32
+//            parameters, which that one has packed by a launch there: n=4 64 8192 11.8 | 12.0, 128 4500 11.6 | 11.6, 256 4500 13.1 | 11.8, n=3
+//            128 4500 11.0 | 10.6, n=2 256 8192 11.7 | 10.8, 640 4500 20.2 | 13.6
 //   float32  n=4 512 1613 16 | 17, 2047 18 | 18;  1280 1613 26 | 27, 2047 30 | 29;  n=3 832 900 14 | 15, 1100 15 | 15;  n=2 1024 900 13 | 14,
 //            1100 15 | 14, 2560 900 19 | 20, 1100 26 | 21
 //   float32 storage  n=4 512 1900 15 | 16, 2200 17 | 17;  1280 1900 28 | 30, 2700 35 | 34;  1920 1000 22 | 28, 1333 31 | 29;  n=3 1280 1333
 //            18 | 20, 1600 23 | 20;  3072 1333 34 | 33;  n=2 2560 1333 27 | 28, 1900 33 | 30;  4096 1000 29 | 25
-bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C) {
+bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C, bool from_params) {
     if (n < 2 || n > 4 || C % held_chunk(x_dtype) != 0 || C / held_chunk(x_dtype) > 8 * held_most_cb(n)) return false;
     const bool types = (x_dtype == kBF16 && y_dtype == kBF16 && phi_dtype == kBF16) || (x_dtype == kF32 && y_dtype == kF32 && phi_dtype == kF32) ||
                        (x_dtype == kF32AsBF16 && y_dtype == kF32 && phi_dtype == kBF16);
@@ -569,7 +571,8 @@ bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, in
     if (x_dtype == kF32) return B >= (n == 4 ? 1850 : (n == 3 ? 1050 : 1000));
     if (x_dtype == kF32AsBF16) return B >= (nC >= 6144 ? 1300 : (n == 4 ? 2200 : 1600));
     // (where the one-launch forward of layer_fwd_onepass.hip stands beside it: from its second round of workgroups on)
-    if (layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C)) return nC >= 1536 && B > 256 * layer_fwd_onepass_most_samples(n, C);
+    if (layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C))
+        return (nC >= 1536 || (from_params && C >= 128)) && B > 256 * layer_fwd_onepass_most_samples(n, C);
     return B >= (nC <= 6144 ? 2100 : (n < 4 && nC >= 9216 ? 1333 : 1600));
 }
 

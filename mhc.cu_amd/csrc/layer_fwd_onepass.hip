@@ -504,6 +504,11 @@ bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C
     return phi_bytes <= 120 * 1024 || (phi_bytes <= 256 * 1024 && B >= (from_params ? 1280 : 1024) && B <= 2048);
 }
 
+// Whether the one-launch forward reads fp32 parameters itself: in one round of workgroups.  That form has one workgroup on a CU, the
+// packed one two, and with more samples it takes two rounds (forward us, packed by a launch | read here: n=1 C=512 B=4000 10.1 | 9.0,
+// 4500 12.2 | 15.7;  n=2 C=512 4000 11.5 | 10.1, 4200 13.4 | 17.1, 8192 14.7 | 18.1;  n=4 C=256 4000 11.5 | 10.6, 4200 13.1 | 17.7).
+bool layer_fwd_onepass_reads_params(int B, int n, int C) { return B <= 256 * layer_fwd_onepass_most_samples(n, C); }
+
 bool layer_fwd_onepass_gathers(const ParamGather &g) {
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     return g.phi_dtype == kF32 && al16(g.phi[0]) && al16(g.phi[1]) && al16(g.phi[2]) && tuning_get(kTuneGather) != 1;
