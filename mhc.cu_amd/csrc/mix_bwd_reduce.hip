@@ -35,7 +35,8 @@ template <typename TG, typename TX, int NP, int V, int FORM>
 __global__ __launch_bounds__(FORM == kWaveCoef ? 64 : 256) void mix_bwd_reduce_small_kernel(BwdReduceArgs a) {
     constexpr bool FUSED = FORM != kSumsOnly;
     constexpr int kSlots = FORM == kWaveCoef ? 4 : FUSED ? 32 : 16;  // kSumsCoef: up to two column parts
-    using CB = CoefBwdSmall<NP, std::is_same<TX, float>::value, false, false, false, FUSED>;
+    // (kSumsCoef, 4 x 4: the denominators by lane, as the launch of its own keeps them: the same results bit for bit)
+    using CB = CoefBwdSmall<NP, std::is_same<TX, float>::value, false, false, false, FORM == kWaveCoef || (FUSED && NP == 8)>;
     using SK = typename CB::SK;
     constexpr int K = CB::K;  // dM | dHpost | A1 | A2 | s1
     extern __shared__ float smem[];
@@ -1523,14 +1524,14 @@ static hipError_t launch_small(BwdReduceArgs a, hipStream_t stream) {
     if (nt > 256) nt = 256;
     if (nt < SkSmall<NP>::kGroup) nt = SkSmall<NP>::kGroup;  // the epilogue runs on the lanes of one matrix
     constexpr int K = NP * NP + 3 * NP + 1;
-    // at most 14 KB (T <= 32 with the coefficient backward)
+    // at most 20 KB (T <= 32 with the coefficient backward)
     if (form == kWaveCoef) {
         if constexpr (NP == 4) {
             const size_t smem = sizeof(float) * (K * 5 + SkSmall<NP, true>::scaling_floats(a.T));
             mix_bwd_reduce_small_kernel<TG, TX, NP, V, kWaveCoef><<<a.B, 64, smem, stream>>>(a);
         }
     } else if (form == kSumsCoef) {
-        const size_t smem = sizeof(float) * (K * 33 + SkSmall<NP, true>::scaling_floats(a.T));
+        const size_t smem = sizeof(float) * (K * 33 + SkSmall<NP, NP == 8>::scaling_floats(a.T));
         mix_bwd_reduce_small_kernel<TG, TX, NP, V, kSumsCoef><<<a.B, nt, smem, stream>>>(a);
     } else {
         mix_bwd_reduce_small_kernel<TG, TX, NP, V, kSumsOnly><<<dim3(a.B, a.parts), nt, sizeof(float) * K * 17, stream>>>(a);

@@ -47,9 +47,19 @@ template <int NP, bool COMPACT = false> struct SkSmall {
     __device__ static __forceinline__ int row(int g) { return g / NP; }
     __device__ static __forceinline__ int col0(int g) { return g % NP; }
 
+    // COMPACT: the lanes of a row or column share what is saved, so that their sums have to be the same to the last bit: pairs add in
+    // either order, and the product that the first sum adds is rounded on either side (the compiler fuses the plain expression)
+    __device__ static __forceinline__ float first_sum(float a, float b) {
+        if constexpr (COMPACT) {
+#pragma clang fp contract(off)
+            return a + b;
+        } else {
+            return a + b;
+        }
+    }
     // sum over the NP consecutive lanes that hold a row
     __device__ static __forceinline__ float row_allreduce(float v) {
-        v += dpp_mov<kDppQuadXor1>(v);
+        v = first_sum(v, dpp_mov<kDppQuadXor1>(v));
         v += dpp_mov<kDppQuadXor2>(v);
         if constexpr (NP == 8) v += dpp_mov<kDppRowHalfMirror>(v);  // the other quad of the 8 lanes
         return v;
@@ -57,10 +67,10 @@ template <int NP, bool COMPACT = false> struct SkSmall {
     // sum over the lanes that hold a column (stride NP)
     __device__ static __forceinline__ float col_allreduce(float v) {
         if constexpr (NP == 4) {
-            v += dpp_mov<kDppRowRor4>(v);
-            v += dpp_mov<kDppRowRor8>(v);
+            v = first_sum(v, COMPACT ? dpp_mov<kDppRowRor8>(v) : dpp_mov<kDppRowRor4>(v));
+            v += COMPACT ? dpp_mov<kDppRowRor4>(v) : dpp_mov<kDppRowRor8>(v);
         } else {
-            v += dpp_mov<kDppRowRor8>(v);
+            v = first_sum(v, dpp_mov<kDppRowRor8>(v));
             v = xor16_add(v);
             v = xor32_add(v);
         }
