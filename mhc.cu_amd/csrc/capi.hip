@@ -91,7 +91,7 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 // n = 5 .. 8, where the slab is bwd_slab8.hip:
 //   n=5 C=64:   1200 23.9 | 22.1, 1600 25.2 | 26.7, 8192 49.0 | 58.4;  C=256: 1200 25.9 | 26.0, 4000 36.0 | 47.6, 8192 51.4 | 80.7
 //       C=384:  565 24.7 | 23.7, 655 26.8 | 26.9, 829 26.0 | 30.0;  C=1280: 382 25.9 | 25.1, 518 31.4 | 36.7;  C=2560: 245 30.3 | 25.1, 273 30.8 | 35.0;  C=4096: 225 36.7 | 30.9, 291 39.6 | 46.9
-//   n=6 C=64:   4000 37.2 | 37.4, 8192 51.8 | 59.1;  C=256: 1200 28.9 | 27.1, 1600 30.4 | 32.1, 8192 55.4 | 76.9
+//   n=6 C=64:   4000 37.2 | 37.4, 4125 42.3 | 39.6, 8192 51.8 | 59.1;  C=256: 1200 28.9 | 27.1, 1600 30.4 | 32.1, 8192 55.4 | 76.9
 //       C=384:  655 29.3 | 27.2, 765 27.3 | 29.0;  C=768: 647 32.8 | 32.0, 790 30.8 | 35.0;  C=1280: 472 29.9 | 27.8, 527 33.5 | 36.1;  C=2560: 256 31.8 | 25.1, 307 35.4 | 36.4;  C=4096: 227 41.3 | 33.3, 291 44.7 | 48.9
 //   n=7 C=64:   4000 40.1 | 37.8, 8192 54.6 | 60.5;  C=256: 1600 32.4 | 32.6, 4000 42.8 | 49.7, 8192 60.7 | 83.0
 //       C=384:  777 35.6 | 31.4, 1024 31.8 | 32.9, 1163 39.3 | 36.9;  C=768: 680 36.0 | 32.7, 832 34.2 | 35.2, 1087 40.4 | 41.4;  C=1280: 455 37.4 | 32.3, 705 42.0 | 44.9;  C=2560: 361 42.7 | 41.7, 448 41.5 | 45.1
@@ -103,7 +103,7 @@ bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;
     if (n > 4) {
         // (large batches of short rows: the channel sums are gram_wave_kernel there)
-        const int upto128[4] = {1500, 4000, 6000, 7000}, upto256[4] = {1200, 1500, 1900, 3700};
+        const int upto128[4] = {1500, 5000, 6000, 7000}, upto256[4] = {1200, 1500, 1900, 3700};
         if (C <= 256) return B <= (C <= 128 ? upto128 : upto256)[n - 5];
         const int per_row[4] = {500'000, 680'000, 880'000, 940'000}, least[4] = {256, 256, 256, 448}, most[4] = {640, 704, 832, 1400};
         return B <= std::min(most[n - 5], std::max(least[n - 5], per_row[n - 5] / C));
