@@ -1494,9 +1494,8 @@ static hipError_t launch_gram_small_static(BwdReduceArgs a, hipStream_t stream) 
 // kSumsCoef has fewer workgroups and, with 104 registers (n <= 4), four waves per SIMD instead of six: it pays while its workgroups are
 // resident together, and with two parts once there are enough of them to fill the chip.  A wave per sample has nobody wait for the
 // coefficient backward, but a long row's loads come one after the other, and those of single elements (!wide) most of all: n=4 C=515
-// B=1500 56.1 | | 57.3, n=2 C=1283 B=1200 57.3 | | 63.6, n=7
-// C=221 B=1026 58.2 | 60.3.  4096 waves are on the chip at once (n=4 C=128 B=4311 43.8 | | 46.7).  Not with a Sinkhorn state that would take the LDS of the
-// workgroups beside it.
+// B=1500 56.1 | | 57.3, n=2 C=1283 B=1200 57.3 | | 63.6, n=7 C=221 B=1026 58.2 | 60.3.  4096 waves are on the chip at once (n=4
+// C=128 B=4311 43.8 | | 46.7).  Not with a Sinkhorn state that would take the LDS of the workgroups beside it.
 static ReduceForm reduce_small_form(const BwdReduceArgs &a, bool wide) {
     const int B = a.B, C = a.C;
     if (a.T > 32) return kSumsOnly;
