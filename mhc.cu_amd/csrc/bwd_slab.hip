@@ -48,7 +48,7 @@ struct BwdSlabArgs {
     float *dphi_part;        // [S][D][nC]
     double *dw_part;         // [S][C]
     double *dt_part;         // [S][D+3]
-    int w_bf16, B, BP, n, C, tiles;  // tiles of the batch (32 samples, bf16 dy: 16); split y takes tiles [y T / S, (y + 1) T / S)
+    int w_bf16, B, BP, n, C, tiles;  // tiles of the batch (32 samples, bf16 dy: 16), see the kernels for a split's
 };
 
 __device__ __forceinline__ bf16x8_t slab_frag_t(const bf16_t *tile, int k0, int col0, int lane) {
@@ -445,9 +445,12 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
     const int C = a.C, nC = N * C;
     const int slab = blockIdx.x, c0 = slab * CW;
     const unsigned nsplit = gridDim.y;
-    const int b_begin = (int)((uint64_t)blockIdx.y * (unsigned)a.tiles / nsplit) * TB;
-    const int b_end = min(a.B, (int)((uint64_t)(blockIdx.y + 1) * (unsigned)a.tiles / nsplit) * TB);
-    const int T = (b_end - b_begin + TB - 1) / TB;
+    // tiles y, y + S, ..: all splits go through the batch together and begin where the channel sums, which go through it from its end,
+    // have just read x and dy: the memory-side cache (256 MB) still holds that part.  Backward us, splits of consecutive tiles | this: n=4 C=2560
+    // B=8192 162.3 | 156.4 (the order of either kernel alone: 161.0, 168.1), 3000 63.3 | 62.6;  C=1920 4096 63.8 | 62.9;  C=1280 8192 84.1 | 84.7
+    // (forward + backward 121.9 | 121.9);  n=3 C=1024 8192 60.0 | 58.4;  n=2 C=2560 8192 91.5 | 90.3;  n=1 C=4096 6000 80.5 | 80.0
+    const int b_begin = blockIdx.y * TB, b_step = nsplit * TB, b_end = a.B;
+    const int T = (a.tiles - 1 - (int)blockIdx.y) / (int)nsplit + 1;
     const int pwg = blockIdx.y * gridDim.x + blockIdx.x;
     (void)pwg;
     MHC_PHASE_ZERO(kPhaseBwdSlab, pwg);
@@ -467,7 +470,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
     const int ld_row = lane_row(lw * kRows), ld_col = min(lane_col(ld_row), C - 8);
     constexpr int kLoads = F32 ? N * TB / kRows / ST::kLoaders : N;  // instructions per loader for a tile of x, or of both
     auto load_tile = [&](const void *src, int t, uint32_t dst) {
-        const int sb = b_begin + t * TB;
+        const int sb = b_begin + t * b_step;
         if constexpr (F32) {
             const char *base = static_cast<const char *>(src) + ((size_t)sb * nC + c0) * 4;
 #pragma unroll
@@ -518,7 +521,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
     for (int i = 0; i < ST::kShareDt; i++) mine[i] = block_of(lw + i * ST::kLoaders);
     auto load_x = [&](int t) {
         const uint32_t st = smem_at + t % ST::kXRing * ST::kXBytes;
-        const int sb = b_begin + t * TB, left = min(b_end - sb, TB);
+        const int sb = b_begin + t * b_step, left = min(b_end - sb, TB);
         load_tile(F32 ? a.dx : static_cast<const void *>(a.x), t, st);
 #pragma unroll
         for (int i = 0; i < ST::kShareDt; i++) {
@@ -595,7 +598,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
             if (p + ST::kGAhead < T) load_dy(p + ST::kGAhead);
             if (slab == 0) {  // dt column sums: 32 columns x 2 kLoaders row groups
                 const char *st = smem + p % ST::kXRing * ST::kXBytes;
-                const int col = tid & 31, rg = (tid >> 5) - 2 * ST::kMixers, left = b_end - (b_begin + p * TB);
+                const int col = tid & 31, rg = (tid >> 5) - 2 * ST::kMixers, left = b_end - (b_begin + p * b_step);
                 const float *dts = reinterpret_cast<const float *>(st + ST::kCoef) + ST::kSegs * 64;
                 if (col < D + 3) {
 #pragma unroll
@@ -631,7 +634,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
         // a tile of dx leaves in pieces of one KiB, kOut for every mixer
         constexpr int kPieces = N * TB / kRows, kOut = (kPieces + ST::kMixers - 1) / ST::kMixers;
         auto store_dx = [&](int t) {
-            const int sb = b_begin + t * TB;
+            const int sb = b_begin + t * b_step;
             const char *g = smem + ST::kG + t % ST::kGRing * ST::kTile;
 #pragma unroll
             for (int i = 0; i < kOut; i++) {
@@ -656,7 +659,7 @@ __global__ __launch_bounds__(CW * 6, 3) void bwd_slab_stage_kernel(BwdSlabArgs a
         for (int t = 0; t < T; t++) {
             const char *st = smem + t % ST::kXRing * ST::kXBytes;
             char *const gs = smem + ST::kG + t % ST::kGRing * ST::kTile;
-            const int sb = b_begin + t * TB;
+            const int sb = b_begin + t * b_step;
             const float *co = reinterpret_cast<const float *>(st + ST::kCoef);
             MHC_PHASE_ADD(kPhaseBwdSlab, pwg, t > 0 ? 2 : 0, pclk);
             stage_barrier();

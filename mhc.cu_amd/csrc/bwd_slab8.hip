@@ -41,7 +41,7 @@ struct BwdSlab8Args {
     float *dphi_part;        // [S][D][N C]
     double *dw_part;         // [S][C]
     double *dt_part;         // [S slabs][D+3]
-    int w_bf16, B, BP, C, tiles;  // tiles of 16 samples; split y takes tiles [y T / S, (y + 1) T / S)
+    int w_bf16, B, BP, C, tiles;  // tiles of 16 samples
 };
 
 // F32: float32 storage, as in bwd_slab.hip: the channel sums have left x and dy in bf16 where dx will be, and the bytes of CW channels
@@ -82,9 +82,12 @@ __global__ __launch_bounds__((Slab8Stage<N, F32>::kThreads), 2) void bwd_slab8_k
     const int C = a.C, nC = N * C;
     const int slab = blockIdx.x, slabs = gridDim.x, c0 = slab * CW;
     const unsigned nsplit = gridDim.y;
-    const int b_begin = (int)((uint64_t)blockIdx.y * (unsigned)a.tiles / nsplit) * TB;
-    const int b_end = min(a.B, (int)((uint64_t)(blockIdx.y + 1) * (unsigned)a.tiles / nsplit) * TB);
-    const int T = (b_end - b_begin + TB - 1) / TB;
+    // tiles y, y + S, ..: all splits go through the batch together and begin where the channel sums, which go through it from its end,
+    // have just read x and dy: the memory-side cache (256 MB) still holds that part.  Backward us, splits of consecutive tiles | this: n=8 C=2560
+    // B=4096 206.2 | 196.3 (the order of either kernel alone: 204.3, 210.9);  C=1280 3000 84.8 | 84.1;  C=512 8192 98.2 | 95.1;  n=5 C=1024
+    // 8192 94.6 | 90.9;  n=6 C=2560 1024 49.6 | 49.0
+    const int b_begin = blockIdx.y * TB, b_step = nsplit * TB, b_end = a.B;
+    const int T = (a.tiles - 1 - (int)blockIdx.y) / (int)nsplit + 1;
     const int pwg = blockIdx.y * gridDim.x + blockIdx.x;
     (void)pwg;
     MHC_PHASE_ZERO(kPhaseBwdSlab, pwg);
@@ -103,7 +106,7 @@ __global__ __launch_bounds__((Slab8Stage<N, F32>::kThreads), 2) void bwd_slab8_k
     const int ld_at = F32 ? c0 * 4 + lane_chunk(ld_row) * 16 : min(lane_col(ld_row), C - 8) * 2;  // bytes behind the row's first
     auto load_tile = [&](const void *src, int t, uint32_t dst) {
         constexpr int ES = F32 ? 4 : 2;
-        const int sb = b_begin + t * TB;
+        const int sb = b_begin + t * b_step;
         const char *base = static_cast<const char *>(src) + (size_t)sb * nC * ES;
         // slots beyond the batch alias its last sample, columns beyond C the last ones: they only meet zero columns of
         // dP^T or land in rows and columns that are not stored (F32: C is a multiple of 64)
@@ -146,7 +149,7 @@ __global__ __launch_bounds__((Slab8Stage<N, F32>::kThreads), 2) void bwd_slab8_k
     };
     auto load_all = [&](int t, const Block (&mine)[ST::kShare]) {
         const uint32_t st = smem_at + t % ST::kXRing * ST::kXBytes;
-        const int sb = b_begin + t * TB;
+        const int sb = b_begin + t * b_step;
         const uint32_t left = min(b_end - sb, TB);
         load_tile(F32 ? a.dx : static_cast<const void *>(a.x), t, st);
 #pragma unroll
@@ -297,7 +300,7 @@ __global__ __launch_bounds__((Slab8Stage<N, F32>::kThreads), 2) void bwd_slab8_k
         const int row_at = row_place(cl >> 3) + (kq & 1) * 8, row_dy = F32 ? row_place(kChunks / 2 + (cl >> 3)) + (kq & 1) * 8 : row_at;
         constexpr int kPieces = N * TB / kRows, kOut = (kPieces + ST::kMixers - 1) / ST::kMixers;
         auto store_dx = [&](int t) {
-            const int sb = b_begin + t * TB;
+            const int sb = b_begin + t * b_step;
             const char *g = smem + ST::kG + t % ST::kGRing * ST::kTile;
 #pragma unroll
             for (int i = 0; i < kOut; i++) {
@@ -313,7 +316,7 @@ __global__ __launch_bounds__((Slab8Stage<N, F32>::kThreads), 2) void bwd_slab8_k
         for (int t = 0; t < T; t++) {
             const char *st = smem + t % ST::kXRing * ST::kXBytes;
             char *const gs = smem + ST::kG + t % ST::kGRing * ST::kTile;
-            const int sb = b_begin + t * TB;
+            const int sb = b_begin + t * b_step;
             const float *co = reinterpret_cast<const float *>(st + ST::kCoef);
             MHC_PHASE_ADD(kPhaseBwdSlab, pwg, t > 0 ? 2 : 0, pclk);
             stage_barrier();

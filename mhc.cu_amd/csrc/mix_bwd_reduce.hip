@@ -277,6 +277,7 @@ __device__ __forceinline__ uint4 masked_halves(uint4 v, bool first, bool second)
 // and the launch of the coefficient kernel is saved.
 // STATIC (with FUSED): shared coefficients; the tail only converts the sums into the sample's row of raw
 // gradients (see CoefBwdSmall).
+// From the batch's end to its start, as in the two kernels below: the slab kernels then begin with what was read last.
 // 128 registers, four workgroups per CU: their coefficient steps, serial chains on one wave each, hide behind each other (8 x 8 with
 // as many registers as it likes, 138, has three; backward us: n=8 B=2000 C=2560 102.9 -> 100.1, B=3000 C=512 65.3 -> 63.1, n=6
 // B=3000 C=768 57.6 -> 55.1, n=5 B=2000 C=1280 51.5 -> 49.6; five workgroups spill: 122.7, 76.9).
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(256, F32 && NP == 4 ? 3 : 4) void gram_small_kernel
     __shared__ float slot_s[K * 16];  // one slot per 16-lane row of the workgroup
     __shared__ float tot_s[FUSED ? K : 1];
     extern __shared__ float sc[];     // FUSED: Sinkhorn denominators, SK::scaling_floats(T), then CB::kXch
-    const int b = blockIdx.x, part = blockIdx.y, n = a.n, C = a.C;
+    const int b = gridDim.x - 1 - blockIdx.x, part = blockIdx.y, n = a.n, C = a.C;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int pwg = blockIdx.y * gridDim.x + blockIdx.x;
     (void)pwg;
@@ -507,7 +508,7 @@ __global__ __launch_bounds__(64 * kGramWaves, 4) void gram_wave_kernel(BwdReduce
     constexpr bool inject = WMODE == kGramInject;
     extern __shared__ float smem[];  // per wave: slots [K][4] | sums [K] | CB::kXch | Sinkhorn denominators
     const int n = a.n, C = a.C, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = blockIdx.x * kGramWaves + wave;
+    const int b = (gridDim.x - 1 - blockIdx.x) * kGramWaves + wave;
     MHC_PHASE_ZERO(kPhaseGramSmall, blockIdx.x);
     if (b >= a.B) return;
     float *slot_s = smem + wave * (5 * K + CB::kXch + CB::SK::scaling_floats(a.T)), *tot_s = slot_s + 4 * K, *xch = tot_s + K, *sc = xch + CB::kXch;
@@ -663,7 +664,7 @@ __global__ __launch_bounds__(768, F32 ? (U <= 2 ? 6 : 4) : (U <= 2 ? 8 : 7)) voi
     constexpr int K = CB::K, Q = SK::kPerWave;
     constexpr bool inject = WMODE == kGramInject;
     extern __shared__ float smem[];  // slots [Q][K][SW] | sums [Q][K] | Sinkhorn denominators, SK::scaling_floats(T) | Q CB::kXch | w, 16-byte aligned
-    const int b0 = blockIdx.x * a.per_wg, n = a.n, C = a.C, tid = threadIdx.x, lane = tid & 63;
+    const int b0 = (gridDim.x - 1 - blockIdx.x) * a.per_wg, n = a.n, C = a.C, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), SW = (blockDim.x >> 6) - 1;
     const int nb = min(a.per_wg, a.B - b0);
     float *slot_s = smem, *tot_s = slot_s + Q * K * SW, *sc = tot_s + Q * K;
