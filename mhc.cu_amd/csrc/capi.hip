@@ -160,20 +160,29 @@ bool f32_as_bf16_accepted(int B, int n, int C, int iters) {
 //       104 | 104;  C=1024 850 58 | 57, 1100 67 | 69, 4400 212 | 273;  C=1920 1100 113 | 112, 1700 164 | 184;  C=2560 1100 149 | 144, 1500
 //       198 | 222;  C=3072 1700 296 | 295
 //   at most 256 channels: n=5 C=64 3000 40 | 32, C=256 1100 32 | 34, 1500 34 | 31, 4400 54 | 55;  n=8 C=256 4400 74 | 63
+// Around the line the resident path is at its best where its last round of workgroups (two to four a CU) is full.  Forward + backward us:
+//   n=4 C=1024 900 45.7 | 44.2, 990 46.0 | 44.4;  C=1088 940 48.4 | 53.1;  C=1280 700 46.1 | 45.0, 768 46.8 | 46.7, 800 49.9 | 51.7;  C=1536 512
+//       43.9 | 38.4, 660 48.4 | 46.1, 768 50.1 | 49.9;  C=1728 512 44.8 | 42.1, 590 50.3 | 51.5;  C=1920 512 46.1 | 44.7, 513 49.9 | 51.0;  C=2176
+//       512 50.2 | 53.6;  C=2560 440 51.9 | 53.4
+//   n=3 C=960 780 40.2 | 38.8;  C=1280 512 37.3 | 34.7, 560 38.9 | 40.5;  C=1536 512 39.8 | 35.6, 600 41.8 | 41.6;  C=1920 400 39.8 | 36.7, 512
+//       41.3 | 39.0, 520 44.2 | 45.2;  n=2 C=1536 512 34.9 | 33.7, 520 35.9 | 38.7;  n=1 C=1536 520 30.8 | 34.4
+//   n=5 C=1280 512 51.6 | 48.2;  C=1024 540 50.0 | 54.0;  C=2048 512 62.4 | 67.7;  n=6 C=1280 512 56.0 | 50.8;  C=1920 512 65.1 | 69.6;  n=8
+//       C=1024 1024 89.4 | 88.6, 1100 103.1 | 104.7
 bool bwd_f32_tiled(int B, int n, int C) {
     if (n > 8 || C % 64 != 0) return false;
     if (const int hook = tuning_get(kTuneResident)) return hook == 1;
-    if (n == 8) return C >= 1024 && B >= std::max(1000, 5 * C / 8);
+    if (n == 8) return C >= 1024 && B >= std::max(1025, 5 * C / 8);
     if (n > 4) {
         const int least[3] = {340, 330, 450}, over_row[3] = {200'000, 215'000, 230'000};
-        return C > 256 && B >= std::max(least[n - 5] + over_row[n - 5] / C, n == 7 ? C / 4 : 0);
+        return C > 256 && B >= std::max(least[n - 5] + over_row[n - 5] / C, n == 7 ? C / 4 : (C <= 1600 ? 513 : 0));
     }
     if (C <= 256) {
         const int from[4] = {700, 850, 1000, 1150}, again[4] = {2000, 2000, 2000, 4000};
         return B > 1536 ? B >= again[n - 1] : B >= from[n - 1];
     }
-    const int least[4] = {280, 280, 320, 420}, most[4] = {620, 740, 950, 1000}, per_row[4] = {720'000, 720'000, 730'000, 880'000};
-    return B >= std::max(least[n - 1], std::min(most[n - 1], per_row[n - 1] / C));
+    if (n >= 3) return B >= (C <= 1024 ? (n == 3 ? 950 : 1000) : (n == 4 && C <= 1600) ? 769 : C <= 2000 ? 513 : (n == 3 ? 320 : 420));
+    const int most[2] = {620, 740};
+    return B >= std::max(C <= 1600 ? 513 : 280, std::min(most[n - 1], 720'000 / C));
 }
 
 int max_ksplit(int B, int n, int C) {
