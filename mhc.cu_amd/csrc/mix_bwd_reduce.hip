@@ -277,7 +277,6 @@ __device__ __forceinline__ uint4 masked_halves(uint4 v, bool first, bool second)
 // and the launch of the coefficient kernel is saved.
 // STATIC (with FUSED): shared coefficients; the tail only converts the sums into the sample's row of raw
 // gradients (see CoefBwdSmall).
-// From the batch's end to its start, as in the two kernels below: the slab kernels then begin with what was read last.
 // 128 registers, four workgroups per CU: their coefficient steps, serial chains on one wave each, hide behind each other (8 x 8 with
 // as many registers as it likes, 138, has three; backward us: n=8 B=2000 C=2560 102.9 -> 100.1, B=3000 C=512 65.3 -> 63.1, n=6
 // B=3000 C=768 57.6 -> 55.1, n=5 B=2000 C=1280 51.5 -> 49.6; five workgroups spill: 122.7, 76.9).
@@ -299,7 +298,7 @@ __global__ __launch_bounds__(256, F32 && NP == 4 ? 3 : 4) void gram_small_kernel
     __shared__ float slot_s[K * 16];  // one slot per 16-lane row of the workgroup
     __shared__ float tot_s[FUSED ? K : 1];
     extern __shared__ float sc[];     // FUSED: Sinkhorn denominators, SK::scaling_floats(T), then CB::kXch
-    const int b = gridDim.x - 1 - blockIdx.x, part = blockIdx.y, n = a.n, C = a.C;
+    const int b = blockIdx.x, part = blockIdx.y, n = a.n, C = a.C;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int pwg = blockIdx.y * gridDim.x + blockIdx.x;
     (void)pwg;
@@ -497,6 +496,8 @@ __global__ __launch_bounds__(256, F32 && NP == 4 ? 3 : 4) void gram_small_kernel
 // and shares nothing with the others.  In gram_small_kernel the sums of a sample wait for three waves and its coefficient backward
 // leaves those three idle; with short rows it is most of a workgroup's life.  Channel sums of n=5 B=8192 C=512 54 us there (84 MB: 17).
 // A step's products have sums of their own: one chain over a row would be three times as long as there.
+// From the batch's end to its start: the slab kernel behind then begins with what was read last (gram_small_kernel, whose batches fit the
+// memory-side cache, forwards: forward + backward n=4 C=2560 B=1000 51.4 us | 52.4 from the end, 1280 58.1 | 58.9).
 // F32: as in gram_small_kernel.
 constexpr int kGramWaves = 4;
 template <int WMODE, bool F32>
@@ -654,7 +655,7 @@ __global__ __launch_bounds__(64 * kGramWaves, 4) void gram_wave_kernel(BwdReduce
 // eight iterations, and four steps per wave (80 registers and spills) lost to gram_small_kernel.
 // B=8192 n=4 C=2560: 72 -> 65 us (336 MB, 5.2 TB/s).
 constexpr int kGramQuadSteps = 33;
-// F32: as in gram_small_kernel.
+// F32: as in gram_small_kernel.  From the batch's end to its start, as in gram_wave_kernel.
 template <int WMODE, int U, bool F32 = false>
 __global__ __launch_bounds__(768, F32 ? (U <= 2 ? 6 : 4) : (U <= 2 ? 8 : 7)) void gram_quad_kernel(BwdReduceArgs a) {
     static_assert(!F32 || WMODE != kGramInject, "an injected f takes the other kernels");
