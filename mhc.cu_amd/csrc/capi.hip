@@ -142,47 +142,66 @@ bool f32_as_bf16_accepted(int B, int n, int C, int iters) {
            bwd_resident_supported(kF32AsBF16, kF32, kBF16, n, C, iters) && proj_bwd_addx_supported(n);
 }
 
-// Whether the backward of float32 storage takes the tiled path (channel sums that leave x and dy in bf16, slab) instead of the
-// resident one.  Backward us, tiled | resident, on either side of the line and beyond:
-//   n=1 C=256 B=600 17 | 17, 1300 20 | 27;  C=1280 510 20 | 20, 580 20 | 24;  C=4096 260 20 | 21, 4369 118 | 192
-//   n=2 C=512 600 18 | 17, 800 19 | 20;  C=1280 510 21 | 20, 580 23 | 25;  C=4096 300 27 | 32, 3000 108 | 177
-//   n=3 C=512 760 20 | 20, 1000 24 | 26;  C=1280 510 25 | 23, 580 25 | 26;  C=2560 330 26 | 27;  C=3136 3000 124 | 199
-//   n=4 C=640 720 25 | 24, 1000 27 | 29, 8000 98 | 131;  C=1280 510 28 | 24, 760 30 | 31, 4369 113 | 142;  C=2560 330 33 | 32, 513 39 | 46,
-//       2000 90 | 133;  C=4096 400 42 | 43
-//   at most 256 channels the resident path splits the batch beyond 1536 samples: n=4 C=256 1536 28 | 30, 2000 28 | 26, 4369 37 | 39
-//   n=5 C=320 925 30 | 34;  C=512 650 30 | 30, 850 32 | 36;  C=1024 450 31 | 30, 650 35 | 40, 4400 110 | 198;  C=2560 300 41 | 40, 450 43 | 46,
-//       2000 115 | 196
-//   n=6 C=512 650 32 | 31, 850 34 | 35;  C=1024 450 34 | 30, 650 38 | 41, 4400 126 | 239;  C=1536 399 37 | 37, 563 44 | 50;  C=2560 300
-//       45 | 42, 450 48 | 49, 2000 143 | 229
-//   n=7 C=512 650 33 | 31, 850 36 | 36, 1100 40 | 43;  C=1024 450 36 | 32, 650 42 | 44, 4400 156 | 273;  C=2560 450 59 | 57, 650 75 | 81, 2000
-//       192 | 282;  C=3136 568 88 | 85, 1183 150 | 164
-//   n=8 (slabs of 32 channels: shorter runs of a row, more partial sums) C=512 2000 63 | 62, 4400 114 | 118;  C=768 1700 75 | 71, 2600
-//       104 | 104;  C=1024 850 58 | 57, 1100 67 | 69, 4400 212 | 273;  C=1920 1100 113 | 112, 1700 164 | 184;  C=2560 1100 149 | 144, 1500
-//       198 | 222;  C=3072 1700 296 | 295
-//   at most 256 channels: n=5 C=64 3000 40 | 32, C=256 1100 32 | 34, 1500 34 | 31, 4400 54 | 55;  n=8 C=256 4400 74 | 63
-// Around the line the resident path is at its best where its last round of workgroups (two to four a CU) is full.  Forward + backward us:
-//   n=4 C=1024 900 45.7 | 44.2, 990 46.0 | 44.4;  C=1088 940 48.4 | 53.1;  C=1280 700 46.1 | 45.0, 768 46.8 | 46.7, 800 49.9 | 51.7;  C=1536 512
-//       43.9 | 38.4, 660 48.4 | 46.1, 768 50.1 | 49.9;  C=1728 512 44.8 | 42.1, 590 50.3 | 51.5;  C=1920 512 46.1 | 44.7, 513 49.9 | 51.0;  C=2176
-//       512 50.2 | 53.6;  C=2560 440 51.9 | 53.4
-//   n=3 C=960 780 40.2 | 38.8;  C=1280 512 37.3 | 34.7, 560 38.9 | 40.5;  C=1536 512 39.8 | 35.6, 600 41.8 | 41.6;  C=1920 400 39.8 | 36.7, 512
-//       41.3 | 39.0, 520 44.2 | 45.2;  n=2 C=1536 512 34.9 | 33.7, 520 35.9 | 38.7;  n=1 C=1536 520 30.8 | 34.4
-//   n=5 C=1280 512 51.6 | 48.2;  C=1024 540 50.0 | 54.0;  C=2048 512 62.4 | 67.7;  n=6 C=1280 512 56.0 | 50.8;  C=1920 512 65.1 | 69.6;  n=8
-//       C=1024 1024 89.4 | 88.6, 1100 103.1 | 104.7
+// Whether the backward of float32 storage takes the tiled path (channel sums that leave x and dy in bf16, slab) instead of the resident
+// one.  The resident path's time is a staircase: a workgroup per sample, two to eight of them on a CU by the registers and waves
+// that the row takes, and it is at its best where its last round of workgroups is full (256 x 2, x 3, x 4 samples).  The lines stand behind
+// the full rounds that it wins, between row lengths at which another form of it begins (items of 512 channels, with n > 4 also of 896
+// and 1280).  n = 8 has slabs of 32 channels (shorter runs of a row, more partial sums) and a slab kernel with 19 registers in scratch
+// memory.  Forward + backward us in graphs of ten, tiled | resident, on either side of the lines:
+//   n=1 C=512: 600 27.4 | 27.6, 680 27.7 | 28.4;  C=1536: 512 30.6 | 29.9, 540 31.5 | 35.4;  C=1600: 256 26.5 | 23.3, 300 28.5 | 30.0;  C=2624:
+//       340 34.2 | 33.3, 1024 51.1 | 48.1, 1060 54.2 | 59.8;  C=3584: 460 40.4 | 39.0, 540 43.3 | 46.4
+//   n=2 C=512: 600 29.4 | 28.8, 768 29.3 | 30.4;  C=1024: 540 32.6 | 33.0, 600 32.6 | 33.8;  C=2048: 512 37.4 | 36.7, 540 39.8 | 43.8;  C=2624:
+//       512 41.1 | 37.9, 800 51.1 | 53.0;  C=3584: 512 46.2 | 45.9, 540 50.5 | 53.2;  C=4096: 256 38.2 | 35.8, 300 42.9 | 45.4
+//   n=3 C=1024: 800 40.7 | 41.1, 1024 41.5 | 43.6;  C=1280: 512 38.0 | 34.8, 540 39.4 | 40.4;  C=1536: 680 43.6 | 43.2, 800 47.0 | 50.2;
+//       C=2048: 512 43.2 | 41.3, 540 46.6 | 48.1;  C=2560: 300 42.5 | 42.6, 460 45.2 | 46.0;  C=2624: 512 46.6 | 44.8, 600 53.0 | 54.1;  C=3584:
+//       384 49.6 | 48.8, 420 50.7 | 52.2
+//   n=4 C=1024: 1024 46.6 | 45.4, 1060 49.8 | 52.0;  C=1536: 512 44.1 | 38.4, 768 50.9 | 50.0, 800 53.8 | 55.4;  C=1600: 512 44.2 | 41.1, 600
+//       47.3 | 48.5;  C=2048: 512 46.7 | 45.9, 600 52.0 | 55.7;  C=2560: 384 50.3 | 49.0, 460 52.6 | 54.4;  C=2624: 512 55.7 | 53.0, 768 69.6 |
+//       72.6;  C=3584: 460 62.9 | 61.2, 540 73.7 | 74.5
+//   n=5 C=384: 600 41.7 | 41.1, 680 42.5 | 44.2;  C=512: 1150 53.4 | 59.4, 1250 55.9 | 54.4, 1300 56.0 | 57.9;  C=896: 768 51.4 | 49.9, 900 57.6
+//       | 59.2;  C=1664: 460 56.8 | 55.0, 540 68.7 | 74.1;  C=2560: 384 71.8 | 71.5, 460 72.3 | 75.4
+//   n=6 C=384: 680 45.0 | 45.1, 768 43.5 | 45.7, 1300 56.8 | 55.6;  C=512: 768 47.4 | 48.5, 1280 58.8 | 57.0, 1300 59.0 | 61.4;  C=768: 768 53.3
+//       | 51.1, 900 59.4 | 60.6;  C=896: 600 54.2 | 48.9, 1024 64.5 | 65.1;  C=1792: 460 64.4 | 62.2, 540 75.7 | 79.2;  C=2624: 512 82.8 | 81.5,
+//       540 100 | 104
+//   n=7 C=640: 820 58.6 | 57.4, 950 62.4 | 62.4;  C=768: 1024 68.0 | 66.1, 1280 75.4 | 78.1;  C=896: 768 64.0 | 58.6, 1280 86.4 | 84.9, 1536
+//       94.7 | 95.3;  C=1024: 512 53.7 | 49.9, 540 59.1 | 59.6;  C=1792: 600 90.7 | 86.2, 800 108 | 110;  C=3072: 1024 205 | 202, 1060 229 | 235
+//   n=8 C=1024: 1024 88.7 | 88.1, 1060 103 | 104;  C=1792: 1400 199 | 185, 1800 249 | 251;  C=2048: 1400 215 | 209, 1537 234 | 241;  C=2560:
+//       1150 245 | 234, 1400 290 | 296;  C=3072: 1060 290 | 269, 2000 495 | 483;  C=3328: 1060 308 | 302, 1280 340 | 349;  C=4096: 1060 340 |
+//       357
+//   at most 256 channels, where the resident path splits larger batches: n=1 C=64 1600 30.0 | 28.6, 2000 29.2 | 28.3, 2100 29.4 | 32.5, n=3
+//       C=128 1024 31.2 | 30.4, 1060 31.8 | 33.4, n=4 C=64 1060 32.8 | 33.7, 2000 36.9 | 33.1, 4000 44.1 | 41.9, 4200 45.5 | 46.1
+//   beyond a full round of larger batches: n=4 C=512 1536 45.9 | 49.5, 1600 47.2 | 45.6, 1800 47.5 | 49.7
+constexpr BatchLine kF32Tiled1[] = {{512, 700}, {1024, 620}, {1536, 513}, {2560, 280}, {2688, 1025}, {3072, 280}, {3584, 513}, {kAnyRow, 280}};
+constexpr BatchLine kF32Tiled2[] = {{256, 850}, {576, 740}, {1024, 600}, {2560, 513}, {2688, 769}, {3584, 513}, {kAnyRow, 280}};
+constexpr BatchLine kF32Tiled3[] = {{256, 1025}, {1024, 950}, {1280, 513}, {1536, 769}, {2048, 513}, {2560, 320}, {2688, 513}, {3072, 320}, {3584, 400}, {kAnyRow, 320}};
+constexpr BatchLine kF32Tiled4[] = {{1024, 1025}, {1536, 769}, {2048, 513}, {2560, 420}, {2688, 680}, {3584, 490}, {kAnyRow, 420}};
+constexpr BatchLine kF32Tiled5[] = {{256, kNever}, {384, 680}, {768, 700}, {896, 800}, {1664, 513}, {2688, 450}, {kAnyRow, 400}};
+constexpr BatchLine kF32Tiled6[] = {{256, kNever}, {384, 768}, {768, 850}, {896, 1000}, {1792, 513}, {2560, 460}, {2688, 513}, {kAnyRow, 400}};
+constexpr BatchLine kF32Tiled7[] = {{256, kNever}, {384, 850}, {640, 920}, {704, 1040}, {768, 1200}, {896, 1500}, {1024, 540}, {1216, 769}, {1408, 600},
+                                    {1536, 680}, {1792, 769}, {2048, 600}, {2496, 769}, {2688, 640}, {3584, 1025}, {kAnyRow, 960}};
+constexpr BatchLine kF32Tiled8[] = {{1023, kNever}, {1600, 1025}, {1792, 1750}, {2112, 1500}, {2688, 1350}, {3072, kNever}, {3519, 1200}, {kAnyRow, 1025}};
+// further full rounds beyond a line
+bool bwd_f32_resident_round(int B, int n, int C) {
+    const auto in = [&](int c_min, int c_max, int b_min, int b_max) { return C >= c_min && C <= c_max && B >= b_min && B <= b_max; };
+    if (n <= 4) return in(0, 256, 1537, n == 4 ? 4096 : 2048) || (n >= 3 && in(257, 512, 1537, 1700));
+    return (n <= 6 && in(385, 512, 1201, 1280)) || (n == 6 && in(257, 384, 1281, 1450));
+}
 bool bwd_f32_tiled(int B, int n, int C) {
     if (n > 8 || C % 64 != 0) return false;
     if (const int hook = tuning_get(kTuneResident)) return hook == 1;
-    if (n == 8) return C >= 1024 && B >= std::max(1025, 5 * C / 8);
-    if (n > 4) {
-        const int least[3] = {340, 330, 450}, over_row[3] = {200'000, 215'000, 230'000};
-        return C > 256 && B >= std::max(least[n - 5] + over_row[n - 5] / C, n == 7 ? C / 4 : (C <= 1600 ? 513 : 0));
-    }
-    if (C <= 256) {
-        const int from[4] = {700, 850, 1000, 1150}, again[4] = {2000, 2000, 2000, 4000};
-        return B > 1536 ? B >= again[n - 1] : B >= from[n - 1];
-    }
-    if (n >= 3) return B >= (C <= 1024 ? (n == 3 ? 950 : 1000) : (n == 4 && C <= 1600) ? 769 : C <= 2000 ? 513 : (n == 3 ? 320 : 420));
-    const int most[2] = {620, 740};
-    return B >= std::max(C <= 1600 ? 513 : 280, std::min(most[n - 1], 720'000 / C));
+    const auto line = [&] {
+        switch (n) {
+            case 1: return batch_line(kF32Tiled1, C);
+            case 2: return batch_line(kF32Tiled2, C);
+            case 3: return batch_line(kF32Tiled3, C);
+            case 4: return batch_line(kF32Tiled4, C);
+            case 5: return batch_line(kF32Tiled5, C);
+            case 6: return batch_line(kF32Tiled6, C);
+            case 7: return batch_line(kF32Tiled7, C);
+            default: return batch_line(kF32Tiled8, C);
+        }
+    };
+    return B >= line() && !bwd_f32_resident_round(B, n, C);
 }
 
 int max_ksplit(int B, int n, int C) {
@@ -346,6 +365,12 @@ __attribute__((visibility("default"))) int mhc_tuning_set(int key, int value) {
 }
 __attribute__((visibility("default"))) int mhc_tuning_get(int key) {
     return (key < 0 || key >= kTuneCount) ? -1 : g_tuning[key];
+}
+__attribute__((visibility("default"))) int mhc_tuning_route(int route, int x_dtype, int B, int n, int C) {
+    switch (route) {
+        case kRouteBackward: return x_dtype == kF32AsBF16 ? bwd_f32_tiled(B, n, C) : !bwd_resident_preferred(B, n, C);
+        default: return -1;
+    }
 }
 #endif
 

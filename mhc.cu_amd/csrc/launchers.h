@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stddef.h>
 
 #include "batch_sums.h"
@@ -30,6 +31,15 @@ template <auto Kernel> inline hipError_t allow_dynamic_lds(size_t bytes) {
     return allowed.raise(dev, (int)bytes, [](int value) {
         return hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, value);
     });
+}
+
+// A line between two launch paths: rows of at most `upto` channels take the second path from `from` samples on.
+struct BatchLine { int upto, from; };
+constexpr int kAnyRow = INT_MAX, kNever = INT_MAX;
+template <int N> constexpr int batch_line(const BatchLine (&lines)[N], int C) {  // the last of them is for kAnyRow
+    int i = 0;
+    while (C > lines[i].upto) i++;
+    return lines[i].from;
 }
 
 // Projection row count padded to whole 32-wide MFMA tiles.

@@ -24,6 +24,11 @@ enum TuneKey {
     kTuneCount = 13
 };
 
+// What mhc_tuning_route() of the same build tells about the built-in heuristic, for tests of its lines.
+enum RouteKey {
+    kRouteBackward = 0,     // n <= 8, bf16 arithmetic: 0 = sample-resident, 1 = tiled
+};
+
 #ifdef MHC_TUNING
 extern int g_tuning[kTuneCount];
 inline int tuning_get(int key) { return g_tuning[key]; }

@@ -83,7 +83,7 @@ _TUNING_LIB = None
 def tuning_lib():
     """The test/experiment build of the same library (libmhc_hip_tuning.so, `build.py --tuning`): the same
     entry points plus mhc_tuning_set / mhc_tuning_get, which override the launch heuristics
-    (csrc/tuning.h) for the whole process.  The product library above has no such hooks; tests load
+    (csrc/tuning.h) for the whole process, and mhc_tuning_route, which tells what they choose.  The product library above has no such hooks; tests load
     this one to compare two launch paths on the same inputs."""
     global _TUNING_LIB
     if _TUNING_LIB is None:
@@ -95,6 +95,8 @@ def tuning_lib():
         handle.mhc_tuning_set.argtypes = [c_int, c_int]
         handle.mhc_tuning_get.restype = c_int
         handle.mhc_tuning_get.argtypes = [c_int]
+        handle.mhc_tuning_route.restype = c_int
+        handle.mhc_tuning_route.argtypes = [c_int] * 5
         _TUNING_LIB = handle
     return _TUNING_LIB
 

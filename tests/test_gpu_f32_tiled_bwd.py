@@ -81,13 +81,15 @@ def test_same_as_the_resident_backward(n, C, wt):
             assert e <= {"dalpha": 1e-3, "dx": 2e-4}.get(k, 2e-5), (B, k, e)
 
 
-@pytest.mark.parametrize("B,n,C", [(1701, 4, 320), (1150, 3, 512), (4100, 4, 256), (1000, 2, 1024), (963, 5, 576), (801, 6, 640),
-                                   (1001, 7, 512), (1003, 8, 1024)])  # (n = 1: dHpre is the difference of equal sums)
+@pytest.mark.parametrize("B,n,C", [(1701, 4, 320), (1150, 3, 512), (4100, 4, 256), (1000, 2, 1024), (963, 5, 576), (1001, 6, 640),
+                                   (1001, 7, 512), (1029, 8, 1024), (1721, 8, 1024)])  # (n = 1: dHpre is the difference of equal sums)
 def test_through_the_module(B, n, C):
-    """Sizes at which the layer takes this path by itself."""
+    """Sizes at which the layer takes this path by itself (the last one with a wave per sample for the channel sums)."""
     import mhc
+    from mhc._lib import tuning_lib
     from oracle import naive_mhc as nm
 
+    assert tuning_lib().mhc_tuning_route(0, F32_AS_BF16, B, n, C) == 1
     torch.manual_seed(2)
     with torch.device("cuda"):
         layer = mhc.MHCLayer(C, n, compute_dtype=torch.bfloat16)
