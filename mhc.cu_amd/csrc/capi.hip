@@ -224,6 +224,20 @@ DynFwdWs carve_dyn_fwd(void *ws, int B, int n, int C) {
     return w;
 }
 
+// How the dynamic forward goes.  direct: the caller's own parameters are whole 16-byte pieces, which a kernel can read (the others are
+// packed by a launch of their own).
+enum ForwardKind { kTwoLaunches, kOneLaunch, kOneLaunchReadsParams, kHeldForward };
+struct ForwardRoute { ForwardKind kind; bool direct; };
+ForwardRoute forward_route(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C, bool inject, const ParamGather *gather, size_t part_bytes) {
+    const bool direct = gather && aligned16(gather->phi[0]) && aligned16(gather->phi[1]) && aligned16(gather->phi[2]);
+    if (!inject && layer_fwd_held_supported(x_dtype, y_dtype, phi_dtype, B, n, C, direct && gather->phi_dtype == kF32) &&
+        layer_fwd_held_bytes(x_dtype, n, C) <= part_bytes)
+        return {kHeldForward, direct};
+    const bool can_gather = gather && layer_fwd_onepass_gathers(*gather);
+    if (!layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C, can_gather)) return {kTwoLaunches, direct};
+    return {can_gather && layer_fwd_onepass_reads_params(B, n, C) ? kOneLaunchReadsParams : kOneLaunch, direct};
+}
+
 // Wide projections (n > 18) without batch split of dphi: four launches, see mhc_layer_bwd_dynamic.
 // Up to 16 M activation elements: the fp32 hand-over costs 4 more bytes per element than completing dx
 // in place, which the shorter chain repays only while the coefficient launch leaves CUs idle
@@ -369,6 +383,11 @@ __attribute__((visibility("default"))) int mhc_tuning_get(int key) {
 __attribute__((visibility("default"))) int mhc_tuning_route(int route, int x_dtype, int B, int n, int C) {
     switch (route) {
         case kRouteBackward: return x_dtype == kF32AsBF16 ? bwd_f32_tiled(B, n, C) : !bwd_resident_preferred(B, n, C);
+        case kRouteForward: {
+            const ParamGather g{{nullptr, nullptr, nullptr}, kF32};
+            const bool exact = x_dtype == kF32;
+            return forward_route(x_dtype, x_dtype == kBF16 ? kBF16 : kF32, exact ? kF32 : kBF16, B, n, C, false, &g, carve_dyn_fwd(nullptr, B, n, C).part_bytes).kind;
+        }
         default: return -1;
     }
 }
@@ -705,22 +724,19 @@ int fwd_dynamic(const void *x, int x_dtype, const void *w, int w_dtype, const Pa
     const DynFwdWs ws = carve_dyn_fwd(workspace, B, n, C);
     if (int s = ws_check(workspace, workspace_bytes, ws.bytes)) return s;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // (parameters that are not whole 16-byte pieces are packed by a launch of their own)
-    const bool direct = gather && aligned16(gather->phi[0]) && aligned16(gather->phi[1]) && aligned16(gather->phi[2]);
-    if (!f_inject && layer_fwd_held_supported(x_dtype, y_dtype, phi_dtype, B, n, C, direct && gather->phi_dtype == kF32) &&
-        layer_fwd_held_bytes(x_dtype, n, C) <= ws.part_bytes) {
-        if (gather && !direct) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
-        MHC_LAUNCH(launch_layer_fwd_held(x, x_dtype, w, w_dtype, y, direct ? gather : nullptr, phi, alpha, bias, ws.Ppart, H_pre, H_post,
-                                         M, P, r, q, sk_state, B, n, C, iters, eps, st));
+    const ForwardRoute route = forward_route(x_dtype, y_dtype, phi_dtype, B, n, C, f_inject != nullptr, gather, ws.part_bytes);
+    if (route.kind == kHeldForward) {
+        if (gather && !route.direct) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
+        MHC_LAUNCH(launch_layer_fwd_held(x, x_dtype, w, w_dtype, y, route.direct ? gather : nullptr, phi, alpha, bias, ws.Ppart, H_pre,
+                                         H_post, M, P, r, q, sk_state, B, n, C, iters, eps, st));
         return MHC_OK;
     }
     // the caller's own parameters: read by the kernel that multiplies with them where it can, otherwise packed by a launch
     // of their own
-    const bool can_gather = gather && layer_fwd_onepass_gathers(*gather);
-    const bool one = layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C, can_gather), in_one = one && can_gather && layer_fwd_onepass_reads_params(B, n, C);
-    const bool in_proj = gather && !one && proj_fwd_gathers(*gather, x_dtype, B, n, C);
+    const bool in_one = route.kind == kOneLaunchReadsParams;
+    const bool in_proj = gather && route.kind == kTwoLaunches && proj_fwd_gathers(*gather, x_dtype, B, n, C);
     if (gather && !in_one && !in_proj) MHC_LAUNCH(launch_pack_params(*gather, n, C, st));
-    if (one) {
+    if (route.kind != kTwoLaunches) {
         // projection, coefficients and mix in one launch; x crosses HBM once
         MHC_LAUNCH(launch_layer_fwd_onepass(x, w, w_dtype, f_inject, y, y_dtype, phi, alpha, bias, H_pre, H_post,
                                             M, P, r, q, sk_state, B, n, C, iters, eps, st, in_one ? gather : nullptr));

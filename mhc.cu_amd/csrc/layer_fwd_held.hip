@@ -556,10 +556,27 @@ size_t layer_fwd_held_bytes(int x_dtype, int n, int C) { return (size_t)held_uni
 //            18 | 22, 2700 34 | 22;  shorter rows n=4 256 8192 12 | 13, 12000 19 | 16, 20000 28 | 28;  from the caller's fp32
 //            parameters, which that one has packed by a launch there: n=4 64 8192 11.8 | 12.0, 128 4500 11.6 | 11.6, 256 4500 13.1 | 11.8, n=3
 //            128 4500 11.0 | 10.6, n=2 256 8192 11.7 | 10.8, 640 4500 20.2 | 13.6
-//   float32  n=4 512 1613 16 | 17, 2047 18 | 18;  1280 1613 26 | 27, 2047 30 | 29;  n=3 832 900 14 | 15, 1100 15 | 15;  n=2 1024 900 13 | 14,
-//            1100 15 | 14, 2560 900 19 | 20, 1100 26 | 21
-//   float32 storage  n=4 512 1900 15 | 16, 2200 17 | 17;  1280 1900 28 | 30, 2700 35 | 34;  1920 1000 22 | 28, 1333 31 | 29;  n=3 1280 1333
-//            18 | 20, 1600 23 | 20;  3072 1333 34 | 33;  n=2 2560 1333 27 | 28, 1900 33 | 30;  4096 1000 29 | 25
+//   float32  n=2 640 1000 12.3 | 12.5, 1060 12.9 | 12.5;  768 1060 13.3 | 13.4, 1350 14.3 | 13.7;  896 1150 13.8 | 15.0, 1350 15.0 | 15.1, 1500
+//            15.5 | 15.3;  1152 1100 16.2 | 16.6, 1250 16.6 | 16.6;  1664 1200 17.5 | 18.3, 1250 18.5 | 18.4;  2048 1030 18.6 | 19.4, 1150 19.5
+//            | 18.4;  2560 1000 20.2 | 21.3, 1030 26.0 | 21.3;  n=3 384 1000 12.2 | 12.1, 1060 13.2 | 12.1;  576 1150 13.5 | 14.5, 1200 14.9 |
+//            14.6;  640 1000 13.4 | 14.5, 1100 15.1 | 14.5;  768 1300 15.4 | 15.9, 1400 16.7 | 16.0;  832 1060 15.7 | 15.8, 1200 15.6 | 15.5;
+//            1152 1150 17.0 | 17.4, 1200 18.5 | 17.5;  1536 1000 19.5 | 19.3, 1060 20.7 | 19.4;  n=4 384 1500 14.7 | 15.0, 1900 15.4 | 15.0;
+//            448 1950 17.0 | 17.4, 2100 18.0 | 17.4;  1024 1500 21.9 | 23.5, 1850 29.3 | 24.6;  1152 1950 26.9 | 28.3, 2100 32.9 | 28.4;  1280
+//            1500 25.6 | 26.5, 1850 29.7 | 28.4
+//   float32 storage  n=2 640 1330 12.5 | 12.3, 1600 13.0 | 12.5;  896 1500 14.1 | 14.4, 1700 14.5 | 14.3;  1280 1500 15.9 | 16.7, 1600 20.0 |
+//            16.5;  n=3 512 1500 13.4 | 12.8, 1650 13.7 | 12.9;  640 1900 15.1 | 15.4, 2100 17.3 | 15.5;  704 1600 15.0 | 15.7, 1750 16.6 |
+//            15.6;  1024 1700 18.3 | 19.5, 1800 22.1 | 19.3;  1152 1500 18.6 | 19.3, 1600 23.0 | 19.1;  1344 1650 25.8 | 26.5, 1850 26.6 | 26.1;
+//            2048 1150 23.4 | 21.5, 1300 29.5 | 21.5;  n=4 320 2200 14.6 | 15.0, 2400 15.2 | 15.3;  512 2300 17.4 | 17.7, 2400 17.7 | 17.0;
+//            1024 2100 28.4 | 24.3, 2200 29.0 | 24.4;  1280 2100 30.6 | 30.9, 2400 32.2 | 32.3;  1536 1150 23.2 | 22.5, 1330 25.2 | 23.0;  2304
+//            1150 32.3 | 34.0, 1400 36.5 | 35.2
+// In float32 and float32 storage the lines go by the registers of a row's form: where another number of chunks per wave begins (768 ->
+// 832 channels at n = 2) a tile costs as much as one of the longest rows of that form.
+constexpr BatchLine kHeldF32N2[] = {{448, 1000}, {640, 1030}, {768, 1150}, {1024, 1350}, {1280, 1200}, {1536, 1000}, {1856, 1250}, {2048, 1080}, {kAnyRow, 1030}};
+constexpr BatchLine kHeldF32N3[] = {{256, 1000}, {384, 1030}, {576, 1200}, {640, 1050}, {768, 1400}, {1024, 1100}, {1344, 1175}, {kAnyRow, 1050}};
+constexpr BatchLine kHeldF32N4[] = {{384, 1850}, {512, 2050}, {1024, 1850}, {1152, 2050}, {kAnyRow, 1850}};
+constexpr BatchLine kHeldStoredN2[] = {{3071, 1600}, {kAnyRow, 1300}};
+constexpr BatchLine kHeldStoredN3[] = {{512, 1600}, {640, 2050}, {768, 1720}, {1024, 1800}, {1280, 1600}, {1344, 1800}, {2047, 1600}, {kAnyRow, 1300}};
+constexpr BatchLine kHeldStoredN4[] = {{256, 2200}, {320, 2400}, {512, 2350}, {1024, 2200}, {1280, 2300}, {1535, 2200}, {kAnyRow, 1300}};
 bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C, bool from_params) {
     if (n < 2 || n > 4 || C % held_chunk(x_dtype) != 0 || C / held_chunk(x_dtype) > 8 * held_most_cb(n)) return false;
     const bool types = (x_dtype == kBF16 && y_dtype == kBF16 && phi_dtype == kBF16) || (x_dtype == kF32 && y_dtype == kF32 && phi_dtype == kF32) ||
@@ -568,8 +585,8 @@ bool layer_fwd_held_supported(int x_dtype, int y_dtype, int phi_dtype, int B, in
     const int hook = tuning_get(kTuneOnepassOff);
     if (hook) return hook == 3;
     const int nC = n * C;
-    if (x_dtype == kF32) return B >= (n == 4 ? 1850 : (n == 3 ? 1050 : 1000));
-    if (x_dtype == kF32AsBF16) return B >= (nC >= 6144 ? 1300 : (n == 4 ? 2200 : 1600));
+    if (x_dtype == kF32) return B >= (n == 4 ? batch_line(kHeldF32N4, C) : n == 3 ? batch_line(kHeldF32N3, C) : batch_line(kHeldF32N2, C));
+    if (x_dtype == kF32AsBF16) return B >= (n == 4 ? batch_line(kHeldStoredN4, C) : n == 3 ? batch_line(kHeldStoredN3, C) : batch_line(kHeldStoredN2, C));
     // (where the one-launch forward of layer_fwd_onepass.hip stands beside it: from its second round of workgroups on)
     if (layer_fwd_onepass_supported(x_dtype, phi_dtype, B, n, C))
         return (nC >= 1536 || (from_params && C >= 128)) && B > 256 * layer_fwd_onepass_most_samples(n, C);

@@ -27,6 +27,7 @@ enum TuneKey {
 // What mhc_tuning_route() of the same build tells about the built-in heuristic, for tests of its lines.
 enum RouteKey {
     kRouteBackward = 0,     // n <= 8, bf16 arithmetic: 0 = sample-resident, 1 = tiled
+    kRouteForward = 1,      // dynamic forward from the caller's fp32 parameters: 0 = two launches, 1 = one launch from packed phi, 2 = one that reads them itself, 3 = held
 };
 
 #ifdef MHC_TUNING

@@ -1,17 +1,42 @@
 """Which launch path a call takes, on either side of the lines at which two paths cost the same (mhc_tuning_route of the tuning
 build: the built-in rules, no GPU needed).  Every row is a size at which one of the two was measured to be the faster one; the
-figures stand beside the rules (csrc/capi.hip)."""
+figures stand beside the rules (csrc/capi.hip, csrc/layer_fwd_held.hip)."""
+import subprocess
+import sys
+
 import pytest
 
 F32, BF16, F32_AS_BF16 = 0, 1, 2
-BACKWARD = 0
+BACKWARD, FORWARD = 0, 1
 RESIDENT, TILED = 0, 1
+TWO, ONE, ONE_READS, HELD = 0, 1, 2, 3
+
+_CHILD = """
+import ctypes, sys
+lib = ctypes.CDLL(sys.argv[1])
+for line in sys.stdin:
+    print(lib.mhc_tuning_route(*map(int, line.split())), flush=True)
+"""
 
 
-def _route(which, dtype, B, n, C):
-    from mhc._lib import tuning_lib
+@pytest.fixture(scope="module")
+def route():
+    """In a process of its own: this one keeps to the product library."""
+    import os
 
-    return tuning_lib().mhc_tuning_route(which, dtype, B, n, C)
+    from mhc import _lib
+
+    path = os.path.join(os.path.dirname(_lib.LIB_PATH), "libmhc_hip_tuning.so")
+    child = subprocess.Popen([sys.executable, "-c", _CHILD, path], stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True)
+
+    def ask(*query):
+        child.stdin.write(" ".join(map(str, query)) + "\n")
+        child.stdin.flush()
+        return int(child.stdout.readline())
+
+    yield ask
+    child.stdin.close()
+    assert child.wait(timeout=60) == 0
 
 
 @pytest.mark.parametrize("n,C,rows", [
@@ -29,6 +54,20 @@ def _route(which, dtype, B, n, C):
     (8, 1792, [(1400, RESIDENT), (1800, TILED)]), (8, 3072, [(2000, RESIDENT)]), (8, 1024, [(1024, RESIDENT), (1060, TILED)]),
     (8, 960, [(8000, RESIDENT)]), (8, 1025, [(8000, RESIDENT)]),  # C % 64 != 0: always the resident path
 ])
-def test_backward_of_float32_storage(n, C, rows):
+def test_backward_of_float32_storage(route, n, C, rows):
     for B, want in rows:
-        assert _route(BACKWARD, F32_AS_BF16, B, n, C) == want, B
+        assert route(BACKWARD, F32_AS_BF16, B, n, C) == want, B
+
+
+@pytest.mark.parametrize("dtype,n,C,rows", [
+    (F32, 2, 640, [(1000, TWO), (1060, HELD)]), (F32, 2, 896, [(1000, TWO), (1150, TWO), (1500, HELD)]),
+    (F32, 2, 1152, [(1100, TWO), (1250, HELD)]), (F32, 2, 1664, [(1150, TWO), (1300, HELD)]), (F32, 2, 2560, [(1000, TWO), (1060, HELD)]),
+    (F32, 3, 576, [(1150, TWO), (1250, HELD)]), (F32, 3, 768, [(1200, TWO), (1500, HELD)]), (F32, 3, 1152, [(1100, TWO), (1250, HELD)]),
+    (F32, 4, 448, [(1950, TWO), (2100, HELD)]), (F32, 4, 1280, [(1500, TWO), (1850, HELD)]),
+    (F32_AS_BF16, 3, 576, [(1700, TWO), (2100, HELD)]), (F32_AS_BF16, 3, 1024, [(1700, TWO), (1850, HELD)]),
+    (F32_AS_BF16, 3, 1152, [(1500, TWO), (1600, HELD)]), (F32_AS_BF16, 4, 320, [(2300, TWO), (2400, HELD)]),
+    (F32_AS_BF16, 4, 1536, [(1150, TWO), (1330, HELD)]),
+])
+def test_forward(route, dtype, n, C, rows):
+    for B, want in rows:
+        assert route(FORWARD, dtype, B, n, C) == want, B
