@@ -45,6 +45,7 @@ struct OnePassArgs {
     PhiSrc src;       // PF32: phi, alpha and bias as the caller stores them
 };
 
+constexpr int kOpReadsPhiBytes = 150 * 1024;  // of packed phi, up to which fp32 parameters are read by the kernel itself
 constexpr int kOpMaxG = 16;      // samples per workgroup: the columns of one 16-wide tile
 constexpr int kOpPadElems = 8;   // LDS row pad (bf16 elements): consecutive rows start 4 banks apart
 constexpr int kOpStagePitch = 72;  // staged phi rows: 128 data bytes + 16 pad (bf16 elements)
@@ -489,11 +490,14 @@ static int onepass_group(int B, int n, int C) {
 // (B=320 C=1280 n=4, 240 KB: 31.4 against 30.3 us); beyond 256 KB it loses everywhere (B=1280 C=2560
 // n=4: 64.1 against 62.2 us).  Elsewhere the two-launch forward (split-K projection, then the fused mix
 // kernel) stays.
-// From the caller's own fp32 parameters (read by the kernel itself, twice the bytes of phi; the two-launch forward reads them in
-// its projection) the window between 120 and 256 KB starts at 1280 samples: n=4 C=1280 B=1024 14.8 against 13.4 us, 1600 16.4 | 16.6;
-// n=2 C=4096 1024 17.5 | 15.2; n=3 C=1920 1024 13.6 | 13.7, 1600 16.2 | 20.2.  Below 120 KB it saves the packing launch (forward
-// us from parameters, packed by a launch -> read here: n=4 C=256 B=7 8.8 -> 7.3, 2048 9.8 -> 8.5, C=512 7 9.9 -> 8.7, n=3 C=640 320 9.4 ->
-// 8.4, n=2 C=1024 7 8.9 -> 7.4).
+// From the caller's own fp32 parameters the two-launch forward reads them in its projection, without a packing launch, and the window
+// between 120 and 256 KB starts later: where this kernel does not read them itself either (layer_fwd_onepass_reads_params()) at 1281
+// samples, forward us, two launches | pack and this: n=4 C=1280 B=1050 14.1 | 15.6, 1400 16.1 | 15.6; n=3 C=1920 1050 14.5 | 15.3, 1400
+// 16.5 | 15.8; C=2560 1200 18.2 | 19.5, 1300 22.7 | 19.4.  Two streams of such rows (C=5120)
+// outgrow the L2 in the two launches from 1025 samples on (1024 18.9 | 20.5, 1050 23.8 | 22.0, 1280 27.0 | 23.6): there this kernel starts
+// at 1025 as well, while one round of workgroups holds the batch (1300 27.3 | 40.8).
+// Below 120 KB reading them here saves the packing launch (forward us from parameters, packed by a launch -> read here: n=4 C=256 B=7
+// 8.8 -> 7.3, 2048 9.8 -> 8.5, C=512 7 9.9 -> 8.7, n=3 C=640 320 9.4 -> 8.4, n=2 C=1024 7 8.9 -> 7.4).
 bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C, bool from_params) {
     const int mode = tuning_get(kTuneOnepassOff);  // 0 = by cost, 1 = never, 2 = whenever the shape allows
     if (mode == 1) return false;
@@ -501,13 +505,20 @@ bool layer_fwd_onepass_supported(int x_dtype, int phi_dtype, int B, int n, int C
     if (OnePassLds(1, n * C, round_up(C / 8, 4), kOnePassWaves).total > 158 * 1024) return false;
     if (mode == 2) return true;
     const long long phi_bytes = 2ll * (n * n + 2 * n) * n * C;
-    return phi_bytes <= 120 * 1024 || (phi_bytes <= 256 * 1024 && B >= (from_params ? 1280 : 1024) && B <= 2048);
+    if (phi_bytes <= 120 * 1024) return true;
+    const bool early = phi_bytes <= kOpReadsPhiBytes || (n <= 2 && B <= 256 * layer_fwd_onepass_most_samples(n, C));
+    return phi_bytes <= 256 * 1024 && B >= (!from_params ? 1024 : early ? 1025 : 1281) && B <= 2048;
 }
 
 // Whether the one-launch forward reads fp32 parameters itself: in one round of workgroups.  That form has one workgroup on a CU, the
 // packed one two, and with more samples it takes two rounds (forward us, packed by a launch | read here: n=1 C=512 B=4000 10.1 | 9.0,
 // 4500 12.2 | 15.7;  n=2 C=512 4000 11.5 | 10.1, 4200 13.4 | 17.1, 8192 14.7 | 18.1;  n=4 C=256 4000 11.5 | 10.6, 4200 13.1 | 17.7).
-bool layer_fwd_onepass_reads_params(int B, int n, int C) { return B <= 256 * layer_fwd_onepass_most_samples(n, C); }
+// And up to 150 KB of phi, twice that as float32 for every workgroup: n=4 C=704 (132 KB) 1200 11.8 | 11.4, C=768 1500 13.7 | 13.5;  n=3 C=1600
+// (141 KB) 1200 13.8 | 13.4, 1400 14.5 | 15.1;  n=2 C=5120 (160 KB) 1100 22.8 | 23.3;  n=4 C=1280 1500 15.8 | 16.5;  n=3 C=2560 1400
+// 19.8 | 20.4, C=2880 1400 21.8 | 22.6.
+bool layer_fwd_onepass_reads_params(int B, int n, int C) {
+    return B <= 256 * layer_fwd_onepass_most_samples(n, C) && 2ll * (n * n + 2 * n) * n * C <= kOpReadsPhiBytes;
+}
 
 bool layer_fwd_onepass_gathers(const ParamGather &g) {
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };

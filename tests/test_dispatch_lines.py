@@ -1,6 +1,6 @@
 """Which launch path a call takes, on either side of the lines at which two paths cost the same (mhc_tuning_route of the tuning
 build: the built-in rules, no GPU needed).  Every row is a size at which one of the two was measured to be the faster one; the
-figures stand beside the rules (csrc/capi.hip, csrc/layer_fwd_held.hip)."""
+figures stand beside the rules (csrc/capi.hip, csrc/layer_fwd_held.hip, csrc/layer_fwd_onepass.hip)."""
 import subprocess
 import sys
 
@@ -67,6 +67,12 @@ def test_backward_of_float32_storage(route, n, C, rows):
     (F32_AS_BF16, 3, 576, [(1700, TWO), (2100, HELD)]), (F32_AS_BF16, 3, 1024, [(1700, TWO), (1850, HELD)]),
     (F32_AS_BF16, 3, 1152, [(1500, TWO), (1600, HELD)]), (F32_AS_BF16, 4, 320, [(2300, TWO), (2400, HELD)]),
     (F32_AS_BF16, 4, 1536, [(1150, TWO), (1330, HELD)]),
+    # the one-launch forward: phi up to 120 KB, up to 150, up to 256, and beyond
+    (BF16, 4, 256, [(7, ONE_READS), (4000, ONE_READS), (4200, HELD)]), (BF16, 4, 64, [(5000, ONE)]),
+    (BF16, 4, 704, [(1024, TWO), (1100, ONE_READS)]), (BF16, 3, 1600, [(1024, TWO), (1100, ONE_READS)]),
+    (BF16, 2, 4096, [(1024, TWO), (1100, ONE_READS)]), (BF16, 2, 5120, [(1024, TWO), (1100, ONE)]),
+    (BF16, 2, 6144, [(1100, TWO)]), (BF16, 4, 1280, [(1100, TWO), (1280, TWO), (1400, ONE), (2048, ONE)]),
+    (BF16, 3, 2560, [(1200, TWO), (1300, ONE)]), (BF16, 4, 1408, [(1400, TWO)]),
 ])
 def test_forward(route, dtype, n, C, rows):
     for B, want in rows:

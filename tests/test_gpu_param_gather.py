@@ -60,7 +60,7 @@ def test_parameters_read_by_the_projection_match_the_packing_launch(B, n, C, mix
 
 @pytest.mark.parametrize("B,n,C,mixed", [
     (1, 4, 64, False), (37, 4, 64, False), (300, 4, 128, False), (3000, 2, 64, False), (9, 3, 640, False), (40, 1, 128, False),
-    (1500, 4, 832, False),                              # one launch: one workgroup, fewer steps than workgroups, two row pieces, steps from each workgroup's own starting point
+    (1500, 4, 768, False),                              # one launch: one workgroup, fewer steps than workgroups, two row pieces, steps from each workgroup's own starting point
     (4112, 4, 384, False), (1700, 3, 192, True),        # sixteen samples per workgroup
 ])
 def test_parameters_read_by_the_one_pass_forwards(B, n, C, mixed):
