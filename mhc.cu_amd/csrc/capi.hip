@@ -388,6 +388,7 @@ __attribute__((visibility("default"))) int mhc_tuning_route(int route, int x_dty
             const bool exact = x_dtype == kF32;
             return forward_route(x_dtype, x_dtype == kBF16 ? kBF16 : kF32, exact ? kF32 : kBF16, B, n, C, false, &g, carve_dyn_fwd(nullptr, B, n, C).part_bytes).kind;
         }
+        case kRouteSums: return x_dtype == kF32 ? bwd_reduce_form_f32(B, n, C) : -1;
         default: return -1;
     }
 }

@@ -173,10 +173,11 @@ hipError_t launch_mix_bwd_reduce(const void *dy, int y_dtype, const void *x, int
 // static_logits / static_state (optional, static H, n > 8): the channel-sum launch also recomputes the
 // Sinkhorn forward of the shared logits and leaves its denominators in static_state ((2 T + 2) * 32 floats)
 // for launch_finalize_static.
-// raw (optional, dynamic H, n <= 8): scratch of B * bwd_reduce_parts() * (NP*NP + 3*NP + 1) floats;
-// when given, the channel sums and the coefficient backward run as two launches.
+// raw (required for dynamic H and for n > 8): scratch of bwd_reduce_raw_floats() floats, the channel sums between two launches; with
+// n <= 8 and dynamic H the coefficient backward may also run in the launch of the sums, which then leaves raw alone.
 int bwd_reduce_parts(int B, int n, int C);
-size_t bwd_reduce_raw_floats(int B, int n, int C);  // size of `raw` (required for n > 8)
+size_t bwd_reduce_raw_floats(int B, int n, int C);  // size of `raw`
+int bwd_reduce_form_f32(int B, int n, int C);  // n <= 8, fp32 tier: 0 = two launches, 1 = one, 2 = one with a wave per sample
 // n > 16, dynamic H, bf16 dy and x: the same two launches, the second also holding the workgroups of
 // the matrix-core dx kernel in the form that needs no result of the coefficient backward
 // (dxp = M^T dy + Hpre (x) da into `dxp`, fp32 [B][n][C]; df or the dw rows u); they run beside the

@@ -1496,18 +1496,31 @@ static hipError_t launch_gram_small_static(BwdReduceArgs a, hipStream_t stream) 
 // kSumsCoef has fewer workgroups and, with 104 registers (n <= 4), four waves per SIMD instead of six: it pays while its workgroups are
 // resident together, and with two parts once there are enough of them to fill the chip.  A wave per sample has nobody wait for the
 // coefficient backward, but a long row's loads come one after the other, and those of single elements (!wide) most of all: n=4 C=515
-// B=1500 56.1 | | 57.3, n=2 C=1283 B=1200 57.3 | | 63.6, n=7 C=221 B=1026 58.2 | 60.3.  4096 waves are on the chip at once (n=4
-// C=128 B=4311 43.8 | | 46.7).  Not with a Sinkhorn state that would take the LDS of the workgroups beside it.
-static ReduceForm reduce_small_form(const BwdReduceArgs &a, bool wide) {
-    const int B = a.B, C = a.C;
-    if (a.T > 32) return kSumsOnly;
-    if (const int hook = tuning_get(kTuneGramFused)) return hook == 3 && a.n <= 4 ? kWaveCoef : hook >= 2 ? kSumsCoef : kSumsOnly;  // experiment hook
-    if (a.n > 4) return (a.parts == 1 ? B <= (!wide ? 768 : C <= 512 ? 2047 : 1024) : B >= 384 && B <= 768) ? kSumsCoef : kSumsOnly;
-    if (C <= 256) return B <= 4096 ? kWaveCoef : kSumsOnly;
-    if (C <= 512 && wide) return B <= 1700 ? kSumsCoef : B <= 6000 ? kWaveCoef : kSumsOnly;
-    if (C <= 3072 && wide && B > 1024) return kWaveCoef;
-    return B <= 1024 && (a.parts == 1 || B > 512) ? kSumsCoef : kSumsOnly;
+// B=1500 56.1 | | 57.3, n=2 C=1283 B=1200 57.3 | | 63.6, n=7 C=221 B=1026 58.2 | 60.3.  Not with a Sinkhorn state that would take the LDS
+// of the workgroups beside it.
+// 4096 waves are on the chip at once, and a wave per sample loses behind them (forward + backward us, two launches | kWaveCoef: n=1 C=512 4096
+// 54.2 | 52.1, 4200 57.4 | 60.5;  C=1280 4096 78.5 | 74.7, 4200 82.0 | 84.9;  n=4 C=768 4096 96.0 | 91.9, 4200 112 | 113) and, with few
+// streams, in long rows of few samples (n=1 C=1600 1030 42.8 | 43.2;  C=1920 1100 47.8 | 49.3, 1500 51.7 | 51.2;  C=2816 1300 65.6 | 67.7, 1800
+// 77.3 | 76.9;  C=3072 1800 75.6 | 78.3;  n=2 C=3072 1100 76.4 | 78.2, 1400 84.9 | 85.1).
+// Two parts, n > 4: a full round of the two launches is 384 samples where a part has four waves, 512 where it has three (two launches |
+// kSumsCoef: n=5 C=1600 384 79.7 | 82.0, 400 85.5 | 82.9;  C=1280 450 78.8 | 80.3, 540 87.6 | 85.0;  n=6 C=2112 450 115 | 116, 512 122 | 119;
+// single elements n=5 C=1285 450 85.1 | 88.9, 540 100.6 | 102.2, n=2 C=1283 800 61.3 | 62.4, n=4 C=1283 800 77.6 | 78.0).
+static ReduceForm reduce_small_form(int B, int n, int C, int T, int parts, bool wide) {
+    if (T > 32) return kSumsOnly;
+    if (const int hook = tuning_get(kTuneGramFused)) return hook == 3 && n <= 4 ? kWaveCoef : hook >= 2 ? kSumsCoef : kSumsOnly;  // experiment hook
+    if (n > 4) {
+        if (parts == 1) return B <= (!wide ? 768 : C <= 512 ? 2047 : 1024) ? kSumsCoef : kSumsOnly;
+        const int per_part = C / 4, waves = (per_part / ((per_part + 255) / 256) + 63) / 64;  // chunks of two channels
+        return wide && B > (waves == 3 ? 512 : 384) && B <= 768 ? kSumsCoef : kSumsOnly;
+    }
+    if (B > 4096) return kSumsOnly;
+    if (C <= 256) return kWaveCoef;
+    if (C <= 512 && wide) return B <= 1700 ? kSumsCoef : kWaveCoef;
+    const int from = n == 1 ? (C <= 1800 ? 1025 : C <= 2560 ? 1500 : C <= 2816 ? 1800 : kNever) : n < 4 && C > 2560 ? 1300 : 1025;
+    if (C <= 3072 && wide && B >= from) return kWaveCoef;
+    return B <= 1024 && (parts == 1 || (wide && B > (n <= 2 ? 640 : 512))) ? kSumsCoef : kSumsOnly;
 }
+int bwd_reduce_form_f32(int B, int n, int C) { return reduce_small_form(B, n, C, 20, bwd_reduce_parts(B, n, C), C % (n <= 4 ? 4 : 2) == 0); }
 
 template <typename TG, typename TX, int NP, int V>
 static hipError_t launch_small(BwdReduceArgs a, hipStream_t stream) {
@@ -1516,7 +1529,7 @@ static hipError_t launch_small(BwdReduceArgs a, hipStream_t stream) {
         // static H: worth it once the batch fills the chip (one workgroup per sample)
         if (a.hstride == 0 && a.C % 8 == 0 && a.B >= 128) return launch_gram_small_static<NP>(a, stream);
     }
-    const ReduceForm form = a.hstride != 0 ? reduce_small_form(a, V > 1) : kSumsOnly;
+    const ReduceForm form = a.hstride != 0 ? reduce_small_form(a.B, a.n, a.C, a.T, a.parts, V > 1) : kSumsOnly;
     if (form != kSumsOnly) a.raw = nullptr;  // (kSumsCoef: at most two parts)
     if (form == kWaveCoef) a.parts = 1;
     const int nch = (a.C / V + a.parts - 1) / a.parts;  // chunks per column part

@@ -28,6 +28,7 @@ enum TuneKey {
 enum RouteKey {
     kRouteBackward = 0,     // n <= 8, bf16 arithmetic: 0 = sample-resident, 1 = tiled
     kRouteForward = 1,      // dynamic forward from the caller's fp32 parameters: 0 = two launches, 1 = one launch from packed phi, 2 = one that reads them itself, 3 = held
+    kRouteSums = 2,         // channel sums of the fp32 tier, n <= 8: 0 = two launches, 1 = one, 2 = one with a wave per sample
 };
 
 #ifdef MHC_TUNING

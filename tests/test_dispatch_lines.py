@@ -1,15 +1,17 @@
 """Which launch path a call takes, on either side of the lines at which two paths cost the same (mhc_tuning_route of the tuning
 build: the built-in rules, no GPU needed).  Every row is a size at which one of the two was measured to be the faster one; the
-figures stand beside the rules (csrc/capi.hip, csrc/layer_fwd_held.hip, csrc/layer_fwd_onepass.hip)."""
+figures stand beside the rules (csrc/capi.hip, csrc/layer_fwd_held.hip, csrc/layer_fwd_onepass.hip,
+csrc/mix_bwd_reduce.hip)."""
 import subprocess
 import sys
 
 import pytest
 
 F32, BF16, F32_AS_BF16 = 0, 1, 2
-BACKWARD, FORWARD = 0, 1
+BACKWARD, FORWARD, SUMS = 0, 1, 2
 RESIDENT, TILED = 0, 1
 TWO, ONE, ONE_READS, HELD = 0, 1, 2, 3
+APART, FUSED, WAVE = 0, 1, 2
 
 _CHILD = """
 import ctypes, sys
@@ -77,3 +79,16 @@ def test_backward_of_float32_storage(route, n, C, rows):
 def test_forward(route, dtype, n, C, rows):
     for B, want in rows:
         assert route(FORWARD, dtype, B, n, C) == want, B
+
+
+@pytest.mark.parametrize("n,C,rows", [
+    (1, 512, [(1500, FUSED), (4096, WAVE), (4200, APART)]), (4, 768, [(1000, FUSED), (4096, WAVE), (4200, APART)]),
+    (4, 1280, [(700, FUSED), (2560, WAVE)]), (1, 1600, [(1100, WAVE)]), (1, 1920, [(1100, APART), (1500, WAVE)]),
+    (1, 2816, [(1300, APART), (1800, WAVE)]), (1, 3072, [(2000, APART)]), (2, 3072, [(1100, APART), (1400, WAVE)]),
+    (2, 2048, [(600, APART), (700, FUSED)]), (5, 1600, [(384, APART), (400, FUSED), (800, APART)]),
+    (5, 1280, [(450, APART), (540, FUSED)]), (6, 2112, [(450, APART), (540, FUSED)]), (5, 1285, [(450, APART), (540, APART)]), (2, 1283, [(800, APART)]),
+    (4, 128, [(4311, APART)]), (6, 640, [(1000, FUSED), (1100, APART)]),
+])
+def test_channel_sums_of_the_float32_tier(route, n, C, rows):
+    for B, want in rows:
+        assert route(SUMS, F32, B, n, C) == want, B
