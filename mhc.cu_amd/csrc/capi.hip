@@ -95,20 +95,21 @@ struct DynBwdWs { float *dt, *dP, *cx, *s1, *u, *upart, *dtpart, *raw, *s1part, 
 //   n=6 C=64: 4000 37.2 | 37.4, 4125 42.3 | 39.6, 8192 51.8 | 59.1; C=256: 1200 28.9 | 27.1, 1600 30.4 | 32.1, 8192 55.4 | 76.9
 //       C=384: 655 29.3 | 27.2, 765 27.3 | 29.0; C=768: 647 32.8 | 32.0, 790 30.8 | 35.0; C=1280: 472 29.9 | 27.8, 527 33.5 |
 //       36.1; C=2560: 256 31.8 | 25.1, 307 35.4 | 36.4; C=4096: 227 41.3 | 33.3, 291 44.7 | 48.9
-//   n=7 C=64: 4000 40.1 | 37.8, 8192 54.6 | 60.5; C=256: 1600 32.4 | 32.6, 4000 42.8 | 49.7, 8192 60.7 | 83.0; C=384: 777 35.6 |
+//   n=7 C=64: 4000 40.1 | 37.8, 8192 54.6 | 60.5; C=256: 1600 32.4 | 32.6, 4000 42.8 | 49.7, 8192 60.7 | 83.0 (with the
+//       forward: C=192 2126 53.8 | 51.3, 2400 54.5 | 53.3, 3000 55.9 | 63.7; C=256 2400 56.0 | 55.0, 3000 56.6 | 62.6); C=384: 777 35.6 |
 //       31.4, 1024 31.8 | 32.9, 1163 39.3 | 36.9; C=768: 680 36.0 | 32.7, 832 34.2 | 35.2, 1087 40.4 | 41.4; C=1280: 455 37.4 |
 //       32.3, 705 42.0 | 44.9; C=2560: 361 42.7 | 41.7, 448 41.5 | 45.1
 //   n=8 C=128: 4000 43.8 | 41.2, 8192 61.7 | 66.4; C=256: 2200 40.8 | 36.5, 4000 48.1 | 50.4, 8192 69.4 | 87.0; C=384: 1200 37.4
-//       | 35.0, 1600 39.9 | 42.8; C=512: 1200 42.2 | 40.0, 1600 43.7 | 49.5; C=1280: 569 43.5 | 42.0, 815 49.3 | 55.7; C=2560:
+//       | 35.0, 1600 39.9 | 42.8 (with the forward: C=320 1500 58.1 | 55.9, 1600 58.2 | 62.6); C=512: 1200 42.2 | 40.0, 1600 43.7 | 49.5; C=1280: 569 43.5 | 42.0, 815 49.3 | 55.7; C=2560:
 //       387 52.5 | 49.6, 532 56.4 | 64.1; C=4096: 344 60.8 | 58.2, 539 73.1 | 85.6
 // Experiment hook: 1 = never, 2 = always.
 bool bwd_resident_preferred(int B, int n, int C) {
     if (const int hook = tuning_get(kTuneResident)) return hook == 2;
     if (n > 4) {
         // (large batches of short rows: the channel sums are gram_wave_kernel there)
-        const int upto128[4] = {1500, 5000, 6000, 7000}, upto256[4] = {1200, 1500, 1900, 3700};
+        const int upto128[4] = {1500, 5000, 6000, 7000}, upto256[4] = {1200, 1500, 2450, 3700};
         if (C <= 256) return B <= (C <= 128 ? upto128 : upto256)[n - 5];
-        const int per_row[4] = {500'000, 680'000, 880'000, 940'000}, least[4] = {256, 256, 256, 448}, most[4] = {640, 704, 832, 1400};
+        const int per_row[4] = {500'000, 680'000, 880'000, 940'000}, least[4] = {256, 256, 256, 448}, most[4] = {640, 704, 832, C <= 384 ? 1500 : 1400};
         return B <= std::min(most[n - 5], std::max(least[n - 5], per_row[n - 5] / C));
     }
     if (C <= 256) {

@@ -92,3 +92,10 @@ def test_forward(route, dtype, n, C, rows):
 def test_channel_sums_of_the_float32_tier(route, n, C, rows):
     for B, want in rows:
         assert route(SUMS, F32, B, n, C) == want, B
+
+
+@pytest.mark.parametrize("n,C,rows", [(7, 192, [(2126, RESIDENT), (2400, RESIDENT), (3000, TILED)]), (7, 256, [(2400, RESIDENT), (3000, TILED)]),
+                                      (8, 320, [(1500, RESIDENT), (1600, TILED)]), (8, 512, [(1500, TILED)])])
+def test_backward_of_bf16_storage(route, n, C, rows):
+    for B, want in rows:
+        assert route(BACKWARD, BF16, B, n, C) == want, B
