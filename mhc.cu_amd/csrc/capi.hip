@@ -230,7 +230,8 @@ DynFwdWs carve_dyn_fwd(void *ws, int B, int n, int C) {
 enum ForwardKind { kTwoLaunches, kOneLaunch, kOneLaunchReadsParams, kHeldForward };
 struct ForwardRoute { ForwardKind kind; bool direct; };
 ForwardRoute forward_route(int x_dtype, int y_dtype, int phi_dtype, int B, int n, int C, bool inject, const ParamGather *gather, size_t part_bytes) {
-    const bool direct = gather && aligned16(gather->phi[0]) && aligned16(gather->phi[1]) && aligned16(gather->phi[2]);
+    const bool direct = gather && aligned16(gather->phi[0]) && aligned16(gather->phi[1]) && aligned16(gather->phi[2]) &&
+                        tuning_get(kTuneGather) != 1;
     if (!inject && layer_fwd_held_supported(x_dtype, y_dtype, phi_dtype, B, n, C, direct && gather->phi_dtype == kF32) &&
         layer_fwd_held_bytes(x_dtype, n, C) <= part_bytes)
         return {kHeldForward, direct};

@@ -18,7 +18,7 @@ enum TuneKey {
     kTuneResident = 7,      // n <= 8 sample-resident backward: 0 = by heuristic, 1 = never, 2 = whenever the shape allows
     kTuneWideDxBeside = 8,  // wide projections (n > 18): dx workgroups beside the coefficient launch: 1 = never, 2 = always
     kTuneSpareB = 9,        // projection forward (matrix-core kernels): K splits, 0 = by heuristic
-    kTuneGather = 10,       // projection reads the caller's fp32 parameters itself: 1 = never, 2 = whenever the shape allows
+    kTuneGather = 10,       // the caller's fp32 parameters read by the kernels of the forward themselves: 1 = never, 2 = whenever the shape allows
     kTuneSlabWidth = 11,    // slab backward (n <= 4, bf16): channels per workgroup, 1 = 64, 2 = 128, 0 = by size
     kTuneSlab8 = 12,        // slab backward of n = 5 .. 8 behind the channel sums: 1 = never (general kernels), 2 = always
     kTuneCount = 13
