@@ -535,8 +535,9 @@ template <typename TS, typename TX, int N, int CB, int NW> static hipError_t lau
 constexpr int held_most_cb(int n) { return n == 4 ? 5 : (n == 3 ? 6 : 10); }
 template <typename TS, typename TX, int N> static hipError_t launch_held_by_size(const HeldArgs &a, hipStream_t stream) {
     const int nch = (a.C + HeldShape<TX, N>::CH - 1) / HeldShape<TX, N>::CH;
+// (eight waves for the rows that four do not hold: no form that nothing reaches)
 #define MHC_HELD(CB, NW) \
-    if constexpr (CB <= held_most_cb(N)) { if (nch <= CB * NW) return launch_held<TS, TX, N, CB, NW>(a, stream); }
+    if constexpr (CB <= held_most_cb(N) && (NW == 4 || CB * NW > 4 * held_most_cb(N))) { if (nch <= CB * NW) return launch_held<TS, TX, N, CB, NW>(a, stream); }
     MHC_HELD(1, 4) MHC_HELD(2, 4) MHC_HELD(3, 4) MHC_HELD(4, 4) MHC_HELD(5, 4) MHC_HELD(6, 4) MHC_HELD(8, 4) MHC_HELD(10, 4)
     MHC_HELD(3, 8) MHC_HELD(4, 8) MHC_HELD(5, 8) MHC_HELD(6, 8) MHC_HELD(8, 8) MHC_HELD(10, 8)
 #undef MHC_HELD
