@@ -23,17 +23,17 @@ def _reset_tuning():
     tuning_lib().mhc_tuning_set(K_FORWARD, 0)
 
 
-def _inputs(kind, B, n, C, seed=0):
+def _inputs(kind, B, n, C, seed=0, wt=None):
     g = torch.Generator(device="cuda").manual_seed(seed + B + n + C)
     rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
     act = torch.bfloat16 if kind == BF16 else torch.float32
-    wt = torch.float32 if kind == F32 else torch.bfloat16
+    pt = torch.float32 if kind == F32 else torch.bfloat16
     D = n * n + 2 * n
-    return dict(x=rn(B, n, C).to(act), w=(1 + 0.1 * rn(C)).to(wt), phi=(0.02 * rn(D, n * C)).to(wt), bias=0.5 * rn(D),
+    return dict(x=rn(B, n, C).to(act), w=(1 + 0.1 * rn(C)).to(wt or pt), phi=(0.02 * rn(D, n * C)).to(pt), bias=0.5 * rn(D),
                 alpha=torch.tensor([0.3, 0.4, 0.5], device="cuda"))
 
 
-def _reference(kind, v):
+def _reference(kind, v, T=T):
     x = v["x"].bfloat16().double() if kind == F32_AS_BF16 else v["x"].double()
     B, n, C = x.shape
     al, b = v["alpha"].double(), v["bias"].double()
@@ -52,10 +52,10 @@ def _reference(kind, v):
     a = (Hp[:, :, None] * x).sum(1)
     q = (a.square().mean(1) + EPS).sqrt()
     y = (M[:, :, :, None] * x[:, None]).sum(2) + Ho[:, :, None] * (a / q[:, None] * v["w"].double())[:, None]
-    return dict(P=P, r=r, Hp=Hp, Ho=Ho, M=M, q=q, y=y, sk=torch.stack(sk, 1))
+    return dict(P=P, r=r, Hp=Hp, Ho=Ho, M=M, q=q, y=y, **(dict(sk=torch.stack(sk, 1)) if T else {}))
 
 
-def _forward(kind, v, hook=3):
+def _forward(kind, v, hook=3, T=T, state=True):
     from mhc import _lib
     from mhc._lib import check, dtype_code, ptr
 
@@ -73,7 +73,7 @@ def _forward(kind, v, hook=3):
     check("mhc_layer_fwd_dynamic",
           lib.mhc_layer_fwd_dynamic(ptr(x), code, ptr(v["w"]), dtype_code(v["w"]), ptr(v["phi"]), dtype_code(v["phi"]),
                                     ptr(v["bias"]), ptr(v["alpha"]), None, ptr(out["y"]), dtype_code(out["y"]), ptr(out["Hp"]),
-                                    ptr(out["Ho"]), ptr(out["M"]), ptr(out["P"]), ptr(out["r"]), ptr(out["q"]), ptr(out["sk"]),
+                                    ptr(out["Ho"]), ptr(out["M"]), ptr(out["P"]), ptr(out["r"]), ptr(out["q"]), ptr(out["sk"]) if state else None,
                                     B, n, C, T, EPS, ptr(ws), ws.numel(), _lib.stream_ptr(x.device)))
     torch.cuda.synchronize()
     assert all(torch.isnan(t[B]).all() for t in out.values()), "wrote behind the batch"
@@ -118,6 +118,40 @@ def test_several_rounds(kind, B, n, C):
     _check(kind, _forward(kind, v), _reference(kind, v))
 
 
+@pytest.mark.parametrize("kind", [BF16, F32, F32_AS_BF16])
+@pytest.mark.parametrize("n,C", [(4, 64), (4, 1344), (3, 832), (2, 2624)])
+def test_without_saved_state(kind, n, C):
+    """As inference calls it: the same results bit for bit, and nothing is written where a state would be."""
+    if kind == F32:
+        C //= 2
+    for B in (1, 53):
+        v = _inputs(kind, B, n, C)
+        want, got = _forward(kind, v), _forward(kind, v, state=False)
+        assert torch.isnan(got.pop("sk")).all()
+        for k in got:
+            assert torch.equal(got[k], want[k]), k
+        _check(kind, {**got, "sk": want["sk"]}, _reference(kind, v))
+
+
+@pytest.mark.parametrize("kind", [BF16, F32, F32_AS_BF16])
+@pytest.mark.parametrize("iters", [0, 1, 32])
+@pytest.mark.parametrize("state", [True, False])
+def test_sinkhorn_iterations(kind, iters, state):
+    for n, C in ((4, 320), (3, 64), (2, 192)):
+        v = _inputs(kind, 35, n, C)
+        ref = _reference(kind, v, iters)
+        if not state:
+            ref.pop("sk", None)
+        _check(kind, _forward(kind, v, T=iters, state=state), ref)
+
+
+@pytest.mark.parametrize("kind", [BF16, F32, F32_AS_BF16])
+def test_the_other_type_of_weight(kind):
+    for n, C in ((4, 1344), (3, 192), (2, 2624)):
+        v = _inputs(kind, 37, n, C, wt=torch.bfloat16 if kind == F32 else torch.float32)
+        _check(kind, _forward(kind, v), _reference(kind, v))
+
+
 def test_samples_are_independent():
     """A sample of infinities and one of NaN leave the others of their tile as they were, bit for bit."""
     v = _inputs(BF16, 40, 3, 192)
@@ -131,10 +165,13 @@ def test_samples_are_independent():
 
 @pytest.mark.parametrize("dtype,B,n,C", [(torch.bfloat16, 4200, 4, 384), (torch.bfloat16, 4100, 2, 128), (torch.float32, 1111, 2, 96), (torch.float32, 1100, 3, 64)])
 def test_through_the_module(dtype, B, n, C):
-    """Sizes at which the layer takes this path by itself: the packed parameters that it leaves serve the backward."""
+    """Sizes at which the layer takes this path by itself: the packed parameters that it leaves serve the backward.  And as inference
+    calls it, without a state to keep: the same y."""
     import mhc
+    from mhc._lib import tuning_lib
     from oracle import naive_mhc as nm
 
+    assert tuning_lib().mhc_tuning_route(1, 1 if dtype == torch.bfloat16 else 0, B, n, C) == 3
     torch.manual_seed(1)
     with torch.device("cuda"):
         layer = mhc.MHCLayer(C, n, output_dtype=dtype if dtype == torch.bfloat16 else None)
@@ -149,6 +186,8 @@ def test_through_the_module(dtype, B, n, C):
         dy = torch.randn(B, n, C, dtype=dtype)
     y = layer(x)
     y.backward(dy)
+    with torch.no_grad():
+        assert torch.equal(layer(x), y)
     torch.cuda.synchronize()
     params = {k: getattr(layer, k).detach().double() for k in nm.DYN_PARAM_NAMES if k != "w"}
     params["w"] = layer.rmsnorm_weight.detach().double()
