@@ -411,7 +411,7 @@ __global__ __launch_bounds__(256, 2) void bwd_slab_f32dy_kernel(BwdSlabArgs a) {
 // through two places of its own.  Backward in graphs of ten, resident path -> channel sums and this: n=4 B=4369 C=1280 142 -> 113 us,
 // 2000 2560 133 -> 90, n=3 3000 3136 199 -> 124, n=2 4369 2560 185 -> 105.
 template <int N, int CW, bool F32> struct SlabStage {
-    static_assert(!F32 || CW == 64, "the pieces of a row are 64 channels wide");
+    static_assert(!F32 || CW == f32_piece_channels(N), "a slab reads whole pieces");
     static constexpr int TB = 16, kLoaders = CW / 32, kMixers = CW / 16, kThreads = 64 * (kLoaders + kMixers);  // 6 CW
     static constexpr int kXAhead = 3, kGAhead = F32 ? 0 : 2;  // tiles requested ahead
     static constexpr int kXRing = kXAhead + 1, kGRing = kGAhead + 2;
@@ -819,7 +819,7 @@ bool bwd_slab_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) {
 //   n=3  1500 x 1920 31.6 | 29.5   n=2  4000 x 1024 34.4 | 32.1   1000 x 2560 29.6 | 27.2
 // The lines: n = 4 up to 1280 channels, or below 12 M activation elements.
 static int slab_width(int B, int n, int C, bool f32 = false) {
-    if (f32) return 64;
+    if (f32) return f32_piece_channels(n);
     if (const int forced = tuning_get(kTuneSlabWidth)) return forced == 1 ? 64 : 128;
     return n == 4 && (C <= 1280 || (long long)B * n * C < 12'000'000) ? 64 : 128;
 }

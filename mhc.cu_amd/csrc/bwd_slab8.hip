@@ -49,7 +49,7 @@ struct BwdSlab8Args {
 // the LDS holds that for 32 channels (two mixers).  Whole backward, resident path -> this: n=5 B=2000 C=2560 198 -> 116 us, n=6 B=3000
 // C=1024 146 -> 83, n=7 B=3000 C=1024 160 -> 109, n=8 B=4369 C=1024 269 -> 211.
 template <int N, bool F32> struct Slab8Stage {
-    static constexpr int CW = F32 && N > 6 ? 32 : 64, TB = 16, kMixers = CW / 16, kHolders = 4, kThreads = 64 * (kMixers + kHolders);  // waves
+    static constexpr int CW = F32 ? f32_piece_channels(N) : 64, TB = 16, kMixers = CW / 16, kHolders = 4, kThreads = 64 * (kMixers + kHolders);  // waves
     static constexpr int kRowBytes = CW * (F32 ? 4 : 2), kChunks = kRowBytes / 16, kRows = 1024 / kRowBytes;  // of a tile's row; rows per KiB
     static constexpr int kRing8 = kChunks * 8;                         // what slab_swizzle() goes by
     static constexpr int D = N * N + 2 * N, NTD = (D + 31) / 32, DP = 32 * NTD;
@@ -457,7 +457,7 @@ bool bwd_slab8_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C) 
     return x_dtype == kBF16 && y_dtype == kBF16 && phi_dtype == kBF16 && n >= 5 && n <= 8 && C % 8 == 0;
 }
 
-static int slab8_width(int n, bool f32) { return f32 && n > 6 ? 32 : 64; }
+static int slab8_width(int n, bool f32) { return f32 ? f32_piece_channels(n) : 64; }
 int bwd_slab8_slabs(int n, int C, bool f32) { return (C + slab8_width(n, f32) - 1) / slab8_width(n, f32); }
 
 // At most one workgroup per CU and at least three tiles each, and within that the splits that cost least: a tile is some 0.2 n us

@@ -156,6 +156,10 @@ struct BwdCoefOut {
     int BP;               // row pitch of dPT, a multiple of 32 that is >= B
 };
 
+// Float32 storage of bf16 arithmetic, the tiled backward (n <= 8, dynamic H, C % 64 == 0): these channel sums round dy and x on their way
+// in and leave both in `copy`, which is dx [B, n, C] as float32: a piece of f32_piece_channels(n) channels of a row becomes as many bf16
+// of x, then as many of dy, in the same bytes.  launch_bwd_slab (n <= 4) and launch_bwd_slab8 read them there and put dx in their place.
+constexpr int f32_piece_channels(int n) { return n > 6 ? 32 : 64; }  // the width of their slabs, too
 hipError_t launch_mix_bwd_reduce_f32_as_bf16(const float *dy, const float *x, const void *w, int w_dtype, const float *Hpre, const float *Hpost,
                                              const float *M, const float *q, const float *P, const float *r, const float *alpha,
                                              const float *b_res, const float *sk_state, BwdCoefOut out, void *copy, int B, int n, int C,
@@ -208,7 +212,8 @@ hipError_t launch_mix_bwd_dx(const void *dy, int y_dtype, const void *x, int x_d
 
 // Slab kernel for n <= 4 in the bf16 tier: dx (complete), df, and the batch-split partial sums of
 // dphi [S][D][nC], dw [S][C] and dt [S][D+3] (the last two in float64) in one pass over dy and x.  With S == 1 pass the final
-// dphi as dphi_part.
+// dphi as dphi_part.  y_dtype kF32AsBF16: dx holds x and dy as launch_mix_bwd_reduce_f32_as_bf16 has just left them, and becomes dx in
+// float32; dy and x are not read, no f_inject.
 bool bwd_slab_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C);
 int bwd_slab_batch_splits(int B, int n, int C, int y_dtype);
 hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const void *w, int w_dtype,
@@ -219,9 +224,9 @@ hipError_t launch_bwd_slab(const void *dy, int y_dtype, const void *x, const voi
                            int B, int n, int C, hipStream_t stream);
 
 // The same for n = 5 .. 8 (bf16 dy and x), behind launch_mix_bwd_reduce (dP fragments, cx, s1, dt of `co`): dw_part [S][C],
-// dt_part [S bwd_slab8_slabs()][D+3].
+// dt_part [S bwd_slab8_slabs()][D+3].  f32: float32 storage, as y_dtype kF32AsBF16 of launch_bwd_slab (dy = x = nullptr).
 bool bwd_slab8_supported(int x_dtype, int y_dtype, int phi_dtype, int n, int C);
-int bwd_slab8_slabs(int n, int C, bool f32);  // f32: float32 storage of bf16 arithmetic, see launch_bwd_slab8
+int bwd_slab8_slabs(int n, int C, bool f32);
 int bwd_slab8_batch_splits(int B, int n, int C, bool f32);
 hipError_t launch_bwd_slab8(const void *dy, const void *x, const void *w, int w_dtype, const void *f_inject, const void *phi,
                             const float *Hpre, const float *Hpost, const float *M, const float *q, const BwdCoefOut &co,

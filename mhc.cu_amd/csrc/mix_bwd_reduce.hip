@@ -1681,7 +1681,7 @@ hipError_t launch_mix_bwd_reduce_f32_as_bf16(const float *dy, const float *x, co
     BwdReduceArgs a{dy, x, w, nullptr, Hpre, Hpost, M, q, P, r, alpha, b_res, sk_state, out,
                     n, w_dtype == kBF16, B, n, C, T, padded_D(n), eps, nullptr, 1};
     a.copy = copy;
-    a.copy_block = n > 6 ? 32 : 64;  // the widths of the slab kernels
+    a.copy_block = f32_piece_channels(n);
     return n <= 4 ? launch_gram_small<4>(a, stream) : launch_gram_small<8>(a, stream);
 }
 
