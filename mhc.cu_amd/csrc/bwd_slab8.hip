@@ -46,8 +46,8 @@ struct BwdSlab8Args {
 
 // F32: float32 storage, as in bwd_slab.hip: the channel sums have left x and dy in bf16 where dx will be, and the bytes of CW channels
 // of dx hold CW of x, then CW of dy.  x and dy are one tile, two ahead, and dx leaves through two places of its own; at n = 7 and 8
-// the LDS holds that for 32 channels (two mixers).  Whole backward, resident path -> this: n=5 B=2000 C=2560 198 -> 116 us, n=6 B=3000
-// C=1024 146 -> 83, n=7 B=3000 C=1024 160 -> 109, n=8 B=4369 C=1024 269 -> 211.
+// the LDS holds that for 32 channels (two mixers); n = 8 keeps 19 registers in scratch memory, 80 bytes a lane.  Whole backward, resident
+// path -> this: n=5 B=2000 C=2560 198 -> 116 us, n=6 B=3000 C=1024 146 -> 83, n=7 B=3000 C=1024 160 -> 109, n=8 B=4369 C=1024 269 -> 211.
 template <int N, bool F32> struct Slab8Stage {
     static constexpr int CW = F32 ? f32_piece_channels(N) : 64, TB = 16, kMixers = CW / 16, kHolders = 4, kThreads = 64 * (kMixers + kHolders);  // waves
     static constexpr int kRowBytes = CW * (F32 ? 4 : 2), kChunks = kRowBytes / 16, kRows = 1024 / kRowBytes;  // of a tile's row; rows per KiB

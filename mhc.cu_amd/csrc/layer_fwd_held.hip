@@ -11,6 +11,8 @@
 //                 its next tile, whose first pieces are requested as registers fall free
 // sixteen samples and no fewer, because every tile reads all of phi; whole lines, because a store of half a line costs
 // as much as a whole one (operand layout instead of rows, n=4 B=8192 C=2560: 88 us, 70 with this one).
+// The registers are full: 19 of the 84 forms keep 1 to 18 of them in scratch memory (bf16 n=4 at five chunks per wave, the form of
+// C=2560: 5; float32 storage, whose loads wait unrounded beside the held rows: up to 18).
 // It is bound by memory in its load and store phases (the tile's arithmetic overlaps with them only between the workgroups of a
 // CU, which is why rows of at most 1280 channels, two or more workgroups per CU, gain most).  Forward us, two launches ->
 // this one, the packing of phi included: bf16 n=4 B=8192 C=2560 87.8 -> 68.8 (4.9 TB/s on x and y), 8192 1280 52.2 -> 38.2,
