@@ -36,22 +36,22 @@ HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 # `--copy-calibration` (a 64 MiB copy).  Filled from the committed counter summary
 # (profiles/hbm_traffic_counters.txt); `commit` is the revision of the kernels the counters ran on.
 MEASURED_TRAFFIC = {
-    "commit": "59765ab",
-    "bytes": {"c1": 13286154, "c2": 39653990, "c3": 251258479, "c4": 66407695, "c5": 577635270},
+    "commit": "a0b948c",
+    "bytes": {"c1": 13286143, "c2": 39653991, "c3": 251311833, "c4": 66407603, "c5": 577618028},
 }
 
 # The kernel with the largest share of a step's device time, from the committed kernel-trace summaries
 # (profiles/layer_step_<config>.txt): average duration per dispatch and the HBM bytes the algorithm
 # needs that kernel to move (its own inputs and outputs once; for the split projections the partial
 # sums are not counted).
-PROFILED_AT = "59765ab"
+PROFILED_AT = "a0b948c"
 PROFILED_DOMINANT = {
-    "c1": dict(kernel="layer_fwd_small_kernel<float,float,4,4,2>", us=6.82, bytes=2 * 4 * 320 * 4 * 1280),
+    "c1": dict(kernel="layer_fwd_small_kernel<float,float,4,4,2>", us=6.58, bytes=2 * 4 * 320 * 4 * 1280),
     # sample-resident backward kernel: reads dy and x, writes the partial dx and the fp32 rows the batch sums are made of
-    "c2": dict(kernel="bwd_resident_kernel<4,bf16 w,2 items,5 tile waves>", us=9.16, bytes=3 * 2 * 320 * 4 * 1280 + 4 * 320 * 1280),
-    "c3": dict(kernel="bwd_slab_stage_kernel<4,128 channels>", us=18.62, bytes=3 * 2 * 1280 * 4 * 2560 + 2 * 24 * 10240 + 4 * 24 * 10240),
-    "c4": dict(kernel="bwd_resident_kernel<8,bf16 w,1 item,10 tile waves>", us=11.29, bytes=3 * 2 * 256 * 8 * 1280 + 4 * 256 * 1280),
-    "c5": dict(kernel="dphi_large_kernel<9,true>", us=36.59, bytes=2 * 128 * 40960 + 4 * 1088 * 40960),
+    "c2": dict(kernel="bwd_resident_kernel<4,bf16 w,2 items,5 tile waves>", us=9.46, bytes=3 * 2 * 320 * 4 * 1280 + 4 * 320 * 1280),
+    "c3": dict(kernel="bwd_slab_stage_kernel<4,128 channels>", us=18.84, bytes=3 * 2 * 1280 * 4 * 2560 + 2 * 24 * 10240 + 4 * 24 * 10240),
+    "c4": dict(kernel="bwd_resident_kernel<8,bf16 w,1 item,10 tile waves>", us=11.22, bytes=3 * 2 * 256 * 8 * 1280 + 4 * 256 * 1280),
+    "c5": dict(kernel="dphi_large_kernel<9,true>", us=35.34, bytes=2 * 128 * 40960 + 4 * 1088 * 40960),
 }
 
 CONFIGS = {
