@@ -77,3 +77,53 @@ def test_layer_beyond_2_31_elements(B, n, C, dyn, bf16):
         assert e <= bar, f"d{k}: full batch vs the two halves {e:.2e}"
     del x, dy, y, dx, dx1, dx2
     torch.cuda.empty_cache()   # tens of GB: hand them back before the next test
+
+
+@pytest.mark.parametrize("compute", [torch.bfloat16, None])
+def test_float32_storage_beyond_2_31_elements(compute):
+    """The one-pass forward, the channel sums that leave x and dy in bf16 in dx, and the slab kernel behind them; the same in float32."""
+    import mhc
+
+    B, n, C = 530000, 4, 1024
+    assert B * n * C > 2 ** 31
+    if torch.cuda.mem_get_info()[0] < 14 * B * n * C * 4:
+        pytest.skip("needs 120 GB of free device memory")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn(B, n, C, device="cuda", generator=g)
+    dy = torch.randn(B, n, C, device="cuda", generator=g)
+    with torch.device("cuda"):
+        layer = mhc.MHCLayer(C, n, compute_dtype=compute)
+        with torch.no_grad():
+            for p in (layer.phi_pre, layer.phi_post, layer.phi_res):
+                p.copy_(p.bfloat16())
+            for a in (layer.alpha_pre, layer.alpha_post, layer.alpha_res):
+                a.fill_(0.1)
+
+    def run(x, dy):
+        x = x.detach().requires_grad_(True)
+        for p in layer.parameters():
+            p.grad = None
+        y = layer(x)
+        y.backward(dy)
+        torch.cuda.synchronize()
+        return y.detach(), x.grad, {k: p.grad.double() for k, p in layer.named_parameters()}
+
+    y, dx, gp = run(x, dy)
+    last_below = 2 ** 31 // (n * C)
+    idx = torch.tensor([0, 1, 31, 32, B // 2 - 1, B // 2, last_below, last_below + 1, B - 33, B - 2, B - 1], device="cuda")
+    rnd = (lambda t: t.bfloat16().double()) if compute else (lambda t: t.double())
+    params = {k: getattr(layer, k).detach().double().cpu() for k in nm.DYN_PARAM_NAMES if k != "w"}
+    params["w"] = layer.rmsnorm_weight.detach().double().cpu()
+    y_ref, g_ref = nm.mhc_dynamic_fwd_bwd(rnd(x[idx]).cpu(), params, rnd(dy[idx]).cpu(), layer.sinkhorn_iters, layer.eps, dtype=torch.float64)
+    assert rel_err(y[idx].double().cpu(), y_ref) <= 1e-5
+    # (dP phi is a product of bf16 operands: 2^-9 of a term that is a part of dx)
+    assert rel_err(dx[idx].double().cpu(), torch.as_tensor(g_ref["x"])) <= (2e-3 if compute else 1e-5)
+    h = B // 2
+    (_, dx1, g1), (_, dx2, g2) = run(x[:h], dy[:h]), run(x[h:], dy[h:])
+    assert torch.equal(dx[:32], dx1[:32]) and torch.equal(dx[-33:], dx2[-33:])
+    for k in gp:
+        # float32 sums in a different order; dw comes back in the parameter's bf16
+        e = rel_err(gp[k].cpu(), (g1[k] + g2[k]).cpu())
+        assert e <= (1e-2 if k == "rmsnorm_weight" else 2e-3 if compute else 1e-4), f"d{k}: full batch vs the two halves {e:.2e}"
+    del x, dy, y, dx, dx1, dx2
+    torch.cuda.empty_cache()
